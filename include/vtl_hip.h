@@ -68,9 +68,17 @@ int vtl_hip_set_device(int device_id);
 /* Name and compute-unit count of the current device (diagnostics only). */
 int vtl_hip_device_info(char *name, size_t name_cap, int *compute_units, int *clock_mhz);
 
-/* C.cudaMalloc storage/cuda_d_cuda.v:39; C.cudaFree :100. */
+/* C.cudaMalloc storage/cuda_d_cuda.v:39; C.cudaFree :100.  Released memory is kept (at most
+ * 8 GiB, blocks of up to 4 GiB) and handed out again.  vtl_hip_free does not wait while
+ * the process has only used the null stream, whose order keeps the old and the new use of a
+ * block apart; once a thread has called vtl_hip_set_stream with a stream of its own, it
+ * waits for the device.  A program that lets work of its own use such memory on a non-blocking
+ * stream that it never named to the library waits for that work before it releases the memory.
+ * When the driver has no memory left, what is kept is given back and the call tried again;
+ * vtl_hip_trim gives it back at once. */
 int vtl_hip_malloc(void **dptr, size_t bytes);
 int vtl_hip_free(void *dptr);
+int vtl_hip_trim(void);
 
 /* C.cudaMemcpy H2D storage/cuda_d_cuda.v:46, D2H :74,:90 (blocking). */
 int vtl_hip_memcpy_h2d(void *dst_device, const void *src_host, size_t bytes);

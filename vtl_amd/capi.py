@@ -29,6 +29,7 @@ SIGNATURES = {
     "vtl_hip_device_info": (_ci, [C.c_char_p, _sz, C.POINTER(_ci), C.POINTER(_ci)]),
     "vtl_hip_malloc": (_ci, [_pp, _sz]),
     "vtl_hip_free": (_ci, [_vp]),
+    "vtl_hip_trim": (_ci, []),
     "vtl_hip_memcpy_h2d": (_ci, [_vp, _vp, _sz]),
     "vtl_hip_memcpy_d2h": (_ci, [_vp, _vp, _sz]),
     "vtl_hip_memcpy_d2d": (_ci, [_vp, _vp, _sz]),

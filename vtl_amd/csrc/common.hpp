@@ -11,6 +11,17 @@ namespace vtlhip {
 // Stream every compute entry point enqueues on (nullptr = the null stream).
 hipStream_t current_stream();
 
+// True while no thread has named a stream of its own with vtl_hip_set_stream: all of the
+// library's work is on the null stream and therefore in one order.
+bool single_stream();
+
+// Whether `st` is being captured into a graph (true also when that cannot be found out).
+bool stream_is_capturing(hipStream_t st);
+
+// hipMalloc; gives the idle blocks of vtl_hip_malloc's pool back to the driver and tries again
+// when memory has run out.
+hipError_t malloc_or_trim(void **ptr, size_t bytes);
+
 // Records a failed HIP runtime call for vtl_hip_last_error() and maps it to a
 // status code of the C ABI.
 int record_hip_error(hipError_t e, const char *what);

@@ -16,7 +16,12 @@ namespace vtlhip {
 static thread_local hipStream_t g_stream = nullptr;
 static thread_local char g_last_error[256] = "";
 
+// Whether every call so far used the null stream (memory.hip).
+static std::atomic<bool> g_single_stream{true};
+
 hipStream_t current_stream() { return g_stream; }
+
+bool single_stream() { return g_single_stream.load(std::memory_order_acquire); }
 
 int record_hip_error(hipError_t e, const char *what)
 {
@@ -234,7 +239,7 @@ void *library_workspace(size_t bytes, int slot)
         cap[dev] = 0;
         in_graph[dev] = false;
         const size_t want = bytes < (size_t(32) << 20) ? (size_t(32) << 20) : bytes;
-        if (hipMalloc(&buf[dev], want) != hipSuccess) {
+        if (malloc_or_trim(&buf[dev], want) != hipSuccess) {
             (void)hipGetLastError();
             buf[dev] = nullptr;
             g_workspace_status = VTL_HIP_ERR_OUT_OF_MEMORY;
@@ -310,23 +315,6 @@ int vtl_hip_device_info(char *name, size_t name_cap, int *compute_units, int *cl
     return VTL_HIP_OK;
 }
 
-int vtl_hip_malloc(void **dptr, size_t bytes)
-{
-    if (!dptr || bytes == 0)
-        return VTL_HIP_ERR_INVALID_ARG;
-    *dptr = nullptr;
-    VTL_HIP_TRY(hipMalloc(dptr, bytes));
-    return VTL_HIP_OK;
-}
-
-int vtl_hip_free(void *dptr)
-{
-    if (!dptr)
-        return VTL_HIP_OK;  // CudaStorage.release() skips nil too
-    VTL_HIP_TRY(hipFree(dptr));
-    return VTL_HIP_OK;
-}
-
 int vtl_hip_memcpy_h2d(void *dst_device, const void *src_host, size_t bytes)
 {
     if (bytes == 0)
@@ -389,7 +377,17 @@ int vtl_hip_sync(void)
 
 int vtl_hip_set_stream(void *hip_stream)
 {
-    g_stream = (hipStream_t)hip_stream;
+    hipStream_t st = (hipStream_t)hip_stream;
+    if (st && single_stream()) {
+        // From here on memory may be used on streams that do not wait for the null stream: what was
+        // handed out again without a wait has to be out of use by then.
+        g_single_stream.store(false, std::memory_order_release);
+        if (!stream_is_capturing(st)) {
+            (void)hipDeviceSynchronize();
+            (void)hipGetLastError();
+        }
+    }
+    g_stream = st;
     return VTL_HIP_OK;
 }
 

@@ -162,7 +162,6 @@ def linear_forward_hip_i8_device(x: HipTensor, qw: QuantizedWeights, relu: bool 
     try:
         return linear_i8_hip(x_q, sx, qw.w_q, qw.sw, qw.bias, relu=relu)
     finally:
-        capi.call("vtl_hip_sync")
         x_q.release()
         sx.release()
 

@@ -23,6 +23,7 @@ class HipParams:
 
 
 _SUPPORTED = (np.float32, np.int8, np.int32, np.float64, np.uint8)
+_DEFAULT = HipParams()
 
 
 class HipStorage:
@@ -38,7 +39,7 @@ class HipStorage:
     # -- construction ------------------------------------------------------
     @staticmethod
     def empty(count: int, dtype, params: HipParams | None = None) -> "HipStorage":
-        params = params or HipParams()
+        params = params or _DEFAULT
         dt = np.dtype(dtype)
         if dt.type not in _SUPPORTED:
             raise TypeError(f"HipStorage: unsupported element type {dt}")

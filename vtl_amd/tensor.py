@@ -7,6 +7,8 @@ for `vtl.Tensor[T]` on the host side.
 """
 from __future__ import annotations
 
+import math
+
 import numpy as np
 
 from . import capi
@@ -28,7 +30,7 @@ class HipTensor:
         self.data = data
         self.memory = "row_major"
         self.shape = [int(s) for s in shape]
-        self.size = int(np.prod(self.shape)) if self.shape else 1
+        self.size = math.prod(self.shape)
         self.strides = _strides_from_shape(self.shape)
         if self.size != data.count:
             raise ValueError(f"HipTensor: shape {self.shape} does not match {data.count} elements")
@@ -42,8 +44,7 @@ class HipTensor:
 
     @staticmethod
     def empty(shape, dtype, params: HipParams | None = None) -> "HipTensor":
-        count = int(np.prod(shape)) if len(shape) else 1
-        return HipTensor(HipStorage.empty(count, dtype, params), shape)
+        return HipTensor(HipStorage.empty(math.prod(shape), dtype, params), shape)
 
     def hip(self, params: HipParams | None = None) -> "HipTensor":
         return self
@@ -261,11 +262,9 @@ def linear_f32_dynquant_hip(x: HipTensor, w_q: HipTensor, sw: HipTensor, bias: H
     try:
         capi.call("vtl_hip_linear_f32_dynquant", x.ptr, w_q.ptr, sw.ptr,
                   bias.ptr if bias is not None else None, y.ptr, M, N, K, int(relu), ws.ptr, ws.size)
-        if own:
-            capi.call("vtl_hip_sync")
     finally:
         if own:
-            ws.release()
+            ws.release()   # what is released stays as it is for work enqueued before
     return y
 
 
