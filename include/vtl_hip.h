@@ -83,6 +83,18 @@ int vtl_hip_trim(void);
 /* C.cudaMemcpy H2D storage/cuda_d_cuda.v:46, D2H :74,:90 (blocking). */
 int vtl_hip_memcpy_h2d(void *dst_device, const void *src_host, size_t bytes);
 int vtl_hip_memcpy_d2h(void *dst_host, const void *src_device, size_t bytes);
+/* vtl_hip_memcpy_h2d for uploads that compute calls follow: returns as soon as src_host may be
+ * reused, with the bytes on their way behind the current stream's earlier work, so that
+ * whatever is enqueued there next finds them.  (It waits for their arrival too once the process has
+ * used a stream of its own, vtl_hip_set_stream.) */
+int vtl_hip_upload(void *dst_device, const void *src_host, size_t bytes);
+/* `count` copies of vtl_hip_memcpy_d2h with one wait for all of them. */
+int vtl_hip_download(int count, void *const *dst_host, const void *const *src_device, const size_t *bytes);
+/* Host memory that downloads reach without a copy by the host.  At most 1 GiB at a time
+ * (VTL_HIP_ERR_OUT_OF_MEMORY beyond: use ordinary memory); up to 256 MiB of what has been freed are
+ * kept for the next call, until vtl_hip_trim. */
+int vtl_hip_host_alloc(void **hptr, size_t bytes);
+int vtl_hip_host_free(void *hptr);
 int vtl_hip_memcpy_d2d(void *dst_device, const void *src_device, size_t bytes);
 /* Byte fill on the current stream, any alignment and size; done by a kernel,
  * so a caller's stream capture records a kernel node, not a memset node. */

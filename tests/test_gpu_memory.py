@@ -68,6 +68,26 @@ for i in range(8):
 capi.call("vtl_hip_trim")
 y = HipTensor.from_host(x)
 assert np.array_equal(y.cpu(), x)
+# uploads that nothing waits for, from memory that is overwritten at once, small and large in turn
+import threading
+bad = []
+def rounds(seed):
+    r = np.random.default_rng(seed)
+    for i in range(12):
+        src = r.integers(0, 255, [100, 70000, (1 << 20) + 5, 3 << 20][i % 4], dtype=np.uint8)
+        keep = src.copy()
+        t = HipTensor.from_host(src)
+        src[:] = 0
+        if not np.array_equal(t.cpu(), keep):
+            bad.append((seed, i))
+        t.release()
+rounds(0)
+threads = [threading.Thread(target=rounds, args=(k,)) for k in range(1, 5)]
+for t in threads:
+    t.start()
+for t in threads:
+    t.join()
+assert not bad, bad
 print("done")
 """
 
@@ -76,6 +96,61 @@ def test_memory_comes_round_again_on_the_null_stream(hip):
     res = subprocess.run([sys.executable, "-c", _NULL_STREAM_ONLY, ROOT], stdout=subprocess.PIPE,
                          stderr=subprocess.PIPE, text=True, timeout=110)
     assert res.returncode == 0 and res.stdout.strip().endswith("done"), res.stderr[-2000:]
+
+
+# bytes: single ones, around a vector, where staging ends and chunks begin (1 MiB), where a chunk is
+# a whole slot (16 MiB and more), once round the ring of 8 slots of 4 MiB and a remainder
+@pytest.mark.parametrize("nbytes", [1, 15, 16, 17, 4096, 131072, 131073, (1 << 20) - 1, 1 << 20, (1 << 20) + 1,
+                                    (4 << 20) + 3, (16 << 20) + 4097, (36 << 20) + 13])
+@pytest.mark.parametrize("offset", [0, 5])
+def test_copies_to_and_from_the_device(hip, nbytes, offset):
+    rng = np.random.default_rng(nbytes + offset)
+    src = rng.integers(0, 256, nbytes, dtype=np.uint8)
+    base = _malloc(nbytes + offset + 64)
+    p = C.c_void_p()
+    capi.call("vtl_hip_host_alloc", C.byref(p), nbytes + 64)
+    pinned = np.frombuffer((C.c_uint8 * (nbytes + 64)).from_address(p.value), np.uint8)
+    for up in ("vtl_hip_memcpy_h2d", "vtl_hip_upload"):
+        capi.call("vtl_hip_memset", base, 0x5a, nbytes + offset + 64)
+        given = src.copy()
+        capi.call(up, base + offset, given.ctypes.data, nbytes)
+        given[:] = 0
+        back = d2h(base, nbytes + offset + 64, np.uint8)                    # memory of numpy's
+        assert np.array_equal(back[offset:offset + nbytes], src)
+        assert np.all(back[:offset] == 0x5a) and np.all(back[offset + nbytes:] == 0x5a)
+        for skew in (offset, 0):                                            # pinned, in step and out of step
+            pinned[:] = 0x33
+            capi.call("vtl_hip_memcpy_d2h", p.value + skew, base + offset, nbytes)
+            assert np.array_equal(pinned[skew:skew + nbytes], src)
+            assert np.all(pinned[:skew] == 0x33) and np.all(pinned[skew + nbytes:] == 0x33)
+    capi.call("vtl_hip_host_free", p)
+    assert capi.status("vtl_hip_host_free", p) == capi.ERR_INVALID_ARG
+    capi.call("vtl_hip_free", base)
+
+
+def test_several_downloads_at_once(hip):
+    """More results than one launch carries, empty ones, small and large ones among them."""
+    rng = np.random.default_rng(9)
+    arrays = [rng.standard_normal(n).astype(np.float32) for n in (3, 0, 300000, 1, 50000, 200000, 250000, 7, 600000)]
+    ts = [HipTensor.from_host(a) for a in arrays]
+    for got, a in zip(HipTensor.cpu_all(ts), arrays):
+        assert np.array_equal(got, a)
+    for t in ts:
+        t.release()
+
+
+def test_results_beyond_the_pinned_memory_are_ordinary_arrays(hip):
+    """Kept results use up the pinned memory; the ones after that still arrive."""
+    x = np.arange(40 << 20, dtype=np.float32)       # 160 MiB
+    t = HipTensor.from_host(x)
+    kept = [t.cpu() for _ in range(8)]
+    assert all(np.array_equal(k, x) for k in kept)
+    p = C.c_void_p()
+    assert capi.status("vtl_hip_host_alloc", C.byref(p), 512 << 20) == capi.ERR_OUT_OF_MEMORY
+    del kept
+    capi.call("vtl_hip_host_alloc", C.byref(p), 512 << 20)
+    capi.call("vtl_hip_host_free", p)
+    t.release()
 
 
 def test_release_waits_for_streams_of_the_caller(hip):

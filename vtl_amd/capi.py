@@ -32,6 +32,10 @@ SIGNATURES = {
     "vtl_hip_trim": (_ci, []),
     "vtl_hip_memcpy_h2d": (_ci, [_vp, _vp, _sz]),
     "vtl_hip_memcpy_d2h": (_ci, [_vp, _vp, _sz]),
+    "vtl_hip_upload": (_ci, [_vp, _vp, _sz]),
+    "vtl_hip_download": (_ci, [_ci, _pp, _pp, C.POINTER(_sz)]),
+    "vtl_hip_host_alloc": (_ci, [_pp, _sz]),
+    "vtl_hip_host_free": (_ci, [_vp]),
     "vtl_hip_memcpy_d2d": (_ci, [_vp, _vp, _sz]),
     "vtl_hip_memset": (_ci, [_vp, _ci, _sz]),
     "vtl_hip_sync": (_ci, []),

@@ -22,6 +22,11 @@ bool stream_is_capturing(hipStream_t st);
 // when memory has run out.
 hipError_t malloc_or_trim(void **ptr, size_t bytes);
 
+// The size that a pooled block of `bytes` gets (memory.hip), and giving back the idle pinned
+// blocks of vtl_hip_host_alloc (host_copy.hip).
+size_t size_class(size_t bytes);
+void trim_pinned_pool();
+
 // Records a failed HIP runtime call for vtl_hip_last_error() and maps it to a
 // status code of the C ABI.
 int record_hip_error(hipError_t e, const char *what);

@@ -1,0 +1,757 @@
+// Pinned host memory and the copies between host and device.
+//
+// What bounds them: below a few hundred KiB the latency of the copy engines and of
+// hipStreamSynchronize, above it the link (57 GB/s each way from pinned memory; the runtime's copies
+// of pageable memory reach 31 to 35 GB/s up and 17 down) and, for results, the page faults of
+// fresh host memory (4.7 GB/s).
+#include <sched.h>
+#include <string.h>
+#include <time.h>
+
+#include <atomic>
+#include <condition_variable>
+#include <deque>
+#include <map>
+#include <memory>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "common.hpp"
+
+namespace vtlhip {
+
+namespace {
+
+// ---- pinned host memory ----------------------------------------------------------
+// Blocks that host tensors are made of (results of downloads): the device writes them directly,
+// and a block that comes round again has its pages in place, where fresh memory costs a page
+// fault of 0.9 us every 4 KiB (4.7 GB/s).
+constexpr size_t kPinnedLiveMost = (size_t)1 << 30;     // beyond, callers use ordinary memory
+constexpr size_t kPinnedIdleMost = (size_t)256 << 20;
+
+struct PinnedPool {
+    std::mutex lock;
+    std::map<uintptr_t, size_t> live;                   // start -> size class
+    std::map<size_t, std::vector<void *>> free_list;
+    size_t live_bytes = 0, idle_bytes = 0;
+};
+
+PinnedPool &pinned_pool()
+{
+    static PinnedPool *p = new PinnedPool;
+    return *p;
+}
+
+bool in_pinned_pool(const void *ptr, size_t bytes)
+{
+    PinnedPool &p = pinned_pool();
+    const uintptr_t a = reinterpret_cast<uintptr_t>(ptr);
+    std::lock_guard<std::mutex> hold(p.lock);
+    auto it = p.live.upper_bound(a);
+    if (it == p.live.begin())
+        return false;
+    --it;
+    return a + bytes <= it->first + it->second;
+}
+
+// ---- copy kernel -------------------------------------------------------------------
+// Copies up to kMaxSegments runs of bytes between device memory and pinned host memory, and, when
+// a flag is given, raises it in pinned memory once every byte is there.  Used instead of the copy
+// engines because a kernel needs no hand-over between queues: host -> device copy, kernel and
+// flag take 11.6 us for 64 KiB and 14.2 us for 196 KiB where the same chain through
+// hipMemcpyAsync takes 23.0 and 25.6 us, and from 4 MiB on both run at the link's 50 to 57 GB/s.
+// 16 to 64 workgroups keep the link full; more only lengthen the tail of fences.
+constexpr int kMaxSegments = 4;
+
+struct Segment {
+    char *dst;
+    const char *src;     // same position within 16 bytes as dst
+    size_t nvec;         // 16-byte vectors
+    unsigned head, tail; // single bytes before and after them
+};
+
+struct CopyArgs {
+    Segment seg[kMaxSegments];
+    int count;
+    unsigned *counter;   // workgroups that have finished, in device memory
+    unsigned target;     // what it reads when all of this launch have
+    unsigned *flag;      // nullptr: no signal
+    unsigned value;
+};
+
+__global__ __launch_bounds__(512) void host_copy_kernel(const CopyArgs g)
+{
+    const size_t first = (size_t)blockIdx.x * 512 + threadIdx.x, step = (size_t)gridDim.x * 512;
+    for (int s = 0; s < g.count; s++) {
+        const Segment &seg = g.seg[s];
+        const uint4 *src = reinterpret_cast<const uint4 *>(seg.src + seg.head);
+        uint4 *dst = reinterpret_cast<uint4 *>(seg.dst + seg.head);
+        size_t i = first;
+        for (; i + 3 * step < seg.nvec; i += 4 * step) {   // four reads of the link in flight per lane
+            const uint4 a = src[i], b = src[i + step], c = src[i + 2 * step], d = src[i + 3 * step];
+            dst[i] = a;
+            dst[i + step] = b;
+            dst[i + 2 * step] = c;
+            dst[i + 3 * step] = d;
+        }
+        for (; i < seg.nvec; i += step)
+            dst[i] = src[i];
+        if (blockIdx.x == 0) {
+            if (threadIdx.x < seg.head)
+                seg.dst[threadIdx.x] = seg.src[threadIdx.x];
+            const size_t end = seg.head + seg.nvec * 16;
+            if (threadIdx.x < seg.tail)
+                seg.dst[end + threadIdx.x] = seg.src[end + threadIdx.x];
+        }
+    }
+    if (!g.flag)
+        return;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        // one system-scope fence per workgroup covers the stores of all of its threads (they
+        // happen before it through the barrier); whoever counts last raises the flag
+        __threadfence_system();
+        const unsigned before = __hip_atomic_fetch_add(g.counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        if (before + 1 == g.target)
+            __hip_atomic_store(g.flag, g.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+Segment make_segment(void *dst, const void *src, size_t bytes)
+{
+    Segment s;
+    s.dst = static_cast<char *>(dst);
+    s.src = static_cast<const char *>(src);
+    size_t head = (16 - (reinterpret_cast<uintptr_t>(dst) & 15)) & 15;
+    if (head > bytes)
+        head = bytes;
+    s.head = (unsigned)head;
+    s.nvec = (bytes - head) >> 4;
+    s.tail = (unsigned)((bytes - head) & 15);
+    return s;
+}
+
+unsigned copy_blocks(size_t bytes)
+{
+    const size_t per = (size_t)512 * 16;
+    const size_t want = (bytes + per - 1) / per;
+    const size_t most = bytes >= ((size_t)1 << 20) ? 32 : 16;
+    return (unsigned)(want < 1 ? 1 : want > most ? most : want);
+}
+
+// ---- lanes: what a download waits with -----------------------------------------------
+// A flag and a staging buffer in pinned memory and a counter in device memory, leased for the
+// length of one call, so that calls on several threads and streams do not meet.
+constexpr size_t kLaneStage = (size_t)1 << 20;
+
+struct Lane {
+    int device = -1;
+    unsigned *flag = nullptr;
+    unsigned *counter = nullptr;
+    unsigned arrived = 0, value = 0;
+    char *stage = nullptr;
+};
+
+struct Lanes {
+    std::mutex lock;
+    std::vector<Lane *> spare;
+};
+
+Lanes &lanes()
+{
+    static Lanes *l = new Lanes;
+    return *l;
+}
+
+__global__ void lane_counter_clear_kernel(unsigned *p) { *p = 0; }
+
+int lease_lane(Lane *&out)
+{
+    int dev = 0;
+    VTL_HIP_TRY(hipGetDevice(&dev));
+    {
+        Lanes &l = lanes();
+        std::lock_guard<std::mutex> hold(l.lock);
+        for (size_t i = l.spare.size(); i-- > 0;)
+            if (l.spare[i]->device == dev) {
+                out = l.spare[i];
+                l.spare.erase(l.spare.begin() + (long)i);
+                return VTL_HIP_OK;
+            }
+    }
+    Lane *lane = new Lane;
+    lane->device = dev;
+    void *pinned = nullptr, *counter = nullptr;
+    hipError_t e = hipHostMalloc(&pinned, kLaneStage + 4096, hipHostMallocDefault);
+    if (e == hipSuccess)
+        e = malloc_or_trim(&counter, 256);
+    if (e != hipSuccess) {
+        if (pinned)
+            (void)hipHostFree(pinned);
+        delete lane;
+        return record_hip_error(e, "memory of a host copy");
+    }
+    lane->flag = static_cast<unsigned *>(pinned);
+    *lane->flag = 0;
+    lane->stage = static_cast<char *>(pinned) + 4096;
+    lane->counter = static_cast<unsigned *>(counter);
+    hipLaunchKernelGGL(lane_counter_clear_kernel, dim3(1), dim3(1), 0, current_stream(), lane->counter);
+    const int st = check_launch("lane_counter_clear_kernel");
+    if (st != VTL_HIP_OK) {
+        (void)hipHostFree(pinned);
+        (void)hipFree(counter);
+        delete lane;
+        return st;
+    }
+    // the next lease may come with another stream
+    if (!single_stream())
+        (void)hipStreamSynchronize(current_stream());
+    out = lane;
+    return VTL_HIP_OK;
+}
+
+void return_lane(Lane *lane)
+{
+    Lanes &l = lanes();
+    std::lock_guard<std::mutex> hold(l.lock);
+    l.spare.push_back(lane);
+}
+
+double seconds()
+{
+    timespec t;
+    clock_gettime(CLOCK_MONOTONIC, &t);
+    return (double)t.tv_sec + 1e-9 * (double)t.tv_nsec;
+}
+
+// Waits for the flag of a launch: polled for two milliseconds, then left to the runtime, which
+// also reports what went wrong if the launch never ends well.
+int wait_flag(const unsigned *flag, unsigned value, hipStream_t st)
+{
+    const double began = seconds();
+    for (;;) {
+        for (int i = 0; i < 64; i++) {
+            if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == value)
+                return VTL_HIP_OK;
+            __builtin_ia32_pause();
+        }
+        if (seconds() - began > 2e-3)
+            break;
+    }
+    VTL_HIP_TRY(hipStreamSynchronize(st));
+    if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == value)
+        return VTL_HIP_OK;
+    return record_hip_error(hipErrorUnknown, "host copy ended without its flag");
+}
+
+// Enqueues the segments with a flag at the end and waits for it.
+int copy_and_wait(CopyArgs &g, size_t bytes, Lane *lane, hipStream_t st)
+{
+    const unsigned blocks = copy_blocks(bytes);
+    g.counter = lane->counter;
+    g.target = lane->arrived + blocks;
+    g.flag = lane->flag;
+    g.value = ++lane->value;
+    hipLaunchKernelGGL(host_copy_kernel, dim3(blocks), dim3(512), 0, st, g);
+    int rc = check_launch("host_copy_kernel");
+    if (rc != VTL_HIP_OK)
+        return rc;
+    lane->arrived += blocks;
+    return wait_flag(lane->flag, g.value, st);
+}
+
+// ---- staging ring ------------------------------------------------------------------------
+// Pinned slots that uploads go through (the host copies in, a kernel carries over), and downloads
+// into memory that is not the library's.  An event stands behind the last kernel that used a slot.
+constexpr int kSlots = 8;
+constexpr size_t kSlotBytes = (size_t)4 << 20;
+constexpr size_t kSlotStride = kSlotBytes + 4096;
+constexpr size_t kSmall = (size_t)1 << 20;      // up to here one host thread copies faster than others wake up
+
+struct Ring {
+    std::mutex lock;         // one transfer at a time
+    char *base = nullptr;
+    hipEvent_t event[kSlots];
+    bool pending[kSlots] = {};
+    int slot = 0;            // slot that small uploads fill
+    size_t used = 0;         // bytes of it that are taken
+
+    char *at(int i) { return base + (size_t)i * kSlotStride; }
+    int leave(int i, hipStream_t st)
+    {
+        VTL_HIP_TRY(hipEventRecord(event[i], st));
+        pending[i] = true;
+        return VTL_HIP_OK;
+    }
+    int enter(int i)
+    {
+        if (pending[i]) {
+            VTL_HIP_TRY(hipEventSynchronize(event[i]));
+            pending[i] = false;
+        }
+        return VTL_HIP_OK;
+    }
+    // enter() that gives up instead of waiting
+    int try_enter(int i, bool &entered)
+    {
+        entered = true;
+        if (pending[i]) {
+            const hipError_t e = hipEventQuery(event[i]);
+            if (e == hipErrorNotReady) {
+                (void)hipGetLastError();
+                entered = false;
+                return VTL_HIP_OK;
+            }
+            VTL_HIP_TRY(e);
+            pending[i] = false;
+        }
+        return VTL_HIP_OK;
+    }
+    // Closes the slot that small uploads were filling; the next transfer starts in a slot of its own.
+    int close(hipStream_t st)
+    {
+        if (used == 0)
+            return VTL_HIP_OK;
+        const int rc = leave(slot, st);
+        slot = (slot + 1) % kSlots;
+        used = 0;
+        return rc;
+    }
+};
+
+constexpr int kMaxDevices = 64;
+
+Ring *ring_of_current_device()
+{
+    static Ring *rings[kMaxDevices] = {};
+    static std::mutex lock;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    std::lock_guard<std::mutex> hold(lock);
+    if (!rings[dev]) {
+        std::unique_ptr<Ring> r(new Ring);
+        void *p = nullptr;
+        bool ok = hipHostMalloc(&p, kSlots * kSlotStride, hipHostMallocDefault) == hipSuccess;
+        for (int i = 0; ok && i < kSlots; i++)
+            ok = hipEventCreateWithFlags(&r->event[i], hipEventDisableTiming) == hipSuccess;
+        if (!ok) {
+            (void)hipGetLastError();
+            if (p)
+                (void)hipHostFree(p);
+            return nullptr;
+        }
+        r->base = static_cast<char *>(p);
+        rings[dev] = r.release();
+    }
+    return rings[dev];
+}
+
+// ---- host threads that share a large transfer's copying ------------------------------------
+// One thread copies 31 GB/s out of memory that is in no cache and touches 4.7 GB/s of fresh pages; the
+// link takes 57.  Three helpers and the caller reach 90 GB/s.
+struct Job {
+    char *dst = nullptr;
+    const char *src = nullptr;
+    size_t bytes = 0;
+    std::atomic<bool> done{false};
+};
+
+struct Crew {
+    std::mutex lock;
+    std::condition_variable wake;
+    std::deque<Job *> queue;
+    int threads = 0;
+
+    static Crew &instance()
+    {
+        static Crew *c = new Crew;   // never destroyed: its threads live as long as the process
+        return *c;
+    }
+    void push(Job *j)
+    {
+        {
+            std::lock_guard<std::mutex> hold(lock);
+            if (threads == 0) {
+                cpu_set_t cpus;
+                const int have = sched_getaffinity(0, sizeof cpus, &cpus) == 0 ? CPU_COUNT(&cpus) : 1;
+                threads = have > 4 ? 3 : have > 1 ? have - 1 : -1;   // -1: the caller does it all
+                for (int i = 0; i < threads; i++)
+                    std::thread([this] {
+                        for (;;)
+                            work(true);
+                    }).detach();
+            }
+            queue.push_back(j);
+        }
+        wake.notify_one();
+    }
+    // Takes one job and does it; the caller of a transfer helps while it would otherwise wait.
+    bool work(bool wait)
+    {
+        Job *j;
+        {
+            std::unique_lock<std::mutex> hold(lock);
+            if (wait)
+                wake.wait(hold, [this] { return !queue.empty(); });
+            else if (queue.empty())
+                return false;
+            j = queue.front();
+            queue.pop_front();
+        }
+        memcpy(j->dst, j->src, j->bytes);
+        j->done.store(true, std::memory_order_release);
+        return true;
+    }
+    void finish(Job &j)
+    {
+        while (!j.done.load(std::memory_order_acquire))
+            if (!work(false))
+                __builtin_ia32_pause();
+    }
+};
+
+int launch_plain_copy(void *dst, const void *src, size_t bytes, hipStream_t st)
+{
+    CopyArgs g = {};
+    g.seg[0] = make_segment(dst, src, bytes);
+    g.count = 1;
+    hipLaunchKernelGGL(host_copy_kernel, dim3(copy_blocks(bytes)), dim3(512), 0, st, g);
+    return check_launch("host_copy_kernel");
+}
+
+// A small upload: its bytes go behind those of the uploads before it in the current slot, one
+// event per slot and not one per upload.
+int upload_small(Ring *r, void *dst, const void *src, size_t bytes, hipStream_t st)
+{
+    const size_t skew = reinterpret_cast<uintptr_t>(dst) & 15;
+    const size_t take = (bytes + skew + 255) & ~(size_t)255;
+    int rc = VTL_HIP_OK;
+    if (r->used + take > kSlotBytes)
+        rc = r->close(st);
+    if (rc == VTL_HIP_OK && r->used == 0)
+        rc = r->enter(r->slot);
+    if (rc != VTL_HIP_OK)
+        return rc;
+    char *stage = r->at(r->slot) + r->used + skew;
+    memcpy(stage, src, bytes);
+    rc = launch_plain_copy(dst, stage, bytes, st);
+    if (rc == VTL_HIP_OK)
+        r->used += take;
+    return rc;
+}
+
+// Chunks of a large transfer: a quarter of it, at least 1 MiB, at most a slot.
+size_t chunk_bytes(size_t bytes)
+{
+    const size_t quarter = (bytes / 4 + 4095) & ~(size_t)4095;
+    return quarter < kSmall ? kSmall : quarter > kSlotBytes ? kSlotBytes : quarter;
+}
+
+// The host threads fill slots while the link empties the ones before them.
+int upload_large(Ring *r, char *dst, const char *src, size_t bytes, hipStream_t st)
+{
+    int rc = r->close(st);
+    if (rc != VTL_HIP_OK)
+        return rc;
+    const size_t skew = reinterpret_cast<uintptr_t>(dst) & 15, chunk = chunk_bytes(bytes);
+    const int n = (int)((bytes + chunk - 1) / chunk), s0 = r->slot;
+    std::unique_ptr<Job[]> jobs(new Job[(size_t)n]);
+    Crew &crew = Crew::instance();
+    int pushed = 0, issued = 0;
+    while (issued < n && rc == VTL_HIP_OK) {
+        while (pushed < n && pushed - issued < kSlots) {
+            const int slot = (s0 + pushed) % kSlots;
+            bool entered = true;
+            rc = pushed == issued ? r->enter(slot) : r->try_enter(slot, entered);
+            if (rc != VTL_HIP_OK || !entered)
+                break;
+            Job &j = jobs[pushed];
+            const size_t at = (size_t)pushed * chunk;
+            j.dst = r->at(slot) + skew;
+            j.src = src + at;
+            j.bytes = bytes - at < chunk ? bytes - at : chunk;
+            crew.push(&j);
+            pushed++;
+        }
+        if (rc != VTL_HIP_OK)
+            break;
+        Job &j = jobs[issued];
+        crew.finish(j);
+        const int slot = (s0 + issued) % kSlots;
+        rc = launch_plain_copy(dst + (size_t)issued * chunk, j.dst, j.bytes, st);
+        if (rc == VTL_HIP_OK)
+            rc = r->leave(slot, st);
+        issued++;
+    }
+    for (int i = issued; i < pushed; i++)   // after a failure: nothing may still write to the slots
+        crew.finish(jobs[i]);
+    r->slot = (s0 + n) % kSlots;
+    return rc;
+}
+
+// The other way round, into memory that the device cannot write itself.
+int download_large(Ring *r, char *dst, const char *src, size_t bytes, hipStream_t st)
+{
+    int rc = r->close(st);
+    if (rc != VTL_HIP_OK)
+        return rc;
+    const size_t skew = reinterpret_cast<uintptr_t>(src) & 15, chunk = chunk_bytes(bytes);
+    const int n = (int)((bytes + chunk - 1) / chunk), s0 = r->slot;
+    std::unique_ptr<Job[]> jobs(new Job[(size_t)n]);
+    Crew &crew = Crew::instance();
+    int issued = 0, pushed = 0, finished = 0;
+    while (finished < n) {
+        while (rc == VTL_HIP_OK && issued < n && issued - finished < kSlots) {
+            const int slot = (s0 + issued) % kSlots;
+            rc = r->enter(slot);
+            Job &j = jobs[issued];
+            const size_t at = (size_t)issued * chunk;
+            j.dst = dst + at;
+            j.src = r->at(slot) + skew;
+            j.bytes = bytes - at < chunk ? bytes - at : chunk;
+            if (rc == VTL_HIP_OK)
+                rc = launch_plain_copy(const_cast<char *>(j.src), src + at, j.bytes, st);
+            if (rc == VTL_HIP_OK)
+                rc = r->leave(slot, st);
+            if (rc == VTL_HIP_OK)
+                issued++;
+        }
+        if (rc == VTL_HIP_OK && pushed < issued) {
+            rc = r->enter((s0 + pushed) % kSlots);   // the chunk has arrived
+            if (rc == VTL_HIP_OK)
+                crew.push(&jobs[pushed++]);
+        }
+        if (rc != VTL_HIP_OK && finished == pushed)
+            break;
+        if (finished < pushed && (pushed == issued || jobs[finished].done.load(std::memory_order_acquire)))
+            crew.finish(jobs[finished++]);
+    }
+    r->slot = (s0 + n) % kSlots;
+    return rc;
+}
+
+}  // namespace
+
+void trim_pinned_pool()
+{
+    PinnedPool &p = pinned_pool();
+    std::vector<void *> out;
+    {
+        std::lock_guard<std::mutex> hold(p.lock);
+        for (auto &e : p.free_list)
+            out.insert(out.end(), e.second.begin(), e.second.end());
+        p.free_list.clear();
+        p.idle_bytes = 0;
+    }
+    for (void *b : out)
+        (void)hipHostFree(b);
+    (void)hipGetLastError();
+}
+
+}  // namespace vtlhip
+
+using namespace vtlhip;
+
+extern "C" {
+
+int vtl_hip_host_alloc(void **hptr, size_t bytes)
+{
+    if (!hptr || bytes == 0)
+        return VTL_HIP_ERR_INVALID_ARG;
+    *hptr = nullptr;
+    PinnedPool &p = pinned_pool();
+    const size_t cls = size_class(bytes < 4096 ? 4096 : bytes);
+    {
+        std::lock_guard<std::mutex> hold(p.lock);
+        if (p.live_bytes + cls > kPinnedLiveMost)
+            return VTL_HIP_ERR_OUT_OF_MEMORY;
+        p.live_bytes += cls;
+        auto it = p.free_list.find(cls);
+        if (it != p.free_list.end() && !it->second.empty()) {
+            *hptr = it->second.back();
+            it->second.pop_back();
+            p.idle_bytes -= cls;
+            p.live[reinterpret_cast<uintptr_t>(*hptr)] = cls;
+            return VTL_HIP_OK;
+        }
+    }
+    const hipError_t e = hipHostMalloc(hptr, cls, hipHostMallocDefault);
+    std::lock_guard<std::mutex> hold(p.lock);
+    if (e != hipSuccess) {
+        p.live_bytes -= cls;
+        *hptr = nullptr;
+        return record_hip_error(e, "hipHostMalloc");
+    }
+    p.live[reinterpret_cast<uintptr_t>(*hptr)] = cls;
+    return VTL_HIP_OK;
+}
+
+int vtl_hip_host_free(void *hptr)
+{
+    if (!hptr)
+        return VTL_HIP_OK;
+    PinnedPool &p = pinned_pool();
+    {
+        std::lock_guard<std::mutex> hold(p.lock);
+        auto it = p.live.find(reinterpret_cast<uintptr_t>(hptr));
+        if (it == p.live.end())
+            return VTL_HIP_ERR_INVALID_ARG;
+        const size_t cls = it->second;
+        p.live.erase(it);
+        p.live_bytes -= cls;
+        if (p.idle_bytes + cls <= kPinnedIdleMost) {
+            p.free_list[cls].push_back(hptr);
+            p.idle_bytes += cls;
+            return VTL_HIP_OK;
+        }
+    }
+    VTL_HIP_TRY(hipHostFree(hptr));
+    return VTL_HIP_OK;
+}
+
+int vtl_hip_upload(void *dst_device, const void *src_host, size_t bytes)
+{
+    if (bytes == 0)
+        return VTL_HIP_OK;
+    if (!dst_device || !src_host)
+        return VTL_HIP_ERR_INVALID_ARG;
+    hipStream_t st = current_stream();
+    const bool one_stream = single_stream();
+    if (one_stream || !stream_is_capturing(st)) {
+        Ring *r = ring_of_current_device();
+        if (r) {
+            std::lock_guard<std::mutex> hold(r->lock);
+            const int rc = bytes <= kSmall ? upload_small(r, dst_device, src_host, bytes, st)
+                                           : upload_large(r, static_cast<char *>(dst_device),
+                                                          static_cast<const char *>(src_host), bytes, st);
+            if (rc != VTL_HIP_OK || one_stream)
+                return rc;
+            // the ring's slots are shared by all streams
+            VTL_HIP_TRY(hipStreamSynchronize(st));
+            return VTL_HIP_OK;
+        }
+    }
+    VTL_HIP_TRY(hipMemcpyAsync(dst_device, src_host, bytes, hipMemcpyHostToDevice, st));
+    VTL_HIP_TRY(hipStreamSynchronize(st));
+    return VTL_HIP_OK;
+}
+
+int vtl_hip_memcpy_h2d(void *dst_device, const void *src_host, size_t bytes)
+{
+    if (bytes == 0)
+        return VTL_HIP_OK;
+    if (!dst_device || !src_host)
+        return VTL_HIP_ERR_INVALID_ARG;
+    hipStream_t st = current_stream();
+    const size_t skew = reinterpret_cast<uintptr_t>(dst_device) & 15;
+    if (bytes + skew > kLaneStage || stream_is_capturing(st)) {
+        const int rc = vtl_hip_upload(dst_device, src_host, bytes);
+        if (rc != VTL_HIP_OK)
+            return rc;
+        VTL_HIP_TRY(hipStreamSynchronize(st));
+        return VTL_HIP_OK;
+    }
+    Lane *lane = nullptr;
+    int rc = lease_lane(lane);
+    if (rc != VTL_HIP_OK)
+        return rc;
+    memcpy(lane->stage + skew, src_host, bytes);
+    CopyArgs g = {};
+    g.seg[0] = make_segment(dst_device, lane->stage + skew, bytes);
+    g.count = 1;
+    rc = copy_and_wait(g, bytes, lane, st);
+    if (rc == VTL_HIP_OK)
+        return_lane(lane);
+    return rc;
+}
+
+int vtl_hip_download(int count, void *const *dst_host, const void *const *src_device, const size_t *bytes)
+{
+    if (count < 0 || (count > 0 && (!dst_host || !src_device || !bytes)))
+        return VTL_HIP_ERR_INVALID_ARG;
+    bool any = false;
+    for (int i = 0; i < count; i++) {
+        if (bytes[i] && (!dst_host[i] || !src_device[i]))
+            return VTL_HIP_ERR_INVALID_ARG;
+        any = any || bytes[i];
+    }
+    if (!any)
+        return VTL_HIP_OK;
+    hipStream_t st = current_stream();
+    // What goes straight into pinned memory or fits a lane's staging buffer travels together, one
+    // wait for all of it; anything else goes through the ring, one by one.
+    CopyArgs g = {};
+    struct { void *dst; const char *stage; size_t bytes; } after[kMaxSegments];
+    int nafter = 0;
+    size_t staged = 0, total = 0;
+    Lane *lane = nullptr;
+    const bool fast = single_stream() || !stream_is_capturing(st);
+    if (fast) {
+        const int rc = lease_lane(lane);
+        if (rc != VTL_HIP_OK)
+            return rc;
+    }
+    int rc = VTL_HIP_OK;
+    auto flush = [&] {
+        if (g.count == 0)
+            return;
+        rc = copy_and_wait(g, total, lane, st);
+        for (int k = 0; rc == VTL_HIP_OK && k < nafter; k++)
+            memcpy(after[k].dst, after[k].stage, after[k].bytes);
+        g.count = nafter = 0;
+        staged = total = 0;
+    };
+    for (int i = 0; i < count && rc == VTL_HIP_OK; i++) {
+        if (bytes[i] == 0)
+            continue;
+        const size_t skew = reinterpret_cast<uintptr_t>(src_device[i]) & 15;
+        const bool direct = fast && (reinterpret_cast<uintptr_t>(dst_host[i]) & 15) == skew &&
+                            bytes[i] > 4096 && in_pinned_pool(dst_host[i], bytes[i]);
+        const size_t take = (bytes[i] + skew + 255) & ~(size_t)255;
+        if (fast && (direct || take <= kLaneStage)) {
+            if (g.count == kMaxSegments || (!direct && staged + take > kLaneStage)) {
+                flush();
+                if (rc != VTL_HIP_OK)
+                    break;
+            }
+            char *to = direct ? static_cast<char *>(dst_host[i]) : lane->stage + staged + skew;
+            g.seg[g.count++] = make_segment(to, src_device[i], bytes[i]);
+            total += bytes[i];
+            if (!direct) {
+                after[nafter++] = {dst_host[i], to, bytes[i]};
+                staged += take;
+            }
+        } else {
+            Ring *r = fast ? ring_of_current_device() : nullptr;
+            if (r) {
+                std::lock_guard<std::mutex> hold(r->lock);
+                rc = download_large(r, static_cast<char *>(dst_host[i]), static_cast<const char *>(src_device[i]),
+                                    bytes[i], st);
+            } else {
+                hipError_t e = hipMemcpyAsync(dst_host[i], src_device[i], bytes[i], hipMemcpyDeviceToHost, st);
+                if (e == hipSuccess)
+                    e = hipStreamSynchronize(st);
+                if (e != hipSuccess)
+                    rc = record_hip_error(e, "hipMemcpyAsync(device to host)");
+            }
+        }
+    }
+    if (rc == VTL_HIP_OK)
+        flush();
+    if (lane) {
+        if (rc == VTL_HIP_OK)
+            return_lane(lane);   // after a failure its counter and flag are unknown: it is left alone
+    }
+    return rc;
+}
+
+int vtl_hip_memcpy_d2h(void *dst_host, const void *src_device, size_t bytes)
+{
+    return vtl_hip_download(1, &dst_host, &src_device, &bytes);
+}
+
+}  // extern "C"

@@ -23,8 +23,6 @@ bool stream_is_capturing(hipStream_t st)
     return capturing != hipStreamCaptureStatusNone;
 }
 
-namespace {
-
 // Sizes are rounded up to eight steps per power of two, so that tensors of nearly the same size
 // share blocks and at most an eighth is wasted.
 size_t size_class(size_t bytes)
@@ -35,6 +33,8 @@ size_t size_class(size_t bytes)
     const size_t step = (size_t)1 << (top < 12 ? 9 : top - 3);
     return (bytes + step - 1) & ~(step - 1);
 }
+
+namespace {
 
 // Released blocks are kept per device and size class.  No wait is needed
 // while every call of the process has used the null stream (single_stream()): whatever still
@@ -226,6 +226,7 @@ int vtl_hip_free(void *dptr)
 int vtl_hip_trim(void)
 {
     trim_device_pool();
+    trim_pinned_pool();
     return VTL_HIP_OK;
 }
 

@@ -315,28 +315,6 @@ int vtl_hip_device_info(char *name, size_t name_cap, int *compute_units, int *cl
     return VTL_HIP_OK;
 }
 
-int vtl_hip_memcpy_h2d(void *dst_device, const void *src_host, size_t bytes)
-{
-    if (bytes == 0)
-        return VTL_HIP_OK;
-    if (!dst_device || !src_host)
-        return VTL_HIP_ERR_INVALID_ARG;
-    VTL_HIP_TRY(hipMemcpyAsync(dst_device, src_host, bytes, hipMemcpyHostToDevice, current_stream()));
-    VTL_HIP_TRY(hipStreamSynchronize(current_stream()));
-    return VTL_HIP_OK;
-}
-
-int vtl_hip_memcpy_d2h(void *dst_host, const void *src_device, size_t bytes)
-{
-    if (bytes == 0)
-        return VTL_HIP_OK;
-    if (!dst_host || !src_device)
-        return VTL_HIP_ERR_INVALID_ARG;
-    VTL_HIP_TRY(hipMemcpyAsync(dst_host, src_device, bytes, hipMemcpyDeviceToHost, current_stream()));
-    VTL_HIP_TRY(hipStreamSynchronize(current_stream()));
-    return VTL_HIP_OK;
-}
-
 int vtl_hip_memcpy_d2d(void *dst_device, const void *src_device, size_t bytes)
 {
     if (bytes == 0)

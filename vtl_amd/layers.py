@@ -357,9 +357,8 @@ def linear_backward_hip_f32(grad: np.ndarray, input: np.ndarray, weight: np.ndar
     outs = []
     try:
         outs = linear_backward_hip(g_dev, x_dev, w_dev, need_db=bias_needs_grad)
-        d_in, d_w = outs[0].cpu(), outs[1].cpu()
-        d_b = outs[2].cpu() if bias_needs_grad else np.zeros((1, w.shape[0]), g.dtype)
-        return [d_in, d_w, d_b]
+        host = HipTensor.cpu_all([t for t in outs if t is not None])
+        return host if bias_needs_grad else [*host, np.zeros((1, w.shape[0]), g.dtype)]
     finally:
         for t in (g_dev, x_dev, w_dev, *outs):
             if t is not None:
@@ -420,7 +419,7 @@ def matmul_gate_backward_hip(grad: np.ndarray, a: np.ndarray, b: np.ndarray):
     try:
         outs.append(matmul_hip(g_dev, b_dev, False, True))    # [M,N] . [K,N]^T -> [M,K]
         outs.append(matmul_hip(a_dev, g_dev, True, False))    # [M,K]^T . [M,N] -> [K,N]
-        return [t.cpu() for t in outs]
+        return HipTensor.cpu_all(outs)
     finally:
         for t in (g_dev, a_dev, b_dev, *outs):
             t.release()

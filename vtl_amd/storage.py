@@ -26,6 +26,36 @@ _SUPPORTED = (np.float32, np.int8, np.int32, np.float64, np.uint8)
 _DEFAULT = HipParams()
 
 
+# Results of more bytes than this are arrays over pinned memory of the library, which the device
+# writes itself; smaller ones are copied into ordinary memory, which the allocator recycles
+# (from 128 KiB on it would map fresh pages for each).
+_PINNED_FROM = 128 << 10
+
+
+class _HostBlock:
+    """Pinned memory under one result array; goes back to the library with the array."""
+
+    __slots__ = ("ptr", "__array_interface__")
+
+    def __init__(self, ptr: int, count: int, dt: np.dtype):
+        self.ptr = ptr
+        self.__array_interface__ = {"shape": (count,), "typestr": dt.str, "data": (ptr, False), "version": 3}
+
+    def __del__(self):
+        capi._lib.vtl_hip_host_free(self.ptr)
+
+
+def _host_array(count: int, dt: np.dtype):
+    """An uninitialised array for a download and its address."""
+    nbytes = count * dt.itemsize
+    if nbytes > _PINNED_FROM:
+        ptr = C.c_void_p(0)
+        if capi.lib().vtl_hip_host_alloc(C.byref(ptr), nbytes) == capi.OK:
+            return np.asarray(_HostBlock(ptr.value, count, dt)), ptr.value
+    out = np.empty(count, dt)
+    return out, out.ctypes.data
+
+
 class HipStorage:
     """`HipStorage[T]{ptr voidptr; size int; count int; device_id int}`."""
 
@@ -56,7 +86,7 @@ class HipStorage:
         flat = np.ascontiguousarray(arr).reshape(-1)
         st = HipStorage.empty(flat.size, flat.dtype, params)
         if st.size:
-            capi.call("vtl_hip_memcpy_h2d", st.ptr, flat.ctypes.data, st.size)
+            capi.call("vtl_hip_upload", st.ptr, flat.ctypes.data, st.size)
         return st
 
     def hip(self, params: HipParams | None = None) -> "HipStorage":
@@ -68,10 +98,19 @@ class HipStorage:
         """`.cpu() !&CpuStorage[T]` (storage/cuda_d_cuda.v:68-81)."""
         if self.count and not self.ptr:
             raise capi.VtlHipError("HipStorage.cpu", capi.ERR_INVALID_ARG, "null pointer")
-        out = np.empty(self.count, self.dtype)
+        out, host = _host_array(self.count, self.dtype)
         if self.size:
-            capi.call("vtl_hip_memcpy_d2h", out.ctypes.data, self.ptr, self.size)
+            capi.call("vtl_hip_memcpy_d2h", host, self.ptr, self.size)
         return out
+
+    @staticmethod
+    def cpu_all(storages) -> list:
+        """`.cpu()` of several storages with one wait for all of them."""
+        n = len(storages)
+        outs = [_host_array(s.count, s.dtype) for s in storages]
+        capi.call("vtl_hip_download", n, (C.c_void_p * n)(*[o[1] for o in outs]),
+                  (C.c_void_p * n)(*[s.ptr for s in storages]), (C.c_size_t * n)(*[s.size for s in storages]))
+        return [o[0] for o in outs]
 
     def to_array(self) -> np.ndarray:
         """`.to_array() ![]T` (storage/cuda_d_cuda.v:84-95)."""

@@ -52,6 +52,11 @@ class HipTensor:
     def cpu(self) -> np.ndarray:
         return self.data.cpu().reshape(self.shape)
 
+    @staticmethod
+    def cpu_all(tensors) -> list:
+        """`.cpu()` of several tensors with one wait for all of them."""
+        return [a.reshape(t.shape) for a, t in zip(HipStorage.cpu_all([t.data for t in tensors]), tensors)]
+
     def release(self) -> None:
         self.data.release()
 
