@@ -77,6 +77,8 @@ int vtl_hip_device_info(char *name, size_t name_cap, int *compute_units, int *cl
  * When the driver has no memory left, what is kept is given back and the call tried again;
  * vtl_hip_trim gives it back at once. */
 int vtl_hip_malloc(void **dptr, size_t bytes);
+/* vtl_hip_set_device and vtl_hip_malloc in one call; no bytes: nullptr. */
+int vtl_hip_malloc_on(int device_id, void **dptr, size_t bytes);
 int vtl_hip_free(void *dptr);
 int vtl_hip_trim(void);
 
@@ -298,6 +300,11 @@ const char *vtl_hip_version(void);
  * reference. */
 int vtl_hip_gemm_tile_choice(int M, int N, int K, int requant, int *config_index, int *tile_m, int *tile_n,
                              int *splits);
+
+/* Fingerprint of a HOST tensor of `count` 4- or 8-byte elements: FNV-1a over the bits of up to 64
+ * elements at even strides and the last one, and the count.  The check that the layers make
+ * before they use the codes of frozen parameters again. */
+int vtl_hip_content_fingerprint(const void *data, int64_t count, int element_bytes, uint64_t *out);
 
 /* The library reads its tuning switches (environment variables VTL_HIP_*, used
  * by tests and tuning runs only) once, at the first call that looks at them;

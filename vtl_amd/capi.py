@@ -28,6 +28,7 @@ SIGNATURES = {
     "vtl_hip_set_device": (_ci, [_ci]),
     "vtl_hip_device_info": (_ci, [C.c_char_p, _sz, C.POINTER(_ci), C.POINTER(_ci)]),
     "vtl_hip_malloc": (_ci, [_pp, _sz]),
+    "vtl_hip_malloc_on": (_ci, [_ci, _pp, _sz]),
     "vtl_hip_free": (_ci, [_vp]),
     "vtl_hip_trim": (_ci, []),
     "vtl_hip_memcpy_h2d": (_ci, [_vp, _vp, _sz]),
@@ -74,6 +75,7 @@ SIGNATURES = {
     "vtl_hip_strerror": (C.c_char_p, [_ci]),
     "vtl_hip_last_error": (C.c_char_p, []),
     "vtl_hip_version": (C.c_char_p, []),
+    "vtl_hip_content_fingerprint": (_ci, [_vp, _i64, _ci, C.POINTER(C.c_uint64)]),
     "vtl_hip_reload_env": (_ci, []),
 }
 

@@ -140,6 +140,8 @@ unsigned copy_blocks(size_t bytes)
     return (unsigned)(want < 1 ? 1 : want > most ? most : want);
 }
 
+constexpr int kMaxDevices = 64;
+
 // ---- lanes: what a download waits with -----------------------------------------------
 // A flag and a staging buffer in pinned memory and a counter in device memory, leased for the
 // length of one call, so that calls on several threads and streams do not meet.
@@ -170,6 +172,8 @@ int lease_lane(Lane *&out)
 {
     int dev = 0;
     VTL_HIP_TRY(hipGetDevice(&dev));
+    if (dev < 0 || dev >= kMaxDevices)
+        return VTL_HIP_ERR_NO_DEVICE;
     {
         Lanes &l = lanes();
         std::lock_guard<std::mutex> hold(l.lock);
@@ -245,9 +249,20 @@ int wait_flag(const unsigned *flag, unsigned value, hipStream_t st)
     return record_hip_error(hipErrorUnknown, "host copy ended without its flag");
 }
 
+// Small uploads enqueued so far and those known to have been read, per device: what a download has
+// waited for tells that every upload before it is done with its staging memory.
+struct UploadCount {
+    std::atomic<uint64_t> enqueued{0}, done{0};
+};
+
+UploadCount g_uploads[kMaxDevices];
+
 // Enqueues the segments with a flag at the end and waits for it.
 int copy_and_wait(CopyArgs &g, size_t bytes, Lane *lane, hipStream_t st)
 {
+    UploadCount &uploads = g_uploads[lane->device];
+    const bool one_stream = single_stream();
+    const uint64_t before = uploads.enqueued.load(std::memory_order_acquire);
     const unsigned blocks = copy_blocks(bytes);
     g.counter = lane->counter;
     g.target = lane->arrived + blocks;
@@ -258,7 +273,13 @@ int copy_and_wait(CopyArgs &g, size_t bytes, Lane *lane, hipStream_t st)
     if (rc != VTL_HIP_OK)
         return rc;
     lane->arrived += blocks;
-    return wait_flag(lane->flag, g.value, st);
+    rc = wait_flag(lane->flag, g.value, st);
+    if (rc == VTL_HIP_OK && one_stream) {
+        uint64_t seen = uploads.done.load(std::memory_order_relaxed);
+        while (seen < before && !uploads.done.compare_exchange_weak(seen, before))
+            ;
+    }
+    return rc;
 }
 
 // ---- staging ring ------------------------------------------------------------------------
@@ -271,6 +292,7 @@ constexpr size_t kSmall = (size_t)1 << 20;      // up to here one host thread co
 
 struct Ring {
     std::mutex lock;         // one transfer at a time
+    UploadCount *uploads = nullptr;
     char *base = nullptr;
     hipEvent_t event[kSlots];
     bool pending[kSlots] = {};
@@ -320,8 +342,6 @@ struct Ring {
     }
 };
 
-constexpr int kMaxDevices = 64;
-
 Ring *ring_of_current_device()
 {
     static Ring *rings[kMaxDevices] = {};
@@ -345,6 +365,7 @@ Ring *ring_of_current_device()
             return nullptr;
         }
         r->base = static_cast<char *>(p);
+        r->uploads = &g_uploads[dev];
         rings[dev] = r.release();
     }
     return rings[dev];
@@ -430,6 +451,11 @@ int upload_small(Ring *r, void *dst, const void *src, size_t bytes, hipStream_t 
     const size_t skew = reinterpret_cast<uintptr_t>(dst) & 15;
     const size_t take = (bytes + skew + 255) & ~(size_t)255;
     int rc = VTL_HIP_OK;
+    // When a download has waited for everything so far, the slot is filled from its start again:
+    // staging memory that is still in the host's caches.
+    if (single_stream() && r->uploads->done.load(std::memory_order_acquire) ==
+                               r->uploads->enqueued.load(std::memory_order_relaxed))
+        r->used = 0;
     if (r->used + take > kSlotBytes)
         rc = r->close(st);
     if (rc == VTL_HIP_OK && r->used == 0)
@@ -439,8 +465,10 @@ int upload_small(Ring *r, void *dst, const void *src, size_t bytes, hipStream_t 
     char *stage = r->at(r->slot) + r->used + skew;
     memcpy(stage, src, bytes);
     rc = launch_plain_copy(dst, stage, bytes, st);
-    if (rc == VTL_HIP_OK)
+    if (rc == VTL_HIP_OK) {
         r->used += take;
+        r->uploads->enqueued.fetch_add(1, std::memory_order_acq_rel);
+    }
     return rc;
 }
 

@@ -169,6 +169,15 @@ int vtl_hip_malloc(void **dptr, size_t bytes)
     return VTL_HIP_OK;
 }
 
+int vtl_hip_malloc_on(int device_id, void **dptr, size_t bytes)
+{
+    if (!dptr)
+        return VTL_HIP_ERR_INVALID_ARG;
+    *dptr = nullptr;
+    const int st = vtl_hip_set_device(device_id);
+    return st != VTL_HIP_OK || bytes == 0 ? st : vtl_hip_malloc(dptr, bytes);
+}
+
 int vtl_hip_free(void *dptr)
 {
     if (!dptr)

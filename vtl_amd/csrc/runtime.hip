@@ -433,6 +433,28 @@ int vtl_hip_reload_env(void)
     return VTL_HIP_OK;
 }
 
+int vtl_hip_content_fingerprint(const void *data, int64_t count, int element_bytes, uint64_t *out)
+{
+    if (!out || count < 0 || (count > 0 && !data) || (element_bytes != 4 && element_bytes != 8))
+        return VTL_HIP_ERR_INVALID_ARG;
+    // the elements lie pages apart: they are all requested before the serial hash takes the first
+    uint64_t v[65];
+    int n = 0;
+    const int64_t step = count >= 64 ? count / 64 : 1;
+    auto take = [&](int64_t i) {
+        v[n++] = element_bytes == 4 ? static_cast<const uint32_t *>(data)[i] : static_cast<const uint64_t *>(data)[i];
+    };
+    for (int64_t i = 0; i < count && n < 64; i += step)
+        take(i);
+    if (count > 0)
+        take(count - 1);
+    uint64_t h = 0xcbf29ce484222325ull ^ (uint64_t)count;
+    for (int i = 0; i < n; i++)
+        h = (h ^ v[i]) * 0x100000001b3ull;
+    *out = h;
+    return VTL_HIP_OK;
+}
+
 const char *vtl_hip_version(void) { return "vtlhip 0.1 (gfx950)"; }
 
 }  // extern "C"

@@ -17,6 +17,7 @@ library's.)
 """
 from __future__ import annotations
 
+import ctypes as C
 import os
 
 import numpy as np
@@ -95,14 +96,10 @@ def content_fingerprint(t: np.ndarray) -> int:
     QuantLinearLayer.quantized): an in-place edit of a frozen parameter - a checkpoint
     loaded into the same tensor, a manual `set` - changes it with near certainty when
     the edit touches most elements, as every optimizer step and every load does."""
-    flat = np.ascontiguousarray(t).reshape(-1).view(np.uint32 if t.dtype.itemsize == 4 else np.uint64)
-    n = flat.size
-    h = 0xcbf29ce484222325 ^ n
-    if n:
-        step = max(1, n // 64)
-        for v in list(flat[::step][:64]) + [flat[n - 1]]:
-            h = ((h ^ int(v)) * 0x100000001b3) & 0xffffffffffffffff
-    return h
+    flat = np.ascontiguousarray(t)
+    h = C.c_uint64()
+    capi.call("vtl_hip_content_fingerprint", flat.ctypes.data, flat.size, flat.itemsize, C.byref(h))
+    return h.value
 
 
 class QuantizedWeights:

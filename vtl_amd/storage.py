@@ -23,7 +23,6 @@ class HipParams:
 
 
 _SUPPORTED = (np.float32, np.int8, np.int32, np.float64, np.uint8)
-_DEFAULT = HipParams()
 
 
 # Results of more bytes than this are arrays over pinned memory of the library, which the device
@@ -63,22 +62,21 @@ class HipStorage:
         self.ptr = ptr
         self.size = size      # bytes
         self.count = count    # elements
-        self.dtype = np.dtype(dtype)
+        self.dtype = dtype if type(dtype) is np.dtype else np.dtype(dtype)
         self.device_id = device_id
 
     # -- construction ------------------------------------------------------
     @staticmethod
     def empty(count: int, dtype, params: HipParams | None = None) -> "HipStorage":
-        params = params or _DEFAULT
+        device_id = params.device_id if params is not None else 0
         dt = np.dtype(dtype)
         if dt.type not in _SUPPORTED:
             raise TypeError(f"HipStorage: unsupported element type {dt}")
-        capi.call("vtl_hip_set_device", params.device_id)
-        nbytes = int(count) * dt.itemsize
-        ptr = C.c_void_p(0)
-        if nbytes:
-            capi.call("vtl_hip_malloc", C.byref(ptr), nbytes)
-        return HipStorage(ptr.value or 0, nbytes, int(count), dt, params.device_id)
+        count = int(count)
+        nbytes = count * dt.itemsize
+        ptr = C.c_void_p()
+        capi.call("vtl_hip_malloc_on", device_id, C.byref(ptr), nbytes)
+        return HipStorage(ptr.value or 0, nbytes, count, dt, device_id)
 
     @staticmethod
     def from_cpu(arr: np.ndarray, params: HipParams | None = None) -> "HipStorage":

@@ -31,9 +31,19 @@ class HipTensor:
         self.memory = "row_major"
         self.shape = [int(s) for s in shape]
         self.size = math.prod(self.shape)
-        self.strides = _strides_from_shape(self.shape)
+        self._strides = None       # those of a dense row-major tensor
         if self.size != data.count:
             raise ValueError(f"HipTensor: shape {self.shape} does not match {data.count} elements")
+
+    @property
+    def strides(self):
+        if self._strides is None:
+            self._strides = _strides_from_shape(self.shape)
+        return self._strides
+
+    @strides.setter
+    def strides(self, value):
+        self._strides = value
 
     # -- construction / transfer (tensor_cuda_d_cuda.v:23-60) ----------------
     @staticmethod
