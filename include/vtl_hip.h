@@ -225,6 +225,39 @@ int vtl_hip_linear_f32_dynquant_noalloc(const float *X, const int8_t *Wq, const 
                                         const float *bias, float *Y, int M, int N, int K,
                                         int relu);
 
+/* ---- whole calls on host tensors ------------------------------------------ */
+
+/* One layer of a stack whose parameters are on the device: an int8 linear with the weights as
+ * stored (codes [out_features, in_features], `out_features` scales when per_channel, else one;
+ * bias or NULL), or a ReLU on what the layer before it gives. */
+enum { VTL_HIP_LAYER_LINEAR = 0, VTL_HIP_LAYER_RELU = 1 };
+typedef struct {
+    int kind;
+    int per_channel;
+    int out_features, in_features;
+    const int8_t *wq;
+    const float *sw;
+    const float *bias;
+} vtl_hip_layer;
+
+/* Sequential.forward / LinearLayer.forward on a host tensor x[rows, cols]: `layers[0 .. count)` in
+ * order, y[rows, out_features of the last linear] on return.  Activations are quantized like the
+ * weights of the layer they enter: per row when per_channel, else with one scale.  Bits of
+ * the calls it is made of (vtl_hip_quantize_f32_i8, vtl_hip_linear_i8_f32 and so on).  The layers'
+ * pointers are device pointers, x and y host pointers. */
+int vtl_hip_forward_i8_host(const float *x_host, int rows, int cols, const vtl_hip_layer *layers, int count,
+                            float *y_host);
+
+/* la.matmul (la/la.v:38-55) and LinearGate.backward (nn/gates/layers/linear.v:57-79) on host
+ * tensors: vtl_hip_matmul_* without transposes and vtl_hip_linear_backward_*, operands and
+ * results on the host. */
+int vtl_hip_matmul_host_f32(const float *A, const float *B, float *C, int M, int N, int K);
+int vtl_hip_matmul_host_f64(const double *A, const double *B, double *C, int M, int N, int K);
+int vtl_hip_linear_backward_host_f32(const float *grad, const float *x, const float *W, float *dx, float *dw,
+                                     float *db, int M, int N, int K);
+int vtl_hip_linear_backward_host_f64(const double *grad, const double *x, const double *W, double *dx, double *dw,
+                                     double *db, int M, int N, int K);
+
 /* ---- f32 / f64 matmul with f64 accumulation ------------------------------ */
 
 /* C[M,N] = op(A) . op(B) with every product and sum in f64 and one rounding

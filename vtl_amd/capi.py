@@ -22,6 +22,15 @@ ERR_UNSUPPORTED = 5
 _i64, _ci, _vp, _sz = C.c_int64, C.c_int, C.c_void_p, C.c_size_t
 _pp = C.POINTER(C.c_void_p)
 
+LAYER_LINEAR, LAYER_RELU = 0, 1
+
+
+class Layer(C.Structure):
+    """`vtl_hip_layer`: one layer of a stack whose parameters are on the device."""
+    _fields_ = [("kind", _ci), ("per_channel", _ci), ("out_features", _ci), ("in_features", _ci),
+                ("wq", _vp), ("sw", _vp), ("bias", _vp)]
+
+
 # name -> (restype, argtypes); kept in step with include/vtl_hip.h
 SIGNATURES = {
     "vtl_hip_device_count": (_ci, [C.POINTER(_ci)]),
@@ -58,6 +67,11 @@ SIGNATURES = {
     "vtl_hip_linear_f32_dynquant_workspace": (_sz, [_ci, _ci]),
     "vtl_hip_linear_f32_dynquant": (_ci, [_vp, _vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp, _sz]),
     "vtl_hip_linear_f32_dynquant_noalloc": (_ci, [_vp, _vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci]),
+    "vtl_hip_forward_i8_host": (_ci, [_vp, _ci, _ci, C.POINTER(Layer), _ci, _vp]),
+    "vtl_hip_matmul_host_f32": (_ci, [_vp, _vp, _vp, _ci, _ci, _ci]),
+    "vtl_hip_matmul_host_f64": (_ci, [_vp, _vp, _vp, _ci, _ci, _ci]),
+    "vtl_hip_linear_backward_host_f32": (_ci, [_vp, _vp, _vp, _vp, _vp, _vp, _ci, _ci, _ci]),
+    "vtl_hip_linear_backward_host_f64": (_ci, [_vp, _vp, _vp, _vp, _vp, _vp, _ci, _ci, _ci]),
     "vtl_hip_matmul_f32": (_ci, [_vp, _vp, _vp, _ci, _ci, _ci, _ci, _ci]),
     "vtl_hip_matmul_f64": (_ci, [_vp, _vp, _vp, _ci, _ci, _ci, _ci, _ci]),
     "vtl_hip_linear_f32": (_ci, [_vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci]),

@@ -34,6 +34,22 @@ int record_hip_error(hipError_t e, const char *what);
 // Checks the launch that was just made.
 int check_launch(const char *kernel_name);
 
+// A small host array in pinned memory, for kernels that read their input once and can take it over
+// the link themselves instead of behind a copy.  The bytes stay until the object is gone and the
+// work enqueued before that is done.  No vtl_hip_upload while one is alive on the same thread.
+struct HostInput {
+    const void *data = nullptr;
+    // False when the bytes have to be uploaded instead: too many, or streams of the caller's.
+    bool stage(const void *src, size_t bytes);
+    HostInput() = default;
+    ~HostInput();
+    HostInput(const HostInput &) = delete;
+    HostInput &operator=(const HostInput &) = delete;
+
+private:
+    void *ring_ = nullptr;
+};
+
 // Streaming copy kernel (quant.hip); false when alignment or size do not qualify.
 bool launch_copy(void *dst, const void *src, size_t bytes, hipStream_t st);
 

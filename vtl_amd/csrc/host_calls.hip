@@ -1,0 +1,245 @@
+// Whole calls on host tensors: upload, kernels and download behind one entry point.
+//
+// A program that keeps its tensors on the host pays, per call, for every step between the
+// kernels: 64 x 784 -> 256 is 10 us of kernels.  Made from the host language step by step,
+// the same call took 41 us, 18 of them outside the library.
+#include "common.hpp"
+
+namespace vtlhip {
+namespace {
+
+// Device memory for the length of a call.  Released while its kernels may still run: the pool hands
+// it out again behind them.
+struct Scratch {
+    void *ptr = nullptr;
+    ~Scratch() { release(); }
+    Scratch() = default;
+    Scratch(const Scratch &) = delete;
+    Scratch &operator=(const Scratch &) = delete;
+    int take(size_t bytes)
+    {
+        release();
+        return bytes ? vtl_hip_malloc(&ptr, bytes) : VTL_HIP_OK;
+    }
+    void release()
+    {
+        if (ptr)
+            (void)vtl_hip_free(ptr);
+        ptr = nullptr;
+    }
+    void swap(Scratch &o)
+    {
+        void *p = ptr;
+        ptr = o.ptr;
+        o.ptr = p;
+    }
+    template <typename T>
+    T *as() { return static_cast<T *>(ptr); }
+};
+
+#define VTL_STEP(expr)            \
+    do {                          \
+        const int rc_ = (expr);   \
+        if (rc_ != VTL_HIP_OK)    \
+            return rc_;           \
+    } while (0)
+
+// Up to this many rows the linear on f32 rows quantizes them inside its own launch, so the
+// activations stay f32 between layers (1 row through 4096 -> 11008 -> 4096 -> 1024: 23.4 against
+// 28.0 us); with more rows per-row codes go from layer to layer.  The bits are the same.
+constexpr int kFewRows = 32;
+
+int check_layers(const vtl_hip_layer *layers, int count, int cols, int &out_cols)
+{
+    for (int i = 0; i < count; i++) {
+        const vtl_hip_layer &l = layers[i];
+        if (l.kind == VTL_HIP_LAYER_RELU)
+            continue;
+        if (l.kind != VTL_HIP_LAYER_LINEAR || l.in_features != cols || l.out_features < 0 || !l.wq || !l.sw)
+            return VTL_HIP_ERR_INVALID_ARG;
+        cols = l.out_features;
+    }
+    out_cols = cols;
+    return VTL_HIP_OK;
+}
+
+int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer *layers, int count, float *y_host)
+{
+    int out_cols = 0;
+    VTL_STEP(check_layers(layers, count, cols, out_cols));
+    if (rows == 0 || cols == 0 || out_cols == 0)
+        return count == 0 ? VTL_HIP_OK : VTL_HIP_ERR_INVALID_ARG;
+    const size_t in_bytes = (size_t)rows * (size_t)cols * sizeof(float);
+    Scratch cur, next;                     // f32 rows
+    Scratch codes, scales, next_codes, next_scales;
+    const float *x = nullptr;              // the f32 rows, or null while the activations are codes
+    int i = 0;
+    if (count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR) {
+        // A quantizer in front reads the input once and takes it over the link itself: 64 x 784,
+        // per tensor, 4 us less than behind an upload.  (A tensor of more than 65536 elements is
+        // read twice, and the launches for a few rows read it in every workgroup.)
+        const bool once = layers[0].per_channel ? rows > kFewRows : (int64_t)rows * cols <= 65536;
+        HostInput input;
+        if (once && input.stage(x_host, in_bytes)) {
+            VTL_STEP(codes.take((size_t)rows * (size_t)cols));
+            VTL_STEP(scales.take((layers[0].per_channel ? (size_t)rows : 1) * sizeof(float)));
+            VTL_STEP(vtl_hip_quantize_f32_i8(static_cast<const float *>(input.data), rows, cols, layers[0].per_channel,
+                                             codes.as<int8_t>(), scales.as<float>()));
+        }
+    }
+    if (!codes.ptr) {
+        VTL_STEP(cur.take(in_bytes));
+        VTL_STEP(vtl_hip_upload(cur.ptr, x_host, in_bytes));
+        x = cur.as<float>();
+    }
+    while (i < count) {
+        const vtl_hip_layer &l = layers[i];
+        if (l.kind == VTL_HIP_LAYER_RELU) {
+            VTL_STEP(vtl_hip_relu_f32(cur.as<float>(), (int64_t)rows * cols));
+            i++;
+            continue;
+        }
+        const int n = l.out_features;
+        const bool relu = i + 1 < count && layers[i + 1].kind == VTL_HIP_LAYER_RELU;
+        i += relu ? 2 : 1;
+        // the next layer takes codes as well
+        const bool feeds = l.per_channel && rows > kFewRows && i < count && layers[i].kind == VTL_HIP_LAYER_LINEAR &&
+                           layers[i].per_channel;
+        if (x && l.per_channel && !feeds) {
+            VTL_STEP(next.take((size_t)rows * (size_t)n * sizeof(float)));
+            const size_t need = vtl_hip_linear_f32_dynquant_workspace(rows, cols);
+            Scratch work;
+            VTL_STEP(work.take(need));
+            VTL_STEP(vtl_hip_linear_f32_dynquant(x, l.wq, l.sw, l.bias, next.as<float>(), rows, n, cols, relu,
+                                                 work.ptr, need));
+            cur.swap(next);
+            x = cur.as<float>();
+            cols = n;
+            continue;
+        }
+        if (x) {
+            VTL_STEP(codes.take((size_t)rows * (size_t)cols));
+            VTL_STEP(scales.take((l.per_channel ? (size_t)rows : 1) * sizeof(float)));
+            VTL_STEP(vtl_hip_quantize_f32_i8(x, rows, cols, l.per_channel, codes.as<int8_t>(), scales.as<float>()));
+            x = nullptr;
+        }
+        if (feeds) {
+            VTL_STEP(next_codes.take((size_t)rows * (size_t)n));
+            VTL_STEP(next_scales.take((size_t)rows * sizeof(float)));
+            VTL_STEP(vtl_hip_linear_i8_requant(codes.as<int8_t>(), scales.as<float>(), 1, l.wq, l.sw, 1, l.bias, relu,
+                                               next_codes.as<int8_t>(), next_scales.as<float>(), nullptr, rows, n,
+                                               cols));
+            codes.swap(next_codes);
+            scales.swap(next_scales);
+        } else {
+            VTL_STEP(cur.take((size_t)rows * (size_t)n * sizeof(float)));
+            VTL_STEP(vtl_hip_linear_i8_f32(codes.as<int8_t>(), scales.as<float>(), l.per_channel, l.wq, l.sw,
+                                           l.per_channel, l.bias, cur.as<float>(), rows, n, cols, relu));
+            x = cur.as<float>();
+        }
+        cols = n;
+    }
+    return vtl_hip_memcpy_d2h(y_host, cur.ptr, (size_t)rows * (size_t)out_cols * sizeof(float));
+}
+
+template <typename T>
+struct Ops;
+template <>
+struct Ops<float> {
+    static constexpr auto matmul = vtl_hip_matmul_f32;
+    static constexpr auto backward = vtl_hip_linear_backward_f32;
+};
+template <>
+struct Ops<double> {
+    static constexpr auto matmul = vtl_hip_matmul_f64;
+    static constexpr auto backward = vtl_hip_linear_backward_f64;
+};
+
+template <typename T>
+int upload(Scratch &to, const T *host, size_t count)
+{
+    VTL_STEP(to.take(count * sizeof(T)));
+    return vtl_hip_upload(to.ptr, host, count * sizeof(T));
+}
+
+template <typename T>
+int matmul_host(const T *a, const T *b, T *c, int m, int n, int k)
+{
+    if (m < 0 || n < 0 || k < 0)
+        return VTL_HIP_ERR_INVALID_ARG;
+    if (m == 0 || n == 0)
+        return VTL_HIP_OK;
+    if (!c || (k > 0 && (!a || !b)))
+        return VTL_HIP_ERR_INVALID_ARG;
+    Scratch da, db, dc;
+    VTL_STEP(upload(da, a, (size_t)m * (size_t)k));
+    VTL_STEP(upload(db, b, (size_t)k * (size_t)n));
+    VTL_STEP(dc.take((size_t)m * (size_t)n * sizeof(T)));
+    VTL_STEP(Ops<T>::matmul(da.as<T>(), db.as<T>(), dc.as<T>(), m, n, k, 0, 0));
+    return vtl_hip_memcpy_d2h(c, dc.ptr, (size_t)m * (size_t)n * sizeof(T));
+}
+
+template <typename T>
+int linear_backward_host(const T *grad, const T *x, const T *w, T *dx, T *dw, T *db, int m, int n, int k)
+{
+    if (m < 0 || n < 0 || k < 0 || !grad || (dx && !w) || (dw && !x))
+        return VTL_HIP_ERR_INVALID_ARG;
+    const size_t mn = (size_t)m * (size_t)n, mk = (size_t)m * (size_t)k, nk = (size_t)n * (size_t)k;
+    Scratch dev_grad, dev_x, dev_w, dev_dx, dev_dw, dev_db;
+    VTL_STEP(upload(dev_grad, grad, mn));
+    if (dw)
+        VTL_STEP(upload(dev_x, x, mk));
+    if (dx)
+        VTL_STEP(upload(dev_w, w, nk));
+    if (dx)
+        VTL_STEP(dev_dx.take(mk * sizeof(T)));
+    if (dw)
+        VTL_STEP(dev_dw.take(nk * sizeof(T)));
+    if (db)
+        VTL_STEP(dev_db.take((size_t)n * sizeof(T)));
+    VTL_STEP(Ops<T>::backward(dev_grad.as<T>(), dev_x.as<T>(), dev_w.as<T>(), dev_dx.as<T>(), dev_dw.as<T>(),
+                              dev_db.as<T>(), m, n, k));
+    void *const host[3] = {dx, dw, db};
+    const void *const dev[3] = {dev_dx.ptr, dev_dw.ptr, dev_db.ptr};
+    const size_t bytes[3] = {dx ? mk * sizeof(T) : 0, dw ? nk * sizeof(T) : 0, db ? (size_t)n * sizeof(T) : 0};
+    return vtl_hip_download(3, host, dev, bytes);
+}
+
+}  // namespace
+}  // namespace vtlhip
+
+using namespace vtlhip;
+
+extern "C" {
+
+int vtl_hip_forward_i8_host(const float *x_host, int rows, int cols, const vtl_hip_layer *layers, int count,
+                            float *y_host)
+{
+    if (rows < 0 || cols < 0 || count < 0 || (count > 0 && !layers) || !x_host || !y_host)
+        return VTL_HIP_ERR_INVALID_ARG;
+    return forward_layers(x_host, rows, cols, layers, count, y_host);
+}
+
+int vtl_hip_matmul_host_f32(const float *a, const float *b, float *c, int m, int n, int k)
+{
+    return matmul_host<float>(a, b, c, m, n, k);
+}
+
+int vtl_hip_matmul_host_f64(const double *a, const double *b, double *c, int m, int n, int k)
+{
+    return matmul_host<double>(a, b, c, m, n, k);
+}
+
+int vtl_hip_linear_backward_host_f32(const float *grad, const float *x, const float *W, float *dx, float *dw,
+                                     float *db, int m, int n, int k)
+{
+    return linear_backward_host<float>(grad, x, W, dx, dw, db, m, n, k);
+}
+
+int vtl_hip_linear_backward_host_f64(const double *grad, const double *x, const double *W, double *dx, double *dw,
+                                     double *db, int m, int n, int k)
+{
+    return linear_backward_host<double>(grad, x, W, dx, dw, db, m, n, k);
+}
+
+}  // extern "C"

@@ -61,7 +61,8 @@ bool in_pinned_pool(const void *ptr, size_t bytes)
 // engines because a kernel needs no hand-over between queues: host -> device copy, kernel and
 // flag take 11.6 us for 64 KiB and 14.2 us for 196 KiB where the same chain through
 // hipMemcpyAsync takes 23.0 and 25.6 us, and from 4 MiB on both run at the link's 50 to 57 GB/s.
-// 16 to 64 workgroups keep the link full; more only lengthen the tail of fences.
+// 16 workgroups keep the link full (50.6 GB/s at 4 MiB up, with 64 of them 46.8); only downloads from
+// 1 MiB on take 32.
 constexpr int kMaxSegments = 4;
 
 struct Segment {
@@ -440,15 +441,14 @@ int launch_plain_copy(void *dst, const void *src, size_t bytes, hipStream_t st)
     CopyArgs g = {};
     g.seg[0] = make_segment(dst, src, bytes);
     g.count = 1;
-    hipLaunchKernelGGL(host_copy_kernel, dim3(copy_blocks(bytes)), dim3(512), 0, st, g);
+    hipLaunchKernelGGL(host_copy_kernel, dim3(copy_blocks(bytes < kSmall ? bytes : kSmall - 1)), dim3(512), 0, st, g);
     return check_launch("host_copy_kernel");
 }
 
-// A small upload: its bytes go behind those of the uploads before it in the current slot, one
-// event per slot and not one per upload.
-int upload_small(Ring *r, void *dst, const void *src, size_t bytes, hipStream_t st)
+// Copies a small upload's bytes into the ring, behind those of the uploads before it in the current
+// slot (one event per slot and not one per upload), `skew` bytes past a 16-byte boundary.
+int stage_small(Ring *r, const void *src, size_t bytes, size_t skew, hipStream_t st, char *&staged)
 {
-    const size_t skew = reinterpret_cast<uintptr_t>(dst) & 15;
     const size_t take = (bytes + skew + 255) & ~(size_t)255;
     int rc = VTL_HIP_OK;
     // When a download has waited for everything so far, the slot is filled from its start again:
@@ -462,13 +462,20 @@ int upload_small(Ring *r, void *dst, const void *src, size_t bytes, hipStream_t 
         rc = r->enter(r->slot);
     if (rc != VTL_HIP_OK)
         return rc;
-    char *stage = r->at(r->slot) + r->used + skew;
-    memcpy(stage, src, bytes);
-    rc = launch_plain_copy(dst, stage, bytes, st);
-    if (rc == VTL_HIP_OK) {
-        r->used += take;
+    staged = r->at(r->slot) + r->used + skew;
+    memcpy(staged, src, bytes);
+    r->used += take;
+    return VTL_HIP_OK;
+}
+
+int upload_small(Ring *r, void *dst, const void *src, size_t bytes, hipStream_t st)
+{
+    char *staged = nullptr;
+    int rc = stage_small(r, src, bytes, reinterpret_cast<uintptr_t>(dst) & 15, st, staged);
+    if (rc == VTL_HIP_OK)
+        rc = launch_plain_copy(dst, staged, bytes, st);
+    if (rc == VTL_HIP_OK)
         r->uploads->enqueued.fetch_add(1, std::memory_order_acq_rel);
-    }
     return rc;
 }
 
@@ -563,6 +570,36 @@ int download_large(Ring *r, char *dst, const char *src, size_t bytes, hipStream_
 }
 
 }  // namespace
+
+HostInput::~HostInput()
+{
+    if (!ring_)
+        return;
+    // counted only now, when the kernels that read the bytes are enqueued: a download that waits
+    // from here on waits for them too
+    Ring *r = static_cast<Ring *>(ring_);
+    r->uploads->enqueued.fetch_add(1, std::memory_order_acq_rel);
+    r->lock.unlock();
+}
+
+// The lock of the ring is held until then, so that no other transfer closes the slot before.
+bool HostInput::stage(const void *src, size_t bytes)
+{
+    if (!single_stream() || bytes > kSmall)
+        return false;
+    Ring *r = ring_of_current_device();
+    if (!r)
+        return false;
+    r->lock.lock();
+    char *staged = nullptr;
+    if (stage_small(r, src, bytes, 0, current_stream(), staged) != VTL_HIP_OK) {
+        r->lock.unlock();
+        return false;
+    }
+    ring_ = r;
+    data = staged;
+    return true;
+}
 
 void trim_pinned_pool()
 {

@@ -23,7 +23,7 @@ import os
 import numpy as np
 
 from . import capi
-from .storage import HipParams, HipStorage
+from .storage import HipParams, HipStorage, host_array
 from .tensor import (HipTensor, linear_backward_hip, linear_f32_dynquant_hip, linear_hip, linear_i8_hip,
                      matmul_hip)
 
@@ -133,6 +133,8 @@ class QuantizedWeights:
             if b.size != self.out_features:
                 raise ValueError(f"bias has {b.size} entries, expected {self.out_features}")
             self.bias = HipTensor.from_host(b, params)
+        self.layer = capi.Layer(capi.LAYER_LINEAR, mode == PER_CHANNEL, self.out_features, self.in_features,
+                                self.w_q.ptr, self.sw.ptr, self.bias.ptr if self.bias is not None else None)
 
     def release(self) -> None:
         self.w_q.release()
@@ -178,16 +180,26 @@ def _linear_host_roundtrip(x, weights, bias, mode) -> np.ndarray:
     if x.ndim != 2 or np.ndim(weights) != 2:
         raise ValueError("Matrix expected")
     qw = QuantizedWeights(weights, bias, mode)
-    x_dev = HipTensor.from_host(x)
     try:
-        y = linear_forward_hip_i8_device(x_dev, qw)
-        try:
-            return y.cpu()
-        finally:
-            y.release()
+        return forward_host(x, [qw.layer], 1, qw.out_features)
     finally:
-        x_dev.release()
         qw.release()
+
+
+def forward_host(x: np.ndarray, layers, count: int, out_features: int) -> np.ndarray:
+    """x[M, K] through `count` layers (`capi.Layer`) whose parameters are on the current device, host
+    to host in one call."""
+    x = np.ascontiguousarray(x)
+    rows, cols = x.shape
+    first = next((l for l in layers if l.kind == capi.LAYER_LINEAR), None)
+    if first is not None and cols != first.in_features:
+        raise ValueError(
+            f"Invalid shapes for matrix multiplication {[rows, cols]} and {[first.in_features, first.out_features]}")
+    y, host = host_array(rows * out_features, x.dtype)
+    if type(layers) is list:
+        layers = (capi.Layer * count)(*layers)
+    capi.call("vtl_hip_forward_i8_host", x.ctypes.data, rows, cols, layers, count, host)
+    return y.reshape(rows, out_features)
 
 
 class QuantLinearLayer:
@@ -261,15 +273,9 @@ class QuantLinearLayer:
         x = np.asarray(x, np.float32)
         if x.ndim != 2:
             raise ValueError("Matrix expected")
-        x_dev = HipTensor.from_host(x, self.params)
-        try:
-            y = self.forward_device(x_dev, no_grad=no_grad)
-            try:
-                return y.cpu()
-            finally:
-                y.release()
-        finally:
-            x_dev.release()
+        capi.call("vtl_hip_set_device", self.params.device_id)
+        qw = self.quantized(no_grad)
+        return forward_host(x, [qw.layer], 1, qw.out_features)
 
     def release(self) -> None:
         if self._cache is not None:
@@ -304,17 +310,15 @@ def matmul_hip_host(a: np.ndarray, b: np.ndarray) -> np.ndarray:
     b = _as_float_matrix(b, "matmul")
     if a.shape[1] != b.shape[0]:
         raise ValueError(f"Invalid shapes for matrix multiplication {list(a.shape)} and {list(b.shape)}")
-    a_dev = HipTensor.from_host(a)
-    b_dev = HipTensor.from_host(b.astype(a.dtype, copy=False))
-    try:
-        c_dev = matmul_hip(a_dev, b_dev)
-        try:
-            return c_dev.cpu()
-        finally:
-            c_dev.release()
-    finally:
-        a_dev.release()
-        b_dev.release()
+    a = np.ascontiguousarray(a)
+    b = np.ascontiguousarray(b, a.dtype)
+    m, k = a.shape
+    n = b.shape[1]
+    capi.call("vtl_hip_set_device", 0)
+    c, host = host_array(m * n, a.dtype)
+    capi.call("vtl_hip_matmul_host_f32" if a.itemsize == 4 else "vtl_hip_matmul_host_f64", a.ctypes.data, b.ctypes.data,
+              host, m, n, k)
+    return c.reshape(m, n)
 
 
 def linear_forward_hip_exact(x: np.ndarray, weights: np.ndarray, bias: np.ndarray | None) -> np.ndarray:
@@ -350,16 +354,17 @@ def linear_backward_hip_f32(grad: np.ndarray, input: np.ndarray, weight: np.ndar
     g = _as_float_matrix(grad, "linear backward")
     x = _as_float_matrix(input, "linear backward").astype(g.dtype, copy=False)
     w = _as_float_matrix(weight, "linear backward").astype(g.dtype, copy=False)
-    g_dev, x_dev, w_dev = HipTensor.from_host(g), HipTensor.from_host(x), HipTensor.from_host(w)
-    outs = []
-    try:
-        outs = linear_backward_hip(g_dev, x_dev, w_dev, need_db=bias_needs_grad)
-        host = HipTensor.cpu_all([t for t in outs if t is not None])
-        return host if bias_needs_grad else [*host, np.zeros((1, w.shape[0]), g.dtype)]
-    finally:
-        for t in (g_dev, x_dev, w_dev, *outs):
-            if t is not None:
-                t.release()
+    m, n = g.shape
+    k = x.shape[1]
+    if x.shape != (m, k) or w.shape != (n, k):
+        raise ValueError(f"linear_backward_hip: grad {list(g.shape)}, input {list(x.shape)}, weight {list(w.shape)}")
+    g, x, w = np.ascontiguousarray(g), np.ascontiguousarray(x), np.ascontiguousarray(w)
+    capi.call("vtl_hip_set_device", 0)
+    (dx, dx_ptr), (dw, dw_ptr) = host_array(m * k, g.dtype), host_array(n * k, g.dtype)
+    db, db_ptr = host_array(n, g.dtype) if bias_needs_grad else (np.zeros(n, g.dtype), None)
+    capi.call("vtl_hip_linear_backward_host_f32" if g.itemsize == 4 else "vtl_hip_linear_backward_host_f64",
+              g.ctypes.data, x.ctypes.data, w.ctypes.data, dx_ptr, dw_ptr, db_ptr, m, n, k)
+    return [dx.reshape(m, k), dw.reshape(n, k), db.reshape(1, n)]
 
 
 # -- activation hooks (cf. relu_forward_f32 / sigmoid_forward_f32,

@@ -44,7 +44,7 @@ class _HostBlock:
         capi._lib.vtl_hip_host_free(self.ptr)
 
 
-def _host_array(count: int, dt: np.dtype):
+def host_array(count: int, dt: np.dtype):
     """An uninitialised array for a download and its address."""
     nbytes = count * dt.itemsize
     if nbytes > _PINNED_FROM:
@@ -96,7 +96,7 @@ class HipStorage:
         """`.cpu() !&CpuStorage[T]` (storage/cuda_d_cuda.v:68-81)."""
         if self.count and not self.ptr:
             raise capi.VtlHipError("HipStorage.cpu", capi.ERR_INVALID_ARG, "null pointer")
-        out, host = _host_array(self.count, self.dtype)
+        out, host = host_array(self.count, self.dtype)
         if self.size:
             capi.call("vtl_hip_memcpy_d2h", host, self.ptr, self.size)
         return out
@@ -105,7 +105,7 @@ class HipStorage:
     def cpu_all(storages) -> list:
         """`.cpu()` of several storages with one wait for all of them."""
         n = len(storages)
-        outs = [_host_array(s.count, s.dtype) for s in storages]
+        outs = [host_array(s.count, s.dtype) for s in storages]
         capi.call("vtl_hip_download", n, (C.c_void_p * n)(*[o[1] for o in outs]),
                   (C.c_void_p * n)(*[s.ptr for s in storages]), (C.c_size_t * n)(*[s.size for s in storages]))
         return [o[0] for o in outs]
