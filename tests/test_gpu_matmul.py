@@ -123,6 +123,33 @@ def test_forced_tile_sizes(hip, tile, knobs):
         assert np.array_equal(run_matmul(Ai, Bi, ta, tb), exact.astype(np.float32))
 
 
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("shape", ["1", "2", "3", "4", "5"])
+def test_direct_shapes_at_their_edges(hip, shape, dt, knobs):
+    """Every shape of the kernel that loads operands straight from memory, all four layouts: single
+    rows and columns, pairs that end inside and at the edge of a tile, one element of K, part of
+    a step, whole steps for some of the waves only, one step more than the loads in flight, K in
+    slices with a part of a step left.  Integers bit for bit."""
+    knobs.setenv("VTL_HIP_MATMUL_TILE", shape)
+    rng = np.random.default_rng(100 + int(shape))
+    for (M, N, K, splits) in [(1, 1, 1, None), (1, 33, 15, None), (31, 1, 16, None), (2, 3, 17, None),
+                              (32, 64, 64, None), (33, 65, 79, None), (63, 127, 257, None), (65, 129, 145, None),
+                              (64, 128, 530, None), (5, 70, 1003, "3"), (130, 31, 1024, "5")]:
+        if splits is None:
+            knobs.delenv("VTL_HIP_MATMUL_SPLITS", raising=False)
+        else:
+            knobs.setenv("VTL_HIP_MATMUL_SPLITS", splits)
+        for ta, tb in [(False, False), (False, True), (True, False), (True, True)]:
+            A = rng.standard_normal((K, M) if ta else (M, K)).astype(dt)
+            B = rng.standard_normal((N, K) if tb else (K, N)).astype(dt)
+            print("direct", shape, dt.__name__, M, N, K, splits, ta, tb, flush=True)
+            absprod = np.abs(A.T if ta else A).astype(np.float64) @ np.abs(B.T if tb else B).astype(np.float64)
+            assert_close_to_oracle(run_matmul(A, B, ta, tb), oracle.matmul(A, B, ta, tb, threads=CPU_THREADS), absprod)
+            Ai, Bi = np.rint(A * 4).astype(dt), np.rint(B * 4).astype(dt)
+            exact = (Ai.T if ta else Ai).astype(np.float64) @ (Bi.T if tb else Bi).astype(np.float64)
+            assert np.array_equal(run_matmul(Ai, Bi, ta, tb), exact.astype(dt))
+
+
 def test_reference_literals(hip):
     # la/la_test.v:30-37
     a = np.array([[1.0, 0], [0.0, 1]])

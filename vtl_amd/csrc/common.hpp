@@ -110,7 +110,7 @@ struct Tuning {
     int stream_weights_mib = 48;    // VTL_HIP_STREAM_WEIGHTS_MIB: weight matrices of this many MiB and more are read with non-temporal loads by the kernels for 2 to 32 rows (0: always)
     int skinny_tiled = -1;          // VTL_HIP_SKINNY_TILED: 1 / 0 force the 32x32-block weight-streaming kernel for M > 32
     int skinny_waves = 4;           // VTL_HIP_SKINNY_WAVES: 2, 4 or 8 waves (K ranges) per workgroup there
-    int matmul_tile = 0;            // VTL_HIP_MATMUL_TILE: 128 / 64 force the f64-accumulating tile
+    int matmul_tile = 0;            // VTL_HIP_MATMUL_TILE: which kernel and tile the f64-accumulating matmul takes (matmul_f64acc.hip)
     int matmul_splits = -1;         // VTL_HIP_MATMUL_SPLITS: K ranges of the f64-accumulating matmul
 };
 const Tuning &tuning();

@@ -5,8 +5,12 @@
 // Also the unquantized Linear forward (nn/layers/linear_forward_f32.v:16-18)
 // and LinearGate.backward (nn/gates/layers/linear.v:69-79) built on it.
 //
-// One workgroup of WR x WC waves owns a BM x BN tile of C.  Both operands are
-// staged through LDS in k-major form (As[k][m], Bs[k][n]) whatever their
+// Two kernels.  matmul_f64acc_kernel stages 128 x 128 tiles through LDS for large products of whole
+// tiles; matmul_f64acc_direct_kernel, for everything else, takes operands from global memory
+// straight to registers.  choose_plan() picks by estimated time.
+//
+// The staged kernel: one workgroup of WR x WC waves owns a BM x BN tile of C.  Both operands go
+// through LDS in k-major form (As[k][m], Bs[k][n]) whatever their
 // layout in memory, so that one 16- or 32-byte LDS read hands a lane the
 // operands of all its 16x16x4 MFMA tiles for one k.  MFMA tile i of a wave
 // holds the rows {TM * r + i : r = 0..15} of the wave's rows (and likewise for
@@ -28,34 +32,15 @@ struct MatmulArgs {
     void *C;            // [M,N] row-major
     const void *bias;   // N values added after rounding to the output type, or nullptr
     int M, N, K;
-    int vec_a, vec_b, vec_c;   // base 16-byte aligned and leading dimension % 4 == 0
     int relu;
-    int k_per_split;           // split-K launches: k range of one grid.y slice (multiple of 32)
-    double *partial;           // split-K launches: [splits][M][N] unrounded sums
+    int k_per_split;    // k range of one grid.y slice (multiple of 16)
+    double *partial;    // launches that slice K: [slices][M][N] unrounded sums, else nullptr
 };
 
 template <typename T>
 struct alignas(16) Vec4 {
     T v[4];
 };
-
-// Four consecutive elements of a row-major matrix starting at (row, col);
-// positions outside rows x cols read as zero.  GUARD == false: the caller
-// knows that every position is inside and 16-byte aligned.
-template <typename T, bool GUARD>
-__device__ __forceinline__ Vec4<T> load4(const T *__restrict__ base, int ld, int rows, int cols, int row,
-                                         int col, bool vec_ok)
-{
-    Vec4<T> out;
-    if (!GUARD || (row < rows && col + 3 < cols && vec_ok)) {
-        out = *reinterpret_cast<const Vec4<T> *>(base + (int64_t)row * ld + col);
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            out.v[j] = (row < rows && col + j < cols) ? base[(int64_t)row * ld + col + j] : T(0);
-    }
-    return out;
-}
 
 // NT consecutive LDS elements (NT = 2 or 4, naturally aligned) widened to f64.
 template <typename T, int NT>
@@ -73,16 +58,14 @@ __device__ __forceinline__ void read_operands(const T *__restrict__ p, double (&
 // One operand tile of BK x BMN elements (k-major in LDS, row stride LDW).
 // KMAJOR: the matrix is stored with the tile's m/n index contiguous ([K, MN]);
 // otherwise it is stored [MN, K] and is transposed on the way into LDS.
-template <typename T, int BK, int BMN, int LDW, int NT, bool KMAJOR, bool GUARD>
+template <typename T, int BK, int BMN, int LDW, int NT, bool KMAJOR>
 struct OperandTile {
-    static constexpr int kGroups = BK * BMN / 4;           // 4-element groups per tile
+    static constexpr int kGroups = BK * BMN / 4;       // 4-element groups per tile
     static constexpr int kPerThread = (kGroups + NT - 1) / NT;   // NT threads in the workgroup
-    Vec4<T> regs[kPerThread];
+    typedef T Group __attribute__((ext_vector_type(4)));   // (a struct of four stays in scratch memory)
+    Group regs[kPerThread];
 
-    // k_total: the matrix's K (its leading dimension when stored [MN, K]);
-    // k_limit <= k_total: positions with k >= k_limit read as zero.
-    __device__ __forceinline__ void fetch(const T *__restrict__ base, int mn_total, int k_total, int k_limit,
-                                          int mn0, int k0, bool vec_ok)
+    __device__ __forceinline__ void fetch(const T *__restrict__ base, int mn_total, int k_total, int mn0, int k0)
     {
         const int t = threadIdx.x;
 #pragma unroll
@@ -90,13 +73,12 @@ struct OperandTile {
             const int g = t + NT * i;
             if (kGroups % NT != 0 && g >= kGroups)
                 break;
-            if constexpr (KMAJOR) {
-                const int krow = g / (BMN / 4), c4 = g % (BMN / 4);
-                regs[i] = load4<T, GUARD>(base, mn_total, k_limit, mn_total, k0 + krow, mn0 + 4 * c4, vec_ok);
-            } else {
-                const int mn = g % BMN, kc = g / BMN;
-                regs[i] = load4<T, GUARD>(base, k_total, mn_total, k_limit, mn0 + mn, k0 + 4 * kc, vec_ok);
-            }
+            const T *__restrict__ p;
+            if constexpr (KMAJOR)
+                p = base + (int64_t)(k0 + g / (BMN / 4)) * mn_total + mn0 + 4 * (g % (BMN / 4));
+            else
+                p = base + (int64_t)(mn0 + g % BMN) * k_total + k0 + 4 * (g / BMN);
+            regs[i] = *reinterpret_cast<const Group *>(p);
         }
     }
 
@@ -110,12 +92,12 @@ struct OperandTile {
                 break;
             if constexpr (KMAJOR) {
                 const int krow = g / (BMN / 4), c4 = g % (BMN / 4);
-                *reinterpret_cast<Vec4<T> *>(lds + krow * LDW + 4 * c4) = regs[i];
+                *reinterpret_cast<Group *>(lds + krow * LDW + 4 * c4) = regs[i];
             } else {
                 const int mn = g % BMN, kc = g / BMN;
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
-                    lds[(4 * kc + j) * LDW + mn] = regs[i].v[j];
+                    lds[(4 * kc + j) * LDW + mn] = regs[i][j];
             }
         }
     }
@@ -131,20 +113,17 @@ __device__ __forceinline__ void lds_barrier()
     asm volatile("" ::: "memory");
 }
 
-// GUARD == false: M, N, K are whole tiles and every row is 16-byte aligned, so
-// the loads and stores carry no bounds checks and the k-loop is straight-line code.
-// SPLIT: grid.y slices K; each slice writes its unrounded f64 sums to g.partial.
+// M, N, K are whole tiles and every row is 16-byte aligned.
 // Workgroup = WR x WC waves, each with TM x TN MFMA tiles of 16x16:
 // BM = 16 * TM * WR, BN = 16 * TN * WC.
-template <typename T, int TM, int TN, int WR, int WC, bool TA, bool TB, bool GUARD, bool SPLIT>
+template <typename T, int TM, int TN, int WR, int WC, bool TA, bool TB>
 __global__ __launch_bounds__(64 * WR * WC) void matmul_f64acc_kernel(const MatmulArgs g)
 {
     constexpr int BM = 16 * TM * WR, BN = 16 * TN * WC, NT = 64 * WR * WC;
-    // bytes of k per tile row: 64 (16 f32 / 8 f64); the small tile takes 128 to halve its barriers
-    constexpr int BK = (BM * BN <= 64 * 64 ? 128 : 64) / (int)sizeof(T);
+    constexpr int BK = 64 / (int)sizeof(T);   // bytes of k per tile row: 64 (16 f32 / 8 f64)
     constexpr int LDA = BM + 4, LDB = BN + 4;
     static_assert(TM == 2 || TM == 4, "wave tile is 32 or 64 rows");
-    static_assert(TN == 2 || TN == 4, "wave tile is 32 or 64 columns");
+    static_assert(TN == 4, "wave tile is 64 columns");
 
     // Three LDS buffers per operand: while tile kt is multiplied, tile kt+1 is
     // written at the start of the step (its global loads were issued a step
@@ -156,7 +135,7 @@ __global__ __launch_bounds__(64 * WR * WC) void matmul_f64acc_kernel(const Matmu
 
     const T *__restrict__ A = static_cast<const T *>(g.A);
     const T *__restrict__ B = static_cast<const T *>(g.B);
-    const int tiles_n = (g.N + BN - 1) / BN;
+    const int tiles_n = g.N / BN;
     const int m0 = (int)(blockIdx.x / tiles_n) * BM;
     const int n0 = (int)(blockIdx.x % tiles_n) * BN;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -164,9 +143,9 @@ __global__ __launch_bounds__(64 * WR * WC) void matmul_f64acc_kernel(const Matmu
     const int r16 = lane & 15, kq = lane >> 4;
 
     // A as op(A)[M,K]: stored [K,M] when transposed (k-major already)
-    OperandTile<T, BK, BM, LDA, NT, TA, GUARD> ta;
+    OperandTile<T, BK, BM, LDA, NT, TA> ta;
     // B as op(B)[K,N]: stored [K,N] when not transposed (k-major already)
-    OperandTile<T, BK, BN, LDB, NT, !TB, GUARD> tb;
+    OperandTile<T, BK, BN, LDB, NT, !TB> tb;
 
     double4_t acc[TM][TN];
 #pragma unroll
@@ -175,19 +154,17 @@ __global__ __launch_bounds__(64 * WR * WC) void matmul_f64acc_kernel(const Matmu
         for (int j = 0; j < TN; ++j)
             acc[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
 
-    const int k_begin = SPLIT ? (int)blockIdx.y * g.k_per_split : 0;
-    const int k_end = SPLIT ? (k_begin + g.k_per_split < g.K ? k_begin + g.k_per_split : g.K) : g.K;
-    const int ktiles = (k_end - k_begin + BK - 1) / BK;
+    const int ktiles = g.K / BK;
     constexpr int S = BK / 4;   // k-groups (one MFMA step each) per tile
     const int aoff = wm + TM * r16 + kq * LDA, boff = wn + TN * r16 + kq * LDB;
 
-    ta.fetch(A, g.M, g.K, k_end, m0, k_begin, g.vec_a != 0);
-    tb.fetch(B, g.N, g.K, k_end, n0, k_begin, g.vec_b != 0);
+    ta.fetch(A, g.M, g.K, m0, 0);
+    tb.fetch(B, g.N, g.K, n0, 0);
     ta.stash(As[0]);
     tb.stash(Bs[0]);
     if (ktiles > 1) {
-        ta.fetch(A, g.M, g.K, k_end, m0, k_begin + BK, g.vec_a != 0);
-        tb.fetch(B, g.N, g.K, k_end, n0, k_begin + BK, g.vec_b != 0);
+        ta.fetch(A, g.M, g.K, m0, BK);
+        tb.fetch(B, g.N, g.K, n0, BK);
     }
     __syncthreads();
     double a[TM], b[TN];
@@ -203,8 +180,8 @@ __global__ __launch_bounds__(64 * WR * WC) void matmul_f64acc_kernel(const Matmu
             tb.stash(Bs[nxt]);
         }
         if (kt + 2 < ktiles) {
-            ta.fetch(A, g.M, g.K, k_end, m0, k_begin + (kt + 2) * BK, g.vec_a != 0);
-            tb.fetch(B, g.N, g.K, k_end, n0, k_begin + (kt + 2) * BK, g.vec_b != 0);
+            ta.fetch(A, g.M, g.K, m0, (kt + 2) * BK);
+            tb.fetch(B, g.N, g.K, n0, (kt + 2) * BK);
         }
 #pragma unroll
         for (int s = 0; s < S; ++s) {
@@ -232,36 +209,19 @@ __global__ __launch_bounds__(64 * WR * WC) void matmul_f64acc_kernel(const Matmu
         cur = nxt;
     }
 
-    if constexpr (SPLIT) {
-        double *__restrict__ P = g.partial + (int64_t)blockIdx.y * g.M * g.N;
-        const int pcol0 = n0 + wn + TN * r16;
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int row = m0 + wm + TM * (4 * e + kq) + i;
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    if (!GUARD || (row < g.M && pcol0 + j < g.N))
-                        P[(int64_t)row * g.N + pcol0 + j] = acc[i][j][e];
-            }
-        return;
-    }
     T *__restrict__ C = static_cast<T *>(g.C);
     const T *__restrict__ bias = static_cast<const T *>(g.bias);
     const int col0 = n0 + wn + TN * r16;
     T bv[TN];
 #pragma unroll
     for (int j = 0; j < TN; ++j)
-        bv[j] = (bias && (!GUARD || col0 + j < g.N)) ? bias[col0 + j] : T(0);
+        bv[j] = bias ? bias[col0 + j] : T(0);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int row = m0 + wm + TM * (4 * e + kq) + i;
-            if (GUARD && row >= g.M)
-                continue;
-            T out[TN];
+            Vec4<T> out;
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 T y = (T)acc[i][j][e];   // the one rounding to the tensor's type
@@ -269,31 +229,211 @@ __global__ __launch_bounds__(64 * WR * WC) void matmul_f64acc_kernel(const Matmu
                     y = y + bv[j];       // Tensor.add in the tensor's type
                 if (g.relu && y < T(0))
                     y = T(0);
-                out[j] = y;
+                out.v[j] = y;
             }
-            T *dst = C + (int64_t)row * g.N + col0;
-            if (!GUARD || (g.vec_c && col0 + TN - 1 < g.N)) {
-                if constexpr (TN == 4) {
-                    Vec4<T> v;
+            *reinterpret_cast<Vec4<T> *>(C + (int64_t)row * g.N + col0) = out;
+        }
+    }
+}
+
+// ---- operands straight from global memory --------------------------------------------------
+// A wave owns 32 x 16 * TN of C.  An f64 MFMA wants two values a lane every 64 cycles, so operands
+// need neither LDS nor barriers, and what bounds a launch is how evenly its MFMAs spread over the
+// SIMDs: the tiles are small, K is cut over the WK waves of a workgroup (partial tiles meet in LDS)
+// and, with few tiles, over grid.y.  With 64 x 64 tiles staged in LDS a wave had four MFMAs for every 4
+// of K, 7 us at K = 256 and 14 us at K = 512 whatever else the chip did, and ragged sizes loaded
+// element by element: 512^3 22.4 -> 8.8 us, 64 x 784 x 256 16.4 -> 5.5, 64 x 256 x 784 44 -> 7.5,
+// 255 x 11007 x 4095 447 -> 367, 333 x 517 x 701 47 -> 13 (f32; f64 alike).
+//
+// Steps of 16 of K are dealt out to the WK waves in turn.  In a step lane l holds four k for the two
+// rows 2 * (l % 16) + {0, 1} of A and for TN / 2 such pairs of columns of B: 16-byte loads where K runs
+// along memory, pairs of 32 neighbouring columns where it does not.  MFMA j of a step takes the j-th of
+// each lane's four: which k they are is free as long as both operands agree.
+// Vector loads need no more than the elements' own alignment on gfx950, so ragged rows take them too;
+// what is left of K after whole steps is a step of its own with checked loads.  CHECKED: every
+// load is (a single row or column of a matrix that has to give pairs).
+template <typename T, bool KROWS, bool CHECKED>
+__device__ __forceinline__ void direct_fetch(T (&out)[2][4], const T *__restrict__ base, int mn_total, int k_total,
+                                            const int (&mn)[2], bool second_only, int k0, int kq)
+{
+    // a 16-byte load holds VK elements; the lane's four are those VK of each run of 4 * VK
+    constexpr int VK = 16 / (int)sizeof(T);
+    struct alignas(sizeof(T)) Run {
+        T v[VK];
+    };
+    struct alignas(sizeof(T)) Pair {
+        T v[2];
+    };
 #pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        v.v[j] = out[j];
-                    *reinterpret_cast<Vec4<T> *>(dst) = v;
+    for (int q = 0; q < 4; q += VK) {
+        const int k = k0 + 4 * q + VK * kq;
+        if constexpr (KROWS) {   // [MN, K]
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const T *__restrict__ p = base + (int64_t)mn[i] * k_total + k;
+                if constexpr (!CHECKED) {
+                    const Run v = *reinterpret_cast<const Run *>(p);
+#pragma unroll
+                    for (int j = 0; j < VK; ++j)
+                        out[i][q + j] = v.v[j];
                 } else {
-                    struct alignas(2 * sizeof(T)) Vec2 {
-                        T v[2];
-                    } v;
-                    v.v[0] = out[0];
-                    v.v[1] = out[1];
-                    *reinterpret_cast<Vec2 *>(dst) = v;
-                }
-            } else {
 #pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    if (col0 + j < g.N)
-                        dst[j] = out[j];
+                    for (int j = 0; j < VK; ++j)
+                        out[i][q + j] = k + j < k_total ? p[j] : T(0);
+                }
+            }
+        } else {                 // [K, MN]
+#pragma unroll
+            for (int j = 0; j < VK; ++j) {
+                if constexpr (!CHECKED) {
+                    // second_only: the pair was moved back by one to stay inside, its second is mn[0]
+                    const Pair v = *reinterpret_cast<const Pair *>(base + (int64_t)(k + j) * mn_total + mn[0] -
+                                                                   (second_only ? 1 : 0));
+                    out[0][q + j] = second_only ? v.v[1] : v.v[0];
+                    out[1][q + j] = v.v[1];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        out[i][q + j] = k + j < k_total ? base[(int64_t)(k + j) * mn_total + mn[i]] : T(0);
+                }
             }
         }
+    }
+}
+
+// The tiles of a workgroup are WM x WN wave tiles of 32 x 16 * TN, K is cut over WK waves each.
+// Blocks are renumbered so that each of the 8 XCDs (own L2) works on a compact patch of tiles, eight
+// tile rows deep: with the plain order the rows that share a column panel of B run on different XCDs.
+template <typename T, int WM, int WN, int WK, int TN, bool TA, bool TB, bool CHECKED>
+__global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel(const MatmulArgs g)
+{
+    constexpr int D = sizeof(T) == 4 && TN == 2 ? 4 : 2;   // steps whose operands are in flight
+    constexpr int P = TN / 2;                              // column pairs of a lane
+    constexpr int V = 8 * TN;                              // values of a lane
+    __shared__ double red[WK > 1 ? WM * WN * WK : 1][WK > 1 ? V : 1][64];
+    const T *__restrict__ A = static_cast<const T *>(g.A);
+    const T *__restrict__ B = static_cast<const T *>(g.B);
+    constexpr int BM = 32 * WM, BN = 16 * TN * WN;
+    const int tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
+    int tm, tn;
+    {
+        const int total = tiles_m * tiles_n, block = (int)blockIdx.x;
+        const int xcd = block & 7, over = total & 7;
+        const int pid = xcd * (total >> 3) + min(xcd, over) + (block >> 3);
+        const int group = 8 * tiles_n, first_m = (pid / group) * 8, gm = min(tiles_m - first_m, 8);
+        tm = first_m + (pid % group) % gm;
+        tn = (pid % group) / gm;
+    }
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wk = wave % WK, tile = wave / WK;
+    const int m0 = tm * BM + (tile / WN) * 32, n0 = tn * BN + (tile % WN) * 16 * TN;
+    const int r16 = lane & 15, kq = lane >> 4;
+    // this workgroup's whole steps of K (all of them, or one of grid.y slices), this wave's among
+    // them, and whether this wave does the part of a step at the end of K
+    const int steps = CHECKED ? (g.K + 15) / 16 : g.K / 16, per = g.k_per_split / 16;
+    const int first = (int)blockIdx.y * per, last = min(first + per, steps) - 1;
+    const int count = first + wk > last ? 0 : (last - first - wk) / WK + 1;
+    const bool rest = !CHECKED && steps * 16 < g.K && blockIdx.y == gridDim.y - 1 && wk == WK - 1;
+
+    // rows and columns past the edge repeat the last ones; what they give is not stored
+    const int row[2] = {min(m0 + 2 * r16, g.M - 1), min(m0 + 2 * r16 + 1, g.M - 1)};
+    const bool row_alone = row[0] == g.M - 1;
+    int col[P][2];
+    bool col_alone[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        col[p][0] = min(n0 + 32 * p + 2 * r16, g.N - 1);
+        col[p][1] = min(n0 + 32 * p + 2 * r16 + 1, g.N - 1);
+        col_alone[p] = col[p][0] == g.N - 1;
+    }
+    T fa[D][2][4], fb[D][P][2][4];
+    auto fetch = [&](int d, int i) {   // the wave's i-th step; past its end the last one again
+        const int k0 = min(first + wk + i * WK, last) * 16;
+        direct_fetch<T, !TA, CHECKED>(fa[d], A, g.M, g.K, row, row_alone, k0, kq);
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+            direct_fetch<T, TB, CHECKED>(fb[d][p], B, g.N, g.K, col[p], col_alone[p], k0, kq);
+    };
+    double4_t acc[2][TN];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+            acc[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
+    auto multiply = [&](int d) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                        (double)fa[d][i][k], (double)fb[d][j >> 1][j & 1][k], acc[i][j], 0, 0, 0);
+    };
+    if (count > 0) {
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            fetch(d, d);
+        int i = 0;
+        for (; i + D <= count; i += D) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                multiply(d);
+                fetch(d, i + d + D);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < D - 1; ++d)
+            if (i + d < count)
+                multiply(d);
+    }
+    if (rest) {
+        const int k0 = steps * 16;
+        direct_fetch<T, !TA, true>(fa[0], A, g.M, g.K, row, false, k0, kq);
+#pragma unroll
+        for (int p = 0; p < P; ++p)
+            direct_fetch<T, TB, true>(fb[0][p], B, g.N, g.K, col[p], false, k0, kq);
+        multiply(0);
+    }
+    T *__restrict__ C = static_cast<T *>(g.C);
+    const T *__restrict__ bias = static_cast<const T *>(g.bias);
+    double *__restrict__ partial = g.partial ? g.partial + (int64_t)blockIdx.y * g.M * g.N : nullptr;
+    // value v of a lane: i = v / (4 TN), j = v / 4 % TN, e = v % 4
+    auto store = [&](int v, double s) {
+        const int j = (v >> 2) & (TN - 1);
+        const int r = m0 + 2 * (4 * (v & 3) + kq) + v / (4 * TN), c = n0 + 32 * (j >> 1) + 2 * r16 + (j & 1);
+        if (r >= g.M || c >= g.N)
+            return;
+        if (partial) {
+            partial[(int64_t)r * g.N + c] = s;
+            return;
+        }
+        T y = (T)s;              // the one rounding to the tensor's type
+        if (bias)
+            y = y + bias[c];     // Tensor.add in the tensor's type
+        if (g.relu && y < T(0))
+            y = T(0);
+        C[(int64_t)r * g.N + c] = y;
+    };
+    if constexpr (WK == 1) {
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            store(v, acc[v / (4 * TN)][(v >> 2) & (TN - 1)][v & 3]);
+        return;
+    }
+    // partial tiles, in the order of the registers
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+        red[wave][v][lane] = acc[v / (4 * TN)][(v >> 2) & (TN - 1)][v & 3];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < V / WK; ++u) {
+        const int v = wk + WK * u;
+        double s = red[tile * WK][v][lane];
+#pragma unroll
+        for (int w = 1; w < WK; ++w)
+            s += red[tile * WK + w][v][lane];
+        store(v, s);
     }
 }
 
@@ -395,62 +535,142 @@ __global__ __launch_bounds__(256) void matmul_splitk_finalize_kernel(const Matmu
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-template <typename T, int TM, int TN, int WR, int WC, bool GUARD, bool SPLIT>
-int launch_tile_guard(const MatmulArgs &g, bool ta, bool tb, int splits, hipStream_t st)
+template <typename T>
+int launch_staged(const MatmulArgs &g, bool ta, bool tb, hipStream_t st)
 {
-    constexpr int BM = 16 * TM * WR, BN = 16 * TN * WC;
-    const int64_t tiles = (int64_t)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
+    // eight waves of 32x64 per 128x128 tile measured a few percent above four waves of 64x64
+    const int64_t tiles = (int64_t)(g.M / 128) * (g.N / 128);
     if (tiles > 0x7fffffff)
         return VTL_HIP_ERR_UNSUPPORTED;
-    const dim3 grid((unsigned)tiles, (unsigned)splits), block(64 * WR * WC);
+    const dim3 grid((unsigned)tiles), block(512);
     if (!ta && !tb)
-        hipLaunchKernelGGL((matmul_f64acc_kernel<T, TM, TN, WR, WC, false, false, GUARD, SPLIT>), grid, block, 0,
-                           st, g);
+        hipLaunchKernelGGL((matmul_f64acc_kernel<T, 2, 4, 4, 2, false, false>), grid, block, 0, st, g);
     else if (!ta && tb)
-        hipLaunchKernelGGL((matmul_f64acc_kernel<T, TM, TN, WR, WC, false, true, GUARD, SPLIT>), grid, block, 0,
-                           st, g);
+        hipLaunchKernelGGL((matmul_f64acc_kernel<T, 2, 4, 4, 2, false, true>), grid, block, 0, st, g);
     else if (ta && !tb)
-        hipLaunchKernelGGL((matmul_f64acc_kernel<T, TM, TN, WR, WC, true, false, GUARD, SPLIT>), grid, block, 0,
-                           st, g);
+        hipLaunchKernelGGL((matmul_f64acc_kernel<T, 2, 4, 4, 2, true, false>), grid, block, 0, st, g);
     else
-        hipLaunchKernelGGL((matmul_f64acc_kernel<T, TM, TN, WR, WC, true, true, GUARD, SPLIT>), grid, block, 0,
-                           st, g);
+        hipLaunchKernelGGL((matmul_f64acc_kernel<T, 2, 4, 4, 2, true, true>), grid, block, 0, st, g);
     return check_launch("matmul_f64acc_kernel");
 }
 
-// Shapes made of whole tiles with 16-byte aligned rows run without bounds checks.
-template <typename T, int TM, int TN, int WR, int WC>
-int launch_tile(const MatmulArgs &g, bool ta, bool tb, hipStream_t st)
+template <typename T>
+int finalize_split(const MatmulArgs &g, int splits, hipStream_t st)
 {
-    constexpr int BM = 16 * TM * WR, BN = 16 * TN * WC;
-    const bool whole = g.M % BM == 0 && g.N % BN == 0 && g.K % 32 == 0 && g.K > 0 && g.vec_a && g.vec_b &&
-                       g.vec_c;
-    return whole ? launch_tile_guard<T, TM, TN, WR, WC, false, false>(g, ta, tb, 1, st)
-                 : launch_tile_guard<T, TM, TN, WR, WC, true, false>(g, ta, tb, 1, st);
-}
-
-// Few output tiles and a long K: slice K over grid.y so that every SIMD holds
-// several waves, f64 partial sums in the library's workspace, then one pass
-// that adds the slices in order and rounds.
-template <typename T, int TM, int TN, int WR, int WC>
-int launch_split(MatmulArgs g, bool ta, bool tb, int splits, hipStream_t st)
-{
-    constexpr int BM = 16 * TM * WR, BN = 16 * TN * WC;
-    const int per = ((g.K + splits - 1) / splits + 31) / 32 * 32;
-    splits = (g.K + per - 1) / per;
-    g.k_per_split = per;
-    g.partial = static_cast<double *>(
-        vtlhip::library_workspace((size_t)splits * (size_t)g.M * (size_t)g.N * sizeof(double)));
-    if (!g.partial)
-        return vtlhip::workspace_status();
-    const bool whole = g.M % BM == 0 && g.N % BN == 0 && g.K % per == 0 && g.vec_a && g.vec_b;
-    int rc = whole ? launch_tile_guard<T, TM, TN, WR, WC, false, true>(g, ta, tb, splits, st)
-                   : launch_tile_guard<T, TM, TN, WR, WC, true, true>(g, ta, tb, splits, st);
-    if (rc != VTL_HIP_OK)
-        return rc;
     const int64_t blocks = ((int64_t)g.M * g.N + 255) / 256;
     hipLaunchKernelGGL((matmul_splitk_finalize_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, st, g, splits);
     return check_launch("matmul_splitk_finalize_kernel");
+}
+
+// How a product runs: the staged kernel, or one of the direct kernel's shapes with K in `slices`.
+enum Shape { kStaged, kK8, kK4, kWide, kPairK2, kPanel, kShapes };
+struct Plan {
+    Shape shape;
+    int slices;
+};
+
+// Wave tiles and waves per tile: what the names above stand for.
+constexpr int kTileM[kShapes] = {128, 32, 32, 32, 64, 64};
+constexpr int kTileN[kShapes] = {128, 32, 32, 64, 64, 128};
+
+// Estimated microseconds: start + rounds * (per_tile + work / rate), where `rounds` is how many
+// workgroups the busiest compute unit gets and `work` the time its matrix cores need for one tile at
+// 2.3 GHz; slicing K adds a launch and its partial sums (per MB).  Fitted to 240 products drawn over
+// m, n up to 11008 and k up to 4096, whole and ragged, all four layouts, every shape timed alternately:
+// the choice is on average 2.6 % and at most 30 % behind the fastest.
+struct Cost {
+    double start, per_tile, inverse_rate, slice_start, slice_mb;
+};
+constexpr Cost kCost[2][kShapes] = {
+    // f32
+    {{2.9, 0.0, 1.12, 0, 0}, {2.8, 1.27, 1.27, 3.5, 0.68}, {3.3, 0.56, 1.31, 3.9, 0.55}, {2.9, 1.61, 1.13, 3.7, 0.60},
+     {3.1, 2.20, 1.13, 4.0, 0.35}, {3.2, 2.85, 1.19, 4.0, 0.35}},
+    // f64
+    {{2.5, 2.5, 1.14, 0, 0}, {1.9, 1.71, 1.41, 3.1, 1.39}, {3.1, 0.68, 1.44, 3.6, 0.73}, {2.8, 1.68, 1.23, 4.0, 0.58},
+     {3.3, 2.21, 1.18, 4.0, 0.27}, {2.5, 3.40, 1.19, 4.0, 0.27}},
+};
+
+Plan choose_plan(bool f64, int m, int n, int k, bool whole)
+{
+    Plan best = {kK4, 1};
+    double best_us = 1e30;
+    for (int s = whole ? kStaged : kK8; s < kShapes; s++) {
+        const Cost &c = kCost[f64 ? 1 : 0][s];
+        const int64_t tiles = (int64_t)((m + kTileM[s] - 1) / kTileM[s]) * ((n + kTileN[s] - 1) / kTileN[s]);
+        // no slices, one workgroup per compute unit in all, or two where K is long
+        int64_t want[3] = {1, 0, 0};
+        if (s != kStaged && k >= 512 && tiles < 256) {
+            want[1] = 256 / tiles;
+            want[2] = k >= 2048 ? 2 * want[1] : 0;
+        }
+        for (int64_t slices : want) {
+            if (slices > k / 96)
+                slices = k / 96;
+            if (slices > 32)
+                slices = 32;
+            if (slices < 1)
+                slices = 1;
+            const double rounds = (double)((tiles * slices + 255) / 256);
+            const double work = (double)kTileM[s] * kTileN[s] * ((double)k / (double)slices) / (64.0 * 2300.0);
+            double us = c.start + rounds * (c.per_tile + work * c.inverse_rate);
+            if (slices > 1)
+                us += c.slice_start + c.slice_mb * 8e-6 * (double)slices * (double)m * (double)n;
+            if (us < best_us) {
+                best_us = us;
+                best = {(Shape)s, (int)slices};
+            }
+        }
+    }
+    return best;
+}
+
+template <typename T, int WM, int WN, int WK, int TN, bool CHECKED = false>
+int launch_direct_shape(const MatmulArgs &g, bool ta, bool tb, int slices, hipStream_t st)
+{
+    constexpr int BM = 32 * WM, BN = 16 * TN * WN;
+    const int64_t tiles = (int64_t)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
+    if (tiles > 0x7fffffff)
+        return VTL_HIP_ERR_UNSUPPORTED;
+    const dim3 grid((unsigned)tiles, (unsigned)slices), block(64 * WM * WN * WK);
+    if (!ta && !tb)
+        hipLaunchKernelGGL((matmul_f64acc_direct_kernel<T, WM, WN, WK, TN, false, false, CHECKED>), grid, block, 0, st, g);
+    else if (!ta && tb)
+        hipLaunchKernelGGL((matmul_f64acc_direct_kernel<T, WM, WN, WK, TN, false, true, CHECKED>), grid, block, 0, st, g);
+    else if (ta && !tb)
+        hipLaunchKernelGGL((matmul_f64acc_direct_kernel<T, WM, WN, WK, TN, true, false, CHECKED>), grid, block, 0, st, g);
+    else
+        hipLaunchKernelGGL((matmul_f64acc_direct_kernel<T, WM, WN, WK, TN, true, true, CHECKED>), grid, block, 0, st, g);
+    return check_launch("matmul_f64acc_direct_kernel");
+}
+
+template <typename T>
+int launch_direct(MatmulArgs g, bool ta, bool tb, Plan plan, hipStream_t st)
+{
+    // pairs of a row or column index that runs along memory need two of them
+    const bool checked = (ta && g.M < 2) || (!tb && g.N < 2);
+    const int steps = checked ? (g.K + 15) / 16 : g.K / 16, per = (steps + plan.slices - 1) / plan.slices;
+    const int slices = per > 0 ? (steps + per - 1) / per : 1;
+    g.k_per_split = 16 * per;
+    if (slices > 1) {
+        g.partial = static_cast<double *>(
+            vtlhip::library_workspace((size_t)slices * (size_t)g.M * (size_t)g.N * sizeof(double)));
+        if (!g.partial)
+            return vtlhip::workspace_status();
+    }
+    int rc;
+    if (checked)
+        rc = launch_direct_shape<T, 1, 1, 8, 2, true>(g, ta, tb, slices, st);
+    else if (plan.shape == kK8)
+        rc = launch_direct_shape<T, 1, 1, 8, 2>(g, ta, tb, slices, st);
+    else if (plan.shape == kWide)
+        rc = launch_direct_shape<T, 1, 1, 4, 4>(g, ta, tb, slices, st);
+    else if (plan.shape == kPairK2)
+        rc = launch_direct_shape<T, 2, 1, 2, 4>(g, ta, tb, slices, st);
+    else if (plan.shape == kPanel)
+        rc = launch_direct_shape<T, 2, 2, 1, 4>(g, ta, tb, slices, st);
+    else
+        rc = launch_direct_shape<T, 1, 1, 4, 2>(g, ta, tb, slices, st);
+    return rc != VTL_HIP_OK || slices == 1 ? rc : finalize_split<T>(g, slices, st);
 }
 
 template <typename T>
@@ -471,51 +691,31 @@ int matmul_impl(const T *a, const T *b, T *c, const T *bias, int m, int n, int k
     g.M = m;
     g.N = n;
     g.K = k;
-    const int lda = trans_a ? m : k, ldb = trans_b ? k : n;
-    g.vec_a = aligned16(a) && lda % 4 == 0;
-    g.vec_b = aligned16(b) && ldb % 4 == 0;
-    g.vec_c = aligned16(c) && n % 4 == 0;
     g.relu = relu;
     g.k_per_split = 0;
     g.partial = nullptr;
-    hipStream_t st = current_stream();
-    // Tile choice by a per-compute-unit estimate, in units of one 128x128 tile at
-    // peak: a compute unit runs two big workgroups together at ~0.84 of peak and
-    // a single one at ~0.75; the 64x64 tile kernel reaches 0.72 (four workgroups
-    // per compute unit) to 0.78 (many) and quantizes four times finer over the
-    // 256 compute units.  Constants fitted to measured times (with many tiles
-    // the big one is 7-12 % faster, e.g. 11008x4096x256: 350 against 377 us).
-    const int64_t big = (int64_t)((m + 127) / 128) * ((n + 127) / 128);
-    const int64_t small = (int64_t)((m + 63) / 64) * ((n + 63) / 64);
-    const int64_t c128 = (big + 255) / 256, c64 = (small + 255) / 256;
-    const double t128 = (double)(c128 / 2) * (2.0 / 0.84) + (double)(c128 % 2) * (1.0 / 0.75);
-    const double t64 = (double)c64 * 0.25 / (0.78 - 0.24 / (double)c64);
-    // eight waves of 32x64 per 128x128 tile measured a few percent above four waves of 64x64
-    const int tile_env = vtlhip::tuning().matmul_tile;   // VTL_HIP_MATMUL_TILE 128 / 64 forces the tile (tuning, tests)
-    if (tile_env ? tile_env == 128 : t128 <= t64)
-        return launch_tile<T, 2, 4, 4, 2>(g, trans_a != 0, trans_b != 0, st);
-    const bool force = vtlhip::tuning().matmul_splits >= 0;   // VTL_HIP_MATMUL_SPLITS (tuning and tests)
-    // Too few big tiles for the chip but a long K: cut K until about 512 big
-    // workgroups exist (two per compute unit); measured 8-12 % faster than
-    // the small tile with its own split (256x4096x11008: 428 -> 386 us).
-    if (!force && m >= 128 && big >= 32 && k >= 2048) {
-        int sp = 1;
-        while (big * sp < 512 && sp < 16 && k / (2 * sp) >= 512)
-            sp *= 2;
-        if (sp > 1)
-            return launch_split<T, 2, 4, 4, 2>(g, trans_a != 0, trans_b != 0, sp, st);
+    // the staged kernel's loads and stores carry no bounds checks
+    const bool whole = m % 128 == 0 && n % 128 == 0 && k % 32 == 0 && k > 0 && aligned16(a) && aligned16(b) &&
+                       aligned16(c);
+    Plan plan = choose_plan(sizeof(T) == 8, m, n, k, whole);
+    // Tuning and tests: VTL_HIP_MATMUL_TILE 128 forces the staged kernel where it can run, 64 the
+    // 64 x 64 tiles, 1 .. 5 a shape of the direct kernel; VTL_HIP_MATMUL_SPLITS the slices of K.
+    const int tile = vtlhip::tuning().matmul_tile, splits = vtlhip::tuning().matmul_splits;
+    if (tile == 128 && whole)
+        plan.shape = kStaged;
+    else if (tile == 64)
+        plan.shape = kPairK2;
+    else if (tile >= kK8 && tile < kShapes)
+        plan.shape = (Shape)tile;
+    if (splits >= 0) {
+        plan.slices = splits > 1 && k >= 32 * splits ? splits : 1;
+        if (plan.shape == kStaged && plan.slices > 1)
+            plan.shape = kK4;
+    } else if (plan.shape == kStaged) {
+        plan.slices = 1;
     }
-    int splits = force ? vtlhip::tuning().matmul_splits : 1;
-    if (!force && small <= 512 && k >= 2048) {
-        splits = (int)(1024 / small);
-        if (splits > k / 512)
-            splits = k / 512;
-        if (splits > 16)
-            splits = 16;
-    }
-    if (splits > 1 && k >= 32 * splits)
-        return launch_split<T, 2, 2, 2, 2>(g, trans_a != 0, trans_b != 0, splits, st);
-    return launch_tile<T, 2, 2, 2, 2>(g, trans_a != 0, trans_b != 0, st);
+    return plan.shape == kStaged ? launch_staged<T>(g, trans_a != 0, trans_b != 0, current_stream())
+                                 : launch_direct<T>(g, trans_a != 0, trans_b != 0, plan, current_stream());
 }
 
 template <typename T>
