@@ -338,6 +338,13 @@ int vtl_hip_gemm_tile_choice(int M, int N, int K, int requant, int *config_index
  * elements at even strides and the last one, and the count.  The check that the layers make
  * before they use the codes of frozen parameters again. */
 int vtl_hip_content_fingerprint(const void *data, int64_t count, int element_bytes, uint64_t *out);
+/* 1 when each of `count` host tensors still has the fingerprint noted beside it, else 0 (not a status). */
+typedef struct {
+    const void *data;
+    int64_t count, element_bytes;
+    uint64_t fingerprint;
+} vtl_hip_watch;
+int vtl_hip_contents_unchanged(int count, const vtl_hip_watch *watched);
 
 /* The library reads its tuning switches (environment variables VTL_HIP_*, used
  * by tests and tuning runs only) once, at the first call that looks at them;

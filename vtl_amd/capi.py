@@ -31,6 +31,11 @@ class Layer(C.Structure):
                 ("wq", _vp), ("sw", _vp), ("bias", _vp)]
 
 
+class Watch(C.Structure):
+    """`vtl_hip_watch`: a host tensor and the fingerprint that its contents had."""
+    _fields_ = [("data", _vp), ("count", _i64), ("element_bytes", _i64), ("fingerprint", C.c_uint64)]
+
+
 # name -> (restype, argtypes); kept in step with include/vtl_hip.h
 SIGNATURES = {
     "vtl_hip_device_count": (_ci, [C.POINTER(_ci)]),
@@ -90,6 +95,7 @@ SIGNATURES = {
     "vtl_hip_last_error": (C.c_char_p, []),
     "vtl_hip_version": (C.c_char_p, []),
     "vtl_hip_content_fingerprint": (_ci, [_vp, _i64, _ci, C.POINTER(C.c_uint64)]),
+    "vtl_hip_contents_unchanged": (_ci, [_ci, C.POINTER(Watch)]),
     "vtl_hip_reload_env": (_ci, []),
 }
 
@@ -107,6 +113,7 @@ class VtlHipError(RuntimeError):
 
 
 _lib = None
+_functions: dict = {}     # name -> bound entry point, filled by call()
 
 
 def lib() -> C.CDLL:
@@ -127,14 +134,22 @@ def lib() -> C.CDLL:
 
 def call(name: str, *args) -> None:
     """Call an int-returning entry point and raise VtlHipError on failure."""
-    L = lib()
-    st = getattr(L, name)(*args)
+    fn = _functions.get(name)
+    if fn is None:
+        fn = _functions[name] = getattr(lib(), name)
+    st = fn(*args)
     if st != OK:
-        detail = L.vtl_hip_strerror(st).decode()
-        last = L.vtl_hip_last_error().decode()
-        if st in (ERR_RUNTIME, ERR_OUT_OF_MEMORY, ERR_NO_DEVICE) and last:
-            detail += " [" + last + "]"
-        raise VtlHipError(name, st, detail)
+        failed(name, st)
+
+
+def failed(name: str, st: int) -> None:
+    """Raise the VtlHipError of a call that returned `st`."""
+    L = lib()
+    detail = L.vtl_hip_strerror(st).decode()
+    last = L.vtl_hip_last_error().decode()
+    if st in (ERR_RUNTIME, ERR_OUT_OF_MEMORY, ERR_NO_DEVICE) and last:
+        detail += " [" + last + "]"
+    raise VtlHipError(name, st, detail)
 
 
 def status(name: str, *args) -> int:

@@ -455,6 +455,17 @@ int vtl_hip_content_fingerprint(const void *data, int64_t count, int element_byt
     return VTL_HIP_OK;
 }
 
+int vtl_hip_contents_unchanged(int count, const vtl_hip_watch *watched)
+{
+    for (int i = 0; i < count; i++) {
+        uint64_t h = 0;
+        if (!watched || vtl_hip_content_fingerprint(watched[i].data, watched[i].count, (int)watched[i].element_bytes,
+                                                    &h) != VTL_HIP_OK || h != watched[i].fingerprint)
+            return 0;
+    }
+    return 1;
+}
+
 const char *vtl_hip_version(void) { return "vtlhip 0.1 (gfx950)"; }
 
 }  // extern "C"

@@ -24,7 +24,7 @@ import numpy as np
 
 from . import capi
 from .storage import HipParams, HipStorage, host_array
-from .tensor import (HipTensor, linear_backward_hip, linear_f32_dynquant_hip, linear_hip, linear_i8_hip,
+from .tensor import (HipTensor, _dynquant_workspace, linear_backward_hip, linear_f32_dynquant_hip, linear_hip, linear_i8_hip,
                      matmul_hip)
 
 
@@ -96,7 +96,7 @@ def content_fingerprint(t: np.ndarray) -> int:
     QuantLinearLayer.quantized): an in-place edit of a frozen parameter - a checkpoint
     loaded into the same tensor, a manual `set` - changes it with near certainty when
     the edit touches most elements, as every optimizer step and every load does."""
-    flat = np.ascontiguousarray(t)
+    flat = np.ascontiguousarray(t, None if t.dtype.itemsize in (4, 8) else np.float64)
     h = C.c_uint64()
     capi.call("vtl_hip_content_fingerprint", flat.ctypes.data, flat.size, flat.itemsize, C.byref(h))
     return h.value
@@ -119,8 +119,16 @@ class QuantizedWeights:
         self.source = weights
         self.bias_source = bias
         self.frozen = frozen
+        # What says whether the parameters are as they were: their addresses (both tensors are
+        # held, so they stay), sizes and fingerprints.
+        parts = [t for t in (weights, bias) if t is not None]
+        self._watchable = all(type(t) is np.ndarray and t.flags.c_contiguous and t.itemsize in (4, 8) for t in parts)
         self.fingerprint = content_fingerprint(weights)
         self.bias_fingerprint = None if bias is None else content_fingerprint(np.asarray(bias))
+        if self._watchable:
+            self._watch = (capi.Watch * len(parts))(*[
+                capi.Watch(t.ctypes.data, t.size, t.itemsize, h)
+                for t, h in zip(parts, (self.fingerprint, self.bias_fingerprint))])
         self.out_features, self.in_features = weights.shape
         w_dev = HipTensor.from_host(np.asarray(weights, np.float32), params)
         try:
@@ -136,6 +144,13 @@ class QuantizedWeights:
         self.layer = capi.Layer(capi.LAYER_LINEAR, mode == PER_CHANNEL, self.out_features, self.in_features,
                                 self.w_q.ptr, self.sw.ptr, self.bias.ptr if self.bias is not None else None)
 
+    def unchanged(self) -> bool:
+        """Whether the parameters still have the contents that the codes were made from."""
+        if self._watchable:
+            return capi.lib().vtl_hip_contents_unchanged(len(self._watch), self._watch) == 1
+        return (self.fingerprint == content_fingerprint(self.source) and
+                (self.bias_source is None or self.bias_fingerprint == content_fingerprint(np.asarray(self.bias_source))))
+
     def release(self) -> None:
         self.w_q.release()
         self.sw.release()
@@ -146,7 +161,7 @@ class QuantizedWeights:
 def linear_forward_hip_i8_device(x: HipTensor, qw: QuantizedWeights, relu: bool = False,
                                  session: HipSession | None = None) -> HipTensor:
     """x[M,K] f32 on the device -> y[M,N] f32 on the device."""
-    if not x.is_matrix():
+    if len(x.shape) != 2:
         raise ValueError("Matrix expected")
     if x.shape[1] != qw.in_features:
         raise ValueError(
@@ -154,8 +169,7 @@ def linear_forward_hip_i8_device(x: HipTensor, qw: QuantizedWeights, relu: bool 
     if qw.mode == PER_CHANNEL:
         ws = None
         if session is not None:
-            need = int(capi.lib().vtl_hip_linear_f32_dynquant_workspace(x.shape[0], x.shape[1]))
-            ws = session.ensure("dynquant", need)
+            ws = session.ensure("dynquant", _dynquant_workspace(*x.shape))
         return linear_f32_dynquant_hip(x, qw.w_q, qw.sw, qw.bias, relu=relu, workspace=ws)
     x_q, sx = x.quantize_i8(-1)
     try:
@@ -256,8 +270,7 @@ class QuantLinearLayer:
         frozen = no_grad or not self.requires_grad
         c = self._cache
         fresh = (c is not None and frozen and c.frozen and c.source is self.weights
-                 and c.bias_source is self.bias and c.fingerprint == content_fingerprint(self.weights)
-                 and c.bias_fingerprint == content_fingerprint(self.bias))
+                 and c.bias_source is self.bias and c.unchanged())
         if not fresh:
             if c is not None:
                 c.release()

@@ -23,6 +23,7 @@ class HipParams:
 
 
 _SUPPORTED = (np.float32, np.int8, np.int32, np.float64, np.uint8)
+_DTYPES = {t: np.dtype(t) for t in _SUPPORTED} | {np.dtype(t): np.dtype(t) for t in _SUPPORTED}
 
 
 # Results of more bytes than this are arrays over pinned memory of the library, which the device
@@ -55,6 +56,9 @@ def host_array(count: int, dt: np.dtype):
     return out, out.ctypes.data
 
 
+_PARAMS: dict = {}
+
+
 class HipStorage:
     """`HipStorage[T]{ptr voidptr; size int; count int; device_id int}`."""
 
@@ -69,7 +73,7 @@ class HipStorage:
     @staticmethod
     def empty(count: int, dtype, params: HipParams | None = None) -> "HipStorage":
         device_id = params.device_id if params is not None else 0
-        dt = np.dtype(dtype)
+        dt = _DTYPES.get(dtype) or np.dtype(dtype)
         if dt.type not in _SUPPORTED:
             raise TypeError(f"HipStorage: unsupported element type {dt}")
         count = int(count)
@@ -86,6 +90,14 @@ class HipStorage:
         if st.size:
             capi.call("vtl_hip_upload", st.ptr, flat.ctypes.data, st.size)
         return st
+
+    @property
+    def params(self) -> HipParams:
+        """What makes another storage on the same device."""
+        p = _PARAMS.get(self.device_id)
+        if p is None:
+            p = _PARAMS[self.device_id] = HipParams(self.device_id)
+        return p
 
     def hip(self, params: HipParams | None = None) -> "HipStorage":
         """Identity, for chaining (storage/cuda_d_cuda.v:62-65)."""

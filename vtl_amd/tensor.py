@@ -29,7 +29,7 @@ class HipTensor:
     def __init__(self, data: HipStorage, shape):
         self.data = data
         self.memory = "row_major"
-        self.shape = [int(s) for s in shape]
+        self.shape = list(map(int, shape))
         self.size = math.prod(self.shape)
         self._strides = None       # those of a dense row-major tensor
         if self.size != data.count:
@@ -119,9 +119,9 @@ class HipTensor:
         return self.is_row_major_contiguous() or self.is_col_major_contiguous()
 
     def _assert(self, dtype, matrix=True, what="tensor"):
-        if self.dtype != np.dtype(dtype):
+        if self.data.dtype.type is not dtype:
             raise TypeError(f"{what}: expected {np.dtype(dtype)}, got {self.dtype}")
-        if matrix and not self.is_matrix():
+        if matrix and len(self.shape) != 2:
             raise ValueError(f"{what}: Matrix expected, got shape {self.shape}")
 
     # -- INT8 quantization vocabulary ------------------------------------------
@@ -130,7 +130,7 @@ class HipTensor:
         self._assert(np.float32, what="absmax")
         rows, cols = self.shape
         per_row = _per_row(axis)
-        out = HipTensor.empty([rows if per_row else 1], np.float32, HipParams(self.data.device_id))
+        out = HipTensor.empty([rows if per_row else 1], np.float32, self.data.params)
         capi.call("vtl_hip_absmax_f32", self.ptr, rows, cols, per_row, out.ptr)
         return out
 
@@ -139,7 +139,7 @@ class HipTensor:
         self._assert(np.float32, what="quantize_i8")
         rows, cols = self.shape
         per_row = _per_row(axis)
-        p = HipParams(self.data.device_id)
+        p = self.data.params
         q = HipTensor.empty([rows, cols], np.int8, p)
         s = HipTensor.empty([rows if per_row else 1], np.float32, p)
         capi.call("vtl_hip_quantize_f32_i8", self.ptr, rows, cols, per_row, q.ptr, s.ptr)
@@ -152,7 +152,7 @@ class HipTensor:
         per_row = _per_row(axis)
         if scales.size != (rows if per_row else 1):
             raise ValueError(f"scales: expected {rows if per_row else 1} entries, got {scales.size}")
-        q = HipTensor.empty([rows, cols], np.int8, HipParams(self.data.device_id))
+        q = HipTensor.empty([rows, cols], np.int8, self.data.params)
         capi.call("vtl_hip_quantize_with_scale_f32_i8", self.ptr, scales.ptr, rows, cols, per_row, q.ptr)
         return q
 
@@ -164,7 +164,7 @@ class HipTensor:
         per_row = _per_row(axis)
         if scales.size != (rows if per_row else 1):
             raise ValueError(f"scales: expected {rows if per_row else 1} entries, got {scales.size}")
-        x = HipTensor.empty([rows, cols], np.float32, HipParams(self.data.device_id))
+        x = HipTensor.empty([rows, cols], np.float32, self.data.params)
         capi.call("vtl_hip_dequantize_i8_f32", self.ptr, scales.ptr, rows, cols, per_row, x.ptr)
         return x
 
@@ -176,7 +176,7 @@ class HipTensor:
 
     def relu_hip(self) -> "HipTensor":
         """`relu_hip() !&HipTensor[T]`: a new tensor, as relu_cuda (tensor_cuda_d_cuda.v:205-235)."""
-        out = HipTensor.empty(self.shape, self.dtype, HipParams(self.data.device_id))
+        out = HipTensor.empty(self.shape, self.dtype, self.data.params)
         capi.call("vtl_hip_memcpy_d2d", out.ptr, self.ptr, self.data.size)
         return out.relu_()
 
@@ -184,7 +184,7 @@ class HipTensor:
         """`sigmoid_hip() !&HipTensor[T]`: 1 / (1 + exp(-x)), as sigmoid_cuda
         (tensor_cuda_d_cuda.v:237-270) with the arithmetic of nn/internal/activation.v:35-40."""
         sfx = _float_suffix(self, "sigmoid_hip")
-        out = HipTensor.empty(self.shape, self.dtype, HipParams(self.data.device_id))
+        out = HipTensor.empty(self.shape, self.dtype, self.data.params)
         capi.call(f"vtl_hip_sigmoid_{sfx}", self.ptr, out.ptr, self.size)
         return out
 
@@ -199,12 +199,13 @@ def _per_row(axis: int) -> int:
 
 def _matmul_shapes(a: HipTensor, bt: HipTensor):
     """Shape rule of la.matmul (la/la.v:38-43) for a second operand stored [N,K]."""
-    if not a.is_matrix() or not bt.is_matrix():
+    if len(a.shape) != 2 or len(bt.shape) != 2:
         raise ValueError("Matrix expected")
-    if a.shape[1] != bt.shape[1]:
+    (m, k), (n, k2) = a.shape, bt.shape
+    if k != k2:
         raise ValueError(
             f"Invalid shapes for matrix multiplication {a.shape} and {[bt.shape[1], bt.shape[0]]}")
-    return a.shape[0], bt.shape[0], a.shape[1]
+    return m, n, k
 
 
 def gemm_i8_hip(dst: HipTensor, a: HipTensor, bt: HipTensor) -> None:
@@ -231,7 +232,7 @@ def linear_i8_hip(x_q: HipTensor, sx: HipTensor, w_q: HipTensor, sw: HipTensor,
         raise ValueError("linear_i8_hip: scale sizes do not match the operands")
     if bias is not None and bias.size != N:
         raise ValueError(f"linear_i8_hip: bias has {bias.size} entries, expected {N}")
-    y = HipTensor.empty([M, N], np.float32, HipParams(x_q.data.device_id))
+    y = HipTensor.empty([M, N], np.float32, x_q.data.params)
     capi.call("vtl_hip_linear_i8_f32", x_q.ptr, sx.ptr, int(sx.size == M), w_q.ptr, sw.ptr,
               int(sw.size == N), bias.ptr if bias is not None else None, y.ptr, M, N, K, int(relu))
     return y
@@ -250,7 +251,7 @@ def linear_i8_requant_hip(x_q: HipTensor, sx: HipTensor, w_q: HipTensor, sw: Hip
         raise ValueError("linear_i8_requant_hip: scale sizes do not match the operands")
     if bias is not None and bias.size != N:
         raise ValueError(f"linear_i8_requant_hip: bias has {bias.size} entries, expected {N}")
-    params = HipParams(x_q.data.device_id)
+    params = x_q.data.params
     y_q = HipTensor.empty([M, N], np.int8, params)
     sy = HipTensor.empty([M], np.float32, params)
     y = HipTensor.empty([M, N], np.float32, params) if keep_f32 else None
@@ -258,6 +259,11 @@ def linear_i8_requant_hip(x_q: HipTensor, sx: HipTensor, w_q: HipTensor, sw: Hip
               int(sw.size == N), bias.ptr if bias is not None else None, int(relu), y_q.ptr, sy.ptr,
               y.ptr if y is not None else None, M, N, K)
     return (y_q, sy, y) if keep_f32 else (y_q, sy)
+
+
+def _dynquant_workspace(m: int, k: int) -> int:
+    """vtl_hip_linear_f32_dynquant_workspace: codes and row scales in whole multiples of 256 bytes."""
+    return (m * k + 255 & ~255) + (4 * m + 255 & ~255) if m > 0 and k > 0 else 0
 
 
 def linear_f32_dynquant_hip(x: HipTensor, w_q: HipTensor, sw: HipTensor, bias: HipTensor | None,
@@ -270,10 +276,10 @@ def linear_f32_dynquant_hip(x: HipTensor, w_q: HipTensor, sw: HipTensor, bias: H
         raise ValueError("linear_f32_dynquant_hip: one weight scale per output channel expected")
     if bias is not None and bias.size != N:
         raise ValueError(f"linear_f32_dynquant_hip: bias has {bias.size} entries, expected {N}")
-    need = int(capi.lib().vtl_hip_linear_f32_dynquant_workspace(M, K))
+    need = _dynquant_workspace(M, K)
     own = workspace is None or workspace.size < need
-    ws = HipStorage.empty(need, np.uint8, HipParams(x.data.device_id)) if own else workspace
-    y = HipTensor.empty([M, N], np.float32, HipParams(x.data.device_id))
+    ws = HipStorage.empty(need, np.uint8, x.data.params) if own else workspace
+    y = HipTensor.empty([M, N], np.float32, x.data.params)
     try:
         capi.call("vtl_hip_linear_f32_dynquant", x.ptr, w_q.ptr, sw.ptr,
                   bias.ptr if bias is not None else None, y.ptr, M, N, K, int(relu), ws.ptr, ws.size)
@@ -304,7 +310,7 @@ def matmul_hip(a: HipTensor, b: HipTensor, trans_a: bool = False, trans_b: bool 
     k2, n = (b.shape[1], b.shape[0]) if trans_b else b.shape
     if k != k2:
         raise ValueError(f"Invalid shapes for matrix multiplication {[m, k]} and {[k2, n]}")
-    c = HipTensor.empty([m, n], a.dtype, HipParams(a.data.device_id))
+    c = HipTensor.empty([m, n], a.dtype, a.data.params)
     capi.call(f"vtl_hip_matmul_{sfx}", a.ptr, b.ptr, c.ptr, m, n, k, int(trans_a), int(trans_b))
     return c
 
@@ -318,7 +324,7 @@ def linear_hip(x: HipTensor, w: HipTensor, bias: HipTensor | None, relu: bool = 
     m, n, k = _matmul_shapes(x, w)
     if bias is not None and bias.size != n:
         raise ValueError(f"linear_hip: bias has {bias.size} entries, expected {n}")
-    y = HipTensor.empty([m, n], x.dtype, HipParams(x.data.device_id))
+    y = HipTensor.empty([m, n], x.dtype, x.data.params)
     capi.call(f"vtl_hip_linear_{sfx}", x.ptr, w.ptr, bias.ptr if bias is not None else None, y.ptr,
               m, n, k, int(relu))
     return y
@@ -329,7 +335,7 @@ def colsum_hip(x: HipTensor) -> HipTensor:
     sfx = _float_suffix(x, "colsum_hip")
     if not x.is_matrix():
         raise ValueError("Matrix expected")
-    out = HipTensor.empty([1, x.shape[1]], x.dtype, HipParams(x.data.device_id))
+    out = HipTensor.empty([1, x.shape[1]], x.dtype, x.data.params)
     capi.call(f"vtl_hip_colsum_{sfx}", x.ptr, x.shape[0], x.shape[1], out.ptr)
     return out
 
@@ -347,7 +353,7 @@ def linear_backward_hip(grad: HipTensor, x: HipTensor, w: HipTensor, need_dx: bo
     k = x.shape[1]
     if x.shape != [m, k] or w.shape != [n, k]:
         raise ValueError(f"linear_backward_hip: grad {grad.shape}, input {x.shape}, weight {w.shape}")
-    params = HipParams(grad.data.device_id)
+    params = grad.data.params
     dx = HipTensor.empty([m, k], grad.dtype, params) if need_dx else None
     dw = HipTensor.empty([n, k], grad.dtype, params) if need_dw else None
     db = HipTensor.empty([1, n], grad.dtype, params) if need_db else None
