@@ -11,9 +11,12 @@ namespace vtlhip {
 // Stream every compute entry point enqueues on (nullptr = the null stream).
 hipStream_t current_stream();
 
-// True while no thread has named a stream of its own with vtl_hip_set_stream: all of the
-// library's work is on the null stream and therefore in one order.
+// True while no thread has named a stream of its own with vtl_hip_set_stream and memory of one
+// device only has been asked for: all of the library's work is on one null stream and therefore in one order.
 bool single_stream();
+
+// Called with the device that memory is asked for on.
+void note_device(int dev);
 
 // Whether `st` is being captured into a graph (true also when that cannot be found out).
 bool stream_is_capturing(hipStream_t st);

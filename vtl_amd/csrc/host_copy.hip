@@ -11,6 +11,7 @@
 #include <atomic>
 #include <condition_variable>
 #include <deque>
+#include <exception>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -421,8 +422,11 @@ struct Crew {
                 started = true;
                 cpu_set_t cpus;
                 const int have = sched_getaffinity(0, sizeof cpus, &cpus) == 0 ? CPU_COUNT(&cpus) : 1;
-                for (int i = 0; i < (have > 4 ? 3 : have - 1); i++)
-                    std::thread([this] { help(); }).detach();
+                try {
+                    for (int i = 0; i < (have > 4 ? 3 : have - 1); i++)
+                        std::thread([this] { help(); }).detach();
+                } catch (const std::exception &) {   // no more threads to be had: the callers copy alone
+                }
             }
         }
         wake.notify_all();
@@ -437,8 +441,14 @@ struct Crew {
         left.store((int)((bytes + kJobBytes - 1) / kJobBytes), std::memory_order_relaxed);
         std::lock_guard<std::mutex> hold(lock);
         for (size_t at = 0; at < bytes; at += kJobBytes) {
-            queue.push_back({dst + at, src + at, bytes - at < kJobBytes ? bytes - at : kJobBytes, &left});
-            queued++;
+            const size_t take = bytes - at < kJobBytes ? bytes - at : kJobBytes;
+            try {
+                queue.push_back({dst + at, src + at, take, &left});
+                queued++;
+            } catch (const std::exception &) {
+                memcpy(dst + at, src + at, take);
+                left.fetch_sub(1, std::memory_order_release);
+            }
         }
     }
     bool work()
@@ -648,7 +658,7 @@ HostInput::~HostInput()
 
 // The lock of the ring is held until then, so that no other transfer closes the slot before.
 bool HostInput::stage(const void *src, size_t bytes)
-{
+try {
     if (!single_stream() || bytes > kSmall)
         return false;
     Ring *r = ring_of_current_device();
@@ -663,6 +673,8 @@ bool HostInput::stage(const void *src, size_t bytes)
     ring_ = r;
     data = staged;
     return true;
+} catch (const std::exception &) {
+    return false;
 }
 
 void trim_pinned_pool()
@@ -688,7 +700,7 @@ using namespace vtlhip;
 extern "C" {
 
 int vtl_hip_host_alloc(void **hptr, size_t bytes)
-{
+try {
     if (!hptr || bytes == 0)
         return VTL_HIP_ERR_INVALID_ARG;
     *hptr = nullptr;
@@ -717,10 +729,19 @@ int vtl_hip_host_alloc(void **hptr, size_t bytes)
     }
     p.live[reinterpret_cast<uintptr_t>(*hptr)] = cls;
     return VTL_HIP_OK;
+} catch (const std::exception &) {
+    if (*hptr) {
+        PinnedPool &p = pinned_pool();
+        std::lock_guard<std::mutex> hold(p.lock);
+        p.live_bytes -= size_class(bytes < 4096 ? 4096 : bytes);
+        (void)hipHostFree(*hptr);
+        *hptr = nullptr;
+    }
+    return VTL_HIP_ERR_OUT_OF_MEMORY;
 }
 
 int vtl_hip_host_free(void *hptr)
-{
+try {
     if (!hptr)
         return VTL_HIP_OK;
     PinnedPool &p = pinned_pool();
@@ -740,10 +761,12 @@ int vtl_hip_host_free(void *hptr)
     }
     VTL_HIP_TRY(hipHostFree(hptr));
     return VTL_HIP_OK;
+} catch (const std::exception &) {
+    return VTL_HIP_ERR_OUT_OF_MEMORY;
 }
 
 int vtl_hip_upload(void *dst_device, const void *src_host, size_t bytes)
-{
+try {
     if (bytes == 0)
         return VTL_HIP_OK;
     if (!dst_device || !src_host)
@@ -767,10 +790,12 @@ int vtl_hip_upload(void *dst_device, const void *src_host, size_t bytes)
     VTL_HIP_TRY(hipMemcpyAsync(dst_device, src_host, bytes, hipMemcpyHostToDevice, st));
     VTL_HIP_TRY(hipStreamSynchronize(st));
     return VTL_HIP_OK;
+} catch (const std::exception &) {
+    return VTL_HIP_ERR_OUT_OF_MEMORY;
 }
 
 int vtl_hip_memcpy_h2d(void *dst_device, const void *src_host, size_t bytes)
-{
+try {
     if (bytes == 0)
         return VTL_HIP_OK;
     if (!dst_device || !src_host)
@@ -796,10 +821,12 @@ int vtl_hip_memcpy_h2d(void *dst_device, const void *src_host, size_t bytes)
     if (rc == VTL_HIP_OK)
         return_lane(lane);
     return rc;
+} catch (const std::exception &) {
+    return VTL_HIP_ERR_OUT_OF_MEMORY;
 }
 
 int vtl_hip_download(int count, void *const *dst_host, const void *const *src_device, const size_t *bytes)
-{
+try {
     if (count < 0 || (count > 0 && (!dst_host || !src_device || !bytes)))
         return VTL_HIP_ERR_INVALID_ARG;
     bool any = false;
@@ -876,6 +903,8 @@ int vtl_hip_download(int count, void *const *dst_host, const void *const *src_de
             return_lane(lane);   // after a failure its counter and flag are unknown: it is left alone
     }
     return rc;
+} catch (const std::exception &) {
+    return VTL_HIP_ERR_OUT_OF_MEMORY;
 }
 
 int vtl_hip_memcpy_d2h(void *dst_host, const void *src_device, size_t bytes)

@@ -4,6 +4,7 @@
 // waits for the device whatever the size (9 us behind the smallest launch), and two 1 GiB
 // results taken in turn cost tens of milliseconds a call: more than the kernels that fill
 // them.  So released blocks are kept and handed out again.
+#include <exception>
 #include <map>
 #include <mutex>
 #include <unordered_map>
@@ -37,7 +38,7 @@ size_t size_class(size_t bytes)
 namespace {
 
 // Released blocks are kept per device and size class.  No wait is needed
-// while every call of the process has used the null stream (single_stream()): whatever still
+// while every call of the process has used the null stream of one device (single_stream()): whatever still
 // reads or writes a released block was enqueued before the release, and whoever gets the
 // block next enqueues behind it.  Once a program has named a stream of its own, a release waits
 // for the device first, as hipFree does, so that a block in the pool is idle on every stream.
@@ -115,7 +116,10 @@ hipError_t malloc_or_trim(void **ptr, size_t bytes)
     hipError_t e = hipMalloc(ptr, bytes);
     if (e != hipSuccess) {
         (void)hipGetLastError();
-        trim_device_pool();
+        try {
+            trim_device_pool();
+        } catch (const std::exception &) {
+        }
         e = hipMalloc(ptr, bytes);
     }
     return e;
@@ -128,12 +132,13 @@ using namespace vtlhip;
 extern "C" {
 
 int vtl_hip_malloc(void **dptr, size_t bytes)
-{
+try {
     if (!dptr || bytes == 0)
         return VTL_HIP_ERR_INVALID_ARG;
     *dptr = nullptr;
     int dev = 0;
     VTL_HIP_TRY(hipGetDevice(&dev));
+    note_device(dev);
     DevicePool &p = device_pool();
     const bool pooled = bytes <= kPooledBlockMost && (single_stream() || !stream_is_capturing(current_stream()));
     const size_t cls = pooled ? size_class(bytes) : bytes;
@@ -167,6 +172,11 @@ int vtl_hip_malloc(void **dptr, size_t bytes)
     rec.device = dev;
     rec.live = true;
     return VTL_HIP_OK;
+} catch (const std::exception &) {   // the pool's own bookkeeping found no host memory
+    if (*dptr)
+        (void)hipFree(*dptr);
+    *dptr = nullptr;
+    return VTL_HIP_ERR_OUT_OF_MEMORY;
 }
 
 int vtl_hip_malloc_on(int device_id, void **dptr, size_t bytes)
@@ -179,7 +189,7 @@ int vtl_hip_malloc_on(int device_id, void **dptr, size_t bytes)
 }
 
 int vtl_hip_free(void *dptr)
-{
+try {
     if (!dptr)
         return VTL_HIP_OK;  // CudaStorage.release() skips nil too
     DevicePool &p = device_pool();
@@ -214,10 +224,10 @@ int vtl_hip_free(void *dptr)
             return record_hip_error(hipErrorInvalidValue, "vtl_hip_free of released memory");
         if (pooled) {
             Block &rec = it->second;
+            p.free_list[{rec.device, rec.bytes}].push_back(dptr);
             rec.live = false;
             rec.idle = idle;
             rec.stamp = ++p.clock;
-            p.free_list[{rec.device, rec.bytes}].push_back(dptr);
             p.idle_bytes += rec.bytes;
             if (p.idle_bytes > kIdleBytesMost)
                 take_oldest(p, kIdleBytesMost, out);
@@ -230,13 +240,17 @@ int vtl_hip_free(void *dptr)
     for (void *b : out)
         VTL_HIP_TRY(hipFree(b));
     return VTL_HIP_OK;
+} catch (const std::exception &) {
+    return VTL_HIP_ERR_OUT_OF_MEMORY;
 }
 
 int vtl_hip_trim(void)
-{
+try {
     trim_device_pool();
     trim_pinned_pool();
     return VTL_HIP_OK;
+} catch (const std::exception &) {
+    return VTL_HIP_ERR_OUT_OF_MEMORY;
 }
 
 }  // extern "C"

@@ -16,12 +16,20 @@ namespace vtlhip {
 static thread_local hipStream_t g_stream = nullptr;
 static thread_local char g_last_error[256] = "";
 
-// Whether every call so far used the null stream (memory.hip).
+// Whether every call so far used the null stream of one device (memory.hip).
 static std::atomic<bool> g_single_stream{true};
 
 hipStream_t current_stream() { return g_stream; }
 
 bool single_stream() { return g_single_stream.load(std::memory_order_acquire); }
+
+void note_device(int dev)
+{
+    static std::atomic<int> first{-1};
+    int seen = -1;
+    if (!first.compare_exchange_strong(seen, dev) && seen != dev && single_stream())
+        g_single_stream.store(false, std::memory_order_release);
+}
 
 int record_hip_error(hipError_t e, const char *what)
 {
