@@ -256,6 +256,34 @@ def test_whole_tensor_quantize_in_two_launches_equals_four(hip, shape, knobs):
         h.release()
 
 
+@pytest.mark.parametrize("n", [4, 4095, 4096, 4097, 16381, 16384, 16385, 65536, 65537, 256 * 4096 - 3, 256 * 4096 + 1,
+                               2 * 256 * 4096 + 3, 8 * 256 * 4096 + 4, 12 * 256 * 4096 + 2, (1 << 24) - 1, 1 << 24,
+                               (1 << 24) + 3, (1 << 24) + 4])
+def test_whole_tensor_quantize_in_one_launch(hip, knobs, n):
+    """Sizes around those where a further workgroup or a further vector per thread comes in and where the
+    registers end; the maximum in the first element, the last, and in between; a wait that gives up
+    at once.  Whole numbers: equal to the oracle."""
+    rng = np.random.Generator(np.random.Philox(n))
+    base = rng.standard_normal(n, dtype=np.float32)
+    X, Q, S = raw_device_buffer(4 * n), raw_device_buffer(n + 16), raw_device_buffer(64)
+    knobs.setenv("VTL_HIP_QUANT_GROUPS", str(1 << 20))   # also after tests that used streams of their own
+    for at, spin in ((0, None), (n - 1, None), (n // 2, None), (n - 1, "0")):
+        if spin is not None:
+            knobs.setenv("VTL_HIP_STAGE_SPIN", spin)
+        x = base.copy()
+        x[at] = -9.0 if at else 7.5
+        h2d(X.ptr, x)
+        want_q, want_s = oracle.quantize(x.reshape(1, n), False, threads=CPU_THREADS)
+        capi.call("vtl_hip_memset", Q.ptr, 0xA5, n + 16)
+        capi.call("vtl_hip_quantize_f32_i8", X.ptr, 1, n, 0, Q.ptr, S.ptr)
+        assert d2h(S.ptr, 1, np.float32).view(np.uint32)[0] == want_s.view(np.uint32).reshape(-1)[0], (at, spin)
+        got = d2h(Q.ptr, n + 16, np.int8)
+        assert np.array_equal(got[:n], want_q.reshape(-1)), (at, spin)
+        assert (got[n:].view(np.uint8) == 0xA5).all()
+    for h in (X, Q, S):
+        h.release()
+
+
 def test_whole_tensor_quantize_on_many_streams(hip):
     """Every stream has absmax cells of its own (the first 16 streams that ask; further ones
     take the four-launch form): calls enqueued on 20 streams without waiting in between, three

@@ -108,6 +108,7 @@ struct Tuning {
     bool no_fused_requant = false;  // VTL_HIP_NO_FUSED_REQUANT: linear, then the row quantizer
     int requant_wide = 0;           // VTL_HIP_REQUANT_WIDE: 1 row maxima in the tile kernel + wide quantizer, 0 one workgroup per row
     bool quant_four_launches = false;  // VTL_HIP_QUANT_FOUR_LAUNCHES: whole-tensor quantize as clear + absmax + scale + quantize (tests)
+    int quant_groups = 0;           // VTL_HIP_QUANT_GROUPS: workgroups of a whole-tensor quantize launch whatever streams there are (tests)
     bool no_fused_decode = false;   // VTL_HIP_NO_FUSED_DECODE: quantizer launch in front of the linear
     int stage_spin = 4096;          // VTL_HIP_STAGE_SPIN: polls a workgroup of the decode launch waits for the quantized rows (0: none, tests)
     int stream_weights_mib = 48;    // VTL_HIP_STREAM_WEIGHTS_MIB: weight matrices of this many MiB and more are read with non-temporal loads by the kernels for 2 to 32 rows (0: always)

@@ -12,6 +12,7 @@
 // The division is the correctly rounded one.  The quotient is first estimated
 // with x * (1/scale); only when that estimate is too close to a rounding tie
 // to decide the integer is the exact division evaluated (see quant_code).
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -184,6 +185,103 @@ __global__ __launch_bounds__(64) void absmax_cells_reduce_kernel(unsigned *cells
     cells[threadIdx.x * kCellStride] = 0u;
     if (threadIdx.x == 0)
         *out = m;
+}
+
+// ---- whole-tensor quantize in one launch ------------------------------------
+
+// Bound by reading the tensor once: every workgroup keeps its share in registers (the chip's hold
+// 64 MiB of it beside their working set) while the workgroups exchange their maxima, so nothing is
+// read again and there is no second launch.  Whole calls against an absmax launch and a quantize launch:
+// 1000 x 1000 6.2 instead of 6.9 us, 3001 x 2049 10.7 instead of 13.5, 3001 x 4099 15.7 instead of
+// 18.7 (3.9 TB/s), 4096 x 4096 20.8 instead of 24.8; against one workgroup that holds the whole tensor,
+// 64 x 784 4.0 instead of 7.0.
+//
+// The exchange: workgroup b stores its maximum together with the call's number as one 8-byte word
+// to part[b], with a device-scope store that goes through to memory, and reads all words until each
+// carries the number; nothing is cleared and no fence is needed, because a word is its own
+// message.  The wait is bounded: after spin_limit polls a workgroup takes the maximum of the whole tensor
+// itself and goes on, so the launch drains whatever else keeps its other workgroups from starting.
+// Calls that share `part` must not overlap and carry different numbers.
+constexpr int kExchangeMost = 256;
+
+template <int T, int NV, bool NT>
+__global__ __launch_bounds__(T) void quantize_tensor_kernel(const float *__restrict__ x, int64_t n, unsigned share,
+                                                            int8_t *__restrict__ q, float *__restrict__ scale_out,
+                                                            unsigned long long *part, unsigned number, int spin_limit)
+{
+    static_assert(T >= kExchangeMost, "one thread per word");
+    __shared__ float smem[T / 64], smem_all[T / 64];
+    __shared__ int gave_up;
+    const float4_t *xv = reinterpret_cast<const float4_t *>(x);
+    unsigned *qv = reinterpret_cast<unsigned *>(q);
+    const int64_t nv = n >> 2;
+    const int64_t base = (int64_t)blockIdx.x * share;
+    const int mine = (int)(nv - base < (int64_t)share ? nv - base : (int64_t)share);   // vectors of this workgroup
+    const int tail = blockIdx.x == gridDim.x - 1 ? (int)(n & 3) : 0;
+
+    float4_t v[NV];
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int idx = i * T + (int)threadIdx.x;
+        if (idx < mine)
+            v[i] = NT ? __builtin_nontemporal_load(xv + base + idx) : xv[base + idx];
+        else
+            v[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    const float last = (int)threadIdx.x < tail ? x[(nv << 2) + threadIdx.x] : 0.0f;
+    float m = fmaxf(0.0f, fabsf(last));
+#pragma unroll
+    for (int i = 0; i < NV; i++)
+        m = absmax4(m, v[i]);
+    m = block_max<T>(m, smem);
+
+    if (gridDim.x > 1) {
+        if (threadIdx.x == 0) {
+            gave_up = 0;
+            __hip_atomic_store(part + blockIdx.x, ((unsigned long long)number << 32) | __float_as_uint(m),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        float other = 0.0f;
+        if (threadIdx.x < gridDim.x) {
+            unsigned long long w = 0;
+            bool here = false;
+            for (int spin = 0; spin < spin_limit && !here; spin++) {
+                w = __hip_atomic_load(part + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                here = (unsigned)(w >> 32) == number;
+            }
+            if (here)
+                other = __uint_as_float((unsigned)w);
+            else
+                gave_up = 1;
+        }
+        m = block_max<T>(other, smem_all);
+        if (gave_up) {   // the same for every thread: written before block_max's barrier
+            float all = 0.0f;
+            for (int64_t i = threadIdx.x; i < nv; i += T)
+                all = absmax4(all, xv[i]);
+            if (threadIdx.x < (n & 3))
+                all = fmaxf(all, fabsf(x[(nv << 2) + threadIdx.x]));
+            m = block_max<T>(all, smem);
+        }
+    }
+
+    const float scale = m / 127.0f;
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        *scale_out = scale;
+    const QuantScale p = make_quant_scale(scale);
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int idx = i * T + (int)threadIdx.x;
+        if (idx < mine) {
+            if (NT)
+                __builtin_nontemporal_store(quant4(v[i], p), qv + base + idx);
+            else
+                qv[base + idx] = quant4(v[i], p);
+        }
+    }
+    if ((int)threadIdx.x < tail)
+        q[(nv << 2) + threadIdx.x] = (int8_t)quant_code(last, p);
 }
 
 // ---- fused per-row absmax + quantize ---------------------------------------
@@ -609,9 +707,14 @@ int check_2d(const void *a, const void *b, int64_t rows, int64_t cols)
 // then goes back to the forms that use the caller's memory only, for good.
 constexpr int kCellSet = kAbsmaxCells * kCellStride;
 __device__ unsigned g_absmax_cells[vtlhip::kStreamSlots * 2 * kCellSet];
+// ... and the words that quantize_tensor_kernel's workgroups exchange, numbered call by call.
+__device__ unsigned long long g_exchange[vtlhip::kStreamSlots * kExchangeMost];
 
 struct AbsmaxCells {
     std::mutex lock;
+    std::atomic<unsigned long long *> exchange{nullptr};
+    unsigned number[vtlhip::kStreamSlots] = {};
+    std::atomic<int> compute_units{0};
     std::atomic<unsigned *> base{nullptr};   // device address of this device's g_absmax_cells
     unsigned char turn[vtlhip::kStreamSlots] = {};
     bool unusable[vtlhip::kStreamSlots] = {};
@@ -627,11 +730,16 @@ AbsmaxCells *absmax_cells_of_device()
     }
     AbsmaxCells &c = cells[dev];
     if (!c.base.load(std::memory_order_acquire)) {
-        void *ptr = nullptr;
-        if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(g_absmax_cells)) != hipSuccess) {
+        void *ptr = nullptr, *words = nullptr;
+        int cus = 0;
+        if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(g_absmax_cells)) != hipSuccess ||
+            hipGetSymbolAddress(&words, HIP_SYMBOL(g_exchange)) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
             (void)hipGetLastError();
             return nullptr;
         }
+        c.exchange.store(static_cast<unsigned long long *>(words), std::memory_order_relaxed);
+        c.compute_units.store(cus, std::memory_order_relaxed);
         c.base.store(static_cast<unsigned *>(ptr), std::memory_order_release);
     }
     return &c;
@@ -686,6 +794,67 @@ int launch_absmax_flat(const float *x, int64_t n, unsigned *cell, hipStream_t s)
                            cell, 1);
     }
     return check_launch("absmax_flat_kernel");
+}
+
+// Whole-tensor quantization in one launch, `groups` workgroups of at most kTensorVecs vectors each.
+constexpr int kTensorThreads = 1024;
+constexpr int64_t kTensorVecs = 16 * kTensorThreads;
+
+int launch_quantize_tensor(const float *x, int64_t n, int groups, int8_t *q, float *scale_out,
+                           unsigned long long *part, unsigned number, hipStream_t s)
+{
+    const int64_t nv = n >> 2;
+    const unsigned share = (unsigned)((nv + groups - 1) / groups);
+#define VTL_Q_TENSOR(NV, NT)                                                                                    \
+    hipLaunchKernelGGL((quantize_tensor_kernel<kTensorThreads, NV, NT>), dim3((unsigned)groups),                \
+                       dim3(kTensorThreads), 0, s, x, n, share, q, scale_out, part, number, tuning().stage_spin)
+    if (share <= 1 * kTensorThreads)
+        VTL_Q_TENSOR(1, false);
+    else if (share <= 2 * kTensorThreads)
+        VTL_Q_TENSOR(2, false);
+    else if (share <= 4 * kTensorThreads)
+        VTL_Q_TENSOR(4, false);
+    else if (share <= 8 * kTensorThreads)
+        VTL_Q_TENSOR(8, true);
+    else if (share <= 12 * kTensorThreads)
+        VTL_Q_TENSOR(12, true);
+    else
+        VTL_Q_TENSOR(16, true);
+#undef VTL_Q_TENSOR
+    return check_launch("quantize_tensor_kernel");
+}
+
+// False when the one-launch form does not take the call: tensors beyond the registers, memory that is not
+// aligned for 16-byte loads and 4-byte stores, streams without a number of their own (stream_slot), and, in
+// a program with several streams, more workgroups than those of all its streams together find room
+// for: launches side by side could each hold what the other's last workgroups wait for, until they give up.
+bool quantize_tensor(const float *x, int64_t n, int8_t *q, float *scale_out, hipStream_t s, int &status)
+{
+    if (n < 4 || !aligned(x, 16) || !aligned(q, 4) || tuning().quant_four_launches)
+        return false;
+    const int64_t nv = n >> 2;
+    int64_t groups = (nv + kTensorThreads - 1) / kTensorThreads;
+    if (groups == 1) {
+        status = launch_quantize_tensor(x, n, 1, q, scale_out, nullptr, 0, s);
+        return true;
+    }
+    const int slot = vtlhip::stream_slot(s);
+    AbsmaxCells *c = slot >= 0 ? absmax_cells_of_device() : nullptr;
+    if (!c)
+        return false;
+    const int64_t most = std::min(kExchangeMost, c->compute_units.load(std::memory_order_relaxed));
+    if (groups > tuning().quant_groups && !single_stream() && groups > most / 8)
+        return false;
+    groups = std::min(groups, most);
+    if (nv > groups * kTensorVecs)
+        return false;
+    std::lock_guard<std::mutex> hold(c->lock);
+    if (++c->number[slot] == 0)   // 0: what the words hold at first
+        c->number[slot] = 1;
+    status = launch_quantize_tensor(x, n, (int)groups, q, scale_out,
+                                    c->exchange.load(std::memory_order_relaxed) + slot * kExchangeMost,
+                                    c->number[slot], s);
+    return true;
 }
 
 int launch_fill_zero(float *p, int64_t n, hipStream_t st);
@@ -953,13 +1122,18 @@ int vtl_hip_quantize_f32_i8(const float *x, int64_t rows, int64_t cols, int per_
     }
     if (per_row)
         return launch_quantize_rows(x, rows, cols, q, scale_out, s);
-    // a small tensor is one "row" of the fused kernel: a single workgroup holds it
-    // in registers between the absmax and the rounding pass, one launch instead of four
+    // A small tensor is one "row" of the fused kernel: a single workgroup holds it in registers between
+    // the absmax and the rounding pass.  Up to 16384 elements: there the exchange between
+    // workgroups costs as much as it saves (64 x 256: 3.8 against 4.0 us, 64 x 784: 7.0 against 4.0).
     const int64_t total = rows * cols;
-    if (total > 0 && total <= 4 * 1024 * 16 && total % 4 == 0 && aligned(x, 16) && aligned(q, 4))
+    if (total > 0 && total <= 4 * 1024 * 4 && total % 4 == 0 && aligned(x, 16) && aligned(q, 4))
         return launch_quantize_rows(x, 1, total, q, scale_out, s);
+    if (quantize_tensor(x, total, q, scale_out, s, st))
+        return st;
+    if (total > 0 && total <= 4 * 1024 * 16 && total % 4 == 0 && aligned(x, 16) && aligned(q, 4))
+        return launch_quantize_rows(x, 1, total, q, scale_out, s);   // (under capture: no number for the exchange)
     if (total > 0 && total <= ((int64_t)1 << 24)) {
-        // whole tensor in two launches: absmax into one of the stream's two sets of cells, then
+        // Unaligned memory, or several streams: two launches, absmax into one of the stream's two sets of cells, then
         // the quantize pass, whose workgroups derive the scale from them (1024 x 1024: 6.0
         // against 10.8 us for the four launches below, 4096 x 4096: 24.6 against 32.6 us).  Up
         // to 16 M elements: beyond, reading the cells in every workgroup costs more than the two

@@ -83,6 +83,7 @@ static const Tuning *read_tuning(bool force)
     t->no_fused_requant = flag("VTL_HIP_NO_FUSED_REQUANT");
     t->requant_wide = number("VTL_HIP_REQUANT_WIDE", 0);
     t->quant_four_launches = flag("VTL_HIP_QUANT_FOUR_LAUNCHES");
+    t->quant_groups = number("VTL_HIP_QUANT_GROUPS", 0);
     t->no_fused_decode = flag("VTL_HIP_NO_FUSED_DECODE");
     t->stage_spin = number("VTL_HIP_STAGE_SPIN", 4096);
     if (t->stage_spin < 0 || t->stage_spin > (1 << 20))
