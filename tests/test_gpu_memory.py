@@ -98,9 +98,9 @@ def test_memory_comes_round_again_on_the_null_stream(hip):
     assert res.returncode == 0 and res.stdout.strip().endswith("done"), res.stderr[-2000:]
 
 
-# bytes: single ones, around a vector, where staging ends and chunks begin (1 MiB), where a chunk is
+# bytes: single ones, around a vector, where a small upload becomes two pieces (384 KiB), where staging ends and chunks begin (1 MiB), where a chunk is
 # a whole slot (16 MiB and more), once round the ring of 8 slots of 4 MiB and a remainder
-@pytest.mark.parametrize("nbytes", [1, 15, 16, 17, 4096, 131072, 131073, (1 << 20) - 1, 1 << 20, (1 << 20) + 1,
+@pytest.mark.parametrize("nbytes", [1, 15, 16, 17, 4096, 131072, 131073, (384 << 10) - 1, 384 << 10, 700001, (1 << 20) - 1, 1 << 20, (1 << 20) + 1,
                                     (4 << 20) + 3, (16 << 20) + 4097, (36 << 20) + 13])
 @pytest.mark.parametrize("offset", [0, 5])
 def test_copies_to_and_from_the_device(hip, nbytes, offset):

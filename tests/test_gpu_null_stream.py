@@ -1,0 +1,55 @@
+"""What the library does only while a process uses the null stream alone, checked in a process of its
+own: other tests of this run name streams, and from then on those paths are off."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PROGRAM = r"""
+import os
+os.environ["VTL_USE_HIP"] = os.environ["VTL_HIP_BACKWARD"] = "1"
+import numpy as np
+import oracle
+from vtl_amd import PER_TENSOR, QuantLinearLayer, linear_backward_hip_f32
+rng = np.random.default_rng(7)
+# Linear backward, host to host: gradients below and above the size from which the device writes them
+# itself while the weights are still on their way up, weights in one piece, in several, in chunks
+for m, n, k, dt in ((5, 33, 17, np.float32), (64, 256, 784, np.float32), (16, 1023, 401, np.float64),
+                    (31, 700, 1301, np.float32), (48, 130, 1, np.float32)):
+    for turn in range(3):
+        g, x, w = (rng.standard_normal(s).astype(dt) for s in ((m, n), (m, k), (n, k)))
+        got = linear_backward_hip_f32(g, x, w, True)
+        eps = np.finfo(dt).eps
+        g64, x64, w64 = g.astype(np.float64), x.astype(np.float64), w.astype(np.float64)
+        for out, want, size in ((got[0], g64 @ w64, abs(g64) @ abs(w64)), (got[1], g64.T @ x64, abs(g64).T @ abs(x64)),
+                                (got[2], g64.sum(0)[None], abs(g64).sum(0)[None])):
+            # one rounding to the type, and sums of up to max(m, n) f64 products in two orders
+            bound = eps * abs(want) + 2 * max(m, n) * np.finfo(np.float64).eps * size
+            assert (abs(out - want) <= bound).all(), (m, n, k, dt, turn)
+    print("backward", m, n, k, np.dtype(dt).name, "ok", flush=True)
+# one scale for x, read over the link by the quantizer (up to 65536 elements) or uploaded
+for m, k in ((1, 16), (64, 784), (3, 21845), (70, 1000)):
+    w = rng.standard_normal((40, k), dtype=np.float32)
+    layer = QuantLinearLayer(w, mode=PER_TENSOR)
+    for turn in range(3):
+        x = rng.standard_normal((m, k), dtype=np.float32)
+        xq, sx = oracle.quantize(x, False)
+        wq, sw = oracle.quantize(w, False)
+        acc = xq.astype(np.int64) @ wq.astype(np.int64).T
+        want = acc.astype(np.float32) * (sx.reshape(()) * sw.reshape(())) + np.float32(0)
+        assert np.array_equal(layer.forward(x), want), (m, k, turn)
+    layer.release()
+    print("layer", m, k, "ok", flush=True)
+"""
+
+
+def test_paths_of_a_program_without_streams(hip):
+    done = subprocess.run([sys.executable, "-c", PROGRAM], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                          text=True, timeout=100)
+    assert done.returncode == 0, done.stdout[-2000:]
+    assert done.stdout.count("ok") == 9, done.stdout[-2000:]
