@@ -80,11 +80,15 @@ struct CopyArgs {
     unsigned target;     // what it reads when all of this launch have
     unsigned *flag;      // nullptr: no signal
     unsigned value;
+    unsigned *behind;    // flag of the launch before this one, which has ended by now, or nullptr
+    unsigned behind_value;
     int to_host;         // the bytes have to be visible to the host when the flag is (else: the source is free)
 };
 
 __global__ __launch_bounds__(512) void host_copy_kernel(const CopyArgs g)
 {
+    if (g.behind && blockIdx.x == 0 && threadIdx.x == 0)
+        __hip_atomic_store(g.behind, g.behind_value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     const size_t first = (size_t)blockIdx.x * 512 + threadIdx.x, step = (size_t)gridDim.x * 512;
     for (int s = 0; s < g.count; s++) {
         const Segment &seg = g.seg[s];
@@ -341,10 +345,47 @@ struct Ring {
     char *at(int i) { return base + (size_t)i * kSlotStride; }
     bool is_free(int i) const { return signal[i].raised(); }
     int wait(int i, hipStream_t st) { return wait_signal(signal[i], st); }
+    // A chunk on its way up, and no launch yet behind it that would raise its slot's flag.
+    int waiting = -1;
+
+    // Chunks on the way up: the next launch on the stream raises the flag of this one, which has ended
+    // when that one begins (counting workgroups and a flag of its own hold a kernel back for
+    // about 1.5 us, on a link that a MiB keeps busy for 18).
+    int launch_up(int i, void *dst, const void *src, size_t bytes, hipStream_t st)
+    {
+        CopyArgs g = {};
+        g.seg[0] = make_segment(dst, src, bytes);
+        g.count = 1;
+        raise_waiting(g);
+        hipLaunchKernelGGL(host_copy_kernel, dim3(copy_blocks(bytes < kSmall ? bytes : kSmall - 1)), dim3(512), 0, st, g);
+        const int rc = check_launch("host_copy_kernel");
+        if (rc == VTL_HIP_OK) {
+            signal[i].value++;
+            waiting = i;
+        }
+        return rc;
+    }
+    void raise_waiting(CopyArgs &g) const
+    {
+        if (waiting >= 0) {
+            g.behind = signal[waiting].flag;
+            g.behind_value = signal[waiting].value;
+        }
+    }
+    // After a failure nothing is under way any more and the host raises the flag.
+    void give_up(hipStream_t st)
+    {
+        (void)hipStreamSynchronize(st);
+        (void)hipGetLastError();
+        if (waiting >= 0)
+            __atomic_store_n(signal[waiting].flag, signal[waiting].value, __ATOMIC_RELEASE);
+        waiting = -1;
+    }
     // Copies with the slot's flag at the end; no bytes: the flag behind the kernels before.
     int launch(int i, void *dst, const void *src, size_t bytes, bool to_host, hipStream_t st)
     {
         CopyArgs g = {};
+        raise_waiting(g);
         if (bytes) {
             g.seg[0] = make_segment(dst, src, bytes);
             g.count = 1;
@@ -353,8 +394,10 @@ struct Ring {
         signal[i].attach(g, blocks, to_host);
         hipLaunchKernelGGL(host_copy_kernel, dim3(blocks), dim3(512), 0, st, g);
         const int rc = check_launch("host_copy_kernel");
-        if (rc == VTL_HIP_OK)
+        if (rc == VTL_HIP_OK) {
             signal[i].launched(blocks);
+            waiting = -1;
+        }
         return rc;
     }
     // Closes the slot that small uploads were filling; the next transfer starts in a slot of its own.
@@ -596,11 +639,16 @@ int upload_large(Ring *r, char *dst, const char *src, size_t bytes, hipStream_t 
         Chunks::Chunk &k = c.chunk[issued];
         crew.finish(k.left);
         const int slot = (s0 + issued) % kSlots;
-        rc = r->launch(slot, dst + k.at, r->at(slot) + skew, k.bytes, false, st);
+        if (issued + 1 < n)
+            rc = r->launch_up(slot, dst + k.at, r->at(slot) + skew, k.bytes, st);
+        else
+            rc = r->launch(slot, dst + k.at, r->at(slot) + skew, k.bytes, false, st);
         issued++;
     }
     for (int i = issued; i < pushed; i++)   // after a failure: nothing may still write to the slots
         crew.finish(c.chunk[i].left);
+    if (rc != VTL_HIP_OK)
+        r->give_up(st);
     crew.end();
     r->slot = (s0 + n) % kSlots;
     return rc;
