@@ -76,9 +76,9 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
     int i = 0;
     if (count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR) {
         // A quantizer in front reads the input once and takes it over the link itself: 64 x 784,
-        // per tensor, 4 us less than behind an upload.  (A tensor of more than 65536 elements is
-        // read twice, and the launches for a few rows read it in every workgroup.)
-        const bool once = layers[0].per_channel ? rows > kFewRows : (int64_t)rows * cols <= 65536;
+        // per tensor, 4 us less than behind an upload.  (The launches for a few rows with a scale each read it in
+        // every workgroup.)
+        const bool once = !layers[0].per_channel || rows > kFewRows;
         HostInput input;
         if (once && input.stage(x_host, in_bytes)) {
             VTL_STEP(codes.take((size_t)rows * (size_t)cols));
