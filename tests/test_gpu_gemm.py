@@ -316,3 +316,19 @@ def test_forced_split_k_is_exact(hip, knobs, k):
     knobs.delenv("VTL_HIP_GEMM_CONFIG")
     for h in (A, B, dsa, dsb, dbias):
         h.release()
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1100, 1001), (3, 700, 2047), (20, 2100, 4081), (33, 300, 4095), (130, 150, 255),
+                                   (64, 520, 8193), (257, 129, 4351)])
+def test_rows_that_are_padded(hip, guard_bands, m, n, k):
+    """K no multiple of 16, around the sizes where a row is padded to whole steps of 256; all operands exact."""
+    rng = np.random.Generator(np.random.Philox(m * 7 + k))
+    a = rng.integers(-127, 128, (m, k)).astype(np.int8)
+    w = rng.integers(-127, 128, (n, k)).astype(np.int8)
+    a[0], w[0] = 127, -127
+    da, dw = HipTensor.from_host(a), HipTensor.from_host(w)
+    c = HipTensor.empty([m, n], np.int32)
+    gemm_i8_hip(c, da, dw)
+    assert np.array_equal(c.cpu(), oracle.gemm_i8_i32(a, w, threads=CPU_THREADS))
+    for t in (da, dw, c):
+        t.release()

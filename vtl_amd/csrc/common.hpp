@@ -96,6 +96,9 @@ struct ScratchArena {
     ScratchArena &operator=(const ScratchArena &) = delete;
 };
 
+// Whether this thread's scratch is the static one just now.
+bool scratch_is_static();
+
 // Tuning and test switches, taken from the environment once (first use) and
 // again only when vtl_hip_reload_env() is called: the dispatch path of a launch
 // reads this struct, never the environment.

@@ -187,6 +187,8 @@ ScratchArena::ScratchArena(void *base_, size_t capacity_) : base(static_cast<cha
 
 ScratchArena::~ScratchArena() { g_arena = nullptr; }
 
+bool scratch_is_static() { return g_arena != nullptr; }
+
 int workspace_status() { return g_workspace_status; }
 
 void *library_workspace(size_t bytes, int slot)
