@@ -136,7 +136,8 @@ int vtl_hip_absmax_f32(const float *x, int64_t rows, int64_t cols, int per_row,
 /* scale = absmax / 127 (f32 division); q = clamp(round_half_even(x / scale),
  * -127, 127) with NaN -> 0 and scale 0 -> all codes 0.  scale_out receives 1
  * (per_row == 0) or `rows` scales.  per_row != 0 is one launch; per_row == 0 is
- * one launch up to 65536 elements, two up to 2^24 (absmax as in
+ * one launch up to 2^24 elements of memory aligned for 16-byte loads (while streams
+ * other than the null stream are in use, up to 131072), else two up to 2^24 (absmax as in
  * vtl_hip_absmax_f32, then a pass that derives the scale from it), four beyond
  * or where vtl_hip_absmax_f32 has no memory of its own for the stream.
  * Replaces divide_scalar (math_op.v:103-111)
@@ -238,7 +239,18 @@ typedef struct {
     const int8_t *wq;
     const float *sw;
     const float *bias;
+    int row_bytes;      /* 0: dense; else the length of wq's rows as vtl_hip_pad_rows_i8 leaves them */
 } vtl_hip_layer;
+
+/* Weights whose row length is no multiple of 16 are copied into padded rows by every call that
+ * multiplies with them.  A program that keeps them does it once: rows of `cols` codes into rows of
+ * vtl_hip_padded_row(cols) bytes (16-byte aligned), zero filled, for vtl_hip_layer. */
+int vtl_hip_padded_row(int cols);
+int vtl_hip_pad_rows_i8(const int8_t *src, int64_t rows, int cols, int8_t *dst);
+
+/* vtl_hip_linear_f32_dynquant with the parameters of a layer (per_channel). */
+int vtl_hip_layer_f32(const vtl_hip_layer *layer, const float *X, float *Y, int M, int relu, void *workspace,
+                      size_t workspace_bytes);
 
 /* Sequential.forward / LinearLayer.forward on a host tensor x[rows, cols]: `layers[0 .. count)` in
  * order, y[rows, out_features of the last linear] on return.  Activations are quantized like the

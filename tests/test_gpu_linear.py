@@ -583,3 +583,39 @@ def test_dynquant_without_caller_workspace(hip, mnk):
         assert np.array_equal(Y.cpu(), want)
     for h in (X, W, SW, B, Y):
         h.release()
+
+
+@pytest.mark.parametrize("m", [1, 2, 8, 33, 130])
+@pytest.mark.parametrize("n,k", [(700, 1001), (300, 4095), (1100, 255), (257, 1030)])
+def test_layers_whose_weights_get_padded_rows(hip, m, n, k):
+    """K no multiple of 16 and enough weights that the layer keeps padded rows: host to host, on the device and in
+    a chain, both granularities, each equal to the oracle on the dense codes."""
+    from vtl_amd import PER_CHANNEL, PER_TENSOR, HipSession, QuantLinearLayer, Sequential
+    rng = np.random.Generator(np.random.Philox(m * 13 + k))
+    x = rng.standard_normal((m, k), dtype=np.float32)
+    w = rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.05)
+    b = rng.standard_normal((1, n), dtype=np.float32)
+    wq, sw = oracle.quantize(w, True)
+    want = oracle.linear_f32_dynquant(x, wq, sw, b.reshape(-1))
+    layer = QuantLinearLayer(w, b, mode=PER_CHANNEL, requires_grad=False)
+    assert (layer.quantized().w_rows is not None) == (n * k >= 1 << 18)
+    assert np.array_equal(layer.forward(x), want)
+    dx = HipTensor.from_host(x)
+    for session in (None, HipSession()):
+        y = layer.forward_device(dx, relu=True, session=session)
+        assert np.array_equal(y.cpu(), np.where(want < 0, np.float32(0), want))
+    layer.release()
+    one = QuantLinearLayer(w, b, mode=PER_TENSOR, requires_grad=False)
+    xq, sx = oracle.quantize(x, False)
+    wq1, sw1 = oracle.quantize(w, False)
+    acc = oracle.gemm_i8_i32(xq, wq1, threads=4).astype(np.float32)
+    assert np.array_equal(one.forward(x), acc * (sx.reshape(()) * sw1.reshape(())) + b)
+    one.release()
+    # a chain: its second layer takes rows of n codes, no multiple of 16 either
+    w2 = rng.standard_normal((1000, n), dtype=np.float32) * np.float32(0.05)
+    net = Sequential().input([k]).linear(n, weights=w, bias=b).relu().linear(1000, weights=w2)
+    w2q, sw2 = oracle.quantize(w2, True)
+    hidden = np.where(want < 0, np.float32(0), want)
+    assert np.array_equal(net.forward(x, no_grad=True),
+                          oracle.linear_f32_dynquant(hidden, w2q, sw2, np.zeros(1000, np.float32)))
+    net.release()

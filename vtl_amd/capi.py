@@ -28,7 +28,7 @@ LAYER_LINEAR, LAYER_RELU = 0, 1
 class Layer(C.Structure):
     """`vtl_hip_layer`: one layer of a stack whose parameters are on the device."""
     _fields_ = [("kind", _ci), ("per_channel", _ci), ("out_features", _ci), ("in_features", _ci),
-                ("wq", _vp), ("sw", _vp), ("bias", _vp)]
+                ("wq", _vp), ("sw", _vp), ("bias", _vp), ("row_bytes", _ci)]
 
 
 class Watch(C.Structure):
@@ -72,6 +72,9 @@ SIGNATURES = {
     "vtl_hip_linear_f32_dynquant_workspace": (_sz, [_ci, _ci]),
     "vtl_hip_linear_f32_dynquant": (_ci, [_vp, _vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci, _vp, _sz]),
     "vtl_hip_linear_f32_dynquant_noalloc": (_ci, [_vp, _vp, _vp, _vp, _vp, _ci, _ci, _ci, _ci]),
+    "vtl_hip_padded_row": (_ci, [_ci]),
+    "vtl_hip_pad_rows_i8": (_ci, [_vp, _i64, _ci, _vp]),
+    "vtl_hip_layer_f32": (_ci, [C.POINTER(Layer), _vp, _vp, _ci, _ci, _vp, _sz]),
     "vtl_hip_forward_i8_host": (_ci, [_vp, _ci, _ci, C.POINTER(Layer), _ci, _vp]),
     "vtl_hip_matmul_host_f32": (_ci, [_vp, _vp, _vp, _ci, _ci, _ci]),
     "vtl_hip_matmul_host_f64": (_ci, [_vp, _vp, _vp, _ci, _ci, _ci]),

@@ -99,6 +99,11 @@ struct ScratchArena {
 // Whether this thread's scratch is the static one just now.
 bool scratch_is_static();
 
+// vtl_hip_linear_i8_f32 and vtl_hip_linear_i8_requant with the parameters of a layer, whose weights may have padded rows.
+int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa, float *Y, int M, int relu);
+int layer_linear_i8_requant(const vtl_hip_layer &l, const int8_t *A, const float *sa, int8_t *Yq, float *sy, int M,
+                            int relu);
+
 // Tuning and test switches, taken from the environment once (first use) and
 // again only when vtl_hip_reload_env() is called: the dispatch path of a launch
 // reads this struct, never the environment.

@@ -2377,9 +2377,88 @@ int check_gemm_args(const void *A, const void *Bt, const void *out, int M, int N
     return VTL_HIP_OK;
 }
 
+// Activation codes [M, K] copied into rows of `row` bytes for weights whose rows are padded to that; nullptr
+// without scratch (workspace_status()) or when the launch fails (status).
+const int8_t *pad_activations(const int8_t *A, int M, int K, int row, int &status)
+{
+    int8_t *ws = static_cast<int8_t *>(vtlhip::library_workspace((size_t)M * (size_t)row, 2));
+    status = ws ? launch_pad_rows(A, M, ws, nullptr, 0, nullptr, K, row, current_stream()) : vtlhip::workspace_status();
+    return status == VTL_HIP_OK ? ws : nullptr;
+}
+
+bool layer_row_fits(const vtl_hip_layer &l)
+{
+    return l.row_bytes == 0 || (l.row_bytes >= l.in_features && l.row_bytes % 16 == 0 && l.row_bytes <= 131072 && aligned16(l.wq));
+}
+
 }  // namespace
 
+namespace vtlhip {
+
+int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa, float *Y, int M, int relu)
+{
+    int st = layer_row_fits(l) && A && M >= 0 ? VTL_HIP_OK : VTL_HIP_ERR_INVALID_ARG;
+    int K = l.in_features;
+    if (st == VTL_HIP_OK && l.row_bytes && M > 0) {
+        A = pad_activations(A, M, K, l.row_bytes, st);
+        K = l.row_bytes;
+    }
+    return st != VTL_HIP_OK ? st : vtl_hip_linear_i8_f32(A, sa, l.per_channel, l.wq, l.sw, l.per_channel, l.bias, Y, M,
+                                                         l.out_features, K, relu);
+}
+
+int layer_linear_i8_requant(const vtl_hip_layer &l, const int8_t *A, const float *sa, int8_t *Yq, float *sy, int M,
+                            int relu)
+{
+    int st = layer_row_fits(l) && A && M >= 0 ? VTL_HIP_OK : VTL_HIP_ERR_INVALID_ARG;
+    int K = l.in_features;
+    if (st == VTL_HIP_OK && l.row_bytes && M > 0) {
+        A = pad_activations(A, M, K, l.row_bytes, st);
+        K = l.row_bytes;
+    }
+    return st != VTL_HIP_OK ? st : vtl_hip_linear_i8_requant(A, sa, 1, l.wq, l.sw, 1, l.bias, relu, Yq, sy, nullptr, M,
+                                                             l.out_features, K);
+}
+
+}  // namespace vtlhip
+
 extern "C" {
+
+int vtl_hip_padded_row(int cols) { return cols <= 0 ? 0 : padded_row(cols); }
+
+int vtl_hip_pad_rows_i8(const int8_t *src, int64_t rows, int cols, int8_t *dst)
+{
+    if (!src || !dst || rows < 0 || cols <= 0 || !aligned16(dst))
+        return VTL_HIP_ERR_INVALID_ARG;
+    return launch_pad_rows(src, rows, dst, nullptr, 0, nullptr, cols, padded_row(cols), current_stream());
+}
+
+int vtl_hip_layer_f32(const vtl_hip_layer *layer, const float *X, float *Y, int M, int relu, void *workspace,
+                      size_t workspace_bytes)
+{
+    if (!layer || layer->kind != VTL_HIP_LAYER_LINEAR || !layer->per_channel || !layer_row_fits(*layer))
+        return VTL_HIP_ERR_INVALID_ARG;
+    const vtl_hip_layer &l = *layer;
+    const int K = l.in_features;
+    if (l.row_bytes == 0 || M <= 0 || l.out_features <= 0 || K <= 0)
+        return vtl_hip_linear_f32_dynquant(X, l.wq, l.sw, l.bias, Y, M, l.out_features, K, relu, workspace,
+                                           workspace_bytes);
+    int st = check_gemm_args(X, l.wq, Y, M, l.out_features, K);
+    if (st != VTL_HIP_OK)
+        return st;
+    if (!l.sw || (workspace && (workspace_bytes < vtl_hip_linear_f32_dynquant_workspace(M, K) ||
+                                (reinterpret_cast<uintptr_t>(workspace) & 15))))
+        return VTL_HIP_ERR_INVALID_ARG;
+    if (!workspace) {
+        workspace = vtlhip::library_workspace(vtl_hip_linear_f32_dynquant_workspace(M, K), 1);
+        if (!workspace)
+            return vtlhip::workspace_status();
+    }
+    int8_t *xq = static_cast<int8_t *>(workspace);
+    float *sx = reinterpret_cast<float *>(xq + ((((size_t)M * (size_t)K) + 255) & ~(size_t)255));
+    st = launch_quantize_rows(X, M, K, xq, sx, current_stream());
+    return st != VTL_HIP_OK ? st : vtlhip::layer_linear_i8_f32(l, xq, sx, Y, M, relu);
+}
 
 int vtl_hip_gemm_i8_i32(const int8_t *A, const int8_t *Bt, int32_t *C, int M, int N, int K)
 {

@@ -110,8 +110,7 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
             const size_t need = vtl_hip_linear_f32_dynquant_workspace(rows, cols);
             Scratch work;
             VTL_STEP(work.take(need));
-            VTL_STEP(vtl_hip_linear_f32_dynquant(x, l.wq, l.sw, l.bias, next.as<float>(), rows, n, cols, relu,
-                                                 work.ptr, need));
+            VTL_STEP(vtl_hip_layer_f32(&l, x, next.as<float>(), rows, relu, work.ptr, need));
             cur.swap(next);
             x = cur.as<float>();
             cols = n;
@@ -126,15 +125,13 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
         if (feeds) {
             VTL_STEP(next_codes.take((size_t)rows * (size_t)n));
             VTL_STEP(next_scales.take((size_t)rows * sizeof(float)));
-            VTL_STEP(vtl_hip_linear_i8_requant(codes.as<int8_t>(), scales.as<float>(), 1, l.wq, l.sw, 1, l.bias, relu,
-                                               next_codes.as<int8_t>(), next_scales.as<float>(), nullptr, rows, n,
-                                               cols));
+            VTL_STEP(layer_linear_i8_requant(l, codes.as<int8_t>(), scales.as<float>(), next_codes.as<int8_t>(),
+                                             next_scales.as<float>(), rows, relu));
             codes.swap(next_codes);
             scales.swap(next_scales);
         } else {
             VTL_STEP(cur.take((size_t)rows * (size_t)n * sizeof(float)));
-            VTL_STEP(vtl_hip_linear_i8_f32(codes.as<int8_t>(), scales.as<float>(), l.per_channel, l.wq, l.sw,
-                                           l.per_channel, l.bias, cur.as<float>(), rows, n, cols, relu));
+            VTL_STEP(layer_linear_i8_f32(l, codes.as<int8_t>(), scales.as<float>(), cur.as<float>(), rows, relu));
             x = cur.as<float>();
         }
         cols = n;
