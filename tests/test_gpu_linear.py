@@ -586,13 +586,17 @@ def test_dynquant_without_caller_workspace(hip, mnk):
 
 
 @pytest.mark.parametrize("m", [1, 2, 8, 33, 130])
-@pytest.mark.parametrize("n,k", [(700, 1001), (300, 4095), (1100, 255), (257, 1030)])
+@pytest.mark.parametrize("n,k", [(700, 1001), (300, 4095), (1100, 255), (257, 1030), (64, 8191), (40, 16385)])
 def test_layers_whose_weights_get_padded_rows(hip, m, n, k):
     """K no multiple of 16 and enough weights that the layer keeps padded rows: host to host, on the device and in
     a chain, both granularities, each equal to the oracle on the dense codes."""
     from vtl_amd import PER_CHANNEL, PER_TENSOR, HipSession, QuantLinearLayer, Sequential
     rng = np.random.Generator(np.random.Philox(m * 13 + k))
     x = rng.standard_normal((m, k), dtype=np.float32)
+    x[0, 0], x[m // 2, k - 1] = np.nan, -40.0       # ignored by the scale, code 0; the maximum in the last place
+    if m > 8:
+        x[3] = 0.0
+        x[5, k // 2] = 1e-30
     w = rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.05)
     b = rng.standard_normal((1, n), dtype=np.float32)
     wq, sw = oracle.quantize(w, True)

@@ -99,6 +99,10 @@ struct ScratchArena {
 // Whether this thread's scratch is the static one just now.
 bool scratch_is_static();
 
+// Per-row quantization into rows of ldq codes, zeros past the end (quant.hip); false when the sizes do not qualify.
+bool launch_quantize_rows_padded(const float *x, int64_t rows, int cols, int8_t *q, int ldq, float *scale_out,
+                                 hipStream_t st, int &status);
+
 // vtl_hip_linear_i8_f32 and vtl_hip_linear_i8_requant with the parameters of a layer, whose weights may have padded rows.
 int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa, float *Y, int M, int relu);
 int layer_linear_i8_requant(const vtl_hip_layer &l, const int8_t *A, const float *sa, int8_t *Yq, float *sy, int M,

@@ -2456,6 +2456,13 @@ int vtl_hip_layer_f32(const vtl_hip_layer *layer, const float *X, float *Y, int 
     }
     int8_t *xq = static_cast<int8_t *>(workspace);
     float *sx = reinterpret_cast<float *>(xq + ((((size_t)M * (size_t)K) + 255) & ~(size_t)255));
+    // straight into padded rows, which need more room than the workspace has
+    int8_t *rows = static_cast<int8_t *>(vtlhip::library_workspace((size_t)M * (size_t)l.row_bytes, 2));
+    if (!rows)
+        return vtlhip::workspace_status();
+    if (vtlhip::launch_quantize_rows_padded(X, M, K, rows, l.row_bytes, sx, current_stream(), st))
+        return st != VTL_HIP_OK ? st : vtl_hip_linear_i8_f32(rows, sx, 1, l.wq, l.sw, 1, l.bias, Y, M, l.out_features,
+                                                             l.row_bytes, relu);
     st = launch_quantize_rows(X, M, K, xq, sx, current_stream());
     return st != VTL_HIP_OK ? st : vtlhip::layer_linear_i8_f32(l, xq, sx, Y, M, relu);
 }
