@@ -2317,10 +2317,17 @@ int launch_gemm(const GemmArgs &g_in, hipStream_t st)
             hipLaunchKernelGGL((gemm_i8_naive_kernel<F32OUT>), grid, dim3(256), 0, st, g);
             return check_launch("gemm_i8_naive_kernel");
         }
-        const int Kp = padded_row(g.K);
-        const size_t a_bytes = ((size_t)g.M * Kp + 255) & ~(size_t)255;
-        const size_t b_bytes = (size_t)g.N * Kp;
-        int8_t *ws = static_cast<int8_t *>(vtlhip::library_workspace(a_bytes + b_bytes, 2));
+        int Kp = padded_row(g.K);
+        size_t a_bytes = 0;
+        auto scratch = [&] {
+            a_bytes = ((size_t)g.M * Kp + 255) & ~(size_t)255;
+            return static_cast<int8_t *>(vtlhip::library_workspace(a_bytes + (size_t)g.N * Kp, 2));
+        };
+        int8_t *ws = scratch();
+        if (!ws && Kp != ((g.K + 15) & ~15)) {   // no memory, or a capture that may not allocate: the shortest rows
+            Kp = (g.K + 15) & ~15;
+            ws = scratch();
+        }
         if (!ws)
             return vtlhip::workspace_status();
         const int rc = launch_pad_rows(g.A, g.M, ws, g.Bt, g.N, ws + a_bytes, g.K, Kp, st);
