@@ -27,7 +27,9 @@
  *   - one host thread per device; the library keeps no pointers to caller
  *     memory after a call returns;
  *   - a few entry points stage data in scratch memory the library owns (the
- *     K-split partial sums of the matmuls, vtl_hip_linear_i8_requant,
+ *     K-split partial sums of the matmuls, with f32 and f64 operands from
+ *     K = 2048 on (for the gradients the dimension that is summed over, for
+ *     column sums 128 rows), vtl_hip_linear_i8_requant,
  *     vtl_hip_linear_f32_dynquant with workspace == NULL, int8 operands that
  *     need repacking).  There is one such buffer per purpose and device,
  *     shared by every stream: calls that use it must not overlap on a device,
@@ -37,7 +39,8 @@
  *     grow one returns VTL_HIP_ERR_UNSUPPORTED instead (pass a workspace of
  *     your own where the entry point takes one, use
  *     vtl_hip_linear_f32_dynquant_noalloc, or run the call once before
- *     capturing).  A buffer that a recorded graph uses is never freed: when a
+ *     capturing; f32 and f64 matmuls multiply in one piece instead).  A
+ *     buffer that a recorded graph uses is never freed: when a
  *     later call needs a larger one it gets a new buffer and the old one stays
  *     allocated until the process ends, so replays of the graph stay valid.
  */

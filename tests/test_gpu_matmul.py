@@ -150,6 +150,53 @@ def test_direct_shapes_at_their_edges(hip, shape, dt, knobs):
             assert np.array_equal(run_matmul(Ai, Bi, ta, tb), exact.astype(dt))
 
 
+def test_short_products_on_two_streams_do_not_meet(hip):
+    """Products with K below 2048 need nothing of the library's: two threads, a non-blocking stream each,
+    many products under way at once, every result exact."""
+    import ctypes as C
+    import threading
+    hiprt = C.CDLL("libamdhip64.so")
+    shapes = [(64, 256, 784), (16, 256, 1024), (64, 256, 2000)]
+    rng = np.random.default_rng(31)
+    work = []
+    for _ in range(2):
+        stream = C.c_void_p()
+        assert hiprt.hipStreamCreateWithFlags(C.byref(stream), C.c_uint(1)) == 0
+        jobs = []
+        for m, n, k in shapes:
+            a, b = rng.integers(-8, 9, (m, k)).astype(np.float32), rng.integers(-8, 9, (k, n)).astype(np.float32)
+            outs = [dev(np.zeros((m, n), np.float32)) for _ in range(8)]
+            jobs.append((m, n, k, dev(a), dev(b), outs, (a.astype(np.float64) @ b).astype(np.float32)))
+        work.append((stream, jobs))
+    capi.call("vtl_hip_sync")
+    failed = []
+
+    def products(stream, jobs):
+        try:
+            capi.call("vtl_hip_set_device", 0)
+            capi.call("vtl_hip_set_stream", stream)
+            for i in range(8):
+                for m, n, k, a, b, outs, _ in jobs:
+                    capi.call("vtl_hip_matmul_f32", a.ptr, b.ptr, outs[i].ptr, m, n, k, 0, 0)
+            capi.call("vtl_hip_sync")
+        except Exception as e:      # noqa: BLE001 - reported by the test
+            failed.append(e)
+
+    threads = [threading.Thread(target=products, args=w) for w in work]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
+    for stream, jobs in work:
+        for m, n, k, a, b, outs, want in jobs:
+            for o in outs:
+                assert np.array_equal(o.cpu(), want), (m, n, k)
+            for t in (a, b, *outs):
+                t.release()
+        assert hiprt.hipStreamDestroy(stream) == 0
+
+
 def test_reference_literals(hip):
     # la/la_test.v:30-37
     a = np.array([[1.0, 0], [0.0, 1]])

@@ -48,6 +48,42 @@ for m, k in ((1, 16), (64, 784), (3, 21845), (70, 1000)):
 """
 
 
+THREADS = r"""
+import threading
+import numpy as np
+from vtl_amd import capi
+from vtl_amd.tensor import HipTensor, matmul_hip
+rng = np.random.default_rng(11)
+# products whose K is cut over the grid, from several threads of a program that has the null stream alone
+bad = []
+def products(seed):
+    r = np.random.default_rng(seed)
+    capi.call("vtl_hip_set_device", 0)
+    for m, n, k in ((64, 256, 784), (16, 256, 1024), (64, 64, 4096), (33, 65, 777)) * 6:
+        a, b = r.integers(-8, 9, (m, k)).astype(np.float32), r.integers(-8, 9, (k, n)).astype(np.float32)
+        da, db = HipTensor.from_host(a), HipTensor.from_host(b)
+        c = [matmul_hip(da, db) for _ in range(4)]
+        want = (a.astype(np.float64) @ b).astype(np.float32)
+        if not all(np.array_equal(t.cpu(), want) for t in c):
+            bad.append((seed, m, n, k))
+        for t in (da, db, *c):
+            t.release()
+threads = [threading.Thread(target=products, args=(s,)) for s in range(4)]
+for t in threads:
+    t.start()
+for t in threads:
+    t.join()
+assert not bad, bad
+print("ok")
+"""
+
+
+def test_products_from_several_threads_on_the_null_stream(hip):
+    done = subprocess.run([sys.executable, "-c", THREADS], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                          text=True, timeout=100)
+    assert done.returncode == 0 and done.stdout.strip().endswith("ok"), done.stdout[-2000:]
+
+
 def test_paths_of_a_program_without_streams(hip):
     done = subprocess.run([sys.executable, "-c", PROGRAM], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
                           text=True, timeout=100)

@@ -590,7 +590,8 @@ constexpr Cost kCost[2][kShapes] = {
      {3.3, 2.21, 1.18, 4.0, 0.27}, {2.5, 3.40, 1.19, 4.0, 0.27}},
 };
 
-Plan choose_plan(bool f64, int m, int n, int k, bool whole)
+// may_slice: whether K may be cut (matmul_impl).
+Plan choose_plan(bool f64, int m, int n, int k, bool whole, bool may_slice)
 {
     Plan best = {kK4, 1};
     double best_us = 1e30;
@@ -599,7 +600,7 @@ Plan choose_plan(bool f64, int m, int n, int k, bool whole)
         const int64_t tiles = (int64_t)((m + kTileM[s] - 1) / kTileM[s]) * ((n + kTileN[s] - 1) / kTileN[s]);
         // no slices, one workgroup per compute unit in all, or two where K is long
         int64_t want[3] = {1, 0, 0};
-        if (s != kStaged && k >= 512 && tiles < 256) {
+        if (may_slice && s != kStaged && k >= 512 && tiles < 256) {
             want[1] = 256 / tiles;
             want[2] = k >= 2048 ? 2 * want[1] : 0;
         }
@@ -643,20 +644,45 @@ int launch_direct_shape(const MatmulArgs &g, bool ta, bool tb, int slices, hipSt
     return check_launch("matmul_f64acc_direct_kernel");
 }
 
+// Memory for the slices' partial sums.  While the process uses the null stream alone (`alone`) it is a block
+// of the call's own, released when the launches that use it are enqueued: the next owner's work comes
+// behind them, and calls of several threads never meet in it.  Once a stream has been named a release would
+// wait for the device, and the library's scratch, one per device, is what there is.
+struct Partial {
+    void *own = nullptr;
+    ~Partial()
+    {
+        if (own)
+            (void)vtl_hip_free(own);
+    }
+    Partial() = default;
+    Partial(const Partial &) = delete;
+    Partial &operator=(const Partial &) = delete;
+    double *take(size_t bytes, bool alone)
+    {
+        if (alone)
+            return vtl_hip_malloc(&own, bytes) == VTL_HIP_OK ? static_cast<double *>(own) : nullptr;
+        return static_cast<double *>(vtlhip::library_workspace(bytes));
+    }
+};
+
 template <typename T>
-int launch_direct(MatmulArgs g, bool ta, bool tb, Plan plan, hipStream_t st)
+int launch_direct(MatmulArgs g, bool ta, bool tb, Plan plan, bool alone, hipStream_t st)
 {
     // pairs of a row or column index that runs along memory need two of them
     const bool checked = (ta && g.M < 2) || (!tb && g.N < 2);
-    const int steps = checked ? (g.K + 15) / 16 : g.K / 16, per = (steps + plan.slices - 1) / plan.slices;
-    const int slices = per > 0 ? (steps + per - 1) / per : 1;
-    g.k_per_split = 16 * per;
+    const int steps = checked ? (g.K + 15) / 16 : g.K / 16;
+    int per = (steps + plan.slices - 1) / plan.slices;
+    int slices = per > 0 ? (steps + per - 1) / per : 1;
+    Partial partial;
     if (slices > 1) {
-        g.partial = static_cast<double *>(
-            vtlhip::library_workspace((size_t)slices * (size_t)g.M * (size_t)g.N * sizeof(double)));
-        if (!g.partial)
-            return vtlhip::workspace_status();
+        g.partial = partial.take((size_t)slices * (size_t)g.M * (size_t)g.N * sizeof(double), alone);
+        if (!g.partial) {   // no memory, or a capture that may not allocate: K in one piece
+            per = steps;
+            slices = 1;
+        }
     }
+    g.k_per_split = 16 * per;
     int rc;
     if (checked)
         rc = launch_direct_shape<T, 1, 1, 8, 2, true>(g, ta, tb, slices, st);
@@ -697,7 +723,11 @@ int matmul_impl(const T *a, const T *b, T *c, const T *bias, int m, int n, int k
     // the staged kernel's loads and stores carry no bounds checks
     const bool whole = m % 128 == 0 && n % 128 == 0 && k % 32 == 0 && k > 0 && aligned16(a) && aligned16(b) &&
                        aligned16(c);
-    Plan plan = choose_plan(sizeof(T) == 8, m, n, k, whole);
+    // Where streams have been named, K is cut from 2048 on only: there the header asks callers to order
+    // calls of different streams, which then share scratch; shorter products stay independent of each other
+    // (64 x 256 x 784 f32: 8.9 us sliced, 10.9 in one piece; 64 x 256 x 2000: 9.3 and 21.9).
+    const bool alone = vtlhip::single_stream();
+    Plan plan = choose_plan(sizeof(T) == 8, m, n, k, whole, alone || k >= 2048);
     // Tuning and tests: VTL_HIP_MATMUL_TILE 128 forces the staged kernel where it can run, 64 the
     // 64 x 64 tiles, 1 .. 5 a shape of the direct kernel; VTL_HIP_MATMUL_SPLITS the slices of K.
     const int tile = vtlhip::tuning().matmul_tile, splits = vtlhip::tuning().matmul_splits;
@@ -715,7 +745,7 @@ int matmul_impl(const T *a, const T *b, T *c, const T *bias, int m, int n, int k
         plan.slices = 1;
     }
     return plan.shape == kStaged ? launch_staged<T>(g, trans_a != 0, trans_b != 0, current_stream())
-                                 : launch_direct<T>(g, trans_a != 0, trans_b != 0, plan, current_stream());
+                                 : launch_direct<T>(g, trans_a != 0, trans_b != 0, plan, alone, current_stream());
 }
 
 template <typename T>
