@@ -85,7 +85,8 @@ int vtl_hip_malloc_on(int device_id, void **dptr, size_t bytes);
 int vtl_hip_free(void *dptr);
 int vtl_hip_trim(void);
 
-/* C.cudaMemcpy H2D storage/cuda_d_cuda.v:46, D2H :74,:90 (blocking). */
+/* C.cudaMemcpy H2D storage/cuda_d_cuda.v:46, D2H :74,:90 (blocking).  These and the copies below take memory
+ * of any device, whichever is current. */
 int vtl_hip_memcpy_h2d(void *dst_device, const void *src_host, size_t bytes);
 int vtl_hip_memcpy_d2h(void *dst_host, const void *src_device, size_t bytes);
 /* vtl_hip_memcpy_h2d for uploads that compute calls follow: returns as soon as src_host may be

@@ -96,3 +96,51 @@ for name in ("f32", "f64"):
     assert st == capi.OK and [e[0] for e in log] == ["launch"], (name, st, log)
 print("done")
 """)
+
+
+def test_copies_run_where_the_memory_is(fake_runtime):
+    """Memory of device 0 is copied after something was allocated on device 1: the kernel that carries the
+    bytes runs on device 0, and device 1 is current again afterwards.  On a stream of the caller's the copy is
+    the runtime's, which takes memory of any device."""
+    _run(fake_runtime, r"""
+runtime(devices=2)
+BIG = 3 << 20
+p = malloc_on(0, BIG + 4096)
+q = malloc_on(1, BIG + 4096)
+host = C.create_string_buffer(BIG)
+def here():
+    d = C.c_int(-1)
+    fake.hipGetDevice(C.byref(d))
+    return d.value
+def downloads(*device):
+    n = len(device)
+    return "vtl_hip_download", (n, (C.c_void_p * n)(*[C.addressof(host)] * n), (C.c_void_p * n)(*device), (C.c_size_t * n)(*[4096] * n))
+for size in (100, 4096, BIG):
+    for name, args in (("vtl_hip_memcpy_h2d", (p + 5, host, size)), ("vtl_hip_upload", (p + 5, host, size)),
+                       ("vtl_hip_memcpy_d2h", (host, p + 5, size)), ("vtl_hip_memcpy_d2d", (p, p + 2048, 1024)),
+                       downloads(p + 64, p)):
+        events()
+        capi.status(name, *args)      # no kernel runs here, so whoever waits for one reports that
+        log = [e for e in events() if e[0] in ("launch", "copy")]
+        assert log and all(e[1] == 0 for e in log), (name, size, log)
+        assert here() == 1, name
+# of both devices in one call, each on its own
+events()
+name, args = downloads(q, p)
+args[3][0] = 0
+capi.status(name, *args)
+assert {e[1] for e in events() if e[0] == "launch"} == {0}
+# device to device between the two: no kernel
+events()
+capi.call("vtl_hip_memcpy_d2d", q, p, 4096)
+assert [e[0] for e in events()] == ["copy"]
+capi.call("vtl_hip_set_stream", 4096)
+for name, args in (("vtl_hip_memcpy_h2d", (p, host, 4096)), ("vtl_hip_upload", (p, host, BIG)),
+                   ("vtl_hip_memcpy_d2h", (host, p, BIG)), downloads(p, q)):
+    events()
+    capi.status(name, *args)
+    log = [e for e in events() if e[0] in ("launch", "copy")]
+    assert log and log[0][0] == "copy" and log[0][2] == 4096, (name, log)
+    assert here() == 1, name
+print("done")
+""")

@@ -18,6 +18,24 @@ bool single_stream();
 // Called with the device that memory is asked for on.
 void note_device(int dev);
 
+// The device whose memory a copy touches.  A copy takes memory of any device, whichever is current: on
+// the null stream the owner is made current for the object's life, so that the copy comes behind the work
+// enqueued there; a stream of the caller's stays where it is, and the copy is left to the runtime.
+class OwnerDevice {
+public:
+    // Memory of two devices (`also` set and elsewhere) is left to the runtime too.
+    explicit OwnerDevice(const void *memory, const void *also = nullptr);
+    ~OwnerDevice();
+    OwnerDevice(const OwnerDevice &) = delete;
+    OwnerDevice &operator=(const OwnerDevice &) = delete;
+    bool kernels() const { return kernels_; }         // whether kernels on the current stream can access the memory
+    bool holds(const void *memory) const;             // whether this memory has the same owner
+
+private:
+    int owner_ = -1, back_ = -1;
+    bool kernels_ = true;
+};
+
 // Whether `st` is being captured into a graph (true also when that cannot be found out).
 bool stream_is_capturing(hipStream_t st);
 

@@ -820,8 +820,9 @@ try {
     if (!dst_device || !src_host)
         return VTL_HIP_ERR_INVALID_ARG;
     hipStream_t st = current_stream();
+    const OwnerDevice owner(dst_device);
     const bool one_stream = single_stream();
-    if (one_stream || !stream_is_capturing(st)) {
+    if (owner.kernels() && (one_stream || !stream_is_capturing(st))) {
         Ring *r = ring_of_current_device();
         if (r) {
             std::lock_guard<std::mutex> hold(r->lock);
@@ -850,7 +851,8 @@ try {
         return VTL_HIP_ERR_INVALID_ARG;
     hipStream_t st = current_stream();
     const size_t skew = reinterpret_cast<uintptr_t>(dst_device) & 15;
-    if (bytes + skew > kLaneStage || stream_is_capturing(st)) {
+    const OwnerDevice owner(dst_device);
+    if (!owner.kernels() || bytes + skew > kLaneStage || stream_is_capturing(st)) {
         const int rc = vtl_hip_upload(dst_device, src_host, bytes);
         if (rc != VTL_HIP_OK)
             return rc;
@@ -877,14 +879,23 @@ int vtl_hip_download(int count, void *const *dst_host, const void *const *src_de
 try {
     if (count < 0 || (count > 0 && (!dst_host || !src_device || !bytes)))
         return VTL_HIP_ERR_INVALID_ARG;
-    bool any = false;
+    const void *first = nullptr;
     for (int i = 0; i < count; i++) {
         if (bytes[i] && (!dst_host[i] || !src_device[i]))
             return VTL_HIP_ERR_INVALID_ARG;
-        any = any || bytes[i];
+        if (!first && bytes[i])
+            first = src_device[i];
     }
-    if (!any)
+    if (!first)
         return VTL_HIP_OK;
+    const OwnerDevice owner(first);
+    for (int i = 0; i < count; i++)
+        if (bytes[i] && src_device[i] != first && !owner.holds(src_device[i])) {   // of several devices: one by one
+            int rc = VTL_HIP_OK;
+            for (int k = 0; k < count && rc == VTL_HIP_OK; k++)
+                rc = vtl_hip_download(1, dst_host + k, src_device + k, bytes + k);
+            return rc;
+        }
     hipStream_t st = current_stream();
     // What goes straight into pinned memory or fits a lane's staging buffer travels together, one
     // wait for all of it; anything else goes through the ring, one by one.
@@ -893,7 +904,7 @@ try {
     int nafter = 0;
     size_t staged = 0, total = 0;
     Lane *lane = nullptr;
-    const bool fast = single_stream() || !stream_is_capturing(st);
+    const bool fast = owner.kernels() && (single_stream() || !stream_is_capturing(st));
     if (fast) {
         const int rc = lease_lane(lane);
         if (rc != VTL_HIP_OK)

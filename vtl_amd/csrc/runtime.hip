@@ -31,6 +31,53 @@ void note_device(int dev)
         g_single_stream.store(false, std::memory_order_release);
 }
 
+static bool several_devices()
+{
+    static const bool several = [] {
+        int n = 0;
+        const bool known = hipGetDeviceCount(&n) == hipSuccess;
+        (void)hipGetLastError();
+        return known && n > 1;
+    }();
+    return several;
+}
+
+// -1: not device memory, or not known to the runtime
+static int device_of(const void *memory)
+{
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, memory) != hipSuccess) {
+        (void)hipGetLastError();
+        return -1;
+    }
+    return a.type == hipMemoryTypeDevice ? a.device : -1;
+}
+
+OwnerDevice::OwnerDevice(const void *memory, const void *also)
+{
+    if (!several_devices())
+        return;
+    owner_ = device_of(memory);
+    int now = -1;
+    if (owner_ < 0 || hipGetDevice(&now) != hipSuccess || (also && device_of(also) != owner_)) {
+        (void)hipGetLastError();
+        kernels_ = false;
+    } else if (owner_ != now) {
+        if (!current_stream() && hipSetDevice(owner_) == hipSuccess)
+            back_ = now;
+        else
+            kernels_ = false;
+    }
+}
+
+OwnerDevice::~OwnerDevice()
+{
+    if (back_ >= 0)
+        (void)hipSetDevice(back_);
+}
+
+bool OwnerDevice::holds(const void *memory) const { return !several_devices() || device_of(memory) == owner_; }
+
 int record_hip_error(hipError_t e, const char *what)
 {
     snprintf(g_last_error, sizeof(g_last_error), "%s: %s (%d)", what, hipGetErrorString(e), (int)e);
@@ -332,7 +379,8 @@ int vtl_hip_memcpy_d2d(void *dst_device, const void *src_device, size_t bytes)
         return VTL_HIP_OK;
     if (!dst_device || !src_device)
         return VTL_HIP_ERR_INVALID_ARG;
-    if (launch_copy(dst_device, src_device, bytes, current_stream()))
+    const OwnerDevice owner(dst_device, src_device);
+    if (owner.kernels() && launch_copy(dst_device, src_device, bytes, current_stream()))
         return check_launch("copy_kernel");
     VTL_HIP_TRY(hipMemcpyAsync(dst_device, src_device, bytes, hipMemcpyDeviceToDevice, current_stream()));
     return VTL_HIP_OK;
