@@ -76,7 +76,9 @@ int vtl_hip_device_info(char *name, size_t name_cap, int *compute_units, int *cl
  * the process has only used the null stream, whose order keeps the old and the new use of a
  * block apart; once a thread has called vtl_hip_set_stream with a stream of its own, it
  * waits for the device.  A program that lets work of its own use such memory on a non-blocking
- * stream that it never named to the library waits for that work before it releases the memory.
+ * stream that it never named to the library waits for that work before it releases the memory, and calls
+ * vtl_hip_sync before that stream uses memory it was just given: calls enqueued on the null stream
+ * may still be at work for the block's last owner.
  * When the driver has no memory left, what is kept is given back and the call tried again;
  * vtl_hip_trim gives it back at once. */
 int vtl_hip_malloc(void **dptr, size_t bytes);
@@ -92,7 +94,8 @@ int vtl_hip_memcpy_d2h(void *dst_host, const void *src_device, size_t bytes);
 /* vtl_hip_memcpy_h2d for uploads that compute calls follow: returns as soon as src_host may be
  * reused, with the bytes on their way behind the current stream's earlier work, so that
  * whatever is enqueued there next finds them.  (It waits for their arrival too once the process has
- * used a stream of its own, vtl_hip_set_stream.) */
+ * used a stream of its own, vtl_hip_set_stream.)  Work on a non-blocking stream that was never named does
+ * not: use vtl_hip_memcpy_h2d for what such a stream reads. */
 int vtl_hip_upload(void *dst_device, const void *src_host, size_t bytes);
 /* `count` copies of vtl_hip_memcpy_d2h with one wait for all of them. */
 int vtl_hip_download(int count, void *const *dst_host, const void *const *src_device, const size_t *bytes);
@@ -110,7 +113,10 @@ int vtl_hip_memset(void *dst_device, int byte_value, size_t bytes);
 int vtl_hip_sync(void);
 
 /* Stream the compute entry points enqueue on (a hipStream_t, NULL = null
- * stream), kept per calling host thread like HIP's current device.  The
+ * stream), kept per calling host thread like HIP's current device.  The first
+ * call that names a stream waits for the device, so that the stream finds what was
+ * enqueued on the null stream before; where that stream is being captured nothing may
+ * wait, and a program calls vtl_hip_sync before it begins the capture.  The
  * reference has no stream concept beyond the unused field at
  * storage/cuda_notd_cuda.v:9. */
 int vtl_hip_set_stream(void *hip_stream);

@@ -84,6 +84,47 @@ def test_products_from_several_threads_on_the_null_stream(hip):
     assert done.returncode == 0 and done.stdout.strip().endswith("ok"), done.stdout[-2000:]
 
 
+OTHER_STREAM = r"""
+import ctypes as C
+import numpy as np
+import oracle
+from vtl_amd import QuantLinearLayer, capi
+from vtl_amd.tensor import HipTensor
+hiprt = C.CDLL("libamdhip64.so")
+capi.call("vtl_hip_set_device", 0)
+stream = C.c_void_p()
+assert hiprt.hipStreamCreateWithFlags(C.byref(stream), C.c_uint(1)) == 0     # non-blocking
+pinned = C.c_void_p()
+capi.call("vtl_hip_host_alloc", C.byref(pinned), 40 << 20)
+def read(t):
+    assert hiprt.hipMemcpyAsync(pinned, C.c_void_p(t.ptr), C.c_size_t(t.data.size), C.c_int(2), stream) == 0
+    assert hiprt.hipStreamSynchronize(stream) == 0
+    return np.frombuffer((C.c_uint8 * t.data.size).from_address(pinned.value), t.dtype).reshape(t.shape)
+rng = np.random.default_rng(3)
+for n in (1, 1000, 262144, 262145, 5 << 20, 9 << 20):
+    x = rng.standard_normal(n, dtype=np.float32)
+    t = HipTensor.from_host(x)
+    assert np.array_equal(read(t), x), n
+    t.release()
+for n, k in ((300, 1024), (1000, 1023), (2048, 4096)):
+    w = rng.standard_normal((n, k), dtype=np.float32)
+    qw = QuantLinearLayer(w, requires_grad=False).quantized()
+    codes, scales = oracle.quantize(w, True)
+    assert np.array_equal(read(qw.w_q), codes) and np.array_equal(read(qw.sw), scales), (n, k)
+    if qw.w_rows is not None:
+        assert np.array_equal(read(qw.w_rows)[:, :k], codes)
+    qw.release()
+assert hiprt.hipStreamDestroy(stream) == 0
+print("ok")
+"""
+
+
+def test_uploads_are_there_for_streams_the_library_does_not_know(hip):
+    done = subprocess.run([sys.executable, "-c", OTHER_STREAM], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                          text=True, timeout=100)
+    assert done.returncode == 0 and done.stdout.strip().endswith("ok"), done.stdout[-2000:]
+
+
 def test_paths_of_a_program_without_streams(hip):
     done = subprocess.run([sys.executable, "-c", PROGRAM], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
                           text=True, timeout=100)

@@ -5,7 +5,11 @@ import os
 import subprocess
 import sys
 
+import numpy as np
 import pytest
+
+from vtl_amd import capi, layers
+from vtl_amd.layers import PER_CHANNEL, PER_TENSOR, QuantizedWeights, QuantLinearLayer
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -144,3 +148,61 @@ for name, args in (("vtl_hip_memcpy_h2d", (p, host, 4096)), ("vtl_hip_upload", (
     assert here() == 1, name
 print("done")
 """)
+
+
+def test_tensors_from_the_host_are_there_on_return(fake_runtime):
+    """HipStorage.from_cpu waits for what it enqueued, so that work on streams the library knows
+    nothing of finds the bytes."""
+    _run(fake_runtime, r"""
+import numpy as np
+from vtl_amd.storage import HipStorage
+runtime()
+def waited(log):
+    enqueued = max(i for i, e in enumerate(log) if e[0] in ("launch", "copy"))
+    return any(e[0] in ("sync", "device_sync") for e in log[enqueued:])
+def run(f, *args, **kw):
+    events()
+    try:
+        f(*args, **kw)
+    except capi.VtlHipError:      # the wait for a kernel that no one runs
+        pass
+    return events()
+for nbytes in (1, 4096, 1 << 20, (1 << 20) + 1, 5 << 20):
+    assert waited(run(HipStorage.from_cpu, np.zeros(nbytes, np.uint8))), nbytes
+print("done")
+""")
+
+
+@pytest.mark.parametrize("mode", [PER_CHANNEL, PER_TENSOR])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("cols", [1024, 1023])
+def test_int8_parameters_are_there_on_return(monkeypatch, cols, bias, mode):
+    """The last of the calls that make a layer's codes waits for all of them; a forward from host to host leaves
+    that to its own end."""
+    calls = []
+
+    def call(name, *args):
+        calls.append(name)
+        if name == "vtl_hip_content_fingerprint":     # no device needed
+            assert capi.status(name, *args) == capi.OK
+
+    monkeypatch.setattr(capi, "call", call)
+    w, b = np.ones((300, cols), np.float32), np.zeros(300, np.float32) if bias else None
+    QuantizedWeights(w, b, mode)
+    assert "vtl_hip_quantize_f32_i8" in calls and ("vtl_hip_pad_rows_i8" in calls) == (cols % 16 != 0)
+    assert calls[-1] == "vtl_hip_sync", calls
+    calls.clear()
+    layer = QuantLinearLayer(w, b, mode, requires_grad=False)
+    layer.forward(np.zeros((4, cols), np.float32))
+    assert calls[-1] == "vtl_hip_forward_i8_host" and "vtl_hip_sync" not in calls
+    calls.clear()
+    layer.quantized()
+    assert "vtl_hip_sync" not in calls                 # the forward has waited
+    layer.invalidate()
+    calls.clear()
+    monkeypatch.setattr(layers, "forward_host", lambda *a: calls.append("failed") or 1 / 0)
+    with pytest.raises(ZeroDivisionError):
+        layer.forward(np.zeros((4, cols), np.float32))
+    del calls[:calls.index("failed") + 1]
+    layer.quantized()
+    assert calls == ["vtl_hip_sync"]                   # no copies a second time, but the wait

@@ -102,15 +102,27 @@ def content_fingerprint(t: np.ndarray) -> int:
     return h.value
 
 
+def _enqueue_upload(t: np.ndarray, params: HipParams | None) -> HipTensor:
+    """HipTensor.from_host without its wait, for what only the library's next calls use."""
+    row = np.ascontiguousarray(t)
+    dev = HipTensor.empty(row.shape, row.dtype, params)
+    if dev.data.size:
+        capi.call("vtl_hip_upload", dev.ptr, row.ctypes.data, dev.data.size)
+    return dev
+
+
 class QuantizedWeights:
     """Device-resident int8 weights of one Linear layer, derived from the f32
     parameter.  `source` / `bias_source` are the host tensors the device copies
     were made from, `fingerprint` / `bias_fingerprint` their content fingerprints at
     that moment and `frozen` whether the parameters were frozen then (see
-    QuantLinearLayer.quantized for the rule that decides re-use)."""
+    QuantLinearLayer.quantized for the rule that decides re-use).
+
+    The device copies are complete on return, for work on any stream.  With `wait` False they
+    are on their way, in order for the library's next calls; wait() makes up for it."""
 
     def __init__(self, weights: np.ndarray, bias: np.ndarray | None, mode: str,
-                 params: HipParams | None = None, frozen: bool = False):
+                 params: HipParams | None = None, frozen: bool = False, wait: bool = True):
         if weights.ndim != 2:
             raise ValueError("Matrix expected")
         if mode not in (PER_TENSOR, PER_CHANNEL):
@@ -130,7 +142,7 @@ class QuantizedWeights:
                 capi.Watch(t.ctypes.data, t.size, t.itemsize, h)
                 for t, h in zip(parts, (self.fingerprint, self.bias_fingerprint))])
         self.out_features, self.in_features = weights.shape
-        w_dev = HipTensor.from_host(np.asarray(weights, np.float32), params)
+        w_dev = _enqueue_upload(np.asarray(weights, np.float32), params)
         try:
             self.w_q, self.sw = w_dev.quantize_i8(0 if mode == PER_CHANNEL else -1)
         finally:
@@ -140,7 +152,7 @@ class QuantizedWeights:
             b = np.asarray(bias, np.float32).reshape(-1)
             if b.size != self.out_features:
                 raise ValueError(f"bias has {b.size} entries, expected {self.out_features}")
-            self.bias = HipTensor.from_host(b, params)
+            self.bias = _enqueue_upload(b, params)
         # Rows of codes that the fast kernels do not take as they are get a padded copy, made with
         # the codes instead of by every forward (8 tokens x 14336 x 4095: 39.7 -> 18.6 us).  Small ones don't: a few
         # tokens take them in one launch.
@@ -152,6 +164,19 @@ class QuantizedWeights:
         self.layer = capi.Layer(capi.LAYER_LINEAR, mode == PER_CHANNEL, self.out_features, self.in_features,
                                 (self.w_q if self.w_rows is None else self.w_rows).ptr, self.sw.ptr,
                                 self.bias.ptr if self.bias is not None else None, row_bytes)
+        self._complete = False
+        if wait:
+            self.wait()
+
+    def wait(self) -> None:
+        """Returns when the device copies are complete."""
+        if not self._complete:
+            capi.call("vtl_hip_sync")
+            self._complete = True
+
+    def known_complete(self) -> None:
+        """Says that something has been waited for that was enqueued after the device copies."""
+        self._complete = True
 
     def unchanged(self) -> bool:
         """Whether the parameters still have the contents that the codes were made from."""
@@ -214,7 +239,7 @@ def _linear_host_roundtrip(x, weights, bias, mode) -> np.ndarray:
     x = np.asarray(x, np.float32)
     if x.ndim != 2 or np.ndim(weights) != 2:
         raise ValueError("Matrix expected")
-    qw = QuantizedWeights(weights, bias, mode)
+    qw = QuantizedWeights(weights, bias, mode, wait=False)
     try:
         return forward_host(x, [qw.layer], 1, qw.out_features)
     finally:
@@ -288,6 +313,12 @@ class QuantLinearLayer:
         forward runs under `no_grad`) and were frozen when the copy was made, `weights` and
         `bias` are still the same tensor objects, and their content fingerprints have not
         changed.  Otherwise the parameters are uploaded and quantized again."""
+        qw = self.enqueue_quantized(no_grad)
+        qw.wait()
+        return qw
+
+    def enqueue_quantized(self, no_grad: bool = False) -> QuantizedWeights:
+        """quantized() without its wait, for a call whose own end is waited for (known_complete)."""
         frozen = no_grad or not self.requires_grad
         c = self._cache
         fresh = (c is not None and frozen and c.frozen and c.source is self.weights
@@ -295,7 +326,8 @@ class QuantLinearLayer:
         if not fresh:
             if c is not None:
                 c.release()
-            self._cache = QuantizedWeights(self.weights, self.bias, self.mode, self.params, frozen=frozen)
+            self._cache = QuantizedWeights(self.weights, self.bias, self.mode, self.params, frozen=frozen,
+                                           wait=False)
             self.quantize_count += 1
         return self._cache
 
@@ -308,8 +340,10 @@ class QuantLinearLayer:
         if x.ndim != 2:
             raise ValueError("Matrix expected")
         capi.call("vtl_hip_set_device", self.params.device_id)
-        qw = self.quantized(no_grad)
-        return forward_host(x, [qw.layer], 1, qw.out_features)
+        qw = self.enqueue_quantized(no_grad)
+        y = forward_host(x, [qw.layer], 1, qw.out_features)
+        qw.known_complete()
+        return y
 
     def release(self) -> None:
         if self._cache is not None:

@@ -66,12 +66,15 @@ class Sequential:
             if layer[0] == "linear":
                 qw = codes.get(layer[1])    # a layer that stands in the stack twice is quantized once
                 if qw is None:
-                    qw = codes[layer[1]] = layer[1].quantized(no_grad)
+                    qw = codes[layer[1]] = layer[1].enqueue_quantized(no_grad)
                 stack.append(qw.layer)
                 width = qw.out_features
             elif layer[0] == "relu":
                 stack.append(_RELU)
-        return forward_host(x, stack, len(stack), width)
+        y = forward_host(x, stack, len(stack), width)
+        for qw in codes.values():
+            qw.known_complete()
+        return y
 
     def release(self) -> None:
         for l in self.layers:

@@ -72,6 +72,8 @@ class HipStorage:
     # -- construction ------------------------------------------------------
     @staticmethod
     def empty(count: int, dtype, params: HipParams | None = None) -> "HipStorage":
+        """Uninitialised memory.  It may be a released storage's, which calls enqueued before still use: a
+        stream that the library was never told of (vtl_hip_set_stream) waits for vtl_hip_sync before it writes there."""
         device_id = params.device_id if params is not None else 0
         dt = _DTYPES.get(dtype) or np.dtype(dtype)
         if dt.type not in _SUPPORTED:
@@ -84,11 +86,12 @@ class HipStorage:
 
     @staticmethod
     def from_cpu(arr: np.ndarray, params: HipParams | None = None) -> "HipStorage":
-        """`(cpu &CpuStorage[T]) hip(params) !&HipStorage[T]` (storage/cuda_d_cuda.v:32-55)."""
+        """`(cpu &CpuStorage[T]) hip(params) !&HipStorage[T]` (storage/cuda_d_cuda.v:32-55).  The bytes
+        are there on return, for work on any stream."""
         flat = np.ascontiguousarray(arr).reshape(-1)
         st = HipStorage.empty(flat.size, flat.dtype, params)
         if st.size:
-            capi.call("vtl_hip_upload", st.ptr, flat.ctypes.data, st.size)
+            capi.call("vtl_hip_memcpy_h2d", st.ptr, flat.ctypes.data, st.size)
         return st
 
     @property

@@ -48,7 +48,7 @@ class HipTensor:
     # -- construction / transfer (tensor_cuda_d_cuda.v:23-60) ----------------
     @staticmethod
     def from_host(t: np.ndarray, params: HipParams | None = None) -> "HipTensor":
-        """`(t &Tensor[T]) hip(params) !&HipTensor[T]`: row-major copy, then upload."""
+        """`(t &Tensor[T]) hip(params) !&HipTensor[T]`: row-major copy, then upload, complete on return."""
         row = np.ascontiguousarray(t)
         return HipTensor(HipStorage.from_cpu(row, params), row.shape)
 
@@ -268,7 +268,9 @@ def _dynquant_workspace(m: int, k: int) -> int:
 
 def linear_f32_dynquant_hip(x: HipTensor, w_q: HipTensor, sw: HipTensor, bias: HipTensor | None,
                             relu: bool = False, workspace: HipStorage | None = None) -> HipTensor:
-    """Per-token quantization of x on the fly, then the int8 linear."""
+    """Per-token quantization of x on the fly, then the int8 linear.  Returns with the work enqueued on the
+    library's stream, as every operation on tensors does: `cpu()` waits for it, a stream that the library was
+    never told of has to be ordered behind it (vtl_hip_sync)."""
     x._assert(np.float32, what="linear_f32_dynquant_hip x")
     w_q._assert(np.int8, what="linear_f32_dynquant_hip w_q")
     M, N, K = _matmul_shapes(x, w_q)
