@@ -173,6 +173,29 @@ print("done")
 """)
 
 
+def test_a_transfer_that_waits_for_the_device_costs_no_host_time(fake_runtime):
+    """A large upload whose staging memory is not free yet: neither the caller nor the threads that help
+    with the copying spin until it is."""
+    _run(fake_runtime, r"""
+import time
+import numpy as np
+runtime(wait_ms=600)
+p = malloc_on(0, 64 << 20)
+src = np.zeros(64 << 20, np.uint8)
+src += 1
+runtime()                                      # what is made on first use does not wait
+small = np.zeros(4, np.uint8)
+capi.call("vtl_hip_upload", p, small.ctypes.data, 4)
+runtime(wait_ms=600)
+cpu, wall = time.process_time(), time.monotonic()
+st = capi.status("vtl_hip_upload", p, src.ctypes.data, src.nbytes)
+cpu, wall = time.process_time() - cpu, time.monotonic() - wall
+assert st == capi.ERR_RUNTIME and wall > 0.6   # no kernel ever frees a slot here
+assert cpu < 0.25, (cpu, wall)
+print("done")
+""")
+
+
 @pytest.mark.parametrize("mode", [PER_CHANNEL, PER_TENSOR])
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("cols", [1024, 1023])

@@ -5,6 +5,7 @@
 // of pageable memory reach 31 to 35 GB/s up and 17 down) and, for results, the page faults of
 // fresh host memory (4.7 GB/s).
 #include <sched.h>
+#include <stdio.h>
 #include <string.h>
 #include <time.h>
 
@@ -434,7 +435,38 @@ Ring *ring_of_current_device()
 
 // ---- host threads that share a large transfer's copying ------------------------------------
 // One thread copies 31 GB/s out of memory that is in no cache and touches 4.7 GB/s of fresh pages; the
-// link takes 57.  Three helpers and the caller reach 90 GB/s.
+// link takes 57.  Three helpers and the caller reach 90 GB/s.  A helper looks for jobs for half a millisecond,
+// seven chunks' time on the link, before it sleeps: a transfer that keeps the link busy never waits for one to wake
+// (50 us), and one that stands behind a long device queue costs no host time.
+constexpr double kHelpersLook = 0.5e-3;
+
+// Up to two numbers from a file, 0 for what is not there.
+void read_numbers(const char *path, double &a, double &b)
+{
+    if (FILE *f = fopen(path, "r")) {
+        if (fscanf(f, "%lf %lf", &a, &b) < 1)
+            a = 0;
+        fclose(f);
+    }
+}
+
+// Processors that this process may keep busy: those it may run on, or its container's share (both
+// generations of control groups) where that is less.
+int processors()
+{
+    cpu_set_t cpus;
+    const int have = sched_getaffinity(0, sizeof cpus, &cpus) == 0 ? CPU_COUNT(&cpus) : 1;
+    double quota = 0, period = 0, unused = 0;
+    read_numbers("/sys/fs/cgroup/cpu.max", quota, period);       // "max <period>" without a limit
+    if (period <= 0) {
+        read_numbers("/sys/fs/cgroup/cpu/cpu.cfs_quota_us", quota, unused);    // -1 without one
+        read_numbers("/sys/fs/cgroup/cpu/cpu.cfs_period_us", period, unused);
+    }
+    if (quota <= 0 || period <= 0 || quota >= period * have)
+        return have;
+    return quota < period ? 1 : (int)(quota / period);
+}
+
 struct Crew {
     struct Job {
         char *dst;
@@ -448,7 +480,9 @@ struct Crew {
     std::condition_variable wake;
     std::deque<Job> queue;
     std::atomic<int> queued{0};      // jobs in the queue, read without the lock
-    std::atomic<int> transfers{0};   // under way: helpers look for jobs instead of sleeping
+    std::atomic<int> transfers{0};   // under way
+    unsigned begun = 0;              // transfers so far (lock held)
+    bool called = false;             // every helper that sleeps has been notified (lock held)
     bool started = false;
 
     static Crew &instance()
@@ -461,10 +495,11 @@ struct Crew {
         {
             std::lock_guard<std::mutex> hold(lock);
             transfers++;
+            begun++;
+            called = true;
             if (!started) {
                 started = true;
-                cpu_set_t cpus;
-                const int have = sched_getaffinity(0, sizeof cpus, &cpus) == 0 ? CPU_COUNT(&cpus) : 1;
+                const int have = processors();
                 try {
                     for (int i = 0; i < (have > 4 ? 3 : have - 1); i++)
                         std::thread([this] { help(); }).detach();
@@ -493,6 +528,10 @@ struct Crew {
                 left.fetch_sub(1, std::memory_order_release);
             }
         }
+        if (!called) {       // one went to sleep since the transfer began
+            called = true;
+            wake.notify_all();
+        }
     }
     bool work()
     {
@@ -520,15 +559,27 @@ struct Crew {
     }
     void help()
     {
+        unsigned seen = 0;
+        double since = seconds();
         for (;;) {
-            if (work())
+            if (work()) {
+                since = seconds();
                 continue;
-            if (transfers.load(std::memory_order_acquire) > 0) {
-                __builtin_ia32_pause();
+            }
+            if (transfers.load(std::memory_order_acquire) > 0 && seconds() - since < kHelpersLook) {
+                for (int i = 0; i < 16; i++)
+                    __builtin_ia32_pause();
                 continue;
             }
             std::unique_lock<std::mutex> hold(lock);
-            wake.wait(hold, [this] { return transfers.load() > 0 || !queue.empty(); });
+            wake.wait(hold, [&] {
+                const bool stay = begun == seen && queue.empty();
+                if (stay)
+                    called = false;
+                return !stay;
+            });
+            seen = begun;
+            since = seconds();
         }
     }
 };
