@@ -98,8 +98,8 @@ def test_memory_comes_round_again_on_the_null_stream(hip):
     assert res.returncode == 0 and res.stdout.strip().endswith("done"), res.stderr[-2000:]
 
 
-# bytes: single ones, around a vector, where a small upload becomes two pieces (384 KiB), where staging ends and chunks begin (1 MiB), where a chunk is
-# a whole slot (16 MiB and more), once round the ring of 8 slots of 4 MiB and a remainder
+# bytes: single ones, around a vector, where a result's array moves to pinned memory (128 KiB), some in between, where staging
+# ends and chunks begin (1 MiB), where chunks have grown to a whole slot (from 3.75 MiB on), once round the ring of 8 slots of 4 MiB and a remainder
 @pytest.mark.parametrize("nbytes", [1, 15, 16, 17, 4096, 131072, 131073, (384 << 10) - 1, 384 << 10, 700001, (1 << 20) - 1, 1 << 20, (1 << 20) + 1,
                                     (4 << 20) + 3, (16 << 20) + 4097, (36 << 20) + 13])
 @pytest.mark.parametrize("offset", [0, 5])

@@ -17,8 +17,8 @@ import numpy as np
 import oracle
 from vtl_amd import PER_TENSOR, QuantLinearLayer, linear_backward_hip_f32
 rng = np.random.default_rng(7)
-# Linear backward, host to host: gradients below and above the size from which the device writes them
-# itself while the weights are still on their way up, weights in one piece, in several, in chunks
+# Linear backward, host to host: gradients below and above the 128 KiB from which the device writes them into
+# pinned memory itself; operands below and above the 1 MiB up to which an upload is one piece
 for m, n, k, dt in ((5, 33, 17, np.float32), (64, 256, 784, np.float32), (16, 1023, 401, np.float64),
                     (31, 700, 1301, np.float32), (48, 130, 1, np.float32)):
     for turn in range(3):
@@ -32,8 +32,8 @@ for m, n, k, dt in ((5, 33, 17, np.float32), (64, 256, 784, np.float32), (16, 10
             bound = eps * abs(want) + 2 * max(m, n) * np.finfo(np.float64).eps * size
             assert (abs(out - want) <= bound).all(), (m, n, k, dt, turn)
     print("backward", m, n, k, np.dtype(dt).name, "ok", flush=True)
-# one scale for x, read over the link by the quantizer (up to 65536 elements) or uploaded
-for m, k in ((1, 16), (64, 784), (3, 21845), (70, 1000)):
+# one scale for x, read over the link by the quantizer (up to 1 MiB, 262144 elements) or uploaded
+for m, k in ((1, 16), (64, 784), (3, 21845), (70, 1000), (3, 87381), (2, 131072), (5, 52429)):
     w = rng.standard_normal((40, k), dtype=np.float32)
     layer = QuantLinearLayer(w, mode=PER_TENSOR)
     for turn in range(3):
@@ -45,6 +45,16 @@ for m, k in ((1, 16), (64, 784), (3, 21845), (70, 1000)):
         assert np.array_equal(layer.forward(x), want), (m, k, turn)
     layer.release()
     print("layer", m, k, "ok", flush=True)
+# a scale per row: the same from 33 rows on, in one pass and (ragged rows) in two
+for m, k in ((32, 785), (33, 785), (33, 788), (64, 4095), (64, 4096), (65, 4033), (128, 2049)):
+    w = rng.standard_normal((40, k), dtype=np.float32)
+    wq, sw = oracle.quantize(w, True)
+    layer = QuantLinearLayer(w)
+    for turn in range(3):
+        x = rng.standard_normal((m, k), dtype=np.float32)
+        assert np.array_equal(layer.forward(x), oracle.linear_f32_dynquant(x, wq, sw, np.zeros(40, np.float32))), (m, k, turn)
+    layer.release()
+    print("rows", m, k, "ok", flush=True)
 """
 
 
@@ -129,4 +139,4 @@ def test_paths_of_a_program_without_streams(hip):
     done = subprocess.run([sys.executable, "-c", PROGRAM], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
                           text=True, timeout=100)
     assert done.returncode == 0, done.stdout[-2000:]
-    assert done.stdout.count("ok") == 9, done.stdout[-2000:]
+    assert done.stdout.count("ok") == 19, done.stdout[-2000:]

@@ -55,8 +55,8 @@ int record_hip_error(hipError_t e, const char *what);
 // Checks the launch that was just made.
 int check_launch(const char *kernel_name);
 
-// A small host array in pinned memory, for kernels that read their input once and can take it over
-// the link themselves instead of behind a copy.  The bytes stay until the object is gone and the
+// A small host array in pinned memory, for kernels that read their input once or twice and can take
+// it over the link themselves instead of behind a copy.  The bytes stay until the object is gone and the
 // work enqueued before that is done.  No vtl_hip_upload while one is alive on the same thread.
 struct HostInput {
     const void *data = nullptr;

@@ -118,6 +118,9 @@ class QuantizedWeights:
     that moment and `frozen` whether the parameters were frozen then (see
     QuantLinearLayer.quantized for the rule that decides re-use).
 
+    Codes whose row length is no multiple of 16 lie on the device twice where there are 2**18 of them or
+    more: dense (`w_q`), and in padded rows (`w_rows`).
+
     The device copies are complete on return, for work on any stream.  With `wait` False they
     are on their way, in order for the library's next calls; wait() makes up for it."""
 
