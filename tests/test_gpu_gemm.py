@@ -4,6 +4,8 @@ Bar: int32 accumulators bit-exact; f32 outputs within 1e-5 relative of the
 oracle applying the same scales (the kernels keep the oracle's operation
 order, so equality is asserted as well).
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -117,6 +119,52 @@ def test_odd_k_and_unaligned_operands_are_repacked(hip, mnk):
                   ybuf.ptr + off_c, m, n, k, 1)
         assert np.array_equal(d2h(ybuf.ptr + off_c, (m, n), np.float32), want), (off_a, off_b, off_c)
     for h in (abuf, bbuf, cbuf, ybuf, dsa, dsb, dbias):
+        h.release()
+
+
+# Rows of any length and address taken as they are: shorter than a vector, a vector and one byte more or less, each
+# side of the matrix-vector kernels' shortest row and of their pieces of 1024, one to eight rows and tiles of
+# 32 with an edge, the limits of the rule (256 tiles, K = 2560), and both routes forced.
+RAGGED_SHAPES = [(1, 1, 1), (3, 40, 15), (33, 31, 17), (32, 33, 31), (1, 300, 33), (40, 64, 63), (1, 65, 255), (1, 4100, 257),
+                 (1, 9, 14335), (2, 70, 1023), (2, 2050, 1025), (3, 129, 4097), (4, 1000, 8191), (5, 31, 2049), (8, 1001, 4095),
+                 (7, 300, 511), (9, 100, 1900), (16, 1001, 1901), (65, 97, 2561), (64, 4096, 129), (513, 511, 127)]
+
+
+@pytest.mark.parametrize("route", ["1", "0", None])
+@pytest.mark.parametrize("mnk", RAGGED_SHAPES)
+def test_ragged_rows_as_they_are_and_padded(hip, mnk, route, knobs):
+    if route is None:
+        knobs.delenv("VTL_HIP_RAGGED", raising=False)
+    else:
+        knobs.setenv("VTL_HIP_RAGGED", route)
+    m, n, k = mnk
+    a, bt, sa, sb, bias = workloads.square_int8_gemm(m, n, k, seed=m + 3 * n + k)
+    ref = oracle.gemm_i8_i32(a, bt, threads=CPU_THREADS)
+    abuf, bbuf = raw_device_buffer(a.size + 64), raw_device_buffer(bt.size + 64)
+    cbuf = raw_device_buffer(m * n * 4)
+    dsa, dsb, dbias = dev(sa), dev(sb), dev(bias)
+    for off_a, off_b in ((0, 0), (1, 2), (16, 3)):
+        h2d(abuf.ptr + off_a, a)
+        h2d(bbuf.ptr + off_b, bt)
+        capi.call("vtl_hip_gemm_i8_i32", abuf.ptr + off_a, bbuf.ptr + off_b, cbuf.ptr, m, n, k)
+        assert np.array_equal(d2h(cbuf.ptr, (m, n), np.int32), ref), (off_a, off_b)
+        capi.call("vtl_hip_linear_i8_f32", abuf.ptr + off_a, dsa.ptr, 1, bbuf.ptr + off_b, dsb.ptr, 1, dbias.ptr,
+                  cbuf.ptr, m, n, k, 1)
+        assert np.array_equal(d2h(cbuf.ptr, (m, n), np.float32), oracle.epilogue(ref, sa, sb, bias, relu=True)), (off_a, off_b)
+    # f32 rows quantized on the way, against dense rows of codes and against padded ones
+    x = np.random.default_rng(k).standard_normal((m, k)).astype(np.float32)
+    want = oracle.linear_f32_dynquant(x, bt, sb, bias)
+    X, Y, ws = dev(x), HipTensor.empty([m, n], np.float32), raw_device_buffer(capi.lib().vtl_hip_linear_f32_dynquant_workspace(m, k))
+    h2d(bbuf.ptr, bt)
+    capi.call("vtl_hip_linear_f32_dynquant", X.ptr, bbuf.ptr, dsb.ptr, dbias.ptr, Y.ptr, m, n, k, 0, ws.ptr, ws.size)
+    assert np.array_equal(Y.cpu(), want)
+    row = capi.lib().vtl_hip_padded_row(k)
+    rows = HipTensor.empty([n, row], np.int8)
+    capi.call("vtl_hip_pad_rows_i8", bbuf.ptr, n, k, rows.ptr)
+    layer = capi.Layer(capi.LAYER_LINEAR, 1, n, k, rows.ptr, dsb.ptr, dbias.ptr, row)
+    capi.call("vtl_hip_layer_f32", ctypes.byref(layer), X.ptr, Y.ptr, m, 0, ws.ptr, ws.size)
+    assert np.array_equal(Y.cpu(), want)
+    for h in (abuf, bbuf, cbuf, dsa, dsb, dbias, X, Y, ws, rows):
         h.release()
 
 

@@ -133,6 +133,7 @@ struct Tuning {
     bool no_gemv = false;           // VTL_HIP_NO_GEMV: keep M <= 8 off the matrix-vector kernels
     int gemv_rows = -1;             // VTL_HIP_GEMV_ROWS: 1 / 0 force the few-token kernel on / off
     int gemm_small = -1;            // VTL_HIP_GEMM_SMALL: 1 / 0 force the small-product kernel on / off
+    int ragged = -1;                // VTL_HIP_RAGGED: 1 / 0 force the kernels that take rows of any length as they are on / off
     int gemm_config = -1;           // VTL_HIP_GEMM_CONFIG "<tile index>,<splits>"
     int gemm_splits = 1;
     bool no_fused_requant = false;  // VTL_HIP_NO_FUSED_REQUANT: linear, then the row quantizer

@@ -68,6 +68,9 @@ struct GemmArgs {
     // Weight-streaming kernel with up to 32 rows (every weight is read once): read the weights
     // with non-temporal loads.  Set by the size of the matrix, see stream_weights_from.
     int stream_weights;
+    // Matrix-vector kernels, RAGGED and quantizing xf32 themselves: its row length (K, or less where the
+    // weights lie in padded rows).
+    int x_cols;
 };
 
 // LDS tiles are rows of BK bytes (BK/16 chunks of 16 bytes).  The chunk index
@@ -1200,6 +1203,74 @@ __device__ __forceinline__ int wave_sum_i32(int v)
     return __builtin_amdgcn_readlane(v, 63);
 }
 
+// 16 bytes from any address, as the whole words they lie in (the words at either end hold at least one of the bytes,
+// so nothing is touched that is not in the same word).
+typedef int v4i_words __attribute__((ext_vector_type(4), aligned(4)));
+
+template <bool NT = false>
+__device__ __forceinline__ v4i load_any16(const int8_t *p)
+{
+    const unsigned by = (unsigned)reinterpret_cast<uintptr_t>(p) & 3;
+    const int *w = reinterpret_cast<const int *>(p - by);
+    const v4i_words *v = reinterpret_cast<const v4i_words *>(w);
+    const v4i_words a = NT ? __builtin_nontemporal_load(v) : *v;
+    const int last = w[by ? 4 : 3];
+    return v4i{(int)__builtin_amdgcn_alignbyte((unsigned)a[1], (unsigned)a[0], by), (int)__builtin_amdgcn_alignbyte((unsigned)a[2], (unsigned)a[1], by),
+               (int)__builtin_amdgcn_alignbyte((unsigned)a[3], (unsigned)a[2], by), (int)__builtin_amdgcn_alignbyte((unsigned)last, (unsigned)a[3], by)};
+}
+
+// The last K % 16 bytes of a ragged row (K >= 16) are taken as the row's last 16 bytes, of which the first
+// 16 - K % 16 belong to the piece before: those of the activations are cleared, and so the
+// ones of the weights need no mask and no shift.
+__device__ __forceinline__ v4i clear_first_bytes(v4i v, int drop)
+{
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+        const int n = drop - 4 * d;   // bytes of this word to clear
+        v[d] = n >= 4 ? 0 : (n > 0 ? v[d] & (int)(0xffffffffu << (8 * n)) : v[d]);
+    }
+    return v;
+}
+
+// The same from the row's last K % 16 bytes at the front and zeros behind them, as the codes lie in LDS.
+__device__ __forceinline__ v4i move_bytes_up(v4i v, int by)
+{
+    v4i r;
+#pragma unroll
+    for (int d = 3; d >= 0; d--) {
+        unsigned lo = 0, hi = 0;   // words d - by / 4 - 1 and d - by / 4
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            if (s == d - (by >> 2))
+                hi = (unsigned)v[s];
+            if (s == d - (by >> 2) - 1)
+                lo = (unsigned)v[s];
+        }
+        r[d] = (int)((((unsigned long long)hi << 32 | lo) << (8 * (by & 3))) >> 32);
+    }
+    return r;
+}
+
+// Four consecutive floats of a row of n, from element c on, zeros past its end; rows start at any element.
+struct alignas(4) AnyFloats {
+    float v[4];
+};
+
+__device__ __forceinline__ f4 load_floats(const float *row, int c, int n)
+{
+    f4 r = {0.f, 0.f, 0.f, 0.f};
+    if (c + 4 <= n) {
+        const AnyFloats t = *reinterpret_cast<const AnyFloats *>(row + c);
+        r = f4{t.v[0], t.v[1], t.v[2], t.v[3]};
+    } else {
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+            if (c + j < n)
+                r[j] = row[c + j];
+    }
+    return r;
+}
+
 // Single token (M = 1): a matrix-vector product bound by reading Wq once, done
 // without LDS staging and without MFMA.  With DYNQ the row arrives as f32 and
 // every workgroup quantizes it itself (K floats from L2, the arithmetic of the
@@ -1211,8 +1282,9 @@ __device__ __forceinline__ int wave_sum_i32(int v)
 // registers (cached loads: between launches the weights stay in the last-level
 // cache, non-temporal ones measured 20-40 % slower), two rows are in flight
 // while the current one goes through 4 * KV dot4 instructions and a
-// cross-lane sum.  Requires K % 16 == 0, the row and Wq 16-byte aligned.
-template <int KV, int NWAVE, bool DYNQ, bool F32OUT, bool WNT = false>
+// cross-lane sum.  Requires K % 16 == 0, the row and Wq 16-byte aligned; RAGGED: K >= 16 of any
+// remainder, codes at any address.
+template <int KV, int NWAVE, bool DYNQ, bool F32OUT, bool WNT = false, bool RAGGED = false>
 __global__ __launch_bounds__(64 * NWAVE) void linear_gemv_kernel(const GemmArgs g)
 {
     constexpr int T = 64 * NWAVE;
@@ -1221,7 +1293,9 @@ __global__ __launch_bounds__(64 * NWAVE) void linear_gemv_kernel(const GemmArgs 
     __shared__ float red[NWAVE];
     __shared__ __attribute__((aligned(16))) int8_t xq[DYNQ ? 1024 * KV : 16];
     const int N = g.N, K = g.K;
-    const int kv = K >> 4;  // 16-byte pieces of a row
+    const int kv = RAGGED ? (K + 15) >> 4 : K >> 4;  // 16-byte pieces of a row
+    // where piece p starts, and the bytes of it that piece p - 1 has already
+    auto piece_at = [&](int p) { return RAGGED && 16 * p + 16 > K ? K - 16 : 16 * p; };
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // rows are dealt out cyclically: wave i of W takes rows i, i + W, i + 2 W, ... so that at any
     // moment the waves of the chip read one contiguous stretch of the matrix
@@ -1235,15 +1309,23 @@ __global__ __launch_bounds__(64 * NWAVE) void linear_gemv_kernel(const GemmArgs 
 #pragma unroll
         for (int i = 0; i < XV; i++) {
             const int idx = i * T + threadIdx.x;
-            xr[i] = idx < (K >> 2) ? xv[idx] : f4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (RAGGED)
+                xr[i] = load_floats(g.xf32, 4 * idx, g.x_cols);
+            else
+                xr[i] = idx < (K >> 2) ? xv[idx] : f4{0.f, 0.f, 0.f, 0.f};
         }
     }
     v4i wb[RING][KV];
     auto load_row = [&](int64_t r, v4i (&dst)[KV]) {
-        const v4i *p = reinterpret_cast<const v4i *>(g.Bt + r * K) + lane;
+        const int8_t *row = g.Bt + r * K;
+        const v4i *p = reinterpret_cast<const v4i *>(row) + lane;
 #pragma unroll
-        for (int j = 0; j < KV; j++)
-            dst[j] = (64 * j + lane < kv) ? (WNT ? __builtin_nontemporal_load(p + 64 * j) : p[64 * j]) : v4i{0, 0, 0, 0};
+        for (int j = 0; j < KV; j++) {
+            if constexpr (RAGGED)
+                dst[j] = (64 * j + lane < kv) ? load_any16<WNT>(row + piece_at(64 * j + lane)) : v4i{0, 0, 0, 0};
+            else
+                dst[j] = (64 * j + lane < kv) ? (WNT ? __builtin_nontemporal_load(p + 64 * j) : p[64 * j]) : v4i{0, 0, 0, 0};
+        }
     };
 #pragma unroll
     for (int d = 0; d < DEPTH; d++)
@@ -1275,14 +1357,25 @@ __global__ __launch_bounds__(64 * NWAVE) void linear_gemv_kernel(const GemmArgs 
         }
         lds_barrier();
 #pragma unroll
-        for (int j = 0; j < KV; j++)
+        for (int j = 0; j < KV; j++) {
             xc[j] = reinterpret_cast<const v4i *>(xq)[64 * j + lane];
+            if (RAGGED && 64 * j + lane == (K >> 4))
+                xc[j] = move_bytes_up(xc[j], 16 - (K & 15));
+        }
     } else {
         sx = F32OUT ? g.sa[0] : 0.0f;
         const v4i *p = reinterpret_cast<const v4i *>(g.A) + lane;
 #pragma unroll
-        for (int j = 0; j < KV; j++)
-            xc[j] = (64 * j + lane < kv) ? p[64 * j] : v4i{0, 0, 0, 0};
+        for (int j = 0; j < KV; j++) {
+            if constexpr (RAGGED) {
+                const int piece = 64 * j + lane;
+                xc[j] = piece < kv ? load_any16(g.A + piece_at(piece)) : v4i{0, 0, 0, 0};
+                if (piece == (K >> 4) && piece < kv)
+                    xc[j] = clear_first_bytes(xc[j], 16 - (K & 15));
+            } else {
+                xc[j] = (64 * j + lane < kv) ? p[64 * j] : v4i{0, 0, 0, 0};
+            }
+        }
     }
 
     // lane u of the wave looks after its u-th row: scale and bias are fetched now, the sum is
@@ -1390,8 +1483,8 @@ __device__ __forceinline__ int wave_sum_rows(int (&a)[MR], int lane)
 // through LDS.  Sums are parked
 // 64 / MR weight rows at a time (lane l: row l % MR, weight row l / MR of the
 // batch) and then scaled and stored.  Requires K % 16 == 0, K <= 1024 * KV,
-// operands 16-byte aligned.
-template <int KV, int MR, int DEPTH, bool DYNQ, bool F32OUT, bool WNT = false>
+// operands 16-byte aligned; RAGGED: K >= 16 of any remainder, codes at any address.
+template <int KV, int MR, int DEPTH, bool DYNQ, bool F32OUT, bool WNT = false, bool RAGGED = false>
 __global__ __launch_bounds__(512) void linear_gemv_rows_kernel(const GemmArgs g)
 {
     constexpr int NWAVE = 8;
@@ -1402,7 +1495,8 @@ __global__ __launch_bounds__(512) void linear_gemv_rows_kernel(const GemmArgs g)
     __shared__ int s_fast[MR];
     __shared__ __attribute__((aligned(16))) int8_t xq[DYNQ ? MR * 1024 * KV : 16];
     const int M = g.M, N = g.N, K = g.K;
-    const int kv = K >> 4;  // 16-byte pieces of a row
+    const int kv = RAGGED ? (K + 15) >> 4 : K >> 4;  // 16-byte pieces of a row
+    auto piece_at = [&](int p) { return RAGGED && 16 * p + 16 > K ? K - 16 : 16 * p; };
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t W = (int64_t)gridDim.x * NWAVE;
     const int64_t r0 = (int64_t)blockIdx.x * NWAVE + w, r1 = N;
@@ -1418,17 +1512,25 @@ __global__ __launch_bounds__(512) void linear_gemv_rows_kernel(const GemmArgs g)
 #pragma unroll
         for (int i = 0; i < XV; i++) {
             const int f = i * 512 + (int)threadIdx.x, row = f / PIECES, col = f % PIECES;
-            xr[i] = (row < M && col < (K >> 2))
-                        ? reinterpret_cast<const f4 *>(g.xf32 + (int64_t)row * K)[col]
-                        : f4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (RAGGED)
+                xr[i] = load_floats(g.xf32 + (int64_t)row * g.x_cols, 4 * col, row < M ? g.x_cols : 0);
+            else
+                xr[i] = (row < M && col < (K >> 2))
+                            ? reinterpret_cast<const f4 *>(g.xf32 + (int64_t)row * K)[col]
+                            : f4{0.f, 0.f, 0.f, 0.f};
         }
     }
     v4i wb[RING][KV];
     auto load_row = [&](int64_t r, v4i (&dst)[KV]) {
-        const v4i *p = reinterpret_cast<const v4i *>(g.Bt + r * K) + lane;
+        const int8_t *row = g.Bt + r * K;
+        const v4i *p = reinterpret_cast<const v4i *>(row) + lane;
 #pragma unroll
-        for (int j = 0; j < KV; j++)
-            dst[j] = (64 * j + lane < kv) ? (WNT ? __builtin_nontemporal_load(p + 64 * j) : p[64 * j]) : v4i{0, 0, 0, 0};
+        for (int j = 0; j < KV; j++) {
+            if constexpr (RAGGED)
+                dst[j] = (64 * j + lane < kv) ? load_any16<WNT>(row + piece_at(64 * j + lane)) : v4i{0, 0, 0, 0};
+            else
+                dst[j] = (64 * j + lane < kv) ? (WNT ? __builtin_nontemporal_load(p + 64 * j) : p[64 * j]) : v4i{0, 0, 0, 0};
+        }
     };
 #pragma unroll
     for (int d = 0; d < DEPTH; d++)
@@ -1471,15 +1573,27 @@ __global__ __launch_bounds__(512) void linear_gemv_rows_kernel(const GemmArgs g)
 #pragma unroll
         for (int m = 0; m < MR; m++)
 #pragma unroll
-            for (int j = 0; j < KV; j++)
+            for (int j = 0; j < KV; j++) {
                 xc[m][j] = reinterpret_cast<const v4i *>(xq)[m * 64 * KV + 64 * j + lane];
+                if (RAGGED && 64 * j + lane == (K >> 4))
+                    xc[m][j] = move_bytes_up(xc[m][j], 16 - (K & 15));
+            }
     } else {
 #pragma unroll
         for (int m = 0; m < MR; m++) {
-            const v4i *p = reinterpret_cast<const v4i *>(g.A + (int64_t)(m < M ? m : 0) * K) + lane;
+            const int8_t *row = g.A + (int64_t)(m < M ? m : 0) * K;
+            const v4i *p = reinterpret_cast<const v4i *>(row) + lane;
 #pragma unroll
-            for (int j = 0; j < KV; j++)
-                xc[m][j] = (m < M && 64 * j + lane < kv) ? p[64 * j] : v4i{0, 0, 0, 0};
+            for (int j = 0; j < KV; j++) {
+                if constexpr (RAGGED) {
+                    const int piece = 64 * j + lane;
+                    xc[m][j] = m < M && piece < kv ? load_any16(row + piece_at(piece)) : v4i{0, 0, 0, 0};
+                    if (piece == (K >> 4) && piece < kv)
+                        xc[m][j] = clear_first_bytes(xc[m][j], 16 - (K & 15));
+                } else {
+                    xc[m][j] = (m < M && 64 * j + lane < kv) ? p[64 * j] : v4i{0, 0, 0, 0};
+                }
+            }
         }
     }
 
@@ -1550,34 +1664,6 @@ __global__ __launch_bounds__(512) void linear_gemv_rows_kernel(const GemmArgs g)
 }
 
 
-// Any shape, any alignment: one output per thread.  Only used when K is not a
-// multiple of 16 or a pointer is not 16-byte aligned.
-template <bool F32OUT>
-__global__ __launch_bounds__(256) void gemm_i8_naive_kernel(const GemmArgs g)
-{
-    const int n = blockIdx.x * 16 + (threadIdx.x & 15);
-    const int m = blockIdx.y * 16 + (threadIdx.x >> 4);
-    if (m >= g.M || n >= g.N)
-        return;
-    const int8_t *a = g.A + (int64_t)m * g.K;
-    const int8_t *b = g.Bt + (int64_t)n * g.K;
-    int acc = 0;
-    for (int k = 0; k < g.K; k++)
-        acc += (int)a[k] * (int)b[k];
-    const int64_t o = (int64_t)m * g.N + n;
-    if (F32OUT) {
-        const float s = g.sa[(int64_t)m * g.sa_stride] * g.sw[(int64_t)n * g.sw_stride];
-        float y = (float)acc * s;
-        if (g.bias)
-            y = y + g.bias[n];
-        if (g.relu && y < 0.0f)
-            y = 0.0f;
-        reinterpret_cast<float *>(g.out)[o] = y;
-    } else {
-        reinterpret_cast<int32_t *>(g.out)[o] = acc;
-    }
-}
-
 // Rows of K bytes copied into rows of Kp >= K bytes (Kp % 16 == 0), zero filled: one or two matrices in one
 // launch, 16 destination bytes per thread.  The source rows start anywhere, which 16-byte loads do not
 // mind; bytes one by one only at the end of a row.  Bound by the copy; with four single bytes a thread and a launch
@@ -1642,13 +1728,14 @@ int launch_pad_rows(const int8_t *a, int64_t a_rows, int8_t *a_dst, const int8_t
 
 // Small products (up to a few hundred 32x32 output tiles): nothing is reused
 // often enough to stage, so each wave feeds the MFMA straight from global memory.
-// One workgroup per 32x32 tile; its NW waves split the K steps (U steps of loads
-// in flight per wave) and the partial tiles meet in LDS.  With sixteen waves a
+// One workgroup per 32x32 tile; its NW waves take groups of four K steps (a cache line
+// of every row) in turn, U steps of loads in flight per wave, and the partial tiles meet in LDS.  With sixteen waves a
 // tile with K = 4096 is two rounds of loads per wave, so a product like
 // 256x1024x4096 (256 tiles, one per compute unit) is one launch whose length is
 // a couple of memory latencies, instead of a K-split launch plus the pass that
-// adds the partial sums.  Needs K % 16 == 0 and 16-byte aligned operands.
-template <bool F32OUT, int NW, int U>
+// adds the partial sums.  Needs K % 16 == 0 and 16-byte aligned operands; RAGGED takes any K and
+// any address.
+template <bool F32OUT, int NW, int U, bool RAGGED = false>
 __global__ __launch_bounds__(64 * NW) void gemm_i8_small_kernel(const GemmArgs g)
 {
     __shared__ int red[NW][16][64];
@@ -1659,25 +1746,45 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_small_kernel(const GemmArgs g
     // rows past the edge repeat the last row; their results are never stored
     const int arow = m0 + r < g.M ? m0 + r : g.M - 1;
     const int brow = n0 + r < g.N ? n0 + r : g.N - 1;
-    const int8_t *__restrict__ ap = g.A + (int64_t)arow * g.K + 16 * half;
-    const int8_t *__restrict__ bp = g.Bt + (int64_t)brow * g.K + 16 * half;
+    const int8_t *__restrict__ ap = g.A + (int64_t)arow * g.K + (RAGGED ? 0 : 16 * half);
+    const int8_t *__restrict__ bp = g.Bt + (int64_t)brow * g.K + (RAGGED ? 0 : 16 * half);
     const int steps = (g.K + 31) / 32;
-    const int per = (steps + NW - 1) / NW;
-    const int t0 = wave * per, t1 = t0 + per < steps ? t0 + per : steps;
     v16i acc;
 #pragma unroll
     for (int i = 0; i < 16; ++i)
         acc[i] = 0;
     const v4i zero = {0, 0, 0, 0};
-    for (int t = t0; t < t1; t += U) {   // U steps of loads in flight
+    for (int t0 = 4 * wave; t0 < steps; t0 += U * NW) {   // U steps of loads in flight
         v4i a[U], b[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int k = 32 * (t + u);
+            const int k = 32 * (t0 + (u / 4) * 4 * NW + u % 4);
             // K % 32 == 16: the upper half of the last step is empty
-            const bool in = t + u < t1 && k + 16 * half < g.K;
-            a[u] = in ? *reinterpret_cast<const v4i *>(ap + k) : zero;
-            b[u] = in ? *reinterpret_cast<const v4i *>(bp + k) : zero;
+            const bool in = k + 16 * half < g.K;
+            if constexpr (RAGGED) {
+                const int c = k + 16 * half;
+                const bool whole = c + 16 <= g.K;
+                if (g.K >= 16) {
+                    a[u] = in ? load_any16(ap + (whole ? c : g.K - 16)) : zero;
+                    b[u] = in ? load_any16(bp + (whole ? c : g.K - 16)) : zero;
+                    if (!whole)
+                        a[u] = clear_first_bytes(a[u], c + 16 - g.K);   // (16 and more: all)
+                } else {   // one step, of which one half holds the row
+                    a[u] = b[u] = zero;
+                    for (int i = 0; in && i < g.K; i++) {
+                        const int at = 8 * (i & 3);
+#pragma unroll
+                        for (int d = 0; d < 4; d++)
+                            if (d == i >> 2) {
+                                a[u][d] |= (int)((unsigned)(uint8_t)ap[i] << at);
+                                b[u][d] |= (int)((unsigned)(uint8_t)bp[i] << at);
+                            }
+                    }
+                }
+            } else {
+                a[u] = in ? *reinterpret_cast<const v4i *>(ap + k) : zero;
+                b[u] = in ? *reinterpret_cast<const v4i *>(bp + k) : zero;
+            }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -2142,8 +2249,8 @@ inline int skinny_blocks_waves(int M, int N, int K)
 // take 150 to 250 registers then).
 inline int gemv_max_waves(int K) { return K <= 6144 ? 4096 : 2048; }
 
-// Single-token linear (M = 1, K % 16 == 0, K <= 14336, operands 16-byte aligned).
-template <bool DYNQ, bool F32OUT>
+// Single-token linear (M = 1, K % 16 == 0, K <= 14336, operands 16-byte aligned; RAGGED: K >= 16).
+template <bool DYNQ, bool F32OUT, bool RAGGED = false>
 int launch_gemv(const GemmArgs &g_in, hipStream_t st)
 {
     const GemmArgs &g = g_in;
@@ -2155,13 +2262,14 @@ int launch_gemv(const GemmArgs &g_in, hipStream_t st)
         return VTL_HIP_ERR_UNSUPPORTED;
     const int64_t waves = (g.N + rows_per_wave - 1) / rows_per_wave;
     const dim3 grid((unsigned)((waves + NWAVE - 1) / NWAVE)), block(64 * NWAVE);
-    const bool wnt = stream_weights_from(g.N, g.K, 8);   // the cache policy is part of the load instruction
+    // the cache policy is part of the load instruction (RAGGED: always cached, half as many kernels to load)
+    const bool wnt = !RAGGED && stream_weights_from(g.N, g.K, 8);
 #define VTL_GEMV(KV)                                                                                        \
     do {                                                                                                    \
         if (wnt)                                                                                            \
-            hipLaunchKernelGGL((linear_gemv_kernel<KV, NWAVE, DYNQ, F32OUT, true>), grid, block, 0, st, g); \
+            hipLaunchKernelGGL((linear_gemv_kernel<KV, NWAVE, DYNQ, F32OUT, !RAGGED, RAGGED>), grid, block, 0, st, g); \
         else                                                                                                \
-            hipLaunchKernelGGL((linear_gemv_kernel<KV, NWAVE, DYNQ, F32OUT, false>), grid, block, 0, st, g); \
+            hipLaunchKernelGGL((linear_gemv_kernel<KV, NWAVE, DYNQ, F32OUT, false, RAGGED>), grid, block, 0, st, g); \
     } while (0)
     switch ((g.K + 1023) / 1024) {
     case 1: VTL_GEMV(1); break;
@@ -2182,7 +2290,7 @@ int launch_gemv(const GemmArgs &g_in, hipStream_t st)
 }
 
 // A few tokens (2 <= M <= 8): rows of up to 11264 (2 tokens), 8192 (4) or 4096 (8) codes.
-template <int KV, int MR, bool DYNQ, bool F32OUT>
+template <int KV, int MR, bool DYNQ, bool F32OUT, bool RAGGED>
 int launch_gemv_rows_kv(const GemmArgs &g, hipStream_t st)
 {
     constexpr int NWAVE = 8;
@@ -2198,43 +2306,43 @@ int launch_gemv_rows_kv(const GemmArgs &g, hipStream_t st)
     if constexpr (DYNQ && MR * KV > 8) {
         return VTL_HIP_ERR_UNSUPPORTED;  // not routed here: a quantizer launch of its own is cheaper
     } else {
-        if (stream_weights_from(g.N, g.K, tuning().stream_weights_mib))   // (the cache policy is part of the load instruction)
-            hipLaunchKernelGGL((linear_gemv_rows_kernel<KV, MR, DEPTH, DYNQ, F32OUT, true>), grid, block, 0, st, g);
+        if (!RAGGED && stream_weights_from(g.N, g.K, tuning().stream_weights_mib))   // (the cache policy is part of the load instruction)
+            hipLaunchKernelGGL((linear_gemv_rows_kernel<KV, MR, DEPTH, DYNQ, F32OUT, !RAGGED, RAGGED>), grid, block, 0, st, g);
         else
-            hipLaunchKernelGGL((linear_gemv_rows_kernel<KV, MR, DEPTH, DYNQ, F32OUT, false>), grid, block, 0, st, g);
+            hipLaunchKernelGGL((linear_gemv_rows_kernel<KV, MR, DEPTH, DYNQ, F32OUT, false, RAGGED>), grid, block, 0, st, g);
         return check_launch("linear_gemv_rows_kernel");
     }
 }
 
-template <int MR, bool DYNQ, bool F32OUT>
+template <int MR, bool DYNQ, bool F32OUT, bool RAGGED>
 int launch_gemv_rows_mr(const GemmArgs &g, hipStream_t st)
 {
     const int kv = (g.K + 1023) / 1024;
     if (kv <= 1)
-        return launch_gemv_rows_kv<1, MR, DYNQ, F32OUT>(g, st);
+        return launch_gemv_rows_kv<1, MR, DYNQ, F32OUT, RAGGED>(g, st);
     if (kv <= 2)
-        return launch_gemv_rows_kv<2, MR, DYNQ, F32OUT>(g, st);
+        return launch_gemv_rows_kv<2, MR, DYNQ, F32OUT, RAGGED>(g, st);
     if (kv <= 4)
-        return launch_gemv_rows_kv<4, MR, DYNQ, F32OUT>(g, st);
+        return launch_gemv_rows_kv<4, MR, DYNQ, F32OUT, RAGGED>(g, st);
     if constexpr (MR <= 4) {
         if (kv <= 8)
-            return launch_gemv_rows_kv<8, MR, DYNQ, F32OUT>(g, st);
+            return launch_gemv_rows_kv<8, MR, DYNQ, F32OUT, RAGGED>(g, st);
     }
     if constexpr (MR <= 2) {
         if (kv <= 11)
-            return launch_gemv_rows_kv<11, MR, DYNQ, F32OUT>(g, st);
+            return launch_gemv_rows_kv<11, MR, DYNQ, F32OUT, RAGGED>(g, st);
     }
     return VTL_HIP_ERR_UNSUPPORTED;  // not reached: see gemv_rows_applies
 }
 
-template <bool DYNQ, bool F32OUT>
+template <bool DYNQ, bool F32OUT, bool RAGGED = false>
 int launch_gemv_rows(const GemmArgs &g, hipStream_t st)
 {
     if (g.M <= 2)
-        return launch_gemv_rows_mr<2, DYNQ, F32OUT>(g, st);
+        return launch_gemv_rows_mr<2, DYNQ, F32OUT, RAGGED>(g, st);
     if (g.M <= 4)
-        return launch_gemv_rows_mr<4, DYNQ, F32OUT>(g, st);
-    return launch_gemv_rows_mr<8, DYNQ, F32OUT>(g, st);
+        return launch_gemv_rows_mr<4, DYNQ, F32OUT, RAGGED>(g, st);
+    return launch_gemv_rows_mr<8, DYNQ, F32OUT, RAGGED>(g, st);
 }
 
 // The codes of the MR rows stay in registers: at most 32 pieces of 16 bytes per lane (22 for two rows:
@@ -2287,6 +2395,39 @@ inline bool gemv_applies(const void *row, const void *w, int N, int K)
            !tuning().no_gemv;
 }
 
+// The matrix-vector kernels' RAGGED forms: rows of K codes, K no multiple of 16 or operands not aligned.
+inline bool gemv_takes_ragged(int M, int N, int K)
+{
+    if (tuning().no_gemv || K < 256)
+        return false;
+    return M == 1 ? K <= 14336 && N <= 64 * gemv_max_waves(K)
+                  : M >= 2 && M <= 8 && K <= (M <= 2 ? 11264 : (M <= 4 ? 8192 : 4096));
+}
+
+// Against padding both operands and the kernel for that (one row, four rows of N = 64 ... 4000, K = 533 ... 4090: 6 to
+// 14 us, here 3.3 to 7).  With five to eight rows the kernel's own work outweighs the padding of few
+// long weight rows (8 x 64 x 4087 7.6 against 9.0 us, 8 x 1001 x 4087 9.5 and 9.2, 8 x 4001 x 2047 12.4 and 6.7).
+inline bool gemv_ragged_faster(int M, int N, int K)
+{
+    return gemv_takes_ragged(M, N, K) && (M <= 4 || K <= 2048 || N >= 1000);
+}
+
+// Where the small-product kernel takes ragged rows as they are faster than padding and the kernel for padded
+// rows (M = 9 ... 1024, N = 64 ... 4000, K = 91 ... 4090): one round of workgroups, and short rows with a few rounds
+// (64 x 1001 x 1029 8.1 -> 5.6 us, 256 x 1001 x 2047 10.1 -> 9.0, 512 x 1001 x 250 8.2 -> 5.5, 512 x 1001 x 1001 9.5
+// against 10.2, 1024 x 1001 x 91 8.0 -> 5.4).  Long rows pay where the padding would be that of many weight rows for few
+// activation rows (64 x 4001 x 4087 19.3 -> 15.2 us, 64 x 1001 x 3583 11.1 against 11.6).  The smallest products
+// never ask for scratch.
+inline bool small_ragged_faster(int M, int N, int K)
+{
+    if ((int64_t)M * N * K <= (int64_t)1 << 20)
+        return true;
+    const int64_t t32 = (int64_t)((M + 31) / 32) * ((N + 31) / 32);
+    if (t32 <= 256)
+        return K <= 2560 || (K <= 4096 && N >= 32 * (int64_t)M);
+    return (t32 <= 512 && K <= 512) || (t32 <= 1024 && K <= 128);
+}
+
 // Where one workgroup per 32x32 tile, fed straight from global memory, beats the tile kernels:
 // few tiles and a short K (nothing to stage), and up to a chip's worth of tiles with a long K,
 // which the tile kernels could only fill the chip with by cutting K (a second launch).
@@ -2302,21 +2443,35 @@ inline int small_product_waves(int64_t t32, int K)
     return K <= 2048 ? 4 : (K <= 4096 ? 8 : 16);
 }
 
+template <bool F32OUT, bool RAGGED>
+int launch_small(const GemmArgs &g, int64_t t32, int waves, hipStream_t st)
+{
+    const dim3 grid((unsigned)t32);
+    if (waves >= 16)
+        hipLaunchKernelGGL((gemm_i8_small_kernel<F32OUT, 16, 8, RAGGED>), grid, dim3(1024), 0, st, g);
+    else if (waves >= 8)
+        hipLaunchKernelGGL((gemm_i8_small_kernel<F32OUT, 8, 8, RAGGED>), grid, dim3(512), 0, st, g);
+    else
+        hipLaunchKernelGGL((gemm_i8_small_kernel<F32OUT, 4, 4, RAGGED>), grid, dim3(256), 0, st, g);
+    return check_launch("gemm_i8_small_kernel");
+}
+
 template <bool F32OUT>
 int launch_gemm(const GemmArgs &g_in, hipStream_t st)
 {
     GemmArgs g = g_in;
     if ((g.K % 16) || !aligned16(g.A) || !aligned16(g.Bt)) {
-        // The fast kernels read 16-byte chunks of rows that start 16-byte
-        // aligned.  A tiny product is done one output per thread; anything
-        // else is first copied into zero-padded rows of the library's scratch
-        // (one more pass over the int8 operands: e.g. 1024x4096x4090 takes
-        // 21 ms output-per-thread and well under 0.1 ms this way).
-        const dim3 grid((unsigned)((g.N + 15) / 16), (unsigned)((g.M + 15) / 16));
-        if ((int64_t)g.M * g.N * g.K <= (int64_t)1 << 20 && grid.y <= 65535) {
-            hipLaunchKernelGGL((gemm_i8_naive_kernel<F32OUT>), grid, dim3(256), 0, st, g);
-            return check_launch("gemm_i8_naive_kernel");
+        // Most kernels read 16-byte chunks of rows that start 16-byte aligned.  What one of the kernels that
+        // take rows as they are does not do faster is first copied into zero-padded rows of the
+        // library's scratch (one more pass over the int8 operands and one more launch).
+        const int ragged = tuning().ragged;
+        if constexpr (F32OUT) {   // (int32 sums of a few ragged rows are nobody's hot path: no kernels for them)
+            if (ragged < 0 ? gemv_ragged_faster(g.M, g.N, g.K) : ragged && gemv_takes_ragged(g.M, g.N, g.K))
+                return g.M == 1 ? launch_gemv<false, true, true>(g, st) : launch_gemv_rows<false, true, true>(g, st);
         }
+        const int64_t t32 = (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32);
+        if (ragged < 0 ? small_ragged_faster(g.M, g.N, g.K) : ragged && t32 <= 0x7fffffff)
+            return launch_small<F32OUT, true>(g, t32, g.K <= 256 || t32 > 256 ? 4 : (g.K <= 1900 ? 8 : 16), st);
         int Kp = padded_row(g.K);
         size_t a_bytes = 0;
         auto scratch = [&] {
@@ -2357,14 +2512,7 @@ int launch_gemm(const GemmArgs &g_in, hipStream_t st)
         if (t32 > 0x7fffffff)
             return VTL_HIP_ERR_UNSUPPORTED;
         const int nw = tn.gemm_small >= 4 ? tn.gemm_small : small_product_waves(t32, g.K);
-        const dim3 grid((unsigned)t32);
-        if (nw >= 16)
-            hipLaunchKernelGGL((gemm_i8_small_kernel<F32OUT, 16, 8>), grid, dim3(1024), 0, st, g);
-        else if (nw >= 8)
-            hipLaunchKernelGGL((gemm_i8_small_kernel<F32OUT, 8, 8>), grid, dim3(512), 0, st, g);
-        else
-            hipLaunchKernelGGL((gemm_i8_small_kernel<F32OUT, 4, 4>), grid, dim3(256), 0, st, g);
-        return check_launch("gemm_i8_small_kernel");
+        return launch_small<F32OUT, false>(g, t32, nw, st);
     }
     int idx, splits;
     choose_config(g.M, g.N, g.K, idx, splits);
@@ -2391,6 +2539,22 @@ const int8_t *pad_activations(const int8_t *A, int M, int K, int row, int &statu
     int8_t *ws = static_cast<int8_t *>(vtlhip::library_workspace((size_t)M * (size_t)row, 2));
     status = ws ? launch_pad_rows(A, M, ws, nullptr, 0, nullptr, K, row, current_stream()) : vtlhip::workspace_status();
     return status == VTL_HIP_OK ? ws : nullptr;
+}
+
+// Up to eight f32 rows of x_cols elements against weights in rows of `row` codes (x_cols, or padded), in one launch
+// where the aligned forms of the kernels would not take them; -1: not taken.
+int launch_ragged_rows(const float *X, int x_cols, const int8_t *Wq, int row, const float *sw, const float *bias, float *Y,
+                       int M, int N, int relu)
+{
+    if ((row == x_cols && row % 16 == 0 && aligned16(X) && aligned16(Wq)) || tuning().no_fused_decode || !tuning().ragged)
+        return -1;
+    GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, row, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
+    g.x_cols = x_cols;
+    if (M == 1 && gemv_takes_ragged(M, N, row))
+        return launch_gemv<true, true, true>(g, current_stream());
+    if (gemv_takes_ragged(M, N, row) && gemv_rows_fused_quant_faster(M, N, row))
+        return launch_gemv_rows<true, true, true>(g, current_stream());
+    return -1;
 }
 
 bool layer_row_fits(const vtl_hip_layer &l)
@@ -2456,6 +2620,9 @@ int vtl_hip_layer_f32(const vtl_hip_layer *layer, const float *X, float *Y, int 
     if (!l.sw || (workspace && (workspace_bytes < vtl_hip_linear_f32_dynquant_workspace(M, K) ||
                                 (reinterpret_cast<uintptr_t>(workspace) & 15))))
         return VTL_HIP_ERR_INVALID_ARG;
+    const int fused = launch_ragged_rows(X, K, l.wq, l.row_bytes, l.sw, l.bias, Y, M, l.out_features, relu);
+    if (fused >= 0)
+        return fused;
     if (!workspace) {
         workspace = vtlhip::library_workspace(vtl_hip_linear_f32_dynquant_workspace(M, K), 1);
         if (!workspace)
@@ -2613,6 +2780,9 @@ int vtl_hip_linear_f32_dynquant(const float *X, const int8_t *Wq, const float *s
         GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
         return launch_gemv<true, true>(g, current_stream());
     }
+    const int fused = launch_ragged_rows(X, K, Wq, K, sw, bias, Y, M, N, relu);
+    if (fused >= 0)
+        return fused;
     if (gemv_rows_applies(X, Wq, M, N, K) && gemv_rows_fused_quant_faster(M, N, K) && !tuning().no_fused_decode) {
         // a few tokens and short rows: same, each workgroup quantizes the rows itself
         GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};

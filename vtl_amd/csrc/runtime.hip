@@ -121,6 +121,7 @@ static const Tuning *read_tuning(bool force)
     t->no_gemv = flag("VTL_HIP_NO_GEMV");
     t->gemv_rows = number("VTL_HIP_GEMV_ROWS", -1);
     t->gemm_small = number("VTL_HIP_GEMM_SMALL", -1);
+    t->ragged = number("VTL_HIP_RAGGED", -1);
     if (const char *v = getenv("VTL_HIP_GEMM_CONFIG")) {
         int idx = -1, splits = 1;
         // a value that does not parse still takes the launch off the special-case kernels

@@ -157,8 +157,8 @@ class QuantizedWeights:
                 raise ValueError(f"bias has {b.size} entries, expected {self.out_features}")
             self.bias = _enqueue_upload(b, params)
         # Rows of codes that the fast kernels do not take as they are get a padded copy, made with
-        # the codes instead of by every forward (8 tokens x 14336 x 4095: 39.7 -> 18.6 us).  Small ones don't: a few
-        # tokens take them in one launch.
+        # the codes instead of by every forward (8 tokens x 14336 x 4095: 39.7 -> 18.6 us).  Small ones don't: kernels
+        # that take rows of any length are as fast there.
         self.w_rows, row_bytes = None, 0
         if self.in_features % 16 and self.w_q.size >= 1 << 18:
             row_bytes = capi.lib().vtl_hip_padded_row(self.in_features)
