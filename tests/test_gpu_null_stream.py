@@ -88,6 +88,80 @@ print("ok")
 """
 
 
+RESULTS = r"""
+import sys
+import threading
+import numpy as np
+import oracle
+from vtl_amd import PER_CHANNEL, PER_TENSOR, QuantLinearLayer, Sequential, capi, matmul_hip_host
+# Results that the last launch writes to the host itself: pieces of eight (up to 8 rows, 2048 results) and ordinary stores
+# behind it, results in staging memory and in the library's own (from 128 KiB on), in 8 MiB and more; the kernels
+# for a few rows, small products, 32-row blocks, tiles, K cut over the grid; inputs over the link (few rows: at most 20 KiB or
+# past 32 KiB) and uploaded
+LAYERS = [(1, 1, 64), (1, 2048, 300), (1, 2049, 512), (2, 1024, 256), (2, 1025, 1100), (3, 9, 1700), (8, 256, 640), (8, 40, 1024),
+          (5, 700, 2100), (17, 2050, 512), (33, 100, 784), (40, 900, 1024), (64, 300, 2100), (65, 4100, 640), (200, 801, 1664),
+          (256, 8191, 72), (256, 8193, 72)]
+def layers(seed):
+    rng = np.random.default_rng(seed)
+    for m, n, k in LAYERS:
+        w, b = rng.standard_normal((n, k), dtype=np.float32), rng.standard_normal((1, n), dtype=np.float32)
+        for mode in (PER_CHANNEL, PER_TENSOR):
+            layer = QuantLinearLayer(w, b, mode=mode, requires_grad=False)
+            wq, sw = oracle.quantize(w, mode == PER_CHANNEL)
+            for turn in range(3):
+                x = rng.standard_normal((m, k), dtype=np.float32)
+                xq, sx = oracle.quantize(x, mode == PER_CHANNEL)
+                want = oracle.epilogue(oracle.gemm_i8_i32(xq, wq, threads=4), sx, sw, b.reshape(-1))
+                assert np.array_equal(layer.forward(x), want), (m, n, k, mode, turn)
+            layer.release()
+def network(seed):   # a ReLU folded into the last layer, and one more that is not
+    rng = np.random.default_rng(seed)
+    w1, w2 = rng.standard_normal((70, 130), dtype=np.float32), rng.standard_normal((40, 70), dtype=np.float32)
+    for relus in (0, 1, 2):
+        net = Sequential().input([130]).linear(70, weights=w1).relu().linear(40, weights=w2)
+        for _ in range(relus):
+            net.relu()
+        for m in (1, 6, 40):
+            x = rng.standard_normal((m, 130), dtype=np.float32)
+            y = x
+            for w, r in ((w1, True), (w2, relus > 0)):
+                wq, sw = oracle.quantize(w, True)
+                y = oracle.linear_f32_dynquant(y, wq, sw, np.zeros(len(w), np.float32), relu=r)
+            assert np.array_equal(net.forward(x, no_grad=True), y), (relus, m)
+        net.release()
+def products(seed):   # whole numbers: every sum is exact; whole tiles of 128, K cut, results past 8 MiB
+    rng = np.random.default_rng(seed)
+    for m, n, k, dt in ((1, 1, 1, "f4"), (37, 41, 100, "f8"), (33, 257, 3000, "f4"), (128, 256, 64, "f8"), (180, 183, 32, "f4"),
+                        (1024, 1024, 8, "f8"), (1030, 1030, 8, "f8")):
+        for turn in range(2):
+            a, b = rng.integers(-8, 9, (m, k)).astype(dt), rng.integers(-8, 9, (k, n)).astype(dt)
+            assert np.array_equal(matmul_hip_host(a, b), (a.astype("f8") @ b.astype("f8")).astype(dt)), (m, n, k, dt, turn)
+capi.call("vtl_hip_set_device", 0)
+for part in (layers, network, products):
+    part(1)
+    print(part.__name__, flush=True)
+bad = []
+def guarded(part, seed):
+    try:
+        part(seed)
+    except BaseException as e:
+        bad.append((part.__name__, seed, repr(e)))
+threads = [threading.Thread(target=guarded, args=(p, s)) for s, p in enumerate((layers, layers, network, products), 2)]
+for t in threads:
+    t.start()
+for t in threads:
+    t.join()
+assert not bad, bad
+print("ok")
+"""
+
+
+def test_results_written_by_the_last_launch(hip):
+    done = subprocess.run([sys.executable, "-c", RESULTS], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                          text=True, timeout=110)
+    assert done.returncode == 0 and done.stdout.strip().endswith("ok"), done.stdout[-2000:]
+
+
 def test_products_from_several_threads_on_the_null_stream(hip):
     done = subprocess.run([sys.executable, "-c", THREADS], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
                           text=True, timeout=100)

@@ -55,21 +55,100 @@ int record_hip_error(hipError_t e, const char *what);
 // Checks the launch that was just made.
 int check_launch(const char *kernel_name);
 
-// A small host array in pinned memory, for kernels that read their input once or twice and can take
-// it over the link themselves instead of behind a copy.  The bytes stay until the object is gone and the
-// work enqueued before that is done.  No vtl_hip_upload while one is alive on the same thread.
+// A small host array in pinned memory, for kernels that can take their input over the link themselves instead
+// of behind a copy (the L2 keeps what comes over the link for the length of a launch, so workgroups that all read it
+// share one transfer per XCD).  The bytes stay until release() and until the work enqueued before that is done.  No
+// vtl_hip_upload in between on the same thread.
 struct HostInput {
     const void *data = nullptr;
     // False when the bytes have to be uploaded instead: too many, or streams of the caller's.
     bool stage(const void *src, size_t bytes);
+    void release();
     HostInput() = default;
-    ~HostInput();
+    ~HostInput() { release(); }
     HostInput(const HostInput &) = delete;
     HostInput &operator=(const HostInput &) = delete;
 
 private:
     void *ring_ = nullptr;
 };
+
+// How a launch tells the host that its results are there: every workgroup counts itself when its stores are
+// complete, and the one that reaches the target raises the flag.  No flag: nothing to tell.
+struct DoneSignal {
+    unsigned *counter;   // in device memory
+    unsigned target;
+    unsigned value;
+    unsigned *flag;      // in pinned host memory
+};
+
+// The result of a whole host-to-host call, written over the link by the launch that computes it instead of by a
+// copy behind it (64 x 256 f32: 0.8 us more than to device memory, where the copy is a launch of 4.3; 256 x 1024 f32 19 against
+// 23, 512 x 512 f64 36 against 43).  Kernels that store whole cache lines, or a few pieces of lines, store them through
+// to the host and raise the flag (attach): a part of a line crosses the link alone (512 x 512 doubles in
+// halves of lines: 17 ms).  When none did, ordinary stores went to the host's memory by way of the caches and finish() lets a small
+// launch raise the flag behind them; a fence in every workgroup instead would write the caches back each time (7.6 us with
+// 256 of them).
+class HostResult {
+public:
+    HostResult() = default;
+    ~HostResult();
+    HostResult(const HostResult &) = delete;
+    HostResult &operator=(const HostResult &) = delete;
+    // Pinned memory to write a result of `bytes` to that finish() leaves in dst (up to kParts of them); nullptr:
+    // compute in device memory and download.
+    void *begin(void *dst, size_t bytes);
+    // For the last launch of the call, right before it, with its number of workgroups.
+    void attach(DoneSignal &signal, unsigned blocks);
+    // After the release() of an input that the launch with the signal has read.
+    bool attached() const { return attached_; }
+    void input_released() { uploads_++; }
+    // Waits for the results and hands them over.
+    int finish();
+
+private:
+    struct Part {
+        void *dst;
+        const char *stage;
+        size_t bytes;
+    };
+    static constexpr int kParts = 3;
+    void *lane_ = nullptr;
+    Part after_[kParts];
+    int nafter_ = 0;
+    size_t staged_ = 0;
+    uint64_t uploads_ = 0;
+    bool attached_ = false;
+};
+
+#ifdef __HIPCC__
+// A result element: with a signal to raise it goes through the caches to where the host sees it.
+template <typename T>
+__device__ __forceinline__ void store_result(T *p, T v, const DoneSignal &done)
+{
+    if (done.flag)
+        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    else
+        *p = v;
+}
+
+// Called by every thread of a workgroup after its last store_result.  Those are written through, so their
+// acknowledgement is enough to count on; the fence of the last workgroup covers results of launches before.
+__device__ __forceinline__ void raise_when_last(const DoneSignal &done)
+{
+    if (!done.flag)
+        return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x != 0)
+        return;
+    const unsigned before = __hip_atomic_fetch_add(done.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (before + 1 == done.target) {
+        __threadfence_system();
+        __hip_atomic_store(done.flag, done.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+#endif
 
 // Streaming copy kernel (quant.hip); false when alignment or size do not qualify.
 bool launch_copy(void *dst, const void *src, size_t bytes, hipStream_t st);
@@ -121,8 +200,17 @@ bool scratch_is_static();
 bool launch_quantize_rows_padded(const float *x, int64_t rows, int cols, int8_t *q, int ldq, float *scale_out,
                                  hipStream_t st, int &status);
 
+// vtl_hip_matmul_* without a transposed b.  `result`: c is its memory, and this is the call's last launch.
+int matmul_to(HostResult *result, const float *a, const float *b, float *c, int m, int n, int k, int trans_a);
+int matmul_to(HostResult *result, const double *a, const double *b, double *c, int m, int n, int k, int trans_a);
+
 // vtl_hip_linear_i8_f32 and vtl_hip_linear_i8_requant with the parameters of a layer, whose weights may have padded rows.
-int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa, float *Y, int M, int relu);
+// `result`: Y is its memory.
+int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa, float *Y, int M, int relu,
+                        HostResult *result = nullptr);
+// vtl_hip_layer_f32.
+int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu, void *workspace, size_t workspace_bytes,
+              HostResult *result = nullptr);
 int layer_linear_i8_requant(const vtl_hip_layer &l, const int8_t *A, const float *sa, int8_t *Yq, float *sy, int M,
                             int relu);
 

@@ -33,6 +33,19 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 #define VTL_GPTR(p) ((const __attribute__((address_space(1))) void *)(p))
 #define VTL_LPTR(p) ((__attribute__((address_space(3))) void *)(p))
 
+using vtlhip::HostResult;
+using vtlhip::raise_when_last;
+using vtlhip::store_result;
+
+// Four of them in a row, 16-byte aligned unless they are written through.
+__device__ __forceinline__ void store_result4(float *p, f4 v, const vtlhip::DoneSignal &done)
+{
+    if (done.flag)   // waited for in raise_when_last
+        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(p), "v"(v) : "memory");
+    else
+        *reinterpret_cast<f4 *>(p) = v;
+}
+
 struct GemmArgs {
     const int8_t *A;   // [M,K]
     const int8_t *Bt;  // [N,K]
@@ -71,6 +84,9 @@ struct GemmArgs {
     // Matrix-vector kernels, RAGGED and quantizing xf32 themselves: its row length (K, or less where the
     // weights lie in padded rows).
     int x_cols;
+    // Where `out` is the memory of a whole host call's result: the kernels that can raise its flag do.
+    vtlhip::DoneSignal done;
+    vtlhip::HostResult *result;   // host side only
 };
 
 // LDS tiles are rows of BK bytes (BK/16 chunks of 16 bytes).  The chunk index
@@ -614,12 +630,8 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_i8_dma_kernel(const GemmArg
 // applies the epilogue.  VEC consecutive outputs of one row per thread, n
 // fastest (VEC = 4 needs N % 4 == 0 and 16-byte aligned buffers).
 template <bool F32OUT, int VEC>
-__global__ __launch_bounds__(256) void splitk_finalize_kernel(const GemmArgs g)
+__device__ __forceinline__ void finalize_outputs(const GemmArgs &g, int64_t idx, int64_t mn)
 {
-    const int64_t idx = ((int64_t)blockIdx.x * 256 + threadIdx.x) * VEC;
-    const int64_t mn = (int64_t)g.M * g.N;
-    if (idx >= mn)
-        return;
     int acc[VEC];
 #pragma unroll
     for (int j = 0; j < VEC; j++)
@@ -650,11 +662,10 @@ __global__ __launch_bounds__(256) void splitk_finalize_kernel(const GemmArgs g)
                 y[j] = 0.0f;
         }
         float *out = reinterpret_cast<float *>(g.out) + idx;
-        if (VEC == 4) {
-            *reinterpret_cast<vtlhip::qdev::float4_t *>(out) = vtlhip::qdev::float4_t{y[0], y[1], y[2], y[3]};
-        } else {
-            out[0] = y[0];
-        }
+        if (VEC == 4)
+            store_result4(out, f4{y[0], y[1], y[2], y[3]}, g.done);
+        else
+            store_result(out, y[0], g.done);
     } else {
         int32_t *out = reinterpret_cast<int32_t *>(g.out) + idx;
         if (VEC == 4) {
@@ -663,6 +674,17 @@ __global__ __launch_bounds__(256) void splitk_finalize_kernel(const GemmArgs g)
             out[0] = acc[0];
         }
     }
+}
+
+template <bool F32OUT, int VEC>
+__global__ __launch_bounds__(256) void splitk_finalize_kernel(const GemmArgs g)
+{
+    const int64_t idx = ((int64_t)blockIdx.x * 256 + threadIdx.x) * VEC;
+    const int64_t mn = (int64_t)g.M * g.N;
+    if (idx < mn)
+        finalize_outputs<F32OUT, VEC>(g, idx, mn);
+    if constexpr (F32OUT)
+        raise_when_last(g.done);
 }
 
 // Epilogue and per-row requantization in one pass over the int32 sums: one
@@ -1167,13 +1189,13 @@ __global__ __launch_bounds__(64 * NWAVE) void linear_skinny_kernel(const GemmArg
                     y[k] = v;
                 }
             }
-            if (n + 3 < N && (N & 3) == 0) {
-                *reinterpret_cast<f4 *>(reinterpret_cast<float *>(g.out) + o) = f4{y[0], y[1], y[2], y[3]};
+            if (n + 3 < N && ((N & 3) == 0 || g.done.flag)) {
+                store_result4(reinterpret_cast<float *>(g.out) + o, f4{y[0], y[1], y[2], y[3]}, g.done);
             } else {
 #pragma unroll
                 for (int k = 0; k < 4; k++)
                     if (n + k < N)
-                        reinterpret_cast<float *>(g.out)[o + k] = y[k];
+                        store_result(reinterpret_cast<float *>(g.out) + o + k, y[k], g.done);
             }
         } else {
             if (n + 3 < N && (N & 3) == 0) {
@@ -1186,6 +1208,8 @@ __global__ __launch_bounds__(64 * NWAVE) void linear_skinny_kernel(const GemmArg
             }
         }
     }
+    if constexpr (F32OUT)
+        raise_when_last(g.done);
 }
 
 // Sum of an int over the 64 lanes of a wave, the same value returned to every
@@ -1290,7 +1314,7 @@ __global__ __launch_bounds__(64 * NWAVE) void linear_gemv_kernel(const GemmArgs 
     constexpr int T = 64 * NWAVE;
     constexpr int XV = (256 * KV + T - 1) / T;  // float4 of x per thread
     constexpr int DEPTH = 2, RING = DEPTH + 1;
-    __shared__ float red[NWAVE];
+    __shared__ float red[NWAVE], parked[F32OUT ? 64 : 1][NWAVE];
     __shared__ __attribute__((aligned(16))) int8_t xq[DYNQ ? 1024 * KV : 16];
     const int N = g.N, K = g.K;
     const int kv = RAGGED ? (K + 15) >> 4 : K >> 4;  // 16-byte pieces of a row
@@ -1416,9 +1440,21 @@ __global__ __launch_bounds__(64 * NWAVE) void linear_gemv_kernel(const GemmArgs 
                 y = y + bv;
             if (g.relu && y < 0.0f)
                 y = 0.0f;
-            reinterpret_cast<float *>(g.out)[my_row] = y;
+            if (g.done.flag)
+                parked[lane][w] = y;
+            else
+                reinterpret_cast<float *>(g.out)[my_row] = y;
         } else {
             reinterpret_cast<int32_t *>(g.out)[my_row] = res;
+        }
+    }
+    if constexpr (F32OUT) {
+        if (g.done.flag) {   // the waves' rows are neighbours: NWAVE floats in a piece
+            __syncthreads();
+            const int64_t row = (int64_t)blockIdx.x * NWAVE + (threadIdx.x / NWAVE) * W + threadIdx.x % NWAVE;
+            if (row < N)
+                store_result(reinterpret_cast<float *>(g.out) + row, parked[threadIdx.x / NWAVE][threadIdx.x % NWAVE], g.done);
+            raise_when_last(g.done);
         }
     }
 }
@@ -1492,6 +1528,7 @@ __global__ __launch_bounds__(512) void linear_gemv_rows_kernel(const GemmArgs g)
     constexpr int SLOTS = 64 / MR;
     __shared__ float s_sa[MR], s_rinv[MR];
     __shared__ unsigned s_amax[MR];
+    __shared__ float parked[F32OUT ? 64 : 1][NWAVE];
     __shared__ int s_fast[MR];
     __shared__ __attribute__((aligned(16))) int8_t xq[DYNQ ? MR * 1024 * KV : 16];
     const int M = g.M, N = g.N, K = g.K;
@@ -1625,7 +1662,10 @@ __global__ __launch_bounds__(512) void linear_gemv_rows_kernel(const GemmArgs g)
                     y = y + bv;
                 if (g.relu && y < 0.0f)
                     y = 0.0f;
-                reinterpret_cast<float *>(g.out)[o] = y;
+                if (g.done.flag)   // (one batch then, see attach_gemv_result)
+                    parked[lane][w] = y;
+                else
+                    reinterpret_cast<float *>(g.out)[o] = y;
             } else {
                 reinterpret_cast<int32_t *>(g.out)[o] = res;
             }
@@ -1661,6 +1701,16 @@ __global__ __launch_bounds__(512) void linear_gemv_rows_kernel(const GemmArgs g)
     }
     if (it % SLOTS != 0)
         flush(it - it % SLOTS);
+    if constexpr (F32OUT) {
+        if (g.done.flag) {   // the waves' weight rows are neighbours: NWAVE floats in a piece
+            __syncthreads();
+            const int l = threadIdx.x / NWAVE, v = threadIdx.x % NWAVE;
+            const int64_t n = (int64_t)blockIdx.x * NWAVE + v + (int64_t)(l / MR) * W;
+            if (l % MR < M && n < N)
+                store_result(reinterpret_cast<float *>(g.out) + (int64_t)(l % MR) * N + n, parked[l][v], g.done);
+            raise_when_last(g.done);
+        }
+    }
 }
 
 
@@ -1812,11 +1862,29 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_small_kernel(const GemmArgs g
                 y = y + g.bias[n];
             if (g.relu && y < 0.0f)
                 y = 0.0f;
-            reinterpret_cast<float *>(g.out)[idx] = y;
+            store_result(reinterpret_cast<float *>(g.out) + idx, y, g.done);
         } else {
             reinterpret_cast<int32_t *>(g.out)[idx] = sum;
         }
     }
+    if constexpr (F32OUT)
+        raise_when_last(g.done);
+}
+
+// Right before the launch that writes g.out, of `blocks` workgroups that call raise_when_last.
+inline void attach_result(GemmArgs &g, unsigned blocks)
+{
+    if (g.result)
+        g.result->attach(g.done, blocks);
+}
+
+// The same for the matrix-vector kernels, whose workgroups store pieces of NWAVE = 8 floats: for few results (layers of
+// one row, 64 -> 256 and 512 -> 1024: 20.9 -> 18.2 and 22.7 -> 20.2 us), while with 4096 the pieces cost more than a launch that
+// raises the flag behind ordinary stores (24.8 against 26.0).  `one_batch`: a lane parks one result.
+inline void attach_gemv_result(GemmArgs &g, unsigned blocks, bool one_batch)
+{
+    if (one_batch && (int64_t)g.M * g.N <= 2048)
+        attach_result(g, blocks);
 }
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -1962,11 +2030,13 @@ int launch_dma(GemmArgs g, int splits, hipStream_t st)
         return launch_finalize_requant(g, st);
     const int64_t mn = (int64_t)g.M * g.N;
     if (g.N % 4 == 0 && aligned16(g.out) && aligned16(g.partials)) {
-        hipLaunchKernelGGL((splitk_finalize_kernel<F32OUT, 4>), dim3((unsigned)((mn / 4 + 255) / 256)), dim3(256), 0,
-                           st, g);
+        const unsigned blocks = (unsigned)((mn / 4 + 255) / 256);
+        attach_result(g, blocks);
+        hipLaunchKernelGGL((splitk_finalize_kernel<F32OUT, 4>), dim3(blocks), dim3(256), 0, st, g);
     } else {
-        hipLaunchKernelGGL((splitk_finalize_kernel<F32OUT, 1>), dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, st,
-                           g);
+        const unsigned blocks = (unsigned)((mn + 255) / 256);
+        attach_result(g, blocks);
+        hipLaunchKernelGGL((splitk_finalize_kernel<F32OUT, 1>), dim3(blocks), dim3(256), 0, st, g);
     }
     return check_launch("splitk_finalize_kernel");
 }
@@ -2118,6 +2188,7 @@ int launch_skinny_cfg(const GemmArgs &g_in, hipStream_t st)
             hipFuncAttributeMaxDynamicSharedMemorySize, lds));
         done.store(true, std::memory_order_release);
     }
+    attach_result(g, (unsigned)((g.N + 31) / 32) * grid.y);   // (the quantizing workgroups are gone by then)
     hipLaunchKernelGGL((linear_skinny_kernel<NWAVE, STAGES, XJ, F32OUT, STAGEQ>), grid, dim3(64 * NWAVE), lds, st, g);
     return check_launch("linear_skinny_kernel");
 }
@@ -2253,7 +2324,7 @@ inline int gemv_max_waves(int K) { return K <= 6144 ? 4096 : 2048; }
 template <bool DYNQ, bool F32OUT, bool RAGGED = false>
 int launch_gemv(const GemmArgs &g_in, hipStream_t st)
 {
-    const GemmArgs &g = g_in;
+    GemmArgs g = g_in;
     constexpr int NWAVE = 8;
     // every wave the same number of rows
     const int max_waves = gemv_max_waves(g.K);
@@ -2262,6 +2333,7 @@ int launch_gemv(const GemmArgs &g_in, hipStream_t st)
         return VTL_HIP_ERR_UNSUPPORTED;
     const int64_t waves = (g.N + rows_per_wave - 1) / rows_per_wave;
     const dim3 grid((unsigned)((waves + NWAVE - 1) / NWAVE)), block(64 * NWAVE);
+    attach_gemv_result(g, grid.x, true);
     // the cache policy is part of the load instruction (RAGGED: always cached, half as many kernels to load)
     const bool wnt = !RAGGED && stream_weights_from(g.N, g.K, 8);
 #define VTL_GEMV(KV)                                                                                        \
@@ -2291,7 +2363,7 @@ int launch_gemv(const GemmArgs &g_in, hipStream_t st)
 
 // A few tokens (2 <= M <= 8): rows of up to 11264 (2 tokens), 8192 (4) or 4096 (8) codes.
 template <int KV, int MR, bool DYNQ, bool F32OUT, bool RAGGED>
-int launch_gemv_rows_kv(const GemmArgs &g, hipStream_t st)
+int launch_gemv_rows_kv(GemmArgs g, hipStream_t st)
 {
     constexpr int NWAVE = 8;
     // Codes and weight rows live in registers, which limits the waves a SIMD holds; with few
@@ -2306,6 +2378,7 @@ int launch_gemv_rows_kv(const GemmArgs &g, hipStream_t st)
     if constexpr (DYNQ && MR * KV > 8) {
         return VTL_HIP_ERR_UNSUPPORTED;  // not routed here: a quantizer launch of its own is cheaper
     } else {
+        attach_gemv_result(g, grid.x, rows_per_wave <= 64 / MR);
         if (!RAGGED && stream_weights_from(g.N, g.K, tuning().stream_weights_mib))   // (the cache policy is part of the load instruction)
             hipLaunchKernelGGL((linear_gemv_rows_kernel<KV, MR, DEPTH, DYNQ, F32OUT, !RAGGED, RAGGED>), grid, block, 0, st, g);
         else
@@ -2444,9 +2517,10 @@ inline int small_product_waves(int64_t t32, int K)
 }
 
 template <bool F32OUT, bool RAGGED>
-int launch_small(const GemmArgs &g, int64_t t32, int waves, hipStream_t st)
+int launch_small(GemmArgs g, int64_t t32, int waves, hipStream_t st)
 {
     const dim3 grid((unsigned)t32);
+    attach_result(g, grid.x);
     if (waves >= 16)
         hipLaunchKernelGGL((gemm_i8_small_kernel<F32OUT, 16, 8, RAGGED>), grid, dim3(1024), 0, st, g);
     else if (waves >= 8)
@@ -2544,12 +2618,13 @@ const int8_t *pad_activations(const int8_t *A, int M, int K, int row, int &statu
 // Up to eight f32 rows of x_cols elements against weights in rows of `row` codes (x_cols, or padded), in one launch
 // where the aligned forms of the kernels would not take them; -1: not taken.
 int launch_ragged_rows(const float *X, int x_cols, const int8_t *Wq, int row, const float *sw, const float *bias, float *Y,
-                       int M, int N, int relu)
+                       int M, int N, int relu, HostResult *result)
 {
     if ((row == x_cols && row % 16 == 0 && aligned16(X) && aligned16(Wq)) || tuning().no_fused_decode || !tuning().ragged)
         return -1;
     GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, row, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
     g.x_cols = x_cols;
+    g.result = result;
     if (M == 1 && gemv_takes_ragged(M, N, row))
         return launch_gemv<true, true, true>(g, current_stream());
     if (gemv_takes_ragged(M, N, row) && gemv_rows_fused_quant_faster(M, N, row))
@@ -2562,11 +2637,96 @@ bool layer_row_fits(const vtl_hip_layer &l)
     return l.row_bytes == 0 || (l.row_bytes >= l.in_features && l.row_bytes % 16 == 0 && l.row_bytes <= 131072 && aligned16(l.wq));
 }
 
+int linear_i8_f32(const int8_t *A, const float *sa, int sa_per_row, const int8_t *Wq,
+                          const float *sw, int sw_per_col, const float *bias, float *Y, int M, int N,
+                          int K, int relu, HostResult *result)
+{
+    int st = check_gemm_args(A, Wq, Y, M, N, K);
+    if (st != VTL_HIP_OK)
+        return st;
+    if (!sa || !sw)
+        return VTL_HIP_ERR_INVALID_ARG;
+    if (M == 0 || N == 0)
+        return VTL_HIP_OK;
+    if (K == 0)
+        return VTL_HIP_ERR_UNSUPPORTED;  // la.matmul rejects empty inner dimensions as well
+    GemmArgs g{A, Wq, Y, sa, sw, bias, M, N, K, sa_per_row ? 1 : 0, sw_per_col ? 1 : 0, relu ? 1 : 0, 1, nullptr, nullptr, 0};
+    g.result = result;
+    return launch_gemm<true>(g, current_stream());
+}
+
+int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, const float *bias,
+                                float *Y, int M, int N, int K, int relu, void *workspace,
+                                size_t workspace_bytes, HostResult *result)
+{
+    int st = check_gemm_args(X, Wq, Y, M, N, K);
+    if (st != VTL_HIP_OK)
+        return st;
+    if (!sw)
+        return VTL_HIP_ERR_INVALID_ARG;
+    if (M == 0 || N == 0)
+        return VTL_HIP_OK;
+    if (K == 0)
+        return VTL_HIP_ERR_UNSUPPORTED;
+    if (workspace && (workspace_bytes < vtl_hip_linear_f32_dynquant_workspace(M, K) ||
+                      (reinterpret_cast<uintptr_t>(workspace) & 15)))
+        return VTL_HIP_ERR_INVALID_ARG;
+    if (M == 1 && gemv_applies(X, Wq, N, K) && !tuning().no_fused_decode) {
+        // a single token: quantized inside the matrix-vector kernel, one launch instead of two
+        // (N = 14336, K = 4096: 9.5 us against 12.8 us).  The workspace stays unused.
+        // VTL_HIP_NO_FUSED_DECODE forces the two-launch path (tests).
+        GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
+        g.result = result;
+        return launch_gemv<true, true>(g, current_stream());
+    }
+    const int fused = launch_ragged_rows(X, K, Wq, K, sw, bias, Y, M, N, relu, result);
+    if (fused >= 0)
+        return fused;
+    if (gemv_rows_applies(X, Wq, M, N, K) && gemv_rows_fused_quant_faster(M, N, K) && !tuning().no_fused_decode) {
+        // a few tokens and short rows: same, each workgroup quantizes the rows itself
+        GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
+        g.result = result;
+        return launch_gemv_rows<true, true>(g, current_stream());
+    }
+    const bool staged = stage_inside_launch_faster(M, N, K, gemv_rows_applies(X, Wq, M, N, K) && gemv_rows_faster(M, N, K, true)) &&
+                        aligned16(X) && aligned16(Wq) && tuning().gemm_config < 0 && !tuning().no_fused_decode;
+    if (!workspace) {   // no caller scratch: stage in the library's own buffer
+        workspace = vtlhip::library_workspace(vtl_hip_linear_f32_dynquant_workspace(M, K), 1);
+        if (!workspace)
+            return vtlhip::workspace_status();
+    }
+    int8_t *xq = reinterpret_cast<int8_t *>(workspace);
+    const size_t codes = (((size_t)M * (size_t)K) + 255) & ~(size_t)255;
+    float *sx = reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + codes);
+    if (staged && (reinterpret_cast<uintptr_t>(workspace) & 127) == 0) {
+        // a few tokens: quantized inside the weight-streaming launch (N = 14336, K = 4096, M = 8:
+        // 14.4 us against 16.0 us).  Its workgroups read the staging buffer as soon as the rows
+        // are counted and rely on no cache holding an older copy of those lines, which holds
+        // when nothing else shares them: the buffer starts on a cache line (anything from
+        // vtl_hip_malloc does) and its size is a whole number of them.
+        GemmArgs g{xq, Wq, Y, sx, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
+        g.stage_codes = xq;
+        g.stage_scales = sx;
+        g.result = result;
+        bool launched = false;
+        st = launch_skinny_staged(g, current_stream(), launched);
+        if (launched || st != VTL_HIP_OK)
+            return st;
+    }
+    st = launch_quantize_rows(X, M, K, xq, sx, current_stream());
+    if (st != VTL_HIP_OK)
+        return st;
+    GemmArgs g{xq, Wq, Y, sx, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, nullptr, 0};
+    g.result = result;
+    return launch_gemm<true>(g, current_stream());
+}
+
 }  // namespace
 
 namespace vtlhip {
 
-int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa, float *Y, int M, int relu)
+int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa, float *Y, int M, int relu,
+                        HostResult *result)
 {
     int st = layer_row_fits(l) && A && M >= 0 ? VTL_HIP_OK : VTL_HIP_ERR_INVALID_ARG;
     int K = l.in_features;
@@ -2574,8 +2734,44 @@ int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa
         A = pad_activations(A, M, K, l.row_bytes, st);
         K = l.row_bytes;
     }
-    return st != VTL_HIP_OK ? st : vtl_hip_linear_i8_f32(A, sa, l.per_channel, l.wq, l.sw, l.per_channel, l.bias, Y, M,
-                                                         l.out_features, K, relu);
+    return st != VTL_HIP_OK ? st : linear_i8_f32(A, sa, l.per_channel, l.wq, l.sw, l.per_channel, l.bias, Y, M,
+                                                         l.out_features, K, relu, result);
+}
+
+int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu, void *workspace, size_t workspace_bytes,
+              HostResult *result)
+{
+    if (l.kind != VTL_HIP_LAYER_LINEAR || !l.per_channel || !layer_row_fits(l))
+        return VTL_HIP_ERR_INVALID_ARG;
+    const int K = l.in_features;
+    if (l.row_bytes == 0 || M <= 0 || l.out_features <= 0 || K <= 0)
+        return linear_f32_dynquant(X, l.wq, l.sw, l.bias, Y, M, l.out_features, K, relu, workspace, workspace_bytes,
+                                   result);
+    int st = check_gemm_args(X, l.wq, Y, M, l.out_features, K);
+    if (st != VTL_HIP_OK)
+        return st;
+    if (!l.sw || (workspace && (workspace_bytes < vtl_hip_linear_f32_dynquant_workspace(M, K) ||
+                                (reinterpret_cast<uintptr_t>(workspace) & 15))))
+        return VTL_HIP_ERR_INVALID_ARG;
+    const int fused = launch_ragged_rows(X, K, l.wq, l.row_bytes, l.sw, l.bias, Y, M, l.out_features, relu, result);
+    if (fused >= 0)
+        return fused;
+    if (!workspace) {
+        workspace = vtlhip::library_workspace(vtl_hip_linear_f32_dynquant_workspace(M, K), 1);
+        if (!workspace)
+            return vtlhip::workspace_status();
+    }
+    int8_t *xq = static_cast<int8_t *>(workspace);
+    float *sx = reinterpret_cast<float *>(xq + ((((size_t)M * (size_t)K) + 255) & ~(size_t)255));
+    // straight into padded rows, which need more room than the workspace has
+    int8_t *rows = static_cast<int8_t *>(vtlhip::library_workspace((size_t)M * (size_t)l.row_bytes, 2));
+    if (!rows)
+        return vtlhip::workspace_status();
+    if (vtlhip::launch_quantize_rows_padded(X, M, K, rows, l.row_bytes, sx, current_stream(), st))
+        return st != VTL_HIP_OK ? st : linear_i8_f32(rows, sx, 1, l.wq, l.sw, 1, l.bias, Y, M, l.out_features,
+                                                     l.row_bytes, relu, result);
+    st = launch_quantize_rows(X, M, K, xq, sx, current_stream());
+    return st != VTL_HIP_OK ? st : layer_linear_i8_f32(l, xq, sx, Y, M, relu, result);
 }
 
 int layer_linear_i8_requant(const vtl_hip_layer &l, const int8_t *A, const float *sa, int8_t *Yq, float *sy, int M,
@@ -2607,38 +2803,7 @@ int vtl_hip_pad_rows_i8(const int8_t *src, int64_t rows, int cols, int8_t *dst)
 int vtl_hip_layer_f32(const vtl_hip_layer *layer, const float *X, float *Y, int M, int relu, void *workspace,
                       size_t workspace_bytes)
 {
-    if (!layer || layer->kind != VTL_HIP_LAYER_LINEAR || !layer->per_channel || !layer_row_fits(*layer))
-        return VTL_HIP_ERR_INVALID_ARG;
-    const vtl_hip_layer &l = *layer;
-    const int K = l.in_features;
-    if (l.row_bytes == 0 || M <= 0 || l.out_features <= 0 || K <= 0)
-        return vtl_hip_linear_f32_dynquant(X, l.wq, l.sw, l.bias, Y, M, l.out_features, K, relu, workspace,
-                                           workspace_bytes);
-    int st = check_gemm_args(X, l.wq, Y, M, l.out_features, K);
-    if (st != VTL_HIP_OK)
-        return st;
-    if (!l.sw || (workspace && (workspace_bytes < vtl_hip_linear_f32_dynquant_workspace(M, K) ||
-                                (reinterpret_cast<uintptr_t>(workspace) & 15))))
-        return VTL_HIP_ERR_INVALID_ARG;
-    const int fused = launch_ragged_rows(X, K, l.wq, l.row_bytes, l.sw, l.bias, Y, M, l.out_features, relu);
-    if (fused >= 0)
-        return fused;
-    if (!workspace) {
-        workspace = vtlhip::library_workspace(vtl_hip_linear_f32_dynquant_workspace(M, K), 1);
-        if (!workspace)
-            return vtlhip::workspace_status();
-    }
-    int8_t *xq = static_cast<int8_t *>(workspace);
-    float *sx = reinterpret_cast<float *>(xq + ((((size_t)M * (size_t)K) + 255) & ~(size_t)255));
-    // straight into padded rows, which need more room than the workspace has
-    int8_t *rows = static_cast<int8_t *>(vtlhip::library_workspace((size_t)M * (size_t)l.row_bytes, 2));
-    if (!rows)
-        return vtlhip::workspace_status();
-    if (vtlhip::launch_quantize_rows_padded(X, M, K, rows, l.row_bytes, sx, current_stream(), st))
-        return st != VTL_HIP_OK ? st : vtl_hip_linear_i8_f32(rows, sx, 1, l.wq, l.sw, 1, l.bias, Y, M, l.out_features,
-                                                             l.row_bytes, relu);
-    st = launch_quantize_rows(X, M, K, xq, sx, current_stream());
-    return st != VTL_HIP_OK ? st : vtlhip::layer_linear_i8_f32(l, xq, sx, Y, M, relu);
+    return layer ? vtlhip::layer_f32(*layer, X, Y, M, relu, workspace, workspace_bytes) : VTL_HIP_ERR_INVALID_ARG;
 }
 
 int vtl_hip_gemm_i8_i32(const int8_t *A, const int8_t *Bt, int32_t *C, int M, int N, int K)
@@ -2658,17 +2823,7 @@ int vtl_hip_linear_i8_f32(const int8_t *A, const float *sa, int sa_per_row, cons
                           const float *sw, int sw_per_col, const float *bias, float *Y, int M, int N,
                           int K, int relu)
 {
-    int st = check_gemm_args(A, Wq, Y, M, N, K);
-    if (st != VTL_HIP_OK)
-        return st;
-    if (!sa || !sw)
-        return VTL_HIP_ERR_INVALID_ARG;
-    if (M == 0 || N == 0)
-        return VTL_HIP_OK;
-    if (K == 0)
-        return VTL_HIP_ERR_UNSUPPORTED;  // la.matmul rejects empty inner dimensions as well
-    GemmArgs g{A, Wq, Y, sa, sw, bias, M, N, K, sa_per_row ? 1 : 0, sw_per_col ? 1 : 0, relu ? 1 : 0, 1, nullptr, nullptr, 0};
-    return launch_gemm<true>(g, current_stream());
+    return linear_i8_f32(A, sa, sa_per_row, Wq, sw, sw_per_col, bias, Y, M, N, K, relu, nullptr);
 }
 
 int vtl_hip_linear_i8_requant(const int8_t *A, const float *sa, int sa_per_row, const int8_t *Wq,
@@ -2761,62 +2916,7 @@ int vtl_hip_linear_f32_dynquant(const float *X, const int8_t *Wq, const float *s
                                 float *Y, int M, int N, int K, int relu, void *workspace,
                                 size_t workspace_bytes)
 {
-    int st = check_gemm_args(X, Wq, Y, M, N, K);
-    if (st != VTL_HIP_OK)
-        return st;
-    if (!sw)
-        return VTL_HIP_ERR_INVALID_ARG;
-    if (M == 0 || N == 0)
-        return VTL_HIP_OK;
-    if (K == 0)
-        return VTL_HIP_ERR_UNSUPPORTED;
-    if (workspace && (workspace_bytes < vtl_hip_linear_f32_dynquant_workspace(M, K) ||
-                      (reinterpret_cast<uintptr_t>(workspace) & 15)))
-        return VTL_HIP_ERR_INVALID_ARG;
-    if (M == 1 && gemv_applies(X, Wq, N, K) && !tuning().no_fused_decode) {
-        // a single token: quantized inside the matrix-vector kernel, one launch instead of two
-        // (N = 14336, K = 4096: 9.5 us against 12.8 us).  The workspace stays unused.
-        // VTL_HIP_NO_FUSED_DECODE forces the two-launch path (tests).
-        GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
-        return launch_gemv<true, true>(g, current_stream());
-    }
-    const int fused = launch_ragged_rows(X, K, Wq, K, sw, bias, Y, M, N, relu);
-    if (fused >= 0)
-        return fused;
-    if (gemv_rows_applies(X, Wq, M, N, K) && gemv_rows_fused_quant_faster(M, N, K) && !tuning().no_fused_decode) {
-        // a few tokens and short rows: same, each workgroup quantizes the rows itself
-        GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
-        return launch_gemv_rows<true, true>(g, current_stream());
-    }
-    const bool staged = stage_inside_launch_faster(M, N, K, gemv_rows_applies(X, Wq, M, N, K) && gemv_rows_faster(M, N, K, true)) &&
-                        aligned16(X) && aligned16(Wq) && tuning().gemm_config < 0 && !tuning().no_fused_decode;
-    if (!workspace) {   // no caller scratch: stage in the library's own buffer
-        workspace = vtlhip::library_workspace(vtl_hip_linear_f32_dynquant_workspace(M, K), 1);
-        if (!workspace)
-            return vtlhip::workspace_status();
-    }
-    int8_t *xq = reinterpret_cast<int8_t *>(workspace);
-    const size_t codes = (((size_t)M * (size_t)K) + 255) & ~(size_t)255;
-    float *sx = reinterpret_cast<float *>(reinterpret_cast<char *>(workspace) + codes);
-    if (staged && (reinterpret_cast<uintptr_t>(workspace) & 127) == 0) {
-        // a few tokens: quantized inside the weight-streaming launch (N = 14336, K = 4096, M = 8:
-        // 14.4 us against 16.0 us).  Its workgroups read the staging buffer as soon as the rows
-        // are counted and rely on no cache holding an older copy of those lines, which holds
-        // when nothing else shares them: the buffer starts on a cache line (anything from
-        // vtl_hip_malloc does) and its size is a whole number of them.
-        GemmArgs g{xq, Wq, Y, sx, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
-        g.stage_codes = xq;
-        g.stage_scales = sx;
-        bool launched = false;
-        st = launch_skinny_staged(g, current_stream(), launched);
-        if (launched || st != VTL_HIP_OK)
-            return st;
-    }
-    st = launch_quantize_rows(X, M, K, xq, sx, current_stream());
-    if (st != VTL_HIP_OK)
-        return st;
-    GemmArgs g{xq, Wq, Y, sx, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, nullptr, 0};
-    return launch_gemm<true>(g, current_stream());
+    return linear_f32_dynquant(X, Wq, sw, bias, Y, M, N, K, relu, workspace, workspace_bytes, nullptr);
 }
 
 int vtl_hip_linear_f32_dynquant_noalloc(const float *X, const int8_t *Wq, const float *sw, const float *bias,

@@ -74,21 +74,34 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
     Scratch codes, scales, next_codes, next_scales;
     const float *x = nullptr;              // the f32 rows, or null while the activations are codes
     int i = 0;
-    if (count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR) {
-        // A quantizer in front takes the input over the link itself: 64 x 784, per tensor, 4 us less than
-        // behind an upload.  Rows that are no whole vectors are read twice, which still is no slower
-        // (forward of 200 x 1001 56.9 against 61.4 us, 64 x 1023 37.9 and 39.3, 64 x 2047 and 64 x 4095 level).
-        // The launches for a few rows with a scale each read it in every workgroup: not those.
-        const bool direct = !layers[0].per_channel || rows > kFewRows;
-        HostInput input;
-        if (direct && input.stage(x_host, in_bytes)) {
+    // the last layer writes y itself, unless a ReLU of its own comes behind it
+    HostResult result;
+    const size_t out_bytes = (size_t)rows * (size_t)out_cols * sizeof(float);
+    const bool ends_linear = count > 0 && (layers[count - 1].kind == VTL_HIP_LAYER_LINEAR ||
+                                           (count > 1 && layers[count - 2].kind == VTL_HIP_LAYER_LINEAR));
+    float *const y = ends_linear ? static_cast<float *>(result.begin(y_host, out_bytes)) : nullptr;
+    HostInput input;
+    // (32 KiB is what the kernels that quantize in every workgroup take at most; near it the eight XCDs' transfers
+    // cost what an upload does)
+    const bool upload_first = rows <= 8 && in_bytes > ((size_t)20 << 10) && in_bytes <= ((size_t)32 << 10);
+    if (count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR && !(upload_first && layers[0].per_channel) &&
+        input.stage(x_host, in_bytes)) {
+        // The first launch takes the input over the link itself: 64 x 784, per tensor, 4 us less than behind an
+        // upload.  Rows that are no whole vectors are read twice, which still is no slower (forward of 200 x 1001
+        // 56.9 against 61.4 us, 64 x 1023 37.9 and 39.3, 64 x 2047 and 64 x 4095 level).  The launches for
+        // a few rows read them in every workgroup, out of the L2 but for the first of each XCD: 0 to 2.6 us more than from
+        // device memory for a row of up to 4096, 10 for 32 such rows (read once), where the upload takes 3 and 13 and a
+        // launch of its own.
+        x = static_cast<const float *>(input.data);
+        if (!layers[0].per_channel || rows > kFewRows) {
             VTL_STEP(codes.take((size_t)rows * (size_t)cols));
             VTL_STEP(scales.take((layers[0].per_channel ? (size_t)rows : 1) * sizeof(float)));
-            VTL_STEP(vtl_hip_quantize_f32_i8(static_cast<const float *>(input.data), rows, cols, layers[0].per_channel,
-                                             codes.as<int8_t>(), scales.as<float>()));
+            VTL_STEP(vtl_hip_quantize_f32_i8(x, rows, cols, layers[0].per_channel, codes.as<int8_t>(), scales.as<float>()));
+            x = nullptr;
+            input.release();
         }
     }
-    if (!codes.ptr) {
+    if (!codes.ptr && !x) {
         VTL_STEP(cur.take(in_bytes));
         VTL_STEP(vtl_hip_upload(cur.ptr, x_host, in_bytes));
         x = cur.as<float>();
@@ -103,15 +116,22 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
         const int n = l.out_features;
         const bool relu = i + 1 < count && layers[i + 1].kind == VTL_HIP_LAYER_RELU;
         i += relu ? 2 : 1;
+        const bool last = y && i == count;
         // the next layer takes codes as well
         const bool feeds = l.per_channel && rows > kFewRows && i < count && layers[i].kind == VTL_HIP_LAYER_LINEAR &&
                            layers[i].per_channel;
         if (x && l.per_channel && !feeds) {
-            VTL_STEP(next.take((size_t)rows * (size_t)n * sizeof(float)));
+            if (!last)
+                VTL_STEP(next.take((size_t)rows * (size_t)n * sizeof(float)));
             const size_t need = vtl_hip_linear_f32_dynquant_workspace(rows, cols);
             Scratch work;
             VTL_STEP(work.take(need));
-            VTL_STEP(vtl_hip_layer_f32(&l, x, next.as<float>(), rows, relu, work.ptr, need));
+            VTL_STEP(layer_f32(l, x, last ? y : next.as<float>(), rows, relu, work.ptr, need, last ? &result : nullptr));
+            if (input.data) {
+                input.release();
+                if (result.attached())
+                    result.input_released();
+            }
             cur.swap(next);
             x = cur.as<float>();
             cols = n;
@@ -131,27 +151,19 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
             codes.swap(next_codes);
             scales.swap(next_scales);
         } else {
-            VTL_STEP(cur.take((size_t)rows * (size_t)n * sizeof(float)));
-            VTL_STEP(layer_linear_i8_f32(l, codes.as<int8_t>(), scales.as<float>(), cur.as<float>(), rows, relu));
+            if (!last)
+                VTL_STEP(cur.take((size_t)rows * (size_t)n * sizeof(float)));
+            VTL_STEP(layer_linear_i8_f32(l, codes.as<int8_t>(), scales.as<float>(), last ? y : cur.as<float>(), rows, relu,
+                                         last ? &result : nullptr));
             x = cur.as<float>();
         }
         cols = n;
     }
-    return vtl_hip_memcpy_d2h(y_host, cur.ptr, (size_t)rows * (size_t)out_cols * sizeof(float));
+    return y ? result.finish() : vtl_hip_memcpy_d2h(y_host, cur.ptr, out_bytes);
 }
 
-template <typename T>
-struct Ops;
-template <>
-struct Ops<float> {
-    static constexpr auto matmul = vtl_hip_matmul_f32;
-    static constexpr auto backward = vtl_hip_linear_backward_f32;
-};
-template <>
-struct Ops<double> {
-    static constexpr auto matmul = vtl_hip_matmul_f64;
-    static constexpr auto backward = vtl_hip_linear_backward_f64;
-};
+int colsum(const float *x, int64_t rows, int64_t cols, float *out) { return vtl_hip_colsum_f32(x, rows, cols, out); }
+int colsum(const double *x, int64_t rows, int64_t cols, double *out) { return vtl_hip_colsum_f64(x, rows, cols, out); }
 
 template <typename T>
 int upload(Scratch &to, const T *host, size_t count)
@@ -172,9 +184,15 @@ int matmul_host(const T *a, const T *b, T *c, int m, int n, int k)
     Scratch da, db, dc;
     VTL_STEP(upload(da, a, (size_t)m * (size_t)k));
     VTL_STEP(upload(db, b, (size_t)k * (size_t)n));
-    VTL_STEP(dc.take((size_t)m * (size_t)n * sizeof(T)));
-    VTL_STEP(Ops<T>::matmul(da.as<T>(), db.as<T>(), dc.as<T>(), m, n, k, 0, 0));
-    return vtl_hip_memcpy_d2h(c, dc.ptr, (size_t)m * (size_t)n * sizeof(T));
+    const size_t bytes = (size_t)m * (size_t)n * sizeof(T);
+    HostResult result;
+    if (T *out = static_cast<T *>(result.begin(c, bytes))) {
+        VTL_STEP(matmul_to(&result, da.as<T>(), db.as<T>(), out, m, n, k, 0));
+        return result.finish();
+    }
+    VTL_STEP(dc.take(bytes));
+    VTL_STEP(matmul_to(nullptr, da.as<T>(), db.as<T>(), dc.as<T>(), m, n, k, 0));
+    return vtl_hip_memcpy_d2h(c, dc.ptr, bytes);
 }
 
 template <typename T>
@@ -184,23 +202,62 @@ int linear_backward_host(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
         return VTL_HIP_ERR_INVALID_ARG;
     const size_t mn = (size_t)m * (size_t)n, mk = (size_t)m * (size_t)k, nk = (size_t)n * (size_t)k;
     Scratch dev_grad, dev_x, dev_w, dev_dx, dev_dw, dev_db;
+    if (mn == 0)
+        return VTL_HIP_ERR_INVALID_ARG;
+    // dW is computed, and on its way to the host, while the host copies W for the upload behind it
+    struct Gradient {
+        T *host;
+        size_t bytes;
+        Scratch &dev;
+        T *out = nullptr;
+        bool direct = false;
+        int take(HostResult &result)
+        {
+            if (!host || bytes == 0)
+                return VTL_HIP_OK;
+            out = static_cast<T *>(result.begin(host, bytes));
+            direct = out != nullptr;
+            if (!direct) {
+                VTL_STEP(dev.take(bytes));
+                out = dev.as<T>();
+            }
+            return VTL_HIP_OK;
+        }
+    };
+    HostResult result;
+    Gradient gw = {dw, nk * sizeof(T), dev_dw}, gx = {dx, mk * sizeof(T), dev_dx}, gb = {db, (size_t)n * sizeof(T), dev_db};
+    VTL_STEP(gw.take(result));
+    VTL_STEP(gx.take(result));
+    VTL_STEP(gb.take(result));
     VTL_STEP(upload(dev_grad, grad, mn));
-    if (dw)
+    if (gb.out && !gx.out)
+        VTL_STEP(colsum(dev_grad.as<T>(), m, n, gb.out));
+    if (gw.out) {   // [N,K] = grad^T[N,M] . x[M,K]
         VTL_STEP(upload(dev_x, x, mk));
-    if (dx)
+        VTL_STEP(matmul_to(gw.direct && !gx.out ? &result : nullptr, dev_grad.as<T>(), dev_x.as<T>(), gw.out, n, k, m, 1));
+    }
+    if (gx.out) {   // [M,K] = grad[M,N] . W[N,K]
+        if (gb.out)
+            VTL_STEP(colsum(dev_grad.as<T>(), m, n, gb.out));
         VTL_STEP(upload(dev_w, w, nk));
-    if (dx)
-        VTL_STEP(dev_dx.take(mk * sizeof(T)));
-    if (dw)
-        VTL_STEP(dev_dw.take(nk * sizeof(T)));
-    if (db)
-        VTL_STEP(dev_db.take((size_t)n * sizeof(T)));
-    VTL_STEP(Ops<T>::backward(dev_grad.as<T>(), dev_x.as<T>(), dev_w.as<T>(), dev_dx.as<T>(), dev_dw.as<T>(),
-                              dev_db.as<T>(), m, n, k));
-    void *const host[3] = {dx, dw, db};
-    const void *const dev[3] = {dev_dx.ptr, dev_dw.ptr, dev_db.ptr};
-    const size_t bytes[3] = {dx ? mk * sizeof(T) : 0, dw ? nk * sizeof(T) : 0, db ? (size_t)n * sizeof(T) : 0};
-    return vtl_hip_download(3, host, dev, bytes);
+        VTL_STEP(matmul_to(gx.direct ? &result : nullptr, dev_grad.as<T>(), dev_w.as<T>(), gx.out, m, k, n, 0));
+    }
+    const Gradient *all[3] = {&gw, &gx, &gb};
+    void *host[3];
+    const void *dev[3];
+    size_t bytes[3];
+    int count = 0;
+    bool direct = false;
+    for (const Gradient *g : all) {
+        direct = direct || g->direct;
+        if (g->out && !g->direct) {
+            host[count] = g->host;
+            dev[count] = g->out;
+            bytes[count++] = g->bytes;
+        }
+    }
+    VTL_STEP(vtl_hip_download(count, host, dev, bytes));
+    return direct ? result.finish() : VTL_HIP_OK;
 }
 
 }  // namespace

@@ -35,6 +35,8 @@ struct MatmulArgs {
     int relu;
     int k_per_split;    // k range of one grid.y slice (multiple of 16)
     double *partial;    // launches that slice K: [slices][M][N] unrounded sums, else nullptr
+    vtlhip::DoneSignal done;     // C is the memory of a whole host call's result
+    vtlhip::HostResult *result;  // host side only
 };
 
 template <typename T>
@@ -301,6 +303,27 @@ __device__ __forceinline__ void direct_fetch(T (&out)[2][4], const T *__restrict
     }
 }
 
+// Two neighbours of a row, aligned as one element is.
+__device__ __forceinline__ void store_pair(float *p, float a, float b, const vtlhip::DoneSignal &done)
+{
+    typedef float Two __attribute__((ext_vector_type(2), aligned(4)));
+    const Two v = {a, b};
+    if (done.flag)   // waited for in raise_when_last
+        asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1" ::"v"(p), "v"(v) : "memory");
+    else
+        *reinterpret_cast<Two *>(p) = v;
+}
+
+__device__ __forceinline__ void store_pair(double *p, double a, double b, const vtlhip::DoneSignal &done)
+{
+    typedef double Two __attribute__((ext_vector_type(2), aligned(8)));
+    const Two v = {a, b};
+    if (done.flag)
+        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(p), "v"(v) : "memory");
+    else
+        *reinterpret_cast<Two *>(p) = v;
+}
+
 // The tiles of a workgroup are WM x WN wave tiles of 32 x 16 * TN, K is cut over WK waves each.
 // Blocks are renumbered so that each of the 8 XCDs (own L2) works on a compact patch of tiles, eight
 // tile rows deep: with the plain order the rows that share a column panel of B run on different XCDs.
@@ -398,43 +421,58 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
     T *__restrict__ C = static_cast<T *>(g.C);
     const T *__restrict__ bias = static_cast<const T *>(g.bias);
     double *__restrict__ partial = g.partial ? g.partial + (int64_t)blockIdx.y * g.M * g.N : nullptr;
-    // value v of a lane: i = v / (4 TN), j = v / 4 % TN, e = v % 4
-    auto store = [&](int v, double s) {
+    // Value v of a lane: i = v / (4 TN), j = v / 4 % TN, e = v % 4.  Values v and v + 4 of an even j are
+    // neighbours in a row and stored together: whole lines of 16 lanes.
+    auto store = [&](int v, double s0, double s1) {
         const int j = (v >> 2) & (TN - 1);
-        const int r = m0 + 2 * (4 * (v & 3) + kq) + v / (4 * TN), c = n0 + 32 * (j >> 1) + 2 * r16 + (j & 1);
+        const int r = m0 + 2 * (4 * (v & 3) + kq) + v / (4 * TN), c = n0 + 32 * (j >> 1) + 2 * r16;
         if (r >= g.M || c >= g.N)
             return;
+        const bool both = c + 1 < g.N;
         if (partial) {
-            partial[(int64_t)r * g.N + c] = s;
+            partial[(int64_t)r * g.N + c] = s0;
+            if (both)
+                partial[(int64_t)r * g.N + c + 1] = s1;
             return;
         }
-        T y = (T)s;              // the one rounding to the tensor's type
-        if (bias)
-            y = y + bias[c];     // Tensor.add in the tensor's type
-        if (g.relu && y < T(0))
-            y = T(0);
-        C[(int64_t)r * g.N + c] = y;
+        T y[2] = {(T)s0, (T)s1};     // the one rounding to the tensor's type
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if (bias)
+                y[u] = y[u] + bias[u && both ? c + 1 : c];     // Tensor.add in the tensor's type
+            if (g.relu && y[u] < T(0))
+                y[u] = T(0);
+        }
+        T *to = C + ((int64_t)r * g.N + c);
+        if (both)
+            store_pair(to, y[0], y[1], g.done);
+        else
+            vtlhip::store_result(to, y[0], g.done);
     };
     if constexpr (WK == 1) {
 #pragma unroll
         for (int v = 0; v < V; ++v)
-            store(v, acc[v / (4 * TN)][(v >> 2) & (TN - 1)][v & 3]);
-        return;
+            if (!(v & 4))
+                store(v, acc[v / (4 * TN)][(v >> 2) & (TN - 1)][v & 3], acc[v / (4 * TN)][((v >> 2) & (TN - 1)) + 1][v & 3]);
+    } else {
+        // partial tiles, in the order of the registers
+#pragma unroll
+        for (int v = 0; v < V; ++v)
+            red[wave][v][lane] = acc[v / (4 * TN)][(v >> 2) & (TN - 1)][v & 3];
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < V / 2 / WK; ++u) {
+            const int pair = wk + WK * u, v = 8 * (pair >> 2) + (pair & 3);
+            double s0 = red[tile * WK][v][lane], s1 = red[tile * WK][v + 4][lane];
+#pragma unroll
+            for (int w = 1; w < WK; ++w) {
+                s0 += red[tile * WK + w][v][lane];
+                s1 += red[tile * WK + w][v + 4][lane];
+            }
+            store(v, s0, s1);
+        }
     }
-    // partial tiles, in the order of the registers
-#pragma unroll
-    for (int v = 0; v < V; ++v)
-        red[wave][v][lane] = acc[v / (4 * TN)][(v >> 2) & (TN - 1)][v & 3];
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < V / WK; ++u) {
-        const int v = wk + WK * u;
-        double s = red[tile * WK][v][lane];
-#pragma unroll
-        for (int w = 1; w < WK; ++w)
-            s += red[tile * WK + w][v][lane];
-        store(v, s);
-    }
+    vtlhip::raise_when_last(g.done);   // (a launch that leaves partial sums has no signal)
 }
 
 // Column sums with f64 accumulation: la.matmul(ones[1,M], grad) of
@@ -519,18 +557,19 @@ __global__ __launch_bounds__(256) void matmul_splitk_finalize_kernel(const Matmu
 {
     const int64_t total = (int64_t)g.M * g.N;
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= total)
-        return;
-    double s = 0.0;
-    for (int i = 0; i < splits; ++i)
-        s += g.partial[(int64_t)i * total + idx];
-    T y = (T)s;
-    const T *__restrict__ bias = static_cast<const T *>(g.bias);
-    if (bias)
-        y = y + bias[idx % g.N];
-    if (g.relu && y < T(0))
-        y = T(0);
-    static_cast<T *>(g.C)[idx] = y;
+    if (idx < total) {
+        double s = 0.0;
+        for (int i = 0; i < splits; ++i)
+            s += g.partial[(int64_t)i * total + idx];
+        T y = (T)s;
+        const T *__restrict__ bias = static_cast<const T *>(g.bias);
+        if (bias)
+            y = y + bias[idx % g.N];
+        if (g.relu && y < T(0))
+            y = T(0);
+        vtlhip::store_result(static_cast<T *>(g.C) + idx, y, g.done);
+    }
+    vtlhip::raise_when_last(g.done);
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
@@ -555,9 +594,11 @@ int launch_staged(const MatmulArgs &g, bool ta, bool tb, hipStream_t st)
 }
 
 template <typename T>
-int finalize_split(const MatmulArgs &g, int splits, hipStream_t st)
+int finalize_split(MatmulArgs g, int splits, hipStream_t st)
 {
     const int64_t blocks = ((int64_t)g.M * g.N + 255) / 256;
+    if (g.result)
+        g.result->attach(g.done, (unsigned)blocks);
     hipLaunchKernelGGL((matmul_splitk_finalize_kernel<T>), dim3((unsigned)blocks), dim3(256), 0, st, g, splits);
     return check_launch("matmul_splitk_finalize_kernel");
 }
@@ -626,13 +667,15 @@ Plan choose_plan(bool f64, int m, int n, int k, bool whole, bool may_slice)
 }
 
 template <typename T, int WM, int WN, int WK, int TN, bool CHECKED = false>
-int launch_direct_shape(const MatmulArgs &g, bool ta, bool tb, int slices, hipStream_t st)
+int launch_direct_shape(MatmulArgs g, bool ta, bool tb, int slices, hipStream_t st)
 {
     constexpr int BM = 32 * WM, BN = 16 * TN * WN;
     const int64_t tiles = (int64_t)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
     if (tiles > 0x7fffffff)
         return VTL_HIP_ERR_UNSUPPORTED;
     const dim3 grid((unsigned)tiles, (unsigned)slices), block(64 * WM * WN * WK);
+    if (g.result && slices == 1)
+        g.result->attach(g.done, grid.x);
     if (!ta && !tb)
         hipLaunchKernelGGL((matmul_f64acc_direct_kernel<T, WM, WN, WK, TN, false, false, CHECKED>), grid, block, 0, st, g);
     else if (!ta && tb)
@@ -701,7 +744,7 @@ int launch_direct(MatmulArgs g, bool ta, bool tb, Plan plan, bool alone, hipStre
 
 template <typename T>
 int matmul_impl(const T *a, const T *b, T *c, const T *bias, int m, int n, int k, int trans_a, int trans_b,
-                int relu)
+                int relu, vtlhip::HostResult *result = nullptr)
 {
     if (m < 0 || n < 0 || k < 0)
         return VTL_HIP_ERR_INVALID_ARG;
@@ -709,7 +752,8 @@ int matmul_impl(const T *a, const T *b, T *c, const T *bias, int m, int n, int k
         return VTL_HIP_OK;
     if (!c || (k > 0 && (!a || !b)))
         return VTL_HIP_ERR_INVALID_ARG;
-    MatmulArgs g;
+    MatmulArgs g = {};
+    g.result = result;
     g.A = a;
     g.B = b;
     g.C = c;
@@ -718,8 +762,6 @@ int matmul_impl(const T *a, const T *b, T *c, const T *bias, int m, int n, int k
     g.N = n;
     g.K = k;
     g.relu = relu;
-    g.k_per_split = 0;
-    g.partial = nullptr;
     // the staged kernel's loads and stores carry no bounds checks
     const bool whole = m % 128 == 0 && n % 128 == 0 && k % 32 == 0 && k > 0 && aligned16(a) && aligned16(b) &&
                        aligned16(c);
@@ -817,6 +859,20 @@ int linear_backward_impl(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
 }
 
 }  // namespace
+
+namespace vtlhip {
+
+int matmul_to(HostResult *result, const float *a, const float *b, float *c, int m, int n, int k, int trans_a)
+{
+    return matmul_impl<float>(a, b, c, nullptr, m, n, k, trans_a, 0, 0, result);
+}
+
+int matmul_to(HostResult *result, const double *a, const double *b, double *c, int m, int n, int k, int trans_a)
+{
+    return matmul_impl<double>(a, b, c, nullptr, m, n, k, trans_a, 0, 0, result);
+}
+
+}  // namespace vtlhip
 
 extern "C" {
 
