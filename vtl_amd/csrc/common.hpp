@@ -73,6 +73,9 @@ private:
     void *ring_ = nullptr;
 };
 
+// Two uploads as vtl_hip_upload makes them, which share their launches; false: to be made one by one.
+bool upload_two(void *dst0, const void *src0, size_t bytes0, void *dst1, const void *src1, size_t bytes1, int &status);
+
 // How a launch tells the host that its results are there: every workgroup counts itself when its stores are
 // complete, and the one that reaches the target raises the flag.  No flag: nothing to tell.
 struct DoneSignal {

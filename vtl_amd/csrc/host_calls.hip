@@ -173,6 +173,18 @@ int upload(Scratch &to, const T *host, size_t count)
 }
 
 template <typename T>
+int upload_both(Scratch &to0, const T *host0, size_t count0, Scratch &to1, const T *host1, size_t count1)
+{
+    VTL_STEP(to0.take(count0 * sizeof(T)));
+    VTL_STEP(to1.take(count1 * sizeof(T)));
+    int status = VTL_HIP_OK;
+    if (upload_two(to0.ptr, host0, count0 * sizeof(T), to1.ptr, host1, count1 * sizeof(T), status))
+        return status;
+    VTL_STEP(vtl_hip_upload(to0.ptr, host0, count0 * sizeof(T)));
+    return vtl_hip_upload(to1.ptr, host1, count1 * sizeof(T));
+}
+
+template <typename T>
 int matmul_host(const T *a, const T *b, T *c, int m, int n, int k)
 {
     if (m < 0 || n < 0 || k < 0)
@@ -182,8 +194,7 @@ int matmul_host(const T *a, const T *b, T *c, int m, int n, int k)
     if (!c || (k > 0 && (!a || !b)))
         return VTL_HIP_ERR_INVALID_ARG;
     Scratch da, db, dc;
-    VTL_STEP(upload(da, a, (size_t)m * (size_t)k));
-    VTL_STEP(upload(db, b, (size_t)k * (size_t)n));
+    VTL_STEP(upload_both(da, a, (size_t)m * (size_t)k, db, b, (size_t)k * (size_t)n));
     const size_t bytes = (size_t)m * (size_t)n * sizeof(T);
     HostResult result;
     if (T *out = static_cast<T *>(result.begin(c, bytes))) {
@@ -229,11 +240,13 @@ int linear_backward_host(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
     VTL_STEP(gw.take(result));
     VTL_STEP(gx.take(result));
     VTL_STEP(gb.take(result));
-    VTL_STEP(upload(dev_grad, grad, mn));
+    if (gw.out)
+        VTL_STEP(upload_both(dev_grad, grad, mn, dev_x, x, mk));
+    else
+        VTL_STEP(upload(dev_grad, grad, mn));
     if (gb.out && !gx.out)
         VTL_STEP(colsum(dev_grad.as<T>(), m, n, gb.out));
     if (gw.out) {   // [N,K] = grad^T[N,M] . x[M,K]
-        VTL_STEP(upload(dev_x, x, mk));
         VTL_STEP(matmul_to(gw.direct && !gx.out ? &result : nullptr, dev_grad.as<T>(), dev_x.as<T>(), gw.out, n, k, m, 1));
     }
     if (gx.out) {   // [M,K] = grad[M,N] . W[N,K]

@@ -74,19 +74,54 @@ struct Segment {
     unsigned head, tail; // single bytes before and after them
 };
 
-struct CopyArgs {
-    Segment seg[kMaxSegments];
-    int count;
+struct LinkSignals {
     DoneSignal done;
     unsigned *behind;    // flag of the launch before this one, which has ended by now, or nullptr
     unsigned behind_value;
     int to_host;         // the bytes have to be visible to the host when the flag is (else: the source is free)
 };
 
+struct CopyArgs {
+    Segment seg[kMaxSegments];
+    int count;
+    LinkSignals signals;
+};
+
+__device__ __forceinline__ void raise_behind(const LinkSignals &s)
+{
+    if (s.behind && blockIdx.x == 0 && threadIdx.x == 0)
+        __hip_atomic_store(s.behind, s.behind_value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// At the end of a workgroup whose pinned source has been read (or, to_host, whose bytes are there).
+__device__ __forceinline__ void raise_done(const LinkSignals &s)
+{
+    const DoneSignal &done = s.done;
+    if (!done.flag)
+        return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every load has returned, every store is acknowledged
+    __syncthreads();
+    if (threadIdx.x != 0)
+        return;
+    if (s.to_host) {
+        // one system-scope fence per workgroup covers the stores of all of its threads (they
+        // happen before it through the barrier); whoever counts last raises the flag
+        __threadfence_system();
+        const unsigned before = __hip_atomic_fetch_add(done.counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        if (before + 1 == done.target)
+            __hip_atomic_store(done.flag, done.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    } else {
+        // nothing to publish: the flag says that the pinned source has been read, which the
+        // returned loads are enough for (a fence would write the caches back at every chunk)
+        const unsigned before = __hip_atomic_fetch_add(done.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (before + 1 == done.target)
+            __hip_atomic_store(done.flag, done.value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 __global__ __launch_bounds__(512) void host_copy_kernel(const CopyArgs g)
 {
-    if (g.behind && blockIdx.x == 0 && threadIdx.x == 0)
-        __hip_atomic_store(g.behind, g.behind_value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    raise_behind(g.signals);
     const size_t first = (size_t)blockIdx.x * 512 + threadIdx.x, step = (size_t)gridDim.x * 512;
     for (int s = 0; s < g.count; s++) {
         const Segment &seg = g.seg[s];
@@ -110,27 +145,7 @@ __global__ __launch_bounds__(512) void host_copy_kernel(const CopyArgs g)
                 seg.dst[end + threadIdx.x] = seg.src[end + threadIdx.x];
         }
     }
-    const DoneSignal &done = g.done;
-    if (!done.flag)
-        return;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every load has returned, every store is acknowledged
-    __syncthreads();
-    if (threadIdx.x != 0)
-        return;
-    if (g.to_host) {
-        // one system-scope fence per workgroup covers the stores of all of its threads (they
-        // happen before it through the barrier); whoever counts last raises the flag
-        __threadfence_system();
-        const unsigned before = __hip_atomic_fetch_add(done.counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if (before + 1 == done.target)
-            __hip_atomic_store(done.flag, done.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    } else {
-        // nothing to publish: the flag says that the pinned source has been read, which the
-        // returned loads are enough for (a fence would write the caches back at every chunk)
-        const unsigned before = __hip_atomic_fetch_add(done.counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (before + 1 == done.target)
-            __hip_atomic_store(done.flag, done.value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
+    raise_done(g.signals);
 }
 
 Segment make_segment(void *dst, const void *src, size_t bytes)
@@ -165,20 +180,22 @@ struct Signal {
     unsigned arrived = 0, value = 0;
 
     DoneSignal next(unsigned blocks) const { return {counter, arrived + blocks, value + 1, flag}; }
-    void attach(CopyArgs &g, unsigned blocks, bool to_host)
+    void attach(LinkSignals &s, unsigned blocks, bool to_host)
     {
-        g.done = next(blocks);
-        g.to_host = to_host;
+        s.done = next(blocks);
+        s.to_host = to_host;
     }
     void launched(unsigned blocks)
     {
         arrived += blocks;
         value++;
     }
-    bool raised() const { return __atomic_load_n(flag, __ATOMIC_ACQUIRE) == value; }
+    bool raised() const { return reached(flag, value); }
+    static bool reached(const unsigned *flag, unsigned value)
+    {
+        return (int)(__atomic_load_n(flag, __ATOMIC_ACQUIRE) - value) >= 0;
+    }
 };
-
-int wait_signal(const Signal &s, hipStream_t st);
 
 __global__ void clear_counters_kernel(unsigned *p) { p[threadIdx.x] = 0; }
 
@@ -274,14 +291,14 @@ double seconds()
     return (double)t.tv_sec + 1e-9 * (double)t.tv_nsec;
 }
 
-// Waits for the last launch: its flag is polled for two milliseconds, then it is left to the
+// Waits for a launch: its flag is polled for two milliseconds, then it is left to the
 // runtime, which also reports what went wrong if the launch never ends well.
-int wait_signal(const Signal &s, hipStream_t st)
+int wait_flag(const unsigned *flag, unsigned value, hipStream_t st)
 {
     const double began = seconds();
     for (;;) {
         for (int i = 0; i < 64; i++) {
-            if (s.raised())
+            if (Signal::reached(flag, value))
                 return VTL_HIP_OK;
             __builtin_ia32_pause();
         }
@@ -289,7 +306,7 @@ int wait_signal(const Signal &s, hipStream_t st)
             break;
     }
     VTL_HIP_TRY(hipStreamSynchronize(st));
-    return s.raised() ? VTL_HIP_OK : record_hip_error(hipErrorUnknown, "host copy ended without its flag");
+    return Signal::reached(flag, value) ? VTL_HIP_OK : record_hip_error(hipErrorUnknown, "host copy ended without its flag");
 }
 
 // Small uploads enqueued so far and those known to have been read, per device: what a download has
@@ -303,7 +320,7 @@ UploadCount g_uploads[kMaxDevices];
 // Waits for a lane's flag behind which `before` uploads were enqueued.
 int wait_behind(Lane *lane, uint64_t before, bool one_stream, hipStream_t st)
 {
-    const int rc = wait_signal(lane->signal, st);
+    const int rc = wait_flag(lane->signal.flag, lane->signal.value, st);
     if (rc == VTL_HIP_OK && one_stream) {
         UploadCount &uploads = g_uploads[lane->device];
         uint64_t seen = uploads.done.load(std::memory_order_relaxed);
@@ -319,7 +336,7 @@ int copy_and_wait(CopyArgs &g, size_t bytes, Lane *lane, hipStream_t st)
     const bool one_stream = single_stream();
     const uint64_t before = g_uploads[lane->device].enqueued.load(std::memory_order_acquire);
     const unsigned blocks = copy_blocks(bytes);
-    lane->signal.attach(g, blocks, true);
+    lane->signal.attach(g.signals, blocks, true);
     hipLaunchKernelGGL(host_copy_kernel, dim3(blocks), dim3(512), 0, st, g);
     int rc = check_launch("host_copy_kernel");
     if (rc != VTL_HIP_OK)
@@ -345,35 +362,41 @@ struct Ring {
     int slot = 0;            // slot that small uploads fill
     size_t used = 0;         // bytes of it that are taken
 
+    // What says that a slot is free again: a launch may read several, and raises the flag of its first.
+    struct Gate {
+        int signal;
+        unsigned value;
+    } gate[kSlots] = {};
+
     char *at(int i) { return base + (size_t)i * kSlotStride; }
-    bool is_free(int i) const { return signal[i].raised(); }
-    int wait(int i, hipStream_t st) { return wait_signal(signal[i], st); }
-    // A chunk on its way up, and no launch yet behind it that would raise its slot's flag.
+    bool is_free(int i) const { return Signal::reached(signal[gate[i].signal].flag, gate[i].value); }
+    int wait(int i, hipStream_t st) { return wait_flag(signal[gate[i].signal].flag, gate[i].value, st); }
+    // Slots on their way up, and no launch yet behind theirs that would raise their flag.
     int waiting = -1;
 
-    // Chunks on the way up: the next launch on the stream raises the flag of this one, which has ended
-    // when that one begins (counting workgroups and a flag of its own hold a kernel back for
-    // about 1.5 us, on a link that a MiB keeps busy for 18).
-    int launch_up(int i, void *dst, const void *src, size_t bytes, hipStream_t st)
+    // A launch that reads the slots first .. first + count - 1.  On the way up the next launch on the
+    // stream raises their flag, which begins when this one has ended (counting workgroups and a flag of its own
+    // hold a launch back for about 1.5 us, on a link that a MiB keeps busy for 18); only the last launch (`own`) counts.
+    LinkSignals signals_for(int first, unsigned blocks, bool own, bool to_host)
     {
-        CopyArgs g = {};
-        g.seg[0] = make_segment(dst, src, bytes);
-        g.count = 1;
-        raise_waiting(g);
-        hipLaunchKernelGGL(host_copy_kernel, dim3(copy_blocks(bytes < kSmall ? bytes : kSmall - 1)), dim3(512), 0, st, g);
-        const int rc = check_launch("host_copy_kernel");
-        if (rc == VTL_HIP_OK) {
-            signal[i].value++;
-            waiting = i;
-        }
-        return rc;
-    }
-    void raise_waiting(CopyArgs &g) const
-    {
+        LinkSignals s = {};
         if (waiting >= 0) {
-            g.behind = signal[waiting].flag;
-            g.behind_value = signal[waiting].value;
+            s.behind = signal[waiting].flag;
+            s.behind_value = signal[waiting].value;
         }
+        if (own)
+            signal[first].attach(s, blocks, to_host);
+        return s;
+    }
+    void launched(int first, int count, unsigned blocks, bool own)
+    {
+        if (own)
+            signal[first].launched(blocks);
+        else
+            signal[first].value++;
+        waiting = own ? -1 : first;
+        for (int i = 0; i < count; i++)
+            gate[(first + i) % kSlots] = {first, signal[first].value};
     }
     // After a failure nothing is under way any more and the host raises the flag.
     void give_up(hipStream_t st)
@@ -388,19 +411,16 @@ struct Ring {
     int launch(int i, void *dst, const void *src, size_t bytes, bool to_host, hipStream_t st)
     {
         CopyArgs g = {};
-        raise_waiting(g);
         if (bytes) {
             g.seg[0] = make_segment(dst, src, bytes);
             g.count = 1;
         }
         const unsigned blocks = copy_blocks(bytes < kSmall || to_host ? bytes : kSmall - 1);
-        signal[i].attach(g, blocks, to_host);
+        g.signals = signals_for(i, blocks, true, to_host);
         hipLaunchKernelGGL(host_copy_kernel, dim3(blocks), dim3(512), 0, st, g);
         const int rc = check_launch("host_copy_kernel");
-        if (rc == VTL_HIP_OK) {
-            signal[i].launched(blocks);
-            waiting = -1;
-        }
+        if (rc == VTL_HIP_OK)
+            launched(i, 1, blocks, true);
         return rc;
     }
     // Closes the slot that small uploads were filling; the next transfer starts in a slot of its own.
@@ -586,53 +606,195 @@ struct Crew {
     }
 };
 
-int launch_plain_copy(void *dst, const void *src, size_t bytes, hipStream_t st)
-{
-    CopyArgs g = {};
-    g.seg[0] = make_segment(dst, src, bytes);
-    g.count = 1;
-    hipLaunchKernelGGL(host_copy_kernel, dim3(copy_blocks(bytes < kSmall ? bytes : kSmall - 1)), dim3(512), 0, st, g);
-    return check_launch("host_copy_kernel");
-}
+// Room for small uploads of `bytes` in all (with the gaps that put_small leaves), behind those before them in
+// the current slot (one flag per slot and not one per upload).
+size_t small_room(size_t bytes) { return (bytes + 15 + 255) & ~(size_t)255; }
 
-// Copies a small upload's bytes into the ring, behind those of the uploads before it in the current
-// slot (one flag per slot and not one per upload), `skew` bytes past a 16-byte boundary.
-int stage_small(Ring *r, const void *src, size_t bytes, size_t skew, hipStream_t st, char *&staged)
+int open_small(Ring *r, size_t room, hipStream_t st)
 {
-    const size_t take = (bytes + skew + 255) & ~(size_t)255;
     int rc = VTL_HIP_OK;
     // When a download has waited for everything so far, the slot is filled from its start again:
     // staging memory that is still in the host's caches.
     if (single_stream() && r->uploads->done.load(std::memory_order_acquire) ==
                                r->uploads->enqueued.load(std::memory_order_relaxed))
         r->used = 0;
-    if (r->used + take > kSlotBytes)
+    if (r->used + room > kSlotBytes)
         rc = r->close(st);
     if (rc == VTL_HIP_OK && r->used == 0)
         rc = r->wait(r->slot, st);
-    if (rc != VTL_HIP_OK)
-        return rc;
-    staged = r->at(r->slot) + r->used + skew;
-    memcpy(staged, src, bytes);
-    r->used += take;
-    return VTL_HIP_OK;
+    return rc;
 }
 
-int upload_small(Ring *r, void *dst, const void *src, size_t bytes, hipStream_t st)
+// Copies bytes there, `skew` past a 16-byte boundary.
+char *put_small(Ring *r, const void *src, size_t bytes, size_t skew)
 {
-    char *staged = nullptr;
-    int rc = stage_small(r, src, bytes, reinterpret_cast<uintptr_t>(dst) & 15, st, staged);
-    if (rc == VTL_HIP_OK)
-        rc = launch_plain_copy(dst, staged, bytes, st);
+    char *staged = r->at(r->slot) + r->used + skew;
+    memcpy(staged, src, bytes);
+    r->used += small_room(bytes);
+    return staged;
+}
+
+// One upload of several.
+struct Source {
+    void *dst;
+    const void *src;
+    size_t bytes;
+};
+
+// Small uploads, kSmall bytes in all at most, in one launch.
+int upload_small(Ring *r, const Source *from, int count, hipStream_t st)
+{
+    size_t bytes = 0, room = 0;
+    for (int i = 0; i < count; i++) {
+        bytes += from[i].bytes;
+        room += small_room(from[i].bytes);
+    }
+    int rc = open_small(r, room, st);
+    if (rc != VTL_HIP_OK)
+        return rc;
+    CopyArgs g = {};
+    for (int i = 0; i < count; i++)
+        g.seg[g.count++] = make_segment(from[i].dst,
+                                        put_small(r, from[i].src, from[i].bytes, reinterpret_cast<uintptr_t>(from[i].dst) & 15),
+                                        from[i].bytes);
+    hipLaunchKernelGGL(host_copy_kernel, dim3(copy_blocks(bytes < kSmall ? bytes : kSmall - 1)), dim3(512), 0, st, g);
+    rc = check_launch("host_copy_kernel");
     if (rc == VTL_HIP_OK)
         r->uploads->enqueued.fetch_add(1, std::memory_order_acq_rel);
     return rc;
 }
 
-// A large transfer's chunks: small ones first, so that the link does not wait for the host's first
-// copy, then twice as large each up to a slot, because every launch costs the link about 3 us.
-constexpr size_t kFirstChunk = (size_t)256 << 10;
+// What goes up in pieces of at most a slot, and the launches that carry up to kMaxSegments pieces each: small ones first, so
+// that the link does not wait for the host's first copy, then larger ones, because a launch costs the link about 3 us (one slot
+// a launch 53.9 GB/s, four 56.1).  Beyond a slot half as large again each: the host copies what a launch carries
+// during the one before, and is not twice as fast as the link.  (180 MB in launches of one slot 3310 us, so 3170; 2 MiB of two
+// operands 88 -> 80.)
+constexpr size_t kFirstLaunch = (size_t)512 << 10;
 
+struct Pieces {
+    struct Piece {
+        const char *src;
+        char *dst;
+        size_t bytes;
+        std::atomic<int> left{0};
+        bool last_of_launch;
+        size_t skew() const { return reinterpret_cast<uintptr_t>(dst) & 15; }
+    };
+    std::unique_ptr<Piece[]> piece;
+    int count = 0;
+
+    Pieces(const Source *from, int sources)
+    {
+        for (int pass = 0; pass < 2; pass++) {
+            size_t ahead = 0, launch = kFirstLaunch, room = launch;
+            for (int s = 0; s < sources; s++)
+                ahead += from[s].bytes;
+            int n = 0, in_launch = 0;
+            for (int s = 0; s < sources; s++)
+                for (size_t at = 0; at < from[s].bytes;) {
+                    if (in_launch == 0 && ahead < launch + launch / 2)   // no small launch at the end
+                        room = ahead;
+                    size_t take = from[s].bytes - at;
+                    if (take > kSlotBytes)
+                        take = kSlotBytes;
+                    if (take > room)
+                        take = room;
+                    if (pass) {
+                        Piece &p = piece[n];
+                        p.src = static_cast<const char *>(from[s].src) + at;
+                        p.dst = static_cast<char *>(from[s].dst) + at;
+                        p.bytes = take;
+                    }
+                    at += take;
+                    ahead -= take;
+                    room -= take;
+                    n++;
+                    in_launch++;
+                    const bool end = room == 0 || in_launch == kMaxSegments || ahead == 0;
+                    if (pass)
+                        piece[n - 1].last_of_launch = end;
+                    if (end) {
+                        launch = launch < kSlotBytes ? 2 * launch : (launch + launch / 2) & ~(size_t)4095;
+                        if (launch > kMaxSegments * kSlotBytes)
+                            launch = kMaxSegments * kSlotBytes;
+                        room = launch;
+                        in_launch = 0;
+                    }
+                }
+            if (!pass)
+                piece.reset(new Piece[(size_t)n]);
+            count = n;
+        }
+    }
+};
+
+// The host threads fill slots while the link empties the ones before them.  launch(first, n, slot of the
+// first, last): pieces first .. first + n - 1, in as many consecutive slots.
+template <typename Launch>
+int send_pieces(Ring *r, Pieces &c, hipStream_t st, Launch launch)
+{
+    int rc = r->close(st);
+    if (rc != VTL_HIP_OK)
+        return rc;
+    const int n = c.count, s0 = r->slot;
+    Crew &crew = Crew::instance();
+    crew.begin();
+    int pushed = 0, issued = 0;
+    while (issued < n && rc == VTL_HIP_OK) {
+        int end = issued;
+        while (!c.piece[end++].last_of_launch)
+            ;
+        // what this launch carries, and as much of the next ones as there are free slots for
+        while (pushed < n && pushed - issued < kSlots) {
+            const int slot = (s0 + pushed) % kSlots;
+            if (!r->is_free(slot)) {
+                if (pushed >= end)
+                    break;
+                if ((rc = r->wait(slot, st)) != VTL_HIP_OK)
+                    break;
+            }
+            Pieces::Piece &p = c.piece[pushed];
+            crew.push(r->at(slot) + p.skew(), p.src, p.bytes, p.left);
+            pushed++;
+        }
+        for (int i = issued; i < end && rc == VTL_HIP_OK; i++)
+            crew.finish(c.piece[i].left);
+        if (rc == VTL_HIP_OK)
+            rc = launch(issued, end - issued, (s0 + issued) % kSlots, end == n);
+        if (rc == VTL_HIP_OK)
+            issued = end;
+    }
+    for (int i = 0; i < pushed; i++)   // after a failure: nothing may still write to the slots
+        crew.finish(c.piece[i].left);
+    if (rc != VTL_HIP_OK)
+        r->give_up(st);
+    crew.end();
+    r->slot = (s0 + n) % kSlots;
+    return rc;
+}
+
+int upload_large(Ring *r, const Source *from, int count, hipStream_t st)
+{
+    Pieces c(from, count);
+    return send_pieces(r, c, st, [&](int first, int n, int slot, bool last) {
+        CopyArgs g = {};
+        size_t bytes = 0;
+        for (int i = 0; i < n; i++) {
+            const Pieces::Piece &p = c.piece[first + i];
+            g.seg[g.count++] = make_segment(p.dst, r->at((slot + i) % kSlots) + p.skew(), p.bytes);
+            bytes += p.bytes;
+        }
+        const unsigned blocks = copy_blocks(bytes < kSmall ? bytes : kSmall - 1);
+        g.signals = r->signals_for(slot, blocks, last, false);
+        hipLaunchKernelGGL(host_copy_kernel, dim3(blocks), dim3(512), 0, st, g);
+        const int rc = check_launch("host_copy_kernel");
+        if (rc == VTL_HIP_OK)
+            r->launched(slot, n, blocks, last);
+        return rc;
+    });
+}
+
+// A large transfer the other way: pieces of a MiB, then twice as large each up to a slot.
 struct Chunks {
     struct Chunk {
         size_t at, bytes;
@@ -663,50 +825,6 @@ struct Chunks {
     }
 };
 
-// The host threads fill slots while the link empties the ones before them.
-int upload_large(Ring *r, char *dst, const char *src, size_t bytes, hipStream_t st)
-{
-    int rc = r->close(st);
-    if (rc != VTL_HIP_OK)
-        return rc;
-    const size_t skew = reinterpret_cast<uintptr_t>(dst) & 15;
-    Chunks c(bytes, kFirstChunk);
-    const int n = c.count, s0 = r->slot;
-    Crew &crew = Crew::instance();
-    crew.begin();
-    int pushed = 0, issued = 0;
-    while (issued < n && rc == VTL_HIP_OK) {
-        while (pushed < n && pushed - issued < kSlots) {
-            const int slot = (s0 + pushed) % kSlots;
-            if (!r->is_free(slot)) {
-                if (pushed > issued)
-                    break;
-                if ((rc = r->wait(slot, st)) != VTL_HIP_OK)
-                    break;
-            }
-            crew.push(r->at(slot) + skew, src + c.chunk[pushed].at, c.chunk[pushed].bytes, c.chunk[pushed].left);
-            pushed++;
-        }
-        if (rc != VTL_HIP_OK)
-            break;
-        Chunks::Chunk &k = c.chunk[issued];
-        crew.finish(k.left);
-        const int slot = (s0 + issued) % kSlots;
-        if (issued + 1 < n)
-            rc = r->launch_up(slot, dst + k.at, r->at(slot) + skew, k.bytes, st);
-        else
-            rc = r->launch(slot, dst + k.at, r->at(slot) + skew, k.bytes, false, st);
-        issued++;
-    }
-    for (int i = issued; i < pushed; i++)   // after a failure: nothing may still write to the slots
-        crew.finish(c.chunk[i].left);
-    if (rc != VTL_HIP_OK)
-        r->give_up(st);
-    crew.end();
-    r->slot = (s0 + n) % kSlots;
-    return rc;
-}
-
 // The other way round, into memory that the device cannot write itself.
 int download_large(Ring *r, char *dst, const char *src, size_t bytes, hipStream_t st)
 {
@@ -714,7 +832,7 @@ int download_large(Ring *r, char *dst, const char *src, size_t bytes, hipStream_
     if (rc != VTL_HIP_OK)
         return rc;
     const size_t skew = reinterpret_cast<uintptr_t>(src) & 15;
-    Chunks c(bytes, kFirstChunk * 4);
+    Chunks c(bytes, (size_t)1 << 20);
     const int n = c.count, s0 = r->slot;
     Crew &crew = Crew::instance();
     crew.begin();
@@ -768,16 +886,32 @@ try {
     if (!r)
         return false;
     r->lock.lock();
-    char *staged = nullptr;
-    if (stage_small(r, src, bytes, 0, current_stream(), staged) != VTL_HIP_OK) {
+    if (open_small(r, small_room(bytes), current_stream()) != VTL_HIP_OK) {
         r->lock.unlock();
         return false;
     }
     ring_ = r;
-    data = staged;
+    data = put_small(r, src, bytes, 0);
     return true;
 } catch (const std::exception &) {
     return false;
+}
+
+bool upload_two(void *dst0, const void *src0, size_t bytes0, void *dst1, const void *src1, size_t bytes1, int &status)
+try {
+    if (!bytes0 || !bytes1 || !single_stream())
+        return false;
+    const OwnerDevice owner(dst0, dst1);
+    Ring *r = owner.kernels() ? ring_of_current_device() : nullptr;
+    if (!r)
+        return false;
+    const Source from[2] = {{dst0, src0, bytes0}, {dst1, src1, bytes1}};
+    std::lock_guard<std::mutex> hold(r->lock);
+    status = bytes0 + bytes1 <= kSmall ? upload_small(r, from, 2, current_stream()) : upload_large(r, from, 2, current_stream());
+    return true;
+} catch (const std::exception &) {
+    status = VTL_HIP_ERR_OUT_OF_MEMORY;
+    return true;
 }
 
 // Results that are written over the link as they are computed: up to here no slower than a copy behind the
@@ -825,8 +959,8 @@ int HostResult::finish()
     int rc = VTL_HIP_OK;
     if (!attached_) {
         CopyArgs g = {};
-        attach(g.done, 1);
-        g.to_host = 1;
+        attach(g.signals.done, 1);
+        g.signals.to_host = 1;
         hipLaunchKernelGGL(host_copy_kernel, dim3(1), dim3(64), 0, st, g);
         rc = check_launch("host_copy_kernel");
     }
@@ -952,9 +1086,8 @@ try {
         Ring *r = ring_of_current_device();
         if (r) {
             std::lock_guard<std::mutex> hold(r->lock);
-            const int rc = bytes <= kSmall ? upload_small(r, dst_device, src_host, bytes, st)
-                                           : upload_large(r, static_cast<char *>(dst_device),
-                                                          static_cast<const char *>(src_host), bytes, st);
+            const Source from = {dst_device, src_host, bytes};
+            const int rc = bytes <= kSmall ? upload_small(r, &from, 1, st) : upload_large(r, &from, 1, st);
             if (rc != VTL_HIP_OK || one_stream)
                 return rc;
             // the ring's slots are shared by all streams
