@@ -104,6 +104,30 @@ def test_split_k_paths(hip, dt, knobs):
         t.release()
 
 
+# (the shapes that only f64 with K along both operands' rows has, and the others at the edges of the largest tiles;
+# columns beyond a lane's 32-bit offset are checked load by load)
+@pytest.mark.parametrize("shape", ["4", "5", "6"])
+@pytest.mark.parametrize("mnk", [(64, 64, 16), (65, 63, 113), (129, 130, 47), (127, 2, 33), (2, 129, 300), (200, 70, 64),
+                                 (3, (1 << 22) + 1, 5)])
+def test_large_shapes_at_their_edges(hip, shape, mnk, knobs):
+    knobs.setenv("VTL_HIP_MATMUL_TILE", shape)
+    M, N, K = mnk
+    rng = np.random.default_rng(M + N + K)
+    bias = rng.integers(-9, 10, N)
+    for dt in (np.float32, np.float64):
+        for ta, tb in [(False, False), (False, True), (True, False), (True, True)][:2 if N > 1 << 20 else 4]:
+            A = rng.integers(-9, 10, (K, M) if ta else (M, K)).astype(dt)
+            B = rng.integers(-9, 10, (N, K) if tb else (K, N)).astype(dt)
+            exact = (A.T if ta else A).astype(np.float64) @ (B.T if tb else B).astype(np.float64)
+            assert np.array_equal(run_matmul(A, B, ta, tb), exact.astype(dt)), (dt, ta, tb)
+            if not ta and tb:
+                x, w, b = dev(A), dev(B), dev(bias.astype(dt))
+                y = linear_hip(x, w, b, relu=True)
+                assert np.array_equal(y.cpu(), np.maximum(exact + bias, 0).astype(dt)), dt
+                for t in (x, w, b, y):
+                    t.release()
+
+
 @pytest.mark.parametrize("tile", ["64", "128"])
 def test_forced_tile_sizes(hip, tile, knobs):
     """VTL_HIP_MATMUL_TILE forces the 64x64 or the 128x128 tile kernel: whole and ragged

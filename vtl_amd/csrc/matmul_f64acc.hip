@@ -5,16 +5,8 @@
 // Also the unquantized Linear forward (nn/layers/linear_forward_f32.v:16-18)
 // and LinearGate.backward (nn/gates/layers/linear.v:69-79) built on it.
 //
-// Two kernels.  matmul_f64acc_kernel stages 128 x 128 tiles through LDS for large products of whole
-// tiles; matmul_f64acc_direct_kernel, for everything else, takes operands from global memory
-// straight to registers.  choose_plan() picks by estimated time.
-//
-// The staged kernel: one workgroup of WR x WC waves owns a BM x BN tile of C.  Both operands go
-// through LDS in k-major form (As[k][m], Bs[k][n]) whatever their
-// layout in memory, so that one 16- or 32-byte LDS read hands a lane the
-// operands of all its 16x16x4 MFMA tiles for one k.  MFMA tile i of a wave
-// holds the rows {TM * r + i : r = 0..15} of the wave's rows (and likewise for
-// columns), which makes those reads and the final stores contiguous per lane.
+// matmul_f64acc_direct_kernel takes operands from global memory straight to registers; choose_plan() picks its
+// shape by estimated time.
 #include "common.hpp"
 
 #include <stdlib.h>
@@ -44,263 +36,130 @@ struct alignas(16) Vec4 {
     T v[4];
 };
 
-// NT consecutive LDS elements (NT = 2 or 4, naturally aligned) widened to f64.
-template <typename T, int NT>
-__device__ __forceinline__ void read_operands(const T *__restrict__ p, double (&out)[NT])
-{
-    struct alignas(NT * sizeof(T) > 16 ? 16 : NT * sizeof(T)) Pack {
-        T v[NT];
-    };
-    const Pack pk = *reinterpret_cast<const Pack *>(p);
-#pragma unroll
-    for (int i = 0; i < NT; ++i)
-        out[i] = (double)pk.v[i];
-}
-
-// One operand tile of BK x BMN elements (k-major in LDS, row stride LDW).
-// KMAJOR: the matrix is stored with the tile's m/n index contiguous ([K, MN]);
-// otherwise it is stored [MN, K] and is transposed on the way into LDS.
-template <typename T, int BK, int BMN, int LDW, int NT, bool KMAJOR>
-struct OperandTile {
-    static constexpr int kGroups = BK * BMN / 4;       // 4-element groups per tile
-    static constexpr int kPerThread = (kGroups + NT - 1) / NT;   // NT threads in the workgroup
-    typedef T Group __attribute__((ext_vector_type(4)));   // (a struct of four stays in scratch memory)
-    Group regs[kPerThread];
-
-    __device__ __forceinline__ void fetch(const T *__restrict__ base, int mn_total, int k_total, int mn0, int k0)
-    {
-        const int t = threadIdx.x;
-#pragma unroll
-        for (int i = 0; i < kPerThread; ++i) {
-            const int g = t + NT * i;
-            if (kGroups % NT != 0 && g >= kGroups)
-                break;
-            const T *__restrict__ p;
-            if constexpr (KMAJOR)
-                p = base + (int64_t)(k0 + g / (BMN / 4)) * mn_total + mn0 + 4 * (g % (BMN / 4));
-            else
-                p = base + (int64_t)(mn0 + g % BMN) * k_total + k0 + 4 * (g / BMN);
-            regs[i] = *reinterpret_cast<const Group *>(p);
-        }
-    }
-
-    __device__ __forceinline__ void stash(T *__restrict__ lds) const
-    {
-        const int t = threadIdx.x;
-#pragma unroll
-        for (int i = 0; i < kPerThread; ++i) {
-            const int g = t + NT * i;
-            if (kGroups % NT != 0 && g >= kGroups)
-                break;
-            if constexpr (KMAJOR) {
-                const int krow = g / (BMN / 4), c4 = g % (BMN / 4);
-                *reinterpret_cast<Group *>(lds + krow * LDW + 4 * c4) = regs[i];
-            } else {
-                const int mn = g % BMN, kc = g / BMN;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    lds[(4 * kc + j) * LDW + mn] = regs[i][j];
-            }
-        }
-    }
-};
-
-// Workgroup barrier that orders LDS traffic only: unlike __syncthreads() it does
-// not wait for outstanding global loads, so the operand loads issued two
-// k-tiles ahead stay in flight across it.
-__device__ __forceinline__ void lds_barrier()
-{
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
-// M, N, K are whole tiles and every row is 16-byte aligned.
-// Workgroup = WR x WC waves, each with TM x TN MFMA tiles of 16x16:
-// BM = 16 * TM * WR, BN = 16 * TN * WC.
-template <typename T, int TM, int TN, int WR, int WC, bool TA, bool TB>
-__global__ __launch_bounds__(64 * WR * WC) void matmul_f64acc_kernel(const MatmulArgs g)
-{
-    constexpr int BM = 16 * TM * WR, BN = 16 * TN * WC, NT = 64 * WR * WC;
-    constexpr int BK = 64 / (int)sizeof(T);   // bytes of k per tile row: 64 (16 f32 / 8 f64)
-    constexpr int LDA = BM + 4, LDB = BN + 4;
-    static_assert(TM == 2 || TM == 4, "wave tile is 32 or 64 rows");
-    static_assert(TN == 4, "wave tile is 64 columns");
-
-    // Three LDS buffers per operand: while tile kt is multiplied, tile kt+1 is
-    // written at the start of the step (its global loads were issued a step
-    // earlier) and the one barrier per step sits before the last k-group, so
-    // that the first operands of tile kt+1 are read from LDS under the last
-    // MFMAs of tile kt and no MFMA waits for a barrier followed by an LDS read.
-    __shared__ __attribute__((aligned(16))) T As[3][BK * LDA];
-    __shared__ __attribute__((aligned(16))) T Bs[3][BK * LDB];
-
-    const T *__restrict__ A = static_cast<const T *>(g.A);
-    const T *__restrict__ B = static_cast<const T *>(g.B);
-    const int tiles_n = g.N / BN;
-    const int m0 = (int)(blockIdx.x / tiles_n) * BM;
-    const int n0 = (int)(blockIdx.x % tiles_n) * BN;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = (wave / WC) * (16 * TM), wn = (wave % WC) * (16 * TN);
-    const int r16 = lane & 15, kq = lane >> 4;
-
-    // A as op(A)[M,K]: stored [K,M] when transposed (k-major already)
-    OperandTile<T, BK, BM, LDA, NT, TA> ta;
-    // B as op(B)[K,N]: stored [K,N] when not transposed (k-major already)
-    OperandTile<T, BK, BN, LDB, NT, !TB> tb;
-
-    double4_t acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-            acc[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
-
-    const int ktiles = g.K / BK;
-    constexpr int S = BK / 4;   // k-groups (one MFMA step each) per tile
-    const int aoff = wm + TM * r16 + kq * LDA, boff = wn + TN * r16 + kq * LDB;
-
-    ta.fetch(A, g.M, g.K, m0, 0);
-    tb.fetch(B, g.N, g.K, n0, 0);
-    ta.stash(As[0]);
-    tb.stash(Bs[0]);
-    if (ktiles > 1) {
-        ta.fetch(A, g.M, g.K, m0, BK);
-        tb.fetch(B, g.N, g.K, n0, BK);
-    }
-    __syncthreads();
-    double a[TM], b[TN];
-    read_operands<T, TM>(As[0] + aoff, a);
-    read_operands<T, TN>(Bs[0] + boff, b);
-
-    int cur = 0;
-    for (int kt = 0; kt < ktiles; ++kt) {
-        const int nxt = cur == 2 ? 0 : cur + 1;
-        if (kt + 1 < ktiles) {
-            // buffer nxt was last read two steps ago; every wave has passed a barrier since
-            ta.stash(As[nxt]);
-            tb.stash(Bs[nxt]);
-        }
-        if (kt + 2 < ktiles) {
-            ta.fetch(A, g.M, g.K, m0, (kt + 2) * BK);
-            tb.fetch(B, g.N, g.K, n0, (kt + 2) * BK);
-        }
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-            double an[TM], bn[TN];
-            if (s + 1 < S) {
-                read_operands<T, TM>(As[cur] + aoff + 4 * (s + 1) * LDA, an);
-                read_operands<T, TN>(Bs[cur] + boff + 4 * (s + 1) * LDB, bn);
-            } else {
-                lds_barrier();   // tile kt+1 is in LDS for every wave; global loads stay in flight
-                read_operands<T, TM>(As[nxt] + aoff, an);
-                read_operands<T, TN>(Bs[nxt] + boff, bn);
-            }
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-                a[i] = an[i];
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-                b[j] = bn[j];
-        }
-        cur = nxt;
-    }
-
-    T *__restrict__ C = static_cast<T *>(g.C);
-    const T *__restrict__ bias = static_cast<const T *>(g.bias);
-    const int col0 = n0 + wn + TN * r16;
-    T bv[TN];
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-        bv[j] = bias ? bias[col0 + j] : T(0);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int row = m0 + wm + TM * (4 * e + kq) + i;
-            Vec4<T> out;
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                T y = (T)acc[i][j][e];   // the one rounding to the tensor's type
-                if (bias)
-                    y = y + bv[j];       // Tensor.add in the tensor's type
-                if (g.relu && y < T(0))
-                    y = T(0);
-                out.v[j] = y;
-            }
-            *reinterpret_cast<Vec4<T> *>(C + (int64_t)row * g.N + col0) = out;
-        }
-    }
-}
-
 // ---- operands straight from global memory --------------------------------------------------
-// A wave owns 32 x 16 * TN of C.  An f64 MFMA wants two values a lane every 64 cycles, so operands
-// need neither LDS nor barriers, and what bounds a launch is how evenly its MFMAs spread over the
-// SIMDs: the tiles are small, K is cut over the WK waves of a workgroup (partial tiles meet in LDS)
-// and, with few tiles, over grid.y.  With 64 x 64 tiles staged in LDS a wave had four MFMAs for every 4
+// A wave owns 16 * TM x 16 * TN of C.  An f64 MFMA wants two values a lane every 64 cycles, so operands
+// need neither LDS nor barriers: the tiles are small, K is cut over the WK waves of a workgroup (partial
+// tiles meet in LDS) and, with few tiles, over grid.y.  With 64 x 64 tiles staged in LDS a wave had four MFMAs for every 4
 // of K, 7 us at K = 256 and 14 us at K = 512 whatever else the chip did, and ragged sizes loaded
 // element by element: 512^3 22.4 -> 8.8 us, 64 x 784 x 256 16.4 -> 5.5, 64 x 256 x 784 44 -> 7.5,
 // 255 x 11007 x 4095 447 -> 367, 333 x 517 x 701 47 -> 13 (f32; f64 alike).
 //
-// Steps of 16 of K are dealt out to the WK waves in turn.  In a step lane l holds four k for the two
+// What bounds a large product: nothing of the vector unit runs beside an f64 MFMA.  An instruction between two of them
+// costs 11 cycles and each further one 5 to 7 (measured, one and two waves on a SIMD, conversions, integer
+// and f32 operations alike), against 64 for the MFMA.  So the loop has no vector instruction but the
+// conversions of f32 operands, all of a step's at once, and those are fewer the larger a wave's tile is:
+// loads take a lane's offset that never changes and scalars for the rest (buffer loads), and a pair of columns at
+// the odd edge of a matrix is moved, not chosen from.
+//
+// Steps of 16 of K are dealt out to the WK waves in turn.  In a step lane l holds four k for TM / 2 pairs of
 // rows 2 * (l % 16) + {0, 1} of A and for TN / 2 such pairs of columns of B: 16-byte loads where K runs
 // along memory, pairs of 32 neighbouring columns where it does not.  MFMA j of a step takes the j-th of
 // each lane's four: which k they are is free as long as both operands agree.
 // Vector loads need no more than the elements' own alignment on gfx950, so ragged rows take them too;
 // what is left of K after whole steps is a step of its own with checked loads.  CHECKED: every
-// load is (a single row or column of a matrix that has to give pairs).
-template <typename T, bool KROWS, bool CHECKED>
-__device__ __forceinline__ void direct_fetch(T (&out)[2][4], const T *__restrict__ base, int mn_total, int k_total,
-                                            const int (&mn)[2], bool second_only, int k0, int kq)
+// load is (a single row or column of a matrix that has to give pairs, sizes beyond a lane's 32-bit offset).
+template <typename T>
+constexpr int kRun = 16 / (int)sizeof(T);   // elements of a 16-byte load; the lane's four are those of each run of 4 * kRun
+
+// N elements at `off` bytes (a lane's own) + `along` from base, one load.
+template <typename T, int N>
+__device__ __forceinline__ void load_run(T (&out)[N], __amdgpu_buffer_rsrc_t base, unsigned off, unsigned along)
 {
-    // a 16-byte load holds VK elements; the lane's four are those VK of each run of 4 * VK
-    constexpr int VK = 16 / (int)sizeof(T);
-    struct alignas(sizeof(T)) Run {
-        T v[VK];
-    };
-    struct alignas(sizeof(T)) Pair {
-        T v[2];
-    };
+    typedef unsigned Two __attribute__((ext_vector_type(2)));
+    typedef unsigned Four __attribute__((ext_vector_type(4)));
+    constexpr int bytes = N * (int)sizeof(T);
+    static_assert(bytes == 8 || bytes == 16, "one load");
+    if constexpr (bytes == 16) {
+        const Four v = __builtin_amdgcn_raw_buffer_load_b128(base, off, along, 0);
+        __builtin_memcpy(out, &v, bytes);
+    } else {
+        const Two v = __builtin_amdgcn_raw_buffer_load_b64(base, off, along, 0);
+        __builtin_memcpy(out, &v, bytes);
+    }
+}
+
+template <bool THROUGH>
+__device__ __forceinline__ void store_run(__amdgpu_buffer_rsrc_t base, unsigned off, unsigned along, float a, float b)
+{
+    typedef unsigned Two __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(Two{__float_as_uint(a), __float_as_uint(b)}, base, off, along, THROUGH ? 17 : 0);   // sc0 sc1
+}
+
+template <bool THROUGH>
+__device__ __forceinline__ void store_run(__amdgpu_buffer_rsrc_t base, unsigned off, unsigned along, double a, double b)
+{
+    typedef unsigned Four __attribute__((ext_vector_type(4)));
+    const unsigned long long ua = (unsigned long long)__double_as_longlong(a), ub = (unsigned long long)__double_as_longlong(b);
+    __builtin_amdgcn_raw_buffer_store_b128(Four{(unsigned)ua, (unsigned)(ua >> 32), (unsigned)ub, (unsigned)(ub >> 32)}, base, off,
+                                           along, THROUGH ? 17 : 0);
+}
+
+// One pair of rows or columns of an operand for the lanes of a wave.
+template <typename T, bool KROWS>
+struct DirectOperand {
+    const char *base;      // of the wave's rows or columns
+    int64_t k_stride;      // bytes from one k to the next
+    unsigned off[2];       // a lane's bytes from there, at k = 0: of its two rows, or of its pair
+
+    // [MN, K], its rows mn[0] and mn[1], or [K, MN], its columns mn[0] and mn[0] + 1
+    __device__ __forceinline__ DirectOperand(const T *p, int mn_total, int k_total, int mn_first, const int (&mn)[2], int kq)
+    {
+        if constexpr (KROWS) {
+            base = reinterpret_cast<const char *>(p + (int64_t)mn_first * k_total);
+            k_stride = (int)sizeof(T);
 #pragma unroll
-    for (int q = 0; q < 4; q += VK) {
-        const int k = k0 + 4 * q + VK * kq;
-        if constexpr (KROWS) {   // [MN, K]
+            for (int i = 0; i < 2; ++i)
+                off[i] = ((unsigned)(mn[i] - mn_first) * (unsigned)k_total + (unsigned)(kRun<T> * kq)) * (unsigned)sizeof(T);
+        } else {
+            base = reinterpret_cast<const char *>(p);
+            k_stride = (int64_t)mn_total * (int)sizeof(T);
+            off[0] = off[1] = ((unsigned)(kRun<T> * kq) * (unsigned)mn_total + (unsigned)mn[0]) * (unsigned)sizeof(T);
+        }
+    }
+    __device__ __forceinline__ void fetch(T (&out)[2][4], int k0) const
+    {
+        constexpr int VK = kRun<T>;
+        const __amdgpu_buffer_rsrc_t at =
+            __builtin_amdgcn_make_buffer_rsrc(const_cast<char *>(base + k0 * k_stride), 0, 0xffffffff, 0x00027000);
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const T *__restrict__ p = base + (int64_t)mn[i] * k_total + k;
-                if constexpr (!CHECKED) {
-                    const Run v = *reinterpret_cast<const Run *>(p);
+        for (int q = 0; q < 4; q += VK) {
+            if constexpr (KROWS) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    T run[VK];
+                    load_run<T, VK>(run, at, off[i], (unsigned)(4 * q) * (unsigned)sizeof(T));
 #pragma unroll
                     for (int j = 0; j < VK; ++j)
-                        out[i][q + j] = v.v[j];
-                } else {
-#pragma unroll
-                    for (int j = 0; j < VK; ++j)
-                        out[i][q + j] = k + j < k_total ? p[j] : T(0);
+                        out[i][q + j] = run[j];
                 }
-            }
-        } else {                 // [K, MN]
+            } else {
 #pragma unroll
-            for (int j = 0; j < VK; ++j) {
-                if constexpr (!CHECKED) {
-                    // second_only: the pair was moved back by one to stay inside, its second is mn[0]
-                    const Pair v = *reinterpret_cast<const Pair *>(base + (int64_t)(k + j) * mn_total + mn[0] -
-                                                                   (second_only ? 1 : 0));
-                    out[0][q + j] = second_only ? v.v[1] : v.v[0];
-                    out[1][q + j] = v.v[1];
-                } else {
-#pragma unroll
-                    for (int i = 0; i < 2; ++i)
-                        out[i][q + j] = k + j < k_total ? base[(int64_t)(k + j) * mn_total + mn[i]] : T(0);
+                for (int j = 0; j < VK; ++j) {
+                    T pair[2];
+                    load_run<T, 2>(pair, at, off[0], (unsigned)(4 * q + j) * (unsigned)k_stride);
+                    out[0][q + j] = pair[0];
+                    out[1][q + j] = pair[1];
                 }
             }
         }
     }
+};
+
+// The same with every load checked and no vector loads, at any size.
+template <typename T, bool KROWS>
+__device__ __forceinline__ void checked_fetch(T (&out)[2][4], const T *__restrict__ base, int mn_total, int k_total,
+                                              const int (&mn)[2], int k0, int kq)
+{
+    constexpr int VK = kRun<T>;
+#pragma unroll
+    for (int q = 0; q < 4; q += VK)
+#pragma unroll
+        for (int j = 0; j < VK; ++j) {
+            const int k = k0 + 4 * q + VK * kq + j;
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                out[i][q + j] = k < k_total ? base[KROWS ? (int64_t)mn[i] * k_total + k : (int64_t)k * mn_total + mn[i]] : T(0);
+        }
 }
 
 // Two neighbours of a row, aligned as one element is.
@@ -324,19 +183,20 @@ __device__ __forceinline__ void store_pair(double *p, double a, double b, const 
         *reinterpret_cast<Two *>(p) = v;
 }
 
-// The tiles of a workgroup are WM x WN wave tiles of 32 x 16 * TN, K is cut over WK waves each.
+// The tiles of a workgroup are WM x WN wave tiles, K is cut over WK waves each.
 // Blocks are renumbered so that each of the 8 XCDs (own L2) works on a compact patch of tiles, eight
 // tile rows deep: with the plain order the rows that share a column panel of B run on different XCDs.
-template <typename T, int WM, int WN, int WK, int TN, bool TA, bool TB, bool CHECKED>
+template <typename T, int WM, int WN, int WK, int TM, int TN, bool TA, bool TB, bool CHECKED>
 __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel(const MatmulArgs g)
 {
-    constexpr int D = sizeof(T) == 4 && TN == 2 ? 4 : 2;   // steps whose operands are in flight
-    constexpr int P = TN / 2;                              // column pairs of a lane
-    constexpr int V = 8 * TN;                              // values of a lane
+    constexpr int PA = TM / 2, PB = TN / 2;                // row and column pairs of a lane
+    // steps whose operands are in flight
+    constexpr int D = sizeof(T) == 4 ? (TM * TN <= 4 ? 4 : 2) : (TM * TN <= 8 ? 3 : 2);
+    constexpr int V = 4 * TM * TN;                         // values of a lane
     __shared__ double red[WK > 1 ? WM * WN * WK : 1][WK > 1 ? V : 1][64];
     const T *__restrict__ A = static_cast<const T *>(g.A);
     const T *__restrict__ B = static_cast<const T *>(g.B);
-    constexpr int BM = 32 * WM, BN = 16 * TN * WN;
+    constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
     const int tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
     int tm, tn;
     {
@@ -349,7 +209,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
     }
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wk = wave % WK, tile = wave / WK;
-    const int m0 = tm * BM + (tile / WN) * 32, n0 = tn * BN + (tile % WN) * 16 * TN;
+    const int m0 = tm * BM + (tile / WN) * 16 * TM, n0 = tn * BN + (tile % WN) * 16 * TN;
     const int r16 = lane & 15, kq = lane >> 4;
     // this workgroup's whole steps of K (all of them, or one of grid.y slices), this wave's among
     // them, and whether this wave does the part of a step at the end of K
@@ -358,40 +218,77 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
     const int count = first + wk > last ? 0 : (last - first - wk) / WK + 1;
     const bool rest = !CHECKED && steps * 16 < g.K && blockIdx.y == gridDim.y - 1 && wk == WK - 1;
 
-    // rows and columns past the edge repeat the last ones; what they give is not stored
-    const int row[2] = {min(m0 + 2 * r16, g.M - 1), min(m0 + 2 * r16 + 1, g.M - 1)};
-    const bool row_alone = row[0] == g.M - 1;
-    int col[P][2];
-    bool col_alone[P];
+    // Rows and columns past the edge repeat the last ones; what they give is not stored.  A pair that would
+    // reach past the edge is moved back by one: its second is then the edge.
+    int row[PA][2], col[PB][2];
+    auto pair_at = [&](int (&mn)[2], int at, int total, bool along) {
+        mn[0] = min(at, total - (along && !CHECKED ? 2 : 1));
+        mn[1] = along && !CHECKED ? mn[0] + 1 : min(at + 1, total - 1);
+    };
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
-        col[p][0] = min(n0 + 32 * p + 2 * r16, g.N - 1);
-        col[p][1] = min(n0 + 32 * p + 2 * r16 + 1, g.N - 1);
-        col_alone[p] = col[p][0] == g.N - 1;
-    }
-    T fa[D][2][4], fb[D][P][2][4];
+    for (int p = 0; p < PA; ++p)
+        pair_at(row[p], m0 + 32 * p + 2 * r16, g.M, TA);
+#pragma unroll
+    for (int p = 0; p < PB; ++p)
+        pair_at(col[p], n0 + 32 * p + 2 * r16, g.N, !TB);
+    T fa[D][PA][2][4], fb[D][PB][2][4];
+    auto checked = [&](int d, int k0) {
+#pragma unroll
+        for (int p = 0; p < PA; ++p)
+            checked_fetch<T, !TA>(fa[d][p], A, g.M, g.K, row[p], k0, kq);
+#pragma unroll
+        for (int p = 0; p < PB; ++p)
+            checked_fetch<T, TB>(fb[d][p], B, g.N, g.K, col[p], k0, kq);
+    };
+    const int row_first = min(m0, g.M - 1), col_first = min(n0, g.N - 1);
     auto fetch = [&](int d, int i) {   // the wave's i-th step; past its end the last one again
         const int k0 = min(first + wk + i * WK, last) * 16;
-        direct_fetch<T, !TA, CHECKED>(fa[d], A, g.M, g.K, row, row_alone, k0, kq);
+        if constexpr (CHECKED) {
+            checked(d, k0);
+        } else {
 #pragma unroll
-        for (int p = 0; p < P; ++p)
-            direct_fetch<T, TB, CHECKED>(fb[d][p], B, g.N, g.K, col[p], col_alone[p], k0, kq);
+            for (int p = 0; p < PA; ++p)
+                DirectOperand<T, !TA>(A, g.M, g.K, row_first, row[p], kq).fetch(fa[d][p], k0);
+#pragma unroll
+            for (int p = 0; p < PB; ++p)
+                DirectOperand<T, TB>(B, g.N, g.K, col_first, col[p], kq).fetch(fb[d][p], k0);
+        }
     };
-    double4_t acc[2][TN];
+    double4_t acc[TM][TN];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
             acc[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
-    auto multiply = [&](int d) {
+    // The products of step d, and behind its conversions (or, of f64, behind its MFMAs) the loads that take its place.
+    auto step = [&](int d, auto &&refill) {
+        double a[TM][4], b[TN][4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                a[i][k] = (double)fa[d][i >> 1][i & 1][k];
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                b[j][k] = (double)fb[d][j >> 1][j & 1][k];
+        }
+        if constexpr (sizeof(T) == 4) {
+            __builtin_amdgcn_sched_barrier(0);
+            refill();
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int k = 0; k < 4; ++k)
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                        (double)fa[d][i][k], (double)fb[d][j >> 1][j & 1][k], acc[i][j], 0, 0, 0);
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][k], b[j][k], acc[i][j], 0, 0, 0);
+        if constexpr (sizeof(T) == 8) {
+            __builtin_amdgcn_sched_barrier(0);
+            refill();
+        }
+        __builtin_amdgcn_sched_barrier(0);
     };
     if (count > 0) {
 #pragma unroll
@@ -400,32 +297,68 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
         int i = 0;
         for (; i + D <= count; i += D) {
 #pragma unroll
-            for (int d = 0; d < D; ++d) {
-                multiply(d);
-                fetch(d, i + d + D);
-            }
+            for (int d = 0; d < D; ++d)
+                step(d, [&] { fetch(d, i + d + D); });
         }
 #pragma unroll
         for (int d = 0; d < D - 1; ++d)
             if (i + d < count)
-                multiply(d);
+                step(d, [] {});
     }
     if (rest) {
-        const int k0 = steps * 16;
-        direct_fetch<T, !TA, true>(fa[0], A, g.M, g.K, row, false, k0, kq);
+        checked(0, steps * 16);
+        step(0, [] {});
+    }
+    if constexpr (!CHECKED) {
+        // the edge of an odd matrix is the second of its pair
+        if (m0 + 16 * TM > g.M - 1)
 #pragma unroll
-        for (int p = 0; p < P; ++p)
-            direct_fetch<T, TB, true>(fb[0][p], B, g.N, g.K, col[p], false, k0, kq);
-        multiply(0);
+            for (int i = 0; i < TM; i += 2)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i][j][e] = m0 + 16 * i + 2 * (4 * e + kq) == g.M - 1 ? acc[i + 1][j][e] : acc[i][j][e];
+        if (n0 + 16 * TN > g.N - 1)
+#pragma unroll
+            for (int j = 0; j < TN; j += 2)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        acc[i][j][e] = n0 + 16 * j + 2 * r16 == g.N - 1 ? acc[i][j + 1][e] : acc[i][j][e];
     }
     T *__restrict__ C = static_cast<T *>(g.C);
     const T *__restrict__ bias = static_cast<const T *>(g.bias);
     double *__restrict__ partial = g.partial ? g.partial + (int64_t)blockIdx.y * g.M * g.N : nullptr;
     // Value v of a lane: i = v / (4 TN), j = v / 4 % TN, e = v % 4.  Values v and v + 4 of an even j are
     // neighbours in a row and stored together: whole lines of 16 lanes.
+    // Inside the matrix a store's address is a scalar and a lane's offset too.
+    const bool inside = !CHECKED && !partial && m0 + 16 * TM <= g.M && n0 + 16 * TN <= g.N;
+    const __amdgpu_buffer_rsrc_t tile_out =
+        __builtin_amdgcn_make_buffer_rsrc(C + (inside ? (int64_t)m0 * g.N + n0 : 0), 0, 0xffffffff, 0x00027000);
+    const unsigned lane_out = (unsigned)(2 * kq * g.N + 2 * r16) * (unsigned)sizeof(T);
     auto store = [&](int v, double s0, double s1) {
-        const int j = (v >> 2) & (TN - 1);
-        const int r = m0 + 2 * (4 * (v & 3) + kq) + v / (4 * TN), c = n0 + 32 * (j >> 1) + 2 * r16;
+        const int i = v / (4 * TN), j = (v >> 2) % TN;
+        if (inside) {
+            T y[2] = {(T)s0, (T)s1};
+            if (bias) {
+                const T *at = bias + n0 + 32 * (j >> 1) + 2 * r16;
+                y[0] = y[0] + at[0];
+                y[1] = y[1] + at[1];
+            }
+            if (g.relu) {
+                y[0] = y[0] < T(0) ? T(0) : y[0];
+                y[1] = y[1] < T(0) ? T(0) : y[1];
+            }
+            const unsigned along = (unsigned)((32 * (i >> 1) + 8 * (v & 3) + (i & 1)) * g.N + 32 * (j >> 1)) * (unsigned)sizeof(T);
+            if (g.done.flag)
+                store_run<true>(tile_out, lane_out, along, y[0], y[1]);
+            else
+                store_run<false>(tile_out, lane_out, along, y[0], y[1]);
+            return;
+        }
+        const int r = m0 + 32 * (i >> 1) + 2 * (4 * (v & 3) + kq) + (i & 1), c = n0 + 32 * (j >> 1) + 2 * r16;
         if (r >= g.M || c >= g.N)
             return;
         const bool both = c + 1 < g.N;
@@ -453,12 +386,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
 #pragma unroll
         for (int v = 0; v < V; ++v)
             if (!(v & 4))
-                store(v, acc[v / (4 * TN)][(v >> 2) & (TN - 1)][v & 3], acc[v / (4 * TN)][((v >> 2) & (TN - 1)) + 1][v & 3]);
+                store(v, acc[v / (4 * TN)][(v >> 2) % TN][v & 3], acc[v / (4 * TN)][(v >> 2) % TN + 1][v & 3]);
     } else {
         // partial tiles, in the order of the registers
 #pragma unroll
         for (int v = 0; v < V; ++v)
-            red[wave][v][lane] = acc[v / (4 * TN)][(v >> 2) & (TN - 1)][v & 3];
+            red[wave][v][lane] = acc[v / (4 * TN)][(v >> 2) % TN][v & 3];
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < V / 2 / WK; ++u) {
@@ -575,25 +508,6 @@ __global__ __launch_bounds__(256) void matmul_splitk_finalize_kernel(const Matmu
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 template <typename T>
-int launch_staged(const MatmulArgs &g, bool ta, bool tb, hipStream_t st)
-{
-    // eight waves of 32x64 per 128x128 tile measured a few percent above four waves of 64x64
-    const int64_t tiles = (int64_t)(g.M / 128) * (g.N / 128);
-    if (tiles > 0x7fffffff)
-        return VTL_HIP_ERR_UNSUPPORTED;
-    const dim3 grid((unsigned)tiles), block(512);
-    if (!ta && !tb)
-        hipLaunchKernelGGL((matmul_f64acc_kernel<T, 2, 4, 4, 2, false, false>), grid, block, 0, st, g);
-    else if (!ta && tb)
-        hipLaunchKernelGGL((matmul_f64acc_kernel<T, 2, 4, 4, 2, false, true>), grid, block, 0, st, g);
-    else if (ta && !tb)
-        hipLaunchKernelGGL((matmul_f64acc_kernel<T, 2, 4, 4, 2, true, false>), grid, block, 0, st, g);
-    else
-        hipLaunchKernelGGL((matmul_f64acc_kernel<T, 2, 4, 4, 2, true, true>), grid, block, 0, st, g);
-    return check_launch("matmul_f64acc_kernel");
-}
-
-template <typename T>
 int finalize_split(MatmulArgs g, int splits, hipStream_t st)
 {
     const int64_t blocks = ((int64_t)g.M * g.N + 255) / 256;
@@ -603,45 +517,56 @@ int finalize_split(MatmulArgs g, int splits, hipStream_t st)
     return check_launch("matmul_splitk_finalize_kernel");
 }
 
-// How a product runs: the staged kernel, or one of the direct kernel's shapes with K in `slices`.
-enum Shape { kStaged, kK8, kK4, kWide, kPairK2, kPanel, kShapes };
+// The kernel's shapes, and K in `slices` over the grid.
+enum Shape { kK8, kK4, kWide, kLarge, kSquare, kBlock, kShapes };
 struct Plan {
     Shape shape;
     int slices;
 };
 
-// Wave tiles and waves per tile: what the names above stand for.
-constexpr int kTileM[kShapes] = {128, 32, 32, 32, 64, 64};
-constexpr int kTileN[kShapes] = {128, 32, 32, 64, 64, 128};
+// Three kinds of product differ in what a shape costs: f32, f64, and f64 with K along both operands' rows (the
+// Linear forward), where a 16-byte load is two k of one row and a small tile waits for its loads.
+enum Kind { kF32, kF64, kF64Rows, kKinds };
 
-// Estimated microseconds: start + rounds * (per_tile + work / rate), where `rounds` is how many
-// workgroups the busiest compute unit gets and `work` the time its matrix cores need for one tile at
-// 2.3 GHz; slicing K adds a launch and its partial sums (per MB).  Fitted to 240 products drawn over
-// m, n up to 11008 and k up to 4096, whole and ragged, all four layouts, every shape timed alternately:
-// the choice is on average 2.6 % and at most 30 % behind the fastest.
+// Wave tiles and waves per tile.  kLarge is one wave of 32 x 64 for f32 (level with 64 x 128 of four waves in large
+// products, up to 3 % ahead with a short K) and that workgroup for f64 (2 % ahead of single waves at 4096^3).
+// kSquare (a 64 x 64 wave tile, K over four) and kBlock (one such wave) are for kF64Rows: 256 x 11008 x 4096 514 ->
+// 366 us, 64 x 10979 x 3840 178 -> 120, 4096^3 2700 -> 1865.
+constexpr int kTileM[kKinds][kShapes] = {{32, 32, 32, 32, 0, 0}, {32, 32, 32, 64, 0, 0}, {32, 32, 32, 0, 64, 64}};
+constexpr int kTileN[kKinds][kShapes] = {{32, 32, 64, 64, 0, 0}, {32, 32, 64, 128, 0, 0}, {32, 32, 64, 0, 64, 64}};
+constexpr int kPerUnit[kKinds][kShapes] = {{1, 1, 1, 4, 0, 0}, {1, 1, 1, 1, 0, 0}, {1, 1, 1, 0, 1, 4}};   // workgroups that fill a compute unit's SIMDs once
+
+// Estimated microseconds: start + rounds * (per_tile + work / rate), where `rounds` is how many times the busiest
+// compute unit is filled and `work` the time its matrix cores need for that at
+// 2.3 GHz; slicing K adds a launch and its partial sums (per MB).  Fitted to 1200 products drawn over
+// m, n up to 11008 and k up to 4096, whole and ragged, the layouts of forward and backward, every shape timed alternately:
+// the choice is on average 2 % (kF64Rows 2.7 %) and at most 26 % behind the fastest.
 struct Cost {
     double start, per_tile, inverse_rate, slice_start, slice_mb;
 };
-constexpr Cost kCost[2][kShapes] = {
-    // f32
-    {{2.9, 0.0, 1.12, 0, 0}, {2.8, 1.27, 1.27, 3.5, 0.68}, {3.3, 0.56, 1.31, 3.9, 0.55}, {2.9, 1.61, 1.13, 3.7, 0.60},
-     {3.1, 2.20, 1.13, 4.0, 0.35}, {3.2, 2.85, 1.19, 4.0, 0.35}},
-    // f64
-    {{2.5, 2.5, 1.14, 0, 0}, {1.9, 1.71, 1.41, 3.1, 1.39}, {3.1, 0.68, 1.44, 3.6, 0.73}, {2.8, 1.68, 1.23, 4.0, 0.58},
-     {3.3, 2.21, 1.18, 4.0, 0.27}, {2.5, 3.40, 1.19, 4.0, 0.27}},
+constexpr Cost kCost[kKinds][kShapes] = {
+    {{1.59, 2.57, 1.18, 4.24, 0.42}, {3.22, 0.88, 1.13, 4.10, 0.43}, {2.89, 1.65, 1.05, 4.71, 0.45}, {2.52, 2.71, 1.08, 4.06, 0.53}, {}, {}},
+    {{1.64, 2.07, 1.22, 4.27, 0.49}, {2.87, 0.83, 1.14, 4.01, 0.55}, {2.81, 1.65, 1.06, 4.57, 0.53}, {2.41, 3.48, 0.97, 5.23, 0.30}, {}, {}},
+    {{1.65, 2.10, 1.89, 4.47, 0.62}, {2.69, 1.09, 1.76, 3.91, 0.75}, {2.57, 2.21, 1.37, 4.47, 0.52}, {}, {1.40, 5.53, 1.04, 4.55, 0.55},
+     {0.0, 8.0, 0.97, 3.93, 0.41}},
 };
 
+Kind kind_of(bool f64, bool ta, bool tb) { return !f64 ? kF32 : (!ta && tb ? kF64Rows : kF64); }
+
 // may_slice: whether K may be cut (matmul_impl).
-Plan choose_plan(bool f64, int m, int n, int k, bool whole, bool may_slice)
+Plan choose_plan(Kind kind, int m, int n, int k, bool may_slice)
 {
     Plan best = {kK4, 1};
     double best_us = 1e30;
-    for (int s = whole ? kStaged : kK8; s < kShapes; s++) {
-        const Cost &c = kCost[f64 ? 1 : 0][s];
-        const int64_t tiles = (int64_t)((m + kTileM[s] - 1) / kTileM[s]) * ((n + kTileN[s] - 1) / kTileN[s]);
+    for (int s = 0; s < kShapes; s++) {
+        const int bm = kTileM[kind][s], bn = kTileN[kind][s], unit = kPerUnit[kind][s];
+        if (bm == 0)
+            continue;
+        const Cost &c = kCost[kind][s];
+        const int64_t tiles = (int64_t)((m + bm - 1) / bm) * ((n + bn - 1) / bn);
         // no slices, one workgroup per compute unit in all, or two where K is long
         int64_t want[3] = {1, 0, 0};
-        if (may_slice && s != kStaged && k >= 512 && tiles < 256) {
+        if (may_slice && k >= 512 && tiles < 256) {
             want[1] = 256 / tiles;
             want[2] = k >= 2048 ? 2 * want[1] : 0;
         }
@@ -652,8 +577,8 @@ Plan choose_plan(bool f64, int m, int n, int k, bool whole, bool may_slice)
                 slices = 32;
             if (slices < 1)
                 slices = 1;
-            const double rounds = (double)((tiles * slices + 255) / 256);
-            const double work = (double)kTileM[s] * kTileN[s] * ((double)k / (double)slices) / (64.0 * 2300.0);
+            const double rounds = (double)((tiles * slices + 256 * unit - 1) / (256 * unit));
+            const double work = (double)bm * bn * unit * ((double)k / (double)slices) / (64.0 * 2300.0);
             double us = c.start + rounds * (c.per_tile + work * c.inverse_rate);
             if (slices > 1)
                 us += c.slice_start + c.slice_mb * 8e-6 * (double)slices * (double)m * (double)n;
@@ -666,24 +591,32 @@ Plan choose_plan(bool f64, int m, int n, int k, bool whole, bool may_slice)
     return best;
 }
 
-template <typename T, int WM, int WN, int WK, int TN, bool CHECKED = false>
+// ROWS_ONLY: the layout of kF64Rows, no other.
+template <typename T, int WM, int WN, int WK, int TM, int TN, bool CHECKED = false, bool ROWS_ONLY = false>
 int launch_direct_shape(MatmulArgs g, bool ta, bool tb, int slices, hipStream_t st)
 {
-    constexpr int BM = 32 * WM, BN = 16 * TN * WN;
+    constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
     const int64_t tiles = (int64_t)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
     if (tiles > 0x7fffffff)
         return VTL_HIP_ERR_UNSUPPORTED;
     const dim3 grid((unsigned)tiles, (unsigned)slices), block(64 * WM * WN * WK);
     if (g.result && slices == 1)
         g.result->attach(g.done, grid.x);
-    if (!ta && !tb)
-        hipLaunchKernelGGL((matmul_f64acc_direct_kernel<T, WM, WN, WK, TN, false, false, CHECKED>), grid, block, 0, st, g);
-    else if (!ta && tb)
-        hipLaunchKernelGGL((matmul_f64acc_direct_kernel<T, WM, WN, WK, TN, false, true, CHECKED>), grid, block, 0, st, g);
-    else if (ta && !tb)
-        hipLaunchKernelGGL((matmul_f64acc_direct_kernel<T, WM, WN, WK, TN, true, false, CHECKED>), grid, block, 0, st, g);
-    else
-        hipLaunchKernelGGL((matmul_f64acc_direct_kernel<T, WM, WN, WK, TN, true, true, CHECKED>), grid, block, 0, st, g);
+#define VTL_DIRECT(TA, TB) \
+    hipLaunchKernelGGL((matmul_f64acc_direct_kernel<T, WM, WN, WK, TM, TN, TA, TB, CHECKED>), grid, block, 0, st, g)
+    if constexpr (ROWS_ONLY) {
+        VTL_DIRECT(false, true);
+    } else {
+        if (!ta && !tb)
+            VTL_DIRECT(false, false);
+        else if (!ta && tb)
+            VTL_DIRECT(false, true);
+        else if (ta && !tb)
+            VTL_DIRECT(true, false);
+        else
+            VTL_DIRECT(true, true);
+    }
+#undef VTL_DIRECT
     return check_launch("matmul_f64acc_direct_kernel");
 }
 
@@ -712,8 +645,9 @@ struct Partial {
 template <typename T>
 int launch_direct(MatmulArgs g, bool ta, bool tb, Plan plan, bool alone, hipStream_t st)
 {
-    // pairs of a row or column index that runs along memory need two of them
-    const bool checked = (ta && g.M < 2) || (!tb && g.N < 2);
+    // pairs of a row or column index that runs along memory need two of them, and a lane's offset is 32 bits
+    constexpr int kMost = 1 << 22;
+    const bool checked = (ta && g.M < 2) || (!tb && g.N < 2) || g.M > kMost || g.N > kMost || g.K > kMost;
     const int steps = checked ? (g.K + 15) / 16 : g.K / 16;
     int per = (steps + plan.slices - 1) / plan.slices;
     int slices = per > 0 ? (steps + per - 1) / per : 1;
@@ -726,19 +660,23 @@ int launch_direct(MatmulArgs g, bool ta, bool tb, Plan plan, bool alone, hipStre
         }
     }
     g.k_per_split = 16 * per;
-    int rc;
+    int rc = VTL_HIP_ERR_UNSUPPORTED;
     if (checked)
-        rc = launch_direct_shape<T, 1, 1, 8, 2, true>(g, ta, tb, slices, st);
+        rc = launch_direct_shape<T, 1, 1, 8, 2, 2, true>(g, ta, tb, slices, st);
     else if (plan.shape == kK8)
-        rc = launch_direct_shape<T, 1, 1, 8, 2>(g, ta, tb, slices, st);
+        rc = launch_direct_shape<T, 1, 1, 8, 2, 2>(g, ta, tb, slices, st);
+    else if (plan.shape == kK4)
+        rc = launch_direct_shape<T, 1, 1, 4, 2, 2>(g, ta, tb, slices, st);
     else if (plan.shape == kWide)
-        rc = launch_direct_shape<T, 1, 1, 4, 4>(g, ta, tb, slices, st);
-    else if (plan.shape == kPairK2)
-        rc = launch_direct_shape<T, 2, 1, 2, 4>(g, ta, tb, slices, st);
-    else if (plan.shape == kPanel)
-        rc = launch_direct_shape<T, 2, 2, 1, 4>(g, ta, tb, slices, st);
+        rc = launch_direct_shape<T, 1, 1, 4, 2, 4>(g, ta, tb, slices, st);
+    else if constexpr (sizeof(T) == 4)
+        rc = launch_direct_shape<T, 1, 1, 1, 2, 4>(g, ta, tb, slices, st);
+    else if (plan.shape == kLarge)
+        rc = launch_direct_shape<T, 2, 2, 1, 2, 4>(g, ta, tb, slices, st);
+    else if (plan.shape == kSquare)
+        rc = launch_direct_shape<T, 1, 1, 4, 4, 4, false, true>(g, ta, tb, slices, st);
     else
-        rc = launch_direct_shape<T, 1, 1, 4, 2>(g, ta, tb, slices, st);
+        rc = launch_direct_shape<T, 1, 1, 1, 4, 4, false, true>(g, ta, tb, slices, st);
     return rc != VTL_HIP_OK || slices == 1 ? rc : finalize_split<T>(g, slices, st);
 }
 
@@ -762,32 +700,22 @@ int matmul_impl(const T *a, const T *b, T *c, const T *bias, int m, int n, int k
     g.N = n;
     g.K = k;
     g.relu = relu;
-    // the staged kernel's loads and stores carry no bounds checks
-    const bool whole = m % 128 == 0 && n % 128 == 0 && k % 32 == 0 && k > 0 && aligned16(a) && aligned16(b) &&
-                       aligned16(c);
     // Where streams have been named, K is cut from 2048 on only: there the header asks callers to order
     // calls of different streams, which then share scratch; shorter products stay independent of each other
     // (64 x 256 x 784 f32: 8.9 us sliced, 10.9 in one piece; 64 x 256 x 2000: 9.3 and 21.9).
     const bool alone = vtlhip::single_stream();
-    Plan plan = choose_plan(sizeof(T) == 8, m, n, k, whole, alone || k >= 2048);
-    // Tuning and tests: VTL_HIP_MATMUL_TILE 128 forces the staged kernel where it can run, 64 the
-    // 64 x 64 tiles, 1 .. 5 a shape of the direct kernel; VTL_HIP_MATMUL_SPLITS the slices of K.
+    const Kind kind = kind_of(sizeof(T) == 8, trans_a != 0, trans_b != 0);
+    Plan plan = choose_plan(kind, m, n, k, alone || k >= 2048);
+    // Tuning and tests: VTL_HIP_MATMUL_TILE 1 .. 6 forces a shape (one that the kind of product does not have gives its
+    // largest), 64 and 128 the larger ones; VTL_HIP_MATMUL_SPLITS the slices of K.
     const int tile = vtlhip::tuning().matmul_tile, splits = vtlhip::tuning().matmul_splits;
-    if (tile == 128 && whole)
-        plan.shape = kStaged;
-    else if (tile == 64)
-        plan.shape = kPairK2;
-    else if (tile >= kK8 && tile < kShapes)
-        plan.shape = (Shape)tile;
-    if (splits >= 0) {
-        plan.slices = splits > 1 && k >= 32 * splits ? splits : 1;
-        if (plan.shape == kStaged && plan.slices > 1)
-            plan.shape = kK4;
-    } else if (plan.shape == kStaged) {
-        plan.slices = 1;
+    if (tile > 0) {
+        const int shape = tile == 64 ? (int)kSquare : (tile <= kShapes ? tile - 1 : (int)kBlock);
+        plan.shape = kTileM[kind][shape] ? (Shape)shape : (kind == kF64Rows ? kBlock : kLarge);
     }
-    return plan.shape == kStaged ? launch_staged<T>(g, trans_a != 0, trans_b != 0, current_stream())
-                                 : launch_direct<T>(g, trans_a != 0, trans_b != 0, plan, alone, current_stream());
+    if (splits >= 0)
+        plan.slices = splits > 1 && k >= 32 * splits ? splits : 1;
+    return launch_direct<T>(g, trans_a != 0, trans_b != 0, plan, alone, current_stream());
 }
 
 template <typename T>
