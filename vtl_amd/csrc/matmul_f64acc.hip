@@ -530,8 +530,8 @@ enum Kind { kF32, kF64, kF64Rows, kKinds };
 
 // Wave tiles and waves per tile.  kLarge is one wave of 32 x 64 for f32 (level with 64 x 128 of four waves in large
 // products, up to 3 % ahead with a short K) and that workgroup for f64 (2 % ahead of single waves at 4096^3).
-// kSquare (a 64 x 64 wave tile, K over four) and kBlock (one such wave) are for kF64Rows: 256 x 11008 x 4096 514 ->
-// 366 us, 64 x 10979 x 3840 178 -> 120, 4096^3 2700 -> 1865.
+// kSquare (a 64 x 64 wave tile, K over four) and kBlock (one such wave) are for kF64Rows: against kWide
+// 256 x 11008 x 4096 523 -> 366 us, 64 x 10979 x 3840 169 -> 119, 4096^3 2760 -> 1865.
 constexpr int kTileM[kKinds][kShapes] = {{32, 32, 32, 32, 0, 0}, {32, 32, 32, 64, 0, 0}, {32, 32, 32, 0, 64, 64}};
 constexpr int kTileN[kKinds][kShapes] = {{32, 32, 64, 64, 0, 0}, {32, 32, 64, 128, 0, 0}, {32, 32, 64, 0, 64, 64}};
 constexpr int kPerUnit[kKinds][kShapes] = {{1, 1, 1, 4, 0, 0}, {1, 1, 1, 1, 0, 0}, {1, 1, 1, 0, 1, 4}};   // workgroups that fill a compute unit's SIMDs once
