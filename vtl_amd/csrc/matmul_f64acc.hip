@@ -383,6 +383,19 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
             vtlhip::store_result(to, y[0], g.done);
     };
     if constexpr (WK == 1) {
+        // Nothing but conversions and stores: what `store` asks of every pair is asked once for the tile.  No vector
+        // instruction runs beside another wave's MFMAs, so with a short K this end of a tile is what a launch waits for:
+        // f32 dW 8192 x 8192 x 64 168 -> 149 us, 11008 x 4096 x 128 197 -> 183, x 256 363 -> 347.
+        if (inside && !bias && !g.relu && !g.done.flag) {
+#pragma unroll
+            for (int v = 0; v < V; ++v)
+                if (!(v & 4)) {
+                    const int i = v / (4 * TN), j = (v >> 2) % TN;
+                    const unsigned along = (unsigned)((32 * (i >> 1) + 8 * (v & 3) + (i & 1)) * g.N + 32 * (j >> 1)) * (unsigned)sizeof(T);
+                    store_run<false>(tile_out, lane_out, along, (T)acc[i][j][v & 3], (T)acc[i][j + 1][v & 3]);
+                }
+            return;   // no signal to raise
+        }
 #pragma unroll
         for (int v = 0; v < V; ++v)
             if (!(v & 4))
