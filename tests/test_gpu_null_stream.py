@@ -100,7 +100,8 @@ from vtl_amd import PER_CHANNEL, PER_TENSOR, QuantLinearLayer, Sequential, capi,
 # past 32 KiB) and uploaded
 LAYERS = [(1, 1, 64), (1, 2048, 300), (1, 2049, 512), (2, 1024, 256), (2, 1025, 1100), (3, 9, 1700), (8, 256, 640), (8, 40, 1024),
           (5, 700, 2100), (17, 2050, 512), (33, 100, 784), (40, 900, 1024), (64, 300, 2100), (65, 4100, 640), (200, 801, 1664),
-          (256, 8191, 72), (256, 8193, 72)]
+          (256, 8191, 72), (256, 8193, 72),
+          (256, 4096, 72), (256, 4128, 72), (100, 6553, 72), (100, 6554, 72)]   # either side of what is written directly
 def layers(seed):
     rng = np.random.default_rng(seed)
     for m, n, k in LAYERS:
@@ -132,7 +133,7 @@ def network(seed):   # a ReLU folded into the last layer, and one more that is n
 def products(seed):   # whole numbers: every sum is exact; whole tiles of 128, K cut, results past 8 MiB
     rng = np.random.default_rng(seed)
     for m, n, k, dt in ((1, 1, 1, "f4"), (37, 41, 100, "f8"), (33, 257, 3000, "f4"), (128, 256, 64, "f8"), (180, 183, 32, "f4"),
-                        (1024, 1024, 8, "f8"), (1030, 1030, 8, "f8"),
+                        (1024, 1024, 8, "f8"), (1030, 1030, 8, "f8"), (300, 655, 40, "f4"), (300, 656, 40, "f4"),
                         # operands that go up together: in one launch (1 MiB in all) or not, several pieces a launch, odd addresses
                         (64, 64, 2048, "f4"), (64, 65, 2048, "f4"), (401, 403, 777, "f8"), (701, 903, 1201, "f4"),
                         (2051, 65, 1103, "f8")):

@@ -99,8 +99,8 @@ public:
     HostResult(const HostResult &) = delete;
     HostResult &operator=(const HostResult &) = delete;
     // Pinned memory to write a result of `bytes` to that finish() leaves in dst (up to kParts of them); nullptr:
-    // compute in device memory and download.
-    void *begin(void *dst, size_t bytes);
+    // compute in device memory and download, as with more than `most`.
+    void *begin(void *dst, size_t bytes, size_t most);
     // For the last launch of the call, right before it, with its number of workgroups.
     void attach(DoneSignal &signal, unsigned blocks);
     // After the release() of an input that the launch with the signal has read.

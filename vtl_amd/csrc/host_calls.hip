@@ -79,7 +79,11 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
     const size_t out_bytes = (size_t)rows * (size_t)out_cols * sizeof(float);
     const bool ends_linear = count > 0 && (layers[count - 1].kind == VTL_HIP_LAYER_LINEAR ||
                                            (count > 1 && layers[count - 2].kind == VTL_HIP_LAYER_LINEAR));
-    float *const y = ends_linear ? static_cast<float *>(result.begin(y_host, out_bytes)) : nullptr;
+    // Written over the link as it is computed, with rows that end where lines do, 4 MiB is no slower than a copy behind the
+    // launch (256 x 4096 126 -> 121 us; 256 x 5000 145 and 158, 256 x 8000 205 and 222).  Other rows leave lines to two
+    // workgroups: 100 x 6001 76 -> 74, but 96 x 8191 90 and 92, 200 x 4999 117 and 126, 200 x 6001 133 and 151, 192 x 10000 186 and 236.
+    const size_t most = out_cols % 32 == 0 ? (size_t)4 << 20 : (size_t)5 << 19;
+    float *const y = ends_linear ? static_cast<float *>(result.begin(y_host, out_bytes, most)) : nullptr;
     HostInput input;
     // (32 KiB is what the kernels that quantize in every workgroup take at most; near it the eight XCDs' transfers
     // cost what an upload does)
@@ -184,6 +188,19 @@ int upload_both(Scratch &to0, const T *host0, size_t count0, Scratch &to1, const
     return vtl_hip_upload(to1.ptr, host1, count1 * sizeof(T));
 }
 
+constexpr size_t kResultMost = (size_t)8 << 20;
+
+// How many bytes a product writes over the link as it is computed.  Rows that do not end where lines do leave lines to two
+// workgroups, which the link takes apart: a copy behind the launch is faster unless there is little to write (us,
+// copied and written over the link: f32 700 x 1001 x 200 122 and 136, 1024 x 1001 x 64 117 and 128, x 320 184 and
+// 195, 256 x 1000 x 800 level, 256 x 700 x 16 38 and 36; whole lines 1024 x 1024 x 16 107 and 102, x 400 200 and 198).
+template <typename T>
+size_t direct_most(int m, int n)
+{
+    const bool whole_lines = (size_t)n * sizeof(T) % 128 == 0;
+    return whole_lines || (int64_t)m * n <= 196608 ? kResultMost : 0;
+}
+
 template <typename T>
 int matmul_host(const T *a, const T *b, T *c, int m, int n, int k)
 {
@@ -197,7 +214,7 @@ int matmul_host(const T *a, const T *b, T *c, int m, int n, int k)
     VTL_STEP(upload_both(da, a, (size_t)m * (size_t)k, db, b, (size_t)k * (size_t)n));
     const size_t bytes = (size_t)m * (size_t)n * sizeof(T);
     HostResult result;
-    if (T *out = static_cast<T *>(result.begin(c, bytes))) {
+    if (T *out = static_cast<T *>(result.begin(c, bytes, direct_most<T>(m, n)))) {
         VTL_STEP(matmul_to(&result, da.as<T>(), db.as<T>(), out, m, n, k, 0));
         return result.finish();
     }
@@ -226,7 +243,7 @@ int linear_backward_host(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
         {
             if (!host || bytes == 0)
                 return VTL_HIP_OK;
-            out = static_cast<T *>(result.begin(host, bytes));
+            out = static_cast<T *>(result.begin(host, bytes, kResultMost));
             direct = out != nullptr;
             if (!direct) {
                 VTL_STEP(dev.take(bytes));

@@ -914,13 +914,9 @@ try {
     return true;
 }
 
-// Results that are written over the link as they are computed: up to here no slower than a copy behind the
-// launch (256 x 11008 f32, 11 MiB: 248 us more against 219).
-constexpr size_t kResultMost = (size_t)8 << 20;
-
-void *HostResult::begin(void *dst, size_t bytes)
+void *HostResult::begin(void *dst, size_t bytes, size_t most)
 {
-    if (bytes == 0 || bytes > kResultMost || nafter_ == kParts || (!single_stream() && stream_is_capturing(current_stream())))
+    if (bytes == 0 || bytes > most || nafter_ == kParts || (!single_stream() && stream_is_capturing(current_stream())))
         return nullptr;
     const bool direct = (reinterpret_cast<uintptr_t>(dst) & 15) == 0 && bytes > 4096 && in_pinned_pool(dst, bytes);
     const size_t take = (bytes + 255) & ~(size_t)255;
