@@ -134,8 +134,9 @@ def products(seed):   # whole numbers: every sum is exact; whole tiles of 128, K
     rng = np.random.default_rng(seed)
     for m, n, k, dt in ((1, 1, 1, "f4"), (37, 41, 100, "f8"), (33, 257, 3000, "f4"), (128, 256, 64, "f8"), (180, 183, 32, "f4"),
                         (1024, 1024, 8, "f8"), (1030, 1030, 8, "f8"), (300, 655, 40, "f4"), (300, 656, 40, "f4"),
-                        # operands that go up together: in one launch (1 MiB in all) or not, several pieces a launch, odd addresses
-                        (64, 64, 2048, "f4"), (64, 65, 2048, "f4"), (401, 403, 777, "f8"), (701, 903, 1201, "f4"),
+                        # operands that go up together: in one launch (640 KiB in all), in turn (1 MiB each) or in pieces, several a
+                        # launch, odd addresses
+                        (80, 80, 1024, "f4"), (80, 81, 1024, "f4"), (256, 256, 1024, "f4"), (257, 256, 1024, "f4"), (64, 64, 2048, "f4"), (64, 65, 2048, "f4"), (401, 403, 777, "f8"), (701, 903, 1201, "f4"),
                         (2051, 65, 1103, "f8")):
         for turn in range(2):
             a, b = rng.integers(-8, 9, (m, k)).astype(dt), rng.integers(-8, 9, (k, n)).astype(dt)
