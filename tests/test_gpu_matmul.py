@@ -104,6 +104,26 @@ def test_split_k_paths(hip, dt, knobs):
         t.release()
 
 
+# K cut for the last round's tiles alone (f64 with K along both operands' rows): rounds of 256 tiles before it, none (every
+# tile is of the last), steps of K that do not divide and a rest of K, all it may be cut into; all values are whole, so
+# every sum is exact
+@pytest.mark.parametrize("slices", ["-2", "-5", "-8"])
+@pytest.mark.parametrize("mnk", [(130, 8301, 113), (301, 7200, 96), (65, 63, 47), (64, 16385, 160), (4, 16449, 769)])
+def test_last_round_cut_by_k(hip, slices, mnk, knobs):
+    knobs.setenv("VTL_HIP_MATMUL_TILE", "5")
+    knobs.setenv("VTL_HIP_MATMUL_SPLITS", slices)
+    M, N, K = mnk
+    rng = np.random.default_rng(M + N + K)
+    A, B, bias = (rng.integers(-9, 10, shape).astype(np.float64) for shape in ((M, K), (N, K), (N,)))
+    exact = A @ B.T
+    assert np.array_equal(run_matmul(A, B, False, True), exact)
+    x, w, b = dev(A), dev(B), dev(bias)
+    y = linear_hip(x, w, b, relu=True)
+    assert np.array_equal(y.cpu(), np.maximum(exact + bias, 0))
+    for t in (x, w, b, y):
+        t.release()
+
+
 # (the shapes that only f64 with K along both operands' rows has, and the others at the edges of the largest tiles;
 # columns beyond a lane's 32-bit offset are checked load by load)
 @pytest.mark.parametrize("shape", ["4", "5", "6"])

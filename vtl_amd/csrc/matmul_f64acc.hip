@@ -26,7 +26,9 @@ struct MatmulArgs {
     int M, N, K;
     int relu;
     int k_per_split;    // k range of one grid.y slice (multiple of 16)
-    double *partial;    // launches that slice K: [slices][M][N] unrounded sums, else nullptr
+    double *partial;    // launches that slice K: [slices][M][N] unrounded sums, or [tail tile][slice][tile]; else nullptr
+    int whole_tiles;    // with tail_slices > 1 the tiles from here on, the last round's, have K in that many slices
+    int tail_slices;
     vtlhip::DoneSignal done;     // C is the memory of a whole host call's result
     vtlhip::HostResult *result;  // host side only
 };
@@ -183,6 +185,16 @@ __device__ __forceinline__ void store_pair(double *p, double a, double b, const 
         *reinterpret_cast<Two *>(p) = v;
 }
 
+__device__ __forceinline__ void tile_of_block(int block, int tiles_m, int tiles_n, int &tm, int &tn)
+{
+    const int total = tiles_m * tiles_n;
+    const int xcd = block & 7, over = total & 7;
+    const int pid = xcd * (total >> 3) + min(xcd, over) + (block >> 3);
+    const int group = 8 * tiles_n, first_m = (pid / group) * 8, gm = min(tiles_m - first_m, 8);
+    tm = first_m + (pid % group) % gm;
+    tn = (pid % group) / gm;
+}
+
 // The tiles of a workgroup are WM x WN wave tiles, K is cut over WK waves each.
 // Blocks are renumbered so that each of the 8 XCDs (own L2) works on a compact patch of tiles, eight
 // tile rows deep: with the plain order the rows that share a column panel of B run on different XCDs.
@@ -190,6 +202,7 @@ template <typename T, int WM, int WN, int WK, int TM, int TN, bool TA, bool TB, 
 __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel(const MatmulArgs g)
 {
     constexpr int PA = TM / 2, PB = TN / 2;                // row and column pairs of a lane
+    constexpr bool TAIL = TM == 4 && WK > 1;               // kSquare: choose_plan
     // steps whose operands are in flight
     constexpr int D = sizeof(T) == 4 ? (TM * TN <= 4 ? 4 : 2) : (TM * TN <= 8 ? 3 : 2);
     constexpr int V = 4 * TM * TN;                         // values of a lane
@@ -198,25 +211,25 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
     const T *__restrict__ B = static_cast<const T *>(g.B);
     constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
     const int tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
-    int tm, tn;
-    {
-        const int total = tiles_m * tiles_n, block = (int)blockIdx.x;
-        const int xcd = block & 7, over = total & 7;
-        const int pid = xcd * (total >> 3) + min(xcd, over) + (block >> 3);
-        const int group = 8 * tiles_n, first_m = (pid / group) * 8, gm = min(tiles_m - first_m, 8);
-        tm = first_m + (pid % group) % gm;
-        tn = (pid % group) / gm;
+    int block = (int)blockIdx.x, slice = (int)blockIdx.y, slices = (int)gridDim.y, of_tail = -1;
+    if (TAIL && g.tail_slices > 1 && block >= g.whole_tiles) {
+        of_tail = block - g.whole_tiles;
+        slices = g.tail_slices;
+        slice = of_tail % slices;
+        block = g.whole_tiles + of_tail / slices;
     }
+    int tm, tn;
+    tile_of_block(block, tiles_m, tiles_n, tm, tn);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wk = wave % WK, tile = wave / WK;
     const int m0 = tm * BM + (tile / WN) * 16 * TM, n0 = tn * BN + (tile % WN) * 16 * TN;
     const int r16 = lane & 15, kq = lane >> 4;
     // this workgroup's whole steps of K (all of them, or one of grid.y slices), this wave's among
     // them, and whether this wave does the part of a step at the end of K
-    const int steps = CHECKED ? (g.K + 15) / 16 : g.K / 16, per = g.k_per_split / 16;
-    const int first = (int)blockIdx.y * per, last = min(first + per, steps) - 1;
+    const int steps = CHECKED ? (g.K + 15) / 16 : g.K / 16, per = TAIL && g.tail_slices > 1 && of_tail < 0 ? steps : g.k_per_split / 16;
+    const int first = slice * per, last = min(first + per, steps) - 1;
     const int count = first + wk > last ? 0 : (last - first - wk) / WK + 1;
-    const bool rest = !CHECKED && steps * 16 < g.K && blockIdx.y == gridDim.y - 1 && wk == WK - 1;
+    const bool rest = !CHECKED && steps * 16 < g.K && slice == slices - 1 && wk == WK - 1;
 
     // Rows and columns past the edge repeat the last ones; what they give is not stored.  A pair that would
     // reach past the edge is moved back by one: its second is then the edge.
@@ -330,7 +343,14 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
     }
     T *__restrict__ C = static_cast<T *>(g.C);
     const T *__restrict__ bias = static_cast<const T *>(g.bias);
-    double *__restrict__ partial = g.partial ? g.partial + (int64_t)blockIdx.y * g.M * g.N : nullptr;
+    double *__restrict__ partial = nullptr;   // and the place of C's first element, were it there
+    int64_t partial_row = g.N;
+    if (TAIL && of_tail >= 0) {
+        partial = g.partial + (int64_t)of_tail * (BM * BN) - ((int64_t)tm * BM * BN + (int64_t)tn * BN);
+        partial_row = BN;
+    } else if (g.partial && !(TAIL && g.tail_slices > 1)) {
+        partial = g.partial + (int64_t)slice * g.M * g.N;
+    }
     // Value v of a lane: i = v / (4 TN), j = v / 4 % TN, e = v % 4.  Values v and v + 4 of an even j are
     // neighbours in a row and stored together: whole lines of 16 lanes.
     // Inside the matrix a store's address is a scalar and a lane's offset too.
@@ -363,9 +383,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
             return;
         const bool both = c + 1 < g.N;
         if (partial) {
-            partial[(int64_t)r * g.N + c] = s0;
+            partial[(int64_t)r * partial_row + c] = s0;
             if (both)
-                partial[(int64_t)r * g.N + c + 1] = s1;
+                partial[(int64_t)r * partial_row + c + 1] = s1;
             return;
         }
         T y[2] = {(T)s0, (T)s1};     // the one rounding to the tensor's type
@@ -518,6 +538,30 @@ __global__ __launch_bounds__(256) void matmul_splitk_finalize_kernel(const Matmu
     vtlhip::raise_when_last(g.done);
 }
 
+// The last round's tiles, 256 elements a workgroup (with a tile each 128 x 8704 x 2049 in eight slices took 117 us, now 86).
+template <typename T>
+__global__ __launch_bounds__(256) void matmul_tail_finalize_kernel(const MatmulArgs g, int bm, int bn)
+{
+    const int per_tile = bm * bn / 256, t = (int)blockIdx.x / per_tile, i = ((int)blockIdx.x % per_tile) * 256 + (int)threadIdx.x;
+    int tm, tn;
+    tile_of_block(g.whole_tiles + t, (g.M + bm - 1) / bm, (g.N + bn - 1) / bn, tm, tn);
+    const int r = tm * bm + i / bn, c = tn * bn + i % bn;
+    if (r >= g.M || c >= g.N)
+        return;
+    const double *__restrict__ partial = g.partial + (int64_t)t * g.tail_slices * (bm * bn) + i;
+    double s = 0.0;
+#pragma unroll 4
+    for (int k = 0; k < g.tail_slices; ++k)
+        s += partial[(int64_t)k * (bm * bn)];
+    T y = (T)s;
+    const T *__restrict__ bias = static_cast<const T *>(g.bias);
+    if (bias)
+        y = y + bias[c];
+    if (g.relu && y < T(0))
+        y = T(0);
+    static_cast<T *>(g.C)[(int64_t)r * g.N + c] = y;
+}
+
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 template <typename T>
@@ -535,6 +579,7 @@ enum Shape { kK8, kK4, kWide, kLarge, kSquare, kBlock, kShapes };
 struct Plan {
     Shape shape;
     int slices;
+    int tail_slices;   // of the last round's tiles alone
 };
 
 // Three kinds of product differ in what a shape costs: f32, f64, and f64 with K along both operands' rows (the
@@ -567,9 +612,9 @@ constexpr Cost kCost[kKinds][kShapes] = {
 Kind kind_of(bool f64, bool ta, bool tb) { return !f64 ? kF32 : (!ta && tb ? kF64Rows : kF64); }
 
 // may_slice: whether K may be cut (matmul_impl).
-Plan choose_plan(Kind kind, int m, int n, int k, bool may_slice)
+Plan choose_plan(Kind kind, int m, int n, int k, bool may_slice, bool may_tail)
 {
-    Plan best = {kK4, 1};
+    Plan best = {kK4, 1, 1};
     double best_us = 1e30;
     for (int s = 0; s < kShapes; s++) {
         const int bm = kTileM[kind][s], bn = kTileN[kind][s], unit = kPerUnit[kind][s];
@@ -597,7 +642,26 @@ Plan choose_plan(Kind kind, int m, int n, int k, bool may_slice)
                 us += c.slice_start + c.slice_mb * 8e-6 * (double)slices * (double)m * (double)n;
             if (us < best_us) {
                 best_us = us;
-                best = {(Shape)s, (int)slices};
+                best = {(Shape)s, (int)slices, 1};
+            }
+        }
+        // The last round with few tiles: K cut until they fill the chip.  For kSquare alone: its sums take 128 KiB of LDS, one
+        // workgroup is all a compute unit holds, and a round is as long as its last (f64 forward, us: 256 x 4352 x 4096
+        // 261 -> 145, 128 x 10240 x 2560 168 -> 110, 100 x 11008 x 4096 262 -> 191, 250 x 5000 x 640 50 -> 44).  The others have
+        // two that share a unit's matrix cores and level that out: f32 256 x 11008 x 4096 came to 343 from 348.
+        const int64_t whole = tiles / (256 * unit), left = tiles % (256 * unit);
+        if (s == kSquare && may_tail && whole > 0 && left > 0) {
+            const int64_t most = k / 96 < 8 ? k / 96 : 8;
+            const int64_t slices = 256 * unit / left < most ? 256 * unit / left : most;
+            if (slices > 1) {
+                const double work = (double)bm * bn * unit * k / (64.0 * 2300.0);
+                const double us = c.start + (double)whole * (c.per_tile + work * c.inverse_rate) + c.per_tile +
+                                  work / (double)slices * c.inverse_rate + c.slice_start +
+                                  c.slice_mb * 8e-6 * (double)(slices * left) * bm * bn;
+                if (us < best_us) {
+                    best_us = us;
+                    best = {(Shape)s, 1, (int)slices};
+                }
             }
         }
     }
@@ -612,7 +676,11 @@ int launch_direct_shape(MatmulArgs g, bool ta, bool tb, int slices, hipStream_t 
     const int64_t tiles = (int64_t)((g.M + BM - 1) / BM) * ((g.N + BN - 1) / BN);
     if (tiles > 0x7fffffff)
         return VTL_HIP_ERR_UNSUPPORTED;
-    const dim3 grid((unsigned)tiles, (unsigned)slices), block(64 * WM * WN * WK);
+    // (whole_tiles + the tail's slices: a few workgroups more than tiles)
+    const int64_t blocks = g.tail_slices > 1 ? g.whole_tiles + (tiles - g.whole_tiles) * g.tail_slices : tiles;
+    if (blocks > 0x7fffffff)
+        return VTL_HIP_ERR_UNSUPPORTED;
+    const dim3 grid((unsigned)blocks, (unsigned)slices), block(64 * WM * WN * WK);
     if (g.result && slices == 1)
         g.result->attach(g.done, grid.x);
 #define VTL_DIRECT(TA, TB) \
@@ -656,7 +724,7 @@ struct Partial {
 };
 
 template <typename T>
-int launch_direct(MatmulArgs g, bool ta, bool tb, Plan plan, bool alone, hipStream_t st)
+int launch_direct(MatmulArgs g, Kind kind, bool ta, bool tb, Plan plan, bool alone, hipStream_t st)
 {
     // pairs of a row or column index that runs along memory need two of them, and a lane's offset is 32 bits
     constexpr int kMost = 1 << 22;
@@ -670,6 +738,18 @@ int launch_direct(MatmulArgs g, bool ta, bool tb, Plan plan, bool alone, hipStre
         if (!g.partial) {   // no memory, or a capture that may not allocate: K in one piece
             per = steps;
             slices = 1;
+        }
+    }
+    const int bm = kTileM[kind][plan.shape], bn = kTileN[kind][plan.shape], unit = 256 * kPerUnit[kind][plan.shape];
+    const int64_t tiles = (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn), left = tiles % unit;
+    g.tail_slices = 1;
+    if (plan.tail_slices > 1 && plan.shape == kSquare && slices == 1 && !checked && !g.result && left > 0 && tiles < 0x7fffffff) {
+        const int tail_per = (steps + plan.tail_slices - 1) / plan.tail_slices;
+        const int tail = tail_per > 0 ? (steps + tail_per - 1) / tail_per : 1;
+        if (tail > 1 && (g.partial = partial.take((size_t)left * (size_t)tail * (size_t)(bm * bn) * sizeof(double), alone))) {
+            g.tail_slices = tail;
+            g.whole_tiles = (int)(tiles - left);
+            per = tail_per;
         }
     }
     g.k_per_split = 16 * per;
@@ -690,7 +770,13 @@ int launch_direct(MatmulArgs g, bool ta, bool tb, Plan plan, bool alone, hipStre
         rc = launch_direct_shape<T, 1, 1, 4, 4, 4, false, true>(g, ta, tb, slices, st);
     else
         rc = launch_direct_shape<T, 1, 1, 1, 4, 4, false, true>(g, ta, tb, slices, st);
-    return rc != VTL_HIP_OK || slices == 1 ? rc : finalize_split<T>(g, slices, st);
+    if (rc != VTL_HIP_OK)
+        return rc;
+    if (g.tail_slices > 1) {
+        hipLaunchKernelGGL((matmul_tail_finalize_kernel<T>), dim3((unsigned)(left * (bm * bn / 256))), dim3(256), 0, st, g, bm, bn);
+        return check_launch("matmul_tail_finalize_kernel");
+    }
+    return slices == 1 ? rc : finalize_split<T>(g, slices, st);
 }
 
 template <typename T>
@@ -718,17 +804,19 @@ int matmul_impl(const T *a, const T *b, T *c, const T *bias, int m, int n, int k
     // (64 x 256 x 784 f32: 8.9 us sliced, 10.9 in one piece; 64 x 256 x 2000: 9.3 and 21.9).
     const bool alone = vtlhip::single_stream();
     const Kind kind = kind_of(sizeof(T) == 8, trans_a != 0, trans_b != 0);
-    Plan plan = choose_plan(kind, m, n, k, alone || k >= 2048);
+    Plan plan = choose_plan(kind, m, n, k, alone || k >= 2048, !result && (alone || k >= 2048));
     // Tuning and tests: VTL_HIP_MATMUL_TILE 1 .. 6 forces a shape (one that the kind of product does not have gives its
-    // largest), 64 and 128 the larger ones; VTL_HIP_MATMUL_SPLITS the slices of K.
+    // largest), 64 and 128 the larger ones; VTL_HIP_MATMUL_SPLITS the slices of K, from -2 down those of the last round.
     const int tile = vtlhip::tuning().matmul_tile, splits = vtlhip::tuning().matmul_splits;
     if (tile > 0) {
         const int shape = tile == 64 ? (int)kSquare : (tile <= kShapes ? tile - 1 : (int)kBlock);
         plan.shape = kTileM[kind][shape] ? (Shape)shape : (kind == kF64Rows ? kBlock : kLarge);
     }
-    if (splits >= 0)
+    if (splits >= 0 || splits < -1) {
         plan.slices = splits > 1 && k >= 32 * splits ? splits : 1;
-    return launch_direct<T>(g, trans_a != 0, trans_b != 0, plan, alone, current_stream());
+        plan.tail_slices = splits < -1 ? -splits : 1;
+    }
+    return launch_direct<T>(g, kind, trans_a != 0, trans_b != 0, plan, alone, current_stream());
 }
 
 template <typename T>
