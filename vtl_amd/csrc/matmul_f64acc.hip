@@ -616,26 +616,31 @@ Plan choose_plan(Kind kind, int m, int n, int k, bool may_slice, bool may_tail)
 {
     Plan best = {kK4, 1, 1};
     double best_us = 1e30;
+    const int most_slices = k / 96;
     for (int s = 0; s < kShapes; s++) {
         const int bm = kTileM[kind][s], bn = kTileN[kind][s], unit = kPerUnit[kind][s];
         if (bm == 0)
             continue;
         const Cost &c = kCost[kind][s];
-        const int64_t tiles = (int64_t)((m + bm - 1) / bm) * ((n + bn - 1) / bn);
+        // (tile sides are powers of two, and so is what fills the chip: no divisions where a small product spends its time)
+        const int fill = unit == 4 ? 10 : 8;
+        const int64_t tiles = (((int64_t)m + bm - 1) >> __builtin_ctz(bm)) * (((int64_t)n + bn - 1) >> __builtin_ctz(bn));
         // no slices, one workgroup per compute unit in all, or two where K is long
         int64_t want[3] = {1, 0, 0};
         if (may_slice && k >= 512 && tiles < 256) {
-            want[1] = 256 / tiles;
+            want[1] = 256 / (int)tiles;
             want[2] = k >= 2048 ? 2 * want[1] : 0;
         }
         for (int64_t slices : want) {
-            if (slices > k / 96)
-                slices = k / 96;
+            if (slices == 0)
+                break;
+            if (slices > most_slices)
+                slices = most_slices;
             if (slices > 32)
                 slices = 32;
             if (slices < 1)
                 slices = 1;
-            const double rounds = (double)((tiles * slices + 256 * unit - 1) / (256 * unit));
+            const double rounds = (double)((tiles * slices + (1 << fill) - 1) >> fill);
             const double work = (double)bm * bn * unit * ((double)k / (double)slices) / (64.0 * 2300.0);
             double us = c.start + rounds * (c.per_tile + work * c.inverse_rate);
             if (slices > 1)
@@ -649,9 +654,9 @@ Plan choose_plan(Kind kind, int m, int n, int k, bool may_slice, bool may_tail)
         // workgroup is all a compute unit holds, and a round is as long as its last (f64 forward, us: 256 x 4352 x 4096
         // 261 -> 145, 128 x 10240 x 2560 168 -> 110, 100 x 11008 x 4096 262 -> 191, 250 x 5000 x 640 50 -> 44).  The others have
         // two that share a unit's matrix cores and level that out: f32 256 x 11008 x 4096 came to 343 from 348.
-        const int64_t whole = tiles / (256 * unit), left = tiles % (256 * unit);
+        const int64_t whole = tiles >> fill, left = tiles & ((1 << fill) - 1);
         if (s == kSquare && may_tail && whole > 0 && left > 0) {
-            const int64_t most = k / 96 < 8 ? k / 96 : 8;
+            const int64_t most = most_slices < 8 ? most_slices : 8;
             const int64_t slices = 256 * unit / left < most ? 256 * unit / left : most;
             if (slices > 1) {
                 const double work = (double)bm * bn * unit * k / (64.0 * 2300.0);
@@ -740,13 +745,15 @@ int launch_direct(MatmulArgs g, Kind kind, bool ta, bool tb, Plan plan, bool alo
             slices = 1;
         }
     }
-    const int bm = kTileM[kind][plan.shape], bn = kTileN[kind][plan.shape], unit = 256 * kPerUnit[kind][plan.shape];
-    const int64_t tiles = (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn), left = tiles % unit;
     g.tail_slices = 1;
-    if (plan.tail_slices > 1 && plan.shape == kSquare && slices == 1 && !checked && !g.result && left > 0 && tiles < 0x7fffffff) {
+    constexpr int bm = 64, bn = 64;   // kSquare
+    int64_t left = 0;
+    if (plan.tail_slices > 1 && plan.shape == kSquare && slices == 1 && !checked && !g.result) {
+        const int64_t tiles = (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn);
+        left = tiles < 0x7fffffff ? tiles % 256 : 0;
         const int tail_per = (steps + plan.tail_slices - 1) / plan.tail_slices;
         const int tail = tail_per > 0 ? (steps + tail_per - 1) / tail_per : 1;
-        if (tail > 1 && (g.partial = partial.take((size_t)left * (size_t)tail * (size_t)(bm * bn) * sizeof(double), alone))) {
+        if (left > 0 && tail > 1 && (g.partial = partial.take((size_t)left * (size_t)tail * (size_t)(bm * bn) * sizeof(double), alone))) {
             g.tail_slices = tail;
             g.whole_tiles = (int)(tiles - left);
             per = tail_per;
