@@ -609,10 +609,15 @@ constexpr Cost kCost[kKinds][kShapes] = {
      {0.0, 8.0, 0.97, 3.93, 0.41}},
 };
 
+// What a second launch has to be worth beyond its time on the device: it takes the host 3.4 us, which a chain of small products
+// waits for (steps of 16 x 2496 x 572 and 204 x 149 x 539, f64: 39.4 and 39.5 us without this, 35.9 and 36.2 with it).  Not
+// in whole host calls, where the link is behind the host (242 x 78 x 765: 60.5, and 62.5 with it).
+constexpr double kLaunch = 1.0;
+
 Kind kind_of(bool f64, bool ta, bool tb) { return !f64 ? kF32 : (!ta && tb ? kF64Rows : kF64); }
 
 // may_slice: whether K may be cut (matmul_impl).
-Plan choose_plan(Kind kind, int m, int n, int k, bool may_slice, bool may_tail)
+Plan choose_plan(Kind kind, int m, int n, int k, bool may_slice, bool may_tail, double launch)
 {
     Plan best = {kK4, 1, 1};
     double best_us = 1e30;
@@ -644,7 +649,7 @@ Plan choose_plan(Kind kind, int m, int n, int k, bool may_slice, bool may_tail)
             const double work = (double)bm * bn * unit * ((double)k / (double)slices) / (64.0 * 2300.0);
             double us = c.start + rounds * (c.per_tile + work * c.inverse_rate);
             if (slices > 1)
-                us += c.slice_start + c.slice_mb * 8e-6 * (double)slices * (double)m * (double)n;
+                us += c.slice_start + launch + c.slice_mb * 8e-6 * (double)slices * (double)m * (double)n;
             if (us < best_us) {
                 best_us = us;
                 best = {(Shape)s, (int)slices, 1};
@@ -811,7 +816,7 @@ int matmul_impl(const T *a, const T *b, T *c, const T *bias, int m, int n, int k
     // (64 x 256 x 784 f32: 8.9 us sliced, 10.9 in one piece; 64 x 256 x 2000: 9.3 and 21.9).
     const bool alone = vtlhip::single_stream();
     const Kind kind = kind_of(sizeof(T) == 8, trans_a != 0, trans_b != 0);
-    Plan plan = choose_plan(kind, m, n, k, alone || k >= 2048, !result && (alone || k >= 2048));
+    Plan plan = choose_plan(kind, m, n, k, alone || k >= 2048, !result && (alone || k >= 2048), result ? 0.0 : kLaunch);
     // Tuning and tests: VTL_HIP_MATMUL_TILE 1 .. 6 forces a shape (one that the kind of product does not have gives its
     // largest), 64 and 128 the larger ones; VTL_HIP_MATMUL_SPLITS the slices of K, from -2 down those of the last round.
     const int tile = vtlhip::tuning().matmul_tile, splits = vtlhip::tuning().matmul_splits;
