@@ -610,9 +610,10 @@ constexpr Cost kCost[kKinds][kShapes] = {
 };
 
 // What a second launch has to be worth beyond its time on the device: it takes the host 3.4 us, which a chain of small products
-// waits for (steps of 16 x 2496 x 572 and 204 x 149 x 539, f64: 39.4 and 39.5 us without this, 35.9 and 36.2 with it).  Not
-// in whole host calls, where the link is behind the host (242 x 78 x 765: 60.5, and 62.5 with it).
-constexpr double kLaunch = 1.0;
+// waits for.  Steps whose forward is cut for an estimated 0.04 and 0.46 us (16 x 2496 x 572 and 204 x 149 x 539, f64): 39.4 and
+// 39.5 us, and 35.9 and 36.2 in one piece; 64 x 256 x 784, 0.84, is 8.9 cut and 10.9 in one piece.  Not in whole host
+// calls, where the link is behind the host (242 x 78 x 765: 60.5 cut, 62.5 in one piece).
+constexpr double kLaunch = 0.6;
 
 Kind kind_of(bool f64, bool ta, bool tb) { return !f64 ? kF32 : (!ta && tb ? kF64Rows : kF64); }
 
