@@ -274,7 +274,7 @@ int vtl_hip_forward_i8_host(const float *x_host, int rows, int cols, const vtl_h
 
 /* la.matmul (la/la.v:38-55) and LinearGate.backward (nn/gates/layers/linear.v:57-79) on host
  * tensors: vtl_hip_matmul_* without transposes and vtl_hip_linear_backward_*, operands and
- * results on the host. */
+ * results on the host.  A result may share memory with an operand, not with another result. */
 int vtl_hip_matmul_host_f32(const float *A, const float *B, float *C, int M, int N, int K);
 int vtl_hip_matmul_host_f64(const double *A, const double *B, double *C, int M, int N, int K);
 int vtl_hip_linear_backward_host_f32(const float *grad, const float *x, const float *W, float *dx, float *dw,

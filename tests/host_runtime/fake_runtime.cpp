@@ -22,13 +22,14 @@ struct Range {
     int device;
 };
 std::map<const char *, Range> g_memory;
+std::map<const void *, std::string> g_kernels;   // mangled names
 
-void note(const char *what, void *stream, unsigned long long n)
+void note(const char *what, void *stream, unsigned long long n, const std::string &more = "")
 {
     char line[128];
-    snprintf(line, sizeof line, "%s %d %llu %llu\n", what, g_device, (unsigned long long)(uintptr_t)stream, n);
+    snprintf(line, sizeof line, "%s %d %llu %llu", what, g_device, (unsigned long long)(uintptr_t)stream, n);
     std::lock_guard<std::mutex> hold(g_lock);
-    g_log += line;
+    g_log += line + more + "\n";
 }
 
 struct Call {
@@ -50,7 +51,8 @@ void fake_set(int devices, int capturing, int refuse_memory, int wait_ms)
     g_wait_ms = wait_ms;
 }
 
-// The lines "<event> <device> <stream> <number>" since the last call.
+// The lines "<event> <device> <stream> <number>" since the last call; of a launch also the kernel's name and, of
+// the f64-accumulating matmul and the column sums, the address they write to.
 size_t fake_log(char *out, size_t cap)
 {
     std::lock_guard<std::mutex> hold(g_lock);
@@ -87,7 +89,13 @@ hipError_t hipFree(void *p)
     return hipSuccess;
 }
 
-hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) { *p = aligned_alloc(4096, (bytes + 4095) / 4096 * 4096); return hipSuccess; }
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned)
+{
+    note("host_malloc", nullptr, bytes);
+    *p = aligned_alloc(4096, (bytes + 4095) / 4096 * 4096);
+    return hipSuccess;
+}
+
 hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
 
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
@@ -150,9 +158,24 @@ hipError_t __hipPopCallConfiguration(dim3 *grid, dim3 *block, size_t *shared, hi
     return hipSuccess;
 }
 
-hipError_t hipLaunchKernel(const void *, dim3 grid, dim3, void **, size_t, hipStream_t st)
+void __hipRegisterFunction(void **, const void *function, char *, const char *name, unsigned, void *, void *, dim3 *, dim3 *,
+                           int *)
 {
-    note("launch", st, (unsigned long long)grid.x * grid.y * grid.z);
+    std::lock_guard<std::mutex> hold(g_lock);
+    g_kernels[function] = name;
+}
+
+hipError_t hipLaunchKernel(const void *function, dim3 grid, dim3, void **args, size_t, hipStream_t st)
+{
+    std::string more = " ?";
+    auto it = g_kernels.find(function);
+    if (it != g_kernels.end())
+        more = " " + it->second;
+    if (more.find("matmul_f64acc_direct_kernel") != std::string::npos)   // its argument begins with A, B, C
+        more += " " + std::to_string((unsigned long long)(uintptr_t) static_cast<void **>(args[0])[2]);
+    else if (more.find("13colsum_kernel") != std::string::npos)              // x, rows, cols, rows of a split, out
+        more += " " + std::to_string((unsigned long long)(uintptr_t) * static_cast<void **>(args[4]));
+    note("launch", st, (unsigned long long)grid.x * grid.y * grid.z, more);
     return hipSuccess;
 }
 

@@ -393,6 +393,26 @@ def test_linear_backward_host_entry(hip, monkeypatch):
     assert zeros.shape == (1, 2) and not zeros.any()
 
 
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("where", ["dw", "dw and db", "db"])
+def test_gradients_into_the_memory_of_w(hip, where, dt):
+    """A program that drops its weights with the step lets dW, or db, take their place: dX is of the weights as they were.
+    Whole values, so every sum is exact; large enough for results that launches write to the host themselves."""
+    from vtl_amd.storage import host_array
+    M, N, K = 64, 2048, 64
+    rng = np.random.default_rng(31)
+    grad, x, w0 = (rng.integers(-9, 10, shape).astype(dt) for shape in ((M, N), (M, K), (N, K)))
+    arena, _ = host_array(N * K + N, np.dtype(dt))
+    w, behind = arena[:N * K].reshape(N, K), arena[N * K:]
+    w[:] = w0
+    dx = np.zeros((M, K), dt)
+    dw = w if "dw" in where else np.zeros((N, K), dt)
+    db = w.reshape(-1)[:N] if where == "db" else behind
+    capi.call("vtl_hip_linear_backward_host_f32" if dt == np.float32 else "vtl_hip_linear_backward_host_f64",
+              grad.ctypes.data, x.ctypes.data, w.ctypes.data, dx.ctypes.data, dw.ctypes.data, db.ctypes.data, M, N, K)
+    assert np.array_equal(dx, grad @ w0) and np.array_equal(dw, grad.T @ x) and np.array_equal(db, grad.sum(0))
+
+
 def test_argument_errors(hip):
     from helpers import raw_device_buffer
     buf = raw_device_buffer(4096)

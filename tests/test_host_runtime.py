@@ -23,11 +23,13 @@ from vtl_amd import capi
 def runtime(devices=1, capturing=False, refuse_memory=False, wait_ms=0):
     fake.fake_set(devices, int(capturing), int(refuse_memory), wait_ms)
 
-def events():
+def lines():
     buf = C.create_string_buffer(1 << 20)
     n = fake.fake_log(buf, C.c_size_t(len(buf)))
-    lines = [l.split() for l in buf.raw[:n].decode().splitlines()]
-    return [(l[0], int(l[1]), int(l[2]), int(l[3])) for l in lines]
+    return [l.split() for l in buf.raw[:n].decode().splitlines()]
+
+def events():
+    return [(l[0], int(l[1]), int(l[2]), int(l[3])) for l in lines()]
 
 def count(what, log):
     return sum(1 for e in log if e[0] == what)
@@ -169,6 +171,33 @@ def run(f, *args, **kw):
     return events()
 for nbytes in (1, 4096, 1 << 20, (1 << 20) + 1, 5 << 20):
     assert waited(run(HipStorage.from_cpu, np.zeros(nbytes, np.uint8))), nbytes
+print("done")
+""")
+
+
+def test_gradients_in_the_memory_of_w_wait_for_its_upload(fake_runtime):
+    """The backward from host to host lets launches write dW and db to the host while it still has W to copy: never to
+    memory that W lies in (dW is all of it, or db its last row)."""
+    _run(fake_runtime, r"""
+runtime()
+M, N, K = 64, 2048, 64
+NK = N * K
+arena = C.c_void_p()
+capi.call("vtl_hip_host_alloc", C.byref(arena), 4 * (NK + N) + 8192)
+host = (C.c_float * (M * (N + K) + NK))()
+grad, x, other = C.addressof(host), C.addressof(host) + 4 * M * N, C.addressof(host) + 4 * M * (N + K)
+w = arena.value + 4096
+def written(dx, dw, db):
+    events()
+    capi.status("vtl_hip_linear_backward_host_f32", grad, x, w, dx, dw, db, M, N, K)    # no kernel runs here
+    return [int(l[5]) for l in lines() if len(l) > 5]
+W = range(w, w + 4 * NK)
+assert written(None, w, None) == [w]                     # W is not read at all
+for dw, db in ((w, None), (w - 4096, None), (w + 4 * 1024, None), (None, w), (None, w + 4 * (NK - N)), (w, w + 4 * NK)):
+    early = written(other, dw, db)[:-1]                  # all but dX, which comes behind the upload
+    assert len(early) == (dw is not None) + (db is not None), (dw, db, early)
+    assert not any(p in W for p in early), (dw, db, early)
+assert w + 4 * NK in written(other, w, w + 4 * NK)       # behind W: straight to the host
 print("done")
 """)
 
