@@ -202,6 +202,32 @@ print("done")
 """)
 
 
+def test_a_call_that_fails_keeps_no_memory(fake_runtime):
+    """Whole host calls that end in an error between their first step and their last, whichever it is: the pinned memory that
+    the result was to come through, and the device memory, serve the next call."""
+    _run(fake_runtime, r"""
+runtime()
+p = malloc_on(0, 1 << 20)
+host = (C.c_float * 65536)()
+def forward(rows, row_bytes):
+    layer = capi.Layer(0, 1, 64, 100, p, p, None, row_bytes)      # a linear, one scale per row
+    return capi.status("vtl_hip_forward_i8_host", host, rows, 100, C.byref(layer), 1, host)
+for rows in (1, 16, 64):
+    for again in range(4):
+        events()
+        assert forward(rows, 100) == capi.ERR_INVALID_ARG       # rows of a layer are padded to whole 16 bytes
+        log = events()
+        assert again == 0 or not count("host_malloc", log) + count("malloc", log), (rows, again, log)
+runtime(refuse_memory=True)
+capi.call("vtl_hip_trim")
+for again in range(4):      # device memory runs out behind the lease of what results come through
+    events()
+    assert capi.status("vtl_hip_linear_backward_host_f32", host, host, host, host, host, host, 64, 64, 64) == capi.ERR_OUT_OF_MEMORY
+    assert not count("host_malloc", events()), again
+print("done")
+""")
+
+
 def test_a_transfer_that_waits_for_the_device_costs_no_host_time(fake_runtime):
     """A large upload whose staging memory is not free yet: neither the caller nor the threads that help
     with the copying spin until it is."""

@@ -984,12 +984,20 @@ int HostResult::finish()
     return VTL_HIP_OK;
 }
 
-// After a failure launches may still write the results, and the lane's counter and flag are unknown: it is left alone.
+// After a failure launches may still write the results: they are waited for.  The lane goes back where its counter and flag are
+// known, no launch having been given its signal, or that launch having raised it; else it is left alone.
 HostResult::~HostResult()
 {
-    if (lane_) {
-        (void)hipStreamSynchronize(current_stream());
-        (void)hipGetLastError();
+    if (!lane_)
+        return;
+    Lane *lane = static_cast<Lane *>(lane_);
+    const bool ended = hipStreamSynchronize(current_stream()) == hipSuccess;
+    (void)hipGetLastError();
+    if (!ended || (attached_ && !lane->signal.raised()))
+        return;
+    try {
+        return_lane(lane);
+    } catch (const std::exception &) {   // no room in the list
     }
 }
 
