@@ -135,6 +135,25 @@ __device__ __forceinline__ void store_result(T *p, T v, const DoneSignal &done)
         *p = v;
 }
 
+// 8 or 16 bytes of a result of less than 4 GiB, `off` bytes from its start and aligned as an element is: one store, through
+// the caches.  (By way of a builtin and not of inline assembly: the compiler puts the wait states in that gfx950 wants
+// between a wide store, or the MFMA before it, and the instructions that touch the same registers.)
+typedef unsigned Words2 __attribute__((ext_vector_type(2)));
+typedef unsigned Words4 __attribute__((ext_vector_type(4)));
+constexpr int kThrough = 17;   // sc0 sc1
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t result_buffer(void *out)
+{
+    return __builtin_amdgcn_make_buffer_rsrc(out, 0, 0xffffffff, 0x00027000);
+}
+__device__ __forceinline__ void store_through(void *out, unsigned off, Words2 v)
+{
+    __builtin_amdgcn_raw_buffer_store_b64(v, result_buffer(out), off, 0, kThrough);
+}
+__device__ __forceinline__ void store_through(void *out, unsigned off, Words4 v)
+{
+    __builtin_amdgcn_raw_buffer_store_b128(v, result_buffer(out), off, 0, kThrough);
+}
+
 // Called by every thread of a workgroup after its last store_result.  Those are written through, so their
 // acknowledgement is enough to count on; the fence of the last workgroup covers results of launches before.
 __device__ __forceinline__ void raise_when_last(const DoneSignal &done)

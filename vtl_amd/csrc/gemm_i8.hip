@@ -37,13 +37,13 @@ using vtlhip::HostResult;
 using vtlhip::raise_when_last;
 using vtlhip::store_result;
 
-// Four of them in a row, 16-byte aligned unless they are written through.
-__device__ __forceinline__ void store_result4(float *p, f4 v, const vtlhip::DoneSignal &done)
+// Four of them from element `at` of out, 16-byte aligned unless they are written through (a host call's result: a few MiB).
+__device__ __forceinline__ void store_result4(float *out, int64_t at, f4 v, const vtlhip::DoneSignal &done)
 {
     if (done.flag)   // waited for in raise_when_last
-        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(p), "v"(v) : "memory");
+        vtlhip::store_through(out, (unsigned)at * 4u, __builtin_bit_cast(vtlhip::Words4, v));
     else
-        *reinterpret_cast<f4 *>(p) = v;
+        *reinterpret_cast<f4 *>(out + at) = v;
 }
 
 struct GemmArgs {
@@ -661,11 +661,11 @@ __device__ __forceinline__ void finalize_outputs(const GemmArgs &g, int64_t idx,
             if (g.relu && y[j] < 0.0f)
                 y[j] = 0.0f;
         }
-        float *out = reinterpret_cast<float *>(g.out) + idx;
+        float *out = reinterpret_cast<float *>(g.out);
         if (VEC == 4)
-            store_result4(out, f4{y[0], y[1], y[2], y[3]}, g.done);
+            store_result4(out, idx, f4{y[0], y[1], y[2], y[3]}, g.done);
         else
-            store_result(out, y[0], g.done);
+            store_result(out + idx, y[0], g.done);
     } else {
         int32_t *out = reinterpret_cast<int32_t *>(g.out) + idx;
         if (VEC == 4) {
@@ -1190,7 +1190,7 @@ __global__ __launch_bounds__(64 * NWAVE) void linear_skinny_kernel(const GemmArg
                 }
             }
             if (n + 3 < N && ((N & 3) == 0 || g.done.flag)) {
-                store_result4(reinterpret_cast<float *>(g.out) + o, f4{y[0], y[1], y[2], y[3]}, g.done);
+                store_result4(reinterpret_cast<float *>(g.out), o, f4{y[0], y[1], y[2], y[3]}, g.done);
             } else {
 #pragma unroll
                 for (int k = 0; k < 4; k++)

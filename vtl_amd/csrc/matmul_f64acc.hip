@@ -7,9 +7,11 @@
 //
 // matmul_f64acc_direct_kernel takes operands from global memory straight to registers; choose_plan() picks its
 // shape by estimated time.
-#include "common.hpp"
-
 #include <stdlib.h>
+
+#include <type_traits>
+
+#include "common.hpp"
 
 namespace {
 
@@ -84,7 +86,7 @@ template <bool THROUGH>
 __device__ __forceinline__ void store_run(__amdgpu_buffer_rsrc_t base, unsigned off, unsigned along, float a, float b)
 {
     typedef unsigned Two __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(Two{__float_as_uint(a), __float_as_uint(b)}, base, off, along, THROUGH ? 17 : 0);   // sc0 sc1
+    __builtin_amdgcn_raw_buffer_store_b64(Two{__float_as_uint(a), __float_as_uint(b)}, base, off, along, THROUGH ? vtlhip::kThrough : 0);
 }
 
 template <bool THROUGH>
@@ -93,7 +95,7 @@ __device__ __forceinline__ void store_run(__amdgpu_buffer_rsrc_t base, unsigned 
     typedef unsigned Four __attribute__((ext_vector_type(4)));
     const unsigned long long ua = (unsigned long long)__double_as_longlong(a), ub = (unsigned long long)__double_as_longlong(b);
     __builtin_amdgcn_raw_buffer_store_b128(Four{(unsigned)ua, (unsigned)(ua >> 32), (unsigned)ub, (unsigned)(ub >> 32)}, base, off,
-                                           along, THROUGH ? 17 : 0);
+                                           along, THROUGH ? vtlhip::kThrough : 0);
 }
 
 // One pair of rows or columns of an operand for the lanes of a wave.
@@ -164,25 +166,18 @@ __device__ __forceinline__ void checked_fetch(T (&out)[2][4], const T *__restric
         }
 }
 
-// Two neighbours of a row, aligned as one element is.
-__device__ __forceinline__ void store_pair(float *p, float a, float b, const vtlhip::DoneSignal &done)
+// Two neighbours of a row from element `at` of out, aligned as one element is (written through, to a host call's result: a
+// few MiB).
+template <typename T>
+__device__ __forceinline__ void store_pair(T *out, int64_t at, T a, T b, const vtlhip::DoneSignal &done)
 {
-    typedef float Two __attribute__((ext_vector_type(2), aligned(4)));
+    typedef T Two __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+    using Words = std::conditional_t<sizeof(T) == 4, vtlhip::Words2, vtlhip::Words4>;
     const Two v = {a, b};
     if (done.flag)   // waited for in raise_when_last
-        asm volatile("global_store_dwordx2 %0, %1, off sc0 sc1" ::"v"(p), "v"(v) : "memory");
+        vtlhip::store_through(out, (unsigned)at * (unsigned)sizeof(T), __builtin_bit_cast(Words, v));
     else
-        *reinterpret_cast<Two *>(p) = v;
-}
-
-__device__ __forceinline__ void store_pair(double *p, double a, double b, const vtlhip::DoneSignal &done)
-{
-    typedef double Two __attribute__((ext_vector_type(2), aligned(8)));
-    const Two v = {a, b};
-    if (done.flag)
-        asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1" ::"v"(p), "v"(v) : "memory");
-    else
-        *reinterpret_cast<Two *>(p) = v;
+        *reinterpret_cast<Two *>(out + at) = v;
 }
 
 __device__ __forceinline__ void tile_of_block(int block, int tiles_m, int tiles_n, int &tm, int &tn)
@@ -396,11 +391,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
             if (g.relu && y[u] < T(0))
                 y[u] = T(0);
         }
-        T *to = C + ((int64_t)r * g.N + c);
+        const int64_t at = (int64_t)r * g.N + c;
         if (both)
-            store_pair(to, y[0], y[1], g.done);
+            store_pair(C, at, y[0], y[1], g.done);
         else
-            vtlhip::store_result(to, y[0], g.done);
+            vtlhip::store_result(C + at, y[0], g.done);
     };
     if constexpr (WK == 1) {
         // Nothing but conversions and stores: what `store` asks of every pair is asked once for the tile.  No vector
