@@ -127,7 +127,9 @@ def test_odd_k_and_unaligned_operands_are_repacked(hip, mnk):
 # 32 with an edge, the limits of the rule (256 tiles, K = 2560), and both routes forced.
 RAGGED_SHAPES = [(1, 1, 1), (3, 40, 15), (33, 31, 17), (32, 33, 31), (1, 300, 33), (40, 64, 63), (1, 65, 255), (1, 4100, 257),
                  (1, 9, 14335), (2, 70, 1023), (2, 2050, 1025), (3, 129, 4097), (4, 1000, 8191), (5, 31, 2049), (8, 1001, 4095),
-                 (7, 300, 511), (9, 100, 1900), (16, 1001, 1901), (65, 97, 2561), (64, 4096, 129), (513, 511, 127)]
+                 (7, 300, 511), (9, 100, 1900), (16, 1001, 1901), (65, 97, 2561), (64, 4096, 129), (513, 511, 127),
+                 # fewer weight rows in flight than where rows are whole, half as many waves, each side of the rule
+                 (1, 2100, 4097), (1, 2100, 11265), (2, 65, 4097), (2, 810, 11263), (3, 40, 8191), (4, 1030, 3585), (6, 800, 2391)]
 
 
 @pytest.mark.parametrize("route", ["1", "0", None])
@@ -165,6 +167,32 @@ def test_ragged_rows_as_they_are_and_padded(hip, mnk, route, knobs):
     capi.call("vtl_hip_layer_f32", ctypes.byref(layer), X.ptr, Y.ptr, m, 0, ws.ptr, ws.size)
     assert np.array_equal(Y.cpu(), want)
     for h in (abuf, bbuf, cbuf, dsa, dsb, dbias, X, Y, ws, rows):
+        h.release()
+
+
+# Weights in padded rows, read as whole ones, with f32 rows of any length at any address: the limits of a piece of
+# 1024, of a wave's share of the chip (6144) and of the longest rows, each number of rows, and rows as long as the padded ones.
+@pytest.mark.parametrize("mnk", [(1, 300, 257), (1, 5000, 1009), (1, 4100, 6143), (1, 2100, 6145), (1, 70, 11265), (1, 9, 14335),
+                                 (2, 600, 1023), (2, 70, 4095), (3, 40, 2047), (4, 1030, 1025), (5, 33, 257), (7, 300, 1001),
+                                 (8, 4097, 1023), (1, 100, 4096), (2, 100, 2048)])
+def test_f32_rows_of_any_length_against_padded_weights(hip, mnk, knobs):
+    m, n, k = mnk
+    rng = np.random.default_rng(m + n + k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    wq, sw, bias = rng.integers(-127, 128, (n, k), dtype=np.int8), rng.uniform(1e-3, 1e-2, n).astype(np.float32), rng.standard_normal(n).astype(np.float32)
+    want = oracle.linear_f32_dynquant(x, wq, sw, bias)
+    row = capi.lib().vtl_hip_padded_row(k)
+    xbuf, Wq, rows, Sw, B, Y = raw_device_buffer(x.nbytes + 16), dev(wq), HipTensor.empty([n, row], np.int8), dev(sw), dev(bias), HipTensor.empty([m, n], np.float32)
+    capi.call("vtl_hip_pad_rows_i8", Wq.ptr, n, k, rows.ptr)
+    layer = capi.Layer(capi.LAYER_LINEAR, 1, n, k, rows.ptr, Sw.ptr, B.ptr, row)
+    for route in (None, "0"):
+        if route:
+            knobs.setenv("VTL_HIP_RAGGED", route)
+        for off in (0, 4) if route is None else (0,):
+            h2d(xbuf.ptr + off, x)
+            capi.call("vtl_hip_layer_f32", ctypes.byref(layer), xbuf.ptr + off, Y.ptr, m, 0, None, 0)
+            assert np.array_equal(Y.cpu(), want), (route, off)
+    for h in (xbuf, Wq, rows, Sw, B, Y):
         h.release()
 
 

@@ -81,8 +81,8 @@ struct GemmArgs {
     // Weight-streaming kernel with up to 32 rows (every weight is read once): read the weights
     // with non-temporal loads.  Set by the size of the matrix, see stream_weights_from.
     int stream_weights;
-    // Matrix-vector kernels, RAGGED and quantizing xf32 themselves: its row length (K, or less where the
-    // weights lie in padded rows).
+    // Matrix-vector kernels that are not for kWhole rows and quantize xf32 themselves: its row length (K, or less
+    // where the weights lie in padded rows).
     int x_cols;
     // Where `out` is the memory of a whole host call's result: the kernels that can raise its flag do.
     vtlhip::DoneSignal done;
@@ -1295,6 +1295,18 @@ __device__ __forceinline__ f4 load_floats(const float *row, int c, int n)
     return r;
 }
 
+// What rows a matrix-vector kernel takes.  kWhole: K % 16 == 0, operands 16-byte aligned.  kPadded: so are the weights, in
+// rows of K codes, and the activations are f32 rows of x_cols <= K values anywhere.  kRagged: K >= 16 of any remainder, codes
+// and values anywhere; a lane reads a fifth word with every 16 bytes of weights.
+enum Rows { kWhole, kPadded, kRagged };
+
+// Ragged weight rows in flight beside the one at work, up to `most`: as many as fit 256 registers with the codes of `mr`
+// rows (four rows of 8192 codes with two spilled 34 registers, one of 14336 66).
+constexpr int ragged_depth(int kv, int mr, int most)
+{
+    return most > 1 && 4 * kv * mr + 5 * kv * (most + 1) + 40 > 256 ? ragged_depth(kv, mr, most - 1) : most;
+}
+
 // Single token (M = 1): a matrix-vector product bound by reading Wq once, done
 // without LDS staging and without MFMA.  With DYNQ the row arrives as f32 and
 // every workgroup quantizes it itself (K floats from L2, the arithmetic of the
@@ -1306,14 +1318,14 @@ __device__ __forceinline__ f4 load_floats(const float *row, int c, int n)
 // registers (cached loads: between launches the weights stay in the last-level
 // cache, non-temporal ones measured 20-40 % slower), two rows are in flight
 // while the current one goes through 4 * KV dot4 instructions and a
-// cross-lane sum.  Requires K % 16 == 0, the row and Wq 16-byte aligned; RAGGED: K >= 16 of any
-// remainder, codes at any address.
-template <int KV, int NWAVE, bool DYNQ, bool F32OUT, bool WNT = false, bool RAGGED = false>
+// cross-lane sum.
+template <int KV, int NWAVE, bool DYNQ, bool F32OUT, bool WNT = false, Rows ROWS = kWhole>
 __global__ __launch_bounds__(64 * NWAVE) void linear_gemv_kernel(const GemmArgs g)
 {
     constexpr int T = 64 * NWAVE;
     constexpr int XV = (256 * KV + T - 1) / T;  // float4 of x per thread
-    constexpr int DEPTH = 2, RING = DEPTH + 1;
+    constexpr bool RAGGED = ROWS == kRagged;
+    constexpr int DEPTH = RAGGED ? ragged_depth(KV, 1, 2) : 2, RING = DEPTH + 1;
     __shared__ float red[NWAVE], parked[F32OUT ? 64 : 1][NWAVE];
     __shared__ __attribute__((aligned(16))) int8_t xq[DYNQ ? 1024 * KV : 16];
     const int N = g.N, K = g.K;
@@ -1333,7 +1345,7 @@ __global__ __launch_bounds__(64 * NWAVE) void linear_gemv_kernel(const GemmArgs 
 #pragma unroll
         for (int i = 0; i < XV; i++) {
             const int idx = i * T + threadIdx.x;
-            if constexpr (RAGGED)
+            if constexpr (ROWS != kWhole)
                 xr[i] = load_floats(g.xf32, 4 * idx, g.x_cols);
             else
                 xr[i] = idx < (K >> 2) ? xv[idx] : f4{0.f, 0.f, 0.f, 0.f};
@@ -1518,12 +1530,12 @@ __device__ __forceinline__ int wave_sum_rows(int (&a)[MR], int lane)
 // the work (the arithmetic of the row quantizer), and the codes are exchanged
 // through LDS.  Sums are parked
 // 64 / MR weight rows at a time (lane l: row l % MR, weight row l / MR of the
-// batch) and then scaled and stored.  Requires K % 16 == 0, K <= 1024 * KV,
-// operands 16-byte aligned; RAGGED: K >= 16 of any remainder, codes at any address.
-template <int KV, int MR, int DEPTH, bool DYNQ, bool F32OUT, bool WNT = false, bool RAGGED = false>
+// batch) and then scaled and stored.  Requires K <= 1024 * KV.
+template <int KV, int MR, int DEPTH, bool DYNQ, bool F32OUT, bool WNT = false, Rows ROWS = kWhole>
 __global__ __launch_bounds__(512) void linear_gemv_rows_kernel(const GemmArgs g)
 {
     constexpr int NWAVE = 8;
+    constexpr bool RAGGED = ROWS == kRagged;
     constexpr int RING = DEPTH + 1;
     constexpr int SLOTS = 64 / MR;
     __shared__ float s_sa[MR], s_rinv[MR];
@@ -1549,7 +1561,7 @@ __global__ __launch_bounds__(512) void linear_gemv_rows_kernel(const GemmArgs g)
 #pragma unroll
         for (int i = 0; i < XV; i++) {
             const int f = i * 512 + (int)threadIdx.x, row = f / PIECES, col = f % PIECES;
-            if constexpr (RAGGED)
+            if constexpr (ROWS != kWhole)
                 xr[i] = load_floats(g.xf32 + (int64_t)row * g.x_cols, 4 * col, row < M ? g.x_cols : 0);
             else
                 xr[i] = (row < M && col < (K >> 2))
@@ -2316,32 +2328,33 @@ inline int skinny_blocks_waves(int M, int N, int K)
 }
 
 // Waves of the single-token kernel's grid: no more than the chip holds at once, sixteen per
-// compute unit up to 6144 codes a row, eight beyond (the codes and three weight rows of a wave
+// compute unit up to 6144 codes a row (4096 where rows are ragged), eight beyond (the codes and three weight rows of a wave
 // take 150 to 250 registers then).
-inline int gemv_max_waves(int K) { return K <= 6144 ? 4096 : 2048; }
+inline int gemv_max_waves(int K, Rows rows = kWhole) { return K <= (rows == kRagged ? 4096 : 6144) ? 4096 : 2048; }
 
-// Single-token linear (M = 1, K % 16 == 0, K <= 14336, operands 16-byte aligned; RAGGED: K >= 16).
-template <bool DYNQ, bool F32OUT, bool RAGGED = false>
+// Single-token linear (M = 1, K <= 14336).
+template <bool DYNQ, bool F32OUT, Rows ROWS = kWhole>
 int launch_gemv(const GemmArgs &g_in, hipStream_t st)
 {
     GemmArgs g = g_in;
     constexpr int NWAVE = 8;
     // every wave the same number of rows
-    const int max_waves = gemv_max_waves(g.K);
+    const int max_waves = gemv_max_waves(g.K, ROWS);
     const int rows_per_wave = (g.N + max_waves - 1) / max_waves;
     if (rows_per_wave > 64)   // more rows than a wave has lanes to park their sums in
         return VTL_HIP_ERR_UNSUPPORTED;
     const int64_t waves = (g.N + rows_per_wave - 1) / rows_per_wave;
     const dim3 grid((unsigned)((waves + NWAVE - 1) / NWAVE)), block(64 * NWAVE);
     attach_gemv_result(g, grid.x, true);
-    // the cache policy is part of the load instruction (RAGGED: always cached, half as many kernels to load)
-    const bool wnt = !RAGGED && stream_weights_from(g.N, g.K, 8);
+    // The cache policy is part of the load instruction.  Ragged rows: always cached, their lines are read for two lanes
+    // (1 x 14336 x 4095 repeated 12.1 us, with non-temporal loads 16.2; from HBM 15.5 and 16.1).
+    const bool wnt = ROWS != kRagged && stream_weights_from(g.N, g.K, 8);
 #define VTL_GEMV(KV)                                                                                        \
     do {                                                                                                    \
         if (wnt)                                                                                            \
-            hipLaunchKernelGGL((linear_gemv_kernel<KV, NWAVE, DYNQ, F32OUT, !RAGGED, RAGGED>), grid, block, 0, st, g); \
+            hipLaunchKernelGGL((linear_gemv_kernel<KV, NWAVE, DYNQ, F32OUT, ROWS != kRagged, ROWS>), grid, block, 0, st, g); \
         else                                                                                                \
-            hipLaunchKernelGGL((linear_gemv_kernel<KV, NWAVE, DYNQ, F32OUT, false, RAGGED>), grid, block, 0, st, g); \
+            hipLaunchKernelGGL((linear_gemv_kernel<KV, NWAVE, DYNQ, F32OUT, false, ROWS>), grid, block, 0, st, g); \
     } while (0)
     switch ((g.K + 1023) / 1024) {
     case 1: VTL_GEMV(1); break;
@@ -2362,13 +2375,14 @@ int launch_gemv(const GemmArgs &g_in, hipStream_t st)
 }
 
 // A few tokens (2 <= M <= 8): rows of up to 11264 (2 tokens), 8192 (4) or 4096 (8) codes.
-template <int KV, int MR, bool DYNQ, bool F32OUT, bool RAGGED>
+template <int KV, int MR, bool DYNQ, bool F32OUT, Rows ROWS>
 int launch_gemv_rows_kv(GemmArgs g, hipStream_t st)
 {
     constexpr int NWAVE = 8;
     // Codes and weight rows live in registers, which limits the waves a SIMD holds; with few
     // waves a third weight row in flight per wave keeps enough bytes on their way from HBM.
-    constexpr int DEPTH = (MR * KV >= 16 && 4 * KV * (MR + 4) + 40 <= 256) ? 3 : 2;
+    constexpr int WHOLE = (MR * KV >= 16 && 4 * KV * (MR + 4) + 40 <= 256) ? 3 : 2;
+    constexpr int DEPTH = ROWS == kRagged ? ragged_depth(KV, MR, WHOLE) : WHOLE;
     constexpr int REGS = 4 * KV * (MR + DEPTH + 1) + 40;
     // a workgroup of 8 waves puts two on every SIMD: whole workgroups only
     constexpr int OCC = 512 / REGS >= 8 ? 8 : (512 / REGS >= 2 ? (512 / REGS) & ~1 : 2);
@@ -2379,43 +2393,43 @@ int launch_gemv_rows_kv(GemmArgs g, hipStream_t st)
         return VTL_HIP_ERR_UNSUPPORTED;  // not routed here: a quantizer launch of its own is cheaper
     } else {
         attach_gemv_result(g, grid.x, rows_per_wave <= 64 / MR);
-        if (!RAGGED && stream_weights_from(g.N, g.K, tuning().stream_weights_mib))   // (the cache policy is part of the load instruction)
-            hipLaunchKernelGGL((linear_gemv_rows_kernel<KV, MR, DEPTH, DYNQ, F32OUT, !RAGGED, RAGGED>), grid, block, 0, st, g);
+        if (ROWS != kRagged && stream_weights_from(g.N, g.K, tuning().stream_weights_mib))   // (the cache policy is part of the load instruction)
+            hipLaunchKernelGGL((linear_gemv_rows_kernel<KV, MR, DEPTH, DYNQ, F32OUT, ROWS != kRagged, ROWS>), grid, block, 0, st, g);
         else
-            hipLaunchKernelGGL((linear_gemv_rows_kernel<KV, MR, DEPTH, DYNQ, F32OUT, false, RAGGED>), grid, block, 0, st, g);
+            hipLaunchKernelGGL((linear_gemv_rows_kernel<KV, MR, DEPTH, DYNQ, F32OUT, false, ROWS>), grid, block, 0, st, g);
         return check_launch("linear_gemv_rows_kernel");
     }
 }
 
-template <int MR, bool DYNQ, bool F32OUT, bool RAGGED>
+template <int MR, bool DYNQ, bool F32OUT, Rows ROWS>
 int launch_gemv_rows_mr(const GemmArgs &g, hipStream_t st)
 {
     const int kv = (g.K + 1023) / 1024;
     if (kv <= 1)
-        return launch_gemv_rows_kv<1, MR, DYNQ, F32OUT, RAGGED>(g, st);
+        return launch_gemv_rows_kv<1, MR, DYNQ, F32OUT, ROWS>(g, st);
     if (kv <= 2)
-        return launch_gemv_rows_kv<2, MR, DYNQ, F32OUT, RAGGED>(g, st);
+        return launch_gemv_rows_kv<2, MR, DYNQ, F32OUT, ROWS>(g, st);
     if (kv <= 4)
-        return launch_gemv_rows_kv<4, MR, DYNQ, F32OUT, RAGGED>(g, st);
+        return launch_gemv_rows_kv<4, MR, DYNQ, F32OUT, ROWS>(g, st);
     if constexpr (MR <= 4) {
         if (kv <= 8)
-            return launch_gemv_rows_kv<8, MR, DYNQ, F32OUT, RAGGED>(g, st);
+            return launch_gemv_rows_kv<8, MR, DYNQ, F32OUT, ROWS>(g, st);
     }
     if constexpr (MR <= 2) {
         if (kv <= 11)
-            return launch_gemv_rows_kv<11, MR, DYNQ, F32OUT, RAGGED>(g, st);
+            return launch_gemv_rows_kv<11, MR, DYNQ, F32OUT, ROWS>(g, st);
     }
     return VTL_HIP_ERR_UNSUPPORTED;  // not reached: see gemv_rows_applies
 }
 
-template <bool DYNQ, bool F32OUT, bool RAGGED = false>
+template <bool DYNQ, bool F32OUT, Rows ROWS = kWhole>
 int launch_gemv_rows(const GemmArgs &g, hipStream_t st)
 {
     if (g.M <= 2)
-        return launch_gemv_rows_mr<2, DYNQ, F32OUT, RAGGED>(g, st);
+        return launch_gemv_rows_mr<2, DYNQ, F32OUT, ROWS>(g, st);
     if (g.M <= 4)
-        return launch_gemv_rows_mr<4, DYNQ, F32OUT, RAGGED>(g, st);
-    return launch_gemv_rows_mr<8, DYNQ, F32OUT, RAGGED>(g, st);
+        return launch_gemv_rows_mr<4, DYNQ, F32OUT, ROWS>(g, st);
+    return launch_gemv_rows_mr<8, DYNQ, F32OUT, ROWS>(g, st);
 }
 
 // The codes of the MR rows stay in registers: at most 32 pieces of 16 bytes per lane (22 for two rows:
@@ -2468,21 +2482,24 @@ inline bool gemv_applies(const void *row, const void *w, int N, int K)
            !tuning().no_gemv;
 }
 
-// The matrix-vector kernels' RAGGED forms: rows of K codes, K no multiple of 16 or operands not aligned.
-inline bool gemv_takes_ragged(int M, int N, int K)
+// The matrix-vector kernels' forms for other rows than whole ones.
+inline bool gemv_takes_ragged(int M, int N, int K, Rows rows = kRagged)
 {
     if (tuning().no_gemv || K < 256)
         return false;
-    return M == 1 ? K <= 14336 && N <= 64 * gemv_max_waves(K)
+    return M == 1 ? K <= 14336 && N <= 64 * gemv_max_waves(K, rows)
                   : M >= 2 && M <= 8 && K <= (M <= 2 ? 11264 : (M <= 4 ? 8192 : 4096));
 }
 
-// Against padding both operands and the kernel for that (one row, four rows of N = 64 ... 4000, K = 533 ... 4090: 6 to
-// 14 us, here 3.3 to 7).  With five to eight rows the kernel's own work outweighs the padding of few
-// long weight rows (8 x 64 x 4087 7.6 against 9.0 us, 8 x 1001 x 4087 9.5 and 9.2, 8 x 4001 x 2047 12.4 and 6.7).
+// Against padding both operands and the kernel for that (codes quantized right before, weights repeated and from HBM; K = 257 ... 14335,
+// N = 64 ... 14336).  One row: always, but for a few weight rows of more than 10000 codes (level).  Two to eight: the
+// kernel's own work grows with the codes that every workgroup reads, the padding with the weights: with more than 14 codes
+// for a weight row it is behind (2 x 64 x 8191 12.6 against 11.1 us, 4 x 1000 x 8191 17.6 and 14.8, 8 x 1000 x 3001 15.3 and 12.7;
+// 2 x 1000 x 8191 13.0 and 14.3, 4 x 3000 x 6143 16.5 and 20.0, 8 x 3000 x 4095 19.0 and 18.8), unless there are few (4 x
+// 64 x 3001 10.7 and 10.9, 8 x 64 x 1800 10.6 and 10.6).
 inline bool gemv_ragged_faster(int M, int N, int K)
 {
-    return gemv_takes_ragged(M, N, K) && (M <= 4 || K <= 2048 || N >= 1000);
+    return gemv_takes_ragged(M, N, K) && (M == 1 || M * K <= 14336 || 14 * (int64_t)N >= M * K);
 }
 
 // Where the small-product kernel takes ragged rows as they are faster than padding and the kernel for padded
@@ -2541,7 +2558,7 @@ int launch_gemm(const GemmArgs &g_in, hipStream_t st)
         const int ragged = tuning().ragged;
         if constexpr (F32OUT) {   // (int32 sums of a few ragged rows are nobody's hot path: no kernels for them)
             if (ragged < 0 ? gemv_ragged_faster(g.M, g.N, g.K) : ragged && gemv_takes_ragged(g.M, g.N, g.K))
-                return g.M == 1 ? launch_gemv<false, true, true>(g, st) : launch_gemv_rows<false, true, true>(g, st);
+                return g.M == 1 ? launch_gemv<false, true, kRagged>(g, st) : launch_gemv_rows<false, true, kRagged>(g, st);
         }
         const int64_t t32 = (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32);
         if (ragged < 0 ? small_ragged_faster(g.M, g.N, g.K) : ragged && t32 <= 0x7fffffff)
@@ -2616,20 +2633,27 @@ const int8_t *pad_activations(const int8_t *A, int M, int K, int row, int &statu
 }
 
 // Up to eight f32 rows of x_cols elements against weights in rows of `row` codes (x_cols, or padded), in one launch
-// where the aligned forms of the kernels would not take them; -1: not taken.
+// where the kernels for whole rows would not take them; -1: not taken.
+template <Rows ROWS>
+int launch_rows_quantized(const GemmArgs &g)
+{
+    if (!gemv_takes_ragged(g.M, g.N, g.K, ROWS))
+        return -1;
+    if (g.M == 1)
+        return launch_gemv<true, true, ROWS>(g, current_stream());
+    return gemv_rows_fused_quant_faster(g.M, g.N, g.K) ? launch_gemv_rows<true, true, ROWS>(g, current_stream()) : -1;
+}
+
 int launch_ragged_rows(const float *X, int x_cols, const int8_t *Wq, int row, const float *sw, const float *bias, float *Y,
                        int M, int N, int relu, HostResult *result)
 {
-    if ((row == x_cols && row % 16 == 0 && aligned16(X) && aligned16(Wq)) || tuning().no_fused_decode || !tuning().ragged)
+    const bool whole_weights = row % 16 == 0 && aligned16(Wq);
+    if ((row == x_cols && whole_weights && aligned16(X)) || tuning().no_fused_decode || !tuning().ragged)
         return -1;
     GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, row, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
     g.x_cols = x_cols;
     g.result = result;
-    if (M == 1 && gemv_takes_ragged(M, N, row))
-        return launch_gemv<true, true, true>(g, current_stream());
-    if (gemv_takes_ragged(M, N, row) && gemv_rows_fused_quant_faster(M, N, row))
-        return launch_gemv_rows<true, true, true>(g, current_stream());
-    return -1;
+    return whole_weights ? launch_rows_quantized<kPadded>(g) : launch_rows_quantized<kRagged>(g);
 }
 
 bool layer_row_fits(const vtl_hip_layer &l)
