@@ -124,8 +124,8 @@ def test_last_round_cut_by_k(hip, slices, mnk, knobs):
         t.release()
 
 
-# (the shapes that only f64 with K along both operands' rows has, and the others at the edges of the largest tiles;
-# columns beyond a lane's 32-bit offset are checked load by load)
+# (the shapes that only f64 with K along both operands' rows has, and the others at the edges of the largest tiles, and
+# of long rows)
 @pytest.mark.parametrize("shape", ["4", "5", "6"])
 @pytest.mark.parametrize("mnk", [(64, 64, 16), (65, 63, 113), (129, 130, 47), (127, 2, 33), (2, 129, 300), (200, 70, 64),
                                  (3, (1 << 22) + 1, 5)])
@@ -146,6 +146,26 @@ def test_large_shapes_at_their_edges(hip, shape, mnk, knobs):
                 assert np.array_equal(y.cpu(), np.maximum(exact + bias, 0).astype(dt)), dt
                 for t in (x, w, b, y):
                     t.release()
+
+
+# Either side of where 32-bit offsets end: rows of C (64 to a wave), rows with K along them (64), rows with K across (16).  Many
+# rows, and K across many, end nowhere.  Whole values: sums are exact, and so is their rounding.
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("case", ["many rows", "long K across", "long K along", "long rows of C", "long rows of B"])
+def test_products_at_the_end_of_32_bit_offsets(hip, case, dt):
+    along, across = ((1 << 32) - 1) // (64 * np.dtype(dt).itemsize), ((1 << 32) - 1) // (16 * np.dtype(dt).itemsize)
+    rng = np.random.default_rng(len(case))
+    for M, N, K, ta, tb in {"many rows": [((1 << 22) + 1, 3, 5, False, True), ((1 << 22) + 1, 3, 18, False, False)],
+                            "long K across": [(3, 5, (1 << 22) + 1, True, False), (34, 2, along + 1, True, False)],
+                            "long K along": [(3, 2, along, False, True), (2, 3, along + 1, False, True), (2, 2, along + 1, False, False)],
+                            "long rows of C": [(34, along, 2, False, True), (34, along + 1, 2, False, True)],
+                            "long rows of B": [(2, across, 3, False, False), (2, across + 1, 3, False, False)]}[case]:
+        print(case, M, N, K, ta, tb, flush=True)
+        A = rng.integers(-9, 10, (K, M) if ta else (M, K), dtype=np.int8).astype(dt)
+        B = rng.integers(-9, 10, (N, K) if tb else (K, N), dtype=np.int8).astype(dt)
+        got = run_matmul(A, B, ta, tb)
+        exact = (A.T if ta else A).astype(np.float64) @ (B.T if tb else B).astype(np.float64)
+        assert np.array_equal(got, exact.astype(dt)), (M, N, K, ta, tb)
 
 
 @pytest.mark.parametrize("tile", ["64", "128"])

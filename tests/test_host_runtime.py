@@ -104,6 +104,31 @@ print("done")
 """)
 
 
+def test_long_products_take_vector_loads(fake_runtime):
+    """Only rows too long for a lane's 32-bit offset are loaded element by element: how many rows there are, or how long K is
+    where it runs across them, does not matter (a forward over five million rows, its dW)."""
+    _run(fake_runtime, _PRODUCTS + r"""
+import re
+def checked(name, m, n, k, ta, tb):
+    events()
+    assert capi.status("vtl_hip_matmul_" + name, p, p, p, m, n, k, ta, tb) == capi.OK     # no kernel runs here
+    flags = [re.search(r"direct_kernelI\wLi.*?Lb(\d)ELb(\d)ELb(\d)E", l[4]) for l in lines() if l[0] == "launch"]
+    flags = [f.groups() for f in flags if f]
+    assert len(flags) == 1 and flags[0][:2] == (str(ta), str(tb)), flags
+    return flags[0][2] == "1"
+MANY = 5000000
+for name, size in (("f32", 4), ("f64", 8)):
+    along, across = ((1 << 32) - 1) // (64 * size), ((1 << 32) - 1) // (16 * size)
+    for case in [(MANY, 64, 64, 0, 1), (MANY, 64, 64, 0, 0), (64, 64, MANY, 1, 0), (64, MANY, 64, 0, 1), (MANY, 7, 5, 1, 0), (5, MANY, 64, 0, 0),
+                 (64, 64, MANY, 0, 0), (64, 64, along, 0, 1), (across, 3, 5, 1, 0), (3, across, 5, 0, 0), (64, 64, 1 << 28, 1, 0)]:
+        assert not checked(name, *case), (name, case)
+    for case in [(64, 64, along + 1, 0, 1), (64, 64, along + 1, 0, 0), (64, 64, along + 1, 1, 1), (across + 1, 3, 5, 1, 0),
+                 (3, across + 1, 5, 0, 0), (1, 64, 64, 1, 0), (64, 1, 64, 0, 0)]:
+        assert checked(name, *case), (name, case)
+print("done")
+""")
+
+
 def test_copies_run_where_the_memory_is(fake_runtime):
     """Memory of device 0 is copied after something was allocated on device 1: the kernel that carries the
     bytes runs on device 0, and device 1 is current again afterwards.  On a stream of the caller's the copy is

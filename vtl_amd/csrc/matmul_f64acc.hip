@@ -61,9 +61,16 @@ struct alignas(16) Vec4 {
 // each lane's four: which k they are is free as long as both operands agree.
 // Vector loads need no more than the elements' own alignment on gfx950, so ragged rows take them too;
 // what is left of K after whole steps is a step of its own with checked loads.  CHECKED: every
-// load is (a single row or column of a matrix that has to give pairs, sizes beyond a lane's 32-bit offset).
+// load is (a single row or column of a matrix that has to give pairs, rows too long for a lane's 32-bit offset).
 template <typename T>
 constexpr int kRun = 16 / (int)sizeof(T);   // elements of a 16-byte load; the lane's four are those of each run of 4 * kRun
+
+// The longest rows that offsets of 32 bits reach over.  Where K runs along them a wave covers up to 64; where it runs across
+// them, a step's 16.  Neither limits how many rows there are: their first is a scalar.
+template <typename T>
+constexpr int kLongest64 = (int)(0xffffffffu / (64 * sizeof(T)));
+template <typename T>
+constexpr int kLongest16 = (int)(0xffffffffu / (16 * sizeof(T)));
 
 // N elements at `off` bytes (a lane's own) + `along` from base, one load.
 template <typename T, int N>
@@ -349,10 +356,10 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
     // Value v of a lane: i = v / (4 TN), j = v / 4 % TN, e = v % 4.  Values v and v + 4 of an even j are
     // neighbours in a row and stored together: whole lines of 16 lanes.
     // Inside the matrix a store's address is a scalar and a lane's offset too.
-    const bool inside = !CHECKED && !partial && m0 + 16 * TM <= g.M && n0 + 16 * TN <= g.N;
+    const bool inside = !CHECKED && !partial && m0 + 16 * TM <= g.M && n0 + 16 * TN <= g.N && g.N <= kLongest64<T>;
     const __amdgpu_buffer_rsrc_t tile_out =
         __builtin_amdgcn_make_buffer_rsrc(C + (inside ? (int64_t)m0 * g.N + n0 : 0), 0, 0xffffffff, 0x00027000);
-    const unsigned lane_out = (unsigned)(2 * kq * g.N + 2 * r16) * (unsigned)sizeof(T);
+    const unsigned lane_out = (2u * kq * (unsigned)g.N + 2u * r16) * (unsigned)sizeof(T);
     auto store = [&](int v, double s0, double s1) {
         const int i = v / (4 * TN), j = (v >> 2) % TN;
         if (inside) {
@@ -366,7 +373,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
                 y[0] = y[0] < T(0) ? T(0) : y[0];
                 y[1] = y[1] < T(0) ? T(0) : y[1];
             }
-            const unsigned along = (unsigned)((32 * (i >> 1) + 8 * (v & 3) + (i & 1)) * g.N + 32 * (j >> 1)) * (unsigned)sizeof(T);
+            const unsigned along = ((unsigned)(32 * (i >> 1) + 8 * (v & 3) + (i & 1)) * (unsigned)g.N + 32u * (j >> 1)) * (unsigned)sizeof(T);
             if (g.done.flag)
                 store_run<true>(tile_out, lane_out, along, y[0], y[1]);
             else
@@ -406,7 +413,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
             for (int v = 0; v < V; ++v)
                 if (!(v & 4)) {
                     const int i = v / (4 * TN), j = (v >> 2) % TN;
-                    const unsigned along = (unsigned)((32 * (i >> 1) + 8 * (v & 3) + (i & 1)) * g.N + 32 * (j >> 1)) * (unsigned)sizeof(T);
+                    const unsigned along = ((unsigned)(32 * (i >> 1) + 8 * (v & 3) + (i & 1)) * (unsigned)g.N + 32u * (j >> 1)) * (unsigned)sizeof(T);
                     store_run<false>(tile_out, lane_out, along, (T)acc[i][j][v & 3], (T)acc[i][j + 1][v & 3]);
                 }
             return;   // no signal to raise
@@ -733,9 +740,9 @@ struct Partial {
 template <typename T>
 int launch_direct(MatmulArgs g, Kind kind, bool ta, bool tb, Plan plan, bool alone, hipStream_t st)
 {
-    // pairs of a row or column index that runs along memory need two of them, and a lane's offset is 32 bits
-    constexpr int kMost = 1 << 22;
-    const bool checked = (ta && g.M < 2) || (!tb && g.N < 2) || g.M > kMost || g.N > kMost || g.K > kMost;
+    // pairs of a row or column index that runs along memory need two of them
+    const bool checked = (ta && (g.M < 2 || g.M > kLongest16<T>)) || (!tb && (g.N < 2 || g.N > kLongest16<T>)) ||
+                         ((!ta || tb) && g.K > kLongest64<T>);
     const int steps = checked ? (g.K + 15) / 16 : g.K / 16;
     int per = (steps + plan.slices - 1) / plan.slices;
     int slices = per > 0 ? (steps + per - 1) / per : 1;
