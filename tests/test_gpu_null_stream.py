@@ -167,6 +167,77 @@ def test_results_written_by_the_last_launch(hip):
     assert done.returncode == 0 and done.stdout.strip().endswith("ok"), done.stdout[-2000:]
 
 
+GRADIENTS = r"""
+import ctypes as C
+import itertools
+import threading
+import numpy as np
+from vtl_amd import capi
+# Every set of gradients that can be asked for.  The last product tells the host that all of them are there (dX's, or dW's where there
+# is no dX), or a launch behind (dB alone, dX or dW too large to be written over the link), and what was not written over the
+# link comes down.  Memory of the caller's own: through staging memory, 1 MiB for the three together; of
+# vtl_hip_host_alloc: written in place beyond 4 KiB and up to 8 MiB.  Whole numbers: every sum is exact.
+SIZES = [(3, 5, 7), (64, 256, 784), (40, 700, 1001), (17, 1030, 2100), (600, 64, 2100), (2, 2049, 1024)]
+def memory(count, dt, pool, kept):
+    if not pool:
+        return np.empty(count, dt)
+    at = C.c_void_p()
+    capi.call("vtl_hip_host_alloc", C.byref(at), count * dt.itemsize)
+    kept.append(at)
+    return np.frombuffer((C.c_char * (count * dt.itemsize)).from_address(at.value), dt)
+def gradients(seed):
+    rng = np.random.default_rng(seed)
+    for (m, n, k), dt in itertools.product(SIZES, (np.dtype("f4"), np.dtype("f8"))):
+        for pools in ((0, 0, 0), (1, 1, 1), (1, 0, 0), (0, 1, 0)):
+            kept = []
+            for wanted in range(1, 8):
+                g, x, w = (rng.integers(-9, 10, s).astype(dt) for s in ((m, n), (m, k), (n, k)))
+                want = [g @ w, g.T @ x, g.sum(0)]
+                out = [memory(a.size, dt, p, kept) if wanted >> i & 1 else None for i, (a, p) in enumerate(zip(want, pools))]
+                for o in out:
+                    if o is not None:
+                        o[:] = -12345
+                capi.call("vtl_hip_linear_backward_host_" + ("f32" if dt.itemsize == 4 else "f64"), g.ctypes.data,
+                          x.ctypes.data if wanted & 2 else None, w.ctypes.data if wanted & 1 else None,
+                          *(None if o is None else o.ctypes.data for o in out), m, n, k)
+                for name, o, a in zip(("dx", "dw", "db"), out, want):
+                    assert o is None or np.array_equal(o, a.reshape(-1)), (m, n, k, dt, pools, wanted, name)
+            for at in kept:
+                capi.call("vtl_hip_host_free", at)
+capi.call("vtl_hip_set_device", 0)
+gradients(1)
+print("null stream", flush=True)
+bad = []
+def guarded(seed, stream=None):
+    try:
+        if stream:
+            capi.call("vtl_hip_set_stream", stream)
+        gradients(seed)
+    except BaseException as e:
+        bad.append((seed, repr(e)))
+def at_once(*calls):
+    threads = [threading.Thread(target=guarded, args=c) for c in calls]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad, bad
+at_once((2,), (3,))
+print("two threads", flush=True)
+hiprt = C.CDLL("libamdhip64.so")
+stream = C.c_void_p()
+assert hiprt.hipStreamCreateWithFlags(C.byref(stream), C.c_uint(1)) == 0
+at_once((4, stream))
+print("ok")
+"""
+
+
+def test_every_set_of_gradients(hip):
+    done = subprocess.run([sys.executable, "-c", GRADIENTS], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                          text=True, timeout=110)
+    assert done.returncode == 0 and done.stdout.rstrip().endswith("ok"), done.stdout[-3000:]
+
+
 def test_products_from_several_threads_on_the_null_stream(hip):
     done = subprocess.run([sys.executable, "-c", THREADS], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
                           text=True, timeout=100)
