@@ -148,6 +148,30 @@ def test_large_shapes_at_their_edges(hip, shape, mnk, knobs):
                     t.release()
 
 
+# What K has beyond steps of 16 is the first step, which loads elements of the second that it clears: around one step, as
+# many as are in flight (2 or 4) and one wave's or eight waves' share of them, with K in one piece and cut.  Whole values, exact
+# sums; a row of A meets an infinity in the elements that two steps load, which twice nothing must not turn into a NaN.
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("shape", ["1", "2", "3", "4", "5", "6"])
+def test_k_of_no_whole_steps(hip, shape, dt, knobs):
+    knobs.setenv("VTL_HIP_MATMUL_TILE", shape)
+    rng = np.random.default_rng(int(shape))
+    M, N = 35, 69
+    for K in (1, 15, 16, 17, 31, 32, 33, 47, 49, 63, 64, 65, 113, 127, 129, 143, 255, 257, 511, 513, 525):
+        for slices in ("0", "2") if K >= 64 else ("0",):
+            knobs.setenv("VTL_HIP_MATMUL_SPLITS", slices)
+            for ta, tb in [(False, False), (False, True), (True, False), (True, True)]:
+                A = rng.integers(-9, 10, (M, K)).astype(dt)
+                B = rng.integers(1, 10, (K, N)).astype(dt)
+                A[3, :] = 1
+                A[3, min(K - 1, K % 16 + 2)] = np.inf
+                A[4, 0] = np.inf
+                A[4, 1:] = 2
+                exact = A.astype(np.float64) @ B.astype(np.float64)
+                got = run_matmul(np.ascontiguousarray(A.T) if ta else A, np.ascontiguousarray(B.T) if tb else B, ta, tb)
+                assert np.array_equal(got, exact.astype(dt)), (K, slices, ta, tb)
+
+
 # Either side of where 32-bit offsets end: rows of C (64 to a wave), rows with K along them (64), rows with K across (16).  Many
 # rows, and K across many, end nowhere.  Whole values: sums are exact, and so is their rounding.
 @pytest.mark.parametrize("dt", [np.float32, np.float64])

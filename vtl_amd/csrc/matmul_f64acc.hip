@@ -27,7 +27,7 @@ struct MatmulArgs {
     const void *bias;   // N values added after rounding to the output type, or nullptr
     int M, N, K;
     int relu;
-    int k_per_split;    // k range of one grid.y slice (multiple of 16)
+    int slice_steps;    // steps of 16 of K in one grid.y slice
     double *partial;    // launches that slice K: [slices][M][N] unrounded sums, or [tail tile][slice][tile]; else nullptr
     int whole_tiles;    // with tail_slices > 1 the tiles from here on, the last round's, have K in that many slices
     int tail_slices;
@@ -59,9 +59,11 @@ struct alignas(16) Vec4 {
 // rows 2 * (l % 16) + {0, 1} of A and for TN / 2 such pairs of columns of B: 16-byte loads where K runs
 // along memory, pairs of 32 neighbouring columns where it does not.  MFMA j of a step takes the j-th of
 // each lane's four: which k they are is free as long as both operands agree.
-// Vector loads need no more than the elements' own alignment on gfx950, so ragged rows take them too;
-// what is left of K after whole steps is a step of its own with checked loads.  CHECKED: every
-// load is (a single row or column of a matrix that has to give pairs, rows too long for a lane's 32-bit offset).
+// Vector loads need no more than the elements' own alignment on gfx950, so ragged rows take them too.  What K has beyond whole
+// steps is the first one: loaded like any other, and what belongs to the second cleared.  (As a last step with checked
+// loads, waited for one after another, it was as long as several: f32 256 x 11008 x 300 44.3 -> 39.5 us, 101 x 720 x 394 8.0 -> 6.9; f64
+// 105 x 653 x 361 7.7 -> 6.8.)  CHECKED: every load is (a single row or column of a matrix that has to give pairs, rows
+// too long for a lane's 32-bit offset); so it is below K = 16.
 template <typename T>
 constexpr int kRun = 16 / (int)sizeof(T);   // elements of a 16-byte load; the lane's four are those of each run of 4 * kRun
 
@@ -156,6 +158,9 @@ struct DirectOperand {
     }
 };
 
+// Steps of 16 that K is.
+__host__ __device__ __forceinline__ int steps_of(int k) { return (k >> 4) + ((k & 15) != 0); }
+
 // The same with every load checked and no vector loads, at any size.
 template <typename T, bool KROWS>
 __device__ __forceinline__ void checked_fetch(T (&out)[2][4], const T *__restrict__ base, int mn_total, int k_total,
@@ -205,8 +210,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
 {
     constexpr int PA = TM / 2, PB = TN / 2;                // row and column pairs of a lane
     constexpr bool TAIL = TM == 4 && WK > 1;               // kSquare: choose_plan
-    // steps whose operands are in flight
-    constexpr int D = sizeof(T) == 4 ? (TM * TN <= 4 ? 4 : 2) : (TM * TN <= 8 ? 3 : 2);
+    // steps whose operands are in flight (f64 with three: no faster in large products, 11008 x 4096 x 256 349 and 345 us, and
+    // up to 15 % slower in short ones, which have the registers for fewer waves and load steps that they have not)
+    constexpr int D = sizeof(T) == 4 && TM * TN <= 4 ? 4 : 2;
     constexpr int V = 4 * TM * TN;                         // values of a lane
     __shared__ double red[WK > 1 ? WM * WN * WK : 1][WK > 1 ? V : 1][64];
     const T *__restrict__ A = static_cast<const T *>(g.A);
@@ -226,12 +232,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
     const int wk = wave % WK, tile = wave / WK;
     const int m0 = tm * BM + (tile / WN) * 16 * TM, n0 = tn * BN + (tile % WN) * 16 * TN;
     const int r16 = lane & 15, kq = lane >> 4;
-    // this workgroup's whole steps of K (all of them, or one of grid.y slices), this wave's among
-    // them, and whether this wave does the part of a step at the end of K
-    const int steps = CHECKED ? (g.K + 15) / 16 : g.K / 16, per = TAIL && g.tail_slices > 1 && of_tail < 0 ? steps : g.k_per_split / 16;
+    // this workgroup's steps of K (all of them, or one of grid.y slices) and this wave's among them
+    const int steps = steps_of(g.K), per = TAIL && g.tail_slices > 1 && of_tail < 0 ? steps : g.slice_steps;
     const int first = slice * per, last = min(first + per, steps) - 1;
     const int count = first + wk > last ? 0 : (last - first - wk) / WK + 1;
-    const bool rest = !CHECKED && steps * 16 < g.K && slice == slices - 1 && wk == WK - 1;
+    // where K is no whole steps the first one has what is left, and loads some of the next one's that it clears
+    const int beyond = CHECKED ? 0 : -g.K & 15;
 
     // Rows and columns past the edge repeat the last ones; what they give is not stored.  A pair that would
     // reach past the edge is moved back by one: its second is then the edge.
@@ -257,7 +263,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
     };
     const int row_first = min(m0, g.M - 1), col_first = min(n0, g.N - 1);
     auto fetch = [&](int d, int i) {   // the wave's i-th step; past its end the last one again
-        const int k0 = min(first + wk + i * WK, last) * 16;
+        const int k0 = max(min(first + wk + i * WK, last) * 16 - beyond, 0);
         if constexpr (CHECKED) {
             checked(d, k0);
         } else {
@@ -305,10 +311,49 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    if (count > 0) {
+    auto clear_beyond = [&] {   // the first step's, once it is loaded
+        if (CHECKED || beyond == 0 || first + wk != 0)
+            return;
+        constexpr int VK = kRun<T>;
+#pragma unroll
+        for (int q = 0; q < 4; q += VK)
+#pragma unroll
+            for (int j = 0; j < VK; ++j) {
+                const bool mine = 4 * q + VK * kq + j < 16 - beyond;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+#pragma unroll
+                    for (int p = 0; p < PA; ++p)
+                        fa[0][p][i][q + j] = mine ? fa[0][p][i][q + j] : T(0);
+#pragma unroll
+                    for (int p = 0; p < PB; ++p)
+                        fb[0][p][i][q + j] = mine ? fb[0][p][i][q + j] : T(0);
+                }
+            }
+    };
+    if (!CHECKED && g.K < 16) {
+        if (count > 0) {
+            checked(0, 0);
+            step(0, [] {});
+        }
+    } else if (TM * TN <= 8 && count < D) {
+        // Fewer steps than can be in flight: none is loaded twice (f32 89 x 123 x 64 4.5 -> 3.6 us, f64 81 x 829 x 70 4.5 -> 4.2).  (Conditions
+        // on the loads before the loop instead have it wait for all that are in flight: f64 256 x 11008 x 4096 368 -> 429.)
+#pragma unroll
+        for (int d = 0; d < D - 1; ++d)
+            if (d < count)
+                fetch(d, d);
+        if (count > 0)
+            clear_beyond();
+#pragma unroll
+        for (int d = 0; d < D - 1; ++d)
+            if (d < count)
+                step(d, [] {});
+    } else if (count > 0) {
 #pragma unroll
         for (int d = 0; d < D; ++d)
             fetch(d, d);
+        clear_beyond();
         int i = 0;
         for (; i + D <= count; i += D) {
 #pragma unroll
@@ -319,10 +364,6 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
         for (int d = 0; d < D - 1; ++d)
             if (i + d < count)
                 step(d, [] {});
-    }
-    if (rest) {
-        checked(0, steps * 16);
-        step(0, [] {});
     }
     if constexpr (!CHECKED) {
         // the edge of an odd matrix is the second of its pair
@@ -743,7 +784,7 @@ int launch_direct(MatmulArgs g, Kind kind, bool ta, bool tb, Plan plan, bool alo
     // pairs of a row or column index that runs along memory need two of them
     const bool checked = (ta && (g.M < 2 || g.M > kLongest16<T>)) || (!tb && (g.N < 2 || g.N > kLongest16<T>)) ||
                          ((!ta || tb) && g.K > kLongest64<T>);
-    const int steps = checked ? (g.K + 15) / 16 : g.K / 16;
+    const int steps = steps_of(g.K);
     int per = (steps + plan.slices - 1) / plan.slices;
     int slices = per > 0 ? (steps + per - 1) / per : 1;
     Partial partial;
@@ -768,7 +809,7 @@ int launch_direct(MatmulArgs g, Kind kind, bool ta, bool tb, Plan plan, bool alo
             per = tail_per;
         }
     }
-    g.k_per_split = 16 * per;
+    g.slice_steps = per;
     int rc = VTL_HIP_ERR_UNSUPPORTED;
     if (checked)
         rc = launch_direct_shape<T, 1, 1, 8, 2, 2, true>(g, ta, tb, slices, st);
