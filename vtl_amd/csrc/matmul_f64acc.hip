@@ -336,19 +336,28 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
             checked(0, 0);
             step(0, [] {});
         }
-    } else if (TM * TN <= 8 && count < D) {
-        // Fewer steps than can be in flight: none is loaded twice (f32 89 x 123 x 64 4.5 -> 3.6 us, f64 81 x 829 x 70 4.5 -> 4.2).  (Conditions
-        // on the loads before the loop instead have it wait for all that are in flight: f64 256 x 11008 x 4096 368 -> 429.)
+    } else if (TM * TN <= 8 && count <= D) {
+        // No more steps than can be in flight: none is loaded twice, and each number of them has code of its own (60 x 500 in tiles
+        // of 32 x 32, K over four waves, loaded twice and now: f32 K = 64 4.5 -> 3.6 us, 128 5.0 -> 4.2, 192 5.4 -> 4.7; f64 64 4.1 -> 4.0, 128 5.3 -> 4.8).
+        // (Conditions on single loads have the compiler move them behind the products before, and wait in the loop for
+        // all that are in flight: f64 256 x 11008 x 4096 368 -> 429.)
+        auto all = [&](auto n) {
 #pragma unroll
-        for (int d = 0; d < D - 1; ++d)
-            if (d < count)
+            for (int d = 0; d < n; ++d)
                 fetch(d, d);
-        if (count > 0)
             clear_beyond();
 #pragma unroll
-        for (int d = 0; d < D - 1; ++d)
-            if (d < count)
+            for (int d = 0; d < n; ++d)
                 step(d, [] {});
+        };
+        if (count == 1)
+            all(std::integral_constant<int, 1>());
+        else if (count == 2)
+            all(std::integral_constant<int, 2>());
+        else if (D > 2 && count == 3)
+            all(std::integral_constant<int, D < 3 ? D : 3>());
+        else if (D > 3 && count == 4)
+            all(std::integral_constant<int, D < 4 ? D : 4>());
     } else if (count > 0) {
 #pragma unroll
         for (int d = 0; d < D; ++d)
