@@ -331,12 +331,14 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
                 }
             }
     };
-    if (!CHECKED && g.K < 16) {
+    // (What is expected here is where the compiler lays the loop: behind the other paths, tiles of one wave each, all of a chip's
+    // workgroups reading the same code, took 4 to 12 % longer, f32 dW 4411 x 1344 x 192 42 -> 51 us, f64 4096 x 2496 x 128 46 -> 49.)
+    if (!CHECKED && __builtin_expect(g.K < 16, 0)) {
         if (count > 0) {
             checked(0, 0);
             step(0, [] {});
         }
-    } else if (TM * TN <= 8 && count <= D) {
+    } else if (TM * TN <= 8 && (WK > 1 ? count <= D : __builtin_expect(count <= D, 0))) {
         // No more steps than can be in flight: none is loaded twice, and each number of them has code of its own (60 x 500 in tiles
         // of 32 x 32, K over four waves, loaded twice and now: f32 K = 64 4.5 -> 3.6 us, 128 5.0 -> 4.2, 192 5.4 -> 4.7; f64 64 4.1 -> 4.0, 128 5.3 -> 4.8).
         // (Conditions on single loads have the compiler move them behind the products before, and wait in the loop for
@@ -366,8 +368,17 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
         int i = 0;
         for (; i + D <= count; i += D) {
 #pragma unroll
-            for (int d = 0; d < D; ++d)
+            for (int d = 0; d < D; ++d) {
+                // All of a step's f32 operands are waited for before the first is converted: conversions that wait one by one lie
+                // between the MFMAs of the workgroup beside this one, and the two end at once instead of one after the other
+                // (f32 229 x 5211 x 1251 in 2.5 rounds 62 us, waiting for each 80; 256 x 11008 x 4096 level).
+                if constexpr (!CHECKED && sizeof(T) == 4 && TM * TN == 8 && WK > 1) {
+                    constexpr int later = ((TA ? 4 : 2) * PA + (TB ? 2 : 4) * PB) * (D - 1);   // loads of the steps behind it
+                    __builtin_amdgcn_s_waitcnt(0x0f70 | (later & 15) | (later >> 4) << 14);    // vmcnt
+                    __builtin_amdgcn_sched_barrier(0);
+                }
                 step(d, [&] { fetch(d, i + d + D); });
+            }
         }
 #pragma unroll
         for (int d = 0; d < D - 1; ++d)
