@@ -35,7 +35,9 @@
  *     vtl_hip_linear_f32_dynquant with workspace == NULL, int8 operands that
  *     need repacking).  There is one such buffer per purpose and device,
  *     shared by every stream: calls that use it must not overlap on a device,
- *     i.e. issue them on one stream (or order the streams yourself).  The
+ *     i.e. issue them on one stream (or order the streams yourself).  Calls
+ *     on whole host tensors have blocks of their own instead while no stream
+ *     has been named, and may run in several threads at once.  The
  *     buffers grow on demand, which waits for the whole device; while the
  *     current stream is being captured into a graph a call that would have to
  *     grow one returns VTL_HIP_ERR_UNSUPPORTED instead (pass a workspace of

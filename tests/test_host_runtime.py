@@ -253,6 +253,29 @@ print("done")
 """)
 
 
+def test_whole_host_calls_share_no_scratch_between_threads(fake_runtime):
+    """Whole host calls run in several threads at once: what two of their launches meet in is memory of the call's own, not
+    the library's one buffer per purpose (32 MiB at least, where these calls take a few)."""
+    _run(fake_runtime, r"""
+runtime()
+p = malloc_on(0, 1 << 20)
+host = (C.c_float * (1 << 20))()
+def shared(name, *args):
+    events()
+    capi.status(name, *args)                                                  # no kernel runs here
+    log = events()
+    assert count("launch", log) > 1, (name, args, log)
+    return [e for e in log if e[0] == "malloc" and e[3] >= 32 << 20]
+for per_channel in (0, 1):
+    for rows, n, k, row in ((256, 1000, 72, 80), (256, 1000, 72, 0), (64, 1000, 1001, 1008), (64, 1024, 4096, 0)):
+        layer = capi.Layer(0, per_channel, n, k, p, p, None, row)             # a linear
+        assert not shared("vtl_hip_forward_i8_host", host, rows, k, C.byref(layer), 1, host), (per_channel, rows, n, k)
+for name in ("f32", "f64"):                                                   # column sums in splits
+    assert not shared("vtl_hip_linear_backward_host_" + name, host, host, host, host, host, host, 256, 64, 16), name
+print("done")
+""")
+
+
 def test_a_transfer_that_waits_for_the_device_costs_no_host_time(fake_runtime):
     """A large upload whose staging memory is not free yet: neither the caller nor the threads that help
     with the copying spin until it is."""

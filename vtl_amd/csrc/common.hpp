@@ -215,6 +215,24 @@ struct ScratchArena {
     ScratchArena &operator=(const ScratchArena &) = delete;
 };
 
+// While one is alive, library_workspace() hands this thread blocks of its own instead of the library's: whole host calls run in
+// several threads at once, and between two launches of one that meet in a slot another's may write it.  A released block's next owner
+// comes behind these launches on the null stream; once the process has named a stream a release would wait for the
+// device, and the library's buffers are what there is.
+class CallScratch {
+public:
+    CallScratch();
+    ~CallScratch();
+    CallScratch(const CallScratch &) = delete;
+    CallScratch &operator=(const CallScratch &) = delete;
+    // nullptr: no memory
+    void *take(size_t bytes, int slot);
+
+private:
+    void *own_[3] = {};
+    size_t bytes_[3] = {};
+};
+
 // Whether this thread's scratch is the static one just now.
 bool scratch_is_static();
 

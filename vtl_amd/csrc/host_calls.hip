@@ -85,6 +85,7 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
     const size_t most = out_cols % 32 == 0 ? (size_t)4 << 20 : (size_t)5 << 19;
     float *const y = ends_linear ? static_cast<float *>(result.begin(y_host, out_bytes, most)) : nullptr;
     HostInput input;
+    vtlhip::CallScratch own;
     // (32 KiB is what the kernels that quantize in every workgroup take at most; near it the eight XCDs' transfers
     // cost what an upload does)
     const bool upload_first = rows <= 8 && in_bytes > ((size_t)20 << 10) && in_bytes <= ((size_t)32 << 10);
@@ -220,6 +221,7 @@ int matmul_host(const T *a, const T *b, T *c, int m, int n, int k)
     VTL_STEP(upload_both(da, a, (size_t)m * (size_t)k, db, b, (size_t)k * (size_t)n));
     const size_t bytes = (size_t)m * (size_t)n * sizeof(T);
     HostResult result;
+    vtlhip::CallScratch own;
     if (T *out = static_cast<T *>(result.begin(c, bytes, direct_most<T>(m, n)))) {
         VTL_STEP(matmul_to(&result, da.as<T>(), db.as<T>(), out, m, n, k, 0));
         return result.finish();
@@ -261,6 +263,7 @@ int linear_backward_host(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
         }
     };
     HostResult result;
+    vtlhip::CallScratch own;
     const size_t dw_bytes = nk * sizeof(T), db_bytes = (size_t)n * sizeof(T);
     Gradient gw = {dw, dw_bytes, dev_dw, dx && overlap(dw, dw_bytes, w, dw_bytes)}, gx = {dx, mk * sizeof(T), dev_dx, false},
              gb = {db, db_bytes, dev_db, dx && overlap(db, db_bytes, w, dw_bytes)};

@@ -235,6 +235,39 @@ ScratchArena::ScratchArena(void *base_, size_t capacity_) : base(static_cast<cha
 
 ScratchArena::~ScratchArena() { g_arena = nullptr; }
 
+static thread_local CallScratch *g_call_scratch = nullptr;
+
+CallScratch::CallScratch()
+{
+    if (!g_call_scratch && single_stream())
+        g_call_scratch = this;
+}
+
+CallScratch::~CallScratch()
+{
+    if (g_call_scratch == this)
+        g_call_scratch = nullptr;
+    for (void *own : own_)
+        if (own)
+            (void)vtl_hip_free(own);
+}
+
+void *CallScratch::take(size_t bytes, int slot)
+{
+    if (bytes > bytes_[slot] || !own_[slot]) {
+        if (own_[slot])
+            (void)vtl_hip_free(own_[slot]);
+        own_[slot] = nullptr;
+        bytes_[slot] = 0;
+        if (vtl_hip_malloc(&own_[slot], bytes ? bytes : 1) != VTL_HIP_OK) {
+            own_[slot] = nullptr;
+            return nullptr;
+        }
+        bytes_[slot] = bytes;
+    }
+    return own_[slot];
+}
+
 bool scratch_is_static() { return g_arena != nullptr; }
 
 int workspace_status() { return g_workspace_status; }
@@ -261,6 +294,12 @@ void *library_workspace(size_t bytes, int slot)
         void *p = g_arena->base + g_arena->used;
         g_arena->used += take;
         return p;
+    }
+    if (g_call_scratch) {
+        void *own = g_call_scratch->take(bytes, slot);
+        if (!own)
+            g_workspace_status = VTL_HIP_ERR_OUT_OF_MEMORY;
+        return own;
     }
     void **buf = bufs[slot];
     size_t *cap = caps[slot];
