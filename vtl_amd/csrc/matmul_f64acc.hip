@@ -210,9 +210,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
 {
     constexpr int PA = TM / 2, PB = TN / 2;                // row and column pairs of a lane
     constexpr bool TAIL = TM == 4 && WK > 1;               // kSquare: choose_plan
-    // steps whose operands are in flight (f64 with three: no faster in large products, 11008 x 4096 x 256 349 and 345 us, and
-    // up to 15 % slower in short ones, which have the registers for fewer waves and load steps that they have not)
-    constexpr int D = sizeof(T) == 4 && TM * TN <= 4 ? 4 : 2;
+    // Steps whose operands are in flight.  f64 with three: no faster in large products (11008 x 4096 x 256 349 and 345 us), and
+    // up to 15 % slower in short ones, which have the registers for fewer waves and load steps that they have not; but where K runs
+    // across the rows of B, in tiles of 32 x 32 with K over four waves, a last round that is not full is a round longer
+    // with two (dW 408 x 3057 x 2373 95 -> 111 us, 396 x 2741 x 2398 94 -> 109, dX 1803 x 1248 x 3212 231 -> 250; K < 400 2 % ahead).
+    constexpr int D = sizeof(T) == 4 ? (TM * TN <= 4 ? 4 : 2) : (TM * TN == 4 && WK == 4 && !TB ? 3 : 2);
     constexpr int V = 4 * TM * TN;                         // values of a lane
     __shared__ double red[WK > 1 ? WM * WN * WK : 1][WK > 1 ? V : 1][64];
     const T *__restrict__ A = static_cast<const T *>(g.A);
@@ -261,6 +263,15 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
         for (int p = 0; p < PB; ++p)
             checked_fetch<T, TB>(fb[d][p], B, g.N, g.K, col[p], k0, kq);
     };
+    // Two workgroups that share a compute unit should end one after the other: where they end at once, a last round that is not
+    // full may find both places of one unit and none of the next.  f32 tiles of 32 x 64, K along the rows of B: the wait in the loop; K
+    // across them, where that wait does not do it: every other 256 workgroups, one per compute unit, go first (dX 144 x 8720 x
+    // 1072, 2.7 rounds, 68 to 75 us -> 61 to 62; dX and dW of 280 to 1800 tiles on average level).
+    constexpr bool in_turn = !CHECKED && sizeof(T) == 4 && TM * TN == 8 && WK > 1;
+    if constexpr (in_turn && !TB) {
+        if (((blockIdx.x + gridDim.x * blockIdx.y) >> 8 & 1) == 0)
+            __builtin_amdgcn_s_setprio(1);
+    }
     const int row_first = min(m0, g.M - 1), col_first = min(n0, g.N - 1);
     auto fetch = [&](int d, int i) {   // the wave's i-th step; past its end the last one again
         const int k0 = max(min(first + wk + i * WK, last) * 16 - beyond, 0);
@@ -372,9 +383,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
                 // All of a step's f32 operands are waited for before the first is converted: conversions that wait one by one lie
                 // between the MFMAs of the workgroup beside this one, and the two end at once instead of one after the other
                 // (f32 229 x 5211 x 1251 in 2.5 rounds 62 us, waiting for each 80; 256 x 11008 x 4096 level).
-                if constexpr (!CHECKED && sizeof(T) == 4 && TM * TN == 8 && WK > 1) {
-                    constexpr int later = ((TA ? 4 : 2) * PA + (TB ? 2 : 4) * PB) * (D - 1);   // loads of the steps behind it
-                    __builtin_amdgcn_s_waitcnt(0x0f70 | (later & 15) | (later >> 4) << 14);    // vmcnt
+                if constexpr (in_turn && TB) {
+                    constexpr int later = ((TA ? 4 : 2) * PA + 2 * PB) * (D - 1);             // loads of the steps behind it
+                    __builtin_amdgcn_s_waitcnt(0x0f70 | (later & 15) | (later >> 4) << 14);   // vmcnt
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 step(d, [&] { fetch(d, i + d + D); });
