@@ -670,18 +670,20 @@ constexpr int kPerUnit[kKinds][kShapes] = {{1, 1, 1, 4, 0, 0}, {1, 1, 1, 1, 0, 0
 
 // Estimated microseconds: start + rounds * (per_tile + work / rate), where `rounds` is how many times the busiest
 // compute unit is filled and `work` the time its matrix cores need for that at
-// 2.3 GHz; slicing K adds a launch and its partial sums (per MB).  Fitted to 1200 products drawn over
-// m, n up to 11008 and k up to 4096, whole and ragged, the layouts of forward and backward, every shape timed alternately:
-// the choice is on average 2 % (kF64Rows 2.7 %) behind the fastest of them, and on 898 others 2.2, 1.8 and 3.7 % (kF32, kF64,
-// kF64Rows), at most 43, 27 and 37 % where K is below 300.
+// 2.3 GHz; slicing K adds a launch and its partial sums (per MB).  Fitted to products drawn over m, n up to 11008 and k up to
+// 4096, half of them with k below 300, whole and ragged, the layouts of forward and backward, every shape timed alternately: kF32 and kF64
+// to 1200 of the forms before this one's for a short K, kF64Rows to 470 of these.  On 700 each the choice is on average 3.6, 2.8 and
+// 1.3 % (kF32, kF64, kF64Rows) behind the fastest, at most 65, 29 and 26 %, the worst with k below 300.  (kF32 and kF64 refitted the same
+// way come to 0.9 % there, but over 160 products with K from 200 to 4000 and rounds that are not full to 0 to 1 % more time than now and up to 15 %
+// in single ones: kept as they were.)
 struct Cost {
     double start, per_tile, inverse_rate, slice_start, slice_mb;
 };
 constexpr Cost kCost[kKinds][kShapes] = {
     {{1.59, 2.57, 1.18, 4.24, 0.42}, {3.22, 0.88, 1.13, 4.10, 0.43}, {2.89, 1.65, 1.05, 4.71, 0.45}, {2.52, 2.71, 1.08, 4.06, 0.53}, {}, {}},
     {{1.64, 2.07, 1.22, 4.27, 0.49}, {2.87, 0.83, 1.14, 4.01, 0.55}, {2.81, 1.65, 1.06, 4.57, 0.53}, {2.41, 3.48, 0.97, 5.23, 0.30}, {}, {}},
-    {{1.65, 2.10, 1.89, 4.47, 0.62}, {2.69, 1.09, 1.76, 3.91, 0.75}, {2.57, 2.21, 1.37, 4.47, 0.52}, {}, {1.40, 5.53, 1.04, 4.55, 0.55},
-     {0.0, 8.0, 0.97, 3.93, 0.41}},
+    {{1.51, 2.26, 2.08, 3.78, 0.67}, {1.59, 0.45, 1.97, 2.65, 0.74}, {2.10, 1.82, 1.42, 3.92, 0.52}, {}, {1.44, 6.76, 0.96, 4.19, 0.42},
+     {0.02, 7.80, 1.07, 3.19, 0.42}},
 };
 
 // What a second launch has to be worth beyond its time on the device: it takes the host 3.4 us, which a chain of small products
