@@ -412,3 +412,26 @@ def test_roundtrip_config_full_size(hip):
     assert np.array_equal(qt.cpu()[sample], oracle.quantize_with_scale(x[sample], st.cpu(), False))
     for h in (t, q, s, d, q2, qt, st):
         h.release()
+
+
+# Four codes are made at once unless one of them has to be looked at alone: what calls for that (no number, a tie, either side of one by some
+# steps, in and out of the band in which the quotient is divided) at each of the four places, the largest value of the row among them
+@pytest.mark.parametrize("axis", [0, -1])
+@pytest.mark.parametrize("cols", [256, 1000, 4096, 20000])
+def test_one_of_four_values_that_is_looked_at_alone(hip, cols, axis):
+    rng = np.random.Generator(np.random.Philox(cols))
+    x = rng.uniform(-1, 1, (24, cols)).astype(np.float32)
+    for r in range(x.shape[0]):
+        most = np.float32([1.0, 3.7, 127.0, 1e-30, 2e30, 5e-39][r % 6]) if axis == 0 else np.float32(127 * 0.37)
+        x[r] *= most * np.float32(0.99)
+        scale = most / np.float32(127)
+        for i in range(r // 6, cols, 4 + r % 5):
+            half = (np.float32(rng.integers(-126, 126)) + np.float32(0.5)) * scale
+            x[r, i] = [np.nan, half, half * np.float32(1 + 2e-7 * rng.integers(-9, 10)), half + scale * np.float32(2.0 ** -14), most, -most][i % 6]
+        x[r, cols // 2] = most
+    t = dev(x)
+    q, s = t.quantize_i8(axis)
+    qr, sr = oracle.quantize(x, axis == 0)
+    assert np.array_equal(s.cpu(), sr) and np.array_equal(q.cpu(), qr)
+    for h in (t, q, s):
+        h.release()

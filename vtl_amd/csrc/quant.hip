@@ -517,7 +517,7 @@ __global__ __launch_bounds__(T) void quantize_scaled_kernel(const float *__restr
         for (int i = 0; i < NV; i++) {
             const int64_t idx = base + i * T + threadIdx.x;
             if (idx < nv)
-                __builtin_nontemporal_store(quant4(v[i], p), qv + idx);
+                __builtin_nontemporal_store(quant4<!FROM_ABSMAX>(v[i], p), qv + idx);
         }
         // ragged tail of a flat tensor (cols % 4 elements)
         if (chunk == 0 && threadIdx.x < (cols & 3)) {
@@ -595,7 +595,7 @@ __global__ __launch_bounds__(T) void quantize_scaled_flat_rows_kernel(const floa
             const QuantScale p = make_quant_scale(scale[row]);
             unsigned packed;
             if (col + 4 <= cols) {
-                packed = quant4(v[i], p);
+                packed = quant4<true>(v[i], p);
             } else {  // the vector runs into the next row
                 const QuantScale p1 = make_quant_scale(scale[row + 1]);
                 const unsigned in0 = cols - col;  // 1..3 elements still in `row`

@@ -132,8 +132,32 @@ __device__ __forceinline__ unsigned pack4(int a, int b, int c, int d)
            ((unsigned)d << 24);
 }
 
+// Four codes at once: a quotient's rounding is what is left of it beside a number whose last place is one, the code its low
+// byte, and one test sees whether any of the four is too close to a tie, or no number (v_maximum3 keeps a NaN): then the
+// codes are made one by one.  6 vector instructions an element instead of 14, which the kernels that quantize a row in every workgroup, or hold
+// a tensor in registers until its scale is known, have nothing to hide behind (us: linear on f32 rows 1 x 4096 x 11008 10.97 -> 10.41,
+// 2 x 14336 x 4096 12.15 -> 11.10, 8 x 13.7 -> 13.35, 128 x 17.1 -> 16.6; 3001 x 4099 quantized with one scale and back 27.4 -> 26.4).
+// GIVEN: the scale is not that of the values' own maximum, so quotients may be out of range.
+template <bool GIVEN = false>
 __device__ __forceinline__ unsigned quant4(float4_t v, const QuantScale &p)
 {
+    constexpr float kOnes = 0x1.8p23f;
+    float n[4], off[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const float t = v[i] * p.rinv;
+        n[i] = t + kOnes;
+        const float r = n[i] - kOnes;
+        off[i] = fabsf(t - r);
+        if (GIVEN)
+            n[i] = __builtin_amdgcn_fmed3f(r, -127.0f, 127.0f) + kOnes;
+    }
+    const float most = __builtin_elementwise_maximum(__builtin_elementwise_maximum(off[0], off[1]), __builtin_elementwise_maximum(off[2], off[3]));
+    if (__builtin_expect(p.fast && most < 0.5f - kTieBand, 1)) {
+        const unsigned lo = __builtin_amdgcn_perm(__float_as_uint(n[1]), __float_as_uint(n[0]), 0x0c0c0400);
+        const unsigned hi = __builtin_amdgcn_perm(__float_as_uint(n[3]), __float_as_uint(n[2]), 0x04000c0c);
+        return lo | hi;
+    }
     return pack4(quant_code(v.x, p), quant_code(v.y, p), quant_code(v.z, p), quant_code(v.w, p));
 }
 
