@@ -414,6 +414,22 @@ def test_linear_backward_against_oracle(hip, dt):
             t.release()
 
 
+@pytest.mark.parametrize("m,n,k", [(16, 2625, 3136), (64, 1024, 2688), (128, 1984, 1615), (128, 1646, 3609)])
+def test_f64_weight_gradient_of_large_tiles(hip, m, n, k):
+    # tiles of 64 x 128 that store pairs of doubles one behind the other: every bit of both has to arrive, each time
+    rng = np.random.default_rng(m + n)
+    g, x = rng.standard_normal((m, n)), rng.standard_normal((m, k))
+    want, bound = g.T @ x, (m + 2) * 2.0 ** -53 * (np.abs(g).T @ np.abs(x))
+    gd, xd, wd = dev(g), dev(x), dev(np.zeros((n, k)))
+    print("weight gradient", m, n, k, flush=True)
+    for _ in range(10):
+        dw = linear_backward_hip(gd, xd, wd, need_dx=False, need_db=False)[1]
+        assert np.all(np.abs(dw.cpu() - want) <= 2 * bound)
+        dw.release()
+    for t in (gd, xd, wd):
+        t.release()
+
+
 def test_linear_backward_host_entry(hip, monkeypatch):
     # operands of autograd_cuda/device_session_test.v:52-60; gradients worked by hand
     g = np.array([[1.0, 0.5]], np.float32)

@@ -105,6 +105,12 @@ __device__ __forceinline__ void store_run(__amdgpu_buffer_rsrc_t base, unsigned 
     const unsigned long long ua = (unsigned long long)__double_as_longlong(a), ub = (unsigned long long)__double_as_longlong(b);
     __builtin_amdgcn_raw_buffer_store_b128(Four{(unsigned)ua, (unsigned)(ua >> 32), (unsigned)ub, (unsigned)(ub >> 32)}, base, off,
                                            along, THROUGH ? vtlhip::kThrough : 0);
+    // A store of more than 8 bytes reads its registers for two more instructions.  The compiler keeps instructions that write them
+    // away only where the offset is no scalar register; left to it, the next pair's first word was moved in behind the store, and
+    // now and then went out with this one (dW 2625 x 3136 x 16: elements in even columns off by 1e-7 of themselves).
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 1");
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 // One pair of rows or columns of an operand for the lanes of a wave.
