@@ -430,6 +430,51 @@ def test_f64_weight_gradient_of_large_tiles(hip, m, n, k):
         t.release()
 
 
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("m,n,k", [(1, 2, 2), (1, 3, 17), (15, 33, 31), (16, 64, 32), (17, 65, 97), (33, 63, 130), (64, 4, 1030),
+                                   (128, 1000, 70), (40, 2500, 65), (512, 66, 34), (513, 66, 34), (129, 1100, 1450)])
+def test_gradients_in_one_launch(hip, knobs, dt, m, n, k):
+    """Edges of the tiles, of the column sums' groups of four and 64, of a step of K, and of the rows that one launch
+    sums; dX's K in one piece and in slices: as launch by launch, within the order of the sums."""
+    rng = np.random.default_rng(m * n + k)
+    g, x, w = (rng.standard_normal(s).astype(dt) for s in ((m, n), (m, k), (n, k)))
+    gd, xd, wd = dev(g), dev(x), dev(w)
+    bounds = (n * (np.abs(g).astype(np.float64) @ np.abs(w)), m * (np.abs(g).T.astype(np.float64) @ np.abs(x)),
+              m * np.abs(g).astype(np.float64).sum(axis=0)[None])
+    want = [g.astype(np.float64) @ w.astype(np.float64), g.T.astype(np.float64) @ x.astype(np.float64),
+            g.astype(np.float64).sum(axis=0)[None]]
+    for mode in ("0", "1"):
+        knobs.setenv("VTL_HIP_BACKWARD_GROUP", mode)
+        for need in ((True, True, True), (True, True, False), (False, True, True), (True, False, True)):
+            print("gradients", dt.__name__, m, n, k, mode, need, flush=True)
+            outs = linear_backward_hip(gd, xd, wd, *need)
+            for o, exact, b in zip(outs, want, bounds):
+                if o is not None:
+                    # sums of m or n products in f64, numpy's too, and one rounding to the tensor's type
+                    got = o.cpu().astype(np.float64)
+                    assert np.all(np.abs(got - exact) <= 2.0 ** -52 * b + (np.abs(exact) * 2.0 ** -24 if dt == np.float32 else 0))
+                    o.release()
+    for t in (gd, xd, wd):
+        t.release()
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_weight_gradient_over_the_weights(hip, knobs, dt):
+    """dX is complete before dW is written: dW may take the place of W."""
+    m, n, k = 64, 192, 160
+    rng = np.random.default_rng(7)
+    g, x, w = (rng.integers(-8, 9, s).astype(dt) for s in ((m, n), (m, k), (n, k)))   # (whole numbers: every sum exact)
+    for mode in ("0", "1"):
+        knobs.setenv("VTL_HIP_BACKWARD_GROUP", mode)
+        gd, xd, wd, dx, db = dev(g), dev(x), dev(w), dev(np.zeros_like(x)), dev(np.zeros((1, n), dt))
+        capi.call("vtl_hip_linear_backward_f32" if dt == np.float32 else "vtl_hip_linear_backward_f64", gd.ptr, xd.ptr, wd.ptr,
+                  dx.ptr, wd.ptr, db.ptr, m, n, k)
+        assert np.array_equal(dx.cpu(), g @ w) and np.array_equal(wd.cpu(), g.T @ x)
+        assert np.array_equal(db.cpu().reshape(-1), g.sum(axis=0))
+        for t in (gd, xd, wd, dx, db):
+            t.release()
+
+
 def test_linear_backward_host_entry(hip, monkeypatch):
     # operands of autograd_cuda/device_session_test.v:52-60; gradients worked by hand
     g = np.array([[1.0, 0.5]], np.float32)

@@ -243,6 +243,9 @@ bool launch_quantize_rows_padded(const float *x, int64_t rows, int cols, int8_t 
 // vtl_hip_matmul_* without a transposed b.  `result`: c is its memory, and this is the call's last launch.
 int matmul_to(HostResult *result, const float *a, const float *b, float *c, int m, int n, int k, int trans_a);
 int matmul_to(HostResult *result, const double *a, const double *b, double *c, int m, int n, int k, int trans_a);
+// dW = grad^T . x and, unless it is null, db = the column sums of grad.
+int weight_gradients_to(HostResult *result, const float *grad, const float *x, float *dw, float *db, int m, int n, int k);
+int weight_gradients_to(HostResult *result, const double *grad, const double *x, double *dw, double *db, int m, int n, int k);
 
 // vtl_hip_linear_i8_f32 and vtl_hip_linear_i8_requant with the parameters of a layer, whose weights may have padded rows.
 // `result`: Y is its memory.
@@ -274,6 +277,7 @@ struct Tuning {
     int skinny_tiled = -1;          // VTL_HIP_SKINNY_TILED: 1 / 0 force the 32x32-block weight-streaming kernel for M > 32
     int skinny_waves = 4;           // VTL_HIP_SKINNY_WAVES: 2, 4 or 8 waves (K ranges) per workgroup there
     int matmul_tile = 0;            // VTL_HIP_MATMUL_TILE: which kernel and tile the f64-accumulating matmul takes (matmul_f64acc.hip)
+    int backward_group = -1;        // VTL_HIP_BACKWARD_GROUP: 1 / 0 force a backward's gradients in one launch on (where it can be) / off
     int matmul_splits = -1;         // VTL_HIP_MATMUL_SPLITS: K ranges of the f64-accumulating matmul
 };
 const Tuning &tuning();

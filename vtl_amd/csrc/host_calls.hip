@@ -274,14 +274,11 @@ int linear_backward_host(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
         VTL_STEP(upload_both(dev_grad, grad, mn, dev_x, x, mk));
     else
         VTL_STEP(upload(dev_grad, grad, mn));
-    if (gb.out && !gx.out)
+    if (gw.out)     // [N,K] = grad^T[N,M] . x[M,K], and the column sums
+        VTL_STEP(weight_gradients_to(gw.direct && !gx.out ? &result : nullptr, dev_grad.as<T>(), dev_x.as<T>(), gw.out, gb.out, m, n, k));
+    else if (gb.out)
         VTL_STEP(colsum(dev_grad.as<T>(), m, n, gb.out));
-    if (gw.out) {   // [N,K] = grad^T[N,M] . x[M,K]
-        VTL_STEP(matmul_to(gw.direct && !gx.out ? &result : nullptr, dev_grad.as<T>(), dev_x.as<T>(), gw.out, n, k, m, 1));
-    }
     if (gx.out) {   // [M,K] = grad[M,N] . W[N,K]
-        if (gb.out)
-            VTL_STEP(colsum(dev_grad.as<T>(), m, n, gb.out));
         VTL_STEP(upload(dev_w, w, nk));
         VTL_STEP(matmul_to(gx.direct ? &result : nullptr, dev_grad.as<T>(), dev_w.as<T>(), gx.out, m, k, n, 0));
     }

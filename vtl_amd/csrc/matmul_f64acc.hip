@@ -208,11 +208,19 @@ __device__ __forceinline__ void tile_of_block(int block, int tiles_m, int tiles_
     tn = (pid % group) / gm;
 }
 
+// The partial tiles of a workgroup whose waves cut K.
+template <int WM, int WN, int WK, int TM, int TN>
+struct PartialTiles {
+    double at[WK > 1 ? WM * WN * WK : 1][WK > 1 ? 4 * TM * TN : 1][64];
+};
+
+// One workgroup's part of a product: tile `block` and slice `slice` of `slices` of K.  `turn`: this workgroup's number in the launch.
 // The tiles of a workgroup are WM x WN wave tiles, K is cut over WK waves each.
 // Blocks are renumbered so that each of the 8 XCDs (own L2) works on a compact patch of tiles, eight
 // tile rows deep: with the plain order the rows that share a column panel of B run on different XCDs.
 template <typename T, int WM, int WN, int WK, int TM, int TN, bool TA, bool TB, bool CHECKED>
-__global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel(const MatmulArgs g)
+__device__ __forceinline__ void direct_tile(const MatmulArgs &g, int block, int slice, int slices, unsigned turn,
+                                            PartialTiles<WM, WN, WK, TM, TN> &red)
 {
     constexpr int PA = TM / 2, PB = TN / 2;                // row and column pairs of a lane
     constexpr bool TAIL = TM == 4 && WK > 1;               // kSquare: choose_plan
@@ -222,12 +230,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
     // with two (dW 408 x 3057 x 2373 95 -> 111 us, 396 x 2741 x 2398 94 -> 109, dX 1803 x 1248 x 3212 231 -> 250; K < 400 2 % ahead).
     constexpr int D = sizeof(T) == 4 ? (TM * TN <= 4 ? 4 : 2) : (TM * TN == 4 && WK == 4 && !TB ? 3 : 2);
     constexpr int V = 4 * TM * TN;                         // values of a lane
-    __shared__ double red[WK > 1 ? WM * WN * WK : 1][WK > 1 ? V : 1][64];
     const T *__restrict__ A = static_cast<const T *>(g.A);
     const T *__restrict__ B = static_cast<const T *>(g.B);
     constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
     const int tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
-    int block = (int)blockIdx.x, slice = (int)blockIdx.y, slices = (int)gridDim.y, of_tail = -1;
+    int of_tail = -1;
     if (TAIL && g.tail_slices > 1 && block >= g.whole_tiles) {
         of_tail = block - g.whole_tiles;
         slices = g.tail_slices;
@@ -275,7 +282,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
     // 1072, 2.7 rounds, 68 to 75 us -> 61 to 62; dX and dW of 280 to 1800 tiles on average level).
     constexpr bool in_turn = !CHECKED && sizeof(T) == 4 && TM * TN == 8 && WK > 1;
     if constexpr (in_turn && !TB) {
-        if (((blockIdx.x + gridDim.x * blockIdx.y) >> 8 & 1) == 0)
+        if ((turn >> 8 & 1) == 0)
             __builtin_amdgcn_s_setprio(1);
     }
     const int row_first = min(m0, g.M - 1), col_first = min(n0, g.N - 1);
@@ -504,21 +511,131 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel
         // partial tiles, in the order of the registers
 #pragma unroll
         for (int v = 0; v < V; ++v)
-            red[wave][v][lane] = acc[v / (4 * TN)][(v >> 2) % TN][v & 3];
+            red.at[wave][v][lane] = acc[v / (4 * TN)][(v >> 2) % TN][v & 3];
         __syncthreads();
 #pragma unroll
         for (int u = 0; u < V / 2 / WK; ++u) {
             const int pair = wk + WK * u, v = 8 * (pair >> 2) + (pair & 3);
-            double s0 = red[tile * WK][v][lane], s1 = red[tile * WK][v + 4][lane];
+            double s0 = red.at[tile * WK][v][lane], s1 = red.at[tile * WK][v + 4][lane];
 #pragma unroll
             for (int w = 1; w < WK; ++w) {
-                s0 += red[tile * WK + w][v][lane];
-                s1 += red[tile * WK + w][v + 4][lane];
+                s0 += red.at[tile * WK + w][v][lane];
+                s1 += red.at[tile * WK + w][v + 4][lane];
             }
             store(v, s0, s1);
         }
     }
     vtlhip::raise_when_last(g.done);   // (a launch that leaves partial sums has no signal)
+}
+
+template <typename T, int WM, int WN, int WK, int TM, int TN, bool TA, bool TB, bool CHECKED>
+__global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel(const MatmulArgs g)
+{
+    __shared__ PartialTiles<WM, WN, WK, TM, TN> red;
+    direct_tile<T, WM, WN, WK, TM, TN, TA, TB, CHECKED>(g, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y,
+                                                        blockIdx.x + gridDim.x * blockIdx.y, red);
+}
+
+// The sums of kSumCols columns by one workgroup of 256 threads: 16 phases of rows, added in order.  Rows start at any element.
+constexpr int kSumCols = 64;
+
+template <typename T>
+struct ColumnSums {
+    const T *x;
+    int rows, cols;
+    T *out;
+};
+
+template <typename T>
+__device__ __forceinline__ void colsum_tile(const ColumnSums<T> &g, int block, const vtlhip::DoneSignal &done,
+                                            double (&red)[16][kSumCols])
+{
+    struct alignas(sizeof(T)) Run {
+        T v[4];
+    };
+    const int group = threadIdx.x & 15, phase = threadIdx.x >> 4, c = block * kSumCols + 4 * group;
+    double acc[4] = {0.0, 0.0, 0.0, 0.0};
+    if (c + 4 <= g.cols) {
+        const T *at = g.x + c;
+        int r = phase;
+        for (; r + 48 < g.rows; r += 64) {   // four loads in flight
+            Run v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                v[u] = *reinterpret_cast<const Run *>(at + (int64_t)(r + 16 * u) * g.cols);
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    acc[j] += (double)v[u].v[j];
+        }
+        for (; r < g.rows; r += 16) {
+            const Run v = *reinterpret_cast<const Run *>(at + (int64_t)r * g.cols);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                acc[j] += (double)v.v[j];
+        }
+    } else {
+        for (int r = phase; r < g.rows; r += 16)
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                if (c + j < g.cols)
+                    acc[j] += (double)g.x[(int64_t)r * g.cols + c + j];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        red[phase][4 * group + j] = acc[j];
+    __syncthreads();
+    const int mine = block * kSumCols + (int)threadIdx.x;
+    if (threadIdx.x < kSumCols && mine < g.cols) {
+        double s = 0.0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            s += red[i][threadIdx.x];
+        vtlhip::store_result(g.out + mine, (T)s, done);
+    }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void colsum_short_kernel(const ColumnSums<T> g)
+{
+    __shared__ double red[16][kSumCols];
+    colsum_tile(g, (int)blockIdx.x, vtlhip::DoneSignal{}, red);
+}
+
+// ---- a Linear layer's gradients in one launch -----------------------------------------------
+// dX = grad . W, dW = grad^T . x and db need nothing of each other, and of a small layer each leaves most of the chip idle for the 3
+// to 5 us that a launch takes at least: workgroups 0 .. dx_blocks - 1 have the tiles of dX (slice by slice of K; the longest first), the next
+// dw_blocks those of dW, the others the column sums.  Fifty sets of gradients of 16 to 256 rows, 64 to 8716 x 64 to 3722 parameters, half f32 and half f64:
+// 19.2 us launch by launch, 12.3 now (geometric mean); 64 x 256 x 640 10.9 -> 5.6, 192 x 832 x 832 22.5 -> 13.8, 192 x 4096 x 1600 123 -> 95; with the
+// forward in front 33 -> 28.
+template <typename T>
+struct BackwardArgs {
+    MatmulArgs dx, dw;
+    int dx_tiles, dx_blocks, dw_blocks;
+    ColumnSums<T> db;
+};
+
+template <typename T, int TNX, int TNW>
+__global__ __launch_bounds__(256) void linear_backward_kernel(const BackwardArgs<T> g)
+{
+    __shared__ union {
+        PartialTiles<1, 1, 4, 2, TNX> dx;
+        PartialTiles<1, 1, 4, 2, TNW> dw;
+        double db[16][kSumCols];
+    } red;
+    int block = (int)blockIdx.x;
+    if (block < g.dx_blocks) {
+        direct_tile<T, 1, 1, 4, 2, TNX, false, false, false>(g.dx, block % g.dx_tiles, block / g.dx_tiles, 1, blockIdx.x, red.dx);
+        return;
+    }
+    block -= g.dx_blocks;
+    if (block < g.dw_blocks) {
+        direct_tile<T, 1, 1, 4, 2, TNW, true, false, false>(g.dw, block, 0, 1, blockIdx.x, red.dw);
+        return;
+    }
+    colsum_tile(g.db, block - g.dw_blocks, g.dw.done, red.db);
+    vtlhip::raise_when_last(g.dw.done);
 }
 
 // Column sums with f64 accumulation: la.matmul(ones[1,M], grad) of
@@ -660,6 +777,7 @@ struct Plan {
     Shape shape;
     int slices;
     int tail_slices;   // of the last round's tiles alone
+    double us;         // estimated
 };
 
 // Three kinds of product differ in what a shape costs: f32, f64, and f64 with K along both operands' rows (the
@@ -701,14 +819,13 @@ constexpr double kLaunch = 0.6;
 Kind kind_of(bool f64, bool ta, bool tb) { return !f64 ? kF32 : (!ta && tb ? kF64Rows : kF64); }
 
 // may_slice: whether K may be cut (matmul_impl).
-Plan choose_plan(Kind kind, int m, int n, int k, bool may_slice, bool may_tail, double launch)
+Plan choose_plan(Kind kind, int m, int n, int k, bool may_slice, bool may_tail, double launch, unsigned shapes = ~0u)
 {
-    Plan best = {kK4, 1, 1};
-    double best_us = 1e30;
+    Plan best = {kK4, 1, 1, 1e30};
     const int most_slices = k / 96;
     for (int s = 0; s < kShapes; s++) {
         const int bm = kTileM[kind][s], bn = kTileN[kind][s], unit = kPerUnit[kind][s];
-        if (bm == 0)
+        if (bm == 0 || !(shapes >> s & 1))
             continue;
         const Cost &c = kCost[kind][s];
         // (tile sides are powers of two, and so is what fills the chip: no divisions where a small product spends its time)
@@ -734,10 +851,8 @@ Plan choose_plan(Kind kind, int m, int n, int k, bool may_slice, bool may_tail, 
             double us = c.start + rounds * (c.per_tile + work * c.inverse_rate);
             if (slices > 1)
                 us += c.slice_start + launch + c.slice_mb * 8e-6 * (double)slices * (double)m * (double)n;
-            if (us < best_us) {
-                best_us = us;
-                best = {(Shape)s, (int)slices, 1};
-            }
+            if (us < best.us)
+                best = {(Shape)s, (int)slices, 1, us};
         }
         // The last round with few tiles: K cut until they fill the chip.  For kSquare alone: its sums take 128 KiB of LDS, one
         // workgroup is all a compute unit holds, and a round is as long as its last (f64 forward, us: 256 x 4352 x 4096
@@ -752,10 +867,8 @@ Plan choose_plan(Kind kind, int m, int n, int k, bool may_slice, bool may_tail, 
                 const double us = c.start + (double)whole * (c.per_tile + work * c.inverse_rate) + c.per_tile +
                                   work / (double)slices * c.inverse_rate + c.slice_start +
                                   c.slice_mb * 8e-6 * (double)(slices * left) * bm * bn;
-                if (us < best_us) {
-                    best_us = us;
-                    best = {(Shape)s, 1, (int)slices};
-                }
+                if (us < best.us)
+                    best = {(Shape)s, 1, (int)slices, us};
             }
         }
     }
@@ -795,6 +908,26 @@ int launch_direct_shape(MatmulArgs g, bool ta, bool tb, int slices, hipStream_t 
     return check_launch("matmul_f64acc_direct_kernel");
 }
 
+MatmulArgs arguments(const void *a, const void *b, void *c, int m, int n, int k)
+{
+    MatmulArgs g = {};
+    g.A = a;
+    g.B = b;
+    g.C = c;
+    g.M = m;
+    g.N = n;
+    g.K = k;
+    g.tail_slices = 1;
+    return g;
+}
+
+// Pairs of a row or column index that runs along memory need two of them.
+template <typename T>
+bool needs_checks(int m, int n, int k, bool ta, bool tb)
+{
+    return (ta && (m < 2 || m > kLongest16<T>)) || (!tb && (n < 2 || n > kLongest16<T>)) || ((!ta || tb) && k > kLongest64<T>);
+}
+
 // Memory for the slices' partial sums.  While the process uses the null stream alone (`alone`) it is a block
 // of the call's own, released when the launches that use it are enqueued: the next owner's work comes
 // behind them, and calls of several threads never meet in it.  Once a stream has been named a release would
@@ -820,9 +953,7 @@ struct Partial {
 template <typename T>
 int launch_direct(MatmulArgs g, Kind kind, bool ta, bool tb, Plan plan, bool alone, hipStream_t st)
 {
-    // pairs of a row or column index that runs along memory need two of them
-    const bool checked = (ta && (g.M < 2 || g.M > kLongest16<T>)) || (!tb && (g.N < 2 || g.N > kLongest16<T>)) ||
-                         ((!ta || tb) && g.K > kLongest64<T>);
+    const bool checked = needs_checks<T>(g.M, g.N, g.K, ta, tb);
     const int steps = steps_of(g.K);
     int per = (steps + plan.slices - 1) / plan.slices;
     int slices = per > 0 ? (steps + per - 1) / per : 1;
@@ -834,7 +965,6 @@ int launch_direct(MatmulArgs g, Kind kind, bool ta, bool tb, Plan plan, bool alo
             slices = 1;
         }
     }
-    g.tail_slices = 1;
     constexpr int bm = 64, bn = 64;   // kSquare
     int64_t left = 0;
     if (plan.tail_slices > 1 && plan.shape == kSquare && slices == 1 && !checked && !g.result) {
@@ -885,15 +1015,9 @@ int matmul_impl(const T *a, const T *b, T *c, const T *bias, int m, int n, int k
         return VTL_HIP_OK;
     if (!c || (k > 0 && (!a || !b)))
         return VTL_HIP_ERR_INVALID_ARG;
-    MatmulArgs g = {};
+    MatmulArgs g = arguments(a, b, c, m, n, k);
     g.result = result;
-    g.A = a;
-    g.B = b;
-    g.C = c;
     g.bias = bias;
-    g.M = m;
-    g.N = n;
-    g.K = k;
     g.relu = relu;
     // Where streams have been named, K is cut from 2048 on only: there the header asks callers to order
     // calls of different streams, which then share scratch; shorter products stay independent of each other
@@ -915,6 +1039,11 @@ int matmul_impl(const T *a, const T *b, T *c, const T *bias, int m, int n, int k
     return launch_direct<T>(g, kind, trans_a != 0, trans_b != 0, plan, alone, current_stream());
 }
 
+// Up to this many rows one launch has the column sums, a workgroup all rows of its columns; beyond, the rows are split and a second
+// launch adds up (us, split and in one: f32 256 x 11008 6.5 and 3.4, 128 x 300 6.3 and 3.6, 512 x 4097 6.7 and 6.4, 1024 x 4097 10.2
+// and 11.1; f64 512 x 11008 11.4 and 7.9, 1024 x 4097 13.2 and 21.0).
+constexpr int64_t kShortSums = 512;
+
 template <typename T>
 int colsum_impl(const T *x, int64_t rows, int64_t cols, T *out)
 {
@@ -925,6 +1054,11 @@ int colsum_impl(const T *x, int64_t rows, int64_t cols, T *out)
     if (!out || (rows > 0 && !x))
         return VTL_HIP_ERR_INVALID_ARG;
     hipStream_t st = current_stream();
+    if (rows <= kShortSums && cols <= 0x7fffffff - kSumCols) {
+        const ColumnSums<T> g = {x, (int)rows, (int)cols, out};
+        hipLaunchKernelGGL((colsum_short_kernel<T>), dim3((unsigned)((cols + kSumCols - 1) / kSumCols)), dim3(256), 0, st, g);
+        return check_launch("colsum_short_kernel");
+    }
     const bool vec = aligned16(x) && cols % 4 == 0;
     const int per_block = vec ? 256 : 64;
     const int64_t col_blocks = (cols + per_block - 1) / per_block;
@@ -966,6 +1100,97 @@ int colsum_impl(const T *x, int64_t rows, int64_t cols, T *out)
     return check_launch("colsum_finalize_kernel");
 }
 
+// Whether memory of `a_bytes` from a and of `b_bytes` from b meet.
+bool meet(const void *a, size_t a_bytes, const void *b, size_t b_bytes)
+{
+    const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+    return a && b && pa < pb + b_bytes && pb < pa + a_bytes;
+}
+
+// dW and what else is asked for (not null) in one launch; false: launch by launch.  `result`: dw and db are its memory, and this is
+// the call's last launch.
+template <typename T>
+bool backward_in_one(vtlhip::HostResult *result, const T *grad, const T *x, const T *w, T *dx, T *dw, T *db, int m, int n, int k,
+                     int &status)
+{
+    const int forced = vtlhip::tuning().backward_group;
+    if (!dw || !(dx || db) || m < 1 || n < 1 || k < 1 || (db && m > kShortSums) || forced == 0 || vtlhip::tuning().matmul_tile > 0 ||
+        vtlhip::tuning().matmul_splits != -1 || needs_checks<T>(n, k, m, true, false) || (dx && needs_checks<T>(m, k, n, false, false)))
+        return false;
+    // launch by launch a gradient may take the place of what those before it were made from
+    const size_t e = sizeof(T), grad_bytes = (size_t)m * n * e, x_bytes = (size_t)m * k * e, w_bytes = (size_t)n * k * e, b_bytes = (size_t)n * e;
+    const struct { const void *at; size_t bytes; } all[6] = {{grad, grad_bytes}, {x, x_bytes}, {dx ? w : nullptr, w_bytes},
+                                                             {dx, x_bytes}, {dw, w_bytes}, {db, b_bytes}};
+    for (int i = 3; i < 6; i++)
+        for (int j = 0; j < i; j++)
+            if (meet(all[i].at, all[i].bytes, all[j].at, all[j].bytes))
+                return false;
+
+    const bool alone = vtlhip::single_stream();
+    const Kind kind = sizeof(T) == 8 ? kF64 : kF32;
+    constexpr unsigned shapes = 1u << kK4 | 1u << kWide;   // workgroups of four waves
+    const Plan pw = choose_plan(kind, n, k, m, false, false, kLaunch, shapes);
+    const Plan px = dx ? choose_plan(kind, m, k, n, alone || n >= 2048, false, kLaunch, shapes) : Plan{kK4, 1, 1, 0.0};
+    const auto tiles = [&](Shape s, int rows, int cols) {
+        return (int64_t)((rows + 31) / 32) * ((cols + kTileN[kind][s] - 1) / kTileN[kind][s]);
+    };
+    const auto tile_us = [&](Shape s, double depth) {
+        const Cost &c = kCost[kind][s];
+        return c.per_tile + 32.0 * kTileN[kind][s] * depth / (64.0 * 2300.0) * c.inverse_rate;
+    };
+    const int64_t tiles_w = tiles(pw.shape, n, k), tiles_x = dx ? tiles(px.shape, m, k) : 0;
+    const int64_t sums = db ? (n + kSumCols - 1) / kSumCols : 0;
+    const int steps = steps_of(n), per = (steps + px.slices - 1) / px.slices, slices = dx ? (steps + per - 1) / per : 1;
+    if (tiles_w + tiles_x * slices + sums > 0x7fffffff)
+        return false;
+    if (forced < 0) {
+        // As choose_plan estimates, the tiles of both products dealt out over the chip.  Sets of gradients from 16 x 92 x 421 to 256 x
+        // 9728 x 320, f32 and f64, in one launch and one by one: up to 0.9 of `apart` 0.39 to 0.86 of the time, up to 1.05 0.8 to 1.01; above 1.2, where
+        // large weight tiles have shapes of their own, 0.98 to 1.26.
+        const double each_x = tile_us(px.shape, (double)n / px.slices), each_w = tile_us(pw.shape, m);
+        const double longest = dx && each_x > each_w ? each_x : each_w;
+        double us = 2.9 + ((double)(tiles_x * px.slices) * each_x + (double)tiles_w * each_w) / 256.0 + 0.5 * longest;
+        if (px.slices > 1)
+            us += kCost[kind][px.shape].slice_start + kLaunch + kCost[kind][px.shape].slice_mb * 8e-6 * px.slices * (double)m * (double)k;
+        double apart = choose_plan(kind, n, k, m, alone || m >= 2048, false, kLaunch).us + (db ? 4.0 : 0.0);
+        if (dx)
+            apart += choose_plan(kind, m, k, n, alone || n >= 2048, false, kLaunch).us;
+        if (us > 1.05 * apart)
+            return false;
+    }
+    BackwardArgs<T> g = {};
+    g.dw = arguments(grad, x, dw, n, k, m);
+    g.dw.slice_steps = steps_of(m);
+    g.dw_blocks = (int)tiles_w;
+    g.dx = arguments(grad, w, dx, m, k, n);
+    g.dx.slice_steps = per;
+    g.db = {grad, m, n, db};
+    Partial partial;
+    int cut = slices;
+    if (cut > 1 && !(g.dx.partial = partial.take((size_t)cut * (size_t)m * (size_t)k * sizeof(double), alone))) {
+        g.dx.slice_steps = steps;   // no memory, or a capture that may not allocate: K in one piece
+        cut = 1;
+    }
+    g.dx_tiles = (int)(tiles_x > 0 ? tiles_x : 1);
+    g.dx_blocks = (int)tiles_x * cut;
+    const dim3 grid((unsigned)(g.dx_blocks + tiles_w + sums));
+    if (result && !dx)
+        result->attach(g.dw.done, grid.x);
+    hipStream_t st = current_stream();
+    if (px.shape == kK4 && pw.shape == kK4)
+        hipLaunchKernelGGL((linear_backward_kernel<T, 2, 2>), grid, dim3(256), 0, st, g);
+    else if (px.shape == kK4)
+        hipLaunchKernelGGL((linear_backward_kernel<T, 2, 4>), grid, dim3(256), 0, st, g);
+    else if (pw.shape == kK4)
+        hipLaunchKernelGGL((linear_backward_kernel<T, 4, 2>), grid, dim3(256), 0, st, g);
+    else
+        hipLaunchKernelGGL((linear_backward_kernel<T, 4, 4>), grid, dim3(256), 0, st, g);
+    status = check_launch("linear_backward_kernel");
+    if (status == VTL_HIP_OK && cut > 1)
+        status = finalize_split<T>(g.dx, cut, st);
+    return true;
+}
+
 template <typename T>
 int linear_backward_impl(const T *grad, const T *x, const T *w, T *dx, T *dw, T *db, int m, int n, int k)
 {
@@ -974,6 +1199,8 @@ int linear_backward_impl(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
     if ((dx && !w) || (dw && !x))
         return VTL_HIP_ERR_INVALID_ARG;
     int rc = VTL_HIP_OK;
+    if (backward_in_one<T>(nullptr, grad, x, w, dx, dw, db, m, n, k, rc))
+        return rc;
     if (dx)   // [M,K] = grad[M,N] . W[N,K]
         rc = matmul_impl<T>(grad, w, dx, nullptr, m, k, n, 0, 0, 0);
     if (rc == VTL_HIP_OK && dw)   // [N,K] = grad^T[N,M] . x[M,K]
@@ -981,6 +1208,18 @@ int linear_backward_impl(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
     if (rc == VTL_HIP_OK && db)   // [1,N] = ones[1,M] . grad[M,N]
         rc = colsum_impl<T>(grad, m, n, db);
     return rc;
+}
+
+// dW and, unless it is null, db.
+template <typename T>
+int weight_gradients(vtlhip::HostResult *result, const T *grad, const T *x, T *dw, T *db, int m, int n, int k)
+{
+    int rc = VTL_HIP_OK;
+    if (backward_in_one<T>(result, grad, x, nullptr, nullptr, dw, db, m, n, k, rc))
+        return rc;
+    if (db)
+        rc = colsum_impl<T>(grad, m, n, db);
+    return rc == VTL_HIP_OK ? matmul_impl<T>(grad, x, dw, nullptr, n, k, m, 1, 0, 0, result) : rc;
 }
 
 }  // namespace
@@ -995,6 +1234,16 @@ int matmul_to(HostResult *result, const float *a, const float *b, float *c, int 
 int matmul_to(HostResult *result, const double *a, const double *b, double *c, int m, int n, int k, int trans_a)
 {
     return matmul_impl<double>(a, b, c, nullptr, m, n, k, trans_a, 0, 0, result);
+}
+
+int weight_gradients_to(HostResult *result, const float *grad, const float *x, float *dw, float *db, int m, int n, int k)
+{
+    return weight_gradients<float>(result, grad, x, dw, db, m, n, k);
+}
+
+int weight_gradients_to(HostResult *result, const double *grad, const double *x, double *dw, double *db, int m, int n, int k)
+{
+    return weight_gradients<double>(result, grad, x, dw, db, m, n, k);
 }
 
 }  // namespace vtlhip
