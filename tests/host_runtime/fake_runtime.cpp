@@ -175,6 +175,18 @@ hipError_t hipLaunchKernel(const void *function, dim3 grid, dim3, void **args, s
         more += " " + std::to_string((unsigned long long)(uintptr_t) static_cast<void **>(args[0])[2]);
     else if (more.find("13colsum_kernel") != std::string::npos)              // x, rows, cols, rows of a split, out
         more += " " + std::to_string((unsigned long long)(uintptr_t) * static_cast<void **>(args[4]));
+    else if (more.find("colsum_short_kernel") != std::string::npos)          // its argument begins with x, rows and cols, out
+        more += " " + std::to_string((unsigned long long)(uintptr_t) static_cast<void **>(args[0])[2]);
+    else if (more.find("linear_backward_kernel") != std::string::npos) {     // that, and those of two products of 104 bytes each
+        void **words = static_cast<void **>(args[0]);
+        const std::string name = more;
+        for (int at : {3 + 2, 3 + 13 + 2})
+            if (words[at])
+                note("launch", st, (unsigned long long)grid.x, name + " " + std::to_string((unsigned long long)(uintptr_t)words[at]));
+        if (!words[2])
+            return hipSuccess;
+        more += " " + std::to_string((unsigned long long)(uintptr_t)words[2]);
+    }
     note("launch", st, (unsigned long long)grid.x * grid.y * grid.z, more);
     return hipSuccess;
 }

@@ -611,9 +611,9 @@ __global__ __launch_bounds__(256) void colsum_short_kernel(const ColumnSums<T> g
 // forward in front 33 -> 28.
 template <typename T>
 struct BackwardArgs {
+    ColumnSums<T> db;
     MatmulArgs dx, dw;
     int dx_tiles, dx_blocks, dw_blocks;
-    ColumnSums<T> db;
 };
 
 template <typename T, int TNX, int TNW>
