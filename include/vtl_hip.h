@@ -101,6 +101,11 @@ int vtl_hip_memcpy_d2h(void *dst_host, const void *src_device, size_t bytes);
  * used a stream of its own, vtl_hip_set_stream.)  Work on a non-blocking stream that was never named does
  * not: use vtl_hip_memcpy_h2d for what such a stream reads. */
 int vtl_hip_upload(void *dst_device, const void *src_host, size_t bytes);
+/* vtl_hip_upload of rows x cols f32 and vtl_hip_quantize_f32_i8 of them, with the f32 values in no memory of the
+ * caller's (with a scale per row they are quantized as they arrive where that can be), and a vtl_hip_upload of
+ * extra_bytes (0: none) with them. */
+int vtl_hip_upload_quantized(const float *src_host, int64_t rows, int64_t cols, int per_row, int8_t *q, float *scale,
+                             void *extra_device, const void *extra_host, size_t extra_bytes);
 /* `count` copies of vtl_hip_memcpy_d2h with one wait for all of them. */
 int vtl_hip_download(int count, void *const *dst_host, const void *const *src_device, const size_t *bytes);
 /* Host memory that downloads reach without a copy by the host.  At most 1 GiB at a time

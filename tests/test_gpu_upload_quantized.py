@@ -1,0 +1,48 @@
+"""Rows that are quantized as they come over the link: the same bits as an upload and the quantizer behind it."""
+import numpy as np
+import pytest
+
+from helpers import dev
+from vtl_amd import capi
+from vtl_amd.tensor import HipTensor
+
+pytestmark = pytest.mark.gpu
+
+
+# 32 MiB and more are quantized on the way: edges of a workgroup's registers, rows that do not divide the pieces a transfer is
+# cut into (rows are not cut); less, longer, shorter and odd rows go in two steps
+@pytest.mark.parametrize("rows,cols", [(8192, 1024), (8191, 1024), (8200, 1028), (4096, 2048), (4100, 2052), (3000, 2800), (2049, 4096), (2100, 4100),
+                                       (1024, 8192), (1031, 8188), (1030, 8196), (33000, 256), (8300, 1023), (300, 1024), (1, 4)])
+@pytest.mark.parametrize("extra", [0, 4096 + 20])
+def test_same_bits_as_upload_and_quantize(hip, rows, cols, extra):
+    rng = np.random.default_rng(rows + cols)
+    x = rng.standard_normal((rows, cols)).astype(np.float32) * np.float32(10.0) ** rng.integers(-3, 4, (rows, 1)).astype(np.float32)
+    x[rows // 2] = 0.0
+    x[rows // 3, :: 5] = np.nan
+    x[-1, cols // 2] = np.inf
+    more = rng.integers(0, 256, extra, dtype=np.uint8)
+    print("rows", rows, cols, extra, flush=True)
+    for per_row in (1, 0):
+        xd = dev(x)
+        want_q, want_s = xd.quantize_i8(0 if per_row else -1)
+        q, s = HipTensor.empty([rows, cols], np.int8), HipTensor.empty([rows if per_row else 1], np.float32)
+        room = HipTensor.empty([extra + 64], np.uint8)
+        for _ in range(2):
+            capi.call("vtl_hip_upload_quantized", x.ctypes.data, rows, cols, per_row, q.ptr, s.ptr, room.ptr + 16 if extra else None,
+                      more.ctypes.data if extra else None, extra)
+            assert np.array_equal(q.cpu(), want_q.cpu())
+            assert np.array_equal(s.cpu().view(np.int32), want_s.cpu().view(np.int32))
+            assert np.array_equal(room.cpu()[16:16 + extra], more)
+        for t in (xd, want_q, want_s, q, s, room):
+            t.release()
+
+
+def test_errors(hip):
+    x, q = np.zeros((4, 8), np.float32), HipTensor.empty([4, 8], np.int8)
+    s = HipTensor.empty([4], np.float32)
+    for args in ((None, 4, 8, 1, q.ptr, s.ptr, None, None, 0), (x.ctypes.data, -1, 8, 1, q.ptr, s.ptr, None, None, 0),
+                 (x.ctypes.data, 4, 8, 1, None, s.ptr, None, None, 0), (x.ctypes.data, 4, 8, 1, q.ptr, None, None, None, 0),
+                 (x.ctypes.data, 4, 8, 1, q.ptr, s.ptr, None, x.ctypes.data, 4)):
+        assert capi.status("vtl_hip_upload_quantized", *args) == capi.ERR_INVALID_ARG
+    for t in (q, s):
+        t.release()

@@ -76,6 +76,10 @@ private:
 // Two uploads as vtl_hip_upload makes them, which share their launches; false: to be made one by one.
 bool upload_two(void *dst0, const void *src0, size_t bytes0, void *dst1, const void *src1, size_t bytes1, int &status);
 
+// Rows that are quantized as they arrive, one scale each, and extra bytes copied with them; false: to be uploaded and quantized.
+bool upload_rows(const float *src, int64_t rows, int64_t cols, int8_t *q, float *scale, void *extra_dst, const void *extra_src,
+                 size_t extra_bytes, int &status);
+
 // How a launch tells the host that its results are there: every workgroup counts itself when its stores are
 // complete, and the one that reaches the target raises the flag.  No flag: nothing to tell.
 struct DoneSignal {

@@ -36,6 +36,7 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 using vtlhip::HostResult;
 using vtlhip::raise_when_last;
 using vtlhip::store_result;
+using vtlhip::qdev::lds_barrier;
 
 // Four of them from element `at` of out, 16-byte aligned unless they are written through (a host call's result: a few MiB).
 __device__ __forceinline__ void store_result4(float *out, int64_t at, f4 v, const vtlhip::DoneSignal &done)
@@ -830,16 +831,6 @@ __global__ __launch_bounds__(256) void requant_rows_wide_kernel(const float *__r
     for (int i = 0; i < 4; i++)
         if (n + 1024 * i < N)
             out[(n + 1024 * i) >> 2] = vtlhip::qdev::quant4(v[i], qp);
-}
-
-// Workgroup barrier that orders LDS traffic only: unlike __syncthreads() it does
-// not wait for outstanding global loads, so direct-to-LDS weight loads issued
-// earlier stay in flight across it.
-__device__ __forceinline__ void lds_barrier()
-{
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
 }
 
 // ---- activations quantized inside the weight-streaming launch ----------------

@@ -315,6 +315,28 @@ int vtl_hip_forward_i8_host(const float *x_host, int rows, int cols, const vtl_h
     return forward_layers(x_host, rows, cols, layers, count, y_host);
 }
 
+int vtl_hip_upload_quantized(const float *src_host, int64_t rows, int64_t cols, int per_row, int8_t *q, float *scale,
+                             void *extra_device, const void *extra_host, size_t extra_bytes)
+{
+    if (rows < 0 || cols < 0 || (rows > 0 && cols > 0 && (!src_host || !q)) || (extra_bytes && (!extra_device || !extra_host)))
+        return VTL_HIP_ERR_INVALID_ARG;
+    int status = VTL_HIP_OK;
+    if (per_row && scale && rows > 0 && cols > 0 &&
+        upload_rows(src_host, rows, cols, q, scale, extra_device, extra_host, extra_bytes, status))
+        return status;
+    const size_t bytes = (size_t)rows * (size_t)cols * sizeof(float);
+    Scratch x;
+    VTL_STEP(x.take(bytes));
+    if (!upload_two(x.ptr, src_host, bytes, extra_device, extra_host, extra_bytes, status)) {
+        if (bytes)
+            VTL_STEP(vtl_hip_upload(x.ptr, src_host, bytes));
+        if (extra_bytes)
+            VTL_STEP(vtl_hip_upload(extra_device, extra_host, extra_bytes));
+    }
+    VTL_STEP(status);
+    return vtl_hip_quantize_f32_i8(x.as<float>(), rows, cols, per_row, q, scale);
+}
+
 int vtl_hip_matmul_host_f32(const float *a, const float *b, float *c, int m, int n, int k)
 {
     return matmul_host<float>(a, b, c, m, n, k);

@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "quant_device.hpp"
 
 namespace vtlhip {
 
@@ -119,33 +120,129 @@ __device__ __forceinline__ void raise_done(const LinkSignals &s)
     }
 }
 
+// One workgroup's share of a segment.
+__device__ __forceinline__ void copy_segment(const Segment &seg)
+{
+    const size_t first = (size_t)blockIdx.x * 512 + threadIdx.x, step = (size_t)gridDim.x * 512;
+    const uint4 *src = reinterpret_cast<const uint4 *>(seg.src + seg.head);
+    uint4 *dst = reinterpret_cast<uint4 *>(seg.dst + seg.head);
+    size_t i = first;
+    for (; i + 3 * step < seg.nvec; i += 4 * step) {   // four reads of the link in flight per lane
+        const uint4 a = src[i], b = src[i + step], c = src[i + 2 * step], d = src[i + 3 * step];
+        dst[i] = a;
+        dst[i + step] = b;
+        dst[i + 2 * step] = c;
+        dst[i + 3 * step] = d;
+    }
+    for (; i < seg.nvec; i += step)
+        dst[i] = src[i];
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < seg.head)
+            seg.dst[threadIdx.x] = seg.src[threadIdx.x];
+        const size_t end = seg.head + seg.nvec * 16;
+        if (threadIdx.x < seg.tail)
+            seg.dst[end + threadIdx.x] = seg.src[end + threadIdx.x];
+    }
+}
+
 __global__ __launch_bounds__(512) void host_copy_kernel(const CopyArgs g)
 {
     raise_behind(g.signals);
-    const size_t first = (size_t)blockIdx.x * 512 + threadIdx.x, step = (size_t)gridDim.x * 512;
+    for (int s = 0; s < g.count; s++)
+        copy_segment(g.seg[s]);
+    raise_done(g.signals);
+}
+
+// f32 rows in pinned memory that arrive as codes and scales, `cols` of the launch each.
+struct Rows {
+    const float *src;    // 16-byte aligned; nullptr: none
+    int8_t *q;
+    float *scale;
+    int count;
+};
+
+struct RowsArgs {
+    Rows rows[kMaxSegments];
+    Segment seg[kMaxSegments];   // copied as they are
+    int count, copies, cols;
+    LinkSignals signals;
+};
+
+// Per-row quantization of what comes over the link: the f32 rows never lie in device memory, and no launch behind the transfer reads
+// them again.  Bound by the link, 56 GB/s as the copy: a workgroup has one row in registers and the next one on its way.  The end of
+// a launch, when the last rows are there, is a microsecond longer than a copy's, so it is for transfers of many MiB a
+// launch (us, copy and quantizer behind it, and this: 11008 x 4096 3659 and 3614 of a forward, 4096 x 4096 1279 and
+// 1265; 512 x 4096 213 and 217, 1000 x 1000 120 and 122).  More workgroups take longer on the link (4096 x 4096 with 16 1270,
+// 32 1303, 64 1308).  Arithmetic as in quant.hip.
+constexpr size_t kRowsFrom = (size_t)32 << 20;
+constexpr int kRowsLeastCols = 1024, kRowsMostCols = 8192;
+
+template <int NV>
+__global__ __launch_bounds__(512) void upload_rows_kernel(const RowsArgs g)
+{
+    using namespace qdev;
+    __shared__ float smem[2][8];
+    raise_behind(g.signals);
+    const int tid = (int)threadIdx.x, nv = g.cols >> 2;
+    int turn = 0;
     for (int s = 0; s < g.count; s++) {
-        const Segment &seg = g.seg[s];
-        const uint4 *src = reinterpret_cast<const uint4 *>(seg.src + seg.head);
-        uint4 *dst = reinterpret_cast<uint4 *>(seg.dst + seg.head);
-        size_t i = first;
-        for (; i + 3 * step < seg.nvec; i += 4 * step) {   // four reads of the link in flight per lane
-            const uint4 a = src[i], b = src[i + step], c = src[i + 2 * step], d = src[i + 3 * step];
-            dst[i] = a;
-            dst[i + step] = b;
-            dst[i + 2 * step] = c;
-            dst[i + 3 * step] = d;
-        }
-        for (; i < seg.nvec; i += step)
-            dst[i] = src[i];
-        if (blockIdx.x == 0) {
-            if (threadIdx.x < seg.head)
-                seg.dst[threadIdx.x] = seg.src[threadIdx.x];
-            const size_t end = seg.head + seg.nvec * 16;
-            if (threadIdx.x < seg.tail)
-                seg.dst[end + threadIdx.x] = seg.src[end + threadIdx.x];
+        const Rows &part = g.rows[s];
+        float4_t next[NV];
+        auto load = [&](int row) {
+#pragma unroll
+            for (int i = 0; i < NV; i++) {
+                const int idx = i * 512 + tid;
+                next[i] = float4_t{0.f, 0.f, 0.f, 0.f};
+                if (row < part.count && idx < nv)
+                    next[i] = reinterpret_cast<const float4_t *>(part.src)[(size_t)row * nv + idx];
+            }
+        };
+        load((int)blockIdx.x);
+        for (int row = (int)blockIdx.x; row < part.count; row += (int)gridDim.x) {
+            float4_t v[NV];
+#pragma unroll
+            for (int i = 0; i < NV; i++)
+                v[i] = next[i];
+            load(row + (int)gridDim.x);
+            float m = 0.0f;
+#pragma unroll
+            for (int i = 0; i < NV; i++)
+                m = absmax4(m, v[i]);
+            m = wave_max(m);
+            if ((tid & 63) == 0)
+                smem[turn][tid >> 6] = m;
+            lds_barrier();   // (the next row stays on its way)
+            m = smem[turn][0];
+#pragma unroll
+            for (int i = 1; i < 8; i++)
+                m = fmaxf(m, smem[turn][i]);
+            turn ^= 1;       // the next row's maxima: others may still read these
+            const float scale = m / 127.0f;
+            if (tid == 0)
+                part.scale[row] = scale;
+            const QuantScale p = make_quant_scale(scale);
+#pragma unroll
+            for (int i = 0; i < NV; i++) {
+                const int idx = i * 512 + tid;
+                if (idx < nv)
+                    reinterpret_cast<unsigned *>(part.q)[(size_t)row * nv + idx] = quant4(v[i], p);
+            }
         }
     }
+    for (int s = 0; s < g.copies; s++)
+        copy_segment(g.seg[s]);
     raise_done(g.signals);
+}
+
+void launch_upload_rows(const RowsArgs &g, unsigned blocks, hipStream_t st)
+{
+    const dim3 grid(blocks), block(512);
+    if (g.cols <= 2048)
+        hipLaunchKernelGGL((upload_rows_kernel<1>), grid, block, 0, st, g);
+    else if (g.cols <= 4096)
+        hipLaunchKernelGGL((upload_rows_kernel<2>), grid, block, 0, st, g);
+    else
+        hipLaunchKernelGGL((upload_rows_kernel<4>), grid, block, 0, st, g);
 }
 
 Segment make_segment(void *dst, const void *src, size_t bytes)
@@ -640,6 +737,40 @@ struct Source {
     void *dst;
     const void *src;
     size_t bytes;
+    // rows that arrive as codes and scales instead, and the bytes of one (they are not cut)
+    int8_t *q = nullptr;
+    float *scale = nullptr;
+    size_t unit = 0;
+};
+
+// What a launch carries: `staged` in pinned memory.
+struct Load {
+    RowsArgs rows = {};
+    CopyArgs copy = {};
+
+    void add(const Source &piece, char *staged)
+    {
+        if (!piece.unit) {
+            copy.seg[copy.count++] = make_segment(piece.dst, staged, piece.bytes);
+            return;
+        }
+        rows.rows[rows.count++] = {reinterpret_cast<const float *>(staged), piece.q, piece.scale, (int)(piece.bytes / piece.unit)};
+        rows.cols = (int)(piece.unit / sizeof(float));
+    }
+    int launch(unsigned blocks, const LinkSignals &signals, hipStream_t st)
+    {
+        if (rows.count == 0) {
+            copy.signals = signals;
+            hipLaunchKernelGGL(host_copy_kernel, dim3(blocks), dim3(512), 0, st, copy);
+            return check_launch("host_copy_kernel");
+        }
+        rows.signals = signals;
+        rows.copies = copy.count;
+        for (int i = 0; i < copy.count; i++)
+            rows.seg[i] = copy.seg[i];
+        launch_upload_rows(rows, blocks, st);
+        return check_launch("upload_rows_kernel");
+    }
 };
 
 // Small uploads, kSmall bytes in all at most, in one launch.
@@ -673,10 +804,7 @@ int upload_small(Ring *r, const Source *from, int count, hipStream_t st)
 constexpr size_t kFirstLaunch = (size_t)512 << 10;
 
 struct Pieces {
-    struct Piece {
-        const char *src;
-        char *dst;
-        size_t bytes;
+    struct Piece : Source {
         std::atomic<int> left{0};
         bool last_of_launch;
         size_t skew() const { return reinterpret_cast<uintptr_t>(dst) & 15; }
@@ -700,18 +828,27 @@ struct Pieces {
                         take = kSlotBytes;
                     if (take > room)
                         take = room;
+                    if (from[s].unit)   // (a slot has room for a row)
+                        take = take < from[s].unit ? from[s].unit : take - take % from[s].unit;
                     if (pass) {
-                        Piece &p = piece[n];
+                        Source &p = piece[n];
+                        p = from[s];
                         p.src = static_cast<const char *>(from[s].src) + at;
-                        p.dst = static_cast<char *>(from[s].dst) + at;
                         p.bytes = take;
+                        if (p.unit) {
+                            p.q += at / sizeof(float);
+                            p.scale += at / p.unit;
+                        } else {
+                            p.dst = static_cast<char *>(from[s].dst) + at;
+                        }
                     }
                     at += take;
                     ahead -= take;
-                    room -= take;
+                    room -= take < room ? take : room;
                     n++;
                     in_launch++;
-                    const bool end = room == 0 || in_launch == kMaxSegments || ahead == 0;
+                    const size_t unit = at < from[s].bytes ? from[s].unit : 0;   // of what comes next
+                    const bool end = room < (unit ? unit : 1) || in_launch == kMaxSegments || ahead == 0;
                     if (pass)
                         piece[n - 1].last_of_launch = end;
                     if (end) {
@@ -755,7 +892,7 @@ int send_pieces(Ring *r, Pieces &c, hipStream_t st, Launch launch)
                     break;
             }
             Pieces::Piece &p = c.piece[pushed];
-            crew.push(r->at(slot) + p.skew(), p.src, p.bytes, p.left);
+            crew.push(r->at(slot) + p.skew(), static_cast<const char *>(p.src), p.bytes, p.left);
             pushed++;
         }
         for (int i = issued; i < end && rc == VTL_HIP_OK; i++)
@@ -778,17 +915,15 @@ int upload_large(Ring *r, const Source *from, int count, hipStream_t st)
 {
     Pieces c(from, count);
     return send_pieces(r, c, st, [&](int first, int n, int slot, bool last) {
-        CopyArgs g = {};
+        Load load;
         size_t bytes = 0;
         for (int i = 0; i < n; i++) {
             const Pieces::Piece &p = c.piece[first + i];
-            g.seg[g.count++] = make_segment(p.dst, r->at((slot + i) % kSlots) + p.skew(), p.bytes);
+            load.add(p, r->at((slot + i) % kSlots) + p.skew());
             bytes += p.bytes;
         }
         const unsigned blocks = copy_blocks(bytes < kSmall ? bytes : kSmall - 1);
-        g.signals = r->signals_for(slot, blocks, last, false);
-        hipLaunchKernelGGL(host_copy_kernel, dim3(blocks), dim3(512), 0, st, g);
-        const int rc = check_launch("host_copy_kernel");
+        const int rc = load.launch(blocks, r->signals_for(slot, blocks, last, false), st);
         if (rc == VTL_HIP_OK)
             r->launched(slot, n, blocks, last);
         return rc;
@@ -920,6 +1055,32 @@ try {
     } else {
         status = upload_large(r, from, 2, current_stream());
     }
+    return true;
+} catch (const std::exception &) {
+    status = VTL_HIP_ERR_OUT_OF_MEMORY;
+    return true;
+}
+
+// Rows over the link as codes, and (extra_bytes of them) something copied with them; false: to be made in two steps.
+bool upload_rows(const float *src, int64_t rows, int64_t cols, int8_t *q, float *scale, void *extra_dst, const void *extra_src,
+                 size_t extra_bytes, int &status)
+try {
+    hipStream_t st = current_stream();
+    const bool one_stream = single_stream();
+    if (rows < 1 || rows > 0x7fffffff || cols < kRowsLeastCols || cols > kRowsMostCols || cols % 4 ||
+        (size_t)rows * (size_t)cols * sizeof(float) < kRowsFrom || (reinterpret_cast<uintptr_t>(q) & 3) || (!one_stream && stream_is_capturing(st)))
+        return false;
+    const OwnerDevice owner(q, extra_bytes ? extra_dst : nullptr);
+    Ring *r = owner.kernels() && owner.holds(scale) ? ring_of_current_device() : nullptr;
+    if (!r)
+        return false;
+    const size_t unit = (size_t)cols * sizeof(float);
+    const Source from[2] = {{nullptr, src, (size_t)rows * unit, q, scale, unit}, {extra_dst, extra_src, extra_bytes}};
+    const int count = extra_bytes ? 2 : 1;
+    std::lock_guard<std::mutex> hold(r->lock);
+    status = upload_large(r, from, count, st);
+    if (status == VTL_HIP_OK && !one_stream && hipStreamSynchronize(st) != hipSuccess)   // the ring's slots are shared by all streams
+        status = record_hip_error(hipErrorUnknown, "upload_rows_kernel");
     return true;
 } catch (const std::exception &) {
     status = VTL_HIP_ERR_OUT_OF_MEMORY;

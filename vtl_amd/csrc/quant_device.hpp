@@ -35,6 +35,16 @@ __device__ __forceinline__ float wave_max(float v)
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
 }
 
+// Workgroup barrier that orders LDS traffic only: unlike __syncthreads() it does
+// not wait for outstanding global loads, so direct-to-LDS weight loads issued
+// earlier stay in flight across it.
+__device__ __forceinline__ void lds_barrier()
+{
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // Max over each group of SEG = 16, 32 or 64 consecutive lanes (a DPP row, two, or the wave),
 // returned to every lane of the group.
 template <int SEG>

@@ -111,6 +111,10 @@ def _enqueue_upload(t: np.ndarray, params: HipParams | None) -> HipTensor:
     return dev
 
 
+# Weights of this many bytes and more are quantized as they come over the link, and the bias comes with them.
+_QUANTIZED_FROM = 32 << 20
+
+
 class QuantizedWeights:
     """Device-resident int8 weights of one Linear layer, derived from the f32
     parameter.  `source` / `bias_source` are the host tensors the device copies
@@ -145,17 +149,30 @@ class QuantizedWeights:
                 capi.Watch(t.ctypes.data, t.size, t.itemsize, h)
                 for t, h in zip(parts, (self.fingerprint, self.bias_fingerprint))])
         self.out_features, self.in_features = weights.shape
-        w_dev = _enqueue_upload(np.asarray(weights, np.float32), params)
-        try:
-            self.w_q, self.sw = w_dev.quantize_i8(0 if mode == PER_CHANNEL else -1)
-        finally:
-            w_dev.release()
+        w = np.asarray(weights, np.float32)
+        b = None if bias is None else np.asarray(bias, np.float32).reshape(-1)
+        if b is not None and b.size != self.out_features:
+            raise ValueError(f"bias has {b.size} entries, expected {self.out_features}")
         self.bias = None
-        if bias is not None:
-            b = np.asarray(bias, np.float32).reshape(-1)
-            if b.size != self.out_features:
-                raise ValueError(f"bias has {b.size} entries, expected {self.out_features}")
-            self.bias = _enqueue_upload(b, params)
+        if mode == PER_CHANNEL and w.nbytes >= _QUANTIZED_FROM:
+            w = np.ascontiguousarray(w)
+            self.w_q = HipTensor.empty(w.shape, np.int8, params)
+            self.sw = HipTensor.empty([self.out_features], np.float32, params)
+            extra = (None, None, 0)
+            if b is not None:
+                b = np.ascontiguousarray(b)
+                self.bias = HipTensor.empty(b.shape, np.float32, params)
+                extra = (self.bias.ptr, b.ctypes.data, b.nbytes)
+            capi.call("vtl_hip_upload_quantized", w.ctypes.data, self.out_features, self.in_features, 1, self.w_q.ptr, self.sw.ptr,
+                      *extra)
+        else:
+            w_dev = _enqueue_upload(w, params)
+            try:
+                self.w_q, self.sw = w_dev.quantize_i8(0 if mode == PER_CHANNEL else -1)
+            finally:
+                w_dev.release()
+            if b is not None:
+                self.bias = _enqueue_upload(b, params)
         # Rows of codes that the fast kernels do not take as they are get a padded copy, made with
         # the codes instead of by every forward (8 tokens x 14336 x 4095: 39.7 -> 18.6 us).  Small ones don't: kernels
         # that take rows of any length are as fast there.
