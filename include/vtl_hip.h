@@ -88,6 +88,8 @@ int vtl_hip_device_info(char *name, size_t name_cap, int *compute_units, int *cl
 int vtl_hip_malloc(void **dptr, size_t bytes);
 /* vtl_hip_set_device and vtl_hip_malloc in one call; no bytes: nullptr. */
 int vtl_hip_malloc_on(int device_id, void **dptr, size_t bytes);
+/* The same with the memory as its result: null for no bytes, and for a failure (vtl_hip_malloc_on says which). */
+void *vtl_hip_alloc(int device_id, size_t bytes);
 int vtl_hip_free(void *dptr);
 int vtl_hip_trim(void);
 

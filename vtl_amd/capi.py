@@ -43,6 +43,7 @@ SIGNATURES = {
     "vtl_hip_device_info": (_ci, [C.c_char_p, _sz, C.POINTER(_ci), C.POINTER(_ci)]),
     "vtl_hip_malloc": (_ci, [_pp, _sz]),
     "vtl_hip_malloc_on": (_ci, [_ci, _pp, _sz]),
+    "vtl_hip_alloc": (_vp, [_ci, _sz]),
     "vtl_hip_free": (_ci, [_vp]),
     "vtl_hip_trim": (_ci, []),
     "vtl_hip_memcpy_h2d": (_ci, [_vp, _vp, _sz]),
@@ -144,6 +145,17 @@ def call(name: str, *args) -> None:
     st = fn(*args)
     if st != OK:
         failed(name, st)
+
+
+_alloc = None
+
+
+def alloc(device_id: int, nbytes: int):
+    """vtl_hip_alloc: an address, or None."""
+    global _alloc
+    if _alloc is None:
+        _alloc = lib().vtl_hip_alloc
+    return _alloc(device_id, nbytes)
 
 
 def failed(name: str, st: int) -> None:

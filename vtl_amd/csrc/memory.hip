@@ -188,6 +188,12 @@ int vtl_hip_malloc_on(int device_id, void **dptr, size_t bytes)
     return st != VTL_HIP_OK || bytes == 0 ? st : vtl_hip_malloc(dptr, bytes);
 }
 
+void *vtl_hip_alloc(int device_id, size_t bytes)
+{
+    void *dptr = nullptr;
+    return vtl_hip_malloc_on(device_id, &dptr, bytes) == VTL_HIP_OK ? dptr : nullptr;
+}
+
 int vtl_hip_free(void *dptr)
 try {
     if (!dptr)

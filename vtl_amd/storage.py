@@ -75,14 +75,19 @@ class HipStorage:
         """Uninitialised memory.  It may be a released storage's, which calls enqueued before still use: a
         stream that the library was never told of (vtl_hip_set_stream) waits for vtl_hip_sync before it writes there."""
         device_id = params.device_id if params is not None else 0
-        dt = _DTYPES.get(dtype) or np.dtype(dtype)
-        if dt.type not in _SUPPORTED:
-            raise TypeError(f"HipStorage: unsupported element type {dt}")
+        dt = _DTYPES.get(dtype)
+        if dt is None:
+            dt = np.dtype(dtype)
+            if dt.type not in _SUPPORTED:
+                raise TypeError(f"HipStorage: unsupported element type {dt}")
         count = int(count)
         nbytes = count * dt.itemsize
-        ptr = C.c_void_p()
-        capi.call("vtl_hip_malloc_on", device_id, C.byref(ptr), nbytes)
-        return HipStorage(ptr.value or 0, nbytes, count, dt, device_id)
+        ptr = capi.alloc(device_id, nbytes)    # an address in one call: small operations on tensors are made of such calls
+        if not ptr:
+            ptr = C.c_void_p()
+            capi.call("vtl_hip_malloc_on", device_id, C.byref(ptr), nbytes)
+            ptr = ptr.value or 0
+        return HipStorage(ptr, nbytes, count, dt, device_id)
 
     @staticmethod
     def from_cpu(arr: np.ndarray, params: HipParams | None = None) -> "HipStorage":
@@ -137,7 +142,7 @@ class HipStorage:
 
     def __del__(self):  # safety net; the reference relies on explicit release()
         try:
-            if getattr(self, "ptr", 0) and capi._lib is not None:
+            if self.ptr:
                 capi._lib.vtl_hip_free(self.ptr)
                 self.ptr = 0
         except Exception:

@@ -54,7 +54,13 @@ class HipTensor:
 
     @staticmethod
     def empty(shape, dtype, params: HipParams | None = None) -> "HipTensor":
-        return HipTensor(HipStorage.empty(math.prod(shape), dtype, params), shape)
+        t = object.__new__(HipTensor)
+        t.shape = shape = list(map(int, shape))
+        t.size = math.prod(shape)
+        t.data = HipStorage.empty(t.size, dtype, params)
+        t.memory = "row_major"
+        t._strides = None
+        return t
 
     def hip(self, params: HipParams | None = None) -> "HipTensor":
         return self
