@@ -459,6 +459,22 @@ def test_gradients_in_one_launch(hip, knobs, dt, m, n, k):
 
 
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("m,n,k", [(1, 1, 1), (1, 2, 3), (17, 33, 65), (64, 64, 64), (40, 700, 64), (16, 256, 256), (64, 300, 300), (64, 256, 512)])
+def test_small_gradients_from_the_host(hip, monkeypatch, dt, m, n, k):
+    """Either side of what goes up together, and sizes that the one launch does not take."""
+    monkeypatch.setenv("VTL_USE_HIP", "1")
+    monkeypatch.setenv("VTL_HIP_BACKWARD", "1")
+    rng = np.random.default_rng(m + n + k)
+    g, x, w = (rng.integers(-8, 9, s).astype(dt) for s in ((m, n), (m, k), (n, k)))   # (whole numbers: every sum exact)
+    for bias in (True, False):
+        for _ in range(3):
+            print("gradients from the host", dt.__name__, m, n, k, bias, flush=True)
+            dx, dw, db = linear_backward_hip_f32(g, x, w, bias)
+            assert np.array_equal(dx, g @ w) and np.array_equal(dw, g.T @ x)
+            assert np.array_equal(db.reshape(-1), g.sum(axis=0) if bias else np.zeros(n))
+
+
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
 def test_weight_gradient_over_the_weights(hip, knobs, dt):
     """dX is complete before dW is written: dW may take the place of W."""
     m, n, k = 64, 192, 160

@@ -76,6 +76,15 @@ private:
 // Two uploads as vtl_hip_upload makes them, which share their launches; false: to be made one by one.
 bool upload_two(void *dst0, const void *src0, size_t bytes0, void *dst1, const void *src1, size_t bytes1, int &status);
 
+// Up to four small uploads, kUploadTogether bytes in all, to one device in one launch; false: to be made one by one.
+constexpr size_t kUploadTogether = (size_t)640 << 10;
+struct HostUpload {
+    void *dst;
+    const void *src;
+    size_t bytes;   // not 0
+};
+bool upload_together(const HostUpload *uploads, int count, int &status);
+
 // Rows that are quantized as they arrive, one scale each, and extra bytes copied with them; false: to be uploaded and quantized.
 bool upload_rows(const float *src, int64_t rows, int64_t cols, int8_t *q, float *scale, void *extra_dst, const void *extra_src,
                  size_t extra_bytes, int &status);
@@ -250,6 +259,11 @@ int matmul_to(HostResult *result, const double *a, const double *b, double *c, i
 // dW = grad^T . x and, unless it is null, db = the column sums of grad.
 int weight_gradients_to(HostResult *result, const float *grad, const float *x, float *dw, float *db, int m, int n, int k);
 int weight_gradients_to(HostResult *result, const double *grad, const double *x, double *dw, double *db, int m, int n, int k);
+// Those, and dX = grad . W, in one launch, the call's last, whose results are `result`'s memory; false: launch by launch.
+bool gradients_in_one(HostResult *result, const float *grad, const float *x, const float *w, float *dx, float *dw, float *db, int m, int n,
+                      int k, int &status);
+bool gradients_in_one(HostResult *result, const double *grad, const double *x, const double *w, double *dx, double *dw, double *db, int m,
+                      int n, int k, int &status);
 
 // vtl_hip_linear_i8_f32 and vtl_hip_linear_i8_requant with the parameters of a layer, whose weights may have padded rows.
 // `result`: Y is its memory.

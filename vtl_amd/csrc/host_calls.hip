@@ -270,6 +270,25 @@ int linear_backward_host(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
     VTL_STEP(gw.take(result));
     VTL_STEP(gx.take(result));
     VTL_STEP(gb.take(result));
+    // Every operand in one upload and all gradients in one launch, where there is less to copy than two more launches take (us, in two
+    // and in one: 64 x 64 x 64 30.6 and 25.2, 256 x 64 x 64 36.0 and 28.6, 64 x 256 x 256 46.4 and 40.9, 64 x 256 x 400
+    // 56.7 and 53.8; f64 64 x 128 x 128 42.7 and 36.1, 16 x 256 x 256 53.9 and 51.5).
+    if (gw.direct && gx.direct && (!gb.out || gb.direct) && (mn + mk + nk) * sizeof(T) <= kUploadTogether) {
+        VTL_STEP(dev_grad.take(mn * sizeof(T)));
+        VTL_STEP(dev_x.take(mk * sizeof(T)));
+        VTL_STEP(dev_w.take(nk * sizeof(T)));
+        const HostUpload operands[3] = {{dev_grad.ptr, grad, mn * sizeof(T)}, {dev_x.ptr, x, mk * sizeof(T)}, {dev_w.ptr, w, nk * sizeof(T)}};
+        int status = VTL_HIP_OK;
+        if (upload_together(operands, 3, status)) {
+            VTL_STEP(status);
+            if (!gradients_in_one(&result, dev_grad.as<T>(), dev_x.as<T>(), dev_w.as<T>(), gx.out, gw.out, gb.out, m, n, k, status)) {
+                VTL_STEP(weight_gradients_to(nullptr, dev_grad.as<T>(), dev_x.as<T>(), gw.out, gb.out, m, n, k));
+                status = matmul_to(&result, dev_grad.as<T>(), dev_w.as<T>(), gx.out, m, k, n, 0);
+            }
+            VTL_STEP(status);
+            return result.finish();
+        }
+    }
     if (gw.out)
         VTL_STEP(upload_both(dev_grad, grad, mn, dev_x, x, mk));
     else

@@ -449,7 +449,6 @@ int copy_and_wait(CopyArgs &g, size_t bytes, Lane *lane, hipStream_t st)
 constexpr int kSlots = 8;
 constexpr size_t kSlotBytes = (size_t)4 << 20;
 constexpr size_t kSlotStride = kSlotBytes + 4096;
-constexpr size_t kTogether = (size_t)640 << 10; // up to here two uploads share a launch
 constexpr size_t kSmall = (size_t)1 << 20;      // up to here one host thread copies faster than others wake up
 
 struct Ring {
@@ -1046,7 +1045,7 @@ try {
     // One launch for both saves its 3 us while they are small; from there on the first is on the link while the host copies
     // the second, and what one host thread copies well needs no others (f32 products, together and in turn: 700 x 1024 x 200 129 and
     // 122 us, 512 x 512 x 300 87 and 83, 1024 x 1000 x 128 139 and 136; 1024 x 1001 x 64 115 and 117).
-    if (bytes0 + bytes1 <= kTogether) {
+    if (bytes0 + bytes1 <= kUploadTogether) {
         status = upload_small(r, from, 2, current_stream());
     } else if (bytes0 <= kSmall && bytes1 <= kSmall) {
         status = upload_small(r, from, 1, current_stream());
@@ -1055,6 +1054,28 @@ try {
     } else {
         status = upload_large(r, from, 2, current_stream());
     }
+    return true;
+} catch (const std::exception &) {
+    status = VTL_HIP_ERR_OUT_OF_MEMORY;
+    return true;
+}
+
+bool upload_together(const HostUpload *uploads, int count, int &status)
+try {
+    Source from[kMaxSegments];
+    size_t bytes = 0;
+    for (int i = 0; i < count; i++) {
+        from[i] = {uploads[i].dst, uploads[i].src, uploads[i].bytes};
+        bytes += uploads[i].bytes;
+    }
+    if (count > kMaxSegments || bytes > kUploadTogether || !single_stream())
+        return false;
+    const OwnerDevice owner(uploads[0].dst, uploads[count - 1].dst);
+    Ring *r = owner.kernels() ? ring_of_current_device() : nullptr;
+    if (!r)
+        return false;
+    std::lock_guard<std::mutex> hold(r->lock);
+    status = upload_small(r, from, count, current_stream());
     return true;
 } catch (const std::exception &) {
     status = VTL_HIP_ERR_OUT_OF_MEMORY;

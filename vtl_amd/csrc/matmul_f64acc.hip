@@ -1130,7 +1130,8 @@ bool backward_in_one(vtlhip::HostResult *result, const T *grad, const T *x, cons
     const Kind kind = sizeof(T) == 8 ? kF64 : kF32;
     constexpr unsigned shapes = 1u << kK4 | 1u << kWide;   // workgroups of four waves
     const Plan pw = choose_plan(kind, n, k, m, false, false, kLaunch, shapes);
-    const Plan px = dx ? choose_plan(kind, m, k, n, alone || n >= 2048, false, kLaunch, shapes) : Plan{kK4, 1, 1, 0.0};
+    const bool may_slice = !(result && dx) && (alone || n >= 2048);   // (sums of slices would come behind the call's last launch)
+    const Plan px = dx ? choose_plan(kind, m, k, n, may_slice, false, kLaunch, shapes) : Plan{kK4, 1, 1, 0.0};
     const auto tiles = [&](Shape s, int rows, int cols) {
         return (int64_t)((rows + 31) / 32) * ((cols + kTileN[kind][s] - 1) / kTileN[kind][s]);
     };
@@ -1174,8 +1175,10 @@ bool backward_in_one(vtlhip::HostResult *result, const T *grad, const T *x, cons
     g.dx_tiles = (int)(tiles_x > 0 ? tiles_x : 1);
     g.dx_blocks = (int)tiles_x * cut;
     const dim3 grid((unsigned)(g.dx_blocks + tiles_w + sums));
-    if (result && !dx)
+    if (result) {
         result->attach(g.dw.done, grid.x);
+        g.dx.done = g.dw.done;
+    }
     hipStream_t st = current_stream();
     if (px.shape == kK4 && pw.shape == kK4)
         hipLaunchKernelGGL((linear_backward_kernel<T, 2, 2>), grid, dim3(256), 0, st, g);
@@ -1234,6 +1237,18 @@ int matmul_to(HostResult *result, const float *a, const float *b, float *c, int 
 int matmul_to(HostResult *result, const double *a, const double *b, double *c, int m, int n, int k, int trans_a)
 {
     return matmul_impl<double>(a, b, c, nullptr, m, n, k, trans_a, 0, 0, result);
+}
+
+bool gradients_in_one(HostResult *result, const float *grad, const float *x, const float *w, float *dx, float *dw, float *db, int m, int n,
+                      int k, int &status)
+{
+    return backward_in_one<float>(result, grad, x, w, dx, dw, db, m, n, k, status);
+}
+
+bool gradients_in_one(HostResult *result, const double *grad, const double *x, const double *w, double *dx, double *dw, double *db, int m,
+                      int n, int k, int &status)
+{
+    return backward_in_one<double>(result, grad, x, w, dx, dw, db, m, n, k, status);
 }
 
 int weight_gradients_to(HostResult *result, const float *grad, const float *x, float *dw, float *db, int m, int n, int k)
