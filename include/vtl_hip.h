@@ -103,6 +103,8 @@ int vtl_hip_memcpy_d2h(void *dst_host, const void *src_device, size_t bytes);
  * used a stream of its own, vtl_hip_set_stream.)  Work on a non-blocking stream that was never named does
  * not: use vtl_hip_memcpy_h2d for what such a stream reads. */
 int vtl_hip_upload(void *dst_device, const void *src_host, size_t bytes);
+/* Two of them, in one launch while they are small. */
+int vtl_hip_upload_two(void *dst0, const void *src0, size_t bytes0, void *dst1, const void *src1, size_t bytes1);
 /* vtl_hip_upload of rows x cols f32 and vtl_hip_quantize_f32_i8 of them, with the f32 values in no memory of the
  * caller's (with a scale per row they are quantized as they arrive where that can be), and a vtl_hip_upload of
  * extra_bytes (0: none) with them. */

@@ -61,6 +61,7 @@ SIGNATURES = {
     "vtl_hip_event_destroy": (_ci, [_vp]),
     "vtl_hip_event_record": (_ci, [_vp]),
     "vtl_hip_event_elapsed_ms": (_ci, [_vp, _vp, C.POINTER(C.c_float)]),
+    "vtl_hip_upload_two": (_ci, [_vp, _vp, _sz, _vp, _vp, _sz]),
     "vtl_hip_upload_quantized": (_ci, [_vp, _i64, _i64, _ci, _vp, _vp, _vp, _vp, _sz]),
     "vtl_hip_absmax_f32": (_ci, [_vp, _i64, _i64, _ci, _vp]),
     "vtl_hip_quantize_f32_i8": (_ci, [_vp, _i64, _i64, _ci, _vp, _vp]),

@@ -334,6 +334,18 @@ int vtl_hip_forward_i8_host(const float *x_host, int rows, int cols, const vtl_h
     return forward_layers(x_host, rows, cols, layers, count, y_host);
 }
 
+int vtl_hip_upload_two(void *dst0, const void *src0, size_t bytes0, void *dst1, const void *src1, size_t bytes1)
+{
+    if ((bytes0 && (!dst0 || !src0)) || (bytes1 && (!dst1 || !src1)))
+        return VTL_HIP_ERR_INVALID_ARG;
+    int status = VTL_HIP_OK;
+    if (upload_two(dst0, src0, bytes0, dst1, src1, bytes1, status))
+        return status;
+    if (bytes0)
+        VTL_STEP(vtl_hip_upload(dst0, src0, bytes0));
+    return bytes1 ? vtl_hip_upload(dst1, src1, bytes1) : VTL_HIP_OK;
+}
+
 int vtl_hip_upload_quantized(const float *src_host, int64_t rows, int64_t cols, int per_row, int8_t *q, float *scale,
                              void *extra_device, const void *extra_host, size_t extra_bytes)
 {
@@ -346,13 +358,7 @@ int vtl_hip_upload_quantized(const float *src_host, int64_t rows, int64_t cols, 
     const size_t bytes = (size_t)rows * (size_t)cols * sizeof(float);
     Scratch x;
     VTL_STEP(x.take(bytes));
-    if (!upload_two(x.ptr, src_host, bytes, extra_device, extra_host, extra_bytes, status)) {
-        if (bytes)
-            VTL_STEP(vtl_hip_upload(x.ptr, src_host, bytes));
-        if (extra_bytes)
-            VTL_STEP(vtl_hip_upload(extra_device, extra_host, extra_bytes));
-    }
-    VTL_STEP(status);
+    VTL_STEP(vtl_hip_upload_two(x.ptr, src_host, bytes, extra_device, extra_host, extra_bytes));
     return vtl_hip_quantize_f32_i8(x.as<float>(), rows, cols, per_row, q, scale);
 }
 

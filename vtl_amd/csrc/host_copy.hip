@@ -449,6 +449,7 @@ int copy_and_wait(CopyArgs &g, size_t bytes, Lane *lane, hipStream_t st)
 constexpr int kSlots = 8;
 constexpr size_t kSlotBytes = (size_t)4 << 20;
 constexpr size_t kSlotStride = kSlotBytes + 4096;
+constexpr size_t kWithAnother = (size_t)64 << 10;
 constexpr size_t kSmall = (size_t)1 << 20;      // up to here one host thread copies faster than others wake up
 
 struct Ring {
@@ -1045,7 +1046,9 @@ try {
     // One launch for both saves its 3 us while they are small; from there on the first is on the link while the host copies
     // the second, and what one host thread copies well needs no others (f32 products, together and in turn: 700 x 1024 x 200 129 and
     // 122 us, 512 x 512 x 300 87 and 83, 1024 x 1000 x 128 139 and 136; 1024 x 1001 x 64 115 and 117).
-    if (bytes0 + bytes1 <= kUploadTogether) {
+    // With little of one there is nothing to overlap (a bias behind its weights).
+    const size_t all = bytes0 + bytes1, less = bytes0 < bytes1 ? bytes0 : bytes1;
+    if (all <= kUploadTogether || (all <= kSmall && less <= kWithAnother)) {
         status = upload_small(r, from, 2, current_stream());
     } else if (bytes0 <= kSmall && bytes1 <= kSmall) {
         status = upload_small(r, from, 1, current_stream());

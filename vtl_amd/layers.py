@@ -102,15 +102,6 @@ def content_fingerprint(t: np.ndarray) -> int:
     return h.value
 
 
-def _enqueue_upload(t: np.ndarray, params: HipParams | None) -> HipTensor:
-    """HipTensor.from_host without its wait, for what only the library's next calls use."""
-    row = np.ascontiguousarray(t)
-    dev = HipTensor.empty(row.shape, row.dtype, params)
-    if dev.data.size:
-        capi.call("vtl_hip_upload", dev.ptr, row.ctypes.data, dev.data.size)
-    return dev
-
-
 # Weights of this many bytes and more are quantized as they come over the link, and the bias comes with them.
 _QUANTIZED_FROM = 32 << 20
 
@@ -153,26 +144,25 @@ class QuantizedWeights:
         b = None if bias is None else np.asarray(bias, np.float32).reshape(-1)
         if b is not None and b.size != self.out_features:
             raise ValueError(f"bias has {b.size} entries, expected {self.out_features}")
-        self.bias = None
+        # enqueued, without a wait: only the library's next calls use them
+        w = np.ascontiguousarray(w)
+        self.bias, extra = None, (None, None, 0)
+        if b is not None:
+            b = np.ascontiguousarray(b)
+            self.bias = HipTensor.empty(b.shape, np.float32, params)
+            extra = (self.bias.ptr, b.ctypes.data, b.nbytes)
         if mode == PER_CHANNEL and w.nbytes >= _QUANTIZED_FROM:
-            w = np.ascontiguousarray(w)
             self.w_q = HipTensor.empty(w.shape, np.int8, params)
             self.sw = HipTensor.empty([self.out_features], np.float32, params)
-            extra = (None, None, 0)
-            if b is not None:
-                b = np.ascontiguousarray(b)
-                self.bias = HipTensor.empty(b.shape, np.float32, params)
-                extra = (self.bias.ptr, b.ctypes.data, b.nbytes)
             capi.call("vtl_hip_upload_quantized", w.ctypes.data, self.out_features, self.in_features, 1, self.w_q.ptr, self.sw.ptr,
                       *extra)
         else:
-            w_dev = _enqueue_upload(w, params)
+            w_dev = HipTensor.empty(w.shape, np.float32, params)
             try:
+                capi.call("vtl_hip_upload_two", w_dev.ptr, w.ctypes.data, w.nbytes, *extra)
                 self.w_q, self.sw = w_dev.quantize_i8(0 if mode == PER_CHANNEL else -1)
             finally:
                 w_dev.release()
-            if b is not None:
-                self.bias = _enqueue_upload(b, params)
         # Rows of codes that the fast kernels do not take as they are get a padded copy, made with
         # the codes instead of by every forward (8 tokens x 14336 x 4095: 39.7 -> 18.6 us).  Small ones don't: kernels
         # that take rows of any length are as fast there.
