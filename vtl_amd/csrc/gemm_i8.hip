@@ -2635,13 +2635,13 @@ int launch_rows_quantized(const GemmArgs &g)
     return gemv_rows_fused_quant_faster(g.M, g.N, g.K) ? launch_gemv_rows<true, true, ROWS>(g, current_stream()) : -1;
 }
 
-int launch_ragged_rows(const float *X, int x_cols, const int8_t *Wq, int row, const float *sw, const float *bias, float *Y,
-                       int M, int N, int relu, HostResult *result)
+int launch_ragged_rows(const float *X, int x_cols, const int8_t *Wq, int row, const float *sw, int sw_stride, const float *bias,
+                       float *Y, int M, int N, int relu, HostResult *result)
 {
     const bool whole_weights = row % 16 == 0 && aligned16(Wq);
     if ((row == x_cols && whole_weights && aligned16(X)) || tuning().no_fused_decode || !tuning().ragged)
         return -1;
-    GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, row, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
+    GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, row, 1, sw_stride, relu ? 1 : 0, 1, nullptr, X, 0};
     g.x_cols = x_cols;
     g.result = result;
     return whole_weights ? launch_rows_quantized<kPadded>(g) : launch_rows_quantized<kRagged>(g);
@@ -2670,7 +2670,8 @@ int linear_i8_f32(const int8_t *A, const float *sa, int sa_per_row, const int8_t
     return launch_gemm<true>(g, current_stream());
 }
 
-int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, const float *bias,
+// sw_stride 0: one scale for all of Wq.
+int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, int sw_stride, const float *bias,
                                 float *Y, int M, int N, int K, int relu, void *workspace,
                                 size_t workspace_bytes, HostResult *result)
 {
@@ -2690,16 +2691,16 @@ int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, const
         // a single token: quantized inside the matrix-vector kernel, one launch instead of two
         // (N = 14336, K = 4096: 9.5 us against 12.8 us).  The workspace stays unused.
         // VTL_HIP_NO_FUSED_DECODE forces the two-launch path (tests).
-        GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
+        GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, K, 1, sw_stride, relu ? 1 : 0, 1, nullptr, X, 0};
         g.result = result;
         return launch_gemv<true, true>(g, current_stream());
     }
-    const int fused = launch_ragged_rows(X, K, Wq, K, sw, bias, Y, M, N, relu, result);
+    const int fused = launch_ragged_rows(X, K, Wq, K, sw, sw_stride, bias, Y, M, N, relu, result);
     if (fused >= 0)
         return fused;
     if (gemv_rows_applies(X, Wq, M, N, K) && gemv_rows_fused_quant_faster(M, N, K) && !tuning().no_fused_decode) {
         // a few tokens and short rows: same, each workgroup quantizes the rows itself
-        GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
+        GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, K, 1, sw_stride, relu ? 1 : 0, 1, nullptr, X, 0};
         g.result = result;
         return launch_gemv_rows<true, true>(g, current_stream());
     }
@@ -2719,7 +2720,7 @@ int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, const
         // are counted and rely on no cache holding an older copy of those lines, which holds
         // when nothing else shares them: the buffer starts on a cache line (anything from
         // vtl_hip_malloc does) and its size is a whole number of them.
-        GemmArgs g{xq, Wq, Y, sx, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, X, 0};
+        GemmArgs g{xq, Wq, Y, sx, sw, bias, M, N, K, 1, sw_stride, relu ? 1 : 0, 1, nullptr, X, 0};
         g.stage_codes = xq;
         g.stage_scales = sx;
         g.result = result;
@@ -2731,7 +2732,7 @@ int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, const
     st = launch_quantize_rows(X, M, K, xq, sx, current_stream());
     if (st != VTL_HIP_OK)
         return st;
-    GemmArgs g{xq, Wq, Y, sx, sw, bias, M, N, K, 1, 1, relu ? 1 : 0, 1, nullptr, nullptr, 0};
+    GemmArgs g{xq, Wq, Y, sx, sw, bias, M, N, K, 1, sw_stride, relu ? 1 : 0, 1, nullptr, nullptr, 0};
     g.result = result;
     return launch_gemm<true>(g, current_stream());
 }
@@ -2756,11 +2757,11 @@ int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa
 int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu, void *workspace, size_t workspace_bytes,
               HostResult *result)
 {
-    if (l.kind != VTL_HIP_LAYER_LINEAR || !l.per_channel || !layer_row_fits(l))
+    if (l.kind != VTL_HIP_LAYER_LINEAR || (!l.per_channel && M != 1) || !layer_row_fits(l))
         return VTL_HIP_ERR_INVALID_ARG;
-    const int K = l.in_features;
+    const int K = l.in_features, sw_stride = l.per_channel ? 1 : 0;
     if (l.row_bytes == 0 || M <= 0 || l.out_features <= 0 || K <= 0)
-        return linear_f32_dynquant(X, l.wq, l.sw, l.bias, Y, M, l.out_features, K, relu, workspace, workspace_bytes,
+        return linear_f32_dynquant(X, l.wq, l.sw, sw_stride, l.bias, Y, M, l.out_features, K, relu, workspace, workspace_bytes,
                                    result);
     int st = check_gemm_args(X, l.wq, Y, M, l.out_features, K);
     if (st != VTL_HIP_OK)
@@ -2768,7 +2769,7 @@ int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu,
     if (!l.sw || (workspace && (workspace_bytes < vtl_hip_linear_f32_dynquant_workspace(M, K) ||
                                 (reinterpret_cast<uintptr_t>(workspace) & 15))))
         return VTL_HIP_ERR_INVALID_ARG;
-    const int fused = launch_ragged_rows(X, K, l.wq, l.row_bytes, l.sw, l.bias, Y, M, l.out_features, relu, result);
+    const int fused = launch_ragged_rows(X, K, l.wq, l.row_bytes, l.sw, sw_stride, l.bias, Y, M, l.out_features, relu, result);
     if (fused >= 0)
         return fused;
     if (!workspace) {
@@ -2783,7 +2784,7 @@ int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu,
     if (!rows)
         return vtlhip::workspace_status();
     if (vtlhip::launch_quantize_rows_padded(X, M, K, rows, l.row_bytes, sx, current_stream(), st))
-        return st != VTL_HIP_OK ? st : linear_i8_f32(rows, sx, 1, l.wq, l.sw, 1, l.bias, Y, M, l.out_features,
+        return st != VTL_HIP_OK ? st : linear_i8_f32(rows, sx, 1, l.wq, l.sw, sw_stride, l.bias, Y, M, l.out_features,
                                                      l.row_bytes, relu, result);
     st = launch_quantize_rows(X, M, K, xq, sx, current_stream());
     return st != VTL_HIP_OK ? st : layer_linear_i8_f32(l, xq, sx, Y, M, relu, result);
@@ -2818,7 +2819,7 @@ int vtl_hip_pad_rows_i8(const int8_t *src, int64_t rows, int cols, int8_t *dst)
 int vtl_hip_layer_f32(const vtl_hip_layer *layer, const float *X, float *Y, int M, int relu, void *workspace,
                       size_t workspace_bytes)
 {
-    return layer ? vtlhip::layer_f32(*layer, X, Y, M, relu, workspace, workspace_bytes) : VTL_HIP_ERR_INVALID_ARG;
+    return layer && layer->per_channel ? vtlhip::layer_f32(*layer, X, Y, M, relu, workspace, workspace_bytes) : VTL_HIP_ERR_INVALID_ARG;
 }
 
 int vtl_hip_gemm_i8_i32(const int8_t *A, const int8_t *Bt, int32_t *C, int M, int N, int K)
@@ -2931,7 +2932,7 @@ int vtl_hip_linear_f32_dynquant(const float *X, const int8_t *Wq, const float *s
                                 float *Y, int M, int N, int K, int relu, void *workspace,
                                 size_t workspace_bytes)
 {
-    return linear_f32_dynquant(X, Wq, sw, bias, Y, M, N, K, relu, workspace, workspace_bytes, nullptr);
+    return linear_f32_dynquant(X, Wq, sw, 1, bias, Y, M, N, K, relu, workspace, workspace_bytes, nullptr);
 }
 
 int vtl_hip_linear_f32_dynquant_noalloc(const float *X, const int8_t *Wq, const float *sw, const float *bias,

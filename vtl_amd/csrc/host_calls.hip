@@ -88,8 +88,14 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
     vtlhip::CallScratch own;
     // (32 KiB is what the kernels that quantize in every workgroup take at most; near it the eight XCDs' transfers
     // cost what an upload does)
+    // One row has one scale either way: a layer with one for all of its weights takes it as one with a scale per row does, in one
+    // launch instead of two (us, per tensor: 1 x 832 x 448 17.4 -> 16.1, 1 x 3000 x 513 21.2 -> 17.5, 1 x 11000 x 4001 29.0 -> 24.8).  Not where
+    // weight rows start at any byte: 1 x 576 x 238 18.3 and 19.1, 1 x 1003 x 130 18.2 and 19.0.
+    const auto by_row = [&](const vtl_hip_layer &l) {
+        return l.per_channel || (rows == 1 && (l.row_bytes || l.in_features % 16 == 0));
+    };
     const bool upload_first = rows <= 8 && in_bytes > ((size_t)20 << 10) && in_bytes <= ((size_t)32 << 10);
-    if (count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR && !(upload_first && layers[0].per_channel) &&
+    if (count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR && !(upload_first && by_row(layers[0])) &&
         input.stage(x_host, in_bytes)) {
         // The first launch takes the input over the link itself: 64 x 784, per tensor, 4 us less than behind an
         // upload.  Rows that are no whole vectors are read twice, which still is no slower (forward of 200 x 1001
@@ -98,7 +104,7 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
         // device memory for a row of up to 4096, 10 for 32 such rows (read once), where the upload takes 3 and 13 and a
         // launch of its own.
         x = static_cast<const float *>(input.data);
-        if (!layers[0].per_channel || rows > kFewRows) {
+        if (!by_row(layers[0]) || rows > kFewRows) {
             VTL_STEP(codes.take((size_t)rows * (size_t)cols));
             VTL_STEP(scales.take((layers[0].per_channel ? (size_t)rows : 1) * sizeof(float)));
             VTL_STEP(vtl_hip_quantize_f32_i8(x, rows, cols, layers[0].per_channel, codes.as<int8_t>(), scales.as<float>()));
@@ -125,7 +131,7 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
         // the next layer takes codes as well
         const bool feeds = l.per_channel && rows > kFewRows && i < count && layers[i].kind == VTL_HIP_LAYER_LINEAR &&
                            layers[i].per_channel;
-        if (x && l.per_channel && !feeds) {
+        if (x && by_row(l) && !feeds) {
             if (!last)
                 VTL_STEP(next.take((size_t)rows * (size_t)n * sizeof(float)));
             const size_t need = vtl_hip_linear_f32_dynquant_workspace(rows, cols);
