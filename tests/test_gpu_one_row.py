@@ -38,6 +38,26 @@ def test_one_row_per_tensor(hip, dims, bias):
         w.release()
 
 
+@pytest.mark.parametrize("k", [15, 16, 17, 31, 33, 100, 127, 238, 255, 257])
+@pytest.mark.parametrize("n", [1, 7, 65, 1003])
+def test_few_short_rows(hip, n, k):
+    """Rows that start at any byte, shorter than the kernels' pieces: quantized in the launch of the product."""
+    rng = np.random.default_rng(n + k)
+    w = QuantizedWeights(rng.standard_normal((n, k)).astype(np.float32), rng.standard_normal(n).astype(np.float32), PER_CHANNEL, frozen=True)
+    for m in (1, 2, 3, 4, 5, 8):
+        x = rng.standard_normal((m, k)).astype(np.float32)
+        print("short rows", m, n, k, flush=True)
+        xd = dev(x)
+        q, s = xd.quantize_i8(0)
+        y = linear_i8_hip(q, s, w.w_q, w.sw, w.bias)
+        want = y.cpu().copy()
+        for t in (xd, q, s, y):
+            t.release()
+        for _ in range(2):
+            assert np.array_equal(forward_host(x, [w.layer], 1, n).view(np.int32), want.view(np.int32))
+    w.release()
+
+
 def test_rows_of_a_layer_with_one_scale_stay_refused(hip):
     w = QuantizedWeights(np.ones((8, 16), np.float32), None, PER_TENSOR, frozen=True)
     x, y = dev(np.ones((1, 16), np.float32)), dev(np.zeros((1, 8), np.float32))

@@ -2474,9 +2474,9 @@ inline bool gemv_applies(const void *row, const void *w, int N, int K)
 }
 
 // The matrix-vector kernels' forms for other rows than whole ones.
-inline bool gemv_takes_ragged(int M, int N, int K, Rows rows = kRagged)
+inline bool gemv_takes_ragged(int M, int N, int K, Rows rows = kRagged, int least = 256)
 {
-    if (tuning().no_gemv || K < 256)
+    if (tuning().no_gemv || K < least)
         return false;
     return M == 1 ? K <= 14336 && N <= 64 * gemv_max_waves(K, rows)
                   : M >= 2 && M <= 8 && K <= (M <= 2 ? 11264 : (M <= 4 ? 8192 : 4096));
@@ -2626,9 +2626,9 @@ const int8_t *pad_activations(const int8_t *A, int M, int K, int row, int &statu
 // Up to eight f32 rows of x_cols elements against weights in rows of `row` codes (x_cols, or padded), in one launch
 // where the kernels for whole rows would not take them; -1: not taken.
 template <Rows ROWS>
-int launch_rows_quantized(const GemmArgs &g)
+int launch_rows_quantized(const GemmArgs &g, int shortest)
 {
-    if (!gemv_takes_ragged(g.M, g.N, g.K, ROWS))
+    if (!gemv_takes_ragged(g.M, g.N, g.K, ROWS, shortest))
         return -1;
     if (g.M == 1)
         return launch_gemv<true, true, ROWS>(g, current_stream());
@@ -2636,7 +2636,7 @@ int launch_rows_quantized(const GemmArgs &g)
 }
 
 int launch_ragged_rows(const float *X, int x_cols, const int8_t *Wq, int row, const float *sw, int sw_stride, const float *bias,
-                       float *Y, int M, int N, int relu, HostResult *result)
+                       float *Y, int M, int N, int relu, HostResult *result, int shortest)
 {
     const bool whole_weights = row % 16 == 0 && aligned16(Wq);
     if ((row == x_cols && whole_weights && aligned16(X)) || tuning().no_fused_decode || !tuning().ragged)
@@ -2644,7 +2644,7 @@ int launch_ragged_rows(const float *X, int x_cols, const int8_t *Wq, int row, co
     GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, row, 1, sw_stride, relu ? 1 : 0, 1, nullptr, X, 0};
     g.x_cols = x_cols;
     g.result = result;
-    return whole_weights ? launch_rows_quantized<kPadded>(g) : launch_rows_quantized<kRagged>(g);
+    return whole_weights ? launch_rows_quantized<kPadded>(g, shortest) : launch_rows_quantized<kRagged>(g, shortest);
 }
 
 bool layer_row_fits(const vtl_hip_layer &l)
@@ -2670,10 +2670,17 @@ int linear_i8_f32(const int8_t *A, const float *sa, int sa_per_row, const int8_t
     return launch_gemm<true>(g, current_stream());
 }
 
+// What the shortest rows are that the launch which quantizes them itself takes where they start at any element.  In device memory:
+// all (dynamic quantization 1, 4 and 8 x 600 x 254 12.4 -> 10.1 us).  Of a host call, whose rows may come over the link, into every
+// workgroup: one or two (1 x 576 x 238 19.5 -> 16.7, 2 x 1003 x 130 19.6 -> 17.0; 4 x 576 x 238 20.0 and 19.8, 8 x 576 x 238 20.9 and
+// 23.7), others from 256 on.
+constexpr int kShortestRow = 16;
+inline int shortest_host_row(int M) { return M <= 2 ? kShortestRow : 256; }
+
 // sw_stride 0: one scale for all of Wq.
 int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, int sw_stride, const float *bias,
                                 float *Y, int M, int N, int K, int relu, void *workspace,
-                                size_t workspace_bytes, HostResult *result)
+                                size_t workspace_bytes, HostResult *result, int shortest)
 {
     int st = check_gemm_args(X, Wq, Y, M, N, K);
     if (st != VTL_HIP_OK)
@@ -2695,7 +2702,7 @@ int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, int s
         g.result = result;
         return launch_gemv<true, true>(g, current_stream());
     }
-    const int fused = launch_ragged_rows(X, K, Wq, K, sw, sw_stride, bias, Y, M, N, relu, result);
+    const int fused = launch_ragged_rows(X, K, Wq, K, sw, sw_stride, bias, Y, M, N, relu, result, shortest);
     if (fused >= 0)
         return fused;
     if (gemv_rows_applies(X, Wq, M, N, K) && gemv_rows_fused_quant_faster(M, N, K) && !tuning().no_fused_decode) {
@@ -2762,14 +2769,15 @@ int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu,
     const int K = l.in_features, sw_stride = l.per_channel ? 1 : 0;
     if (l.row_bytes == 0 || M <= 0 || l.out_features <= 0 || K <= 0)
         return linear_f32_dynquant(X, l.wq, l.sw, sw_stride, l.bias, Y, M, l.out_features, K, relu, workspace, workspace_bytes,
-                                   result);
+                                   result, shortest_host_row(M));
     int st = check_gemm_args(X, l.wq, Y, M, l.out_features, K);
     if (st != VTL_HIP_OK)
         return st;
     if (!l.sw || (workspace && (workspace_bytes < vtl_hip_linear_f32_dynquant_workspace(M, K) ||
                                 (reinterpret_cast<uintptr_t>(workspace) & 15))))
         return VTL_HIP_ERR_INVALID_ARG;
-    const int fused = launch_ragged_rows(X, K, l.wq, l.row_bytes, l.sw, sw_stride, l.bias, Y, M, l.out_features, relu, result);
+    const int fused = launch_ragged_rows(X, K, l.wq, l.row_bytes, l.sw, sw_stride, l.bias, Y, M, l.out_features, relu, result,
+                                         shortest_host_row(M));
     if (fused >= 0)
         return fused;
     if (!workspace) {
@@ -2932,7 +2940,7 @@ int vtl_hip_linear_f32_dynquant(const float *X, const int8_t *Wq, const float *s
                                 float *Y, int M, int N, int K, int relu, void *workspace,
                                 size_t workspace_bytes)
 {
-    return linear_f32_dynquant(X, Wq, sw, 1, bias, Y, M, N, K, relu, workspace, workspace_bytes, nullptr);
+    return linear_f32_dynquant(X, Wq, sw, 1, bias, Y, M, N, K, relu, workspace, workspace_bytes, nullptr, kShortestRow);
 }
 
 int vtl_hip_linear_f32_dynquant_noalloc(const float *X, const int8_t *Wq, const float *sw, const float *bias,

@@ -89,11 +89,9 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
     // (32 KiB is what the kernels that quantize in every workgroup take at most; near it the eight XCDs' transfers
     // cost what an upload does)
     // One row has one scale either way: a layer with one for all of its weights takes it as one with a scale per row does, in one
-    // launch instead of two (us, per tensor: 1 x 832 x 448 17.4 -> 16.1, 1 x 3000 x 513 21.2 -> 17.5, 1 x 11000 x 4001 29.0 -> 24.8).  Not where
-    // weight rows start at any byte: 1 x 576 x 238 18.3 and 19.1, 1 x 1003 x 130 18.2 and 19.0.
-    const auto by_row = [&](const vtl_hip_layer &l) {
-        return l.per_channel || (rows == 1 && (l.row_bytes || l.in_features % 16 == 0));
-    };
+    // launch instead of two (us, per tensor: 1 x 832 x 448 17.4 -> 15.9, 1 x 3000 x 513 20.9 -> 17.3, 1 x 11000 x 4001 28.4 -> 24.6, 1 x
+    // 576 x 238 18.4 -> 16.9).
+    const auto by_row = [&](const vtl_hip_layer &l) { return l.per_channel || rows == 1; };
     const bool upload_first = rows <= 8 && in_bytes > ((size_t)20 << 10) && in_bytes <= ((size_t)32 << 10);
     if (count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR && !(upload_first && by_row(layers[0])) &&
         input.stage(x_host, in_bytes)) {
