@@ -18,7 +18,7 @@
  *     from vtl_hip_malloc (the owner is the V-side HipStorage, released
  *     explicitly as in storage/cuda_d_cuda.v:98-102); host memory is touched
  *     by the copies and by the calls on whole host tensors (..._host), all of
- *     which are done with it on return (and all but vtl_hip_upload with the
+ *     which are done with it on return (and all but the vtl_hip_uploads with the
  *     device's work too), and read by the content fingerprints;
  *   - compute entry points enqueue on the library's current stream (the null
  *     stream unless vtl_hip_set_stream was called) and return without
