@@ -276,6 +276,25 @@ print("done")
 """)
 
 
+def test_a_small_backward_on_a_stream_of_its_own_waits_for_no_other(fake_runtime):
+    """Once a stream has been named a release waits for the whole device: a backward from host to host releases nothing while it
+    still has something to launch."""
+    _run(fake_runtime, r"""
+runtime()
+host, dx, dw, db = [(C.c_float * 65536)() for _ in range(4)]
+capi.call("vtl_hip_set_stream", 4096)
+for name in ("f32", "f64"):
+    for m, n, k in ((16, 24, 40), (64, 64, 64), (600, 16, 16)):
+        for want_db in (db, None):
+            events()
+            capi.status("vtl_hip_linear_backward_host_" + name, host, host, host, dx, dw, want_db, m, n, k)    # no kernel runs here
+            log = [e[0] for e in events()]
+            last = max(i for i, e in enumerate(log) if e == "launch")
+            assert "device_sync" not in log[:last], (name, m, n, k, log)
+print("done")
+""")
+
+
 def test_a_transfer_that_waits_for_the_device_costs_no_host_time(fake_runtime):
     """A large upload whose staging memory is not free yet: neither the caller nor the threads that help
     with the copying spin until it is."""

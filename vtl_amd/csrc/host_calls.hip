@@ -277,7 +277,7 @@ int linear_backward_host(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
     // Every operand in one upload and all gradients in one launch, where there is less to copy than two more launches take (us, in two
     // and in one: 64 x 64 x 64 30.6 and 25.2, 256 x 64 x 64 36.0 and 28.6, 64 x 256 x 256 46.4 and 40.9, 64 x 256 x 400
     // 56.7 and 53.8; f64 64 x 128 x 128 42.7 and 36.1, 16 x 256 x 256 53.9 and 51.5).
-    if (gw.direct && gx.direct && (!gb.out || gb.direct) && (mn + mk + nk) * sizeof(T) <= kUploadTogether) {
+    if (single_stream() && gw.direct && gx.direct && (!gb.out || gb.direct) && (mn + mk + nk) * sizeof(T) <= kUploadTogether) {
         VTL_STEP(dev_grad.take(mn * sizeof(T)));
         VTL_STEP(dev_x.take(mk * sizeof(T)));
         VTL_STEP(dev_w.take(nk * sizeof(T)));
