@@ -295,6 +295,28 @@ print("done")
 """)
 
 
+def test_column_sums_within_their_input_come_behind_all_of_it(fake_runtime):
+    """Sums that are written into the tensor they are made from, from 128 rows on: by a launch behind the one that reads it, for other
+    workgroups still read what one has summed."""
+    _run(fake_runtime, r"""
+runtime()
+p = malloc_on(0, 8 << 20)
+def kernels(name, *args):
+    events()
+    assert capi.status(name, *args) == capi.OK
+    return [k for l in lines() if l[0] == "launch" for k in ("colsum_finalize", "13colsum_kernel", "colsum_short") if k in l[4]]
+for name, size in (("f32", 4), ("f64", 8)):
+    for rows, cols in ((128, 700), (300, 64), (512, 129)):
+        for out in (p + 5 * size, p + size * (rows * cols - 1), p + size * 3 * cols):
+            assert kernels("vtl_hip_colsum_" + name, p, rows, cols, out) == ["13colsum_kernel", "colsum_finalize"], (name, rows, cols, out - p)
+            x, w, dx, dw = (p + (i << 20) for i in range(2, 6))
+            got = kernels("vtl_hip_linear_backward_" + name, p, x, w, dx, dw, out, rows, cols, 16)
+            assert got == ["13colsum_kernel", "colsum_finalize"], (name, rows, cols, out - p)
+        assert kernels("vtl_hip_colsum_" + name, p, rows, cols, p + size * rows * cols) == ["colsum_short"]     # behind it
+print("done")
+""")
+
+
 def test_a_transfer_that_waits_for_the_device_costs_no_host_time(fake_runtime):
     """A large upload whose staging memory is not free yet: neither the caller nor the threads that help
     with the copying spin until it is."""

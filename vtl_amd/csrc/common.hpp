@@ -36,6 +36,13 @@ private:
     bool kernels_ = true;
 };
 
+// Whether memory of `a_bytes` from a and of `b_bytes` from b meet.
+inline bool meet(const void *a, size_t a_bytes, const void *b, size_t b_bytes)
+{
+    const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+    return a && b && pa < pb + b_bytes && pb < pa + a_bytes;
+}
+
 // Whether `st` is being captured into a graph (true also when that cannot be found out).
 bool stream_is_capturing(hipStream_t st);
 

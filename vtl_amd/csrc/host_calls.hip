@@ -195,12 +195,6 @@ int upload_both(Scratch &to0, const T *host0, size_t count0, Scratch &to1, const
 
 constexpr size_t kResultMost = (size_t)8 << 20;
 
-bool overlap(const void *a, size_t a_bytes, const void *b, size_t b_bytes)
-{
-    const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
-    return pa < pb + b_bytes && pb < pa + a_bytes;
-}
-
 // How many bytes a product writes over the link as it is computed.  Rows that do not end where lines do leave lines to two
 // workgroups, which the link takes apart: a copy behind the launch is faster unless there is little to write (us,
 // copied and written over the link: f32 700 x 1001 x 200 122 and 136, 1024 x 1001 x 64 117 and 128, x 320 184 and
@@ -269,8 +263,8 @@ int linear_backward_host(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
     HostResult result;
     vtlhip::CallScratch own;
     const size_t dw_bytes = nk * sizeof(T), db_bytes = (size_t)n * sizeof(T);
-    Gradient gw = {dw, dw_bytes, dev_dw, dx && overlap(dw, dw_bytes, w, dw_bytes)}, gx = {dx, mk * sizeof(T), dev_dx, false},
-             gb = {db, db_bytes, dev_db, dx && overlap(db, db_bytes, w, dw_bytes)};
+    Gradient gw = {dw, dw_bytes, dev_dw, dx && meet(dw, dw_bytes, w, dw_bytes)}, gx = {dx, mk * sizeof(T), dev_dx, false},
+             gb = {db, db_bytes, dev_db, dx && meet(db, db_bytes, w, dw_bytes)};
     VTL_STEP(gw.take(result));
     VTL_STEP(gx.take(result));
     VTL_STEP(gb.take(result));

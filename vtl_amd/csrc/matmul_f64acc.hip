@@ -1042,7 +1042,8 @@ int matmul_impl(const T *a, const T *b, T *c, const T *bias, int m, int n, int k
 
 // Up to this many rows one launch has the column sums, a workgroup all rows of its columns; beyond, the rows are split and a second
 // launch adds up (us, split and in one: f32 256 x 11008 6.5 and 3.4, 128 x 300 6.3 and 3.6, 512 x 4097 6.7 and 6.4, 1024 x 4097 10.2
-// and 11.1; f64 512 x 11008 11.4 and 7.9, 1024 x 4097 13.2 and 21.0).
+// and 11.1; f64 512 x 11008 11.4 and 7.9, 1024 x 4097 13.2 and 21.0).  Not where the sums lie within x: a workgroup would write over
+// columns that another still reads.
 constexpr int64_t kShortSums = 512;
 
 template <typename T>
@@ -1055,7 +1056,8 @@ int colsum_impl(const T *x, int64_t rows, int64_t cols, T *out)
     if (!out || (rows > 0 && !x))
         return VTL_HIP_ERR_INVALID_ARG;
     hipStream_t st = current_stream();
-    if (rows <= kShortSums && cols <= 0x7fffffff - kSumCols) {
+    const size_t out_bytes = (size_t)cols * sizeof(T);
+    if (rows <= kShortSums && cols <= 0x7fffffff - kSumCols && !vtlhip::meet(x, (size_t)rows * out_bytes, out, out_bytes)) {
         const ColumnSums<T> g = {x, (int)rows, (int)cols, out};
         hipLaunchKernelGGL((colsum_short_kernel<T>), dim3((unsigned)((cols + kSumCols - 1) / kSumCols)), dim3(256), 0, st, g);
         return check_launch("colsum_short_kernel");
@@ -1101,13 +1103,6 @@ int colsum_impl(const T *x, int64_t rows, int64_t cols, T *out)
     return check_launch("colsum_finalize_kernel");
 }
 
-// Whether memory of `a_bytes` from a and of `b_bytes` from b meet.
-bool meet(const void *a, size_t a_bytes, const void *b, size_t b_bytes)
-{
-    const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
-    return a && b && pa < pb + b_bytes && pb < pa + a_bytes;
-}
-
 // dW and what else is asked for (not null) in one launch; false: launch by launch.  `result`: dw and db are its memory, and this is
 // the call's last launch.
 template <typename T>
@@ -1124,7 +1119,7 @@ bool backward_in_one(vtlhip::HostResult *result, const T *grad, const T *x, cons
                                                              {dx, x_bytes}, {dw, w_bytes}, {db, b_bytes}};
     for (int i = 3; i < 6; i++)
         for (int j = 0; j < i; j++)
-            if (meet(all[i].at, all[i].bytes, all[j].at, all[j].bytes))
+            if (vtlhip::meet(all[i].at, all[i].bytes, all[j].at, all[j].bytes))
                 return false;
 
     const bool alone = vtlhip::single_stream();
