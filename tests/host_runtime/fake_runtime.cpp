@@ -69,6 +69,8 @@ hipError_t hipGetLastError() { return hipSuccess; }
 
 hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int) { *v = 256; return hipSuccess; }
 
+hipError_t hipFuncSetAttribute(const void *, hipFuncAttribute, int) { return hipSuccess; }
+
 hipError_t hipMalloc(void **p, size_t bytes)
 {
     note("malloc", nullptr, bytes);

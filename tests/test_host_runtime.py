@@ -317,6 +317,72 @@ print("done")
 """)
 
 
+_SHORT_ROWS = r"""
+import re
+runtime()
+p = malloc_on(0, 64 << 20)
+host = (C.c_float * (1 << 20))()
+def in_one(name, *args):
+    events()
+    assert capi.status(name, *args) == capi.OK, args
+    kernels = [l[4] for l in lines() if l[0] == "launch"]
+    return len(kernels) == 1 and "linear_gemv" in kernels[0]
+def dense(m, n, k):
+    return in_one("vtl_hip_linear_f32_dynquant", p, p, p, None, p, m, n, k, 0, None, 0)
+def padded(m, n, k):
+    return in_one("vtl_hip_layer_f32", C.byref(capi.Layer(0, 1, n, k, p, p, None, (k + 15) & ~15)), p, p, m, 0, None, 0)
+"""
+
+
+def test_where_short_rows_are_quantized(fake_runtime):
+    """A few rows of fewer than 256 codes that start anywhere: in the launch of the product where that is the faster form for this many
+    rows, weights and the memory they lie in."""
+    _run(fake_runtime, _SHORT_ROWS + r"""
+for m, n in ((1, 14336), (2, 16384), (3, 8192), (4, 8192), (5, 2048), (8, 2048), (8, 1)):
+    for k in (17, 100, 239):
+        assert dense(m, n, k) and padded(m, n, k), (m, n, k)
+for m, n in ((2, 16385), (3, 8193), (4, 16384), (5, 2049), (6, 14336), (8, 16384)):
+    for k in (17, 100):
+        assert not dense(m, n, k) and not padded(m, n, k), (m, n, k)
+# weights that a call in two launches pads: three
+for m, n, k, one in ((1, 100000, 100, 1), (2, 40000, 100, 1), (2, 25000, 200, 1), (4, 40000, 100, 1), (4, 60000, 200, 1), (4, 60000, 100, 0),
+                     (6, 17000, 200, 0)):
+    assert dense(m, n, k) == bool(one), (m, n, k)
+assert padded(1, 65536, 100) and not padded(1, 80000, 100)
+for k in (15, 16, 240):                                        # too short, or whole rows
+    assert not dense(8, 64, k), k
+# where the rows lie, not which entry point: the first layer reads them over the link, the second has them in device memory, the
+# last one's results go over the link
+def forward(rows, *dims):
+    layers = (capi.Layer * (len(dims) - 1))(*[capi.Layer(0, 1, n, k, p, p, None, 0) for k, n in zip(dims, dims[1:])])
+    events()
+    capi.status("vtl_hip_forward_i8_host", host, rows, dims[0], layers, len(dims) - 1, host)     # no kernel runs here
+    found = [re.search("linear_gemv|quantize", l[4]) for l in lines() if l[0] == "launch"]
+    return [f.group() for f in found if f]
+assert forward(2, 100, 200, 300, 64) == ["linear_gemv"] * 3
+assert forward(1, 100, 20000) == ["quantize"]
+assert forward(4, 100, 200, 250, 64) == ["quantize", "linear_gemv", "quantize"]
+print("done")
+""")
+
+
+def test_short_rows_are_not_refused_for_want_of_scratch(fake_runtime):
+    """Where a call that would take two launches may not allocate, the launch that needs no scratch serves."""
+    _run(fake_runtime, _SHORT_ROWS + r"""
+capi.call("vtl_hip_set_stream", 4096)
+runtime(capturing=True)
+for m, n, k in ((2, 20000, 100), (4, 9000, 239), (4, 60000, 100), (8, 8000, 239)):
+    assert dense(m, n, k), (m, n, k)
+for m, n, k in ((1, 80000, 100), (2, 20000, 100)):
+    assert padded(m, n, k), (m, n, k)
+# the caller's workspace, and none for padded weights
+events()
+assert capi.status("vtl_hip_linear_f32_dynquant", p, p, p, None, p, 4, 60000, 100, 0, p, 1 << 20) == capi.OK
+assert "linear_gemv" in lines()[-1][4]
+print("done")
+""")
+
+
 def test_a_transfer_that_waits_for_the_device_costs_no_host_time(fake_runtime):
     """A large upload whose staging memory is not free yet: neither the caller nor the threads that help
     with the copying spin until it is."""

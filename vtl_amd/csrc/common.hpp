@@ -276,9 +276,9 @@ bool gradients_in_one(HostResult *result, const double *grad, const double *x, c
 // `result`: Y is its memory.
 int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa, float *Y, int M, int relu,
                         HostResult *result = nullptr);
-// vtl_hip_layer_f32; of one row with one scale for the weights too.
+// vtl_hip_layer_f32; of one row with one scale for the weights too.  `x_on_host`: X is in pinned memory (HostInput).
 int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu, void *workspace, size_t workspace_bytes,
-              HostResult *result = nullptr);
+              HostResult *result = nullptr, bool x_on_host = false);
 int layer_linear_i8_requant(const vtl_hip_layer &l, const int8_t *A, const float *sa, int8_t *Yq, float *sy, int M,
                             int relu);
 

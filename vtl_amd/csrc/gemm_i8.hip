@@ -2509,6 +2509,28 @@ inline bool small_ragged_faster(int M, int N, int K)
     return (t32 <= 512 && K <= 512) || (t32 <= 1024 && K <= 128);
 }
 
+// Rows of fewer than 256 codes: quantized in the launch of the product, or in one before it.  Two launches take the host 7 us whatever there
+// is to do, three, where dense weights have to be padded (small_ragged_faster says no), 10 and more; in one, every workgroup quantizes
+// all rows and a wave's sums grow with them.  us a call among others, in one launch and in two or three, K = 100 (17 to 254 alike).  Dense: 1 x 14336 4.9 and
+// 7.1; 2 x 16000 6.3 and 6.9, x 25000 7.3 and 6.9; 3 and 4 x 8000 6.0 and 5.7 against 6.8, x 9000 7.2 and 6.8 against 6.8, x 14336 7.9 and 7.4
+// against 6.9; 5 and 8 x 2000 6.0 and 5.5 against 6.4, x 2500 7.8 and 7.1 against 6.9, x 14336 11.6 and 10.6 against 6.9.  Dense and padded by the call:
+// 2 x 40000 8.2 and 11.2, x 100000 x 30 13.5 and 13.1; 4 x 17000 x 200 7.6 and 10.8, x 40000 10.4 and 11.3, x 60000 12.6 and 12.5, x 100000 x 200 20.1 and 25.2, x 30 18.1
+// and 13.2; 6 x 17000 x 200 11.4 and 10.9.  Padded rows: 1 x 65536 6.8 and 7.8, from 8 MiB on, where weights are streamed, 1 x 80000 9.8 and 7.8; 2 x
+// 20000 5.6 and 7.8, x 65536 8.2 and 7.9; 3 and 4 x 8000 5.2 and 4.9 against 7.7; 8 x 2500 5.7 and 6.2, 5 x 5000 8.2 and 7.7.
+// Over the link, rows or results: 1 x 14336 17.7 and 19.3, x 40000 21.5 and 20.3; 2 x 6000 17.8 and 19.4, x 40000 27.6 and 23.3; 3 x 1003 18.1 and
+// 16.6, 8 x 600 21.9 and 17.4.
+constexpr int kShortestRow = 16;
+inline bool short_rows_fused_faster(int M, int N, int K, Rows rows, bool over_link)
+{
+    if (over_link)
+        return M <= 2 && N <= 16384;
+    if (rows == kRagged && (M == 1 || (M <= 4 && !small_ragged_faster(M, N, K))))
+        return M <= 2 || N <= 40000 || K >= 128;
+    if (M == 1)
+        return (int64_t)N * K < (int64_t)8 << 20;
+    return N <= (M == 2 ? 16384 : (M <= 4 ? 8192 : 2048));
+}
+
 // Where one workgroup per 32x32 tile, fed straight from global memory, beats the tile kernels:
 // few tiles and a short K (nothing to stage), and up to a chip's worth of tiles with a long K,
 // which the tile kernels could only fill the chip with by cutting K (a second launch).
@@ -2624,11 +2646,14 @@ const int8_t *pad_activations(const int8_t *A, int M, int K, int row, int &statu
 }
 
 // Up to eight f32 rows of x_cols elements against weights in rows of `row` codes (x_cols, or padded), in one launch
-// where the kernels for whole rows would not take them; -1: not taken.
+// where the kernels for whole rows would not take them; -1: not taken.  kNoScratch: short rows that go another way while there is
+// memory for it.
+enum RowsIn { kDevice, kOverLink, kNoScratch };
 template <Rows ROWS>
-int launch_rows_quantized(const GemmArgs &g, int shortest)
+int launch_rows_quantized(const GemmArgs &g, RowsIn in)
 {
-    if (!gemv_takes_ragged(g.M, g.N, g.K, ROWS, shortest))
+    if (!gemv_takes_ragged(g.M, g.N, g.K, ROWS, kShortestRow) ||
+        (g.K < 256 && in != kNoScratch && !short_rows_fused_faster(g.M, g.N, g.K, ROWS, in == kOverLink)))
         return -1;
     if (g.M == 1)
         return launch_gemv<true, true, ROWS>(g, current_stream());
@@ -2636,7 +2661,7 @@ int launch_rows_quantized(const GemmArgs &g, int shortest)
 }
 
 int launch_ragged_rows(const float *X, int x_cols, const int8_t *Wq, int row, const float *sw, int sw_stride, const float *bias,
-                       float *Y, int M, int N, int relu, HostResult *result, int shortest)
+                       float *Y, int M, int N, int relu, HostResult *result, RowsIn in)
 {
     const bool whole_weights = row % 16 == 0 && aligned16(Wq);
     if ((row == x_cols && whole_weights && aligned16(X)) || tuning().no_fused_decode || !tuning().ragged)
@@ -2644,7 +2669,7 @@ int launch_ragged_rows(const float *X, int x_cols, const int8_t *Wq, int row, co
     GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, row, 1, sw_stride, relu ? 1 : 0, 1, nullptr, X, 0};
     g.x_cols = x_cols;
     g.result = result;
-    return whole_weights ? launch_rows_quantized<kPadded>(g, shortest) : launch_rows_quantized<kRagged>(g, shortest);
+    return whole_weights ? launch_rows_quantized<kPadded>(g, in) : launch_rows_quantized<kRagged>(g, in);
 }
 
 bool layer_row_fits(const vtl_hip_layer &l)
@@ -2670,17 +2695,10 @@ int linear_i8_f32(const int8_t *A, const float *sa, int sa_per_row, const int8_t
     return launch_gemm<true>(g, current_stream());
 }
 
-// What the shortest rows are that the launch which quantizes them itself takes where they start at any element.  In device memory:
-// all (dynamic quantization 1, 4 and 8 x 600 x 254 12.4 -> 10.1 us).  Of a host call, whose rows may come over the link, into every
-// workgroup: one or two (1 x 576 x 238 19.5 -> 16.7, 2 x 1003 x 130 19.6 -> 17.0; 4 x 576 x 238 20.0 and 19.8, 8 x 576 x 238 20.9 and
-// 23.7), others from 256 on.
-constexpr int kShortestRow = 16;
-inline int shortest_host_row(int M) { return M <= 2 ? kShortestRow : 256; }
-
 // sw_stride 0: one scale for all of Wq.
 int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, int sw_stride, const float *bias,
                                 float *Y, int M, int N, int K, int relu, void *workspace,
-                                size_t workspace_bytes, HostResult *result, int shortest)
+                                size_t workspace_bytes, HostResult *result, bool x_on_host)
 {
     int st = check_gemm_args(X, Wq, Y, M, N, K);
     if (st != VTL_HIP_OK)
@@ -2702,9 +2720,14 @@ int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, int s
         g.result = result;
         return launch_gemv<true, true>(g, current_stream());
     }
-    const int fused = launch_ragged_rows(X, K, Wq, K, sw, sw_stride, bias, Y, M, N, relu, result, shortest);
+    const auto ragged_rows = [&](RowsIn in) { return launch_ragged_rows(X, K, Wq, K, sw, sw_stride, bias, Y, M, N, relu, result, in); };
+    const int fused = ragged_rows(x_on_host || result ? kOverLink : kDevice);
     if (fused >= 0)
         return fused;
+    const auto no_scratch = [&](int status) {
+        const int alone = ragged_rows(kNoScratch);
+        return alone >= 0 ? alone : status;
+    };
     if (gemv_rows_applies(X, Wq, M, N, K) && gemv_rows_fused_quant_faster(M, N, K) && !tuning().no_fused_decode) {
         // a few tokens and short rows: same, each workgroup quantizes the rows itself
         GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, K, 1, sw_stride, relu ? 1 : 0, 1, nullptr, X, 0};
@@ -2716,7 +2739,7 @@ int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, int s
     if (!workspace) {   // no caller scratch: stage in the library's own buffer
         workspace = vtlhip::library_workspace(vtl_hip_linear_f32_dynquant_workspace(M, K), 1);
         if (!workspace)
-            return vtlhip::workspace_status();
+            return no_scratch(vtlhip::workspace_status());
     }
     int8_t *xq = reinterpret_cast<int8_t *>(workspace);
     const size_t codes = (((size_t)M * (size_t)K) + 255) & ~(size_t)255;
@@ -2741,7 +2764,8 @@ int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, int s
         return st;
     GemmArgs g{xq, Wq, Y, sx, sw, bias, M, N, K, 1, sw_stride, relu ? 1 : 0, 1, nullptr, nullptr, 0};
     g.result = result;
-    return launch_gemm<true>(g, current_stream());
+    st = launch_gemm<true>(g, current_stream());
+    return st == VTL_HIP_ERR_OUT_OF_MEMORY || st == VTL_HIP_ERR_UNSUPPORTED ? no_scratch(st) : st;
 }
 
 }  // namespace
@@ -2762,35 +2786,41 @@ int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa
 }
 
 int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu, void *workspace, size_t workspace_bytes,
-              HostResult *result)
+              HostResult *result, bool x_on_host)
 {
     if (l.kind != VTL_HIP_LAYER_LINEAR || (!l.per_channel && M != 1) || !layer_row_fits(l))
         return VTL_HIP_ERR_INVALID_ARG;
     const int K = l.in_features, sw_stride = l.per_channel ? 1 : 0;
     if (l.row_bytes == 0 || M <= 0 || l.out_features <= 0 || K <= 0)
         return linear_f32_dynquant(X, l.wq, l.sw, sw_stride, l.bias, Y, M, l.out_features, K, relu, workspace, workspace_bytes,
-                                   result, shortest_host_row(M));
+                                   result, x_on_host);
     int st = check_gemm_args(X, l.wq, Y, M, l.out_features, K);
     if (st != VTL_HIP_OK)
         return st;
     if (!l.sw || (workspace && (workspace_bytes < vtl_hip_linear_f32_dynquant_workspace(M, K) ||
                                 (reinterpret_cast<uintptr_t>(workspace) & 15))))
         return VTL_HIP_ERR_INVALID_ARG;
-    const int fused = launch_ragged_rows(X, K, l.wq, l.row_bytes, l.sw, sw_stride, l.bias, Y, M, l.out_features, relu, result,
-                                         shortest_host_row(M));
+    const auto ragged_rows = [&](RowsIn in) {
+        return launch_ragged_rows(X, K, l.wq, l.row_bytes, l.sw, sw_stride, l.bias, Y, M, l.out_features, relu, result, in);
+    };
+    const int fused = ragged_rows(x_on_host || result ? kOverLink : kDevice);
     if (fused >= 0)
         return fused;
+    const auto no_scratch = [&] {
+        const int status = vtlhip::workspace_status(), alone = ragged_rows(kNoScratch);
+        return alone >= 0 ? alone : status;
+    };
     if (!workspace) {
         workspace = vtlhip::library_workspace(vtl_hip_linear_f32_dynquant_workspace(M, K), 1);
         if (!workspace)
-            return vtlhip::workspace_status();
+            return no_scratch();
     }
     int8_t *xq = static_cast<int8_t *>(workspace);
     float *sx = reinterpret_cast<float *>(xq + ((((size_t)M * (size_t)K) + 255) & ~(size_t)255));
     // straight into padded rows, which need more room than the workspace has
     int8_t *rows = static_cast<int8_t *>(vtlhip::library_workspace((size_t)M * (size_t)l.row_bytes, 2));
     if (!rows)
-        return vtlhip::workspace_status();
+        return no_scratch();
     if (vtlhip::launch_quantize_rows_padded(X, M, K, rows, l.row_bytes, sx, current_stream(), st))
         return st != VTL_HIP_OK ? st : linear_i8_f32(rows, sx, 1, l.wq, l.sw, sw_stride, l.bias, Y, M, l.out_features,
                                                      l.row_bytes, relu, result);
@@ -2940,7 +2970,7 @@ int vtl_hip_linear_f32_dynquant(const float *X, const int8_t *Wq, const float *s
                                 float *Y, int M, int N, int K, int relu, void *workspace,
                                 size_t workspace_bytes)
 {
-    return linear_f32_dynquant(X, Wq, sw, 1, bias, Y, M, N, K, relu, workspace, workspace_bytes, nullptr, kShortestRow);
+    return linear_f32_dynquant(X, Wq, sw, 1, bias, Y, M, N, K, relu, workspace, workspace_bytes, nullptr, false);
 }
 
 int vtl_hip_linear_f32_dynquant_noalloc(const float *X, const int8_t *Wq, const float *sw, const float *bias,

@@ -135,7 +135,8 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
             const size_t need = vtl_hip_linear_f32_dynquant_workspace(rows, cols);
             Scratch work;
             VTL_STEP(work.take(need));
-            VTL_STEP(layer_f32(l, x, last ? y : next.as<float>(), rows, relu, work.ptr, need, last ? &result : nullptr));
+            VTL_STEP(layer_f32(l, x, last ? y : next.as<float>(), rows, relu, work.ptr, need, last ? &result : nullptr,
+                               input.data != nullptr));
             if (input.data) {
                 input.release();
                 if (result.attached())
