@@ -214,13 +214,13 @@ struct PartialTiles {
     double at[WK > 1 ? WM * WN * WK : 1][WK > 1 ? 4 * TM * TN : 1][64];
 };
 
-// One workgroup's part of a product: tile `block` and slice `slice` of `slices` of K.  `turn`: this workgroup's number in the launch.
+// One workgroup's part of a product: tile `block` and slice `slice` of K, of g.slice_steps steps.  `turn`: this workgroup's number in the launch.
 // (The arguments by value: by reference the compiler lays the branches of the end out otherwise, 512^3 f64 to the host 48.4 -> 48.7 us.)
 // The tiles of a workgroup are WM x WN wave tiles, K is cut over WK waves each.
 // Blocks are renumbered so that each of the 8 XCDs (own L2) works on a compact patch of tiles, eight
 // tile rows deep: with the plain order the rows that share a column panel of B run on different XCDs.
 template <typename T, int WM, int WN, int WK, int TM, int TN, bool TA, bool TB, bool CHECKED>
-__device__ __forceinline__ void direct_tile(const MatmulArgs g, int block, int slice, int slices, unsigned turn,
+__device__ __forceinline__ void direct_tile(const MatmulArgs g, int block, int slice, unsigned turn,
                                             PartialTiles<WM, WN, WK, TM, TN> &red)
 {
     constexpr int PA = TM / 2, PB = TN / 2;                // row and column pairs of a lane
@@ -238,9 +238,8 @@ __device__ __forceinline__ void direct_tile(const MatmulArgs g, int block, int s
     int of_tail = -1;
     if (TAIL && g.tail_slices > 1 && block >= g.whole_tiles) {
         of_tail = block - g.whole_tiles;
-        slices = g.tail_slices;
-        slice = of_tail % slices;
-        block = g.whole_tiles + of_tail / slices;
+        slice = of_tail % g.tail_slices;
+        block = g.whole_tiles + of_tail / g.tail_slices;
     }
     int tm, tn;
     tile_of_block(block, tiles_m, tiles_n, tm, tn);
@@ -248,7 +247,7 @@ __device__ __forceinline__ void direct_tile(const MatmulArgs g, int block, int s
     const int wk = wave % WK, tile = wave / WK;
     const int m0 = tm * BM + (tile / WN) * 16 * TM, n0 = tn * BN + (tile % WN) * 16 * TN;
     const int r16 = lane & 15, kq = lane >> 4;
-    // this workgroup's steps of K (all of them, or one of grid.y slices) and this wave's among them
+    // this workgroup's steps of K (all of them, or a slice) and this wave's among them
     const int steps = steps_of(g.K), per = TAIL && g.tail_slices > 1 && of_tail < 0 ? steps : g.slice_steps;
     const int first = slice * per, last = min(first + per, steps) - 1;
     const int count = first + wk > last ? 0 : (last - first - wk) / WK + 1;
@@ -533,8 +532,7 @@ template <typename T, int WM, int WN, int WK, int TM, int TN, bool TA, bool TB, 
 __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel(const MatmulArgs g)
 {
     __shared__ PartialTiles<WM, WN, WK, TM, TN> red;
-    direct_tile<T, WM, WN, WK, TM, TN, TA, TB, CHECKED>(g, (int)blockIdx.x, (int)blockIdx.y, (int)gridDim.y,
-                                                        blockIdx.x + gridDim.x * blockIdx.y, red);
+    direct_tile<T, WM, WN, WK, TM, TN, TA, TB, CHECKED>(g, (int)blockIdx.x, (int)blockIdx.y, blockIdx.x + gridDim.x * blockIdx.y, red);
 }
 
 // The sums of kSumCols columns by one workgroup of 256 threads: 16 phases of rows, added in order.  Rows start at any element.
@@ -627,12 +625,12 @@ __global__ __launch_bounds__(256) void linear_backward_kernel(const BackwardArgs
     } red;
     int block = (int)blockIdx.x;
     if (block < g.dx_blocks) {
-        direct_tile<T, 1, 1, 4, 2, TNX, false, false, false>(g.dx, block % g.dx_tiles, block / g.dx_tiles, 1, blockIdx.x, red.dx);
+        direct_tile<T, 1, 1, 4, 2, TNX, false, false, false>(g.dx, block % g.dx_tiles, block / g.dx_tiles, blockIdx.x, red.dx);
         return;
     }
     block -= g.dx_blocks;
     if (block < g.dw_blocks) {
-        direct_tile<T, 1, 1, 4, 2, TNW, true, false, false>(g.dw, block, 0, 1, blockIdx.x, red.dw);
+        direct_tile<T, 1, 1, 4, 2, TNW, true, false, false>(g.dw, block, 0, blockIdx.x, red.dw);
         return;
     }
     colsum_tile(g.db, block - g.dw_blocks, g.dw.done, red.db);
