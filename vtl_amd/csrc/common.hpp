@@ -157,7 +157,8 @@ __device__ __forceinline__ void store_result(T *p, T v, const DoneSignal &done)
 
 // 8 or 16 bytes of a result of less than 4 GiB, `off` bytes from its start and aligned as an element is: one store, through
 // the caches.  (By way of a builtin and not of inline assembly: the compiler puts the wait states in that gfx950 wants
-// between a wide store, or the MFMA before it, and the instructions that touch the same registers.)
+// between a wide store, or the MFMA before it, and the instructions that touch the same registers.  Behind a store of 16 bytes
+// it does so only where the scalar offset is a constant, as here; store_run in matmul_f64acc.hip, where it is a register, adds them.)
 typedef unsigned Words2 __attribute__((ext_vector_type(2)));
 typedef unsigned Words4 __attribute__((ext_vector_type(4)));
 constexpr int kThrough = 17;   // sc0 sc1
