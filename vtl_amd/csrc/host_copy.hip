@@ -1065,13 +1065,15 @@ try {
 
 bool upload_together(const HostUpload *uploads, int count, int &status)
 try {
+    if (count < 1 || count > kMaxSegments || !single_stream())
+        return false;
     Source from[kMaxSegments];
     size_t bytes = 0;
     for (int i = 0; i < count; i++) {
         from[i] = {uploads[i].dst, uploads[i].src, uploads[i].bytes};
         bytes += uploads[i].bytes;
     }
-    if (count > kMaxSegments || bytes > kUploadTogether || !single_stream())
+    if (bytes > kUploadTogether)
         return false;
     const OwnerDevice owner(uploads[0].dst, uploads[count - 1].dst);
     Ring *r = owner.kernels() ? ring_of_current_device() : nullptr;
