@@ -270,8 +270,12 @@ for per_channel in (0, 1):
     for rows, n, k, row in ((256, 1000, 72, 80), (256, 1000, 72, 0), (64, 1000, 1001, 1008), (64, 1024, 4096, 0)):
         layer = capi.Layer(0, per_channel, n, k, p, p, None, row)             # a linear
         assert not shared("vtl_hip_forward_i8_host", host, rows, k, C.byref(layer), 1, host), (per_channel, rows, n, k)
-for name in ("f32", "f64"):                                                   # column sums in splits
-    assert not shared("vtl_hip_linear_backward_host_" + name, host, host, host, host, host, host, 256, 64, 16), name
+for name in ("f32", "f64"):
+    backward = "vtl_hip_linear_backward_host_" + name
+    assert not shared(backward, host, host, host, host, host, host, 256, 64, 16), name    # gradients in one launch
+    assert not shared(backward, host, host, host, host, host, host, 2048, 64, 16), name   # column sums in splits
+    capi.status(backward, host, host, host, host, host, host, 2048, 64, 16)
+    assert any("colsum_finalize_kernel" in l[4] for l in lines() if l[0] == "launch"), name
 print("done")
 """)
 
@@ -313,6 +317,38 @@ for name, size in (("f32", 4), ("f64", 8)):
             got = kernels("vtl_hip_linear_backward_" + name, p, x, w, dx, dw, out, rows, cols, 16)
             assert got == ["13colsum_kernel", "colsum_finalize"], (name, rows, cols, out - p)
         assert kernels("vtl_hip_colsum_" + name, p, rows, cols, p + size * rows * cols) == ["colsum_short"]     # behind it
+print("done")
+""")
+
+
+def test_small_host_calls_take_the_launches_they_are_to(fake_runtime):
+    """While the process uses the null stream alone: a small backward is one upload and one launch, one row through a layer with one scale
+    is one launch that reads it over the link, and large weights are quantized as they arrive."""
+    _run(fake_runtime, r"""
+import re
+runtime()
+p = malloc_on(0, 64 << 20)
+host, dx, dw, db = [(C.c_float * (1 << 20))() for _ in range(4)]
+def kernels(name, *args):
+    events()
+    capi.status(name, *args)                                                  # no kernel runs here
+    found = [re.search("host_copy|upload_rows|linear_backward|f64acc_direct|linear_gemv|quantize", l[4]) for l in lines() if l[0] == "launch"]
+    names = [f.group() for f in found if f]
+    return [n for i, n in enumerate(names) if i == 0 or n != names[i - 1]]    # (a launch's gradients are noted one by one)
+one = ["host_copy", "linear_backward"]
+for name, fits, beyond in (("f32", (64, 345, 346), (64, 346, 346)), ("f64", (64, 229, 229), (64, 230, 230))):
+    backward = "vtl_hip_linear_backward_host_" + name
+    assert kernels(backward, host, host, host, dx, dw, db, 64, 64, 64) == one
+    assert kernels(backward, host, host, host, dx, dw, db, *fits) == one
+    got = kernels(backward, host, host, host, dx, dw, db, *beyond)
+    assert got[0] == "host_copy" and "host_copy" in got[2:] and got[-1] != "linear_backward", got
+layer = capi.Layer(0, 0, 64, 784, p, p, None, 0)                              # one scale
+assert kernels("vtl_hip_forward_i8_host", host, 1, 784, C.byref(layer), 1, host) == ["linear_gemv"]
+layer = capi.Layer(0, 0, 64, 6000, p, p, None, 0)                             # 24 KB: uploaded first
+assert kernels("vtl_hip_forward_i8_host", host, 1, 6000, C.byref(layer), 1, host) == ["host_copy", "linear_gemv"]
+rows = (C.c_float * (9 << 20))()
+got = [kernels("vtl_hip_upload_quantized", rows, n, 1024, 1, p, p, None, None, 0) for n in (8191, 8192)]
+assert [g[0] for g in got] == ["host_copy", "upload_rows"], got
 print("done")
 """)
 
