@@ -461,7 +461,8 @@ def test_gradients_in_one_launch(hip, knobs, dt, m, n, k):
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
 @pytest.mark.parametrize("m,n,k", [(1, 1, 1), (1, 2, 3), (17, 33, 65), (64, 64, 64), (40, 700, 64), (16, 256, 256), (64, 300, 300), (64, 256, 512)])
 def test_small_gradients_from_the_host(hip, monkeypatch, dt, m, n, k):
-    """Either side of what goes up together, and sizes that the one launch does not take."""
+    """Small layers, host to host.  (Here beside tests that name streams, so each operand goes up by itself; what goes up together is in
+    test_gpu_null_stream.py.)"""
     monkeypatch.setenv("VTL_USE_HIP", "1")
     monkeypatch.setenv("VTL_HIP_BACKWARD", "1")
     rng = np.random.default_rng(m + n + k)

@@ -238,6 +238,129 @@ def test_every_set_of_gradients(hip):
     assert done.returncode == 0 and done.stdout.rstrip().endswith("ok"), done.stdout[-3000:]
 
 
+SMALL_GRADIENTS = r"""
+import os
+os.environ["VTL_USE_HIP"] = os.environ["VTL_HIP_BACKWARD"] = "1"
+import threading
+import numpy as np
+from vtl_amd import capi, linear_backward_hip_f32
+# Operands of up to 640 KiB in all go up together and one launch has every gradient: either side of that, and sizes that the one
+# launch does not take (a row or a column of one).  Whole numbers: every sum is exact.
+SIZES = {"f4": [(64, 345, 346), (64, 346, 346), (513, 64, 64), (40, 700, 64)], "f8": [(64, 229, 229), (64, 230, 230), (513, 33, 47)]}
+def gradients(seed):
+    rng = np.random.default_rng(seed)
+    for dt in SIZES:
+        for m, n, k in [(1, 1, 1), (1, 2, 3), (5, 1, 7), (3, 9, 1), (17, 33, 65), (64, 64, 64), (16, 256, 256)] + SIZES[dt]:
+            for bias in (True, False):
+                for turn in range(2):
+                    g, x, w = (rng.integers(-8, 9, s).astype(dt) for s in ((m, n), (m, k), (n, k)))
+                    dx, dw, db = linear_backward_hip_f32(g, x, w, bias)
+                    assert np.array_equal(dx, g @ w) and np.array_equal(dw, g.T @ x), (dt, m, n, k)
+                    assert np.array_equal(db.reshape(-1), g.sum(axis=0) if bias else np.zeros(n)), (dt, m, n, k)
+capi.call("vtl_hip_set_device", 0)
+gradients(1)
+print("one thread", flush=True)
+bad = []
+def guarded(seed):
+    try:
+        gradients(seed)
+    except BaseException as e:
+        bad.append((seed, repr(e)))
+threads = [threading.Thread(target=guarded, args=(s,)) for s in (2, 3)]
+for t in threads:
+    t.start()
+for t in threads:
+    t.join()
+assert not bad, bad
+print("ok")
+"""
+
+
+def test_small_gradients_in_one_upload_and_one_launch(hip):
+    done = subprocess.run([sys.executable, "-c", SMALL_GRADIENTS], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                          text=True, timeout=110)
+    assert done.returncode == 0 and done.stdout.rstrip().endswith("ok"), done.stdout[-3000:]
+
+
+ONE_ROW = r"""
+import numpy as np
+import oracle
+from vtl_amd import PER_CHANNEL, PER_TENSOR, capi
+from vtl_amd.layers import QuantizedWeights, forward_host
+# One row through layers with one scale for their weights, and a few short rows, read over the link by the launch that quantizes
+# them or (20 to 32 KiB) uploaded: whole, ragged and padded rows, rows too long for the matrix-vector kernels, several layers
+capi.call("vtl_hip_set_device", 0)
+rng = np.random.default_rng(5)
+for dims, rows in [((16, 16), (1,)), ((1, 1), (1,)), ((17, 5), (1, 2, 8)), ((784, 256), (1,)), ((1001, 300), (1, 2)), ((1000, 1000), (1,)), ((1001, 1000), (1,)),
+                   ((6000, 70), (1,)), ((20000, 33), (1,)), ((20001, 40), (1,)), ((300, 500, 64), (1,)), ((64, 1001, 300, 7), (1, 3)),
+                   ((100, 2700), (1, 2, 3, 8)), ((238, 1003), (1, 2, 3, 8)), ((100, 16385), (1, 2)), ((100, 200, 250, 64), (1, 2, 4, 8))]:
+    for mode in (PER_TENSOR, PER_CHANNEL):
+        weights = [(rng.standard_normal((n, k)) / np.sqrt(k)).astype(np.float32) for k, n in zip(dims, dims[1:])]
+        qw = [QuantizedWeights(w, None, mode, frozen=True) for w in weights]
+        for m in rows if mode == PER_CHANNEL else (1,):
+            for turn in range(3):
+                x = rng.standard_normal((m, dims[0])).astype(np.float32)
+                y = x
+                for w in weights:
+                    wq, sw = oracle.quantize(w, mode == PER_CHANNEL)
+                    xq, sx = oracle.quantize(y, mode == PER_CHANNEL)
+                    y = oracle.epilogue(oracle.gemm_i8_i32(xq, wq, threads=4), sx, sw, None)
+                assert np.array_equal(forward_host(x, [w.layer for w in qw], len(qw), dims[-1]), y), (dims, mode, m, turn)
+        for w in qw:
+            w.release()
+    print(dims, flush=True)
+print("ok")
+"""
+
+
+def test_one_row_and_short_rows_over_the_link(hip):
+    done = subprocess.run([sys.executable, "-c", ONE_ROW], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                          text=True, timeout=110)
+    assert done.returncode == 0 and done.stdout.rstrip().endswith("ok"), done.stdout[-3000:]
+
+
+QUANTIZED_UPLOADS = r"""
+import numpy as np
+import oracle
+from vtl_amd import capi
+from vtl_amd.tensor import HipTensor
+# Rows that are quantized as they come over the link, without a wait: the caller's memory is its own again on return, and small
+# and large transfers come directly behind, through the same staging memory
+capi.call("vtl_hip_set_device", 0)
+rng = np.random.default_rng(9)
+def tensor(shape, dtype):
+    return HipTensor.empty(shape, dtype)
+for rows, cols, extra in ((8192, 1024, 0), (8200, 1028, 4100), (2049, 4096, 65537), (1031, 8188, 20), (4100, 2052, 3 << 20), (300, 1024, 64)):
+    held, waiting = [], []
+    for turn in range(2):
+        x = rng.standard_normal((rows, cols), dtype=np.float32)
+        x[rows // 2] = 0.0
+        more, small, large = (rng.integers(0, 256, n, dtype=np.uint8) for n in (extra, 5000, 21 << 20))
+        want = oracle.quantize(x, True, threads=8) + (more.copy(), small.copy(), large.copy())
+        q, s, e, a, b = tensor([rows, cols], np.int8), tensor([rows], np.float32), tensor([extra + 16], np.uint8), tensor([5000], np.uint8), tensor([21 << 20], np.uint8)
+        capi.call("vtl_hip_upload_quantized", x.ctypes.data, rows, cols, 1, q.ptr, s.ptr, e.ptr if extra else None,
+                  more.ctypes.data if extra else None, extra)
+        x[:] = np.nan
+        more[:] = 0
+        for t, src in ((a, small), (b, large))[:: 1 - 2 * turn]:
+            capi.call("vtl_hip_upload", t.ptr, src.ctypes.data, src.nbytes)
+            src[:] = 0
+        waiting.append(((q, s, e, a, b), want))
+    for tensors, want in waiting:
+        for t, w in zip(tensors, want):
+            assert np.array_equal(t.cpu().reshape(-1)[:w.size], w.reshape(-1)), (rows, cols, extra)
+            t.release()
+    print(rows, cols, extra, flush=True)
+print("ok")
+"""
+
+
+def test_uploads_behind_rows_quantized_on_their_way(hip):
+    done = subprocess.run([sys.executable, "-c", QUANTIZED_UPLOADS], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                          text=True, timeout=110)
+    assert done.returncode == 0 and done.stdout.rstrip().endswith("ok"), done.stdout[-3000:]
+
+
 def test_products_from_several_threads_on_the_null_stream(hip):
     done = subprocess.run([sys.executable, "-c", THREADS], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
                           text=True, timeout=100)

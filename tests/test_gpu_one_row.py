@@ -1,5 +1,6 @@
 """One row through layers with one scale for all weights, and a few short rows: in one launch a layer, the same bits as the same rows
-quantized by themselves and then multiplied, which the other tests hold against the CPU oracle."""
+quantized by themselves and then multiplied, which the other tests hold against the CPU oracle.  (Beside tests that name streams a host
+call's rows are uploaded; over the link: test_gpu_null_stream.py.)"""
 import numpy as np
 import pytest
 

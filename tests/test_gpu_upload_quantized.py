@@ -1,4 +1,5 @@
-"""Rows that are quantized as they come over the link: the same bits as an upload and the quantizer behind it."""
+"""Rows that are quantized as they come over the link: the same bits as an upload and the quantizer behind it.  (Beside tests that name
+streams each call waits for its end; without a wait, and with transfers behind it: test_gpu_null_stream.py.)"""
 import numpy as np
 import pytest
 
