@@ -2455,9 +2455,9 @@ inline bool gemv_rows_faster(int M, int N, int K, bool against_staged_launch = f
     return (int64_t)N * K <= ((int64_t)8 << 20);
 }
 
-// Quantizing the rows inside every workgroup of the few-token kernel costs about 15 instructions
+// Quantizing the rows inside every workgroup of the few-token kernel costs about 6 vector instructions
 // per element and workgroup; past 8192 elements (rows rounded up to 2, 4 or 8) a quantizer launch
-// of its own is cheaper.
+// of its own is cheaper.  (The limit is from when a code took about 15.)
 inline bool gemv_rows_fused_quant_faster(int M, int N, int K)
 {
     const int mr = M <= 2 ? 2 : (M <= 4 ? 4 : 8);

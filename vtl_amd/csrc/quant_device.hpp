@@ -145,8 +145,9 @@ __device__ __forceinline__ unsigned pack4(int a, int b, int c, int d)
 // Four codes at once: a quotient's rounding is what is left of it beside a number whose last place is one, the code its low
 // byte, and one test sees whether any of the four is too close to a tie, or no number (v_maximum3 keeps a NaN): then the
 // codes are made one by one.  6 vector instructions an element instead of 14, which the kernels that quantize a row in every workgroup, or hold
-// a tensor in registers until its scale is known, have nothing to hide behind (us: linear on f32 rows 1 x 4096 x 11008 10.97 -> 10.41,
-// 2 x 14336 x 4096 12.15 -> 11.10, 8 x 13.7 -> 13.35, 128 x 17.1 -> 16.6; 3001 x 4099 quantized with one scale and back 27.4 -> 26.4).
+// a tensor in registers until its scale is known, have nothing to hide behind (us, one at a time before: linear on f32 rows 1 x 4096 x 11008 8.3 -> 7.75,
+// 1 x 14336 x 4096 10.0 -> 8.8, 2 x 11.45 -> 10.2, 8 x 12.7 -> 11.5; 128 rows, in a launch of their own, level; 3001 x 4099 quantized with one scale and
+// back 27.15 -> 26.5, 16384 x 16384 per row and back 425 -> 422).
 // GIVEN: the scale is not that of the values' own maximum, so quotients may be out of range.
 template <bool GIVEN = false>
 __device__ __forceinline__ unsigned quant4(float4_t v, const QuantScale &p)
