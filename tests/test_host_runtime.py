@@ -353,6 +353,25 @@ print("done")
 """)
 
 
+def test_narrow_weight_gradients_have_a_launch_of_their_own(fake_runtime):
+    """Many rows of a few bytes, which a launch that writes over the link as it computes would send one by one."""
+    _run(fake_runtime, r"""
+runtime()
+host, dx, dw, db = [(C.c_float * (1 << 20))() for _ in range(4)]
+def in_one(name, m, n, k):
+    events()
+    capi.status("vtl_hip_linear_backward_host_" + name, host, host, host, dx, dw, db, m, n, k)    # no kernel runs here
+    return not any("f64acc_direct" in l[4] for l in lines() if l[0] == "launch")                 # that of dX
+for name, m, n, k in (("f32", 5, 48, 3), ("f32", 5, 128, 4), ("f32", 5, 400, 9), ("f32", 5, 1024, 8), ("f32", 3, 1024, 17), ("f32", 3, 2048, 33),
+                      ("f64", 5, 128, 2), ("f64", 5, 1024, 4), ("f64", 3, 400, 5), ("f64", 3, 1024, 7), ("f64", 3, 2048, 16)):
+    assert in_one(name, m, n, k), (name, m, n, k)
+for name, m, n, k in (("f32", 5, 49, 2), ("f32", 10, 778, 2), ("f32", 64, 1500, 5), ("f32", 5, 129, 6), ("f32", 5, 401, 10), ("f32", 3, 1025, 16),
+                      ("f32", 3, 2049, 40), ("f64", 10, 778, 3), ("f64", 3, 2000, 4), ("f64", 3, 401, 5), ("f64", 3, 2049, 16)):
+    assert not in_one(name, m, n, k), (name, m, n, k)
+print("done")
+""")
+
+
 _SHORT_ROWS = r"""
 import re
 runtime()

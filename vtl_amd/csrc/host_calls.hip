@@ -230,6 +230,22 @@ int matmul_host(const T *a, const T *b, T *c, int m, int n, int k)
     return vtl_hip_memcpy_d2h(c, dc.ptr, bytes);
 }
 
+// How many rows of dW the launch of all gradients may write over the link.  What a launch writes there as it computes goes as it is
+// stored, a row of a few bytes by itself; dW by a launch of its own is gathered to lines in the cache, and crosses while W comes up
+// (us, launch by launch and in one: f32 10 x 778 x 2 30 and 73, 64 x 1500 x 3 40 and 171, 5 x 100 x 3 24 and 31, 5 x 40 x 3 24 and 22; 10 x 1000 x 9
+// 30 and 42, 150 x 300 x 9 35 and 33; 10 x 1000 x 8 30 and 28, 3 x 2000 x 8 33 and 36, 3 x 5000 x 16 57 and 76; 3 x 2000 x 33 49 and 48, 3 x 4500 x 33 81
+// and 89; f64 10 x 778 x 2 29 and 43, 10 x 1000 x 4 30 and 27, 3 x 2000 x 4 32 and 36).
+int64_t rows_over_link(size_t row_bytes)
+{
+    if (row_bytes >= 128)
+        return 2048;
+    if (row_bytes >= 48 || row_bytes == 32)
+        return 1024;
+    if (row_bytes > 32)
+        return 400;
+    return row_bytes >= 16 && row_bytes % 8 == 0 ? 128 : 48;
+}
+
 template <typename T>
 int linear_backward_host(const T *grad, const T *x, const T *w, T *dx, T *dw, T *db, int m, int n, int k)
 {
@@ -280,7 +296,8 @@ int linear_backward_host(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
         int status = VTL_HIP_OK;
         if (upload_together(operands, 3, status)) {
             VTL_STEP(status);
-            if (!gradients_in_one(&result, dev_grad.as<T>(), dev_x.as<T>(), dev_w.as<T>(), gx.out, gw.out, gb.out, m, n, k, status)) {
+            if (n > rows_over_link(k * sizeof(T)) ||
+                !gradients_in_one(&result, dev_grad.as<T>(), dev_x.as<T>(), dev_w.as<T>(), gx.out, gw.out, gb.out, m, n, k, status)) {
                 VTL_STEP(weight_gradients_to(nullptr, dev_grad.as<T>(), dev_x.as<T>(), gw.out, gb.out, m, n, k));
                 status = matmul_to(&result, dev_grad.as<T>(), dev_w.as<T>(), gx.out, m, k, n, 0);
             }
