@@ -230,7 +230,7 @@ int matmul_host(const T *a, const T *b, T *c, int m, int n, int k)
     return vtl_hip_memcpy_d2h(c, dc.ptr, bytes);
 }
 
-// How many rows of dW the launch of all gradients may write over the link.  What a launch writes there as it computes goes as it is
+// Up to how many rows of dW one launch writes all gradients over the link.  What a launch writes there as it computes goes as it is
 // stored, a row of a few bytes by itself; dW by a launch of its own is gathered to lines in the cache, and crosses while W comes up
 // (us, launch by launch and in one: f32 10 x 778 x 2 30 and 73, 64 x 1500 x 3 40 and 171, 5 x 100 x 3 24 and 31, 5 x 40 x 3 24 and 22; 10 x 1000 x 9
 // 30 and 42, 150 x 300 x 9 35 and 33; 10 x 1000 x 8 30 and 28, 3 x 2000 x 8 33 and 36, 3 x 5000 x 16 57 and 76; 3 x 2000 x 33 49 and 48, 3 x 4500 x 33 81
@@ -288,7 +288,8 @@ int linear_backward_host(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
     // Every operand in one upload and all gradients in one launch, where there is less to copy than two more launches take (us, in two
     // and in one: 64 x 64 x 64 30.6 and 25.2, 256 x 64 x 64 36.0 and 28.6, 64 x 256 x 256 46.4 and 40.9, 64 x 256 x 400
     // 56.7 and 53.8; f64 64 x 128 x 128 42.7 and 36.1, 16 x 256 x 256 53.9 and 51.5).
-    if (single_stream() && gw.direct && gx.direct && (!gb.out || gb.direct) && (mn + mk + nk) * sizeof(T) <= kUploadTogether) {
+    if (single_stream() && gw.direct && gx.direct && (!gb.out || gb.direct) && (mn + mk + nk) * sizeof(T) <= kUploadTogether &&
+        n <= rows_over_link(k * sizeof(T))) {
         VTL_STEP(dev_grad.take(mn * sizeof(T)));
         VTL_STEP(dev_x.take(mk * sizeof(T)));
         VTL_STEP(dev_w.take(nk * sizeof(T)));
@@ -296,8 +297,7 @@ int linear_backward_host(const T *grad, const T *x, const T *w, T *dx, T *dw, T 
         int status = VTL_HIP_OK;
         if (upload_together(operands, 3, status)) {
             VTL_STEP(status);
-            if (n > rows_over_link(k * sizeof(T)) ||
-                !gradients_in_one(&result, dev_grad.as<T>(), dev_x.as<T>(), dev_w.as<T>(), gx.out, gw.out, gb.out, m, n, k, status)) {
+            if (!gradients_in_one(&result, dev_grad.as<T>(), dev_x.as<T>(), dev_w.as<T>(), gx.out, gw.out, gb.out, m, n, k, status)) {
                 VTL_STEP(weight_gradients_to(nullptr, dev_grad.as<T>(), dev_x.as<T>(), gw.out, gb.out, m, n, k));
                 status = matmul_to(&result, dev_grad.as<T>(), dev_w.as<T>(), gx.out, m, k, n, 0);
             }
