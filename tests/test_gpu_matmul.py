@@ -391,6 +391,20 @@ def test_column_sums(hip, dt, rows, cols):
     s.release()
 
 
+@pytest.mark.parametrize("cols", [1, 2, 3, 4, 5, 6, 7, 63, 64, 65, 66, 67, 68, 130])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_column_sums_of_few_rows(hip, guard_bands, dt, cols):
+    """Where the last columns' loads begin before them: whole numbers, so every sum is exact; a tensor that ends where its memory does."""
+    rng = np.random.default_rng(cols)
+    for rows in (1, 15, 16, 17, 48, 49, 63, 64, 65, 112, 512):
+        x = rng.integers(-1000, 1001, (rows, cols)).astype(dt)
+        xd = dev(x)
+        s = colsum_hip(xd)
+        assert np.array_equal(s.cpu().reshape(-1), x.sum(axis=0)), (rows, cols)
+        xd.release()
+        s.release()
+
+
 @pytest.mark.parametrize("dt", [np.float32, np.float64])
 def test_linear_backward_against_oracle(hip, dt):
     rng = np.random.default_rng(26)

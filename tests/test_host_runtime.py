@@ -321,6 +321,27 @@ print("done")
 """)
 
 
+def test_where_column_sums_take_one_launch(fake_runtime):
+    _run(fake_runtime, r"""
+runtime()
+p = malloc_on(0, 1 << 20)
+out = p + (1 << 36)                    # (no kernel runs here)
+def kernels(name, rows, cols, off=0):
+    events()
+    assert capi.status("vtl_hip_colsum_" + name, p + off, rows, cols, out) == capi.OK
+    return [k for l in lines() if l[0] == "launch" for k in ("colsum_finalize", "13colsum_kernel", "colsum_short") if k in l[4]]
+for name in ("f32", "f64"):
+    for rows, cols in ((0, 5), (1, 1), (512, 1), (512, 32768), (127, 32767)):
+        assert kernels(name, rows, cols) == ["colsum_short"], (name, rows, cols)
+    assert kernels(name, 127, 100003) == kernels(name, 256, 32771) == ["13colsum_kernel"]         # nothing to split
+    assert kernels(name, 513, 64) == ["13colsum_kernel", "colsum_finalize"], name
+assert kernels("f32", 320, 65536) == kernels("f32", 96, 65536) == ["colsum_short"]
+assert kernels("f64", 320, 65536) == ["13colsum_kernel", "colsum_finalize"] and kernels("f64", 96, 65536) == ["13colsum_kernel"]
+assert kernels("f32", 96, 65536, 4) == ["13colsum_kernel"]                    # rows that start anywhere
+print("done")
+""")
+
+
 def test_small_host_calls_take_the_launches_they_are_to(fake_runtime):
     """While the process uses the null stream alone: a small backward is one upload and one launch, one row through a layer with one scale
     is one launch that reads it over the link, and large weights are quantized as they arrive."""

@@ -553,9 +553,10 @@ __device__ __forceinline__ void colsum_tile(const ColumnSums<T> &g, int block, c
         T v[4];
     };
     const int group = threadIdx.x & 15, phase = threadIdx.x >> 4, c = block * kSumCols + 4 * group;
+    const int first = min(c, g.cols - 4);   // the last columns with some of those before them
     double acc[4] = {0.0, 0.0, 0.0, 0.0};
-    if (c + 4 <= g.cols) {
-        const T *at = g.x + c;
+    if (first >= 0 && c < g.cols) {
+        const T *at = g.x + first;
         int r = phase;
         for (; r + 48 < g.rows; r += 64) {   // four loads in flight
             Run v[4];
@@ -574,16 +575,18 @@ __device__ __forceinline__ void colsum_tile(const ColumnSums<T> &g, int block, c
             for (int j = 0; j < 4; ++j)
                 acc[j] += (double)v.v[j];
         }
-    } else {
+    } else if (c < g.cols) {   // fewer than four columns
         for (int r = phase; r < g.rows; r += 16)
 #pragma unroll
             for (int j = 0; j < 3; ++j)
-                if (c + j < g.cols)
-                    acc[j] += (double)g.x[(int64_t)r * g.cols + c + j];
+                if (j < g.cols)
+                    acc[j] += (double)g.x[(int64_t)r * g.cols + j];
     }
+    const int shift = first >= 0 ? c - first : 0;   // 0 but for the last columns
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-        red[phase][4 * group + j] = acc[j];
+        if (j >= shift)
+            red[phase][4 * group + j - shift] = acc[j];
     __syncthreads();
     const int mine = block * kSumCols + (int)threadIdx.x;
     if (threadIdx.x < kSumCols && mine < g.cols) {
@@ -1038,11 +1041,19 @@ int matmul_impl(const T *a, const T *b, T *c, const T *bias, int m, int n, int k
     return launch_direct<T>(g, kind, trans_a != 0, trans_b != 0, plan, alone, current_stream());
 }
 
-// Up to this many rows one launch has the column sums, a workgroup all rows of its columns; beyond, the rows are split and a second
-// launch adds up (us, split and in one: f32 256 x 11008 6.5 and 3.4, 128 x 300 6.3 and 3.6, 512 x 4097 6.7 and 6.4, 1024 x 4097 10.2
-// and 11.1; f64 512 x 11008 11.4 and 7.9, 1024 x 4097 13.2 and 21.0).  Not where the sums lie within x: a workgroup would write over
-// columns that another still reads.
-constexpr int64_t kShortSums = 512;
+// Where one launch has the column sums, a workgroup all rows of its columns; elsewhere the rows are split from 128 on and a second
+// launch adds up (us, split and in one: f32 256 x 11008 6.5 and 3.4, 128 x 300 6.3 and 3.6, 512 x 4097 6.7 and 4.4, 1024 x 4097 10.2
+// and 11.1; f64 512 x 11008 11.4 and 7.9, 512 x 32768 24.6 and 20.0, 1024 x 4097 13.2 and 21.0).  Of wider rows a wave reads four times
+// as much of one at a time in the split form, or, where they start anywhere, a word a lane: f64 127 x 65536 11.2 and 16.8, 96 x 65536 8.9
+// and 12.2, 256 x 65536 23.5 and 25.4, 192 x 100003 27.6 and 28.7, f32 127 x 100003 12.4 and 12.9; but f32 320 x 65536 17.1 and 13.8.
+constexpr int64_t kShortSums = 512, kShortSumsWidth = 32768;
+
+template <typename T>
+bool sums_in_one(const T *x, int64_t rows, int64_t cols)
+{
+    return rows <= kShortSums &&
+           (cols <= kShortSumsWidth || (sizeof(T) == 4 && cols % 4 == 0 && aligned16(x) && cols <= 0x7fffffff - kSumCols));
+}
 
 template <typename T>
 int colsum_impl(const T *x, int64_t rows, int64_t cols, T *out)
@@ -1055,7 +1066,8 @@ int colsum_impl(const T *x, int64_t rows, int64_t cols, T *out)
         return VTL_HIP_ERR_INVALID_ARG;
     hipStream_t st = current_stream();
     const size_t out_bytes = (size_t)cols * sizeof(T);
-    if (rows <= kShortSums && cols <= 0x7fffffff - kSumCols && !vtlhip::meet(x, (size_t)rows * out_bytes, out, out_bytes)) {
+    // (Not where the sums lie within x: a workgroup would write over columns that another still reads.)
+    if (sums_in_one(x, rows, cols) && !vtlhip::meet(x, (size_t)rows * out_bytes, out, out_bytes)) {
         const ColumnSums<T> g = {x, (int)rows, (int)cols, out};
         hipLaunchKernelGGL((colsum_short_kernel<T>), dim3((unsigned)((cols + kSumCols - 1) / kSumCols)), dim3(256), 0, st, g);
         return check_launch("colsum_short_kernel");
