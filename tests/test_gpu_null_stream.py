@@ -330,7 +330,7 @@ capi.call("vtl_hip_set_device", 0)
 rng = np.random.default_rng(9)
 def tensor(shape, dtype):
     return HipTensor.empty(shape, dtype)
-for rows, cols, extra in ((8192, 1024, 0), (8200, 1028, 4100), (2049, 4096, 65537), (1031, 8188, 20), (4100, 2052, 3 << 20), (300, 1024, 64)):
+for rows, cols, extra in ((8192, 1024, 0), (8200, 1028, 4100), (4096, 2048, 0), (4111, 2048, 4100), (2049, 4096, 65537), (1031, 8188, 20), (4100, 2052, 3 << 20), (300, 1024, 64)):
     held, waiting = [], []
     for turn in range(2):
         x = rng.standard_normal((rows, cols), dtype=np.float32)

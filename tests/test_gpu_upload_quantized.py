@@ -10,9 +10,9 @@ from vtl_amd.tensor import HipTensor
 pytestmark = pytest.mark.gpu
 
 
-# 32 MiB and more are quantized on the way: edges of a workgroup's registers, rows that do not divide the pieces a transfer is
+# 32 MiB and more in rows of 2048 and more are quantized on the way: edges of a workgroup's registers, rows that do not divide the pieces a transfer is
 # cut into (rows are not cut); less, longer, shorter and odd rows go in two steps
-@pytest.mark.parametrize("rows,cols", [(8192, 1024), (8191, 1024), (8200, 1028), (4096, 2048), (4100, 2052), (3000, 2800), (2049, 4096), (2100, 4100),
+@pytest.mark.parametrize("rows,cols", [(8192, 1024), (8191, 1024), (8200, 1028), (4096, 2048), (4095, 2048), (4200, 2044), (4100, 2052), (3000, 2800), (2049, 4096), (2100, 4100),
                                        (1024, 8192), (1031, 8188), (1030, 8196), (33000, 256), (8300, 1023), (300, 1024), (1, 4)])
 @pytest.mark.parametrize("extra", [0, 4096 + 20])
 def test_same_bits_as_upload_and_quantize(hip, rows, cols, extra):

@@ -173,9 +173,10 @@ struct RowsArgs {
 // a launch, when the last rows are there, is a microsecond longer than a copy's, so it is for transfers of many MiB a
 // launch (us, copy and quantizer behind it, and this: 11008 x 4096 3659 and 3614 of a forward, 4096 x 4096 1279 and
 // 1265; 512 x 4096 213 and 217, 1000 x 1000 120 and 122).  More workgroups take longer on the link (4096 x 4096 with 16 1270,
-// 32 1303, 64 1308).  Arithmetic as in quant.hip.
+// 32 1303, 64 1308).  Of rows of fewer than 2048 values too little is on its way at a time: 8192 x 1024 705 and 1000, 32768 x 1024 2525 and
+// 3760, 20000 x 1536 2305 and 2500, x 1800 2710 and 2790; 20000 x 2048 3040 and 3030.  Arithmetic as in quant.hip.
 constexpr size_t kRowsFrom = (size_t)32 << 20;
-constexpr int kRowsLeastCols = 1024, kRowsMostCols = 8192;
+constexpr int kRowsLeastCols = 2048, kRowsMostCols = 8192;
 
 template <int NV>
 __global__ __launch_bounds__(512) void upload_rows_kernel(const RowsArgs g)

@@ -102,7 +102,7 @@ def content_fingerprint(t: np.ndarray) -> int:
     return h.value
 
 
-# Weights of this many bytes and more go to the call that quantizes them as they come over the link where it can (rows of 1024 to
+# Weights of this many bytes and more go to the call that quantizes them as they come over the link where it can (rows of 2048 to
 # 8192 values), and takes the bias along.
 _QUANTIZED_FROM = 32 << 20
 
