@@ -365,8 +365,14 @@ for name, fits, beyond in (("f32", (64, 345, 346), (64, 346, 346)), ("f64", (64,
     assert got[0] == "host_copy" and "host_copy" in got[2:] and got[-1] != "linear_backward", got
 layer = capi.Layer(0, 0, 64, 784, p, p, None, 0)                              # one scale
 assert kernels("vtl_hip_forward_i8_host", host, 1, 784, C.byref(layer), 1, host) == ["linear_gemv"]
-layer = capi.Layer(0, 0, 64, 6000, p, p, None, 0)                             # 24 KB: uploaded first
-assert kernels("vtl_hip_forward_i8_host", host, 1, 6000, C.byref(layer), 1, host) == ["host_copy", "linear_gemv"]
+# that where every workgroup's reading of the row is not the longer, else it is quantized by a launch of its own (uploaded, 20 to 32 KB, for neither)
+for n, k, want in ((5500, 4096, 1), (17, 5120, 0), (16, 5120, 1), (17, 5136, 0), (1, 8192, 0), (16, 8208, 1), (17, 8208, 0), (64, 14336, 0), (64, 4999, 1),
+                   (4000, 11001, 1), (33, 11017, 0), (32, 14001, 1), (4000, 6001, 2)):
+    layer = capi.Layer(0, 0, n, k, p, p, None, 0)
+    got = kernels("vtl_hip_forward_i8_host", host, 1, k, C.byref(layer), 1, host)
+    assert got[:max(want, 1)] == [["quantize"], ["linear_gemv"], ["host_copy", "linear_gemv"]][want], (n, k, got)
+layers = (capi.Layer * 2)(capi.Layer(0, 0, 10000, 16, p, p, None, 0), capi.Layer(0, 0, 64, 10000, p, p, None, 0))
+assert kernels("vtl_hip_forward_i8_host", host, 1, 16, layers, 2, host) == ["linear_gemv"]      # twice: the second row is on the device
 rows = (C.c_float * (9 << 20))()
 got = [kernels("vtl_hip_upload_quantized", rows, n, k, 1, p, p, None, None, 0) for n, k in ((4200, 2044), (4096, 2048))]
 assert "upload_rows" not in got[0] and got[1] == ["upload_rows"], got        # (in short rows too little would be on its way)

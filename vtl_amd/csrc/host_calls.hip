@@ -63,6 +63,19 @@ int check_layers(const vtl_hip_layer *layers, int count, int cols, int &out_cols
     return VTL_HIP_OK;
 }
 
+// Whether one row of the caller's, against weights with one scale, is quantized in the launch of the product.  That every workgroup
+// reads a long row over the link, or that it is uploaded first (20 to 32 KiB), is more than a second launch behind one that reads it once; rows
+// that start anywhere are read twice there and hold out longer (us, in two launches and in one: 64 x 4096 15.9 and 15.8, 48 x 5120 15.9
+// and 16.4, 16 x 5120 15.6 and 14.3, 64 x 6000 16.3 and 17.2, 600 x 8192 18.4 and 18.0, 64 x 10000 18.0 and 20.4, 2500 x 10000 22.8 and 24.9, 16 x 10000 17.8
+// and 16.1, 64 x 14336 19.6 and 24.1, 16 x 14336 19.1 and 18.7; 64 x 6001 19.5 and 17.2, 64 x 11001 21.1 and 21.1, 5500 x 11001 29.6 and 28.6, 64 x 14001 21.6
+// and 23.8, 32 x 14001 21.2 and 20.1).  Beyond 14336 both take two.
+bool row_in_one(int n, int k)
+{
+    if (k % 16 != 0)
+        return k <= 11008 || n <= 32 || k > 14336;
+    return k <= 4096 || ((k <= 5120 || k > 8192) && n <= 16) || k > 14336;
+}
+
 int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer *layers, int count, float *y_host)
 {
     int out_cols = 0;
@@ -89,11 +102,12 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
     // (32 KiB is what the kernels that quantize in every workgroup take at most; near it the eight XCDs' transfers
     // cost what an upload does)
     // One row has one scale either way: a layer with one for all of its weights takes it as one with a scale per row does, in one
-    // launch instead of two (us, per tensor: 1 x 832 x 448 17.4 -> 15.9, 1 x 3000 x 513 20.9 -> 17.3, 1 x 11000 x 4001 28.4 -> 24.6, 1 x
-    // 576 x 238 18.4 -> 16.9).
+    // launch instead of two (us, per tensor: 1 x 832 x 448 17.4 -> 15.9, 1 x 3000 x 513 20.9 -> 17.3, 1 x 576 x 238 18.4 -> 16.9; a second layer of
+    // 64 x 256 20.9 -> 17.0, of 2500 x 11008 29.3 -> 24.6).
     const auto by_row = [&](const vtl_hip_layer &l) { return l.per_channel || rows == 1; };
+    const bool first_by_row = count > 0 && by_row(layers[0]) && (layers[0].per_channel || row_in_one(layers[0].out_features, cols));
     const bool upload_first = rows <= 8 && in_bytes > ((size_t)20 << 10) && in_bytes <= ((size_t)32 << 10);
-    if (count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR && !(upload_first && by_row(layers[0])) &&
+    if (count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR && !(upload_first && first_by_row) &&
         input.stage(x_host, in_bytes)) {
         // The first launch takes the input over the link itself: 64 x 784, per tensor, 4 us less than behind an
         // upload.  Rows that are no whole vectors are read twice, which still is no slower (forward of 200 x 1001
@@ -102,7 +116,7 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
         // device memory for a row of up to 4096, 10 for 32 such rows (read once), where the upload takes 3 and 13 and a
         // launch of its own.
         x = static_cast<const float *>(input.data);
-        if (!by_row(layers[0]) || rows > kFewRows) {
+        if (!first_by_row || rows > kFewRows) {
             VTL_STEP(codes.take((size_t)rows * (size_t)cols));
             VTL_STEP(scales.take((layers[0].per_channel ? (size_t)rows : 1) * sizeof(float)));
             VTL_STEP(vtl_hip_quantize_f32_i8(x, rows, cols, layers[0].per_channel, codes.as<int8_t>(), scales.as<float>()));
