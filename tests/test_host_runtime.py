@@ -321,6 +321,24 @@ print("done")
 """)
 
 
+def test_small_uploads_share_a_launch_with_little_else(fake_runtime):
+    _run(fake_runtime, r"""
+runtime()
+host = (C.c_float * (1 << 19))()
+def launches(*sizes):
+    p = [malloc_on(0, n) for n in sizes]
+    events()
+    assert capi.status("vtl_hip_upload_two", p[0], host, sizes[0], p[1], host, sizes[1]) == capi.OK
+    found = [l[4] for l in lines() if l[0] == "launch"]
+    assert all("host_copy" in k or "clear_counters" in k for k in found), found
+    return sum("host_copy" in k for k in found)
+launches(16, 16)
+for a, b, n in ((4, 4, 1), (320 << 10, 321 << 10, 2), (2048, 1 << 20, 1), (1 << 20, 64 << 10, 1), (1 << 20, 65 << 10, 2)):    # (a slot's 4 MiB in all)
+    assert launches(a, b) == n, (a, b)
+print("done")
+""")
+
+
 def test_where_column_sums_take_one_launch(fake_runtime):
     _run(fake_runtime, r"""
 runtime()

@@ -1047,9 +1047,9 @@ try {
     // One launch for both saves its 3 us while they are small; from there on the first is on the link while the host copies
     // the second, and what one host thread copies well needs no others (f32 products, together and in turn: 700 x 1024 x 200 129 and
     // 122 us, 512 x 512 x 300 87 and 83, 1024 x 1000 x 128 139 and 136; 1024 x 1001 x 64 115 and 117).
-    // With little of one there is nothing to overlap (a bias behind its weights).
+    // With little of one there is nothing to overlap (a bias behind its weights; of 512 x 512, 1 MiB exactly, 74.0 us together, 76.5 in turn).
     const size_t all = bytes0 + bytes1, less = bytes0 < bytes1 ? bytes0 : bytes1;
-    if (all <= kUploadTogether || (all <= kSmall && less <= kWithAnother)) {
+    if (all <= kUploadTogether || (all - less <= kSmall && less <= kWithAnother)) {
         status = upload_small(r, from, 2, current_stream());
     } else if (bytes0 <= kSmall && bytes1 <= kSmall) {
         status = upload_small(r, from, 1, current_stream());
