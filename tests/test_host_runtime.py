@@ -321,6 +321,25 @@ print("done")
 """)
 
 
+def test_where_gradients_share_a_launch(fake_runtime):
+    """Not where dW is few rows of millions of values, or large enough for shapes of its own."""
+    _run(fake_runtime, r"""
+runtime()
+p = [malloc_on(0, 1 << 20) + (i << 36) for i in range(6)]             # (no kernel runs here)
+def in_one(name, m, n, k, dx, db):
+    events()
+    assert capi.status("vtl_hip_linear_backward_" + name, p[0], p[1], p[2], p[3] if dx else None, p[4], p[5] if db else None, m, n, k) == capi.OK
+    found = [l[4] for l in lines() if l[0] == "launch"]
+    return "linear_backward" in found[0]                              # (and what adds up slices behind it)
+for name, m, n, k, dx, db in (("f32", 64, 256, 640, 1, 1), ("f32", 192, 832, 832, 1, 1), ("f64", 13, 664, 2861, 1, 0), ("f32", 3, 742, 1465, 1, 1), ("f64", 13, 4511, 120, 0, 1)):
+    assert in_one(name, m, n, k, dx, db), (name, m, n, k)
+for name, m, n, k, dx, db in (("f32", 9, 1899, 2356, 1, 1), ("f64", 7, 927, 4509, 0, 1), ("f32", 2, 1072, 1284, 1, 0), ("f32", 31, 1870, 1608, 1, 1), ("f32", 256, 11008, 4096, 1, 1),
+                              ("f64", 442, 6, 3774, 1, 0), ("f32", 88, 1150, 4098, 0, 1), ("f64", 15, 1993, 769, 0, 1)):
+    assert not in_one(name, m, n, k, dx, db), (name, m, n, k)
+print("done")
+""")
+
+
 def test_small_uploads_share_a_launch_with_little_else(fake_runtime):
     _run(fake_runtime, r"""
 runtime()

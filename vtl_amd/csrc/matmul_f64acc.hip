@@ -1151,9 +1151,11 @@ bool backward_in_one(vtlhip::HostResult *result, const T *grad, const T *x, cons
     if (tiles_w + tiles_x * slices + sums > 0x7fffffff)
         return false;
     if (forced < 0) {
-        // As choose_plan estimates, the tiles of both products dealt out over the chip.  Sets of gradients from 16 x 92 x 421 to 256 x
-        // 9728 x 320, f32 and f64, in one launch and one by one: up to 0.9 of `apart` 0.39 to 0.86 of the time, up to 1.05 0.8 to 1.01; above 1.2, where
-        // large weight tiles have shapes of their own, 0.98 to 1.26.
+        // As choose_plan estimates, the tiles of both products dealt out over the chip.  Five hundred sets of gradients of 2 to 600 rows, n and k
+        // of 2 to 6000, half f32 and half f64, in one launch and one by one: up to 0.8 of `apart` 0.34 to 0.97 of the time, up to 0.9 0.74 to 0.99, up to
+        // 1.05 0.77 to 1.03; above 1.2, where large weight tiles have shapes of their own, 1.21 to 1.85.  Less sure are tiles that are mostly
+        // stores or partial sums: from 0.85 on f32 9 x 1899 x 2356 27.0 and 33.1 us, 31 x 1870 x 1608 23.0 and 23.9, f64 7 x 927 x 4509 15.3 and 17.4, 442 x 6 x 3774
+        // 15.0 and 15.9, without dX f32 88 x 1150 x 4098 31.7 and 34.4, f64 15 x 1993 x 769 8.8 and 9.6.
         const double each_x = tile_us(px.shape, (double)n / px.slices), each_w = tile_us(pw.shape, m);
         const double longest = dx && each_x > each_w ? each_x : each_w;
         double us = 2.9 + ((double)(tiles_x * px.slices) * each_x + (double)tiles_w * each_w) / 256.0 + 0.5 * longest;
@@ -1162,7 +1164,8 @@ bool backward_in_one(vtlhip::HostResult *result, const T *grad, const T *x, cons
         double apart = choose_plan(kind, n, k, m, alone || m >= 2048, false, kLaunch).us + (db ? 4.0 : 0.0);
         if (dx)
             apart += choose_plan(kind, m, k, n, alone || n >= 2048, false, kLaunch).us;
-        if (us > 1.05 * apart)
+        const bool slim = n < 32 || (m < 32 && (!dx || px.slices > 1)) || (m < 128 && w_bytes > (size_t)16 << 20);
+        if (us > (slim ? 0.85 : 1.05) * apart)
             return false;
     }
     BackwardArgs<T> g = {};
