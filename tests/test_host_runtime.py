@@ -299,6 +299,26 @@ print("done")
 """)
 
 
+def test_a_forward_on_a_stream_of_its_own_waits_for_no_other(fake_runtime):
+    """Nor does a forward from host to host whose results are flagged by a launch of their own."""
+    _run(fake_runtime, r"""
+runtime()
+p = malloc_on(0, 8 << 20)
+host, y = (C.c_float * (1 << 16))(), (C.c_float * (1 << 16))()
+capi.call("vtl_hip_set_stream", 4096)
+for per_channel in (0, 1):
+    for rows, n, k in ((1, 3358, 150), (1, 3358, 160), (1, 64, 64), (2, 3271, 50), (8, 3000, 512)):
+        for row in (0, (k + 15) // 16 * 16):
+            layer = capi.Layer(0, per_channel, n, k, p, p, None, row)
+            events()
+            capi.status("vtl_hip_forward_i8_host", host, rows, k, C.byref(layer), 1, y)    # no kernel runs here
+            log = [e[0] for e in events()]
+            last = max(i for i, e in enumerate(log) if e == "launch")
+            assert "device_sync" not in log[:last], (per_channel, rows, n, k, row, log)
+print("done")
+""")
+
+
 def test_column_sums_within_their_input_come_behind_all_of_it(fake_runtime):
     """Sums that are written into the tensor they are made from, from 128 rows on: by a launch behind the one that reads it, for other
     workgroups still read what one has summed."""

@@ -84,6 +84,8 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
         return count == 0 ? VTL_HIP_OK : VTL_HIP_ERR_INVALID_ARG;
     const size_t in_bytes = (size_t)rows * (size_t)cols * sizeof(float);
     Scratch cur, next;                     // f32 rows
+    Scratch work;                          // of layers on f32 rows, to the call's last launch: once a stream has been named a release waits
+    size_t work_bytes = 0;
     Scratch codes, scales, next_codes, next_scales;
     const float *x = nullptr;              // the f32 rows, or null while the activations are codes
     int i = 0;
@@ -147,8 +149,10 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
             if (!last)
                 VTL_STEP(next.take((size_t)rows * (size_t)n * sizeof(float)));
             const size_t need = vtl_hip_linear_f32_dynquant_workspace(rows, cols);
-            Scratch work;
-            VTL_STEP(work.take(need));
+            if (need > work_bytes) {
+                VTL_STEP(work.take(need));
+                work_bytes = need;
+            }
             VTL_STEP(layer_f32(l, x, last ? y : next.as<float>(), rows, relu, work.ptr, need, last ? &result : nullptr,
                                input.data != nullptr));
             if (input.data) {
@@ -183,7 +187,13 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
         }
         cols = n;
     }
-    return y ? result.finish() : vtl_hip_memcpy_d2h(y_host, cur.ptr, out_bytes);
+    if (!y)
+        return vtl_hip_memcpy_d2h(y_host, cur.ptr, out_bytes);
+    if (result.attached() || !single_stream()) {   // nothing more to launch: what a release waits for is what the results are waited for
+        for (Scratch *s : {&work, &cur, &next, &codes, &scales, &next_codes, &next_scales})
+            s->release();
+    }
+    return result.finish();
 }
 
 int colsum(const float *x, int64_t rows, int64_t cols, float *out) { return vtl_hip_colsum_f32(x, rows, cols, out); }

@@ -1153,15 +1153,17 @@ int HostResult::finish()
     hipStream_t st = current_stream();
     const bool one_stream = single_stream();
     int rc = VTL_HIP_OK;
-    if (!attached_) {
+    if (!attached_ && one_stream) {
         CopyArgs g = {};
         attach(g.signals.done, 1);
         g.signals.to_host = 1;
         hipLaunchKernelGGL(host_copy_kernel, dim3(1), dim3(64), 0, st, g);
         rc = check_launch("host_copy_kernel");
     }
-    if (rc == VTL_HIP_OK)
+    if (rc == VTL_HIP_OK && attached_)
         rc = wait_behind(lane, uploads_, one_stream, st);
+    else if (rc == VTL_HIP_OK)   // a release has waited for the device, or will: no launch more to raise a flag
+        VTL_HIP_TRY(hipStreamSynchronize(st));
     if (rc != VTL_HIP_OK)
         return rc;
     for (int i = 0; i < nafter_; i++)
