@@ -106,7 +106,7 @@ int vtl_hip_upload(void *dst_device, const void *src_host, size_t bytes);
 /* Two of them, in one launch while they are small. */
 int vtl_hip_upload_two(void *dst0, const void *src0, size_t bytes0, void *dst1, const void *src1, size_t bytes1);
 /* vtl_hip_upload of rows x cols f32 and vtl_hip_quantize_f32_i8 of them, with the f32 values in no memory of the
- * caller's (with a scale per row they are quantized as they arrive where that can be), and a vtl_hip_upload of
+ * caller's (made codes of by the host's threads, or as they arrive, where that is the faster way), and a vtl_hip_upload of
  * extra_bytes (0: none) with them. */
 int vtl_hip_upload_quantized(const float *src_host, int64_t rows, int64_t cols, int per_row, int8_t *q, float *scale,
                              void *extra_device, const void *extra_host, size_t extra_bytes);

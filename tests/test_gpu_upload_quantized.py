@@ -4,7 +4,8 @@ import numpy as np
 import pytest
 
 from helpers import dev
-from vtl_amd import capi
+from vtl_amd import PER_CHANNEL, PER_TENSOR, QuantLinearLayer, capi
+from vtl_amd.layers import QuantizedWeights
 from vtl_amd.tensor import HipTensor
 
 pytestmark = pytest.mark.gpu
@@ -47,3 +48,29 @@ def test_errors(hip):
         assert capi.status("vtl_hip_upload_quantized", *args) == capi.ERR_INVALID_ARG
     for t in (q, s):
         t.release()
+
+
+# The same by the host's units and by the device's: what one thread makes and what several do, pieces that rows do not divide, rows too short
+# for it, one scale for all, and whole forwards whose first layer takes codes (more than 32 rows, dense and padded)
+@pytest.mark.parametrize("rows,cols", [(64, 784), (33, 15), (300, 1023), (257, 1021), (263, 4099), (1000, 17), (70, 70001), (5000, 1027)])
+def test_by_the_host_and_by_the_device(hip, knobs, rows, cols):
+    rng = np.random.default_rng(rows * 31 + cols)
+    x = rng.standard_normal((rows, cols)).astype(np.float32)
+    x[rows // 3, :: 5] = np.nan
+    w = rng.standard_normal((40, cols)).astype(np.float32)
+    bias = rng.standard_normal((1, 40)).astype(np.float32)
+    print("rows", rows, cols, flush=True)
+    got = []
+    for by_host in ("0", "1"):
+        knobs.setenv("VTL_HIP_HOST_QUANTIZE", by_host)
+        out = []
+        for mode in (PER_CHANNEL, PER_TENSOR):
+            qw = QuantizedWeights(x, None, mode)
+            out += [qw.w_q.cpu().copy(), qw.sw.cpu().view(np.int32).copy()]
+            qw.release()
+            layer = QuantLinearLayer(w, bias, mode=mode, requires_grad=False)
+            out += [layer.forward(x).copy(), layer.forward(x[: rows // 2]).copy()]
+            layer.release()
+        got.append(out)
+    for a, b in zip(*got):
+        assert np.array_equal(a, b, equal_nan=a.dtype == np.float32)

@@ -13,7 +13,7 @@ LIB_PATH = os.path.join(PKG_DIR, "libvtlhip.so")
 OBJ_DIR = os.path.join(PKG_DIR, "_build")
 # bench.py's measurement aid (an MFMA-only loop): a library of its own, no part of the product
 BENCH_PROBE_PATH = os.path.join(PKG_DIR, "libvtlbenchprobe.so")
-SOURCES = ["runtime.hip", "memory.hip", "host_copy.hip", "quant.hip", "gemm_i8.hip", "matmul_f64acc.hip", "tensor_ops.hip",
+SOURCES = ["runtime.hip", "memory.hip", "host_copy.hip", "host_quant.hip", "quant.hip", "gemm_i8.hip", "matmul_f64acc.hip", "tensor_ops.hip",
            "host_calls.hip"]
 
 HIPCC_FLAGS = [

@@ -96,6 +96,11 @@ bool upload_together(const HostUpload *uploads, int count, int &status);
 bool upload_rows(const float *src, int64_t rows, int64_t cols, int8_t *q, float *scale, void *extra_dst, const void *extra_src,
                  size_t extra_bytes, int &status);
 
+// Rows that the host's threads quantize in front of the link, which then carries a quarter of their bytes: per_row, or with one
+// scale; `row` bytes from one row of codes to the next (zeros behind the codes).  False: to be quantized by the device.
+bool upload_codes(const float *src, int64_t rows, int64_t cols, int per_row, int8_t *q, int64_t row, float *scale, void *extra_dst,
+                  const void *extra_src, size_t extra_bytes, int &status);
+
 // How a launch tells the host that its results are there: every workgroup counts itself when its stores are
 // complete, and the one that reaches the target raises the flag.  No flag: nothing to tell.
 struct DoneSignal {
@@ -274,14 +279,14 @@ bool gradients_in_one(HostResult *result, const double *grad, const double *x, c
                       int n, int k, int &status);
 
 // vtl_hip_linear_i8_f32 and vtl_hip_linear_i8_requant with the parameters of a layer, whose weights may have padded rows.
-// `result`: Y is its memory.
+// `result`: Y is its memory.  `padded`: so have the codes A.
 int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa, float *Y, int M, int relu,
-                        HostResult *result = nullptr);
+                        HostResult *result = nullptr, bool padded = false);
 // vtl_hip_layer_f32; of one row with one scale for the weights too.  `x_on_host`: X is in pinned memory (HostInput).
 int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu, void *workspace, size_t workspace_bytes,
               HostResult *result = nullptr, bool x_on_host = false);
 int layer_linear_i8_requant(const vtl_hip_layer &l, const int8_t *A, const float *sa, int8_t *Yq, float *sy, int M,
-                            int relu);
+                            int relu, bool padded = false);
 
 // Tuning and test switches, taken from the environment once (first use) and
 // again only when vtl_hip_reload_env() is called: the dispatch path of a launch
@@ -303,6 +308,7 @@ struct Tuning {
     int skinny_tiled = -1;          // VTL_HIP_SKINNY_TILED: 1 / 0 force the 32x32-block weight-streaming kernel for M > 32
     int skinny_waves = 4;           // VTL_HIP_SKINNY_WAVES: 2, 4 or 8 waves (K ranges) per workgroup there
     int matmul_tile = 0;            // VTL_HIP_MATMUL_TILE: which kernel and tile the f64-accumulating matmul takes (matmul_f64acc.hip)
+    int host_quantize = -1;         // VTL_HIP_HOST_QUANTIZE: 1 / 0 force rows in host memory to be quantized by the host's / the device's units
     int backward_group = -1;        // VTL_HIP_BACKWARD_GROUP: 1 / 0 force a backward's gradients in one launch on (where it can be) / off
     int matmul_splits = -1;         // VTL_HIP_MATMUL_SPLITS: K ranges of the f64-accumulating matmul
 };

@@ -2773,12 +2773,13 @@ int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, int s
 namespace vtlhip {
 
 int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa, float *Y, int M, int relu,
-                        HostResult *result)
+                        HostResult *result, bool padded)
 {
     int st = layer_row_fits(l) && A && M >= 0 ? VTL_HIP_OK : VTL_HIP_ERR_INVALID_ARG;
     int K = l.in_features;
     if (st == VTL_HIP_OK && l.row_bytes && M > 0) {
-        A = pad_activations(A, M, K, l.row_bytes, st);
+        if (!padded)
+            A = pad_activations(A, M, K, l.row_bytes, st);
         K = l.row_bytes;
     }
     return st != VTL_HIP_OK ? st : linear_i8_f32(A, sa, l.per_channel, l.wq, l.sw, l.per_channel, l.bias, Y, M,
@@ -2829,12 +2830,13 @@ int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu,
 }
 
 int layer_linear_i8_requant(const vtl_hip_layer &l, const int8_t *A, const float *sa, int8_t *Yq, float *sy, int M,
-                            int relu)
+                            int relu, bool padded)
 {
     int st = layer_row_fits(l) && A && M >= 0 ? VTL_HIP_OK : VTL_HIP_ERR_INVALID_ARG;
     int K = l.in_features;
     if (st == VTL_HIP_OK && l.row_bytes && M > 0) {
-        A = pad_activations(A, M, K, l.row_bytes, st);
+        if (!padded)
+            A = pad_activations(A, M, K, l.row_bytes, st);
         K = l.row_bytes;
     }
     return st != VTL_HIP_OK ? st : vtl_hip_linear_i8_requant(A, sa, 1, l.wq, l.sw, 1, l.bias, relu, Yq, sy, nullptr, M,

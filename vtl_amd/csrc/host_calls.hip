@@ -108,8 +108,25 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
     // 64 x 256 20.9 -> 17.0, of 2500 x 11008 29.3 -> 24.6).
     const auto by_row = [&](const vtl_hip_layer &l) { return l.per_channel || rows == 1; };
     const bool first_by_row = count > 0 && by_row(layers[0]) && (layers[0].per_channel || row_in_one(layers[0].out_features, cols));
+    // More than a few rows that a quantizer's launch would only make codes of go up as codes: of 200 KB the copies and the launches
+    // take less, of 4 MiB the link too.
+    bool padded = false;                   // whether the codes lie in rows of l.row_bytes
+    if (count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR && rows > kFewRows) {
+        const vtl_hip_layer &l = layers[0];
+        const int row = l.row_bytes > cols ? l.row_bytes : cols;
+        VTL_STEP(codes.take((size_t)rows * (size_t)row));
+        VTL_STEP(scales.take((l.per_channel ? (size_t)rows : 1) * sizeof(float)));
+        int status = VTL_HIP_OK;
+        if (upload_codes(x_host, rows, cols, l.per_channel, codes.as<int8_t>(), row, scales.as<float>(), nullptr, nullptr, 0, status)) {
+            VTL_STEP(status);
+            padded = l.row_bytes != 0;
+        } else {
+            codes.release();
+            scales.release();
+        }
+    }
     const bool upload_first = rows <= 8 && in_bytes > ((size_t)20 << 10) && in_bytes <= ((size_t)32 << 10);
-    if (count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR && !(upload_first && first_by_row) &&
+    if (!codes.ptr && count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR && !(upload_first && first_by_row) &&
         input.stage(x_host, in_bytes)) {
         // The first launch takes the input over the link itself: 64 x 784, per tensor, 4 us less than behind an
         // upload.  Rows that are no whole vectors are read twice, which still is no slower (forward of 200 x 1001
@@ -175,16 +192,17 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
             VTL_STEP(next_codes.take((size_t)rows * (size_t)n));
             VTL_STEP(next_scales.take((size_t)rows * sizeof(float)));
             VTL_STEP(layer_linear_i8_requant(l, codes.as<int8_t>(), scales.as<float>(), next_codes.as<int8_t>(),
-                                             next_scales.as<float>(), rows, relu));
+                                             next_scales.as<float>(), rows, relu, padded));
             codes.swap(next_codes);
             scales.swap(next_scales);
         } else {
             if (!last)
                 VTL_STEP(cur.take((size_t)rows * (size_t)n * sizeof(float)));
             VTL_STEP(layer_linear_i8_f32(l, codes.as<int8_t>(), scales.as<float>(), last ? y : cur.as<float>(), rows, relu,
-                                         last ? &result : nullptr));
+                                         last ? &result : nullptr, padded));
             x = cur.as<float>();
         }
+        padded = false;
         cols = n;
     }
     if (!y)
@@ -392,6 +410,9 @@ int vtl_hip_upload_quantized(const float *src_host, int64_t rows, int64_t cols, 
     if (rows < 0 || cols < 0 || (rows > 0 && cols > 0 && (!src_host || !q)) || (extra_bytes && (!extra_device || !extra_host)))
         return VTL_HIP_ERR_INVALID_ARG;
     int status = VTL_HIP_OK;
+    if (scale && rows > 0 && cols > 0 &&
+        upload_codes(src_host, rows, cols, per_row, q, cols, scale, extra_device, extra_host, extra_bytes, status))
+        return status;
     if (per_row && scale && rows > 0 && cols > 0 &&
         upload_rows(src_host, rows, cols, q, scale, extra_device, extra_host, extra_bytes, status))
         return status;

@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "host_quant.hpp"
 #include "quant_device.hpp"
 
 namespace vtlhip {
@@ -451,6 +452,8 @@ constexpr int kSlots = 8;
 constexpr size_t kSlotBytes = (size_t)4 << 20;
 constexpr size_t kSlotStride = kSlotBytes + 4096;
 constexpr size_t kWithAnother = (size_t)64 << 10;
+constexpr size_t kManyHelpersFrom = (size_t)16 << 20;   // below, more than three helpers cost more to wake than they do (4 MiB, us of a forward: 157 and 171)
+constexpr int kCodesLeastCols = 16;             // rows of fewer values are hardly fewer bytes as codes and a scale
 constexpr size_t kSmall = (size_t)1 << 20;      // up to here one host thread copies faster than others wake up
 
 struct Ring {
@@ -588,21 +591,39 @@ int processors()
     return quota < period ? 1 : (int)(quota / period);
 }
 
+// Quantization of rows: what a source or a piece of one becomes on its way, if anything (no codes: its bytes are copied).
+struct Quantized {
+    int8_t *q = nullptr;         // codes on the device
+    float *scale = nullptr;      // one for each row there
+    size_t unit = 0;             // bytes of a row of f32 (they are not cut)
+    // by the host's threads: bytes from one row of codes to the next, and the scale of all rows (with `one`)
+    const HostQuantizer *host = nullptr;
+    size_t row = 0;
+    bool one = false;
+    float given = 0.0f;
+};
+
 struct Crew {
     struct Job {
         char *dst;
         const char *src;
         size_t bytes;
-        std::atomic<int> *left;   // jobs of the same chunk that are not done
+        std::atomic<int> *left;         // jobs of the same chunk that are not done
+        const Quantized *codes;         // makes codes at dst (with none there: the largest magnitude for `scales`) instead of a copy
+        float *scales;
     };
+    // (us, 180 MB made codes of and their forward, in jobs of 64 / 128 / 256 KiB: 2780 / 1670 / 1480; they meet at the lock)
     static constexpr size_t kJobBytes = (size_t)256 << 10;
+    // How many helpers there are, where processors are many, and how many of them a copy takes: the link needs no more, but what reads four
+    // bytes to send one does (us, as above with 3 / 7 / 11 helpers: 2240 / 1480 / 1430).
+    static constexpr int kHelpers = 7, kCopyHelpers = 3;
 
     std::mutex lock;
-    std::condition_variable wake;
+    std::condition_variable wake, wake_more;     // the first kCopyHelpers, and the others
     std::deque<Job> queue;
     std::atomic<int> queued{0};      // jobs in the queue, read without the lock
     std::atomic<int> transfers{0};   // under way
-    unsigned begun = 0;              // transfers so far (lock held)
+    unsigned begun = 0, begun_more = 0;    // transfers so far, and those that take every helper (lock held)
     bool called = false;             // every helper that sleeps has been notified (lock held)
     bool started = false;
 
@@ -611,42 +632,52 @@ struct Crew {
         static Crew *c = new Crew;   // never destroyed: its threads live as long as the process
         return *c;
     }
-    void begin()
+    void begin(bool more = false)
     {
         {
             std::lock_guard<std::mutex> hold(lock);
             transfers++;
             begun++;
+            begun_more += more;
             called = true;
             if (!started) {
                 started = true;
-                const int have = processors();
+                const int have = processors(), helpers = have > 2 * kHelpers ? kHelpers : have > 4 ? kCopyHelpers : have - 1;
                 try {
-                    for (int i = 0; i < (have > 4 ? 3 : have - 1); i++)
-                        std::thread([this] { help(); }).detach();
+                    for (int i = 0; i < helpers; i++)
+                        std::thread([this, i] { help(i >= kCopyHelpers); }).detach();
                 } catch (const std::exception &) {   // no more threads to be had: the callers copy alone
                 }
             }
         }
         wake.notify_all();
+        if (more)
+            wake_more.notify_all();
     }
     void end()
     {
         std::lock_guard<std::mutex> hold(lock);
         transfers--;
     }
-    void push(char *dst, const char *src, size_t bytes, std::atomic<int> &left)
+    // Cut into jobs of `size` bytes (of whole rows).
+    void push(char *dst, const char *src, size_t bytes, std::atomic<int> &left, const Quantized *codes = nullptr, float *scales = nullptr,
+              size_t size = kJobBytes)
     {
-        left.store((int)((bytes + kJobBytes - 1) / kJobBytes), std::memory_order_relaxed);
+        left.store((int)((bytes + size - 1) / size), std::memory_order_relaxed);
         std::lock_guard<std::mutex> hold(lock);
-        for (size_t at = 0; at < bytes; at += kJobBytes) {
-            const size_t take = bytes - at < kJobBytes ? bytes - at : kJobBytes;
+        for (size_t at = 0; at < bytes; at += size) {
+            Job j = {dst, src + at, bytes - at < size ? bytes - at : size, &left, codes, scales};
+            if (!codes) {
+                j.dst = dst + at;
+            } else if (dst) {
+                j.dst = dst + at / codes->unit * codes->row;
+                j.scales = scales ? scales + at / codes->unit : nullptr;
+            }
             try {
-                queue.push_back({dst + at, src + at, take, &left});
+                queue.push_back(j);
                 queued++;
             } catch (const std::exception &) {
-                memcpy(dst + at, src + at, take);
-                left.fetch_sub(1, std::memory_order_release);
+                run(j);
             }
         }
         if (!called) {       // one went to sleep since the transfer began
@@ -654,21 +685,52 @@ struct Crew {
             wake.notify_all();
         }
     }
+    static void run(const Job &j)
+    {
+        if (!j.codes) {
+            memcpy(j.dst, j.src, j.bytes);
+        } else {
+            const Quantized &c = *j.codes;
+            const float *x = reinterpret_cast<const float *>(j.src);
+            const int64_t rows = (int64_t)(j.bytes / c.unit), cols = (int64_t)(c.unit / sizeof(float));
+            int8_t *q = reinterpret_cast<int8_t *>(j.dst);
+            if (!q)
+                raise(j.scales, c.host->absmax(x, (int64_t)(j.bytes / sizeof(float))));
+            else if (c.one)
+                c.host->scaled(x, rows, cols, q, (int64_t)c.row, c.given);
+            else
+                c.host->rows(x, rows, cols, q, (int64_t)c.row, j.scales);
+        }
+        j.left->fetch_sub(1, std::memory_order_release);
+    }
+    static void raise(float *most, float v)
+    {
+        float seen;
+        __atomic_load(most, &seen, __ATOMIC_RELAXED);
+        while (v > seen && !__atomic_compare_exchange(most, &seen, &v, true, __ATOMIC_RELAXED, __ATOMIC_RELAXED))
+            ;
+    }
     bool work()
     {
         if (queued.load(std::memory_order_acquire) == 0)
             return false;
         Job j;
         {
-            std::lock_guard<std::mutex> hold(lock);
+            // (held for a few instructions: to be put to sleep for it, and woken, takes longer than a job)
+            std::unique_lock<std::mutex> hold(lock, std::try_to_lock);
+            for (int i = 0; i < 1000 && !hold; i++) {
+                __builtin_ia32_pause();
+                hold.try_lock();
+            }
+            if (!hold)
+                hold.lock();
             if (queue.empty())
                 return false;
             j = queue.front();
             queue.pop_front();
             queued--;
         }
-        memcpy(j.dst, j.src, j.bytes);
-        j.left->fetch_sub(1, std::memory_order_release);
+        run(j);
         return true;
     }
     // The caller of a transfer copies too while it would otherwise wait.
@@ -678,7 +740,7 @@ struct Crew {
             if (!work())
                 __builtin_ia32_pause();
     }
-    void help()
+    void help(bool more)
     {
         unsigned seen = 0;
         double since = seconds();
@@ -693,13 +755,18 @@ struct Crew {
                 continue;
             }
             std::unique_lock<std::mutex> hold(lock);
-            wake.wait(hold, [&] {
-                const bool stay = begun == seen && queue.empty();
-                if (stay)
-                    called = false;
-                return !stay;
-            });
-            seen = begun;
+            if (more) {
+                wake_more.wait(hold, [&] { return begun_more != seen; });
+                seen = begun_more;
+            } else {
+                wake.wait(hold, [&] {
+                    const bool stay = begun == seen && queue.empty();
+                    if (stay)
+                        called = false;
+                    return !stay;
+                });
+                seen = begun;
+            }
             since = seconds();
         }
     }
@@ -734,14 +801,36 @@ char *put_small(Ring *r, const void *src, size_t bytes, size_t skew)
 }
 
 // One upload of several.
-struct Source {
+struct Source : Quantized {
     void *dst;
     const void *src;
     size_t bytes;
-    // rows that arrive as codes and scales instead, and the bytes of one (they are not cut)
-    int8_t *q = nullptr;
-    float *scale = nullptr;
-    size_t unit = 0;
+
+    Source() = default;
+    Source(void *dst_, const void *src_, size_t bytes_, const Quantized &codes = {}) : Quantized(codes), dst(dst_), src(src_), bytes(bytes_) {}
+    // Where it lies in pinned memory, from a 64-byte boundary: bytes or codes as far behind a 16-byte boundary as on the
+    // device, and behind the codes that the host has made the scales.
+    size_t skew() const { return reinterpret_cast<uintptr_t>(host ? static_cast<void *>(q) : dst) & 15; }
+    size_t codes_bytes() const { return bytes / unit * row; }
+    size_t scales_at() const { return ((skew() + codes_bytes() + 15) & ~(size_t)15) + (reinterpret_cast<uintptr_t>(scale) & 15); }
+    size_t link_bytes() const { return host ? codes_bytes() + (one ? 0 : bytes / unit * sizeof(float)) : bytes; }
+    size_t staged_bytes() const { return host ? scales_at() + (one ? 0 : bytes / unit * sizeof(float)) : bytes; }
+    // By the calling thread.
+    void stage(char *staged) const
+    {
+        std::atomic<int> left{1};
+        Crew::run({staged + skew(), static_cast<const char *>(src), bytes, &left, host ? this : nullptr,
+                   host && !one ? reinterpret_cast<float *>(staged + scales_at()) : nullptr});
+    }
+    // The segments that carry it.
+    int segments(char *staged, Segment *seg) const
+    {
+        seg[0] = host ? make_segment(q, staged + skew(), codes_bytes()) : make_segment(dst, staged + skew(), bytes);
+        if (!host || one)
+            return 1;
+        seg[1] = make_segment(scale, staged + scales_at(), bytes / unit * sizeof(float));
+        return 2;
+    }
 };
 
 // What a launch carries: `staged` in pinned memory.
@@ -749,13 +838,14 @@ struct Load {
     RowsArgs rows = {};
     CopyArgs copy = {};
 
+    // `staged`: 16-byte aligned
     void add(const Source &piece, char *staged)
     {
-        if (!piece.unit) {
-            copy.seg[copy.count++] = make_segment(piece.dst, staged, piece.bytes);
+        if (!piece.unit || piece.host) {
+            copy.count += piece.segments(staged, copy.seg + copy.count);
             return;
         }
-        rows.rows[rows.count++] = {reinterpret_cast<const float *>(staged), piece.q, piece.scale, (int)(piece.bytes / piece.unit)};
+        rows.rows[rows.count++] = {reinterpret_cast<const float *>(staged + piece.skew()), piece.q, piece.scale, (int)(piece.bytes / piece.unit)};
         rows.cols = (int)(piece.unit / sizeof(float));
     }
     int launch(unsigned blocks, const LinkSignals &signals, hipStream_t st)
@@ -779,17 +869,19 @@ int upload_small(Ring *r, const Source *from, int count, hipStream_t st)
 {
     size_t bytes = 0, room = 0;
     for (int i = 0; i < count; i++) {
-        bytes += from[i].bytes;
-        room += small_room(from[i].bytes);
+        bytes += from[i].link_bytes();
+        room += small_room(from[i].staged_bytes());
     }
     int rc = open_small(r, room, st);
     if (rc != VTL_HIP_OK)
         return rc;
     CopyArgs g = {};
-    for (int i = 0; i < count; i++)
-        g.seg[g.count++] = make_segment(from[i].dst,
-                                        put_small(r, from[i].src, from[i].bytes, reinterpret_cast<uintptr_t>(from[i].dst) & 15),
-                                        from[i].bytes);
+    for (int i = 0; i < count; i++) {
+        char *const staged = r->at(r->slot) + r->used;
+        from[i].stage(staged);
+        r->used += small_room(from[i].staged_bytes());
+        g.count += from[i].segments(staged, g.seg + g.count);
+    }
     hipLaunchKernelGGL(host_copy_kernel, dim3(copy_blocks(bytes < kSmall ? bytes : kSmall - 1)), dim3(512), 0, st, g);
     rc = check_launch("host_copy_kernel");
     if (rc == VTL_HIP_OK)
@@ -808,13 +900,16 @@ struct Pieces {
     struct Piece : Source {
         std::atomic<int> left{0};
         bool last_of_launch;
-        size_t skew() const { return reinterpret_cast<uintptr_t>(dst) & 15; }
     };
     std::unique_ptr<Piece[]> piece;
     int count = 0;
 
-    Pieces(const Source *from, int sources)
+    // `host`: the host makes codes of (some of) it, and not the link but the host is what it waits for: launches of one slot at most,
+    // and ever smaller ones at the end, where the link has to carry what the threads made last.
+    Pieces(const Source *from, int sources, bool host)
     {
+        const size_t most = host ? kSlotBytes : kMaxSegments * kSlotBytes;
+        const int pieces = host ? kMaxSegments / 2 : kMaxSegments;   // of a launch (codes take two segments)
         for (int pass = 0; pass < 2; pass++) {
             size_t ahead = 0, launch = kFirstLaunch, room = launch;
             for (int s = 0; s < sources; s++)
@@ -822,7 +917,9 @@ struct Pieces {
             int n = 0, in_launch = 0;
             for (int s = 0; s < sources; s++)
                 for (size_t at = 0; at < from[s].bytes;) {
-                    if (in_launch == 0 && ahead < launch + launch / 2)   // no small launch at the end
+                    if (in_launch == 0 && host)
+                        room = ahead < 2 * kFirstLaunch ? ahead : ahead / 3 < kFirstLaunch ? kFirstLaunch : ahead / 3 < launch ? ahead / 3 : launch;
+                    else if (in_launch == 0 && ahead < launch + launch / 2)   // no small launch at the end
                         room = ahead;
                     size_t take = from[s].bytes - at;
                     if (take > kSlotBytes)
@@ -837,8 +934,9 @@ struct Pieces {
                         p.src = static_cast<const char *>(from[s].src) + at;
                         p.bytes = take;
                         if (p.unit) {
-                            p.q += at / sizeof(float);
-                            p.scale += at / p.unit;
+                            p.q += p.host ? at / p.unit * p.row : at / sizeof(float);
+                            if (!p.one)
+                                p.scale += at / p.unit;
                         } else {
                             p.dst = static_cast<char *>(from[s].dst) + at;
                         }
@@ -849,13 +947,13 @@ struct Pieces {
                     n++;
                     in_launch++;
                     const size_t unit = at < from[s].bytes ? from[s].unit : 0;   // of what comes next
-                    const bool end = room < (unit ? unit : 1) || in_launch == kMaxSegments || ahead == 0;
+                    const bool end = room < (unit ? unit : 1) || in_launch == pieces || ahead == 0;
                     if (pass)
                         piece[n - 1].last_of_launch = end;
                     if (end) {
                         launch = launch < kSlotBytes ? 2 * launch : (launch + launch / 2) & ~(size_t)4095;
-                        if (launch > kMaxSegments * kSlotBytes)
-                            launch = kMaxSegments * kSlotBytes;
+                        if (launch > most)
+                            launch = most;
                         room = launch;
                         in_launch = 0;
                     }
@@ -867,17 +965,19 @@ struct Pieces {
     }
 };
 
+// Of whole rows.
+size_t job_bytes(size_t unit) { return unit > Crew::kJobBytes ? unit : Crew::kJobBytes - Crew::kJobBytes % unit; }
+
 // The host threads fill slots while the link empties the ones before them.  launch(first, n, slot of the
 // first, last): pieces first .. first + n - 1, in as many consecutive slots.
 template <typename Launch>
-int send_pieces(Ring *r, Pieces &c, hipStream_t st, Launch launch)
+int send_pieces(Ring *r, Pieces &c, hipStream_t st, Launch launch)   // between Crew::begin() and end()
 {
     int rc = r->close(st);
     if (rc != VTL_HIP_OK)
         return rc;
     const int n = c.count, s0 = r->slot;
     Crew &crew = Crew::instance();
-    crew.begin();
     int pushed = 0, issued = 0;
     while (issued < n && rc == VTL_HIP_OK) {
         int end = issued;
@@ -893,7 +993,12 @@ int send_pieces(Ring *r, Pieces &c, hipStream_t st, Launch launch)
                     break;
             }
             Pieces::Piece &p = c.piece[pushed];
-            crew.push(r->at(slot) + p.skew(), static_cast<const char *>(p.src), p.bytes, p.left);
+            char *const staged = r->at(slot);
+            if (p.host)
+                crew.push(staged + p.skew(), static_cast<const char *>(p.src), p.bytes, p.left, &p,
+                          p.one ? nullptr : reinterpret_cast<float *>(staged + p.scales_at()), job_bytes(p.unit));
+            else
+                crew.push(staged + p.skew(), static_cast<const char *>(p.src), p.bytes, p.left);
             pushed++;
         }
         for (int i = issued; i < end && rc == VTL_HIP_OK; i++)
@@ -907,21 +1012,30 @@ int send_pieces(Ring *r, Pieces &c, hipStream_t st, Launch launch)
         crew.finish(c.piece[i].left);
     if (rc != VTL_HIP_OK)
         r->give_up(st);
-    crew.end();
     r->slot = (s0 + n) % kSlots;
     return rc;
 }
 
-int upload_large(Ring *r, const Source *from, int count, hipStream_t st)
+// A transfer that host threads share, for the length of a scope.
+struct CrewWork {
+    Crew &crew = Crew::instance();
+    explicit CrewWork(bool more) { crew.begin(more); }
+    ~CrewWork() { crew.end(); }
+    CrewWork(const CrewWork &) = delete;
+    CrewWork &operator=(const CrewWork &) = delete;
+};
+
+int upload_large(Ring *r, const Source *from, int count, hipStream_t st, bool host = false)
 {
-    Pieces c(from, count);
+    Pieces c(from, count, host);
+    const CrewWork work(host && from[count - 1].bytes >= kManyHelpersFrom);
     return send_pieces(r, c, st, [&](int first, int n, int slot, bool last) {
         Load load;
         size_t bytes = 0;
         for (int i = 0; i < n; i++) {
             const Pieces::Piece &p = c.piece[first + i];
-            load.add(p, r->at((slot + i) % kSlots) + p.skew());
-            bytes += p.bytes;
+            load.add(p, r->at((slot + i) % kSlots));
+            bytes += p.link_bytes();
         }
         const unsigned blocks = copy_blocks(bytes < kSmall ? bytes : kSmall - 1);
         const int rc = load.launch(blocks, r->signals_for(slot, blocks, last, false), st);
@@ -1102,12 +1216,70 @@ try {
     if (!r)
         return false;
     const size_t unit = (size_t)cols * sizeof(float);
-    const Source from[2] = {{nullptr, src, (size_t)rows * unit, q, scale, unit}, {extra_dst, extra_src, extra_bytes}};
+    const Quantized codes = {q, scale, unit};
+    const Source from[2] = {{nullptr, src, (size_t)rows * unit, codes}, {extra_dst, extra_src, extra_bytes}};
     const int count = extra_bytes ? 2 : 1;
     std::lock_guard<std::mutex> hold(r->lock);
     status = upload_large(r, from, count, st);
     if (status == VTL_HIP_OK && !one_stream && hipStreamSynchronize(st) != hipSuccess)   // the ring's slots are shared by all streams
         status = record_hip_error(hipErrorUnknown, "upload_rows_kernel");
+    return true;
+} catch (const std::exception &) {
+    status = VTL_HIP_ERR_OUT_OF_MEMORY;
+    return true;
+}
+
+// The host makes codes of f32 rows, and the link carries those: 180 MB of weights with their scales and the forward behind them 3640 -> 1480 us, 4 MiB
+// of activations through three layers 208 -> 157, 200 KB 28.7 -> 25.4 (16 processors).  Only above so many processors that the
+// caller and its helpers are about half of them: with fewer, memory is what a copy and the codes wait for alike (8 processors, GB/s of f32 by 4
+// threads: copied 35, quantized 32).
+constexpr int kQuantizeProcessors = 2 * Crew::kHelpers;
+
+bool upload_codes(const float *src, int64_t rows, int64_t cols, int per_row, int8_t *q, int64_t row, float *scale, void *extra_dst,
+                  const void *extra_src, size_t extra_bytes, int &status)
+try {
+    static const bool many = processors() > kQuantizeProcessors;
+    const int asked = tuning().host_quantize;
+    const HostQuantizer *host = (asked < 0 ? many : asked != 0) ? host_quantizer() : nullptr;
+    hipStream_t st = current_stream();
+    const bool one_stream = single_stream();
+    const size_t unit = (size_t)cols * sizeof(float), bytes = (size_t)rows * unit;
+    // (a slot has room for a row, and for the codes and scales of as many bytes of f32)
+    if (!host || rows < 1 || cols < kCodesLeastCols || unit > kSlotBytes || (size_t)row + sizeof(float) > unit || extra_bytes > kWithAnother ||
+        (!one_stream && stream_is_capturing(st)))
+        return false;
+    const OwnerDevice owner(q, extra_bytes ? extra_dst : nullptr);
+    Ring *r = owner.kernels() && owner.holds(scale) ? ring_of_current_device() : nullptr;
+    if (!r)
+        return false;
+    Quantized codes = {q, scale, unit, host, (size_t)row, !per_row};
+    std::lock_guard<std::mutex> hold(r->lock);
+    std::unique_ptr<CrewWork> work;        // of the scale of all rows
+    const char *const x = reinterpret_cast<const char *>(src);
+    if (bytes > kSmall && !per_row)
+        work.reset(new CrewWork(bytes >= kManyHelpersFrom));
+    float most = 0.0f;
+    if (!per_row) {
+        if (work) {
+            std::atomic<int> left{0};
+            work->crew.push(nullptr, x, bytes, left, &codes, &most);
+            work->crew.finish(left);
+        } else {
+            most = host->absmax(src, rows * cols);
+        }
+        codes.given = host->scale(most);
+    }
+    // the scale of all rows and the extra bytes in front: what the host makes last is then carried by a small launch
+    Source from[3];
+    int count = 0;
+    if (extra_bytes)
+        from[count++] = {extra_dst, extra_src, extra_bytes};
+    if (!per_row)
+        from[count++] = {scale, &codes.given, sizeof(float)};
+    from[count++] = {nullptr, src, bytes, codes};
+    status = bytes > kSmall ? upload_large(r, from, count, st, true) : upload_small(r, from, count, st);
+    if (status == VTL_HIP_OK && !one_stream && hipStreamSynchronize(st) != hipSuccess)   // the ring's slots are shared by all streams
+        status = record_hip_error(hipErrorUnknown, "host_copy_kernel");
     return true;
 } catch (const std::exception &) {
     status = VTL_HIP_ERR_OUT_OF_MEMORY;

@@ -142,6 +142,7 @@ static const Tuning *read_tuning(bool force)
     t->skinny_tiled = number("VTL_HIP_SKINNY_TILED", -1);
     t->skinny_waves = number("VTL_HIP_SKINNY_WAVES", 4);
     t->matmul_tile = number("VTL_HIP_MATMUL_TILE", 0);
+    t->host_quantize = number("VTL_HIP_HOST_QUANTIZE", -1);
     t->backward_group = number("VTL_HIP_BACKWARD_GROUP", -1);
     t->matmul_splits = number("VTL_HIP_MATMUL_SPLITS", -1);
     g_tuning.store(t, std::memory_order_release);

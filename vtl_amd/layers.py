@@ -102,9 +102,8 @@ def content_fingerprint(t: np.ndarray) -> int:
     return h.value
 
 
-# Weights of this many bytes and more go to the call that quantizes them as they come over the link where it can (rows of 2048 to
-# 8192 values), and takes the bias along.
-_QUANTIZED_FROM = 32 << 20
+# Weights of this many bytes and more go to the call that quantizes them on their way to the device, and takes the bias along.
+_QUANTIZED_FROM = 2 << 20
 
 
 class QuantizedWeights:
@@ -152,11 +151,12 @@ class QuantizedWeights:
             b = np.ascontiguousarray(b)
             self.bias = HipTensor.empty(b.shape, np.float32, params)
             extra = (self.bias.ptr, b.ctypes.data, b.nbytes)
-        if mode == PER_CHANNEL and w.nbytes >= _QUANTIZED_FROM:
+        if w.nbytes >= _QUANTIZED_FROM:
+            per_row = mode == PER_CHANNEL
             self.w_q = HipTensor.empty(w.shape, np.int8, params)
-            self.sw = HipTensor.empty([self.out_features], np.float32, params)
-            capi.call("vtl_hip_upload_quantized", w.ctypes.data, self.out_features, self.in_features, 1, self.w_q.ptr, self.sw.ptr,
-                      *extra)
+            self.sw = HipTensor.empty([self.out_features if per_row else 1], np.float32, params)
+            capi.call("vtl_hip_upload_quantized", w.ctypes.data, self.out_features, self.in_features, int(per_row), self.w_q.ptr,
+                      self.sw.ptr, *extra)
         else:
             w_dev = HipTensor.empty(w.shape, np.float32, params)
             try:
