@@ -47,22 +47,29 @@ int8_t code(float x, float scale)
 // Whether scale and 1 / scale are normal numbers with headroom.
 bool by_estimate(float scale) { return scale >= 0x1p-100f && scale <= 0x1p100f; }
 
+#define VTL_AVX512 __attribute__((target("avx512f,avx512bw,avx512vl,avx512dq")))
+#define VTL_AVX2 __attribute__((target("avx2")))
+
+// The largest magnitude of n values (NaNs are passed over: of a NaN and a number the maximum is the second operand), and their codes
+// where an estimated quotient decides; the others are made again.
 struct Avx512 {
-    static constexpr int kStep = 64;
-    // NaNs are passed over: of a NaN and a number the maximum is the second operand.
-    __attribute__((target("avx512f,avx512bw,avx512vl,avx512dq"))) static float absmax(const float *x, int64_t n)
+    VTL_AVX512 static __mmask16 lanes(int64_t left) { return left >= 16 ? (__mmask16)0xffff : (__mmask16)((1u << left) - 1); }
+    VTL_AVX512 static float absmax(const float *x, int64_t n)
     {
         __m512 m[4] = {_mm512_setzero_ps(), _mm512_setzero_ps(), _mm512_setzero_ps(), _mm512_setzero_ps()};
-        for (int64_t i = 0; i < n; i += kStep)
+        int64_t i = 0;
+        for (; i + 64 <= n; i += 64)
             for (int j = 0; j < 4; j++)
                 m[j] = _mm512_max_ps(_mm512_abs_ps(_mm512_loadu_ps(x + i + 16 * j)), m[j]);
+        for (; i < n; i += 16)
+            m[0] = _mm512_max_ps(_mm512_abs_ps(_mm512_maskz_loadu_ps(lanes(n - i), x + i)), m[0]);
         return _mm512_reduce_max_ps(_mm512_max_ps(_mm512_max_ps(m[0], m[1]), _mm512_max_ps(m[2], m[3])));
     }
-    // Codes where an estimate decides; the others are made again.
-    __attribute__((target("avx512f,avx512bw,avx512vl,avx512dq"))) static void codes(const float *x, int64_t n, int8_t *q, float scale)
+    VTL_AVX512 static void codes(const float *x, int64_t n, int8_t *q, float scale)
     {
         const __m512 inv = _mm512_set1_ps(1.0f / scale), tie = _mm512_set1_ps(kTie);
-        for (int64_t i = 0; i < n; i += kStep) {
+        int64_t i = 0;
+        for (; i + 64 <= n; i += 64) {
             uint64_t near = 0;
             for (int j = 0; j < 4; j++) {
                 const __m512 t = _mm512_mul_ps(_mm512_loadu_ps(x + i + 16 * j), inv);
@@ -70,85 +77,83 @@ struct Avx512 {
                 near |= (uint64_t)_mm512_cmp_ps_mask(_mm512_abs_ps(_mm512_sub_ps(t, r)), tie, _CMP_NLT_UQ) << (16 * j);   // (a NaN too)
                 _mm_storeu_si128(reinterpret_cast<__m128i *>(q + i + 16 * j), _mm512_cvtsepi32_epi8(_mm512_cvtps_epi32(r)));
             }
-            for (; __builtin_expect(near != 0, 0); near &= near - 1) {
-                const int64_t at = i + __builtin_ctzll(near);
-                q[at] = code(x[at], scale);
-            }
+            again(x + i, q + i, near, scale);
         }
+        for (; i < n; i += 16) {
+            const __mmask16 in = lanes(n - i);
+            const __m512 t = _mm512_mul_ps(_mm512_maskz_loadu_ps(in, x + i), inv);
+            const __m512 r = _mm512_roundscale_ps(t, _MM_FROUND_TO_NEAREST_INT | _MM_FROUND_NO_EXC);
+            _mm_mask_storeu_epi8(q + i, in, _mm512_cvtsepi32_epi8(_mm512_cvtps_epi32(r)));
+            again(x + i, q + i, _mm512_mask_cmp_ps_mask(in, _mm512_abs_ps(_mm512_sub_ps(t, r)), tie, _CMP_NLT_UQ), scale);
+        }
+    }
+    static void again(const float *x, int8_t *q, uint64_t which, float scale)
+    {
+        for (; __builtin_expect(which != 0, 0); which &= which - 1)
+            q[__builtin_ctzll(which)] = code(x[__builtin_ctzll(which)], scale);
     }
 };
 
+// What is beyond whole steps of 32 is a step that ends with the row; rows shorter than one are made value by value.
 struct Avx2 {
-    static constexpr int kStep = 32;
-    __attribute__((target("avx2"))) static float absmax(const float *x, int64_t n)
+    VTL_AVX2 static float absmax(const float *x, int64_t n)
     {
+        float most = 0.0f;
+        if (n < 32) {
+            for (int64_t i = 0; i < n; i++)
+                most = __builtin_fabsf(x[i]) > most ? __builtin_fabsf(x[i]) : most;
+            return most;
+        }
         const __m256 magnitude = _mm256_castsi256_ps(_mm256_set1_epi32(0x7fffffff));
         __m256 m[4] = {_mm256_setzero_ps(), _mm256_setzero_ps(), _mm256_setzero_ps(), _mm256_setzero_ps()};
-        for (int64_t i = 0; i < n; i += kStep)
+        for (int64_t i = 0; i < n; i += 32) {
+            const float *at = x + (i + 32 <= n ? i : n - 32);
             for (int j = 0; j < 4; j++)
-                m[j] = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(x + i + 8 * j), magnitude), m[j]);
-        float lane[8], most = 0.0f;
+                m[j] = _mm256_max_ps(_mm256_and_ps(_mm256_loadu_ps(at + 8 * j), magnitude), m[j]);
+        }
+        float lane[8];
         _mm256_storeu_ps(lane, _mm256_max_ps(_mm256_max_ps(m[0], m[1]), _mm256_max_ps(m[2], m[3])));
         for (float v : lane)
             most = v > most ? v : most;
         return most;
     }
-    __attribute__((target("avx2"))) static void codes(const float *x, int64_t n, int8_t *q, float scale)
+    VTL_AVX2 static void codes(const float *x, int64_t n, int8_t *q, float scale)
     {
+        if (n < 32) {
+            for (int64_t i = 0; i < n; i++)
+                q[i] = code(x[i], scale);
+            return;
+        }
         const __m256 magnitude = _mm256_castsi256_ps(_mm256_set1_epi32(0x7fffffff));
         const __m256 inv = _mm256_set1_ps(1.0f / scale), tie = _mm256_set1_ps(kTie);
         const __m256i order = _mm256_setr_epi32(0, 4, 1, 5, 2, 6, 3, 7);
-        for (int64_t i = 0; i < n; i += kStep) {
+        for (int64_t i = 0; i < n; i += 32) {
+            const int64_t at = i + 32 <= n ? i : n - 32;
             __m256i c[4];
             unsigned near = 0;
             for (int j = 0; j < 4; j++) {
-                const __m256 t = _mm256_mul_ps(_mm256_loadu_ps(x + i + 8 * j), inv);
+                const __m256 t = _mm256_mul_ps(_mm256_loadu_ps(x + at + 8 * j), inv);
                 const __m256 r = _mm256_round_ps(t, _MM_FROUND_TO_NEAREST_INT | _MM_FROUND_NO_EXC);
                 near |= (unsigned)_mm256_movemask_ps(_mm256_cmp_ps(_mm256_and_ps(_mm256_sub_ps(t, r), magnitude), tie, _CMP_NLT_UQ)) << (8 * j);
                 c[j] = _mm256_cvtps_epi32(r);
             }
             const __m256i all = _mm256_packs_epi16(_mm256_packs_epi32(c[0], c[1]), _mm256_packs_epi32(c[2], c[3]));
-            _mm256_storeu_si256(reinterpret_cast<__m256i *>(q + i), _mm256_permutevar8x32_epi32(all, order));
-            for (; __builtin_expect(near != 0, 0); near &= near - 1) {
-                const int64_t at = i + __builtin_ctz(near);
-                q[at] = code(x[at], scale);
-            }
+            _mm256_storeu_si256(reinterpret_cast<__m256i *>(q + at), _mm256_permutevar8x32_epi32(all, order));
+            for (; __builtin_expect(near != 0, 0); near &= near - 1)
+                q[at + __builtin_ctz(near)] = code(x[at + __builtin_ctz(near)], scale);
         }
     }
 };
 
-// Whole steps by V, the rest of a row in a step of its own with zeros behind it.
-template <typename V>
-float absmax_of(const float *x, int64_t n)
-{
-    const int64_t whole = n - n % V::kStep;
-    float m = V::absmax(x, whole);
-    if (whole < n) {
-        float rest[V::kStep] = {};
-        memcpy(rest, x + whole, (size_t)(n - whole) * sizeof(float));
-        const float more = V::absmax(rest, V::kStep);
-        m = more > m ? more : m;
-    }
-    return m;
-}
-
 template <typename V>
 void codes_of(const float *x, int64_t n, int8_t *q, float scale)
 {
-    if (!by_estimate(scale)) {
-        for (int64_t i = 0; i < n; i++)
-            q[i] = code(x[i], scale);
+    if (by_estimate(scale)) {
+        V::codes(x, n, q, scale);
         return;
     }
-    const int64_t whole = n - n % V::kStep;
-    V::codes(x, whole, q, scale);
-    if (whole < n) {
-        float rest[V::kStep] = {};
-        int8_t some[V::kStep];
-        memcpy(rest, x + whole, (size_t)(n - whole) * sizeof(float));
-        V::codes(rest, V::kStep, some, scale);
-        memcpy(q + whole, some, (size_t)(n - whole));
-    }
+    for (int64_t i = 0; i < n; i++)
+        q[i] = code(x[i], scale);
 }
 
 template <typename V>
@@ -167,7 +172,7 @@ void rows_of(const float *x, int64_t rows, int64_t cols, int8_t *q, int64_t row,
 {
     const DefaultFloats mode;
     for (int64_t r = 0; r < rows; r++, x += cols, q += row) {
-        scales[r] = absmax_of<V>(x, cols) / 127.0f;
+        scales[r] = V::absmax(x, cols) / 127.0f;
         codes_of<V>(x, cols, q, scales[r]);
         memset(q + cols, 0, (size_t)(row - cols));
     }
@@ -179,7 +184,7 @@ float absmax(const float *x, int64_t count)
     float m;
     {
         const DefaultFloats mode;
-        m = absmax_of<V>(x, count);
+        m = V::absmax(x, count);
         asm volatile("" : "+m"(m));
     }
     return m;

@@ -102,8 +102,10 @@ def content_fingerprint(t: np.ndarray) -> int:
     return h.value
 
 
-# Weights of this many bytes and more go to the call that quantizes them on their way to the device, and takes the bias along.
-_QUANTIZED_FROM = 2 << 20
+# Weights of up to so many bytes, which one host thread makes codes of, and from so many on, which several do, go to the call that quantizes
+# them on their way to the device and takes the bias along.  (us of a forward, uploaded and then quantized, and so: 16 x 256 x 256 46 and 42,
+# 64 x 512 x 512 80 and 63, 64 x 600 x 1024 118 and 82.)
+_QUANTIZED_UP_TO, _QUANTIZED_FROM = 1 << 20, 2 << 20
 
 
 class QuantizedWeights:
@@ -151,7 +153,7 @@ class QuantizedWeights:
             b = np.ascontiguousarray(b)
             self.bias = HipTensor.empty(b.shape, np.float32, params)
             extra = (self.bias.ptr, b.ctypes.data, b.nbytes)
-        if w.nbytes >= _QUANTIZED_FROM:
+        if 0 < w.nbytes <= _QUANTIZED_UP_TO or w.nbytes >= _QUANTIZED_FROM:
             per_row = mode == PER_CHANNEL
             self.w_q = HipTensor.empty(w.shape, np.int8, params)
             self.sw = HipTensor.empty([self.out_features if per_row else 1], np.float32, params)
