@@ -408,3 +408,26 @@ def test_rows_that_are_padded(hip, guard_bands, m, n, k):
     assert np.array_equal(c.cpu(), oracle.gemm_i8_i32(a, w, threads=CPU_THREADS))
     for t in (da, dw, c):
         t.release()
+
+
+# Either side of where one workgroup per 32x32 tile is taken (256 and 512 tiles, rows of 256 and 3400), of its rounds of loads (K = 1024, 2048) and of
+# the waves' shares of a tile; with codes for the next layer up to 1024 columns and K = 512, 2048
+@pytest.mark.parametrize("mnk", [(250, 1024, 1008), (256, 1024, 3392), (257, 1024, 784), (256, 1028, 3408), (500, 1024, 240), (513, 1020, 240),
+                                 (512, 1024, 256), (33, 100, 1040), (64, 1000, 2064), (128, 1024, 512), (129, 1024, 528), (65, 1024, 2048),
+                                 (65, 1028, 2032), (40, 4, 16), (256, 1024, 1600), (99, 252, 4096), (90, 250, 4112)])
+def test_small_products_at_the_edges_of_their_rule(hip, mnk):
+    m, n, k = mnk
+    a, bt, sa, sb, bias = workloads.square_int8_gemm(m, n, k, seed=m * 31 + n * 3 + k)
+    ref = oracle.gemm_i8_i32(a, bt, threads=CPU_THREADS)
+    print(mnk, flush=True)
+    assert np.array_equal(_gemm(a, bt), ref)
+    A, B, dsa, dsb, dbias = dev(a), dev(bt), dev(sa), dev(sb), dev(bias)
+    want = oracle.epilogue(ref, sa, sb, bias, relu=True)
+    y = linear_i8_hip(A, dsa, B, dsb, dbias, relu=True)
+    assert np.array_equal(y.cpu(), want)
+    q, s = HipTensor.empty([m, n], np.int8), HipTensor.empty([m], np.float32)
+    capi.call("vtl_hip_linear_i8_requant", A.ptr, dsa.ptr, 1, B.ptr, dsb.ptr, 1, dbias.ptr, 1, q.ptr, s.ptr, None, m, n, k)
+    want_q, want_s = oracle.quantize(want, True)
+    assert np.array_equal(q.cpu(), want_q) and np.array_equal(s.cpu(), want_s)
+    for h in (A, B, dsa, dsb, dbias, y, q, s):
+        h.release()

@@ -1782,11 +1782,8 @@ int launch_pad_rows(const int8_t *a, int64_t a_rows, int8_t *a_dst, const int8_t
 // Small products (up to a few hundred 32x32 output tiles): nothing is reused
 // often enough to stage, so each wave feeds the MFMA straight from global memory.
 // One workgroup per 32x32 tile; its NW waves take groups of four K steps (a cache line
-// of every row) in turn, U steps of loads in flight per wave, and the partial tiles meet in LDS.  With sixteen waves a
-// tile with K = 4096 is two rounds of loads per wave, so a product like
-// 256x1024x4096 (256 tiles, one per compute unit) is one launch whose length is
-// a couple of memory latencies, instead of a K-split launch plus the pass that
-// adds the partial sums.  Needs K % 16 == 0 and 16-byte aligned operands; RAGGED takes any K and
+// of every row) in turn, U steps of loads in flight per wave, and the partial tiles meet in LDS: a launch whose length is
+// a couple of memory latencies.  Needs K % 16 == 0 and 16-byte aligned operands; RAGGED takes any K and
 // any address.
 template <bool F32OUT, int NW, int U, bool RAGGED = false>
 __global__ __launch_bounds__(64 * NW) void gemm_i8_small_kernel(const GemmArgs g)
@@ -1802,6 +1799,19 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_small_kernel(const GemmArgs g
     const int8_t *__restrict__ ap = g.A + (int64_t)arow * g.K + (RAGGED ? 0 : 16 * half);
     const int8_t *__restrict__ bp = g.Bt + (int64_t)brow * g.K + (RAGGED ? 0 : 16 * half);
     const int steps = (g.K + 31) / 32;
+    // This thread's outputs, registers wave, wave + NW, ... of accumulator lane `lane` (register reg: row 8 * (reg / 4) + 4 * (lane / 32) + reg % 4, column
+    // lane % 32).  Their scales and bias are asked for now: read behind the sums they add a memory latency to the launch (64 x 784 -> 256 3.96 -> 3.68 us).
+    constexpr int OUT = 16 / NW;
+    const int n = n0 + r;
+    auto row_of = [&](int i) { return m0 + 8 * ((wave + NW * i) >> 2) + 4 * half + ((wave + NW * i) & 3); };
+    float sa[OUT], sw = 0.0f, bias = 0.0f;
+    if constexpr (F32OUT) {
+        sw = g.sw[(int64_t)brow * g.sw_stride];
+        bias = g.bias ? g.bias[brow] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < OUT; ++i)
+            sa[i] = g.sa[(int64_t)min(row_of(i), g.M - 1) * g.sa_stride];
+    }
     v16i acc;
 #pragma unroll
     for (int i = 0; i < 16; ++i)
@@ -1847,22 +1857,21 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_small_kernel(const GemmArgs g
     for (int i = 0; i < 16; ++i)
         red[wave][i][lane] = acc[i];
     __syncthreads();
-    for (int o = threadIdx.x; o < 1024; o += 64 * NW) {
-        const int reg = o >> 6, l = o & 63;
+#pragma unroll
+    for (int i = 0; i < OUT; ++i) {
         int sum = 0;
 #pragma unroll
         for (int w = 0; w < NW; ++w)
-            sum += red[w][reg][l];
-        // accumulator register reg of lane l: row 8 * (reg / 4) + 4 * (l / 32) + reg % 4, column l % 32
-        const int m = m0 + 8 * (reg >> 2) + 4 * (l >> 5) + (reg & 3), n = n0 + (l & 31);
+            sum += red[w][wave + NW * i][lane];
+        const int m = row_of(i);
         if (m >= g.M || n >= g.N)
             continue;
         const int64_t idx = (int64_t)m * g.N + n;
-        if (F32OUT) {
-            const float sc = g.sa[(int64_t)m * g.sa_stride] * g.sw[(int64_t)n * g.sw_stride];
+        if constexpr (F32OUT) {
+            const float sc = sa[i] * sw;
             float y = (float)sum * sc;
             if (g.bias)
-                y = y + g.bias[n];
+                y = y + bias;
             if (g.relu && y < 0.0f)
                 y = 0.0f;
             store_result(reinterpret_cast<float *>(g.out) + idx, y, g.done);
@@ -2531,31 +2540,27 @@ inline bool short_rows_fused_faster(int M, int N, int K, Rows rows, bool over_li
     return N <= (M == 2 ? 16384 : (M <= 4 ? 8192 : 2048));
 }
 
-// Where one workgroup per 32x32 tile, fed straight from global memory, beats the tile kernels:
-// few tiles and a short K (nothing to stage), and up to a chip's worth of tiles with a long K,
-// which the tile kernels could only fill the chip with by cutting K (a second launch).
-inline bool small_product_faster(int64_t t32, int K)
-{
-    // (up to 128 tiles below K = 1024, where the 32 x 32-block route does not go: 256 x 512 x 512
-    // 3.8 against 4.5 us on the tile kernels)
-    return (t32 <= 64 && K <= 2048) || (t32 <= 128 && K < 1024);
-}
-inline int small_product_waves(int64_t t32, int K)
-{
-    (void)t32;
-    return K <= 2048 ? 4 : (K <= 4096 ? 8 : 16);
-}
+// Where one workgroup per 32x32 tile, fed straight from global memory, beats the tile kernels (and K in ranges, which takes a second
+// launch): while every tile has a compute unit of its own and few waits for memory, or two have and the sum is one wait (us on the device, tile kernels and
+// this one: 250 x 640 x 256 4.0 and 3.2, x 784 5.3 and 3.6, x 2000 7.6 and 5.2, x 2608 8.9 and 6.7; 256 x 1024 x 512 4.1 and 3.7, x 3312 11.0 and 9.0, x 4016 12.0 and
+// 10.2; 64 x 4000 x 3312 11.0 and 10.1; but 32 x 1024 x 4016, in K ranges, 8.0 and 9.6.  300 x 1024 x 160 4.1 and 3.2, 256 x 2048 x 128 3.6 and 3.5, x 256 3.8 and
+// 3.9; 1024 x 640 x 128 3.7 and 3.9).
+inline bool small_product_faster(int64_t t32, int K) { return (t32 <= 256 && K <= 3400) || (t32 <= 512 && K < 256); }
 
 template <bool F32OUT, bool RAGGED>
 int launch_small(GemmArgs g, int64_t t32, int waves, hipStream_t st)
 {
+    // Eight waves of four steps: one round of loads up to K = 1024 (64 x 784 -> 256 3.7 us with four waves, 3.3; 48 x 1536 -> 300 4.2 and
+    // 3.8), beyond 2048 twice as many in flight.  Ragged rows, whose loads take more registers, start that earlier, and short ones are few waves' work.
     const dim3 grid((unsigned)t32);
     attach_result(g, grid.x);
     if (waves >= 16)
         hipLaunchKernelGGL((gemm_i8_small_kernel<F32OUT, 16, 8, RAGGED>), grid, dim3(1024), 0, st, g);
-    else if (waves >= 8)
+    else if (waves >= 8 && g.K > (RAGGED ? 1024 : 2048))
         hipLaunchKernelGGL((gemm_i8_small_kernel<F32OUT, 8, 8, RAGGED>), grid, dim3(512), 0, st, g);
-    else
+    else if (waves >= 8)
+        hipLaunchKernelGGL((gemm_i8_small_kernel<F32OUT, 8, 4, RAGGED>), grid, dim3(512), 0, st, g);
+    else if constexpr (RAGGED)
         hipLaunchKernelGGL((gemm_i8_small_kernel<F32OUT, 4, 4, RAGGED>), grid, dim3(256), 0, st, g);
     return check_launch("gemm_i8_small_kernel");
 }
@@ -2611,12 +2616,11 @@ int launch_gemm(const GemmArgs &g_in, hipStream_t st)
             return launch_skinny<F32OUT>(g, nwave == 2 ? 2 : 4, st);
     }
     const int64_t t32 = (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32);
-    // VTL_HIP_GEMM_SMALL 1 / 0 forces the choice (tests, tuning); 4, 8, 16 also the number of waves
+    // VTL_HIP_GEMM_SMALL 1 / 0 forces the choice (tests, tuning); 16 also the number of waves
     if (small_set ? tn.gemm_small != 0 : small_product_faster(t32, g.K)) {
         if (t32 > 0x7fffffff)
             return VTL_HIP_ERR_UNSUPPORTED;
-        const int nw = tn.gemm_small >= 4 ? tn.gemm_small : small_product_waves(t32, g.K);
-        return launch_small<F32OUT, false>(g, t32, nw, st);
+        return launch_small<F32OUT, false>(g, t32, tn.gemm_small >= 16 || g.K > 4096 ? 16 : 8, st);
     }
     int idx, splits;
     choose_config(g.M, g.N, g.K, idx, splits);
