@@ -2927,6 +2927,23 @@ int vtl_hip_linear_i8_requant(const int8_t *A, const float *sa, int sa_per_row, 
         if (!separate_faster) {
             g.requant_codes = Yq;
             g.requant_scales = sy;
+            // The sums by the kernels that launch_gemm has for small products, whose sums need no scratch of their own.  Up to 1024 columns: beyond, and of
+            // longer rows, the tile kernels' cheaper stores are what the row kernel gains (us, tile kernels and these: 33 x 256 x 784 7.8 and 6.1, 64 x 512 x 1600 8.1
+            // and 6.3, 128 x 1024 x 512 6.4 and 5.7, 256 x 1024 x 1600 10.5 and 9.3; but 256 x 512 x 512 5.9 and 6.4, 64 x 512 x 3072 8.1 and 9.3, 64 x 3200 x 512 6.7 and
+            // 7.0).
+            const int64_t t32 = (int64_t)((M + 31) / 32) * ((N + 31) / 32);
+            if (!config_set && tn.requant_wide <= 0 &&
+                (tn.gemm_small >= 0 ? tn.gemm_small != 0 && t32 <= 0x7fffffff
+                                    : N <= 1024 && K <= 2048 && (K > 512 || M <= 128) && small_product_faster(t32, K))) {
+                g.partials = static_cast<int32_t *>(vtlhip::library_workspace((size_t)M * (size_t)N * sizeof(int32_t)));
+                if (!g.partials)
+                    return vtlhip::workspace_status();
+                GemmArgs sums = g;
+                sums.out = g.partials;
+                sums.requant_codes = nullptr;
+                st = launch_gemm<false>(sums, current_stream());
+                return st != VTL_HIP_OK ? st : launch_finalize_requant(g, current_stream());
+            }
             return launch_config<true>(idx, g, splits, current_stream());
         }
     }
