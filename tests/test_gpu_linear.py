@@ -623,3 +623,45 @@ def test_layers_whose_weights_get_padded_rows(hip, m, n, k):
     assert np.array_equal(net.forward(x, no_grad=True),
                           oracle.linear_f32_dynquant(hidden, w2q, sw2, np.zeros(1000, np.float32)))
     net.release()
+
+
+# Rows quantized by the workgroup of each tile: edges of tiles, of its rounds of values (256, 512, 768) and of its rule (256 and 512 tiles, K = 400 and 768),
+# whole and padded weight rows, rows that start anywhere, values that are no numbers
+@pytest.mark.parametrize("mnk", [(9, 300, 256), (33, 100, 272), (32, 3000, 256), (64, 1000, 512), (65, 31, 528), (100, 2047, 768), (128, 1024, 784), (250, 1030, 400),
+                                 (500, 1024, 400), (512, 1025, 400), (2, 2000, 64), (40, 4, 16), (70, 1200, 767), (70, 1200, 385), (33, 2000, 241),
+                                 (16, 1000, 768)])
+def test_rows_quantized_by_each_tile(hip, mnk):
+    m, n, k = mnk
+    rng = np.random.default_rng(m * 7 + n * 3 + k)
+    x = rng.standard_normal((m, k)).astype(np.float32) * np.float32(10.0) ** rng.integers(-3, 4, (m, 1)).astype(np.float32)
+    x[m // 2] = 0.0
+    x[m // 3, :: 7] = np.nan
+    w = rng.standard_normal((n, k)).astype(np.float32)
+    bias = rng.standard_normal(n).astype(np.float32)
+    print(mnk, flush=True)
+    wq, sw = oracle.quantize(w, True)
+    want = oracle.linear_f32_dynquant(x, wq, sw, bias)
+    layer = QuantLinearLayer(w, bias.reshape(1, n), requires_grad=False)
+    room = HipTensor.from_host(np.concatenate([np.zeros(1, np.float32), x.reshape(-1)]))
+    got = layer.forward_device(HipTensor.from_host(x))
+    assert np.array_equal(got.cpu(), want, equal_nan=True)
+    y = HipTensor.empty([m, n], np.float32)
+    qw = layer.quantized()
+    capi.call("vtl_hip_layer_f32", C.byref(qw.layer), room.ptr + 4, y.ptr, m, 1, None, 0)
+    assert np.array_equal(y.cpu(), np.where(want < 0, np.float32(0), want), equal_nan=True)
+    layer.release()
+
+
+@pytest.mark.parametrize("rows", [9, 33, 250])
+@pytest.mark.parametrize("dims", [(300, 512, 640, 40), (784, 700, 1024, 1100, 10), (64, 2000, 384, 384)])
+def test_layers_hand_rows_on_as_values_or_codes(hip, knobs, rows, dims):
+    rng = np.random.default_rng(rows + sum(dims))
+    net = Sequential().input([dims[0]])
+    for i in range(1, len(dims)):
+        net.linear(dims[i], weights=rng.standard_normal((dims[i], dims[i - 1])).astype(np.float32))
+        if i + 1 < len(dims):
+            net.relu()
+    x = rng.standard_normal((rows, dims[0])).astype(np.float32)
+    got = net.forward(x, no_grad=True).copy()
+    knobs.setenv("VTL_HIP_NO_FUSED_DECODE", "1")     # codes from a launch of their own everywhere
+    assert np.array_equal(got, net.forward(x, no_grad=True))

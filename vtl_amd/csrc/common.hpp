@@ -285,6 +285,8 @@ int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa
 // vtl_hip_layer_f32; of one row with one scale for the weights too.  `x_on_host`: X is in pinned memory (HostInput).
 int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu, void *workspace, size_t workspace_bytes,
               HostResult *result = nullptr, bool x_on_host = false);
+// Whether layer_f32 has more than a few rows in device memory in one launch.
+bool layer_takes_rows(const vtl_hip_layer &l, int M);
 int layer_linear_i8_requant(const vtl_hip_layer &l, const int8_t *A, const float *sa, int8_t *Yq, float *sy, int M,
                             int relu, bool padded = false);
 

@@ -1883,6 +1883,102 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_small_kernel(const GemmArgs g
         raise_when_last(g.done);
 }
 
+// The same for f32 rows that are quantized on the way: a workgroup makes the codes of its 32 rows (K <= 256 * KV) itself, while the weights of its
+// tile are under way, and feeds the MFMA from LDS.  Every tile of a row of tiles does so again, out of the L2: 6 vector instructions for four
+// values, where a quantizer's launch in front is 2.5 us on the device and 3.4 on the host.  Rows of codes are 16 bytes further apart in LDS than
+// they are long: the 32 rows of an operand then start in different banks.  ROWS: kWhole, or kPadded (x rows of x_cols values anywhere).
+template <int KV, Rows ROWS>
+__global__ __launch_bounds__(512) void linear_small_kernel(const GemmArgs g)
+{
+    constexpr int NW = 8, MINE = 32 / NW, OUT = 16 / NW;
+    constexpr int STRIDE = 256 * KV + 16;
+    __shared__ union {
+        __attribute__((aligned(16))) int8_t codes[32 * STRIDE];
+        int red[NW][16][64];
+    } lds;
+    __shared__ float scales[32];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tiles_n = (g.N + 31) / 32;
+    const int m0 = (int)(blockIdx.x / tiles_n) * 32, n0 = (int)(blockIdx.x % tiles_n) * 32;
+    const int r = lane & 31, half = lane >> 5;
+    const int n = n0 + r, brow = min(n, g.N - 1);
+    const int x_cols = ROWS == kWhole ? g.K : g.x_cols;
+    // four of the tile's rows; those past the edge repeat the last one, and their results are never stored
+    f4 x[MINE][KV];
+#pragma unroll
+    for (int j = 0; j < MINE; ++j) {
+        const float *row = g.xf32 + (int64_t)min(m0 + MINE * wave + j, g.M - 1) * x_cols;
+#pragma unroll
+        for (int i = 0; i < KV; ++i) {
+            const int c = 4 * (64 * i + lane);
+            if constexpr (ROWS == kWhole)
+                x[j][i] = c < x_cols ? *reinterpret_cast<const f4 *>(row + c) : f4{0.f, 0.f, 0.f, 0.f};
+            else
+                x[j][i] = load_floats(row, c, x_cols);
+        }
+    }
+    // K steps KV * wave + 0 .. KV - 1
+    const int8_t *bp = g.Bt + (int64_t)brow * g.K + 16 * half;
+    const auto k_of = [&](int u) { return 32 * (KV * wave + u); };
+    v4i b[KV];
+#pragma unroll
+    for (int u = 0; u < KV; ++u)
+        b[u] = k_of(u) + 16 * half < g.K ? *reinterpret_cast<const v4i *>(bp + k_of(u)) : v4i{0, 0, 0, 0};
+    const float sw = g.sw[(int64_t)brow * g.sw_stride], bias = g.bias ? g.bias[brow] : 0.0f;
+#pragma unroll
+    for (int j = 0; j < MINE; ++j) {
+        float am = 0.0f;
+#pragma unroll
+        for (int i = 0; i < KV; ++i)
+            am = vtlhip::qdev::absmax4(am, x[j][i]);
+        am = vtlhip::qdev::wave_max(am);
+        const float scale = am / 127.0f;
+        const vtlhip::qdev::QuantScale qp = vtlhip::qdev::make_quant_scale(scale);
+        if (lane == 0)
+            scales[MINE * wave + j] = scale;
+#pragma unroll
+        for (int i = 0; i < KV; ++i) {
+            const int c = 4 * (64 * i + lane);
+            if (c < g.K)
+                *reinterpret_cast<unsigned *>(lds.codes + (MINE * wave + j) * STRIDE + c) = vtlhip::qdev::quant4(x[j][i], qp);
+        }
+    }
+    lds_barrier();   // (the weights stay under way)
+    v16i acc;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+        acc[i] = 0;
+#pragma unroll
+    for (int u = 0; u < KV; ++u) {
+        const int k = k_of(u) + 16 * half;
+        const v4i a = k < g.K ? *reinterpret_cast<const v4i *>(lds.codes + r * STRIDE + k) : v4i{0, 0, 0, 0};
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, b[u], acc, 0, 0, 0);
+    }
+    __syncthreads();   // the codes have been read
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+        lds.red[wave][i][lane] = acc[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < OUT; ++i) {
+        const int reg = wave + NW * i, at = 8 * (reg >> 2) + 4 * half + (reg & 3), m = m0 + at;
+        int sum = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w)
+            sum += lds.red[w][reg][lane];
+        if (m >= g.M || n >= g.N)
+            continue;
+        const float sc = scales[at] * sw;
+        float y = (float)sum * sc;
+        if (g.bias)
+            y = y + bias;
+        if (g.relu && y < 0.0f)
+            y = 0.0f;
+        store_result(reinterpret_cast<float *>(g.out) + (int64_t)m * g.N + n, y, g.done);
+    }
+    raise_when_last(g.done);
+}
+
 // Right before the launch that writes g.out, of `blocks` workgroups that call raise_when_last.
 inline void attach_result(GemmArgs &g, unsigned blocks)
 {
@@ -2565,6 +2661,54 @@ int launch_small(GemmArgs g, int64_t t32, int waves, hipStream_t st)
     return check_launch("gemm_i8_small_kernel");
 }
 
+template <Rows ROWS>
+int launch_linear_small(GemmArgs g)
+{
+    const dim3 grid((unsigned)(((g.M + 31) / 32) * ((g.N + 31) / 32)));
+    attach_result(g, grid.x);
+    const dim3 block(512);
+    hipStream_t st = current_stream();
+    if (g.K <= 256)
+        hipLaunchKernelGGL((linear_small_kernel<1, ROWS>), grid, block, 0, st, g);
+    else if (g.K <= 512)
+        hipLaunchKernelGGL((linear_small_kernel<2, ROWS>), grid, block, 0, st, g);
+    else
+        hipLaunchKernelGGL((linear_small_kernel<3, ROWS>), grid, block, 0, st, g);
+    return check_launch("linear_small_kernel");
+}
+
+// Where that beats a quantizer's launch and the product's: as long as a tile's workgroup has its compute unit for itself, or there is little to quantize
+// (us on the device, and a call among others, in two launches and in one: 32 x 512 x 256 5.6 and 4.5, 7.1 and 4.5; 64 x 1000 x 512 6.4 and 5.6, 7.4 and 5.5;
+// 128 x 1024 x 768 7.2 and 6.9, 6.9 and 6.7, x 912 7.2 and 7.6, 7.0 and 7.2; 128 x 2560 x 256 6.7 and 6.0, 8.0 and 5.8, x 400 7.8 and 7.3, 7.7 and 7.0, x 512 7.2 and
+// 7.8; 64 x 8192 x 400 7.5 and 7.6, 9.1 and 7.2; 256 x 4096 x 256 7.1 and 12.3).  Against the launch that stages rows (`staged`) it is ahead in short rows alone:
+// 32 x 3000 x 256 5.5 and 4.7, x 512 5.5 and 5.6, x 768 6.1 and 6.4, 20 x 14336 x 256 6.0 and 6.0.
+inline bool small_quantized_faster(int M, int N, int K, bool staged)
+{
+    const int64_t t32 = (int64_t)((M + 31) / 32) * ((N + 31) / 32);
+    if (staged)
+        return t32 <= 256 && K <= 256;
+    return (t32 <= 256 && K <= 768) || (t32 <= 512 && K <= 400);
+}
+
+// Whether weights in rows of `row` codes are taken so.
+inline bool small_rows_apply(const int8_t *Wq, int row, int M, int N, bool staged)
+{
+    return row % 16 == 0 && aligned16(Wq) && !tuning().no_fused_decode && tuning().gemm_config < 0 && tuning().gemm_small != 0 &&
+           small_quantized_faster(M, N, row, staged);
+}
+
+// f32 rows of x_cols values, in device memory, against weights in rows of `row` codes (x_cols, or padded); -1: not taken.
+int launch_small_rows(const float *X, int x_cols, const int8_t *Wq, int row, const float *sw, int sw_stride, const float *bias, float *Y, int M,
+                      int N, int relu, HostResult *result, bool staged)
+{
+    if (!small_rows_apply(Wq, row, M, N, staged))
+        return -1;
+    GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, row, 1, sw_stride, relu ? 1 : 0, 1, nullptr, X, 0};
+    g.x_cols = x_cols;
+    g.result = result;
+    return row == x_cols && aligned16(X) ? launch_linear_small<kWhole>(g) : launch_linear_small<kPadded>(g);
+}
+
 template <bool F32OUT>
 int launch_gemm(const GemmArgs &g_in, hipStream_t st)
 {
@@ -2740,6 +2884,11 @@ int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, int s
     }
     const bool staged = stage_inside_launch_faster(M, N, K, gemv_rows_applies(X, Wq, M, N, K) && gemv_rows_faster(M, N, K, true)) &&
                         aligned16(X) && aligned16(Wq) && tuning().gemm_config < 0 && !tuning().no_fused_decode;
+    if (!x_on_host) {   // (every tile would read its rows over the link)
+        const int small = launch_small_rows(X, K, Wq, K, sw, sw_stride, bias, Y, M, N, relu, result, staged);
+        if (small >= 0)
+            return small;
+    }
     if (!workspace) {   // no caller scratch: stage in the library's own buffer
         workspace = vtlhip::library_workspace(vtl_hip_linear_f32_dynquant_workspace(M, K), 1);
         if (!workspace)
@@ -2811,6 +2960,11 @@ int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu,
     const int fused = ragged_rows(x_on_host || result ? kOverLink : kDevice);
     if (fused >= 0)
         return fused;
+    if (!x_on_host) {
+        const int small = launch_small_rows(X, K, l.wq, l.row_bytes, l.sw, sw_stride, l.bias, Y, M, l.out_features, relu, result, false);
+        if (small >= 0)
+            return small;
+    }
     const auto no_scratch = [&] {
         const int status = vtlhip::workspace_status(), alone = ragged_rows(kNoScratch);
         return alone >= 0 ? alone : status;
@@ -2831,6 +2985,12 @@ int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu,
                                                      l.row_bytes, relu, result);
     st = launch_quantize_rows(X, M, K, xq, sx, current_stream());
     return st != VTL_HIP_OK ? st : layer_linear_i8_f32(l, xq, sx, Y, M, relu, result);
+}
+
+bool layer_takes_rows(const vtl_hip_layer &l, int M)
+{
+    return l.per_channel && layer_row_fits(l) && l.out_features > 0 &&
+           small_rows_apply(l.wq, l.row_bytes ? l.row_bytes : l.in_features, M, l.out_features, false);
 }
 
 int layer_linear_i8_requant(const vtl_hip_layer &l, const int8_t *A, const float *sa, int8_t *Yq, float *sy, int M,

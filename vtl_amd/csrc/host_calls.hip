@@ -159,9 +159,9 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
         const bool relu = i + 1 < count && layers[i + 1].kind == VTL_HIP_LAYER_RELU;
         i += relu ? 2 : 1;
         const bool last = y && i == count;
-        // the next layer takes codes as well
+        // the next layer takes codes as well, and does not make them in its own launch
         const bool feeds = l.per_channel && rows > kFewRows && i < count && layers[i].kind == VTL_HIP_LAYER_LINEAR &&
-                           layers[i].per_channel;
+                           layers[i].per_channel && !layer_takes_rows(layers[i], rows);
         if (x && by_row(l) && !feeds) {
             if (!last)
                 VTL_STEP(next.take((size_t)rows * (size_t)n * sizeof(float)));
