@@ -24,6 +24,14 @@ def hip():
     return capi
 
 
+@pytest.fixture(autouse=True)
+def _few_processors(request, monkeypatch):
+    """The launches that test_host_runtime.py pins are those of a machine with few processors, wherever it runs; on others the
+    host makes codes in front of some of them (test_host_quant.py)."""
+    if request.module.__name__ == "test_host_runtime":
+        monkeypatch.setenv("VTL_HIP_HOST_QUANTIZE", "0")
+
+
 class _Knobs:
     """Environment switches of the library for one test: the library reads its
     VTL_HIP_* switches once, so every change here is followed by

@@ -52,7 +52,8 @@ def test_errors(hip):
 
 # The same by the host's units and by the device's: what one thread makes and what several do, pieces that rows do not divide, rows too short
 # for it, one scale for all, and whole forwards whose first layer takes codes (more than 32 rows, dense and padded)
-@pytest.mark.parametrize("rows,cols", [(64, 784), (33, 15), (300, 1023), (257, 1021), (263, 4099), (1000, 17), (70, 70001), (5000, 1027)])
+@pytest.mark.parametrize("rows,cols", [(64, 784), (33, 15), (300, 1023), (257, 1021), (263, 4099), (1000, 17), (70, 70001), (5000, 1027),
+                                       (4, 100), (20, 800), (32, 512), (33, 497), (64, 256), (65, 256), (128, 128), (18, 900), (1000, 16)])
 def test_by_the_host_and_by_the_device(hip, knobs, rows, cols):
     rng = np.random.default_rng(rows * 31 + cols)
     x = rng.standard_normal((rows, cols)).astype(np.float32)

@@ -123,7 +123,11 @@ for on in (0, 1):
         assert weights(8, 15, per_row) == ["host_copy", "quantize"]
         assert weights(8, 784, per_row, 65540) == ["host_copy", "quantize"]
         assert forward(33, 784, per_row)[:2] == (["host_copy"] if on else ["quantize"]) + ["gemm_i8"]
-        assert forward(32, 784, per_row)[0] != "host_copy"
+        assert forward(32, 784, per_row)[0] == ("host_copy" if on else "quantize")
+        assert forward(64, 256, per_row)[0] == forward(16, 1008, 0)[0] == ("gemm_i8" if on else "quantize")     # 16 KiB of codes: read over the link
+        assert forward(65, 256, per_row)[0] == forward(17, 1008, 0)[0] == ("host_copy" if on else "quantize")
+        assert forward(16, 1000, per_row, 1008)[0] == ("gemm_i8" if on else "quantize")
+        assert forward(1, 784, per_row) == ["linear_gemv"] and forward(8, 240, 1)[0] == "quantize"
         got = forward(40, 1000, per_row, 1008)
         assert got[:2] == (["host_copy", "gemm_i8"] if on else ["quantize", "pad_rows"]), (on, per_row, got)
         assert forward(40, 1000, per_row, 8)[-1:] != ["gemm_i8"]               # rows that do not fit are refused either way

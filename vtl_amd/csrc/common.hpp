@@ -70,6 +70,9 @@ struct HostInput {
     const void *data = nullptr;
     // False when the bytes have to be uploaded instead: too many, or streams of the caller's.
     bool stage(const void *src, size_t bytes);
+    // As codes and scales (data, scales), made by the host as upload_codes has them made.
+    bool stage_codes(const float *src, int64_t rows, int64_t cols, int per_row, int64_t row);
+    const float *scales = nullptr;
     void release();
     HostInput() = default;
     ~HostInput() { release(); }
@@ -97,7 +100,9 @@ bool upload_rows(const float *src, int64_t rows, int64_t cols, int8_t *q, float 
                  size_t extra_bytes, int &status);
 
 // Rows that the host's threads quantize in front of the link, which then carries a quarter of their bytes: per_row, or with one
-// scale; `row` bytes from one row of codes to the next (zeros behind the codes).  False: to be quantized by the device.
+// scale; `row` bytes from one row of codes to the next (zeros behind the codes).  False: to be quantized by the device, as always
+// where the host does not make codes of such rows.
+bool host_makes_codes(int64_t rows, int64_t cols, int64_t row);
 bool upload_codes(const float *src, int64_t rows, int64_t cols, int per_row, int8_t *q, int64_t row, float *scale, void *extra_dst,
                   const void *extra_src, size_t extra_bytes, int &status);
 
@@ -285,8 +290,9 @@ int layer_linear_i8_f32(const vtl_hip_layer &l, const int8_t *A, const float *sa
 // vtl_hip_layer_f32; of one row with one scale for the weights too.  `x_on_host`: X is in pinned memory (HostInput).
 int layer_f32(const vtl_hip_layer &l, const float *X, float *Y, int M, int relu, void *workspace, size_t workspace_bytes,
               HostResult *result = nullptr, bool x_on_host = false);
-// Whether layer_f32 has more than a few rows in device memory in one launch.
+// Whether layer_f32 has rows in device memory, or of a host call's input, in one launch (more than eight of them).
 bool layer_takes_rows(const vtl_hip_layer &l, int M);
+bool layer_takes_input(const vtl_hip_layer &l, int M);
 int layer_linear_i8_requant(const vtl_hip_layer &l, const int8_t *A, const float *sa, int8_t *Yq, float *sy, int M,
                             int relu, bool padded = false);
 

@@ -2993,6 +2993,11 @@ bool layer_takes_rows(const vtl_hip_layer &l, int M)
            small_rows_apply(l.wq, l.row_bytes ? l.row_bytes : l.in_features, M, l.out_features, false);
 }
 
+bool layer_takes_input(const vtl_hip_layer &l, int M)
+{
+    return l.per_channel && l.row_bytes == 0 && aligned16(l.wq) && stage_inside_launch_faster(M, l.out_features, l.in_features, false);
+}
+
 int layer_linear_i8_requant(const vtl_hip_layer &l, const int8_t *A, const float *sa, int8_t *Yq, float *sy, int M,
                             int relu, bool padded)
 {

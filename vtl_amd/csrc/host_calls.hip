@@ -49,6 +49,11 @@ struct Scratch {
 // 28.0 us); with more rows per-row codes go from layer to layer.  The bits are the same.
 constexpr int kFewRows = 32;
 
+// Up to how many bytes of codes the first product reads over the link: each XCD fetches them, which from here on takes what a launch that carries
+// them up does (us, carried and read: 7 x 128 x 128 17.3 and 14.1, 64 x 256 x 128 20.8 and 18.1, 200 x 300 x 64 23.3 and 20.0, 32 x 512 x 512 22.2 and 20.7, 20 x 500 x
+// 1100 21.9 and 22.4, 64 x 256 x 784 24.2 and 29.3).
+constexpr size_t kCodesOverLink = (size_t)16 << 10;
+
 int check_layers(const vtl_hip_layer *layers, int count, int cols, int &out_cols)
 {
     for (int i = 0; i < count; i++) {
@@ -108,25 +113,35 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
     // 64 x 256 20.9 -> 17.0, of 2500 x 11008 29.3 -> 24.6).
     const auto by_row = [&](const vtl_hip_layer &l) { return l.per_channel || rows == 1; };
     const bool first_by_row = count > 0 && by_row(layers[0]) && (layers[0].per_channel || row_in_one(layers[0].out_features, cols));
-    // More than a few rows that a quantizer's launch would only make codes of go up as codes: of 200 KB the copies and the launches
-    // take less, of 4 MiB the link too.
+    // Rows that a launch would only make codes of are made codes of by the host: few bytes of them are read over the link by the product's launch,
+    // more go up.
+    const int8_t *in = nullptr;            // the activations where they are codes, and their scales
+    const float *in_scales = nullptr;
     bool padded = false;                   // whether the codes lie in rows of l.row_bytes
-    if (count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR && rows > kFewRows) {
+    if (count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR &&
+        (rows > kFewRows || (rows > 1 && !layers[0].per_channel) || (rows > 8 && !layer_takes_input(layers[0], rows)))) {
         const vtl_hip_layer &l = layers[0];
         const int row = l.row_bytes > cols ? l.row_bytes : cols;
-        VTL_STEP(codes.take((size_t)rows * (size_t)row));
-        VTL_STEP(scales.take((l.per_channel ? (size_t)rows : 1) * sizeof(float)));
-        int status = VTL_HIP_OK;
-        if (upload_codes(x_host, rows, cols, l.per_channel, codes.as<int8_t>(), row, scales.as<float>(), nullptr, nullptr, 0, status)) {
-            VTL_STEP(status);
-            padded = l.row_bytes != 0;
-        } else {
-            codes.release();
-            scales.release();
+        if ((size_t)rows * (size_t)row <= kCodesOverLink && input.stage_codes(x_host, rows, cols, l.per_channel, row)) {
+            in = static_cast<const int8_t *>(input.data);
+            in_scales = input.scales;
+        } else if (host_makes_codes(rows, cols, row)) {
+            VTL_STEP(codes.take((size_t)rows * (size_t)row));
+            VTL_STEP(scales.take((l.per_channel ? (size_t)rows : 1) * sizeof(float)));
+            int status = VTL_HIP_OK;
+            if (upload_codes(x_host, rows, cols, l.per_channel, codes.as<int8_t>(), row, scales.as<float>(), nullptr, nullptr, 0, status)) {
+                VTL_STEP(status);
+                in = codes.as<int8_t>();
+                in_scales = scales.as<float>();
+            } else {
+                codes.release();
+                scales.release();
+            }
         }
+        padded = in && l.row_bytes != 0;
     }
     const bool upload_first = rows <= 8 && in_bytes > ((size_t)20 << 10) && in_bytes <= ((size_t)32 << 10);
-    if (!codes.ptr && count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR && !(upload_first && first_by_row) &&
+    if (!in && count > 0 && layers[0].kind == VTL_HIP_LAYER_LINEAR && !(upload_first && first_by_row) &&
         input.stage(x_host, in_bytes)) {
         // The first launch takes the input over the link itself: 64 x 784, per tensor, 4 us less than behind an
         // upload.  Rows that are no whole vectors are read twice, which still is no slower (forward of 200 x 1001
@@ -140,10 +155,12 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
             VTL_STEP(scales.take((layers[0].per_channel ? (size_t)rows : 1) * sizeof(float)));
             VTL_STEP(vtl_hip_quantize_f32_i8(x, rows, cols, layers[0].per_channel, codes.as<int8_t>(), scales.as<float>()));
             x = nullptr;
+            in = codes.as<int8_t>();
+            in_scales = scales.as<float>();
             input.release();
         }
     }
-    if (!codes.ptr && !x) {
+    if (!in && !x) {
         VTL_STEP(cur.take(in_bytes));
         VTL_STEP(vtl_hip_upload(cur.ptr, x_host, in_bytes));
         x = cur.as<float>();
@@ -187,20 +204,29 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
             VTL_STEP(scales.take((l.per_channel ? (size_t)rows : 1) * sizeof(float)));
             VTL_STEP(vtl_hip_quantize_f32_i8(x, rows, cols, l.per_channel, codes.as<int8_t>(), scales.as<float>()));
             x = nullptr;
+            in = codes.as<int8_t>();
+            in_scales = scales.as<float>();
         }
         if (feeds) {
             VTL_STEP(next_codes.take((size_t)rows * (size_t)n));
             VTL_STEP(next_scales.take((size_t)rows * sizeof(float)));
-            VTL_STEP(layer_linear_i8_requant(l, codes.as<int8_t>(), scales.as<float>(), next_codes.as<int8_t>(),
+            VTL_STEP(layer_linear_i8_requant(l, in, in_scales, next_codes.as<int8_t>(),
                                              next_scales.as<float>(), rows, relu, padded));
             codes.swap(next_codes);
             scales.swap(next_scales);
+            in = codes.as<int8_t>();
+            in_scales = scales.as<float>();
         } else {
             if (!last)
                 VTL_STEP(cur.take((size_t)rows * (size_t)n * sizeof(float)));
-            VTL_STEP(layer_linear_i8_f32(l, codes.as<int8_t>(), scales.as<float>(), last ? y : cur.as<float>(), rows, relu,
+            VTL_STEP(layer_linear_i8_f32(l, in, in_scales, last ? y : cur.as<float>(), rows, relu,
                                          last ? &result : nullptr, padded));
             x = cur.as<float>();
+        }
+        if (input.data) {
+            input.release();
+            if (result.attached())
+                result.input_released();
         }
         padded = false;
         cols = n;

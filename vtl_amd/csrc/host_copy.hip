@@ -1115,6 +1115,19 @@ int download_large(Ring *r, char *dst, const char *src, size_t bytes, hipStream_
 
 }  // namespace
 
+// The host makes codes of f32 rows, and the link carries those: 180 MB of weights with their scales and the forward behind them 3640 -> 1480 us, 4 MiB
+// of activations through three layers 208 -> 157, 200 KB 28.7 -> 25.4 (16 processors).  Only above so many processors that the
+// caller and its helpers are about half of them: with fewer, memory is what a copy and the codes wait for alike (8 processors, GB/s of f32 by 4
+// threads: copied 35, quantized 32).
+constexpr int kQuantizeProcessors = 2 * Crew::kHelpers;
+
+const HostQuantizer *quantizer_to_use()
+{
+    static const bool many = processors() > kQuantizeProcessors;
+    const int asked = tuning().host_quantize;
+    return (asked < 0 ? many : asked != 0) ? host_quantizer() : nullptr;
+}
+
 void HostInput::release()
 {
     if (!ring_)
@@ -1143,6 +1156,37 @@ try {
     }
     ring_ = r;
     data = put_small(r, src, bytes, 0);
+    return true;
+} catch (const std::exception &) {
+    return false;
+}
+
+bool HostInput::stage_codes(const float *src, int64_t rows, int64_t cols, int per_row, int64_t row)
+try {
+    const HostQuantizer *host = quantizer_to_use();
+    const size_t codes = ((size_t)rows * (size_t)row + 15) & ~(size_t)15, room = small_room(codes + (size_t)rows * sizeof(float));
+    if (!host || !single_stream() || rows < 1 || cols < 1 || row < cols || room > kSmall)
+        return false;
+    Ring *r = ring_of_current_device();
+    if (!r)
+        return false;
+    r->lock.lock();
+    if (open_small(r, room, current_stream()) != VTL_HIP_OK) {
+        r->lock.unlock();
+        return false;
+    }
+    ring_ = r;
+    char *const staged = r->at(r->slot) + r->used;
+    float *const s = reinterpret_cast<float *>(staged + codes);
+    if (per_row) {
+        host->rows(src, rows, cols, reinterpret_cast<int8_t *>(staged), row, s);
+    } else {
+        *s = host->scale(host->absmax(src, rows * cols));
+        host->scaled(src, rows, cols, reinterpret_cast<int8_t *>(staged), row, *s);
+    }
+    r->used += room;
+    data = staged;
+    scales = s;
     return true;
 } catch (const std::exception &) {
     return false;
@@ -1229,25 +1273,23 @@ try {
     return true;
 }
 
-// The host makes codes of f32 rows, and the link carries those: 180 MB of weights with their scales and the forward behind them 3640 -> 1480 us, 4 MiB
-// of activations through three layers 208 -> 157, 200 KB 28.7 -> 25.4 (16 processors).  Only above so many processors that the
-// caller and its helpers are about half of them: with fewer, memory is what a copy and the codes wait for alike (8 processors, GB/s of f32 by 4
-// threads: copied 35, quantized 32).
-constexpr int kQuantizeProcessors = 2 * Crew::kHelpers;
+bool host_makes_codes(int64_t rows, int64_t cols, int64_t row)
+{
+    // (a slot has room for a row, and for the codes and scales of as many bytes of f32)
+    return rows >= 1 && cols >= kCodesLeastCols && (size_t)cols * sizeof(float) <= kSlotBytes && row >= cols &&
+           (size_t)row + sizeof(float) <= (size_t)cols * sizeof(float) && quantizer_to_use() &&
+           (single_stream() || !stream_is_capturing(current_stream()));
+}
 
 bool upload_codes(const float *src, int64_t rows, int64_t cols, int per_row, int8_t *q, int64_t row, float *scale, void *extra_dst,
                   const void *extra_src, size_t extra_bytes, int &status)
 try {
-    static const bool many = processors() > kQuantizeProcessors;
-    const int asked = tuning().host_quantize;
-    const HostQuantizer *host = (asked < 0 ? many : asked != 0) ? host_quantizer() : nullptr;
+    if (!host_makes_codes(rows, cols, row) || extra_bytes > kWithAnother)
+        return false;
+    const HostQuantizer *host = quantizer_to_use();
     hipStream_t st = current_stream();
     const bool one_stream = single_stream();
     const size_t unit = (size_t)cols * sizeof(float), bytes = (size_t)rows * unit;
-    // (a slot has room for a row, and for the codes and scales of as many bytes of f32)
-    if (!host || rows < 1 || cols < kCodesLeastCols || unit > kSlotBytes || (size_t)row + sizeof(float) > unit || extra_bytes > kWithAnother ||
-        (!one_stream && stream_is_capturing(st)))
-        return false;
     const OwnerDevice owner(q, extra_bytes ? extra_dst : nullptr);
     Ring *r = owner.kernels() && owner.holds(scale) ? ring_of_current_device() : nullptr;
     if (!r)
