@@ -620,7 +620,7 @@ def bench_full_precision(timer: Timer, steps: int, warmup: int):
         "us": us, "TFLOP/s": tf,
         "roofline": {"bound": "mfma", "achieved": tf, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                      "frac": tf / PEAK_FP64_TFLOPS, "traffic": measured_traffic("linear_f32"),
-                     "kernel": "matmul_f64acc_direct_kernel<float, 1, 1, 4, 2, 4, false, true, false>"}}
+                     "kernel": "matmul_f64acc_direct_kernel<float, 1, 1, 4, 2, 4, false, true, false, false>"}}
     for h in (X, W, B, Y):
         h.release()
 

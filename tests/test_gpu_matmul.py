@@ -586,3 +586,31 @@ def test_matmul_gate_backward(hip, monkeypatch):
         assert_close_to_oracle(db, want_b, absb)
     with pytest.raises(ValueError, match="Invalid shapes"):
         matmul_gate_backward_hip(np.zeros((3, 3)), np.zeros((3, 4)), np.zeros((5, 3)))
+
+
+# Slices of K whose sums meet within their launch: every shape, tiles at the edges, one and many slices, a K on either side of where that begins, more
+# tiles than there are counters, and the same launches again (the counters are left at zero).  Whole numbers: every order of the sums is exact.
+@pytest.mark.parametrize("mnk", [(33, 65, 800), (1, 70, 1616), (64, 1, 2047), (100, 300, 3001), (17, 33, 799), (130, 129, 848), (1100, 1100, 800), (64, 256, 2000)])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+def test_slices_that_meet_within_their_launch(hip, mnk, dt, knobs):
+    m, n, k = mnk
+    rng = np.random.default_rng(m * 3 + n * 5 + k)
+    a, w = rng.integers(-8, 9, (m, k)).astype(dt), rng.integers(-8, 9, (n, k)).astype(dt)
+    bias = rng.integers(-500, 500, n).astype(dt)
+    want = (a.astype(np.int64) @ w.astype(np.int64).T).astype(dt)
+    A, W, B, Wt = dev(a), dev(w), dev(bias), dev(np.ascontiguousarray(w.T))
+    print(mnk, dt.__name__, flush=True)
+    for tile in ("0", "1", "2", "3", "4", "5", "6"):
+        knobs.setenv("VTL_HIP_MATMUL_TILE", tile)
+        for splits in ("-1", "2", "7", "25"):
+            knobs.setenv("VTL_HIP_MATMUL_SPLITS", splits)
+            for _ in range(2):
+                y = matmul_hip(A, Wt)
+                assert np.array_equal(y.cpu(), want), (tile, splits)
+                y.release()
+            y = linear_hip(A, W, B, relu=True)
+            assert np.array_equal(y.cpu(), np.maximum(want + bias, 0)), (tile, splits)
+            y.release()
+            assert np.array_equal(matmul_hip_host(a, np.ascontiguousarray(w.T)), want), (tile, splits)
+    for t in (A, W, B, Wt):
+        t.release()

@@ -180,9 +180,10 @@ __device__ __forceinline__ void store_through(void *out, unsigned off, Words2 v)
 {
     __builtin_amdgcn_raw_buffer_store_b64(v, result_buffer(out), off, 0, kThrough);
 }
+template <int HOW = kThrough>
 __device__ __forceinline__ void store_through(void *out, unsigned off, Words4 v)
 {
-    __builtin_amdgcn_raw_buffer_store_b128(v, result_buffer(out), off, 0, kThrough);
+    __builtin_amdgcn_raw_buffer_store_b128(v, result_buffer(out), off, 0, HOW);
 }
 
 // Called by every thread of a workgroup after its last store_result.  Those are written through, so their

@@ -31,6 +31,8 @@ struct MatmulArgs {
     double *partial;    // launches that slice K: [slices][M][N] unrounded sums, or [tail tile][slice][tile]; else nullptr
     int whole_tiles;    // with tail_slices > 1 the tiles from here on, the last round's, have K in that many slices
     int tail_slices;
+    int fold_slices;    // > 1: K in so many slices (grid.y), whose sums the last workgroup of each tile adds up; partial: [tile][slice][tile]
+    int fold_slot;      // which counters
     vtlhip::DoneSignal done;     // C is the memory of a whole host call's result
     vtlhip::HostResult *result;  // host side only
 };
@@ -214,12 +216,37 @@ struct PartialTiles {
     double at[WK > 1 ? WM * WN * WK : 1][WK > 1 ? 4 * TM * TN : 1][64];
 };
 
+// Slices of K that meet within a launch.  Each workgroup writes its sums through to memory (16 bytes a thread, whole lines), waits until that is
+// acknowledged and counts itself at its tile; who completes the count reads the slices back, past the caches, adds them up in
+// their order and leaves the counter at 0 for the next launch.  Nobody waits for another, and no fence writes a cache back.  A launch that adds them up
+// instead is 3.4 to 4.7 us on the device, a gap, and 3.4 us on the host (us, with one and so: f32 64 x 256 x 2000 12.2 -> 8.0, 32 x 1024 x 1024 8.3 -> 6.8, 128 x 1024 x 4096
+// 27.2 -> 24.2, f64 64 x 64 x 4096 16.4 -> 10.9, 64 x 1024 x 1024 11.5 -> 8.5).  The counters belong to a stream, whose launches follow one another.
+constexpr int kFoldTiles = 1024, kFoldStride = 16;
+__device__ unsigned g_fold_count[vtlhip::kStreamSlots * kFoldTiles * kFoldStride];
+
+// Whether this workgroup, whose sums are written, is the last of its tile's.
+__device__ __forceinline__ bool last_of_tile(const MatmulArgs &g, int block)
+{
+    __shared__ int s_last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();   // every thread's are
+    if (threadIdx.x == 0) {
+        unsigned *const count = g_fold_count + ((int64_t)g.fold_slot * kFoldTiles + block) * kFoldStride;
+        const bool last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 == (unsigned)g.fold_slices;
+        if (last)
+            __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s_last = last;
+    }
+    __syncthreads();
+    return s_last;
+}
+
 // One workgroup's part of a product: tile `block` and slice `slice` of K, of g.slice_steps steps.  `turn`: this workgroup's number in the launch.
 // (The arguments by value: by reference the compiler lays the branches of the end out otherwise, 512^3 f64 to the host 48.4 -> 48.7 us.)
 // The tiles of a workgroup are WM x WN wave tiles, K is cut over WK waves each.
 // Blocks are renumbered so that each of the 8 XCDs (own L2) works on a compact patch of tiles, eight
 // tile rows deep: with the plain order the rows that share a column panel of B run on different XCDs.
-template <typename T, int WM, int WN, int WK, int TM, int TN, bool TA, bool TB, bool CHECKED>
+template <typename T, int WM, int WN, int WK, int TM, int TN, bool TA, bool TB, bool CHECKED, bool FOLD = false>
 __device__ __forceinline__ void direct_tile(const MatmulArgs g, int block, int slice, unsigned turn,
                                             PartialTiles<WM, WN, WK, TM, TN> &red)
 {
@@ -435,7 +462,7 @@ __device__ __forceinline__ void direct_tile(const MatmulArgs g, int block, int s
     if (TAIL && of_tail >= 0) {
         partial = g.partial + (int64_t)of_tail * (BM * BN) - ((int64_t)tm * BM * BN + (int64_t)tn * BN);
         partial_row = BN;
-    } else if (g.partial && !(TAIL && g.tail_slices > 1)) {
+    } else if (!FOLD && g.partial && !(TAIL && g.tail_slices > 1)) {
         partial = g.partial + (int64_t)slice * g.M * g.N;
     }
     // Value v of a lane: i = v / (4 TN), j = v / 4 % TN, e = v % 4.  Values v and v + 4 of an even j are
@@ -508,6 +535,11 @@ __device__ __forceinline__ void direct_tile(const MatmulArgs g, int block, int s
             if (!(v & 4))
                 store(v, acc[v / (4 * TN)][(v >> 2) % TN][v & 3], acc[v / (4 * TN)][(v >> 2) % TN + 1][v & 3]);
     } else {
+        static_assert(!FOLD || !(TAIL || CHECKED), "slices meet in the launch for the shapes that are cut most");
+        typedef double Pair __attribute__((ext_vector_type(2)));
+        constexpr int kDevice = 16;   // sc1: past the caches of the XCD
+        double *const slices_of_tile = FOLD ? g.partial + (int64_t)block * g.fold_slices * (BM * BN) : nullptr;
+        const auto pair_at_tile = [](int u) { return (unsigned)(u * (64 * WM * WN * WK) + (int)threadIdx.x) * 16u; };
         // partial tiles, in the order of the registers
 #pragma unroll
         for (int v = 0; v < V; ++v)
@@ -522,17 +554,49 @@ __device__ __forceinline__ void direct_tile(const MatmulArgs g, int block, int s
                 s0 += red.at[tile * WK + w][v][lane];
                 s1 += red.at[tile * WK + w][v + 4][lane];
             }
-            store(v, s0, s1);
+            if constexpr (FOLD)
+                vtlhip::store_through<kDevice>(slices_of_tile + (int64_t)slice * (BM * BN), pair_at_tile(u), __builtin_bit_cast(vtlhip::Words4, Pair{s0, s1}));
+            else
+                store(v, s0, s1);
+        }
+        if constexpr (FOLD) {
+            if (!last_of_tile(g, block))
+                return;
+            // four slices' pairs on their way at a time
+            const __amdgpu_buffer_rsrc_t from = vtlhip::result_buffer(slices_of_tile);
+            constexpr int PAIRS = V / 2 / WK, AT_ONCE = 4;
+            Pair sum[PAIRS] = {};
+            for (int s = 0; s < g.fold_slices; s += AT_ONCE) {
+                Pair p[AT_ONCE][PAIRS];
+#pragma unroll
+                for (int q = 0; q < AT_ONCE; ++q)
+#pragma unroll
+                    for (int u = 0; u < PAIRS; ++u) {
+                        const unsigned slice_at = (unsigned)min(s + q, g.fold_slices - 1) * (BM * BN * 8u);   // (the last one again, not added)
+                        p[q][u] = __builtin_bit_cast(Pair, __builtin_amdgcn_raw_buffer_load_b128(from, pair_at_tile(u) + slice_at, 0, kDevice));
+                    }
+#pragma unroll
+                for (int q = 0; q < AT_ONCE; ++q)
+                    if (s + q < g.fold_slices)
+#pragma unroll
+                        for (int u = 0; u < PAIRS; ++u)
+                            sum[u] += p[q][u];
+            }
+#pragma unroll
+            for (int u = 0; u < PAIRS; ++u) {
+                const int pair = wk + WK * u;
+                store(8 * (pair >> 2) + (pair & 3), sum[u].x, sum[u].y);
+            }
         }
     }
     vtlhip::raise_when_last(g.done);   // (a launch that leaves partial sums has no signal)
 }
 
-template <typename T, int WM, int WN, int WK, int TM, int TN, bool TA, bool TB, bool CHECKED>
+template <typename T, int WM, int WN, int WK, int TM, int TN, bool TA, bool TB, bool CHECKED, bool FOLD = false>
 __global__ __launch_bounds__(64 * WM * WN * WK) void matmul_f64acc_direct_kernel(const MatmulArgs g)
 {
     __shared__ PartialTiles<WM, WN, WK, TM, TN> red;
-    direct_tile<T, WM, WN, WK, TM, TN, TA, TB, CHECKED>(g, (int)blockIdx.x, (int)blockIdx.y, blockIdx.x + gridDim.x * blockIdx.y, red);
+    direct_tile<T, WM, WN, WK, TM, TN, TA, TB, CHECKED, FOLD>(g, (int)blockIdx.x, (int)blockIdx.y, blockIdx.x + gridDim.x * blockIdx.y, red);
 }
 
 // The sums of kSumCols columns by one workgroup of 256 threads: 16 phases of rows, added in order.  Rows start at any element.
@@ -618,7 +682,7 @@ struct BackwardArgs {
     int dx_tiles, dx_blocks, dw_blocks;
 };
 
-template <typename T, int TNX, int TNW>
+template <typename T, int TNX, int TNW, bool FOLD>
 __global__ __launch_bounds__(256) void linear_backward_kernel(const BackwardArgs<T> g)
 {
     __shared__ union {
@@ -628,7 +692,7 @@ __global__ __launch_bounds__(256) void linear_backward_kernel(const BackwardArgs
     } red;
     int block = (int)blockIdx.x;
     if (block < g.dx_blocks) {
-        direct_tile<T, 1, 1, 4, 2, TNX, false, false, false>(g.dx, block % g.dx_tiles, block / g.dx_tiles, blockIdx.x, red.dx);
+        direct_tile<T, 1, 1, 4, 2, TNX, false, false, false, FOLD>(g.dx, block % g.dx_tiles, block / g.dx_tiles, blockIdx.x, red.dx);
         return;
     }
     block -= g.dx_blocks;
@@ -890,21 +954,26 @@ int launch_direct_shape(MatmulArgs g, bool ta, bool tb, int slices, hipStream_t 
     if (blocks > 0x7fffffff)
         return VTL_HIP_ERR_UNSUPPORTED;
     const dim3 grid((unsigned)blocks, (unsigned)slices), block(64 * WM * WN * WK);
-    if (g.result && slices == 1)
+    if (g.result && (slices == 1 || g.fold_slices > 1))
         g.result->attach(g.done, grid.x);
-#define VTL_DIRECT(TA, TB) \
-    hipLaunchKernelGGL((matmul_f64acc_direct_kernel<T, WM, WN, WK, TM, TN, TA, TB, CHECKED>), grid, block, 0, st, g)
+    constexpr bool FOLDS = WK > 1 && TM == 2 && !CHECKED;   // (fold_slices asks for no other)
+#define VTL_DIRECT(TA, TB)                                                                                                                 \
+    if (FOLDS && g.fold_slices > 1)                                                                                                        \
+        hipLaunchKernelGGL((matmul_f64acc_direct_kernel<T, WM, WN, WK, TM, TN, TA, TB, CHECKED, FOLDS>), grid, block, 0, st, g);           \
+    else                                                                                                                                   \
+        hipLaunchKernelGGL((matmul_f64acc_direct_kernel<T, WM, WN, WK, TM, TN, TA, TB, CHECKED>), grid, block, 0, st, g)
     if constexpr (ROWS_ONLY) {
         VTL_DIRECT(false, true);
     } else {
-        if (!ta && !tb)
+        if (!ta && !tb) {
             VTL_DIRECT(false, false);
-        else if (!ta && tb)
+        } else if (!ta && tb) {
             VTL_DIRECT(false, true);
-        else if (ta && !tb)
+        } else if (ta && !tb) {
             VTL_DIRECT(true, false);
-        else
+        } else {
             VTL_DIRECT(true, true);
+        }
     }
 #undef VTL_DIRECT
     return check_launch("matmul_f64acc_direct_kernel");
@@ -952,6 +1021,22 @@ struct Partial {
     }
 };
 
+// From how long a K on slices meet within their launch: shorter ones are level with a launch that adds them up (64 x 256 x 784 f32 7.4 and 7.2 us a
+// call, f64 7.6 and 7.5).
+constexpr int kFoldFrom = 800;
+
+// The slices of a launch with tiles of bm x bn (kK8, kK4 or kWide) meet within it, where the stream has counters (not while it is being captured: replays of two graphs
+// may meet) and the memory is there; else g is left as it is.
+void fold_slices(MatmulArgs &g, int bm, int bn, int slices, Partial &partial, bool alone, hipStream_t st)
+{
+    const int64_t tiles = (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn);
+    const int slot = tiles <= kFoldTiles && g.K >= kFoldFrom ? vtlhip::stream_slot(st) : -1;
+    if (slot < 0 || !(g.partial = partial.take((size_t)tiles * (size_t)slices * (size_t)(bm * bn) * sizeof(double), alone)))
+        return;
+    g.fold_slices = slices;
+    g.fold_slot = slot;
+}
+
 template <typename T>
 int launch_direct(MatmulArgs g, Kind kind, bool ta, bool tb, Plan plan, bool alone, hipStream_t st)
 {
@@ -961,7 +1046,10 @@ int launch_direct(MatmulArgs g, Kind kind, bool ta, bool tb, Plan plan, bool alo
     int slices = per > 0 ? (steps + per - 1) / per : 1;
     Partial partial;
     if (slices > 1) {
-        g.partial = partial.take((size_t)slices * (size_t)g.M * (size_t)g.N * sizeof(double), alone);
+        if (!checked && (plan.shape == kK8 || plan.shape == kK4 || plan.shape == kWide))
+            fold_slices(g, kTileM[kind][plan.shape], kTileN[kind][plan.shape], slices, partial, alone, st);
+        if (!g.partial)
+            g.partial = partial.take((size_t)slices * (size_t)g.M * (size_t)g.N * sizeof(double), alone);
         if (!g.partial) {   // no memory, or a capture that may not allocate: K in one piece
             per = steps;
             slices = 1;
@@ -1004,7 +1092,7 @@ int launch_direct(MatmulArgs g, Kind kind, bool ta, bool tb, Plan plan, bool alo
         hipLaunchKernelGGL((matmul_tail_finalize_kernel<T>), dim3((unsigned)(left * (bm * bn / 256))), dim3(256), 0, st, g, bm, bn);
         return check_launch("matmul_tail_finalize_kernel");
     }
-    return slices == 1 ? rc : finalize_split<T>(g, slices, st);
+    return slices == 1 || g.fold_slices > 1 ? rc : finalize_split<T>(g, slices, st);
 }
 
 template <typename T>
@@ -1177,7 +1265,9 @@ bool backward_in_one(vtlhip::HostResult *result, const T *grad, const T *x, cons
     g.db = {grad, m, n, db};
     Partial partial;
     int cut = slices;
-    if (cut > 1 && !(g.dx.partial = partial.take((size_t)cut * (size_t)m * (size_t)k * sizeof(double), alone))) {
+    if (cut > 1)
+        fold_slices(g.dx, 32, kTileN[kind][px.shape], cut, partial, alone, current_stream());
+    if (cut > 1 && !g.dx.partial && !(g.dx.partial = partial.take((size_t)cut * (size_t)m * (size_t)k * sizeof(double), alone))) {
         g.dx.slice_steps = steps;   // no memory, or a capture that may not allocate: K in one piece
         cut = 1;
     }
@@ -1189,16 +1279,23 @@ bool backward_in_one(vtlhip::HostResult *result, const T *grad, const T *x, cons
         g.dx.done = g.dw.done;
     }
     hipStream_t st = current_stream();
-    if (px.shape == kK4 && pw.shape == kK4)
-        hipLaunchKernelGGL((linear_backward_kernel<T, 2, 2>), grid, dim3(256), 0, st, g);
-    else if (px.shape == kK4)
-        hipLaunchKernelGGL((linear_backward_kernel<T, 2, 4>), grid, dim3(256), 0, st, g);
-    else if (pw.shape == kK4)
-        hipLaunchKernelGGL((linear_backward_kernel<T, 4, 2>), grid, dim3(256), 0, st, g);
-    else
-        hipLaunchKernelGGL((linear_backward_kernel<T, 4, 4>), grid, dim3(256), 0, st, g);
+#define VTL_BACKWARD(TNX, TNW)                                                                        \
+    if (g.dx.fold_slices > 1)                                                                         \
+        hipLaunchKernelGGL((linear_backward_kernel<T, TNX, TNW, true>), grid, dim3(256), 0, st, g);   \
+    else                                                                                              \
+        hipLaunchKernelGGL((linear_backward_kernel<T, TNX, TNW, false>), grid, dim3(256), 0, st, g)
+    if (px.shape == kK4 && pw.shape == kK4) {
+        VTL_BACKWARD(2, 2);
+    } else if (px.shape == kK4) {
+        VTL_BACKWARD(2, 4);
+    } else if (pw.shape == kK4) {
+        VTL_BACKWARD(4, 2);
+    } else {
+        VTL_BACKWARD(4, 4);
+    }
+#undef VTL_BACKWARD
     status = check_launch("linear_backward_kernel");
-    if (status == VTL_HIP_OK && cut > 1)
+    if (status == VTL_HIP_OK && cut > 1 && g.dx.fold_slices <= 1)
         status = finalize_split<T>(g.dx, cut, st);
     return true;
 }
