@@ -629,7 +629,8 @@ def test_layers_whose_weights_get_padded_rows(hip, m, n, k):
 # whole and padded weight rows, rows that start anywhere, values that are no numbers
 @pytest.mark.parametrize("mnk", [(9, 300, 256), (33, 100, 272), (32, 3000, 256), (64, 1000, 512), (65, 31, 528), (100, 2047, 768), (128, 1024, 784), (250, 1030, 400),
                                  (500, 1024, 400), (512, 1025, 400), (2, 2000, 64), (40, 4, 16), (70, 1200, 767), (70, 1200, 385), (33, 2000, 241),
-                                 (16, 1000, 768)])
+                                 (16, 1000, 768), (5, 600, 256), (8, 4000, 512), (8, 8200, 512), (8, 14336, 256), (8, 16400, 256), (4, 4000, 256),
+                                 (3, 3900, 256), (6, 3969, 320)])
 def test_rows_quantized_by_each_tile(hip, mnk):
     m, n, k = mnk
     rng = np.random.default_rng(m * 7 + n * 3 + k)

@@ -2690,6 +2690,17 @@ inline bool small_quantized_faster(int M, int N, int K, bool staged)
     return (t32 <= 256 && K <= 768) || (t32 <= 512 && K <= 400);
 }
 
+// And where beats the matrix-vector kernel that quantizes three to eight rows in every workgroup: that reads whole rows of them for eight weight rows, and its sums
+// grow with them (us on the device, that and this: 8 x 500 x 256 4.6 and 4.0, 8 x 14336 x 256 8.6 and 5.6, 6 x 4000 x 512 6.3 and 5.2, 8 x 8000 x 512 6.6 and 5.4, 4 x 8000 x
+// 256 5.2 and 4.3; but 8 x 2000 x 512 4.8 and 5.1, 4 x 2000 x 256 3.7 and 4.0, 4 x 8000 x 512 5.2 and 5.4, 2 x 4000 x 256 3.8 and 4.0).
+inline bool few_rows_by_tiles(int M, int N, int K)
+{
+    const int tiles = (N + 31) / 32;
+    if (M < 3 || M > 8 || tiles > 512)
+        return false;
+    return (K <= 256 && (M >= 5 || tiles >= 125)) || (K <= 512 && M >= 5 && tiles >= 125 && tiles <= 256);
+}
+
 // Whether weights in rows of `row` codes are taken so.
 inline bool small_rows_apply(const int8_t *Wq, int row, int M, int N, bool staged)
 {
@@ -2876,6 +2887,11 @@ int linear_f32_dynquant(const float *X, const int8_t *Wq, const float *sw, int s
         const int alone = ragged_rows(kNoScratch);
         return alone >= 0 ? alone : status;
     };
+    if (gemv_rows_applies(X, Wq, M, N, K) && few_rows_by_tiles(M, N, K) && !x_on_host) {
+        const int small = launch_small_rows(X, K, Wq, K, sw, sw_stride, bias, Y, M, N, relu, result, false);
+        if (small >= 0)
+            return small;
+    }
     if (gemv_rows_applies(X, Wq, M, N, K) && gemv_rows_fused_quant_faster(M, N, K) && !tuning().no_fused_decode) {
         // a few tokens and short rows: same, each workgroup quantizes the rows itself
         GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, K, 1, sw_stride, relu ? 1 : 0, 1, nullptr, X, 0};
