@@ -653,6 +653,25 @@ def test_rows_quantized_by_each_tile(hip, mnk):
     layer.release()
 
 
+# Y in the memory of X: all of it has been quantized before the product's launch stores anything
+@pytest.mark.parametrize("mnk", [(64, 256, 256), (33, 512, 512), (250, 1000, 768), (20, 200, 256), (70, 700, 500)])
+def test_results_over_their_input(hip, mnk):
+    m, n, k = mnk
+    rng = np.random.default_rng(m + n + k)
+    x, w = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    want = _oracle_linear(x, w, None, PER_CHANNEL)
+    layer = QuantLinearLayer(w, None, requires_grad=False)
+    qw = layer.quantized()
+    room = HipTensor.empty([m * max(n, k) + 64], np.float32)
+    print(mnk, flush=True)
+    for at in (0, 4, 64):
+        capi.call("vtl_hip_upload", room.ptr, x.ctypes.data, x.nbytes)
+        capi.call("vtl_hip_layer_f32", C.byref(qw.layer), room.ptr, room.ptr + 4 * at, m, 0, None, 0)
+        assert np.array_equal(room.cpu()[at:at + m * n].reshape(m, n), want), at
+    layer.release()
+    room.release()
+
+
 @pytest.mark.parametrize("rows", [9, 33, 250])
 @pytest.mark.parametrize("dims", [(300, 512, 640, 40), (784, 700, 1024, 1100, 10), (64, 2000, 384, 384)])
 def test_layers_hand_rows_on_as_values_or_codes(hip, knobs, rows, dims):

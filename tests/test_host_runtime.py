@@ -341,6 +341,32 @@ print("done")
 """)
 
 
+def test_results_over_what_they_are_made_from_come_behind_the_quantizer(fake_runtime):
+    """A quantized linear whose Y lies over X, or over the weights, is not made by tiles that read their rows while others are stored."""
+    _run(fake_runtime, r"""
+import re
+runtime()
+p = malloc_on(0, 16 << 20)
+far = p + (8 << 20)
+def kernels(x, y, m, n, k, row=0, w=p + (4 << 20)):
+    events()
+    layer = capi.Layer(0, 1, n, k, w, far, None, row)
+    st = capi.status("vtl_hip_layer_f32", C.byref(layer), x, y, m, 0, None, 0)
+    found = [re.search("linear_small|linear_gemv|quantize|gemm_i8_small", l[4]) for l in lines() if l[0] == "launch"]
+    return [f.group() for f in found if f]
+for m, n, k, row in ((64, 256, 256, 0), (33, 1000, 512, 0), (64, 128, 500, 512), (20, 100, 256, 0)):
+    assert kernels(p, far, m, n, k, row) == ["linear_small"]
+    ends = p + 4 * m * k
+    for y in (p, p + 16, ends - 4, p + 64):
+        assert kernels(p, y, m, n, k, row)[0] == "quantize", (m, n, k, y - p)
+        assert kernels(y, p + 16, m, n, k, row)[0] == ("quantize" if p + 16 + 4 * m * n > y else "linear_small"), (m, n, k, y - p)
+    assert kernels(p, ends, m, n, k, row) == ["linear_small"]                     # behind it
+    assert kernels(p, p + (4 << 20) + 16, m, n, k, row)[0] == "quantize"
+assert kernels(p, far, 8, 14336, 256) == ["linear_small"] and kernels(p, p, 8, 14336, 256, w=p + (1 << 20)) == ["linear_gemv"]
+print("done")
+""")
+
+
 def test_where_gradients_share_a_launch(fake_runtime):
     """Not where dW is few rows of millions of values, or large enough for shapes of its own."""
     _run(fake_runtime, r"""

@@ -2708,11 +2708,14 @@ inline bool small_rows_apply(const int8_t *Wq, int row, int M, int N, bool stage
            small_quantized_faster(M, N, row, staged);
 }
 
-// f32 rows of x_cols values, in device memory, against weights in rows of `row` codes (x_cols, or padded); -1: not taken.
+// f32 rows of x_cols values, in device memory, against weights in rows of `row` codes (x_cols, or padded); -1: not taken, as where Y lies over
+// what it is made from: each tile reads its rows while others of the same rows are stored, where a quantizer's launch has read them all before.
 int launch_small_rows(const float *X, int x_cols, const int8_t *Wq, int row, const float *sw, int sw_stride, const float *bias, float *Y, int M,
                       int N, int relu, HostResult *result, bool staged)
 {
-    if (!small_rows_apply(Wq, row, M, N, staged))
+    const size_t y_bytes = (size_t)M * (size_t)N * sizeof(float);
+    if (!small_rows_apply(Wq, row, M, N, staged) || vtlhip::meet(X, (size_t)M * (size_t)x_cols * sizeof(float), Y, y_bytes) ||
+        vtlhip::meet(Wq, (size_t)N * (size_t)row, Y, y_bytes))
         return -1;
     GemmArgs g{nullptr, Wq, Y, nullptr, sw, bias, M, N, row, 1, sw_stride, relu ? 1 : 0, 1, nullptr, X, 0};
     g.x_cols = x_cols;
