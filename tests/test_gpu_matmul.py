@@ -614,3 +614,26 @@ def test_slices_that_meet_within_their_launch(hip, mnk, dt, knobs):
             assert np.array_equal(matmul_hip_host(a, np.ascontiguousarray(w.T)), want), (tile, splits)
     for t in (A, W, B, Wt):
         t.release()
+
+
+# C in the memory of A or of B, K in slices: what the slices are made from has been read before anything is stored
+@pytest.mark.parametrize("mnk", [(64, 256, 2000), (64, 64, 4096), (33, 65, 800)])
+@pytest.mark.parametrize("dt", [np.float32, np.float64])
+@pytest.mark.parametrize("over", ["a", "b"])
+def test_products_over_their_operands(hip, mnk, dt, over, knobs):
+    m, n, k = mnk
+    rng = np.random.default_rng(m + n * 3 + k * 5)
+    a, w = rng.integers(-8, 9, (m, k)).astype(dt), rng.integers(-8, 9, (n, k)).astype(dt)
+    want = (a.astype(np.int64) @ w.astype(np.int64).T).astype(dt)
+    name = "vtl_hip_linear_f32" if dt == np.float32 else "vtl_hip_linear_f64"
+    print(mnk, dt.__name__, over, flush=True)
+    knobs.setenv("VTL_HIP_MATMUL_TILE", "2")
+    for splits in ("2", "7", "25"):
+        knobs.setenv("VTL_HIP_MATMUL_SPLITS", splits)
+        A, W = dev(a), dev(w)
+        at = (A if over == "a" else W).ptr + 3 * dt().itemsize
+        capi.call(name, A.ptr, W.ptr, None, at, m, n, k, 0)
+        got = (A if over == "a" else W).cpu().reshape(-1)[3:3 + m * n].reshape(m, n)
+        assert np.array_equal(got, want), splits
+        A.release()
+        W.release()

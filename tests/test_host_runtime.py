@@ -367,6 +367,29 @@ print("done")
 """)
 
 
+def test_products_over_their_operands_come_behind_all_of_them(fake_runtime):
+    """Slices of K meet within their launch only where C is memory of its own: elsewhere a launch behind it adds them up."""
+    _run(fake_runtime, r"""
+runtime()
+p = malloc_on(0, 32 << 20)
+far = p + (16 << 20)
+def launches(name, *args):
+    events()
+    assert capi.status(name, *args) == capi.OK
+    return count("launch", events())
+for name, size in (("f32", 4), ("f64", 8)):
+    for m, n, k in ((64, 256, 2000), (64, 64, 4096), (32, 1024, 1024)):
+        a, b = p, p + m * k * size
+        end = b + n * k * size
+        assert launches("vtl_hip_matmul_" + name, a, b, far, m, n, k, 0, 0) == 1, (name, m, n, k)
+        assert launches("vtl_hip_matmul_" + name, a, b, end, m, n, k, 0, 1) == 1
+        for c in (a, a + 4 * size, b - size, b, end - size):
+            assert launches("vtl_hip_matmul_" + name, a, b, c, m, n, k, 0, 0) == 2, (name, m, n, k, c - p)
+            assert launches("vtl_hip_linear_" + name, a, b, None, c, m, n, k, 0) == 2, (name, m, n, k, c - p)
+print("done")
+""")
+
+
 def test_where_gradients_share_a_launch(fake_runtime):
     """Not where dW is few rows of millions of values, or large enough for shapes of its own."""
     _run(fake_runtime, r"""

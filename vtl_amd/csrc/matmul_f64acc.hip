@@ -1026,11 +1026,14 @@ struct Partial {
 constexpr int kFoldFrom = 800;
 
 // The slices of a launch with tiles of bm x bn (kK8, kK4 or kWide) meet within it, where the stream has counters (not while it is being captured: replays of two graphs
-// may meet) and the memory is there; else g is left as it is.
+// may meet) and the memory is there; else g is left as it is.  Nor where C lies over A or B: a tile is stored while others still read them.
+template <typename T>
 void fold_slices(MatmulArgs &g, int bm, int bn, int slices, Partial &partial, bool alone, hipStream_t st)
 {
     const int64_t tiles = (int64_t)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn);
-    const int slot = tiles <= kFoldTiles && g.K >= kFoldFrom ? vtlhip::stream_slot(st) : -1;
+    const size_t m = (size_t)g.M, n = (size_t)g.N, k = (size_t)g.K, c_bytes = m * n * sizeof(T);
+    const bool over = vtlhip::meet(g.C, c_bytes, g.A, m * k * sizeof(T)) || vtlhip::meet(g.C, c_bytes, g.B, n * k * sizeof(T));
+    const int slot = tiles <= kFoldTiles && g.K >= kFoldFrom && !over ? vtlhip::stream_slot(st) : -1;
     if (slot < 0 || !(g.partial = partial.take((size_t)tiles * (size_t)slices * (size_t)(bm * bn) * sizeof(double), alone)))
         return;
     g.fold_slices = slices;
@@ -1047,7 +1050,7 @@ int launch_direct(MatmulArgs g, Kind kind, bool ta, bool tb, Plan plan, bool alo
     Partial partial;
     if (slices > 1) {
         if (!checked && (plan.shape == kK8 || plan.shape == kK4 || plan.shape == kWide))
-            fold_slices(g, kTileM[kind][plan.shape], kTileN[kind][plan.shape], slices, partial, alone, st);
+            fold_slices<T>(g, kTileM[kind][plan.shape], kTileN[kind][plan.shape], slices, partial, alone, st);
         if (!g.partial)
             g.partial = partial.take((size_t)slices * (size_t)g.M * (size_t)g.N * sizeof(double), alone);
         if (!g.partial) {   // no memory, or a capture that may not allocate: K in one piece
@@ -1266,7 +1269,7 @@ bool backward_in_one(vtlhip::HostResult *result, const T *grad, const T *x, cons
     Partial partial;
     int cut = slices;
     if (cut > 1)
-        fold_slices(g.dx, 32, kTileN[kind][px.shape], cut, partial, alone, current_stream());
+        fold_slices<T>(g.dx, 32, kTileN[kind][px.shape], cut, partial, alone, current_stream());
     if (cut > 1 && !g.dx.partial && !(g.dx.partial = partial.take((size_t)cut * (size_t)m * (size_t)k * sizeof(double), alone))) {
         g.dx.slice_steps = steps;   // no memory, or a capture that may not allocate: K in one piece
         cut = 1;
