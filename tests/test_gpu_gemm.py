@@ -431,3 +431,21 @@ def test_small_products_at_the_edges_of_their_rule(hip, mnk):
     assert np.array_equal(q.cpu(), want_q) and np.array_equal(s.cpu(), want_s)
     for h in (A, B, dsa, dsb, dbias, y, q, s):
         h.release()
+
+
+# Sums in the memory of an operand, K in ranges: both operands have been read before anything is stored
+@pytest.mark.parametrize("mnk", [(100, 500, 3312), (64, 640, 3312)])
+@pytest.mark.parametrize("over", ["a", "b"])
+def test_products_over_their_operands(hip, mnk, over):
+    m, n, k = mnk
+    a, bt, *_ = workloads.square_int8_gemm(m, n, k, seed=m + n + k)
+    if over == "a":     # room for the sums
+        a = np.concatenate([a, np.zeros((max(0, -(-4 * m * n // k) - m), k), np.int8)])
+    A, B = dev(a), dev(bt)
+    print(mnk, over, flush=True)
+    t = A if over == "a" else B
+    capi.call("vtl_hip_gemm_i8_i32", A.ptr, B.ptr, t.ptr, m, n, k)
+    got = t.cpu().reshape(-1)[:4 * m * n].copy().view(np.int32).reshape(m, n)
+    assert np.array_equal(got, oracle.gemm_i8_i32(a[:m].copy(), bt, threads=CPU_THREADS))
+    A.release()
+    B.release()

@@ -390,6 +390,28 @@ print("done")
 """)
 
 
+def test_int8_products_over_their_operands_come_behind_all_of_them(fake_runtime):
+    """Small int8 products whose K the tile kernels cut: with the results over an operand they are cut, and added up behind it."""
+    _run(fake_runtime, r"""
+import re
+runtime()
+p = malloc_on(0, 32 << 20)
+far = p + (16 << 20)
+def kernels(name, *args):
+    events()
+    assert capi.status(name, *args) == capi.OK
+    found = [re.search("gemm_i8_small|gemm_i8|finalize", l[4]) for l in lines() if l[0] == "launch"]
+    return [f.group() for f in found if f]
+for m, n, k in ((100, 500, 3312), (64, 640, 3312)):
+    a, b = p, p + m * k
+    for y, want in ((far, ["gemm_i8_small"]), (b + n * k, ["gemm_i8_small"]), (a, ["gemm_i8", "finalize"]), (b - 16, ["gemm_i8", "finalize"]),
+                    (b + n * k - 16, ["gemm_i8", "finalize"])):
+        assert kernels("vtl_hip_linear_i8_f32", a, far + (8 << 20), 1, b, far + (9 << 20), 1, None, y, m, n, k, 0) == want, (m, n, k, y - p)
+        assert kernels("vtl_hip_gemm_i8_i32", a, b, y, m, n, k) == want, (m, n, k, y - p)
+print("done")
+""")
+
+
 def test_where_gradients_share_a_launch(fake_runtime):
     """Not where dW is few rows of millions of values, or large enough for shapes of its own."""
     _run(fake_runtime, r"""

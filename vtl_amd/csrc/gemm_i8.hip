@@ -2774,8 +2774,13 @@ int launch_gemm(const GemmArgs &g_in, hipStream_t st)
             return launch_skinny<F32OUT>(g, nwave == 2 ? 2 : 4, st);
     }
     const int64_t t32 = (int64_t)((g.M + 31) / 32) * ((g.N + 31) / 32);
-    // VTL_HIP_GEMM_SMALL 1 / 0 forces the choice (tests, tuning); 16 also the number of waves
-    if (small_set ? tn.gemm_small != 0 : small_product_faster(t32, g.K)) {
+    // VTL_HIP_GEMM_SMALL 1 / 0 forces the choice (tests, tuning); 16 also the number of waves.  (Not where the results lie over an operand: K in
+    // ranges, as the tile kernels may have it, has read both before anything is stored.)
+    const size_t out_bytes = (size_t)g.M * (size_t)g.N * 4;
+    const auto over = [&] {
+        return vtlhip::meet(g.out, out_bytes, g.A, (size_t)g.M * (size_t)g.K) || vtlhip::meet(g.out, out_bytes, g.Bt, (size_t)g.N * (size_t)g.K);
+    };
+    if (small_set ? tn.gemm_small != 0 : small_product_faster(t32, g.K) && !over()) {
         if (t32 > 0x7fffffff)
             return VTL_HIP_ERR_UNSUPPORTED;
         return launch_small<F32OUT, false>(g, t32, tn.gemm_small >= 16 || g.K > 4096 ? 16 : 8, st);
