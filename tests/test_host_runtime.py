@@ -576,6 +576,33 @@ print("done")
 """)
 
 
+def test_a_kernel_that_is_asked_for_is_the_one(fake_runtime):
+    """The switches that name a kernel for a few rows, or for more, come before the rule for rows that each tile quantizes."""
+    _run(fake_runtime, r"""
+import os, re
+runtime()
+p = malloc_on(0, 64 << 20)
+def kernels(m, n, k, **knobs):
+    os.environ.update(knobs)
+    capi.call("vtl_hip_reload_env")
+    for name in knobs:
+        del os.environ[name]
+    events()
+    capi.status("vtl_hip_linear_f32_dynquant", p, p + (16 << 20), p, None, p + (32 << 20), m, n, k, 0, None, 0)
+    found = [re.search("linear_small|linear_gemv_rows|quantize|skinny|streamk|gemm_i8", l[4]) for l in lines() if l[0] == "launch"]
+    return [f.group() for f in found if f]
+for m, n, k in ((8, 4000, 512), (8, 8192, 512), (5, 600, 256), (3, 4000, 256), (8, 14336, 256)):
+    assert kernels(m, n, k) == ["linear_small"], (m, n, k)
+    assert kernels(m, n, k, VTL_HIP_GEMV_ROWS="1") == ["linear_gemv_rows"], (m, n, k)
+    got = kernels(m, n, k, VTL_HIP_GEMV_ROWS="0")
+    assert "linear_gemv_rows" not in got and "linear_small" not in got, (m, n, k, got)
+for m, n, k in ((64, 256, 512), (33, 1000, 256)):
+    assert kernels(m, n, k) == kernels(m, n, k, VTL_HIP_GEMV_ROWS="1") == ["linear_small"], (m, n, k)
+    assert kernels(m, n, k, VTL_HIP_SKINNY_TILED="1") == ["quantize", "skinny"], (m, n, k)
+print("done")
+""")
+
+
 def test_short_rows_are_not_refused_for_want_of_scratch(fake_runtime):
     """Where a call that would take two launches may not allocate, the launch that needs no scratch serves."""
     _run(fake_runtime, _SHORT_ROWS + r"""

@@ -2701,9 +2701,11 @@ inline bool few_rows_by_tiles(int M, int N, int K)
     return (K <= 256 && (M >= 5 || tiles >= 125)) || (K <= 512 && M >= 5 && tiles >= 125 && tiles <= 256);
 }
 
-// Whether weights in rows of `row` codes are taken so.
+// Whether weights in rows of `row` codes are taken so.  (Not where VTL_HIP_GEMV_ROWS or VTL_HIP_SKINNY_TILED=1 names the kernel for so many rows.)
 inline bool small_rows_apply(const int8_t *Wq, int row, int M, int N, bool staged)
 {
+    if (M <= 32 ? M >= 2 && M <= 8 && tuning().gemv_rows >= 0 : tuning().skinny_tiled > 0)
+        return false;
     return row % 16 == 0 && aligned16(Wq) && !tuning().no_fused_decode && tuning().gemm_config < 0 && tuning().gemm_small != 0 &&
            small_quantized_faster(M, N, row, staged);
 }
