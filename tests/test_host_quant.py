@@ -159,3 +159,22 @@ for capturing in (False, True):
     assert any("host_copy" in l[4] for l in lines() if l[0] == "launch") != capturing
 print("done")
 """)
+
+
+# (a process for each: no kernel empties a slot here)
+@pytest.mark.parametrize("per_row,extra", [(0, 0), (0, 4096), (0, 65536), (1, 0), (1, 4096), (1, 65536)])
+def test_little_beside_codes_takes_no_launch_of_its_own(fake_runtime, per_row, extra):  # noqa: F811
+    """A bias, and the scale of all rows, go up with the first of three launches of codes."""
+    _run(fake_runtime, r"""
+import os
+os.environ["VTL_HIP_HOST_QUANTIZE"] = "1"
+runtime()
+p = malloc_on(0, 64 << 20)
+host = (C.c_float * (1 << 20))()
+events()
+extra = EXTRA
+assert capi.status("vtl_hip_upload_quantized", host, 768, 512, PER_ROW, p, p, p if extra else None, host if extra else None, extra) == capi.OK
+log = [l[4] for l in lines() if l[0] == "launch"]
+assert sum("host_copy" in k for k in log) == 3, log
+print("done")
+""".replace("PER_ROW", str(per_row)).replace("EXTRA", str(extra)))

@@ -909,12 +909,12 @@ struct Pieces {
     Pieces(const Source *from, int sources, bool host)
     {
         const size_t most = host ? kSlotBytes : kMaxSegments * kSlotBytes;
-        const int pieces = host ? kMaxSegments / 2 : kMaxSegments;   // of a launch (codes take two segments)
+        const auto segments = [&](int s) { return from[s].host && !from[s].one ? 2 : 1; };   // (codes with a scale a row take two)
         for (int pass = 0; pass < 2; pass++) {
             size_t ahead = 0, launch = kFirstLaunch, room = launch;
             for (int s = 0; s < sources; s++)
                 ahead += from[s].bytes;
-            int n = 0, in_launch = 0;
+            int n = 0, in_launch = 0;   // pieces, and segments of the launch that is being filled
             for (int s = 0; s < sources; s++)
                 for (size_t at = 0; at < from[s].bytes;) {
                     if (in_launch == 0 && host)
@@ -945,9 +945,10 @@ struct Pieces {
                     ahead -= take;
                     room -= take < room ? take : room;
                     n++;
-                    in_launch++;
+                    in_launch += segments(s);
                     const size_t unit = at < from[s].bytes ? from[s].unit : 0;   // of what comes next
-                    const bool end = room < (unit ? unit : 1) || in_launch == pieces || ahead == 0;
+                    const bool end = ahead == 0 || room < (unit ? unit : 1) ||
+                                     in_launch + segments(at < from[s].bytes || s + 1 == sources ? s : s + 1) > kMaxSegments;
                     if (pass)
                         piece[n - 1].last_of_launch = end;
                     if (end) {
