@@ -324,7 +324,7 @@ import numpy as np
 import oracle
 from vtl_amd import capi
 from vtl_amd.tensor import HipTensor
-# Rows that are quantized as they come over the link, without a wait: the caller's memory is its own again on return, and small
+# Rows that are quantized on their way to the device, without a wait: the caller's memory is its own again on return, and small
 # and large transfers come directly behind, through the same staging memory
 capi.call("vtl_hip_set_device", 0)
 rng = np.random.default_rng(9)
@@ -355,9 +355,10 @@ print("ok")
 """
 
 
-def test_uploads_behind_rows_quantized_on_their_way(hip):
+@pytest.mark.parametrize("by_host", ["0", "1"])      # as they come over the link, and by the host's threads (with up to 64 KiB beside them)
+def test_uploads_behind_rows_quantized_on_their_way(hip, by_host):
     done = subprocess.run([sys.executable, "-c", QUANTIZED_UPLOADS], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
-                          text=True, timeout=110)
+                          text=True, timeout=110, env={**os.environ, "VTL_HIP_HOST_QUANTIZE": by_host})
     assert done.returncode == 0 and done.stdout.rstrip().endswith("ok"), done.stdout[-3000:]
 
 

@@ -1,4 +1,4 @@
-"""Rows that are quantized as they come over the link: the same bits as an upload and the quantizer behind it.  (Beside tests that name
+"""Rows that are quantized on their way to the device, by the host's threads or as they come over the link: the same bits as an upload and the quantizer behind it.  (Beside tests that name
 streams each call waits for its end; without a wait, and with transfers behind it: test_gpu_null_stream.py.)"""
 import numpy as np
 import pytest
@@ -11,19 +11,22 @@ from vtl_amd.tensor import HipTensor
 pytestmark = pytest.mark.gpu
 
 
-# 32 MiB and more in rows of 2048 and more are quantized on the way: edges of a workgroup's registers, rows that do not divide the pieces a transfer is
-# cut into (rows are not cut); less, longer, shorter and odd rows go in two steps
+# By the host's threads, rows of any of these lengths: more and less than what one thread makes, rows that do not divide the pieces a transfer is cut into
+# (rows are not cut).  By the device, 32 MiB and more in rows of 2048 to 8192 values as they come over the link: edges of a workgroup's registers, rows
+# that do not divide the pieces; less, longer, shorter and odd rows go in two steps.
 @pytest.mark.parametrize("rows,cols", [(8192, 1024), (8191, 1024), (8200, 1028), (4096, 2048), (4095, 2048), (4200, 2044), (4100, 2052), (3000, 2800), (2049, 4096), (2100, 4100),
                                        (1024, 8192), (1031, 8188), (1030, 8196), (33000, 256), (8300, 1023), (300, 1024), (1, 4)])
 @pytest.mark.parametrize("extra", [0, 4096 + 20])
-def test_same_bits_as_upload_and_quantize(hip, rows, cols, extra):
+@pytest.mark.parametrize("by_host", ["0", "1"])
+def test_same_bits_as_upload_and_quantize(hip, rows, cols, extra, by_host, knobs):
+    knobs.setenv("VTL_HIP_HOST_QUANTIZE", by_host)
     rng = np.random.default_rng(rows + cols)
     x = rng.standard_normal((rows, cols)).astype(np.float32) * np.float32(10.0) ** rng.integers(-3, 4, (rows, 1)).astype(np.float32)
     x[rows // 2] = 0.0
     x[rows // 3, :: 5] = np.nan
     x[-1, cols // 2] = np.inf
     more = rng.integers(0, 256, extra, dtype=np.uint8)
-    print("rows", rows, cols, extra, flush=True)
+    print("rows", rows, cols, extra, "by host" if by_host == "1" else "by device", flush=True)
     for per_row in (1, 0):
         xd = dev(x)
         want_q, want_s = xd.quantize_i8(0 if per_row else -1)
