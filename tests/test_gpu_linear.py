@@ -280,7 +280,7 @@ def test_session_reuses_buffers_on_second_forward(hip):
                                  (3, 2048, 1024), (4, 4099, 1040), (4, 2048, 2048), (3, 2051, 272),
                                  (5, 2048, 512), (8, 2050, 1024), (7, 9000, 1008), (6, 2048, 16 * 17),
                                  (8, 70001, 256), (2, 1, 256), (3, 7, 2048), (8, 64, 1024), (4, 100, 272),
-                                 (2, 1536, 4096), (8, 4000, 512), (3, 4000, 256),   # (not forced, the last two are quantized by tiles)
+                                 (2, 1536, 4096),
                                  # 48 MiB of weights and more: the instances with non-temporal weight loads
                                  (2, 14336, 4096), (4, 16400, 3072), (2, 8192, 8192), (7, 12300, 4096)])
 def test_few_token_fused_decode_equals_two_launch_path(hip, mnk, knobs):
@@ -319,6 +319,12 @@ def test_few_token_fused_decode_equals_two_launch_path(hip, mnk, knobs):
         S.release()
     for h in (X, W, SW, B):
         h.release()
+
+
+# Sizes that the tiles quantize where the kernel is not asked for
+@pytest.mark.parametrize("mnk", [(8, 4000, 512), (3, 4000, 256)])
+def test_few_token_fused_decode_is_the_one_that_was_asked_for(hip, mnk, knobs):
+    test_few_token_fused_decode_equals_two_launch_path(hip, mnk, knobs)
 
 
 @pytest.mark.parametrize("mnk", [(2, 2048, 256), (8, 14336, 4096), (8, 2077, 1280), (9, 3001, 512), (16, 12300, 8192),

@@ -355,11 +355,16 @@ print("ok")
 """
 
 
-@pytest.mark.parametrize("by_host", ["0", "1"])      # as they come over the link, and by the host's threads (with up to 64 KiB beside them)
-def test_uploads_behind_rows_quantized_on_their_way(hip, by_host):
+def test_uploads_behind_rows_quantized_on_their_way(hip):
     done = subprocess.run([sys.executable, "-c", QUANTIZED_UPLOADS], cwd=ROOT, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
-                          text=True, timeout=110, env={**os.environ, "VTL_HIP_HOST_QUANTIZE": by_host})
+                          text=True, timeout=110)
     assert done.returncode == 0 and done.stdout.rstrip().endswith("ok"), done.stdout[-3000:]
+
+
+@pytest.mark.parametrize("by_host", ["0", "1"])      # as they come over the link, and by the host's threads (with up to 64 KiB beside them)
+def test_uploads_behind_rows_quantized_by_the_host_and_on_the_link(hip, monkeypatch, by_host):
+    monkeypatch.setenv("VTL_HIP_HOST_QUANTIZE", by_host)     # (of the process that it starts)
+    test_uploads_behind_rows_quantized_on_their_way(hip)
 
 
 def test_products_from_several_threads_on_the_null_stream(hip):

@@ -17,16 +17,14 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("rows,cols", [(8192, 1024), (8191, 1024), (8200, 1028), (4096, 2048), (4095, 2048), (4200, 2044), (4100, 2052), (3000, 2800), (2049, 4096), (2100, 4100),
                                        (1024, 8192), (1031, 8188), (1030, 8196), (33000, 256), (8300, 1023), (300, 1024), (1, 4)])
 @pytest.mark.parametrize("extra", [0, 4096 + 20])
-@pytest.mark.parametrize("by_host", ["0", "1"])
-def test_same_bits_as_upload_and_quantize(hip, rows, cols, extra, by_host, knobs):
-    knobs.setenv("VTL_HIP_HOST_QUANTIZE", by_host)
+def test_same_bits_as_upload_and_quantize(hip, rows, cols, extra):
     rng = np.random.default_rng(rows + cols)
     x = rng.standard_normal((rows, cols)).astype(np.float32) * np.float32(10.0) ** rng.integers(-3, 4, (rows, 1)).astype(np.float32)
     x[rows // 2] = 0.0
     x[rows // 3, :: 5] = np.nan
     x[-1, cols // 2] = np.inf
     more = rng.integers(0, 256, extra, dtype=np.uint8)
-    print("rows", rows, cols, extra, "by host" if by_host == "1" else "by device", flush=True)
+    print("rows", rows, cols, extra, flush=True)
     for per_row in (1, 0):
         xd = dev(x)
         want_q, want_s = xd.quantize_i8(0 if per_row else -1)
@@ -40,6 +38,16 @@ def test_same_bits_as_upload_and_quantize(hip, rows, cols, extra, by_host, knobs
             assert np.array_equal(room.cpu()[16:16 + extra], more)
         for t in (xd, want_q, want_s, q, s, room):
             t.release()
+
+
+# Whatever processors the machine has: the rows of 32 MiB and more, by the device's kernel and by the host's threads
+@pytest.mark.parametrize("rows,cols", [(4096, 2048), (4095, 2048), (4200, 2044), (4100, 2052), (3000, 2800), (2049, 4096), (2100, 4100), (1024, 8192), (1031, 8188),
+                                       (1030, 8196)])
+@pytest.mark.parametrize("extra", [0, 4096 + 20])
+@pytest.mark.parametrize("by_host", ["0", "1"])
+def test_same_bits_by_the_host_and_on_the_link(hip, knobs, rows, cols, extra, by_host):
+    knobs.setenv("VTL_HIP_HOST_QUANTIZE", by_host)
+    test_same_bits_as_upload_and_quantize(hip, rows, cols, extra)
 
 
 def test_errors(hip):
