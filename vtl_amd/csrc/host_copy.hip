@@ -1119,7 +1119,7 @@ int download_large(Ring *r, char *dst, const char *src, size_t bytes, hipStream_
 // The host makes codes of f32 rows, and the link carries those: 180 MB of weights with their scales and the forward behind them 3640 -> 1480 us, 4 MiB
 // of activations through three layers 208 -> 157, 200 KB 28.7 -> 25.4 (16 processors).  Only above so many processors that the
 // caller and its helpers are about half of them: with fewer, memory is what a copy and the codes wait for alike (8 processors, GB/s of f32 by 4
-// threads: copied 35, quantized 32).
+// threads: copied 35, quantized 32; what one thread makes, up to kSmall, was not timed on such machines).
 constexpr int kQuantizeProcessors = 2 * Crew::kHelpers;
 
 const HostQuantizer *quantizer_to_use()

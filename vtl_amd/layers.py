@@ -104,7 +104,8 @@ def content_fingerprint(t: np.ndarray) -> int:
 
 # Weights of up to so many bytes, which one host thread makes codes of, and from so many on, which several do, go to the call that quantizes
 # them on their way to the device and takes the bias along.  (us of a forward, uploaded and then quantized, and so: 16 x 256 x 256 46 and 42,
-# 64 x 512 x 512 80 and 63, 64 x 600 x 1024 118 and 82.)
+# 64 x 512 x 512 80 and 63, 64 x 600 x 1024 118 and 82.  Codes are ahead in between too, 64 x 400 x 1024 100 and 78, but those sizes still
+# take the upload.)
 _QUANTIZED_UP_TO, _QUANTIZED_FROM = 1 << 20, 2 << 20
 
 
