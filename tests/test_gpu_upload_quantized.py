@@ -86,3 +86,24 @@ def test_by_the_host_and_by_the_device(hip, knobs, rows, cols):
         got.append(out)
     for a, b in zip(*got):
         assert np.array_equal(a, b, equal_nan=a.dtype == np.float32)
+
+
+# Forwards and weights where sizes say who quantizes, by them and by the device: few dense rows with one scale that are no whole vectors
+@pytest.mark.parametrize("rows,cols", [(2, 1023), (2, 1025), (3, 255), (3, 257), (8, 300), (8, 2047), (8, 2049), (5, 4001), (9, 1372)])
+def test_same_bits_whoever_quantizes(hip, knobs, rows, cols):
+    rng = np.random.default_rng(rows * 37 + cols)
+    x, w = rng.standard_normal((rows, cols)).astype(np.float32), rng.standard_normal((40, cols)).astype(np.float32)
+    print("rows", rows, cols, flush=True)
+    got = []
+    for who in ("0", "2"):
+        knobs.setenv("VTL_HIP_HOST_QUANTIZE", who)
+        out = []
+        for mode in (PER_CHANNEL, PER_TENSOR):
+            qw = QuantizedWeights(x, None, mode)
+            layer = QuantLinearLayer(w, None, mode=mode, requires_grad=False)
+            out += [qw.w_q.cpu().copy(), qw.sw.cpu().view(np.int32).copy(), layer.forward(x).copy()]
+            qw.release()
+            layer.release()
+        got.append(out)
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)

@@ -178,3 +178,31 @@ log = [l[4] for l in lines() if l[0] == "launch"]
 assert sum("host_copy" in k for k in log) == 3, log
 print("done")
 """.replace("PER_ROW", str(per_row)).replace("EXTRA", str(extra)))
+
+
+def test_few_ragged_rows_are_not_read_as_codes_over_the_link(fake_runtime):  # noqa: F811
+    """Two to eight rows with one scale that are no whole vectors, from 256 values on (two rows: 1024) and up to 16 KiB of codes: a launch of the device's quantizes them."""
+    _run(fake_runtime, r"""
+import os, re
+os.environ["VTL_HIP_HOST_QUANTIZE"] = "2"
+runtime()
+p = malloc_on(0, 64 << 20)
+host = (C.c_float * (1 << 20))()
+def first(rows, cols, per_channel=0, row_bytes=0, n=61):
+    layer = capi.Layer(0, per_channel, n, cols, p, p, None, row_bytes)
+    events()
+    capi.status("vtl_hip_forward_i8_host", host, rows, cols, C.byref(layer), 1, host)
+    found = [re.search("host_copy|linear_gemv|quantize|gemm_i8|pad_rows", l[4]) for l in lines() if l[0] == "launch"]
+    return [f.group() for f in found if f][0]
+for rows in range(2, 9):
+    start = 1024 if rows == 2 else 256
+    for cols in (17, 250, 255, 257, 1001, 1023, 1025, 1372, 2047, 4001):
+        got = first(rows, cols)
+        assert (got == "quantize") == (cols >= start and rows * cols <= 16384), (rows, cols, got)     # more codes are carried up
+    assert first(rows, 1372, 0, 1376) != "quantize" and first(rows, 1376) != "quantize"    # padded, whole
+assert first(9, 1372) != "quantize"
+os.environ["VTL_HIP_HOST_QUANTIZE"] = "1"
+capi.call("vtl_hip_reload_env")
+assert first(8, 1372) != "quantize"
+print("done")
+""")

@@ -317,7 +317,8 @@ struct Tuning {
     int skinny_tiled = -1;          // VTL_HIP_SKINNY_TILED: 1 / 0 force the 32x32-block weight-streaming kernel for M > 32
     int skinny_waves = 4;           // VTL_HIP_SKINNY_WAVES: 2, 4 or 8 waves (K ranges) per workgroup there
     int matmul_tile = 0;            // VTL_HIP_MATMUL_TILE: which kernel and tile the f64-accumulating matmul takes (matmul_f64acc.hip)
-    int host_quantize = -1;         // VTL_HIP_HOST_QUANTIZE: 1 / 0 force rows in host memory to be quantized by the host's / the device's units
+    int host_quantize = -1;         // VTL_HIP_HOST_QUANTIZE: 1 / 0 force rows in host memory to be quantized by the host's / the device's units; 2: by
+                                    // the host's where it is faster, with any number of processors
     int backward_group = -1;        // VTL_HIP_BACKWARD_GROUP: 1 / 0 force a backward's gradients in one launch on (where it can be) / off
     int matmul_splits = -1;         // VTL_HIP_MATMUL_SPLITS: K ranges of the f64-accumulating matmul
 };

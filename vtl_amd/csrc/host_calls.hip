@@ -54,6 +54,15 @@ constexpr int kFewRows = 32;
 // 1100 21.9 and 22.4, 64 x 256 x 784 24.2 and 29.3).
 constexpr size_t kCodesOverLink = (size_t)16 << 10;
 
+// Not two to eight dense rows with one scale that are no whole vectors: the product's matrix-vector kernel reads those in every workgroup, in parts, and from so many codes
+// on that is slower over the link than a quantizer's launch that reads f32 there once (us, quantized by a launch and read as codes: 3 x 80 x 251 17.2 and 15.7, but 7 x 48 x
+// 309 19.3 and 24.2, 5 x 126 x 422 18.6 and 21.0, 8 x 61 x 1372 23.7 and 36.3; 2 x 48 x 907 18.4 and 17.4, 2 x 48 x 1187 17.8 and 18.9).  Carried up they are 1 to 8 % behind
+// that launch as well, up to kCodesOverLink.
+bool few_ragged_rows(int rows, int cols, int row)
+{
+    return rows <= 8 && row % 16 != 0 && cols >= (rows == 2 ? 1024 : 256) && (size_t)rows * (size_t)row <= kCodesOverLink;
+}
+
 int check_layers(const vtl_hip_layer *layers, int count, int cols, int &out_cols)
 {
     for (int i = 0; i < count; i++) {
@@ -122,7 +131,9 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
         (rows > kFewRows || (rows > 1 && !layers[0].per_channel) || (rows > 8 && !layer_takes_input(layers[0], rows)))) {
         const vtl_hip_layer &l = layers[0];
         const int row = l.row_bytes > cols ? l.row_bytes : cols;
-        if ((size_t)rows * (size_t)row <= kCodesOverLink && input.stage_codes(x_host, rows, cols, l.per_channel, row)) {
+        if (few_ragged_rows(rows, cols, row) && vtlhip::tuning().host_quantize != 1) {
+            // (by the device, below)
+        } else if ((size_t)rows * (size_t)row <= kCodesOverLink && input.stage_codes(x_host, rows, cols, l.per_channel, row)) {
             in = static_cast<const int8_t *>(input.data);
             in_scales = input.scales;
         } else if (host_makes_codes(rows, cols, row)) {
