@@ -88,8 +88,10 @@ def test_by_the_host_and_by_the_device(hip, knobs, rows, cols):
         assert np.array_equal(a, b, equal_nan=a.dtype == np.float32)
 
 
-# Forwards and weights where sizes say who quantizes, by them and by the device: few dense rows with one scale that are no whole vectors
-@pytest.mark.parametrize("rows,cols", [(2, 1023), (2, 1025), (3, 255), (3, 257), (8, 300), (8, 2047), (8, 2049), (5, 4001), (9, 1372)])
+# Forwards and weights where sizes say who quantizes, by them and by the device: few dense rows with one scale that are no whole vectors, and short rows
+@pytest.mark.parametrize("rows,cols", [(2, 1023), (2, 1025), (3, 255), (3, 257), (8, 300), (8, 2047), (8, 2049), (5, 4001), (9, 1372),
+                                       (264, 31), (265, 31), (512, 32), (513, 32), (86, 191), (86, 192), (129, 128), (341, 192), (64, 256), (64, 257), (8456, 31),
+                                       (8457, 32)])
 def test_same_bits_whoever_quantizes(hip, knobs, rows, cols):
     rng = np.random.default_rng(rows * 37 + cols)
     x, w = rng.standard_normal((rows, cols)).astype(np.float32), rng.standard_normal((40, cols)).astype(np.float32)

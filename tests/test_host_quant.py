@@ -206,3 +206,38 @@ capi.call("vtl_hip_reload_env")
 assert first(8, 1372) != "quantize"
 print("done")
 """)
+
+
+_SHORT_ROWS = r"""
+import os
+os.environ["VTL_HIP_HOST_QUANTIZE"] = "WHO"
+runtime()
+p = malloc_on(0, 64 << 20)
+host = (C.c_float * (3 << 20))()
+events()
+if "WHAT" == "forward":
+    layer = capi.Layer(0, PER_ROW, 24, NCOLS, p, p, None, 0)
+    capi.status("vtl_hip_forward_i8_host", host, NROWS, NCOLS, C.byref(layer), 1, host)
+else:
+    capi.status("vtl_hip_upload_quantized", host, NROWS, NCOLS, PER_ROW, p, p, None, None, 0)
+by = "device" if any("quantize" in l[4] for l in lines() if l[0] == "launch") else "host"
+assert by == "BY", by
+print("done")
+"""
+
+
+# (a process for each call: no kernel empties a slot here)
+@pytest.mark.parametrize("what,per_row,device,host", [
+    ("forward", 1, [(1000, 31), (178, 160), (2100, 48), (104, 256), (341, 192), (1400, 187), (9000, 31)],
+     [(342, 192), (513, 128), (64, 257), (120, 2000), (9000, 32)]),
+    ("forward", 0, [(1000, 31), (1000, 63), (9000, 31)], [(257, 64), (9000, 32)]),
+    ("weights", 1, [(300, 31), (513, 32), (178, 160), (86, 191), (1400, 127), (9000, 31)], [(264, 31), (512, 32), (86, 192), (129, 128), (9000, 32)]),
+    ("weights", 0, [(1000, 31), (9000, 31)], [(500, 31), (1000, 32), (9000, 32)])])
+def test_short_rows_are_quantized_by_the_device(fake_runtime, what, per_row, device, host):  # noqa: F811
+    """Rows that cost the host's units more than the link saves: activations, and weights."""
+    calls = [(r, c, 2, "device") for r, c in device] + [(r, c, 2, "host") for r, c in host] + [(*device[0], 1, "host")]
+    for rows, cols, asked, by in calls:
+        program = _SHORT_ROWS
+        for name, value in (("WHO", asked), ("WHAT", what), ("PER_ROW", per_row), ("NROWS", rows), ("NCOLS", cols), ("BY", by)):
+            program = program.replace(name, str(value))
+        _run(fake_runtime, program)

@@ -103,6 +103,8 @@ bool upload_rows(const float *src, int64_t rows, int64_t cols, int8_t *q, float 
 // scale; `row` bytes from one row of codes to the next (zeros behind the codes).  False: to be quantized by the device, as always
 // where the host does not make codes of such rows.
 bool host_makes_codes(int64_t rows, int64_t cols, int64_t row);
+// Whether such rows are long enough for the host to be the faster.
+bool rows_long_enough(int64_t rows, int64_t cols, int per_row);
 bool upload_codes(const float *src, int64_t rows, int64_t cols, int per_row, int8_t *q, int64_t row, float *scale, void *extra_dst,
                   const void *extra_src, size_t extra_bytes, int &status);
 

@@ -63,6 +63,20 @@ bool few_ragged_rows(int rows, int cols, int row)
     return rows <= 8 && row % 16 != 0 && cols >= (rows == 2 ? 1024 : 256) && (size_t)rows * (size_t)row <= kCodesOverLink;
 }
 
+// Whether activations beyond that are made codes of by the host, where rows_long_enough says so too.  On the null stream alone the launch that quantizes them
+// reads up to 1 MiB of them over the link itself, where weights are uploaded first, so the host is behind it for longer (us, by the device and by the host, rows x
+// values: scales per row 130 x 256 25.2 and 26.3, 98 x 200 21.6 and 23.1, but 106 x 363 24.0 and 23.1, 766 x 240 49.5 and 43.2; one scale 763 x 36 25.7 and 27.3, 1437 x
+// 35 39.2 and 40.8, but 400 x 67 25.6 and 24.9).
+bool activations_long_enough(const vtl_hip_layer &l, int rows, int cols)
+{
+    const size_t codes = (size_t)rows * (size_t)cols;
+    if (!vtlhip::rows_long_enough(rows, cols, l.per_channel))
+        return false;
+    if (!vtlhip::single_stream() || codes * sizeof(float) > (size_t)1 << 20 || vtlhip::tuning().host_quantize == 1)
+        return true;
+    return l.per_channel ? cols > 256 || codes >= (size_t)64 << 10 : cols >= 64;
+}
+
 int check_layers(const vtl_hip_layer *layers, int count, int cols, int &out_cols)
 {
     for (int i = 0; i < count; i++) {
@@ -136,7 +150,7 @@ int forward_layers(const float *x_host, int rows, int cols, const vtl_hip_layer 
         } else if ((size_t)rows * (size_t)row <= kCodesOverLink && input.stage_codes(x_host, rows, cols, l.per_channel, row)) {
             in = static_cast<const int8_t *>(input.data);
             in_scales = input.scales;
-        } else if (host_makes_codes(rows, cols, row)) {
+        } else if (activations_long_enough(l, rows, cols) && host_makes_codes(rows, cols, row)) {
             VTL_STEP(codes.take((size_t)rows * (size_t)row));
             VTL_STEP(scales.take((l.per_channel ? (size_t)rows : 1) * sizeof(float)));
             int status = VTL_HIP_OK;
@@ -447,7 +461,8 @@ int vtl_hip_upload_quantized(const float *src_host, int64_t rows, int64_t cols, 
     if (rows < 0 || cols < 0 || (rows > 0 && cols > 0 && (!src_host || !q)) || (extra_bytes && (!extra_device || !extra_host)))
         return VTL_HIP_ERR_INVALID_ARG;
     int status = VTL_HIP_OK;
-    if (scale && rows > 0 && cols > 0 &&
+    // (once a stream has been named, a release of the f32 memory would wait for the device: 868 x 64 with a small forward 80 us, as codes 56)
+    if (scale && rows > 0 && cols > 0 && (!single_stream() || rows_long_enough(rows, cols, per_row)) &&
         upload_codes(src_host, rows, cols, per_row, q, cols, scale, extra_device, extra_host, extra_bytes, status))
         return status;
     if (per_row && scale && rows > 0 && cols > 0 &&

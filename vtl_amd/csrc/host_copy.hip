@@ -1282,6 +1282,22 @@ bool host_makes_codes(int64_t rows, int64_t cols, int64_t row)
            (single_stream() || !stream_is_capturing(current_stream()));
 }
 
+// A row costs the host's units two divisions and two ends that are no whole vectors beside its values: up to kSmall, which one thread makes, that of short rows outweighs
+// what the link saves, and that of rows of fewer than 32 values for several threads too.  A layer's weights and a small forward, parts of the time with the upload that was
+// there before, by the device and by the host: scales per row, from 16 K codes on, 16 to 31 values 0.97 and 1.21 to 1.65, 32 to 63 0.97 and 1.05 to 1.40, 64 to 127 0.97 and
+// 0.96 to 1.09, 128 to 191 0.96 and 0.99, whole steps of 64 of them 0.97 and 0.94, 192 to 255 0.96 and 0.95, 256 and more 0.96 and 0.93; one scale, 16 to 31 values 0.93 and
+// 0.95, from 64 K codes on 0.96 and 1.03, 32 to 63 0.95 and 0.92.  Forward, scales per row: 178 x 160 26.9 us before, 30.3 by the host, 1770 x 48 33.3 and 40.7, 185 x 196 22.5
+// and 24.0; beyond kSmall 16 to 31 values 1 and 1.06 to 1.19, 32 to 63 1 and 0.96.
+bool rows_long_enough(int64_t rows, int64_t cols, int per_row)
+{
+    const size_t codes = (size_t)rows * (size_t)cols;
+    if (tuning().host_quantize == 1 || codes <= (size_t)(per_row && cols < 32 ? 8 : 16) << 10)
+        return true;
+    if (!per_row || codes * sizeof(float) > kSmall)
+        return cols >= 32;
+    return cols >= 192 || (cols >= 128 && cols % 64 == 0);
+}
+
 bool upload_codes(const float *src, int64_t rows, int64_t cols, int per_row, int8_t *q, int64_t row, float *scale, void *extra_dst,
                   const void *extra_src, size_t extra_bytes, int &status)
 try {
