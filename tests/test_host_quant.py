@@ -241,3 +241,21 @@ def test_short_rows_are_quantized_by_the_device(fake_runtime, what, per_row, dev
         for name, value in (("WHO", asked), ("WHAT", what), ("PER_ROW", per_row), ("NROWS", rows), ("NCOLS", cols), ("BY", by)):
             program = program.replace(name, str(value))
         _run(fake_runtime, program)
+
+
+def test_few_ragged_rows_go_up_as_codes_on_a_stream(fake_runtime):  # noqa: F811
+    """Once a stream has been named a launch that quantizes them would have an upload in front."""
+    _run(fake_runtime, r"""
+import os
+os.environ["VTL_HIP_HOST_QUANTIZE"] = "2"
+runtime()
+p = malloc_on(0, 64 << 20)
+host = (C.c_float * (1 << 16))()
+capi.call("vtl_hip_set_stream", 4096)
+events()
+layer = capi.Layer(0, 0, 61, 1372, p, p, None, 0)
+capi.status("vtl_hip_forward_i8_host", host, 8, 1372, C.byref(layer), 1, host)
+names = [l[4] for l in lines() if l[0] == "launch"]
+assert any("host_copy" in n for n in names) and not any("quantize" in n for n in names), names
+print("done")
+""")

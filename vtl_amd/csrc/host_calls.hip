@@ -57,10 +57,10 @@ constexpr size_t kCodesOverLink = (size_t)16 << 10;
 // Not two to eight dense rows with one scale that are no whole vectors: the product's matrix-vector kernel reads those in every workgroup, in parts, and from so many codes
 // on that is slower over the link than a quantizer's launch that reads f32 there once (us, quantized by a launch and read as codes: 3 x 80 x 251 17.2 and 15.7, but 7 x 48 x
 // 309 19.3 and 24.2, 5 x 126 x 422 18.6 and 21.0, 8 x 61 x 1372 23.7 and 36.3; 2 x 48 x 907 18.4 and 17.4, 2 x 48 x 1187 17.8 and 18.9).  Carried up they are 1 to 8 % behind
-// that launch as well, up to kCodesOverLink.
+// that launch as well, up to kCodesOverLink; once a stream has been named that launch has an upload in front, and codes are 1 to 10 % ahead (5 x 48 x 1162 39.1 and 35.0).
 bool few_ragged_rows(int rows, int cols, int row)
 {
-    return rows <= 8 && row % 16 != 0 && cols >= (rows == 2 ? 1024 : 256) && (size_t)rows * (size_t)row <= kCodesOverLink;
+    return vtlhip::single_stream() && rows <= 8 && row % 16 != 0 && cols >= (rows == 2 ? 1024 : 256) && (size_t)rows * (size_t)row <= kCodesOverLink;
 }
 
 // Whether activations beyond that are made codes of by the host, where rows_long_enough says so too.  On the null stream alone the launch that quantizes them
